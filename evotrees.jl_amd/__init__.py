@@ -13,9 +13,6 @@ Julia is not available where this package is developed, so the host side is Pyth
 streams are numpy's (PCG64), not Julia's Xoshiro, hence models are not stream-identical to a
 Julia run with the same seed — the trees are identical for identical masks/column samples.
 """
-import os
-from concurrent.futures import ThreadPoolExecutor
-
 import numpy as np
 
 from . import _lib
@@ -147,30 +144,38 @@ class EvoTree:
         return predict(self, data, ntree_limit=ntree_limit, device=device)
 
 
-def _per_feature(fn, F):
-    """[fn(0), ..., fn(F - 1)], on a few threads when there are enough features (numpy's sorts release the GIL)."""
-    workers = min(16, os.cpu_count() or 1, F)
-    if workers < 2 or F < 8:
-        return [fn(j) for j in range(F)]
-    with ThreadPoolExecutor(workers) as ex:
-        return list(ex.map(fn, range(F)))
+def _sample_rows(N, nbins, rng):
+    """The rows the edges are computed on, ascending (None: all of them), and how many."""
+    nobs = min(N, 1000 * nbins)
+    return (np.sort(rng.choice(N, nobs, replace=False)) if nobs < N else None), nobs
+
+
+def _quantiles(cols, idx, n, nbins):
+    """Type-7 quantiles at (1..nbins-1)/nbins of every column's values at the rows idx (None: the first n), as np.quantile computes
+    them in Float64: between the order statistics a and b around position (n - 1) q, from the nearer of the two."""
+    at = (n - 1) * (np.arange(1, nbins) / nbins)
+    lo = np.floor(at)
+    t = at - lo
+    lo = lo.astype(np.int64)
+    ranks, back = np.unique(np.concatenate([lo, np.minimum(lo + 1, n - 1)]), return_inverse=True)
+    v = _lib.order_stats(cols, idx, n, ranks)[:, back]
+    a, b = v[:, :nbins - 1], v[:, nbins - 1:]
+    with np.errstate(invalid="ignore", over="ignore"):
+        d = b - a
+        return np.where(t >= 0.5, b - d * (1 - t), a + d * t)
 
 
 def get_edges(x, nbins, rng):
     """get_edges, src/fit-utils.jl:7-24: type-7 quantiles at (1..nbins-1)/nbins of <= 1000*nbins sampled rows."""
     N, F = x.shape
-    nobs = min(N, 1000 * nbins)
-    idx = np.sort(rng.choice(N, nobs, replace=False)) if nobs < N else np.arange(N)
-    q = np.arange(1, nbins) / nbins
-
-    def one(j):
-        col = np.asarray(x[idx, j], np.float64)
-        e = np.quantile(col, q)  # numpy's default is the linear (type 7) rule Statistics.quantile uses
-        if e.shape[0] == 1:
-            e = np.array([col.min()])
-        return np.ascontiguousarray(e)
-
-    edges = _per_feature(one, F)  # `@threads for j`, src/fit-utils.jl:15: the features are independent
+    idx, nobs = _sample_rows(N, nbins, rng)
+    if x.dtype not in _lib.DTYPE_IDS:
+        x, idx = np.asarray(x if idx is None else x[idx], np.float64), None
+    cols = _lib.matrix_columns(x)
+    if nbins == 2:
+        edges = list(_lib.order_stats(cols, idx, nobs, [0]))
+    else:
+        edges = list(_quantiles(cols, idx, nobs, nbins))
     featbins = np.array([len(e) + 1 for e in edges], np.uint8)
     feattypes = np.ones(F, np.uint8)
     return edges, featbins, feattypes
@@ -294,12 +299,14 @@ def get_edges_table(data, feature_names, nbins, rng):
     categorical column is split on its levels (`==`, or `<=` when its levels are ordered), a Real column on the unique
     quantiles of the sampled rows."""
     nrow = len(_column(data, feature_names[0]))
-    nobs = min(nrow, 1000 * nbins)
-    idx = np.sort(rng.choice(nrow, nobs, replace=False)) if nobs < nrow else np.arange(nrow)
-    q = np.arange(1, nbins) / nbins
+    idx, nobs = _sample_rows(nrow, nbins, rng)
+    cols = [_column(data, name) for name in feature_names]
+    real = [j for j, col in enumerate(cols) if not _is_categorical(col) and col.dtype.kind in "iuf"]
+    q = _quantiles(_lib.table_columns([_real_column(cols[j]) for j in real]), idx, nobs, nbins) if real else None
+    q = dict(zip(real, q)) if real else {}
     edges, featbins, feattypes = [], [], []
-    for name in feature_names:
-        col = _column(data, name)
+    for j, name in enumerate(feature_names):
+        col = cols[j]
         if _is_categorical(col):
             e = list(col.categories)
             nb, ft = len(e), bool(col.ordered)
@@ -308,11 +315,10 @@ def get_edges_table(data, feature_names, nbins, rng):
                                    "`nbins`, up to 255." % (nbins, name, nb))
         elif col.dtype == np.bool_:
             e, nb, ft = [False, True], 2, False
-        elif col.dtype.kind in "iuf":
-            sub = np.asarray(col[idx], np.float64)
-            e = np.unique(np.quantile(sub, q))
+        elif j in q:
+            e = np.unique(q[j])
             if e.shape[0] == 1:
-                e = np.array([sub.min()])
+                e = np.array([np.asarray(col if idx is None else col[idx], np.float64).min()])
             e = np.ascontiguousarray(e)
             nb, ft = len(e) + 1, True
         else:
@@ -323,10 +329,15 @@ def get_edges_table(data, feature_names, nbins, rng):
     return edges, np.array(featbins, np.uint8), np.array(feattypes, np.uint8)
 
 
+def _real_column(col):
+    """A Real column as the library reads it: as it is, or as Float64 when its type is none the library knows."""
+    return col if col.dtype in _lib.DTYPE_IDS else np.asarray(col, np.float64)
+
+
 def binarize_table(data, feature_names, edges):
     """binarize for Tables input, src/fit-utils.jl:74-92 -> (F, N) uint8 (the memory order of Julia's N x F matrix)."""
     nrow = len(_column(data, feature_names[0]))
-    out = np.empty((len(feature_names), nrow), np.uint8)
+    cols, search = [], []
     for j, name in enumerate(feature_names):
         col = _column(data, name)
         if _is_categorical(col):
@@ -335,14 +346,19 @@ def binarize_table(data, feature_names, edges):
             codes = np.asarray(col.codes)
             if (codes < 0).any():
                 raise RuntimeError("feature %s holds missing values or levels the model was not trained on" % name)
-            out[j] = codes + 1
+            cols.append(codes)
+            search.append(())  # code + 1
         elif col.dtype == np.bool_:
-            out[j] = col.astype(np.uint8) + 1
+            cols.append(col)
+            search.append(())
         elif col.dtype.kind in "iuf":
-            out[j] = binarize(np.asarray(col, np.float64)[:, None], [edges[j]])[0]
+            cols.append(_real_column(col))
+            search.append(edges[j])
         else:
             raise RuntimeError("Invalid feature eltype: %s is %s" % (name, col.dtype))
-    return out
+        if len(cols[j]) != nrow:
+            raise ValueError("feature %s has %d rows, %s has %d" % (name, len(cols[j]), feature_names[0], nrow))
+    return _lib.bin_columns(_lib.table_columns(cols), nrow, search)
 
 
 def _table_features(data, target_names, weight_name, offset_name, feature_names):
@@ -421,9 +437,7 @@ def init(config, x_train, y_train=None, w_train=None, offset_train=None, feature
     if table:  # Bool and categorical columns have no edges to search: binned on the host as the reference does
         h.set_xbin(binarize_table(x_train, feature_names, edges))
     else:
-        # the library takes the reference's memory order (column-major, a Julia matrix as it lies): free for a Fortran-ordered
-        # numpy array, a transposing host copy for a C-ordered one
-        h.binarize(np.ascontiguousarray(x.T, np.float64), edges)
+        h.binarize_matrix(x, edges)
     mono = np.zeros(F, np.int32)
     for k, v in config.monotone_constraints.items():
         mono[int(k) - 1] = int(v)
@@ -533,7 +547,7 @@ class CallBack:
             if table:
                 h.set_xbin(x_bin)
             else:
-                h.binarize(np.ascontiguousarray(x.T, np.float64), m.info["edges"])
+                h.binarize_matrix(x, m.info["edges"])
             h.set_feature_meta(m.info["feattypes"], None)
             _set_levels(h, config)
             h.set_target(y32, w, np.zeros(m.K, np.float32), offset)  # p = zeros (+ offset'), src/callback.jl:104, :82
@@ -647,20 +661,11 @@ def update(config, m, cache, x_train=None, y_train=None, w_train=None):
 
 
 def binarize(x, edges):
-    """binarize, src/fit-utils.jl:66-72 — host version used for inference inputs (searchsortedfirst)."""
+    """binarize, src/fit-utils.jl:66-72 — host version used for inference inputs (searchsortedfirst, in the order of isless)."""
     x = np.asarray(x)
-    F = x.shape[1]
-    out = np.empty((F, x.shape[0]), np.uint8)
-    for j in range(F):
-        e = np.asarray(edges[j], np.float64)
-        col = np.asarray(x[:, j], np.float64)
-        idx = np.searchsorted(e, col, side="left")  # numpy orders NaN last, as isless does
-        # isless also puts -0.0 before 0.0: a +0.0 value passes the -0.0 edges that `<` treats as equal
-        pz = (col == 0) & ~np.signbit(col)
-        if pz.any() and (e == 0).any():
-            idx[pz] = np.searchsorted(e, 0.0, side="left") + int(((e == 0) & np.signbit(e)).sum())
-        out[j] = idx + 1
-    return out
+    if x.dtype not in _lib.DTYPE_IDS:
+        x = x.astype(np.float64)
+    return _lib.bin_columns(_lib.matrix_columns(x), x.shape[0], edges)
 
 
 def predict(m, data, ntree_limit=None, device="gpu"):

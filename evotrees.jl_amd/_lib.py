@@ -27,7 +27,7 @@ EXPORTS = [
     "evt_predict_tree", "evt_get_xbin", "evt_get_pred", "evt_get_grads", "evt_get_nidx", "evt_get_hist", "evt_get_quant",
     "evt_predict", "evt_predict_f64", "evt_predict_leaf_idx", "evt_eval_metric", "evt_set_profiling", "evt_get_profile", "evt_reset_profile",
     "evt_set_option", "evt_synchronize", "evt_copy_bandwidth", "evt_read_bandwidth", "evt_predict_static",
-    "evt_lds_atomic_rate", "evt_global_atomic_rate",
+    "evt_lds_atomic_rate", "evt_global_atomic_rate", "evt_trim", "evt_binarize", "evt_bin_columns", "evt_order_stats",
 ]
 
 
@@ -68,6 +68,10 @@ def load():
         "evt_destroy": [vp],
         "evt_set_xbin": [vp, vp],
         "evt_binarize_f64": [vp, vp, vp, vp],
+        "evt_trim": [],
+        "evt_binarize": [vp, vp, i32, i64, i64, vp, vp],
+        "evt_bin_columns": [vp, i32, i64, vp, vp, vp],
+        "evt_order_stats": [vp, i32, vp, i64, vp, i32, vp],
         "evt_set_target": [vp, vp, vp, vp, vp],
         "evt_set_feature_meta": [vp, vp, vp],
         "evt_set_alphas": [vp, vp, i32],
@@ -158,6 +162,68 @@ def read_bandwidth(nbytes=1 << 30, iters=10):
     return out.value
 
 
+# evt_column, and the element types a column may have
+COLUMN = np.dtype([("data", np.uint64), ("stride", np.int64), ("dtype", np.int64)])
+DTYPE_IDS = {np.dtype(t): k for k, t in enumerate(("f4", "f8", "i1", "i2", "i4", "i8", "u1", "u2", "u4", "u8"))}
+
+
+def matrix_columns(x):
+    """The columns of a matrix (of a type in DTYPE_IDS) as evt_column records; they point into x."""
+    cols = np.empty(x.shape[1], COLUMN)
+    cols["data"] = x.ctypes.data + x.strides[1] * np.arange(x.shape[1])
+    cols["stride"] = x.strides[0]
+    cols["dtype"] = DTYPE_IDS[x.dtype]
+    return cols
+
+
+def table_columns(arrays):
+    """Vectors (Bool or of a type in DTYPE_IDS) as evt_column records; they point into the vectors."""
+    cols = np.empty(len(arrays), COLUMN)
+    for j, a in enumerate(arrays):
+        cols[j] = (a.ctypes.data, a.strides[0], 6 if a.dtype == np.bool_ else DTYPE_IDS[a.dtype])
+    return cols
+
+
+def strided_matrix(x):
+    """(x, row stride, column stride) in elements, one of them 1, of a Float32 or Float64 matrix: x itself as it lies, or a copy."""
+    es = x.itemsize
+    a, b = x.strides
+    N, F = x.shape
+    if x.dtype.char not in "fd" or not x.dtype.isnative:
+        x = x.astype(np.float64)
+        return strided_matrix(x)
+    if (b == es or F == 1) and a > 0 and a % es == 0:
+        return x, a // es, 1
+    if (a == es or N == 1) and b > 0 and b % es == 0:
+        return x, 1, b // es
+    return np.ascontiguousarray(x), F, 1
+
+
+def flat_edges(edges):
+    """Edges of all features one after the other, and where each feature's start."""
+    off = np.zeros(len(edges) + 1, np.int32)
+    off[1:] = np.cumsum([len(e) for e in edges])
+    flat = np.concatenate([np.asarray(e, np.float64) for e in edges]) if len(edges) else np.zeros(0)
+    return np.ascontiguousarray(flat), off
+
+
+def bin_columns(cols, nobs, edges):
+    """Bins (F, nobs) of table columns, on the host: a column whose edges are empty gets value + 1."""
+    flat, off = flat_edges(edges)
+    out = np.empty((len(cols), nobs), np.uint8)
+    check(load().evt_bin_columns(ptr(cols), len(cols), nobs, ptr(flat), ptr(off), ptr(out)))
+    return out
+
+
+def order_stats(cols, idx, n, ranks):
+    """(F, len(ranks)) order statistics of every column over the rows idx (None: the first n)."""
+    ranks = np.ascontiguousarray(ranks, np.int64)
+    idx = None if idx is None else np.ascontiguousarray(idx, np.int64)
+    out = np.empty((len(cols), len(ranks)), np.float64)
+    check(load().evt_order_stats(ptr(cols), len(cols), ptr(idx), n, ptr(ranks), len(ranks), ptr(out)))
+    return out
+
+
 class TreeArrays:
     """Host arrays in the layout of Tree{L,K} (src/structs.jl:77-106)."""
 
@@ -207,6 +273,13 @@ class Handle:
         off[1:] = np.cumsum([len(e) for e in edges])
         flat = np.ascontiguousarray(np.concatenate([np.asarray(e, np.float64) for e in edges]))
         check(load().evt_binarize_f64(self._h, ptr(x_FN), ptr(flat), ptr(off)))
+
+    def binarize_matrix(self, x, edges):
+        """x: (N, F) matrix as the program holds it, rows or columns contiguous; edges as for binarize."""
+        assert x.shape == (self.N, self.F)
+        x, rs, cs = strided_matrix(x)
+        flat, off = flat_edges(edges)
+        check(load().evt_binarize(self._h, ptr(x), DTYPE_IDS[x.dtype], rs, cs, ptr(flat), ptr(off)))
 
     def set_target(self, y, w, mu, offset=None):
         y = np.ascontiguousarray(y, np.float32)

@@ -1,5 +1,6 @@
 // C ABI of libevotrees_hip.so: handle lifecycle, uploads, the per-tree level loop, read-back.
 #include "evt_internal.h"
+#include "upload.h"
 
 #include <stdarg.h>
 #include <stdio.h>
@@ -506,10 +507,8 @@ static int check_errflag(evt_ctx *c, const char *what) {
     return EVT_OK;
 }
 
-// A Float64 matrix in host memory (column-major, nobs x nfeats) -> bins, written in place at xcm (column j at xcm + j * nobs).
-// The matrix goes up in pieces (whole columns while they are short, row ranges of one column otherwise) through three pinned
-// buffers: a few worker threads copy piece k + 1 into its buffer while the DMA engine moves piece k, and the kernel that bins
-// a piece runs behind its copy on the same stream.  A copy straight from the caller's pageable memory is staged by the runtime
+// Large host buffers go up in pieces through three pinned buffers: a few worker threads copy piece k + 1 into its buffer while
+// the DMA engine moves piece k.  A copy straight from the caller's pageable memory is staged by the runtime
 // at about half the rate the bus gives pinned memory (31 against 57 GB/s on the box this was measured on), and one thread's
 // memcpy is no faster than that either.  The workers only copy memory, never call back into the caller's runtime, and are
 // joined before the call returns.
@@ -594,46 +593,7 @@ static int upload_workers(int64_t total_bytes) {
     if (total_bytes < 2 * UPLOAD_PIECE) return 0;
     return (int)std::min<unsigned>(6, std::max(1u, std::thread::hardware_concurrency() / 2));
 }
-static int upload_binarize_f64(hipStream_t s, const double *x, int64_t nobs, int nfeats, const double *d_edges, const int32_t *d_eoff,
-                               uint8_t *xcm) {
-    const int64_t rows_max = UPLOAD_PIECE / 8;
-    const int64_t rows_piece = std::min(nobs, rows_max);
-    const int cols_piece = (nobs <= rows_max) ? (int)std::max<int64_t>(1, std::min<int64_t>(nfeats, rows_max / nobs)) : 1;
-    const size_t bytes = sizeof(double) * (size_t)rows_piece * cols_piece;
-    UploadSlots U;
-    int r0 = U.init(bytes, true);
-    if (r0 != EVT_OK) return r0;
-    // small inputs are copied by the calling thread; from a few pieces on, by up to six workers
-    std::unique_ptr<CopyPool> pool;
-    if (upload_workers((int64_t)sizeof(double) * nobs * nfeats) > 1) pool.reset(new CopyPool(upload_workers((int64_t)sizeof(double) * nobs * nfeats)));
-    std::vector<CopyJob> jobs;
-    int64_t piece = 0;
-    for (int j0 = 0; j0 < nfeats; j0 += cols_piece) {
-        const int nc = std::min(cols_piece, nfeats - j0);
-        for (int64_t r0 = 0; r0 < nobs; r0 += rows_piece, piece++) {
-            const int64_t n = std::min(rows_piece, nobs - r0);
-            const int k = (int)(piece % UploadSlots::NS);
-            if (piece >= UploadSlots::NS) HIPCHK(hipEventSynchronize(U.ev[k])); // the piece that used this buffer has been binned
-            double *h = static_cast<double *>(U.host[k]);
-            jobs.clear();
-            for (int j = 0; j < nc; j++)
-                jobs.push_back({reinterpret_cast<const char *>(x + (size_t)(j0 + j) * nobs + r0), reinterpret_cast<char *>(h + (size_t)j * n), sizeof(double) * (size_t)n});
-            if (pool) {
-                pool->copy(jobs);
-            } else {
-                for (const CopyJob &job : jobs) memcpy(job.dst, job.src, job.n);
-            }
-            HIPCHK(hipMemcpyAsync(U.dev[k], h, sizeof(double) * (size_t)n * nc, hipMemcpyHostToDevice, s));
-            const int r = launch_binarize_cols(s, U.dev[k], d_edges, d_eoff + j0, xcm + (size_t)j0 * nobs + r0, n, nc, n, nobs);
-            if (r != EVT_OK) return r;
-            HIPCHK(hipEventRecord(U.ev[k], s));
-        }
-    }
-    HIPCHK(hipStreamSynchronize(s));
-    return EVT_OK;
-}
-
-// nbytes from the caller's memory to the device: large host buffers go through the pinned buffers (see upload_binarize_f64),
+// nbytes from the caller's memory to the device: large host buffers go through pinned buffers,
 // everything else is a plain copy.  The data has arrived when the call returns.
 static int upload_bytes(hipStream_t s, const void *src, void *dst, size_t nbytes) {
     hipPointerAttribute_t attr;
@@ -681,22 +641,56 @@ extern "C" int evt_set_xbin(evt_handle c, const uint8_t *x_bin_colmajor) {
     });
 }
 
+// bins are in xcm: the records
+static int bins_arrived(evt_ctx *c) {
+    int r = launch_transpose_validate(c);
+    if (r == EVT_OK) r = check_errflag(c, "binarize produced values outside 1..nbins");
+    if (r != EVT_OK) return r;
+    c->have_xbin = true;
+    return EVT_OK;
+}
+
+extern "C" int evt_binarize(evt_handle c, const void *x, int32_t dtype, int64_t row_stride, int64_t col_stride, const double *edges,
+                            const int32_t *edge_off) {
+    return guarded([&]() -> int {
+    CTXCHK(c);
+    ARGCHK(x && edges && edge_off, "NULL argument");
+    ARGCHK(dtype == EVT_F32 || dtype == EVT_F64, "dtype must be EVT_F32 or EVT_F64");
+    ARGCHK(row_stride == 1 || col_stride == 1, "one of the two strides must be 1");
+    for (int j = 0; j < c->F; j++) {
+        const int ne = edge_off[j + 1] - edge_off[j];
+        ARGCHK(ne >= 1 && ne <= c->B - 1 && edge_off[j] >= 0, "each feature needs 1..nbins-1 edges");
+    }
+    c->have_xbin = false;
+    c->planes_ready = false;
+    HbPlan P;
+    P.build(edges, edge_off, c->F, dtype);
+    const int r = upload_bins(c->stream, P, HbSource{x, dtype, row_stride, col_stride}, c->N, c->xcm, c->N);
+    return r == EVT_OK ? bins_arrived(c) : r;
+    });
+}
+
 extern "C" int evt_binarize_f64(evt_handle c, const double *x_colmajor, const double *edges, const int32_t *edge_off) {
     return guarded([&]() -> int {
     CTXCHK(c);
     ARGCHK(x_colmajor && edges && edge_off, "NULL argument");
-    c->have_xbin = false;
-    c->planes_ready = false;
     hipPointerAttribute_t attr;
     bool on_dev = (hipPointerGetAttributes(&attr, x_colmajor) == hipSuccess) && attr.type == hipMemoryTypeDevice;
     (void)hipGetLastError();
-    // edge_off is read on the host to size the edges upload (works for host pointers only)
+    // edge_off is read on the host to size the edges
     std::vector<int32_t> off(c->F + 1);
     HIPCHK(hipMemcpy(off.data(), edge_off, sizeof(int32_t) * (c->F + 1), hipMemcpyDefault));
     for (int j = 0; j < c->F; j++) {
         int ne = off[j + 1] - off[j];
         ARGCHK(ne >= 1 && ne <= c->B - 1 && off[j] >= 0, "each feature needs 1..nbins-1 edges");
     }
+    if (!on_dev) {
+        std::vector<double> ev(off[c->F]);
+        HIPCHK(hipMemcpy(ev.data(), edges, sizeof(double) * off[c->F], hipMemcpyDefault));
+        return evt_binarize(c, x_colmajor, EVT_F64, 1, c->N, ev.data(), off.data());
+    }
+    c->have_xbin = false;
+    c->planes_ready = false;
     double *d_edges = nullptr;
     int32_t *d_off = nullptr;
     HIPCHK(hipMalloc((void **)&d_edges, sizeof(double) * std::max(1, off[c->F])));
@@ -705,9 +699,7 @@ extern "C" int evt_binarize_f64(evt_handle c, const double *x_colmajor, const do
     if (e == hipSuccess) e = hipMemcpyAsync(d_off, off.data(), sizeof(int32_t) * (c->F + 1), hipMemcpyHostToDevice, c->stream);
     int r = EVT_OK;
     if (e == hipSuccess) {
-        if (on_dev) r = launch_binarize(c, x_colmajor, d_edges, d_off);
-        else r = upload_binarize_f64(c->stream, x_colmajor, c->N, c->F, d_edges, d_off, c->xcm);
-        if (r == EVT_OK) r = launch_transpose_validate(c);
+        r = launch_binarize(c, x_colmajor, d_edges, d_off);
         e = hipStreamSynchronize(c->stream);
     }
     if (d_off) (void)hipFree(d_off);
@@ -717,10 +709,7 @@ extern "C" int evt_binarize_f64(evt_handle c, const double *x_colmajor, const do
         evt_set_error("binarize failed: %s", hipGetErrorString(e));
         return EVT_ERR_HIP;
     }
-    r = check_errflag(c, "binarize produced values outside 1..nbins");
-    if (r != EVT_OK) return r;
-    c->have_xbin = true;
-    return EVT_OK;
+    return bins_arrived(c);
     });
 }
 
@@ -1706,23 +1695,26 @@ static int predict_common(int64_t nobs, int32_t nfeats, const uint8_t *x_bin, co
     else if (e == hipSuccess && !leaf_out) e = hipMalloc((void **)&d_out, sizeof(float) * (size_t)nobs * K);
     if (e == hipSuccess && leaf_out) e = hipMalloc((void **)&d_leaf, sizeof(uint32_t) * (size_t)nobs * ntrees);
     if (e == hipSuccess && !x_f64 && !x_in_place) r = upload_bytes(s, x_bin, d_x, (size_t)nobs * nfeats);
-    if (e == hipSuccess && x_f64) {
-        // binarize on the device: the matrix goes up in pieces through pinned buffers and is binned into place
-        double *d_xf = nullptr, *d_edges = nullptr;
+    if (e == hipSuccess && x_f64 && !on_device(x_f64)) {
+        std::vector<double> ev(eoff[nfeats]);
+        e = hipMemcpy(ev.data(), edges, sizeof(double) * eoff[nfeats], hipMemcpyDefault);
+        if (e == hipSuccess) {
+            HbPlan P;
+            P.build(ev.data(), eoff.data(), nfeats, EVT_F64);
+            r = upload_bins(s, P, HbSource{x_f64, EVT_F64, 1, nobs}, nobs, d_x, nobs);
+        }
+    } else if (e == hipSuccess && x_f64) {
+        double *d_edges = nullptr;
         int32_t *d_eoff = nullptr;
         e = hipMalloc((void **)&d_edges, sizeof(double) * eoff[nfeats]);
         if (e == hipSuccess) e = hipMalloc((void **)&d_eoff, sizeof(int32_t) * (nfeats + 1));
         if (e == hipSuccess) e = hipMemcpy(d_edges, edges, sizeof(double) * eoff[nfeats], hipMemcpyDefault);
         if (e == hipSuccess) e = hipMemcpy(d_eoff, eoff.data(), sizeof(int32_t) * (nfeats + 1), hipMemcpyHostToDevice);
         if (e == hipSuccess) {
-            if (on_device(x_f64)) {
-                r = launch_binarize_cols(s, x_f64, d_edges, d_eoff, d_x, nobs, nfeats, nobs, nobs);
-                if (r == EVT_OK) e = hipStreamSynchronize(s);
-            } else {
-                r = upload_binarize_f64(s, x_f64, nobs, nfeats, d_edges, d_eoff, d_x);
-            }
+            r = launch_binarize_cols(s, x_f64, d_edges, d_eoff, d_x, nobs, nfeats, nobs, nobs);
+            if (r == EVT_OK) e = hipStreamSynchronize(s);
         }
-        void *tmp[] = {d_xf, d_edges, d_eoff};
+        void *tmp[] = {d_edges, d_eoff};
         for (void *p : tmp)
             if (p) (void)hipFree(p);
     }

@@ -21,10 +21,10 @@
  *    stream.  Calls on one handle must not overlap; different handles may be used from
  *    different threads.
  *  - The library installs no signal handlers and never calls back into the caller's runtime.
- *    The calls that take a whole matrix from host memory (evt_binarize_f64, evt_predict_f64,
- *    and evt_set_xbin / evt_predict from 64 MB up) copy it into pinned memory with up to six
- *    worker threads of their own, which only copy memory and are joined before the call
- *    returns; no other call starts a thread.
+ *    The calls that take a whole matrix or table from host memory (evt_binarize, evt_binarize_f64,
+ *    evt_predict_f64, evt_bin_columns, evt_order_stats, and evt_set_xbin / evt_predict from 64 MB up)
+ *    bin or copy it with worker threads of their own, up to one per core, which only read the
+ *    caller's memory and are joined before the call returns; no other call starts a thread.
  */
 #ifndef EVOTREES_HIP_H
 #define EVOTREES_HIP_H
@@ -87,6 +87,16 @@ enum {
 /* params.tree_type, src/learners.jl:45 */
 enum { EVT_TREE_BINARY = 0, EVT_TREE_OBLIVIOUS = 1 };
 
+/* element types of a feature matrix (the first two) and of a table's column */
+enum { EVT_F32 = 0, EVT_F64 = 1, EVT_I8 = 2, EVT_I16 = 3, EVT_I32 = 4, EVT_I64 = 5, EVT_U8 = 6, EVT_U16 = 7, EVT_U32 = 8, EVT_U64 = 9 };
+
+/* A column of a table in host memory: row i at data + i * stride bytes (a Bool column is EVT_U8). */
+typedef struct {
+    const void *data;
+    int64_t stride;
+    int64_t dtype;
+} evt_column;
+
 /* Per-tree hyper-parameters read by the kernels (fields of EvoTreeRegressor & co,
  * src/learners.jl:1-23). */
 typedef struct {
@@ -117,6 +127,9 @@ const char *evt_last_error(void);
 /* Number of visible HIP devices; fails (EVT_ERR_HIP) when the runtime finds none. */
 int evt_device_count(int32_t *count);
 
+/* Gives back the pinned buffers that matrices go up through and that are kept between calls (at most 32 MB). */
+int evt_trim(void);
+
 /* ---- training cache ------------------------------------------------------------------
  * Replaces init_core(params, ::Type{<:GPU}, ...) device allocation
  * (ext/EvoTreesKernelAbstractionsExt/init.jl:1-151): sizes every device buffer.
@@ -139,10 +152,22 @@ int evt_set_xbin(evt_handle h, const uint8_t *x_bin_colmajor);
 
 /* Device binarize: searchsortedfirst(edges[j], x[i,j]) for every cell (src/fit-utils.jl:66-72),
  * written straight into the cache's x_bin.  x is nobs x nfeats column-major Float64; edges are
- * concatenated per feature, edge_off has nfeats+1 entries.  A matrix in host memory goes up in
- * 32 MB pieces through pinned buffers, each binned behind its copy (8 bytes per value over the bus:
- * 0.16 s for 10M x 100 where a plain copy from pageable memory takes 0.30 s). */
+ * concatenated per feature, edge_off has nfeats+1 entries.  A matrix in device memory is binned there,
+ * one in host memory by the host's cores (evt_binarize). */
 int evt_binarize_f64(evt_handle h, const double *x_colmajor, const double *edges, const int32_t *edge_off);
+
+/* The same for a matrix in host memory as the program holds it: element (i, j) at x + i * row_stride + j * col_stride
+ * elements of dtype (EVT_F32 or EVT_F64), one of the two strides being 1 (rows, or columns, one after the other); values are
+ * compared as the Float64 they convert to.  Binned by the host's cores and sent as bytes. */
+int evt_binarize(evt_handle h, const void *x, int32_t dtype, int64_t row_stride, int64_t col_stride, const double *edges, const int32_t *edge_off);
+
+/* Host only, no device needed.  binarize for Tables input (src/fit-utils.jl:74-92): column j's bins go to x_bin_out + j * nobs;
+ * a column with edges is searched as above, one without (Bool, level codes from 0) gets value + 1. */
+int evt_bin_columns(const void *cols /* evt_column[ncols] */, int32_t ncols, int64_t nobs, const double *edges, const int32_t *edge_off, uint8_t *x_bin_out);
+/* Host only.  The order statistics that quantile edges are made of (src/fit-utils.jl:15-21, :48): out[j * n_ranks + i] = the ranks[i]-th
+ * smallest (from 0; ranks ascending) of column j's values at the n rows idx (NULL: rows 0 .. n - 1); NaN throughout for a column
+ * that holds one there. */
+int evt_order_stats(const void *cols /* evt_column[ncols] */, int32_t ncols, const int64_t *idx, int64_t n, const int64_t *ranks, int32_t n_ranks, double *out);
 
 /* Target, weights and initial prediction: y Float32[nobs] (for mlogloss the 1-based level code of each row,
  * as _init_target builds it, src/init.jl:43-67) or, with T > 1 targets, the reference's T x nobs column-major matrix

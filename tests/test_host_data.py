@@ -1,0 +1,80 @@
+"""Features in host memory on their way in: binning by the host's cores and the quantile edges, for every layout and type a program
+may hold them in, against numpy's search in the order of isless and numpy's quantiles."""
+import numpy as np
+import pytest
+
+
+def _values(rng, kind, n):
+    x = rng.standard_normal(n)
+    if kind == "float32":
+        x = x.astype(np.float32)
+    elif kind == "tenths":  # Float64 values that are no Float32 and meet the edges
+        x = np.round(x * 20) * 0.1
+    elif kind == "whole":
+        x = np.round(x * 5)
+    elif kind == "huge":
+        x = x * 1e300
+    elif kind == "skewed":
+        x = np.exp(9 * x)
+    return x
+
+
+def _search(e, v):
+    """searchsortedfirst in the order of isless: NaN last, -0.0 before 0.0."""
+    def key(a):
+        a = np.asarray(a, np.float64)
+        i = a.view(np.int64)
+        k = np.where(i < 0, np.int64(-2 ** 63) - i - 1, i)
+        return np.where(np.isnan(a), np.int64(2 ** 63 - 1), k)
+    return (np.searchsorted(key(e), key(v), side="left") + 1).astype(np.uint8)
+
+
+@pytest.mark.parametrize("kind", ["float32", "float64", "tenths", "whole", "huge"])
+@pytest.mark.parametrize("shape", [(1, 1), (15, 3), (16, 16), (17, 17), (64, 33), (67, 5), (4200, 2)])
+def test_bins_of_every_layout(evt, kind, shape):
+    rng = np.random.default_rng(shape[0] + 7 * len(kind))
+    N, F = shape
+    edges = [np.sort(_values(rng, kind, rng.choice([1, 15, 16, 31, 63, 64, 127, 254])).astype(np.float64)) + 0.0 for _ in range(F)]
+    x = _values(rng, kind, N * F).reshape(N, F)
+    special = [np.nan, np.inf, -np.inf, 0.0, -0.0, 1e-310, edges[0][0], edges[-1][-1]]
+    for v in special:
+        x[rng.integers(N), rng.integers(F)] = v
+    edges[0][np.abs(edges[0]) == 0] = -0.0  # compared value by value
+    want = np.stack([_search(edges[j], x[:, j]) for j in range(F)])
+    for lay, bins in ((x, want), (np.asfortranarray(x), want), (np.repeat(x, 2, axis=1)[:, ::2], want), (x[::-1], want[:, ::-1])):
+        assert np.array_equal(evt.binarize(lay, edges), bins)
+
+
+@pytest.mark.parametrize("kind", ["float32", "float64", "whole", "huge", "skewed"])
+@pytest.mark.parametrize("shape,nbins", [((1, 3), 4), ((64, 9), 2), ((65, 8), 255), ((3000, 17), 64), ((9000, 2), 8)])
+def test_edges_are_numpys_quantiles(evt, kind, shape, nbins):
+    rng = np.random.default_rng(1)
+    x = _values(rng, kind, shape[0] * shape[1]).reshape(shape)
+    x[0, 0] = np.inf
+    x[-1, -1] = np.nan
+    q = np.arange(1, nbins) / nbins
+    for lay in (x, np.asfortranarray(x), x[:, ::-1][:, ::-1]):
+        r1, r2 = np.random.default_rng(7), np.random.default_rng(7)
+        edges, _, _ = evt.get_edges(lay, nbins, r1)
+        n = min(shape[0], 1000 * nbins)
+        idx = np.sort(r2.choice(shape[0], n, replace=False)) if n < shape[0] else np.arange(n)
+        for j in range(shape[1]):
+            col = np.asarray(x[idx, j], np.float64)
+            want = np.quantile(col, q) if nbins > 2 else np.array([col.min()])
+            assert np.array_equal(edges[j], want, equal_nan=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("order", ["C", "F"])
+@pytest.mark.parametrize("shape", [(1, 40), (1000, 1), (77, 19), (70_001, 24), (400_003, 50), (9_000_001, 2)])
+def test_upload_of_a_matrix_as_it_lies(evt, dtype, order, shape):
+    """One piece, several, more pieces than buffers; rows and columns contiguous: the handle holds the host's bins."""
+    rng = np.random.default_rng(3)
+    N, F = shape
+    x = np.asarray(rng.random(shape, np.float32) if N * F > 10 ** 6 else rng.random(shape), dtype, order=order)
+    edges = [np.sort(rng.random(15)) for _ in range(F)]
+    h = evt.Handle(N, F, 16, 1, 3, "mse")
+    h.binarize_matrix(x, edges)
+    assert np.array_equal(h.get_xbin(), evt.binarize(x, edges))
+    h.close()
