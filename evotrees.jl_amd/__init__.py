@@ -13,6 +13,8 @@ Julia is not available where this package is developed, so the host side is Pyth
 streams are numpy's (PCG64), not Julia's Xoshiro, hence models are not stream-identical to a
 Julia run with the same seed — the trees are identical for identical masks/column samples.
 """
+import weakref
+
 import numpy as np
 
 from . import _lib
@@ -668,28 +670,47 @@ def binarize(x, edges):
     return _lib.bin_columns(_lib.matrix_columns(x), x.shape[0], edges)
 
 
-def predict(m, data, ntree_limit=None, device="gpu"):
-    """_predict, ext/.../predict.jl:115-135: binarize, walk the first ntree_limit trees, apply the link."""
+_kept = weakref.WeakKeyDictionary()  # EvoTree -> its KeptModel
+
+
+def _kept_model(m):
+    k = _kept.get(m)
+    if k is None or k.loss != m.loss_type or k.K != m.K:
+        k = _kept[m] = _lib.KeptModel(m.loss_type, m.K)
+    return k
+
+
+def _trees_used(m, ntree_limit, device):
     _device_check(device)
     ntrees = len(m.trees)
     ntree_limit = ntrees if ntree_limit is None else ntree_limit
     if ntree_limit > ntrees:
         raise RuntimeError("ntree_limit is larger than number of trees %d." % ntrees)
-    if _is_table(data):  # Bool / categorical columns: binned on the host (src/fit-utils.jl:74-92), walked on the device
-        x_bin = binarize_table(data, m.info["feature_names"], m.info["edges"])
-        p = _lib.predict_model(x_bin, m.info["feattypes"], m.loss_type, m.K, m.trees[:ntree_limit], apply_link=True)
-        return p[:, 0].copy() if m.K == 1 else p
-    x_FN = np.ascontiguousarray(np.asarray(data).T, np.float64)
-    p = _lib.predict_model_f64(x_FN, m.info["edges"], m.info["feattypes"], m.loss_type, m.K, m.trees[:ntree_limit], apply_link=True)
-    return p[:, 0].copy() if m.K == 1 else p
+    return ntree_limit
+
+
+def predict(m, data, ntree_limit=None, device="gpu"):
+    """_predict, ext/.../predict.jl:115-135: binarize, walk the first ntree_limit trees, apply the link."""
+    n = _trees_used(m, ntree_limit, device)
+    edges, ft = m.info["edges"], m.info["feattypes"]
+    if _is_table(data):  # Bool / categorical columns have no edges to search: binned as a table, walked on the device
+        x_bin = binarize_table(data, m.info["feature_names"], edges)
+        p = _kept_model(m).predict(x_bin, m.trees, None, ft, n)
+        if p is None:
+            p = _lib.predict_model(x_bin, ft, m.loss_type, m.K, m.trees[:n], apply_link=True)
+    else:
+        x = np.asarray(data)
+        p = _kept_model(m).predict(x, m.trees, edges, ft, n)
+        if p is None:
+            p = _lib.predict_model_f64(np.ascontiguousarray(x.T, np.float64), edges, ft, m.loss_type, m.K, m.trees[:n], apply_link=True)
+    return p.reshape(-1) if m.K == 1 else p
 
 
 def predict_leaf_idx(m, data, ntree_limit=None, device="gpu"):
     """predict_leaf_idx, src/predict.jl:173-185 -> (nobs, ntree_limit) uint32."""
-    _device_check(device)
-    ntrees = len(m.trees)
-    ntree_limit = ntrees if ntree_limit is None else ntree_limit
-    if ntree_limit > ntrees:
-        raise RuntimeError("ntree_limit is larger than number of trees %d." % ntrees)
-    x_bin = binarize_table(data, m.info["feature_names"], m.info["edges"]) if _is_table(data) else binarize(data, m.info["edges"])
-    return _lib.predict_leaf_idx(x_bin, m.info["feattypes"], m.trees[:ntree_limit])
+    n = _trees_used(m, ntree_limit, device)
+    edges, ft = m.info["edges"], m.info["feattypes"]
+    table = _is_table(data)
+    x = binarize_table(data, m.info["feature_names"], edges) if table else np.asarray(data)
+    p = _kept_model(m).predict(x, m.trees, None if table else edges, ft, n, leaf=True)
+    return p if p is not None else _lib.predict_leaf_idx(x if table else binarize(x, edges), ft, m.trees[:n])

@@ -4,7 +4,9 @@ The library is mandatory: there is no CPU fallback.  Loading fails loudly when t
 object has not been built, and every compute entry point fails when no MI355X is visible.
 """
 import ctypes as C
+import operator
 import os
+import threading
 
 import numpy as np
 
@@ -28,6 +30,7 @@ EXPORTS = [
     "evt_predict", "evt_predict_f64", "evt_predict_leaf_idx", "evt_eval_metric", "evt_set_profiling", "evt_get_profile", "evt_reset_profile",
     "evt_set_option", "evt_synchronize", "evt_copy_bandwidth", "evt_read_bandwidth", "evt_predict_static",
     "evt_lds_atomic_rate", "evt_global_atomic_rate", "evt_trim", "evt_binarize", "evt_bin_columns", "evt_order_stats",
+    "evt_model_create", "evt_model_destroy", "evt_model_predict",
 ]
 
 
@@ -99,6 +102,9 @@ def load():
         "evt_predict": [i64, i32, vp, vp, i32, i32, i32, vp, vp, vp, vp, vp, i32, vp],
         "evt_predict_leaf_idx": [i64, i32, vp, vp, i32, vp, vp, vp, vp, vp],
         "evt_predict_f64": [i64, i32, vp, vp, vp, vp, i32, i32, i32, vp, vp, vp, vp, vp, i32, vp],
+        "evt_model_create": [i32, i32, vp],
+        "evt_model_destroy": [vp],
+        "evt_model_predict": [vp, i32, vp, vp, vp, vp, vp, vp, i32, vp, vp, vp, i32, i64, i64, i64, i32, i32, i32, vp, vp],
         "evt_eval_metric": [vp, i32, vp],
         "evt_set_profiling": [vp, i32],
         "evt_get_profile": [vp, vp, vp, vp],
@@ -227,13 +233,16 @@ def order_stats(cols, idx, n, ranks):
 class TreeArrays:
     """Host arrays in the layout of Tree{L,K} (src/structs.jl:77-106)."""
 
+    replaced = 0  # how often an array of any tree has been replaced by another: KeptModel looks at the trees again then
+
     def __init__(self, K, nnodes):
-        self.feat = np.zeros(nnodes, np.int64)
-        self.cond_bin = np.zeros(nnodes, np.uint8)
-        self.w = np.zeros(nnodes, np.float32)
-        self.gain = np.zeros(nnodes, np.float32)
-        self.pred = np.zeros((nnodes, K), np.float32)  # memory order of Julia's K x nnodes matrix
-        self.split = np.zeros(nnodes, np.uint8)
+        self.__dict__.update(feat=np.zeros(nnodes, np.int64), cond_bin=np.zeros(nnodes, np.uint8), w=np.zeros(nnodes, np.float32),
+                             gain=np.zeros(nnodes, np.float32), pred=np.zeros((nnodes, K), np.float32),  # memory order of Julia's K x nnodes matrix
+                             split=np.zeros(nnodes, np.uint8))
+
+    def __setattr__(self, name, value):
+        self.__dict__[name] = value
+        TreeArrays.replaced += 1
 
     def as_out(self):
         return EvtTreeOut(ptr(self.feat), ptr(self.cond_bin), ptr(self.w), ptr(self.gain), ptr(self.pred), ptr(self.split))
@@ -501,6 +510,93 @@ def predict_model_f64(x_FN, edges, feattypes, loss, K, trees, apply_link=True):
     check(load().evt_predict_f64(N, F, ptr(x_FN), ptr(eflat), ptr(eoff), ptr(ft), LOSS_IDS[loss], K, len(trees), ptr(off), ptr(feat),
                                  ptr(cb), ptr(pr), ptr(sp), 1 if apply_link else 0, ptr(out)))
     return out
+
+
+class KeptModel:
+    """A model's device form (evt_model), kept between predictions.  The library compares the contents of the arrays on every call;
+    what this class keeps are their addresses, which hold as long as the trees, their arrays and the edges are the same objects."""
+
+    def __init__(self, loss, K):
+        self.loss, self.K = loss, K
+        self._h = C.c_void_p(None)
+        self.trees, self.edges, self._lock = None, None, threading.Lock()
+        check(load().evt_model_create(LOSS_IDS[loss], K, C.byref(self._h)))
+
+    def __del__(self):
+        try:
+            if self._h:
+                load().evt_model_destroy(self._h)
+        except Exception:
+            pass
+
+    def _take_trees(self, trees):
+        arrays = []
+        for t in trees:
+            a = (t.feat, t.cond_bin, t.pred, t.split)
+            for v, dt in zip(a, (np.int64, np.uint8, np.float32, np.uint8)):
+                if not (isinstance(v, np.ndarray) and v.dtype == dt and v.flags.c_contiguous):
+                    return False
+            n = a[0].size
+            if a[1].size != n or a[2].size != n * self.K or a[3].size != n or not 1 <= n < 1 << 20:
+                return False
+            arrays.append(a)
+        at = np.array([[v.ctypes.data for v in a] for a in arrays], np.uint64).T.copy()
+        nn = np.array([a[0].size for a in arrays], np.int64)
+        # the completed trees are stored at the width of the deepest
+        if len(arrays) * max(1, int(nn.max())) > 1 << 28:
+            return False
+        self._tree = ((len(trees), nn.ctypes.data) + tuple(at[k].ctypes.data for k in range(4)), at, nn, arrays)
+        self.trees = list(trees)
+        return True
+
+    def _take_edges(self, edges):
+        own = [e if isinstance(e, np.ndarray) and e.dtype == np.float64 and e.flags.c_contiguous else np.ascontiguousarray(e, np.float64) for e in edges]
+        at = np.array([e.ctypes.data for e in own], np.uint64)
+        ne = np.array([e.size for e in own], np.int32)
+        self._edge = ((at.ctypes.data, ne.ctypes.data), at, ne, own)
+        # converted copies do not follow the caller's: looked at again on every call
+        self.edges = list(edges) if all(a is b for a, b in zip(own, edges)) else None
+
+    def _take(self, trees, edges):
+        """The addresses of the trees' arrays and of the edges, with the objects that keep them valid; None when the arrays are of
+        types that are not kept."""
+        with self._lock:
+            seen = TreeArrays.replaced
+            if self.trees is None or self._seen != seen or len(self.trees) != len(trees) or not all(map(operator.is_, self.trees, trees)):
+                self.trees = None
+                if not self._take_trees(trees):
+                    return None
+                self._seen = seen
+            if edges is not None and (self.edges is None or len(self.edges) != len(edges) or not all(map(operator.is_, self.edges, edges))):
+                self._take_edges(edges)
+            return self._tree, self._edge if edges is not None else None
+
+    def predict(self, x, trees, edges, feattypes, ntrees, leaf=False):
+        """(N, K) float32 with the link applied, or (N, ntrees) leaf ids, of the first ntrees trees; None when the trees cannot be kept.
+        x: an (N, F) matrix, or with edges=None (F, N) bins."""
+        held = self._take(trees, edges)
+        if held is None:
+            return None
+        tree, edge = held
+        if edge is None:
+            F, N = x.shape
+            args = (None, None, x.ctypes.data, DTYPE_IDS[x.dtype], 1, N)
+        else:
+            N, F = x.shape
+            x, rs, cs = strided_matrix(x)
+            if F > len(edge[3]):
+                raise ValueError("the matrix has %d columns, the model %d features" % (F, len(edge[3])))
+            args = edge[0] + (x.ctypes.data, DTYPE_IDS[x.dtype], rs, cs)
+        ft = None if feattypes is None else np.ascontiguousarray(feattypes, np.uint8)
+        fta = (None, 0) if ft is None else (ft.ctypes.data, ft.size)
+        if leaf:
+            out = np.empty((ntrees, N), np.uint32)  # Julia: N x ntrees column-major
+            outs = (None, out.ctypes.data)
+        else:
+            out = np.empty((N, self.K), np.float32)
+            outs = (out.ctypes.data, None)
+        check(load().evt_model_predict(self._h, *tree[0], *fta, *args, N, F, ntrees, 0 if leaf else 1, *outs))
+        return out.T if leaf else out
 
 
 def predict_leaf_idx(x_bin_FN, feattypes, trees):

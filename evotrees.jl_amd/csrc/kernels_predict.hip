@@ -441,3 +441,137 @@ int launch_leaf_idx_model(hipStream_t s, const uint32_t *nodes, const int64_t *o
     HIPCHK(hipGetLastError());
     return EVT_OK;
 }
+
+// Few rows, many trees: a block takes R rows and spreads the trees over its 256 / R lanes per row, so that a handful of rows still
+// occupies whole wavefronts (and a few thousand rows the chip), where a row per lane leaves a single chain of dependent reads.  A lane
+// walks WALK_U trees side by side over the completed trees (fixed depth, nodes from the caches: a model of 200 trees of
+// depth 8 is 100 KB); the leaf values of a run of trees meet in LDS, and one lane per row adds them in tree order with predict!'s
+// clamps, so the sum has the bits of the sequential one.  The bins may lie in pinned host memory, and so may the output.
+// Latency bound: three steps of a level (node, bin, next node) cost about 0.4 us from L2, whatever the number of rows in flight.
+// LEAF: the leaf's node id of every row and tree instead, tree by tree, in LB-byte words.
+#define WALK_U 4
+template <int KMAX, int R, bool LEAF, int LB>
+__global__ __launch_bounds__(256) void k_walk_rows(const uint32_t *__restrict__ cnodes, int stride, const ModelTree *__restrict__ meta,
+                                                  const float *__restrict__ cleaf, const uint32_t *__restrict__ cid, int ntrees, int run,
+                                                  const uint8_t *__restrict__ x, int64_t ldx, int64_t n, int F, int wide, int K, int loss, int link,
+                                                  float *__restrict__ out, void *__restrict__ leaf_out, int64_t leaf_ld) {
+    constexpr int G = 256 / R;
+    extern __shared__ uint32_t smem[];
+    uint8_t *s_x = reinterpret_cast<uint8_t *>(smem);                      // [F][R]
+    float *s_v = reinterpret_cast<float *>(smem + ((size_t)F * R + 3) / 4); // [run][R][K]
+    const int tid = threadIdx.x, r = tid % R, g = tid / R;
+    const int64_t i0 = (int64_t)blockIdx.x * R;
+    for (int k = tid; k < F * R; k += 256) {
+        const int64_t i = i0 + k % R;
+        s_x[k] = x[(size_t)(k / R) * ldx + (i < n ? i : n - 1)];
+    }
+    __syncthreads();
+    float acc[KMAX];
+#pragma unroll
+    for (int k = 0; k < KMAX; k++) acc[k] = 0.0f;
+    for (int t0 = 0; t0 < ntrees; t0 += run) {
+        const int t1 = t0 + run < ntrees ? t0 + run : ntrees;
+        for (int tb = t0 + g; tb < t1; tb += G * WALK_U) {
+            uint32_t nid[WALK_U];
+            int levels[WALK_U], most = 0;
+            const uint32_t *cn[WALK_U];
+#pragma unroll
+            for (int u = 0; u < WALK_U; u++) {
+                const int t = tb + u * G;
+                nid[u] = 1;
+                levels[u] = t < t1 ? meta[t].levels : 0;
+                cn[u] = cnodes + (size_t)(t < t1 ? t : t0) * stride;
+                most = levels[u] > most ? levels[u] : most;
+            }
+            for (int l = 0; l < most; l++) {
+                uint32_t nd[WALK_U];
+#pragma unroll
+                for (int u = 0; u < WALK_U; u++) nd[u] = l < levels[u] ? cn[u][nid[u] - 1] : 0u;
+#pragma unroll
+                for (int u = 0; u < WALK_U; u++) {
+                    if (l >= levels[u]) continue;
+                    const uint32_t f = wide ? nd[u] & 0xFFFFu : ((nd[u] >> 6) & 0x3FCu) | (nd[u] & 3u);
+                    nid[u] = step_node<false>(nid[u], nd[u], s_x[f * R + r]);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < WALK_U; u++) {
+                const int t = tb + u * G;
+                if (t >= t1) continue;
+                const size_t at = (size_t)meta[t].leaf_off + (nid[u] - (1u << levels[u]));
+                if (LEAF) {
+                    const uint32_t id = cid[at];
+                    const size_t o = (size_t)t * leaf_ld + i0 + r;
+                    if (i0 + r < n) {
+                        if (LB == 1) static_cast<uint8_t *>(leaf_out)[o] = (uint8_t)id;
+                        else if (LB == 2) static_cast<uint16_t *>(leaf_out)[o] = (uint16_t)id;
+                        else static_cast<uint32_t *>(leaf_out)[o] = id;
+                    }
+                } else {
+                    float *v = s_v + ((size_t)(t - t0) * R + r) * K;
+                    for (int k = 0; k < K; k++) v[k] = cleaf[at * K + k];
+                }
+            }
+        }
+        if (LEAF) continue;
+        __syncthreads();
+        if (tid < R) {
+#pragma unroll 4
+            for (int t = 0; t < t1 - t0; t++) {
+                float lp[KMAX];
+#pragma unroll
+                for (int k = 0; k < KMAX; k++) lp[k] = k < K ? s_v[((size_t)t * R + tid) * K + k] : 0.0f;
+                add_tree<KMAX>(acc, lp, K, loss);
+            }
+        }
+        __syncthreads();
+    }
+    if (!LEAF && tid < R && i0 + tid < n) {
+        if (link) apply_link<KMAX>(acc, K, loss);
+#pragma unroll
+        for (int k = 0; k < KMAX; k++)
+            if (k < K) out[(size_t)K * (i0 + tid) + k] = acc[k];
+    }
+}
+
+template <int KMAX, int R, bool LEAF, int LB>
+static int launch_walk(hipStream_t s, const uint32_t *cnodes, int stride, const void *meta, const float *cleaf, const uint32_t *cid, int ntrees,
+                       const uint8_t *x, int64_t ldx, int64_t n, int F, int wide, int K, int loss, int link, float *out, void *leaf_out, int64_t leaf_ld) {
+    static EvtDevOnce once;
+    const int dev = EvtDevOnce::current();
+    if (once.pending(dev)) {
+        HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_walk_rows<KMAX, R, LEAF, LB>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        once.mark(dev);
+    }
+    const int G = 256 / R;
+    const int run = LEAF ? ntrees : std::max(G, 8192 / (R * K) / G * G); // trees whose values fit 32 KB of LDS
+    const size_t lds = ((size_t)F * R + 3) / 4 * 4 + (LEAF ? 0 : (size_t)std::min(run, ntrees) * R * K * 4);
+    hipLaunchKernelGGL((k_walk_rows<KMAX, R, LEAF, LB>), dim3((unsigned)((n + R - 1) / R)), dim3(256), lds, s, cnodes, stride,
+                       static_cast<const ModelTree *>(meta), cleaf, cid, ntrees, run, x, ldx, n, F, wide, K, loss, link, out, leaf_out, leaf_ld);
+    HIPCHK(hipGetLastError());
+    return EVT_OK;
+}
+
+int launch_walk_rows(hipStream_t s, const uint32_t *cnodes, int stride, const void *meta, const float *cleaf, const uint32_t *cid, int ntrees,
+                     const uint8_t *x, int64_t ldx, int64_t n, int F, int wide, int K, int loss, int apply_link, float *out, void *leaf_out, int leaf_bytes,
+                     int64_t leaf_ld) {
+    // rows per block: as few as fill the chip (1024 blocks of four wavefronts, eight of which share a compute unit), and no more than
+    // 64 KB of bins
+    int R = n <= 1024 ? 1 : (n <= 8192 ? 4 : (n <= 65536 ? 16 : 64));
+    while (R > 1 && (size_t)R * F > 65536) R /= 4;
+#define EVT_WALK(KM_, LEAF_, LB_)                                                                                                                    \
+    switch (R) {                                                                                                                                     \
+        case 1: return launch_walk<KM_, 1, LEAF_, LB_>(s, cnodes, stride, meta, cleaf, cid, ntrees, x, ldx, n, F, wide, K, loss, apply_link, out, leaf_out, leaf_ld); \
+        case 4: return launch_walk<KM_, 4, LEAF_, LB_>(s, cnodes, stride, meta, cleaf, cid, ntrees, x, ldx, n, F, wide, K, loss, apply_link, out, leaf_out, leaf_ld); \
+        case 16: return launch_walk<KM_, 16, LEAF_, LB_>(s, cnodes, stride, meta, cleaf, cid, ntrees, x, ldx, n, F, wide, K, loss, apply_link, out, leaf_out, leaf_ld); \
+        default: return launch_walk<KM_, 64, LEAF_, LB_>(s, cnodes, stride, meta, cleaf, cid, ntrees, x, ldx, n, F, wide, K, loss, apply_link, out, leaf_out, leaf_ld); \
+    }
+    if (leaf_out) {
+        if (leaf_bytes == 1) { EVT_WALK(1, true, 1) }
+        if (leaf_bytes == 2) { EVT_WALK(1, true, 2) }
+        EVT_WALK(1, true, 4)
+    }
+    if (K <= 4) { EVT_WALK(4, false, 0) }
+    EVT_WALK(EVT_MAX_K, false, 0)
+#undef EVT_WALK
+}

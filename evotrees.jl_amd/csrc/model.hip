@@ -1,0 +1,375 @@
+// A model kept on the device between predictions: _predict(m, data) (src/predict.jl:118-136) and predict_leaf_idx (:138-185) for a program
+// that calls them again and again.  The host arrays of the trees stay the caller's; a copy of them is kept beside the packed device
+// form, and every call compares before it uses the latter.
+#include "upload.h"
+
+#include <math.h>
+#include <string.h>
+
+#include <algorithm>
+#include <memory>
+#include <mutex>
+
+int predict_lds_shape(int F, int max_int, int K, int hint);
+int launch_predict_model_lds(hipStream_t s, const uint32_t *cnodes, const float *cleaf, const void *meta, int ntrees, const uint8_t *xcm, int64_t N,
+                             int F, int max_int, int K, int loss, int apply_link, int all_numeric, int shape, float *out);
+int launch_walk_rows(hipStream_t s, const uint32_t *cnodes, int stride, const void *meta, const float *cleaf, const uint32_t *cid, int ntrees,
+                     const uint8_t *x, int64_t ldx, int64_t n, int F, int wide, int K, int loss, int apply_link, float *out, void *leaf_out, int leaf_bytes,
+                     int64_t leaf_ld);
+
+namespace {
+
+struct CompletedTree { // as k_predict_model_lds and k_walk_rows read it
+    int32_t node_off, leaf_off, levels, n_int;
+};
+
+struct Model {
+    std::mutex mu;
+    int device = 0, loss = 0, K = 0;
+    hipStream_t s = nullptr;
+    // the caller's arrays as they were when the device form was built
+    std::vector<int32_t> nn;
+    std::vector<int64_t> feat;
+    std::vector<uint8_t> cond_bin, split, feattypes;
+    std::vector<float> pred;
+    std::vector<double> edges;
+    std::vector<int32_t> edge_off;
+    // device form: trees completed to their depth, `stride` node words each, padded to a multiple of four trees
+    bool built = false;
+    int ntrees = 0, max_int = 0, max_feat = 0, max_nodes = 0;
+    bool all_numeric = true, wide = false;
+    uint32_t *d_nodes = nullptr, *d_cid = nullptr;
+    float *d_leaf = nullptr;
+    CompletedTree *d_meta = nullptr;
+    size_t cap_nodes = 0, cap_leaf = 0, cap_cid = 0, cap_meta = 0;
+    std::vector<CompletedTree> meta;
+    std::unique_ptr<HbPlan> plan[2]; // by source type
+    uint8_t *d_x = nullptr;          // bins of the pieces in flight
+    size_t cap_x = 0;
+
+    ~Model() {
+        (void)hipSetDevice(device);
+        if (s) (void)hipStreamSynchronize(s);
+        void *p[] = {d_nodes, d_cid, d_leaf, d_meta, d_x};
+        for (void *q : p)
+            if (q) (void)hipFree(q);
+        if (s) (void)hipStreamDestroy(s);
+    }
+};
+
+template <typename T>
+int grow(T **p, size_t *cap, size_t n) {
+    if (*cap >= n) return EVT_OK;
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+    *cap = 0;
+    const hipError_t e = hipMalloc((void **)p, n * sizeof(T));
+    if (e != hipSuccess) {
+        evt_set_error("hipMalloc of %zu bytes failed: %s", n * sizeof(T), hipGetErrorString(e));
+        return EVT_ERR_NOMEM;
+    }
+    *cap = n;
+    return EVT_OK;
+}
+
+struct TreePtrs {
+    int32_t n;
+    const int64_t *nn;
+    const int64_t *const *feat;
+    const uint8_t *const *cond_bin;
+    const uint8_t *const *split;
+    const float *const *pred;
+};
+
+bool same_trees(const Model &m, const TreePtrs &t) {
+    if (!m.built || (size_t)t.n != m.nn.size()) return false;
+    size_t o = 0;
+    for (int i = 0; i < t.n; i++) {
+        const size_t n = (size_t)m.nn[i];
+        if ((int64_t)n != t.nn[i] || memcmp(m.feat.data() + o, t.feat[i], 8 * n) || memcmp(m.cond_bin.data() + o, t.cond_bin[i], n) ||
+            memcmp(m.split.data() + o, t.split[i], n) || memcmp(m.pred.data() + o * m.K, t.pred[i], 4 * n * m.K))
+            return false;
+        o += n;
+    }
+    return true;
+}
+
+// Copies the caller's arrays, checks them by the rules of evt_predict, completes the trees and uploads them.
+int build(Model &m, const TreePtrs &t, const uint8_t *feattypes, int nft) {
+    m.built = false;
+    size_t total = 0;
+    int levels_max = 0;
+    for (int i = 0; i < t.n; i++) {
+        ARGCHK(t.nn[i] >= 1 && t.nn[i] <= ((int64_t)1 << 20) - 1, "a kept model takes trees of up to 2^20 - 1 nodes");
+        total += (size_t)t.nn[i];
+        int d = 0;
+        while (((int64_t)1 << d) - 1 < t.nn[i]) d++;
+        levels_max = std::max(levels_max, d - 1);
+    }
+    const int npad = (t.n + 3) / 4 * 4;
+    m.max_int = (1 << levels_max) - 1;
+    const int stride = std::max(1, m.max_int);
+    ARGCHK((size_t)npad * stride <= ((size_t)1 << 28), "the completed trees of a kept model exceed 2^28 nodes");
+    m.nn.resize(t.n);
+    m.feat.resize(total);
+    m.cond_bin.resize(total);
+    m.split.resize(total);
+    m.pred.resize(total * m.K);
+    m.feattypes.assign(feattypes ? feattypes : nullptr, feattypes ? feattypes + nft : nullptr);
+    size_t o = 0;
+    m.max_feat = m.max_nodes = 0;
+    for (int i = 0; i < t.n; i++) {
+        const int64_t n = t.nn[i];
+        m.nn[i] = (int32_t)n;
+        m.max_nodes = std::max(m.max_nodes, (int)n);
+        memcpy(m.feat.data() + o, t.feat[i], 8 * n);
+        memcpy(m.cond_bin.data() + o, t.cond_bin[i], n);
+        memcpy(m.split.data() + o, t.split[i], n);
+        memcpy(m.pred.data() + o * m.K, t.pred[i], 4 * n * m.K);
+        for (int64_t k = 0; k < n; k++)
+            if (m.split[o + k]) {
+                ARGCHK(2 * k + 3 <= n, "split node without children inside the tree arrays");
+                ARGCHK(m.feat[o + k] >= 1 && m.feat[o + k] <= EVT_MAX_FEATS && (!feattypes || m.feat[o + k] <= nft), "tree feature id outside 1..nfeats");
+                m.max_feat = std::max(m.max_feat, (int)m.feat[o + k]);
+            }
+        o += (size_t)n;
+    }
+    m.wide = m.max_feat > 1024;
+    m.all_numeric = true;
+    m.ntrees = t.n;
+    std::vector<uint32_t> nodes((size_t)npad * stride, 0u), cid;
+    std::vector<float> leaf;
+    m.meta.assign(npad, CompletedTree{0, 0, 0, 0});
+    std::vector<int32_t> src; // 0: a split node of the tree; otherwise the leaf whose value the node carries
+    const uint32_t always_left = (255u << 16) | EVT_NODE_NUMERIC; // feature 1, bin <= 255
+    o = 0;
+    for (int i = 0; i < t.n; i++) {
+        const int n = m.nn[i];
+        int d = 0;
+        while ((1 << d) - 1 < n) d++;
+        const int full = (1 << d) - 1, n_int = full / 2, n_leaf = n_int + 1;
+        m.meta[i] = {(int32_t)((size_t)i * stride), (int32_t)(leaf.size() / m.K), d - 1, n_int};
+        src.assign(full + 1, 0);
+        for (int k = 1; k <= full; k++) {
+            const int32_t up = k == 1 ? 0 : src[k >> 1];
+            src[k] = up ? up : (m.split[o + k - 1] ? 0 : k); // a split node's children lie inside the arrays: k <= n here
+        }
+        uint32_t *cn = nodes.data() + (size_t)i * stride;
+        for (int k = 1; k <= n_int; k++) {
+            uint32_t w = always_left;
+            if (src[k] == 0) {
+                const int f0 = (int)m.feat[o + k - 1] - 1;
+                const bool numeric = m.feattypes.empty() || m.feattypes[f0] != 0;
+                m.all_numeric = m.all_numeric && numeric;
+                w = (m.wide ? (uint32_t)f0 : (uint32_t)(((f0 >> 2) << 8) | (f0 & 3))) | ((uint32_t)m.cond_bin[o + k - 1] << 16) | (numeric ? EVT_NODE_NUMERIC : 0u);
+            }
+            cn[k - 1] = w;
+        }
+        for (int q = 0; q < n_leaf; q++) {
+            const int32_t at = src[n_int + 1 + q];
+            cid.push_back((uint32_t)at);
+            for (int k = 0; k < m.K; k++) leaf.push_back(m.pred[m.K * (o + at - 1) + k]);
+        }
+        o += (size_t)n;
+    }
+    ARGCHK(leaf.size() < ((size_t)1 << 31), "the leaves of a kept model exceed 2^31 values");
+    HIPCHK(hipStreamSynchronize(m.s));
+    int r = grow(&m.d_nodes, &m.cap_nodes, nodes.size());
+    if (r == EVT_OK) r = grow(&m.d_leaf, &m.cap_leaf, leaf.size());
+    if (r == EVT_OK) r = grow(&m.d_cid, &m.cap_cid, cid.size());
+    if (r == EVT_OK) r = grow(&m.d_meta, &m.cap_meta, m.meta.size());
+    if (r != EVT_OK) return r;
+    HIPCHK(hipMemcpyAsync(m.d_nodes, nodes.data(), 4 * nodes.size(), hipMemcpyHostToDevice, m.s));
+    HIPCHK(hipMemcpyAsync(m.d_leaf, leaf.data(), 4 * leaf.size(), hipMemcpyHostToDevice, m.s));
+    HIPCHK(hipMemcpyAsync(m.d_cid, cid.data(), 4 * cid.size(), hipMemcpyHostToDevice, m.s));
+    HIPCHK(hipMemcpyAsync(m.d_meta, m.meta.data(), sizeof(CompletedTree) * m.meta.size(), hipMemcpyHostToDevice, m.s));
+    HIPCHK(hipStreamSynchronize(m.s));
+    m.built = true;
+    return EVT_OK;
+}
+
+// Rows from this many on in one launch take the kernel that walks 1024 rows per block from LDS (k_predict_model_lds), fewer the one
+// that spreads a row's trees over lanes: below it the former leaves compute units without a block.
+const int64_t WALK_LDS_MIN_ROWS = 131072;
+
+struct Request {
+    const HbPlan *plan; // null: `bins` are the host's, column-major with N rows
+    HbSource src;
+    const uint8_t *bins;
+    int64_t N;
+    int F, ntrees, link;
+    float *out;
+    uint32_t *leaf_out;
+};
+
+int walk(Model &m, const Request &q, const uint8_t *x, int64_t n, void *out, int leaf_bytes) {
+    if (q.leaf_out)
+        return launch_walk_rows(m.s, m.d_nodes, std::max(1, m.max_int), m.d_meta, m.d_leaf, m.d_cid, q.ntrees, x, n, n, q.F, m.wide, m.K, m.loss, 0, nullptr, out,
+                                leaf_bytes, n);
+    const int shape = n >= WALK_LDS_MIN_ROWS ? predict_lds_shape(q.F, m.max_int, m.K, 0) : 0;
+    if (shape > 0)
+        return launch_predict_model_lds(m.s, m.d_nodes, m.d_leaf, m.d_meta, q.ntrees, x, n, q.F, m.max_int, m.K, m.loss, q.link, m.all_numeric ? 1 : 0, shape,
+                                        static_cast<float *>(out));
+    return launch_walk_rows(m.s, m.d_nodes, std::max(1, m.max_int), m.d_meta, m.d_leaf, m.d_cid, q.ntrees, x, n, n, q.F, m.wide, m.K, m.loss, q.link,
+                            static_cast<float *>(out), nullptr, 0, 0);
+}
+
+template <typename T>
+void widen(const T *src, uint32_t *dst, int64_t n) {
+    for (int64_t i = 0; i < n; i++) dst[i] = src[i];
+}
+
+int run(Model &m, const Request &q) {
+    const int leaf_bytes = !q.leaf_out ? 0 : m.max_nodes <= 255 ? 1 : m.max_nodes <= 65535 ? 2 : 4;
+    const int64_t back = q.leaf_out ? (int64_t)q.ntrees * leaf_bytes : (int64_t)m.K * 4; // bytes a row sends back
+    const int64_t per_row = q.F + back;
+    // pieces of a sixth of the whole, so that binning, copies and kernels overlap; 256 KB at least, a buffer at most
+    const int64_t goal = std::min<int64_t>((int64_t)PINNED_BYTES - 4096, std::max<int64_t>(256 << 10, q.N * per_row / 6));
+    ARGCHK(64 * per_row <= (int64_t)PINNED_BYTES - 4096, "too many trees for one piece");
+    const int64_t rows_most = std::max<int64_t>(64, goal / per_row / 64 * 64);
+    const bool rowwise = q.plan && q.src.rows_contiguous();
+    const BinPieces B(q.N, q.F, rowwise, true, rows_most, 0);
+    const int NS = (int)std::min<int64_t>(PinnedSlots::NS, B.np);
+    const size_t xs = ((size_t)B.rows * q.F + 255) / 256 * 256; // a buffer holds a piece's bins, then what comes back
+    PinnedSlots U(m.s);
+    int r = U.init(NS);
+    if (r != EVT_OK) return r;
+    const bool direct = B.np == 1 && (int64_t)q.N * q.F <= 65536; // a few bins are read over the bus by the kernel itself
+    if (!direct) {
+        r = grow(&m.d_x, &m.cap_x, xs * NS);
+        if (r != EVT_OK) return r;
+    }
+    auto piece = [&](int64_t p, int64_t *r0, int64_t *n) {
+        int f0, f1;
+        B.at(p, r0, n, &f0, &f1);
+    };
+    auto fill = [&](int64_t p, int t) {
+        uint8_t *h = static_cast<uint8_t *>(U.host[p % NS]);
+        if (q.plan) {
+            B.bin(*q.plan, q.src, p, t, h);
+        } else {
+            int64_t r0, n;
+            piece(p, &r0, &n);
+            const int64_t b0 = (int64_t)(t % B.row_blocks) * B.block;
+            const int f = t / B.row_blocks;
+            if (b0 < n) memcpy(h + (size_t)f * n + b0, q.bins + (size_t)f * q.N + r0 + b0, (size_t)std::min(B.block, n - b0));
+        }
+    };
+    auto send = [&](int64_t p) -> int {
+        int64_t r0, n;
+        piece(p, &r0, &n);
+        uint8_t *h = static_cast<uint8_t *>(U.host[p % NS]);
+        const uint8_t *x = h;
+        if (!direct) {
+            HIPCHK(hipMemcpyAsync(m.d_x + (p % NS) * xs, h, (size_t)n * q.F, hipMemcpyHostToDevice, m.s));
+            x = m.d_x + (p % NS) * xs;
+        }
+        const int rw = walk(m, q, x, n, h + xs, leaf_bytes); // the kernel writes what comes back over the bus itself
+        if (rw != EVT_OK) return rw;
+        if (!direct) HIPCHK(hipEventRecord(U.ev[p % NS], m.s));
+        return EVT_OK;
+    };
+    auto retire = [&](int64_t p) {
+        int64_t r0, n;
+        piece(p, &r0, &n);
+        const uint8_t *h = static_cast<const uint8_t *>(U.host[p % NS]) + xs;
+        if (q.leaf_out) {
+            hb_parallel(q.ntrees, (int)std::min<int64_t>(hb_workers(n * q.ntrees / 2), 8), [&](int t) {
+                uint32_t *d = q.leaf_out + (size_t)t * q.N + r0;
+                const size_t at = (size_t)t * n;
+                if (leaf_bytes == 1) widen(h + at, d, n);
+                else if (leaf_bytes == 2) widen(reinterpret_cast<const uint16_t *>(h) + at, d, n);
+                else widen(reinterpret_cast<const uint32_t *>(h) + at, d, n);
+            });
+        } else {
+            memcpy(q.out + (size_t)r0 * m.K, h, (size_t)n * m.K * 4);
+        }
+    };
+    if (direct) {
+        for (int t = 0; t < B.per_piece; t++) fill(0, t);
+        r = send(0);
+        if (r != EVT_OK) return r;
+        HIPCHK(hipStreamSynchronize(m.s));
+        U.idle = true;
+        retire(0);
+        return EVT_OK;
+    }
+    return run_pieces(U, NS, B.np, B.per_piece, hb_workers(q.plan ? q.N * q.F : q.N * q.F / 8), fill, send, retire);
+}
+
+} // namespace
+
+extern "C" int evt_model_create(int32_t loss, int32_t K, void **out) {
+    return guarded([&]() -> int {
+    ARGCHK(out, "out is NULL");
+    *out = nullptr;
+    ARGCHK(K >= 1 && K <= EVT_MAX_K && loss >= 0 && loss <= EVT_LOSS_LAST, "invalid loss or number of outputs");
+    int ndev = 0;
+    const int r = evt_device_count(&ndev);
+    if (r != EVT_OK) return r;
+    std::unique_ptr<Model> m(new Model());
+    m->loss = loss;
+    m->K = K;
+    HIPCHK(hipGetDevice(&m->device));
+    HIPCHK(hipStreamCreateWithFlags(&m->s, hipStreamNonBlocking));
+    *out = m.release();
+    return EVT_OK;
+    });
+}
+extern "C" int evt_model_destroy(void *model) {
+    return guarded([&]() -> int {
+    delete static_cast<Model *>(model);
+    return EVT_OK;
+    });
+}
+
+extern "C" int evt_model_predict(void *model, int32_t n_model, const int64_t *nnodes, const int64_t *const *feat, const uint8_t *const *cond_bin,
+                                 const float *const *pred, const uint8_t *const *split, const uint8_t *feattypes, int32_t nfeattypes,
+                                 const double *const *edges, const int32_t *n_edges, const void *x, int32_t dtype, int64_t row_stride, int64_t col_stride,
+                                 int64_t nobs, int32_t nfeats, int32_t ntrees, int32_t apply_link, float *out, uint32_t *leaf_out) {
+    return guarded([&]() -> int {
+    ARGCHK(model && nnodes && feat && cond_bin && pred && split && x, "NULL argument");
+    ARGCHK(n_model >= 1 && ntrees >= 1 && ntrees <= n_model && nobs >= 1 && nfeats >= 1 && nfeats <= EVT_MAX_FEATS, "nobs, nfeats, ntrees must be >= 1");
+    ARGCHK((out != nullptr) != (leaf_out != nullptr), "one of out and leaf_out");
+    Model &m = *static_cast<Model *>(model);
+    std::lock_guard<std::mutex> lock(m.mu);
+    HIPCHK(hipSetDevice(m.device));
+    const TreePtrs t{n_model, nnodes, feat, cond_bin, split, pred};
+    const size_t nft = feattypes ? (size_t)nfeattypes : 0;
+    if (m.feattypes.size() != nft || (nft && memcmp(m.feattypes.data(), feattypes, nft)) || !same_trees(m, t)) {
+        const int r = build(m, t, feattypes, nfeattypes);
+        if (r != EVT_OK) return r;
+    }
+    ARGCHK(m.max_feat <= nfeats, "tree feature id outside 1..nfeats");
+    Request q{nullptr, {}, nullptr, nobs, nfeats, ntrees, apply_link, out, leaf_out};
+    if (!edges) {
+        ARGCHK(dtype == EVT_U8, "a matrix of bins is EVT_U8");
+        q.bins = static_cast<const uint8_t *>(x);
+        return run(m, q);
+    }
+    ARGCHK((dtype == EVT_F32 || dtype == EVT_F64) && (row_stride == 1 || col_stride == 1), "dtype must be EVT_F32 or EVT_F64 and one of the two strides 1");
+    bool same = m.edge_off.size() == (size_t)nfeats + 1;
+    for (int j = 0; j < nfeats; j++) {
+        ARGCHK(edges[j] && n_edges[j] >= 1 && n_edges[j] <= 254, "each feature needs 1..254 edges");
+        same = same && m.edge_off[j + 1] - m.edge_off[j] == n_edges[j] && !memcmp(m.edges.data() + m.edge_off[j], edges[j], 8 * (size_t)n_edges[j]);
+    }
+    if (!same) {
+        m.plan[0].reset();
+        m.plan[1].reset();
+        m.edges.clear();
+        m.edge_off.assign(1, 0);
+        for (int j = 0; j < nfeats; j++) {
+            m.edges.insert(m.edges.end(), edges[j], edges[j] + n_edges[j]);
+            m.edge_off.push_back((int32_t)m.edges.size());
+        }
+    }
+    std::unique_ptr<HbPlan> &plan = m.plan[dtype];
+    if (!plan) {
+        plan.reset(new HbPlan());
+        plan->build(m.edges.data(), m.edge_off.data(), nfeats, dtype);
+    }
+    q.plan = plan.get();
+    q.src = HbSource{x, dtype, row_stride, col_stride};
+    return run(m, q);
+    });
+}

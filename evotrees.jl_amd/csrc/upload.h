@@ -7,7 +7,7 @@
 // PINNED_KEPT stay behind when nobody uses them (32 MB); evt_trim gives those back.  Any thread, any device (portable).
 static const size_t PINNED_BYTES = (size_t)8 << 20;
 static const int PINNED_KEPT = 4;
-void *pinned_take();          // nullptr: out of memory (the error is set)
+void *pinned_take();          // nullptr: out of memory (the error is set); the device uses the same address
 void pinned_give(void *p);    // nothing on the device may still use it
 
 struct PinnedSlots { // NS of them, with an event each for the work that reads or writes them
@@ -34,16 +34,96 @@ struct PinnedSlots { // NS of them, with an event each for the work that reads o
     }
 };
 
-// How a matrix of N rows and F features is cut into pieces of at most `bytes` bins: row ranges of all features where its rows are
-// contiguous, whole columns (or row ranges of one) where its columns are.
+// How a matrix of N rows and F features is cut into pieces: row ranges of all features, or whole columns (or row ranges of one).
 struct BinPieces {
     int64_t N, rows; // rows of a piece
     int F, cols;     // features of a piece
     int64_t np;      // pieces
     int64_t row_pieces;
-    BinPieces(int64_t N_, int F_, bool rows_contiguous, size_t bytes);
+    bool rowwise;    // the source's rows are contiguous
+    // tasks of a piece: blocks of rows, of all its features or of one
+    int64_t block;
+    int per_piece, row_blocks;
+    BinPieces(int64_t N_, int F_, bool src_rows_contiguous, bool by_rows, int64_t rows_most, int64_t cells_most);
     void at(int64_t p, int64_t *r0, int64_t *n, int *f0, int *f1) const;
+    void bin(const HbPlan &P, const HbSource &S, int64_t p, int t, uint8_t *out) const; // the bin of (r, f) to out[(f - f0) * n + r - r0]
 };
-// Binned matrix -> device, column j to xcm + j * ldo.  Workers bin pieces into pinned buffers while earlier ones are copied; the
-// data has arrived when the call returns.
+
+// The pieces 0 .. np - 1 through NS buffers: piece p is filled by its `tasks` calls of fill(p, t), on worker threads; then send(p) queues
+// what the device does with it and records U.ev[p % NS]; when that event has come, retire(p), on the calling thread, and the buffer
+// is free for piece p + NS.  Everything has been retired when the call returns EVT_OK.
+template <typename Fill, typename Send, typename Retire>
+static int run_pieces(PinnedSlots &U, int NS, int64_t np, int tasks, int workers, Fill fill, Send send, Retire retire) {
+    if (np <= 2 || workers == 0) { // the calling thread fills too
+        int64_t back = 0;
+        for (int64_t p = 0; p < np; p++) {
+            if (p >= NS) {
+                HIPCHK(hipEventSynchronize(U.ev[back % NS]));
+                retire(back++);
+            }
+            hb_parallel(tasks, workers, [&](int t) { fill(p, t); });
+            const int r = send(p);
+            if (r != EVT_OK) return r;
+        }
+        for (; back < np; back++) {
+            HIPCHK(hipEventSynchronize(U.ev[back % NS]));
+            retire(back);
+        }
+        U.idle = true;
+        return EVT_OK;
+    }
+    // Many pieces: the workers run through the tasks of all of them, as far as buffers are free
+    const int64_t total = np * tasks;
+    std::atomic<int64_t> next{0}, released{NS};
+    std::vector<std::atomic<int>> done((size_t)np);
+    for (auto &d : done) d.store(0, std::memory_order_relaxed);
+    std::atomic<bool> stop{false};
+    auto work = [&] {
+        for (int64_t t; (t = next.fetch_add(1, std::memory_order_relaxed)) < total;) {
+            const int64_t p = t / tasks;
+            while (p >= released.load(std::memory_order_acquire)) {
+                if (stop.load(std::memory_order_relaxed)) return;
+                std::this_thread::yield();
+            }
+            fill(p, (int)(t % tasks));
+            done[(size_t)p].fetch_add(1, std::memory_order_release);
+        }
+    };
+    struct Joined {
+        std::atomic<bool> &stop;
+        std::vector<std::thread> th;
+        ~Joined() {
+            stop.store(true);
+            for (auto &t : th) t.join();
+        }
+    } ws{stop, {}};
+    for (int w = 0; w < workers; w++) ws.th.emplace_back(work);
+    int64_t back = 0;
+    for (int64_t p = 0; p < np; p++) {
+        while (done[(size_t)p].load(std::memory_order_acquire) < tasks) {
+            if (back < p) { // the oldest piece sent that has not been retired
+                const hipError_t q = hipEventQuery(U.ev[back % NS]);
+                if (q == hipSuccess) {
+                    retire(back++);
+                    released.store(back + NS, std::memory_order_release);
+                } else if (q == hipErrorNotReady) {
+                    (void)hipGetLastError();
+                } else {
+                    HIPCHK(q);
+                }
+            }
+            std::this_thread::yield();
+        }
+        const int r = send(p);
+        if (r != EVT_OK) return r;
+    }
+    for (; back < np; back++) {
+        HIPCHK(hipEventSynchronize(U.ev[back % NS]));
+        retire(back);
+    }
+    U.idle = true;
+    return EVT_OK;
+}
+
+// Binned matrix -> device, column j to xcm + j * ldo.  The data has arrived when the call returns.
 int upload_bins(hipStream_t s, const HbPlan &P, const HbSource &S, int64_t N, uint8_t *xcm, int64_t ldo);

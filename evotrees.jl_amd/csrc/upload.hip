@@ -20,9 +20,17 @@ void *pinned_take() {
     }
     void *p = nullptr;
     const hipError_t e = hipHostMalloc(&p, PINNED_BYTES, hipHostMallocPortable);
-    if (e == hipSuccess) return p;
-    evt_set_error("hipHostMalloc failed: %s", hipGetErrorString(e));
-    return nullptr;
+    if (e != hipSuccess) {
+        evt_set_error("hipHostMalloc failed: %s", hipGetErrorString(e));
+        return nullptr;
+    }
+    void *dev = nullptr;
+    if (hipHostGetDevicePointer(&dev, p, 0) != hipSuccess || dev != p) {
+        evt_set_error("pinned buffer is not addressable from the device");
+        (void)hipHostFree(p);
+        return nullptr;
+    }
+    return p;
 }
 void pinned_give(void *p) {
     {
@@ -46,20 +54,24 @@ extern "C" int evt_trim(void) {
     });
 }
 
-BinPieces::BinPieces(int64_t N_, int F_, bool rows_contiguous, size_t bytes) : N(N_), F(F_) {
-    const int64_t cells = (int64_t)bytes;
-    if (rows_contiguous) {
+BinPieces::BinPieces(int64_t N_, int F_, bool src_rows_contiguous, bool by_rows, int64_t rows_most, int64_t cells_most)
+    : N(N_), F(F_), rowwise(src_rows_contiguous) {
+    if (by_rows) {
         cols = F;
-        rows = std::min(N, std::max<int64_t>(64, cells / F / 64 * 64));
-    } else if (N <= cells) {
+        rows = std::min(N, rows_most);
+    } else if (N <= cells_most) {
         rows = N;
-        cols = (int)std::max<int64_t>(1, std::min<int64_t>(F, cells / N));
+        cols = (int)std::max<int64_t>(1, std::min<int64_t>(F, cells_most / N));
     } else {
-        rows = cells;
+        rows = cells_most;
         cols = 1;
     }
     row_pieces = (N + rows - 1) / rows;
     np = row_pieces * ((F + cols - 1) / cols);
+    // a task is about 64k cells: 25 us of work, against 0.1 us to hand it out
+    block = rowwise ? std::max<int64_t>(64, 65536 / F / 64 * 64) : 65536;
+    row_blocks = (int)((rows + block - 1) / block);
+    per_piece = rowwise ? row_blocks : row_blocks * cols;
 }
 void BinPieces::at(int64_t p, int64_t *r0, int64_t *n, int *f0, int *f1) const {
     *r0 = (p % row_pieces) * rows;
@@ -67,109 +79,41 @@ void BinPieces::at(int64_t p, int64_t *r0, int64_t *n, int *f0, int *f1) const {
     *f0 = (int)(p / row_pieces) * cols;
     *f1 = std::min(F, *f0 + cols);
 }
-
-// the bins of task t of a piece: a block of rows of all its features, or a block of rows of one
-struct PieceTasks {
-    int64_t block;
-    int per_piece, row_blocks;
-    bool rowwise;
-    PieceTasks(const BinPieces &B, bool rows_contiguous) : rowwise(rows_contiguous) {
-        // about 64k cells: 25 us of work, against 0.1 us to hand it out
-        block = rowwise ? std::max<int64_t>(64, 65536 / B.F / 64 * 64) : 65536;
-        row_blocks = (int)((B.rows + block - 1) / block);
-        per_piece = rowwise ? row_blocks : row_blocks * B.cols;
+void BinPieces::bin(const HbPlan &P, const HbSource &S, int64_t p, int t, uint8_t *out) const {
+    int64_t r0, n;
+    int f0, f1;
+    at(p, &r0, &n, &f0, &f1);
+    const int64_t b0 = (int64_t)(t % row_blocks) * block;
+    if (b0 >= n) return;
+    const int64_t m = std::min(block, n - b0);
+    if (rowwise) {
+        hb_bin(P, S, r0 + b0, m, f0, f1, out + b0, n);
+    } else {
+        const int f = f0 + t / row_blocks;
+        if (f < f1) hb_bin(P, S, r0 + b0, m, f, f + 1, out + (size_t)(f - f0) * n + b0, n);
     }
-    void run(const HbPlan &P, const HbSource &S, int64_t r0, int64_t n, int f0, int f1, uint8_t *out, int t) const {
-        const int64_t b0 = (int64_t)(t % row_blocks) * block;
-        if (b0 >= n) return;
-        const int64_t m = std::min(block, n - b0);
-        if (rowwise) {
-            hb_bin(P, S, r0 + b0, m, f0, f1, out + b0, n);
-        } else {
-            const int f = f0 + t / row_blocks;
-            if (f < f1) hb_bin(P, S, r0 + b0, m, f, f + 1, out + (size_t)(f - f0) * n + b0, n);
-        }
-    }
-};
+}
 
 int upload_bins(hipStream_t s, const HbPlan &P, const HbSource &S, int64_t N, uint8_t *xcm, int64_t ldo) {
     const bool rowwise = S.rows_contiguous();
-    const BinPieces B(N, P.F, rowwise, PINNED_BYTES);
-    const PieceTasks T(B, rowwise);
+    const BinPieces B(N, P.F, rowwise, rowwise, std::max<int64_t>(64, (int64_t)PINNED_BYTES / P.F / 64 * 64), (int64_t)PINNED_BYTES);
     const int NS = (int)std::min<int64_t>(PinnedSlots::NS, B.np);
     PinnedSlots U(s);
-    int r = U.init(NS);
+    const int r = U.init(NS);
     if (r != EVT_OK) return r;
-    auto send = [&](int64_t p) -> hipError_t {
+    auto send = [&](int64_t p) -> int {
         int64_t r0, n;
         int f0, f1;
         B.at(p, &r0, &n, &f0, &f1);
         uint8_t *dst = xcm + (size_t)f0 * ldo + r0;
         const void *src = U.host[p % NS];
-        hipError_t e = (n == ldo || f1 - f0 == 1) ? hipMemcpyAsync(dst, src, (size_t)n * (f1 - f0), hipMemcpyHostToDevice, s)
-                                                  : hipMemcpy2DAsync(dst, (size_t)ldo, src, (size_t)n, (size_t)n, (size_t)(f1 - f0), hipMemcpyHostToDevice, s);
-        return e == hipSuccess ? hipEventRecord(U.ev[p % NS], s) : e;
-    };
-    auto bin = [&](int64_t p, int t) {
-        int64_t r0, n;
-        int f0, f1;
-        B.at(p, &r0, &n, &f0, &f1);
-        T.run(P, S, r0, n, f0, f1, static_cast<uint8_t *>(U.host[p % NS]), t);
-    };
-    const int workers = hb_workers(N * P.F);
-    if (B.np <= 2 || workers == 0) { // the calling thread works too
-        for (int64_t p = 0; p < B.np; p++) {
-            if (p >= NS) HIPCHK(hipEventSynchronize(U.ev[p % NS]));
-            hb_parallel(T.per_piece, workers, [&](int t) { bin(p, t); });
-            HIPCHK(send(p));
-        }
-        HIPCHK(hipStreamSynchronize(s));
-        U.idle = true;
+        if (n == ldo || f1 - f0 == 1) HIPCHK(hipMemcpyAsync(dst, src, (size_t)n * (f1 - f0), hipMemcpyHostToDevice, s));
+        else HIPCHK(hipMemcpy2DAsync(dst, (size_t)ldo, src, (size_t)n, (size_t)n, (size_t)(f1 - f0), hipMemcpyHostToDevice, s));
+        HIPCHK(hipEventRecord(U.ev[p % NS], s));
         return EVT_OK;
-    }
-    // Many pieces: the workers run through the tasks of all of them, as far as buffers are free; the calling thread sends a piece when
-    // its last task is done and frees a buffer when its copy has arrived.
-    const int64_t total = B.np * T.per_piece;
-    std::atomic<int64_t> next{0}, released{NS};
-    std::vector<std::atomic<int>> done((size_t)B.np);
-    for (auto &d : done) d.store(0, std::memory_order_relaxed);
-    std::atomic<bool> stop{false};
-    auto work = [&] {
-        for (int64_t t; (t = next.fetch_add(1, std::memory_order_relaxed)) < total;) {
-            const int64_t p = t / T.per_piece;
-            while (p >= released.load(std::memory_order_acquire)) {
-                if (stop.load(std::memory_order_relaxed)) return;
-                std::this_thread::yield();
-            }
-            bin(p, (int)(t % T.per_piece));
-            done[(size_t)p].fetch_add(1, std::memory_order_release);
-        }
     };
-    struct Joined {
-        std::atomic<bool> &stop;
-        std::vector<std::thread> th;
-        ~Joined() {
-            stop.store(true);
-            for (auto &t : th) t.join();
-        }
-    } ws{stop, {}};
-    for (int w = 0; w < workers; w++) ws.th.emplace_back(work);
-    int64_t freed = NS; // pieces whose buffer is free for binning, as far as released
-    for (int64_t p = 0; p < B.np; p++) {
-        while (done[(size_t)p].load(std::memory_order_acquire) < T.per_piece) {
-            if (freed < B.np && freed - NS < p) { // the oldest piece sent whose buffer has not been handed on
-                const hipError_t q = hipEventQuery(U.ev[freed % NS]);
-                if (q == hipSuccess) released.store(++freed, std::memory_order_release);
-                else if (q == hipErrorNotReady) (void)hipGetLastError();
-                else HIPCHK(q);
-            }
-            std::this_thread::yield();
-        }
-        HIPCHK(send(p));
-    }
-    HIPCHK(hipStreamSynchronize(s));
-    U.idle = true;
-    return EVT_OK;
+    return run_pieces(U, NS, B.np, B.per_piece, hb_workers(N * P.F), [&](int64_t p, int t) { B.bin(P, S, p, t, static_cast<uint8_t *>(U.host[p % NS])); }, send,
+                      [](int64_t) {});
 }
 
 // ---- host-only entry points ---------------------------------------------------------------------

@@ -22,7 +22,7 @@
  *    different threads.
  *  - The library installs no signal handlers and never calls back into the caller's runtime.
  *    The calls that take a whole matrix or table from host memory (evt_binarize, evt_binarize_f64,
- *    evt_predict_f64, evt_bin_columns, evt_order_stats, and evt_set_xbin / evt_predict from 64 MB up)
+ *    evt_predict_f64, evt_model_predict, evt_bin_columns, evt_order_stats, and evt_set_xbin / evt_predict from 64 MB up)
  *    bin or copy it with worker threads of their own, up to one per core, which only read the
  *    caller's memory and are joined before the call returns; no other call starts a thread.
  */
@@ -335,6 +335,21 @@ int evt_predict_f64(int64_t nobs, int32_t nfeats, const double *x_colmajor, cons
 int evt_predict_leaf_idx(int64_t nobs, int32_t nfeats, const uint8_t *x_bin_colmajor, const uint8_t *feattypes,
                          int32_t ntrees, const int64_t *tree_off, const int64_t *feat, const uint8_t *cond_bin,
                          const uint8_t *split, uint32_t *out);
+
+/* _predict and predict_leaf_idx for a program that keeps its model: the packed trees, the searchable edges and the work buffers stay
+ * with the model handle.  The arrays of the trees remain the caller's and are given with every call, an array of pointers for each
+ * field (tree t: nnodes[t] <= 2^20 - 1 entries of feat / cond_bin / split, K times that of pred); the call compares them with what it
+ * packed before and packs again what has changed, so a call on other trees is right, and only then slow.  The first ntrees
+ * of the n_model trees are walked.  edges: nfeats pointers to ascending Float64 arrays of n_edges entries, and x is a matrix in
+ * host memory as evt_binarize takes it; edges == NULL: x holds nobs x nfeats column-major bins (EVT_U8).  Exactly one of out
+ * (K x nobs, link applied when apply_link != 0) and leaf_out (nobs x ntrees column-major) is not NULL; both are host memory.
+ * Results equal evt_predict's and evt_predict_leaf_idx's, bit for bit.  Calls on one model from several threads take turns. */
+int evt_model_create(int32_t loss, int32_t K, void **out);
+int evt_model_destroy(void *model);
+int evt_model_predict(void *model, int32_t n_model, const int64_t *nnodes, const int64_t *const *feat, const uint8_t *const *cond_bin,
+                      const float *const *pred, const uint8_t *const *split, const uint8_t *feattypes, int32_t nfeattypes,
+                      const double *const *edges, const int32_t *n_edges, const void *x, int32_t dtype, int64_t row_stride, int64_t col_stride,
+                      int64_t nobs, int32_t nfeats, int32_t ntrees, int32_t apply_link, float *out, uint32_t *leaf_out);
 
 /* No counterpart in the reference: evt_predict for callers that cannot allocate - code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc.  Every pointer is device memory: x_bin (nobs x nfeats column-major),

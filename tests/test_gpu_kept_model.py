@@ -1,0 +1,74 @@
+"""Predictions of a kept model (evt_model_predict) against the whole-model calls that pack their trees every time, bit for bit: every
+rows-per-block of the row kernel and the hand-over to the 1024-row kernel, output counts, tree sizes, feature counts."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import _random_tree
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(evt, rng, F, B, K, loss, depths, cat=False):
+    trees = []
+    for d in depths:
+        r, t = _random_tree(rng, d, F, B, K), evt.Tree(K, (1 << d) - 1)
+        for f in ("feat", "cond_bin", "pred", "split"):
+            getattr(t, f)[...] = getattr(r, f)
+        trees.append(t)
+    ft = (rng.random(F) > 0.3).astype(np.uint8) if cat else np.ones(F, np.uint8)
+    return evt.EvoTree(loss, K, trees, dict(edges=[np.sort(rng.random(B - 1)) for _ in range(F)], feattypes=ft, feature_names=["f%d" % j for j in range(F)]))
+
+
+def _check(evt, m, x, n=None):
+    L = evt._lib
+    trees, ft = m.trees[:n], m.info["feattypes"]
+    want = L.predict_model_f64(np.ascontiguousarray(x.T, np.float64), m.info["edges"], ft, m.loss_type, m.K, trees)
+    got = evt.predict(m, x, ntree_limit=n)
+    assert np.array_equal(got.reshape(want.shape).view(np.uint32), want.view(np.uint32))
+    assert np.array_equal(evt.predict_leaf_idx(m, x, ntree_limit=n), L.predict_leaf_idx(evt.binarize(x, m.info["edges"]), ft, trees))
+
+
+@pytest.mark.parametrize("N,F,B,K,loss,depths,cat", [
+    (1, 1, 2, 1, "mse", [1], False),
+    (1, 20, 64, 1, "mse", [1] + [6] * 100, False),
+    (3, 7, 16, 2, "gaussian_mle", [1, 4, 2, 5, 7], True),
+    (1024, 28, 128, 1, "logloss", [1] + [8] * 40, False),
+    (1025, 5, 32, 4, "mlogloss", [6, 3, 6], True),
+    (8193, 13, 255, 16, "mlogloss", [5] * 70, False),
+    (65_537, 3, 8, 5, "mlogloss", [9, 1, 9], False),
+    (140_001, 9, 32, 1, "mse", [6] * 9, True),
+    (300_001, 30, 32, 2, "gaussian_mle", [1] + [6] * 5, False),
+    (130, 1030, 16, 1, "mse", [9] * 6, False),
+    (5, 40_000, 4, 1, "mse", [10] * 3, False),
+    (70, 4, 16, 1, "mse", [3] * 2100, False),
+])
+def test_equals_the_unkept_calls(evt, N, F, B, K, loss, depths, cat):
+    rng = np.random.default_rng(N + F)
+    m = _model(evt, rng, F, B, K, loss, depths, cat)
+    x = rng.random((N, F), np.float32)
+    _check(evt, m, x)
+    _check(evt, m, np.asfortranarray(x.astype(np.float64)), max(1, len(depths) // 2))
+
+
+def test_follows_changes_of_the_model(evt):
+    rng = np.random.default_rng(9)
+    m = _model(evt, rng, 6, 32, 1, "mse", [5] * 8)
+    x = rng.random((50, 6))
+    _check(evt, m, x)
+    m.trees[3].pred *= 2  # in place
+    _check(evt, m, x)
+    m.trees[2].pred = m.trees[2].pred + 1  # another array
+    _check(evt, m, x)
+    m.info["edges"][1] += 0.01
+    _check(evt, m, x)
+    m.info["edges"][2] = m.info["edges"][2][:7] * 0.5
+    _check(evt, m, x)
+    m.trees[4] = m.trees[0]
+    m.trees.append(m.trees[1])
+    _check(evt, m, x)
+    with pytest.raises(ValueError):
+        evt.predict(m, np.zeros((3, 7)))
+    m.trees[1].split[-1] = 1  # a split node whose children do not exist
+    m.trees[1].feat[-1] = 1
+    with pytest.raises(evt.EvtError):
+        evt.predict(m, x)
