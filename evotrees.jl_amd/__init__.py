@@ -160,11 +160,11 @@ def _quantiles(cols, idx, n, nbins):
     t = at - lo
     lo = lo.astype(np.int64)
     ranks, back = np.unique(np.concatenate([lo, np.minimum(lo + 1, n - 1)]), return_inverse=True)
-    v = _lib.order_stats(cols, idx, n, ranks)[:, back]
+    v = np.take(_lib.order_stats(cols, idx, n, ranks), back, axis=1)
     a, b = v[:, :nbins - 1], v[:, nbins - 1:]
     with np.errstate(invalid="ignore", over="ignore"):
         d = b - a
-        return np.where(t >= 0.5, b - d * (1 - t), a + d * t)
+        return np.ascontiguousarray(np.where(t >= 0.5, b - d * (1 - t), a + d * t))
 
 
 def get_edges(x, nbins, rng):

@@ -2,8 +2,11 @@
 
 #include <math.h>
 #include <string.h>
+#include <unistd.h>
 
 #include <algorithm>
+#include <condition_variable>
+#include <mutex>
 
 bool hb_has_avx512() {
 #if defined(__x86_64__)
@@ -16,9 +19,91 @@ bool hb_has_avx512() {
 }
 
 int hb_workers(int64_t cells) {
-    // a thread costs about 15 us to start and join and bins 4 cells per ns at most: one for every 128k cells
-    const int64_t most = std::max(1, (int)std::thread::hardware_concurrency()) - 1;
-    return (int)std::max<int64_t>(0, std::min<int64_t>(most, cells / 131072 - 1));
+    // a worker takes about 5 us to wake, in which the calling thread bins 8k cells
+    static const int64_t most = std::max(1, (int)std::thread::hardware_concurrency()) - 1;
+    return (int)std::max<int64_t>(0, std::min<int64_t>(most, cells / 16384 - 1));
+}
+
+// The worker threads: started when first needed, kept asleep between calls (waking one costs about 5 us, starting one 15 and more), at
+// most one per core.  One parallel region uses them at a time; a region that finds them taken starts threads of its own.
+namespace {
+struct Pool {
+    const pid_t pid = getpid();
+    std::mutex region; // held by the region that uses the workers
+    std::mutex m;
+    std::condition_variable cv, cv_done;
+    int threads = 0;
+    const std::function<void()> *job = nullptr; // null: nothing to join
+    uint64_t gen = 0;
+    int wanted = 0, active = 0;
+    void loop() {
+        uint64_t seen = 0;
+        std::unique_lock<std::mutex> lk(m);
+        for (;;) {
+            cv.wait(lk, [&] { return job && gen != seen && wanted > 0; });
+            seen = gen;
+            wanted--;
+            active++;
+            const std::function<void()> *j = job;
+            lk.unlock();
+            (*j)();
+            lk.lock();
+            if (--active == 0) cv_done.notify_all();
+        }
+    }
+    void start(int n, const std::function<void()> *j) {
+        std::lock_guard<std::mutex> lk(m);
+        for (; threads < n; threads++) std::thread([this] { loop(); }).detach();
+        job = j;
+        gen++;
+        wanted = n;
+        for (int i = 0; i < n; i++) cv.notify_one();
+    }
+    void finish() { // workers that have not joined by now do not; those that have are waited for
+        std::unique_lock<std::mutex> lk(m);
+        job = nullptr;
+        wanted = 0;
+        cv_done.wait(lk, [&] { return active == 0; });
+    }
+    static Pool &get() { // never destroyed: its threads outlive main.  After a fork the child has none of them and starts afresh
+        static std::mutex gm;
+        static Pool *p = nullptr;
+        std::lock_guard<std::mutex> lk(gm);
+        if (!p || p->pid != getpid()) p = new Pool();
+        return *p;
+    }
+};
+} // namespace
+
+HbWorkers::HbWorkers(int n, std::function<void()> f) : fn(std::move(f)) {
+    if (n <= 0) return;
+    Pool &p = Pool::get();
+    if (p.region.try_lock()) {
+        pool = &p;
+        try {
+            p.start(n, &fn);
+        } catch (...) {
+            join();
+            throw;
+        }
+    } else {
+        try {
+            for (int w = 0; w < n; w++) own.emplace_back(fn);
+        } catch (...) {
+            join();
+            throw;
+        }
+    }
+}
+void HbWorkers::join() {
+    if (pool) {
+        Pool *p = static_cast<Pool *>(pool);
+        p->finish();
+        p->region.unlock();
+        pool = nullptr;
+    }
+    for (auto &t : own) t.join();
+    own.clear();
 }
 
 void hb_parallel(int ntasks, int nworkers, const std::function<void(int)> &fn) {
@@ -26,14 +111,7 @@ void hb_parallel(int ntasks, int nworkers, const std::function<void(int)> &fn) {
     auto loop = [&] {
         for (int t; (t = next.fetch_add(1, std::memory_order_relaxed)) < ntasks;) fn(t);
     };
-    struct Joined { // joined also when a thread cannot be started
-        std::vector<std::thread> th;
-        ~Joined() {
-            for (auto &t : th) t.join();
-        }
-    } ws;
-    nworkers = std::min(nworkers, ntasks - 1);
-    for (int w = 0; w < nworkers; w++) ws.th.emplace_back(loop);
+    HbWorkers ws(std::min(nworkers, ntasks - 1), loop);
     loop();
 }
 

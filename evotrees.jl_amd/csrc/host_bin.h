@@ -62,5 +62,17 @@ void hb_bin_columns(const HbColumn *cols, int nc, int64_t n, const double *edges
 // a column with a NaN among them gets NaN throughout
 void hb_order_stats(const HbColumn *cols, int nc, const int64_t *idx, int64_t n, const int64_t *ranks, int nr, double *out);
 
-// fn(0) .. fn(ntasks - 1) on the calling thread and nworkers more, which are joined before it returns
+// f() on up to n worker threads (fewer, or none, when they come too late to join) until join(), which waits for those that joined
+class HbWorkers {
+    std::function<void()> fn;
+    void *pool = nullptr;
+    std::vector<std::thread> own;
+
+  public:
+    HbWorkers(int n, std::function<void()> f);
+    ~HbWorkers() { join(); }
+    HbWorkers(const HbWorkers &) = delete;
+    void join();
+};
+// fn(0) .. fn(ntasks - 1) on the calling thread and up to nworkers more; all are done when it returns
 void hb_parallel(int ntasks, int nworkers, const std::function<void(int)> &fn);

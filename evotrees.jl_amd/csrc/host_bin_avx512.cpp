@@ -182,14 +182,21 @@ void hb512_col(const void *x, int dtype, int64_t n, const HbFeature &f, const fl
 }
 
 // Rows one after the other in memory: tiles of 64 rows x 16 features are turned over in registers (16 x 16 keys at a time)
-// into a 4 KB buffer of columns, then binned a feature at a time and written as whole 64-byte lines.
+// into a 4 KB buffer of columns, then binned a feature at a time and written as whole 64-byte lines.  The next tile's rows are one
+// run of memory, read here in strides no hardware prefetcher follows: it is requested a share with every group of features.
 void hb512_rows(const void *x, int dtype, int64_t rs, int64_t n, const HbFeature *feat, int nf, const float *heap, uint8_t *out, int64_t ldo) {
     alignas(64) float key[16][64] = {};
     alignas(64) uint8_t bins[64];
+    const int64_t row_bytes = rs * (dtype == EVT_F32 ? 4 : 8), used = nf * (dtype == EVT_F32 ? 4 : 8);
+    const int groups = (nf + 15) / 16;
     for (int64_t r0 = 0; r0 < n; r0 += 64) {
         const int64_t nr = n - r0 < 64 ? n - r0 : 64;
+        const char *ahead = static_cast<const char *>(x) + (r0 + 64) * row_bytes;
+        const int64_t na = n - r0 - 64 < 64 ? n - r0 - 64 : 64;                                   // rows of the next tile
+        const int64_t dense = na <= 0 ? 0 : (row_bytes <= used + 64 ? (na - 1) * row_bytes + used : 0); // bytes, when nearly all are used
         for (int f0 = 0; f0 < nf; f0 += 16) {
             const int fc = nf - f0 < 16 ? nf - f0 : 16;
+            for (int64_t b = dense * (f0 / 16) / groups, e = dense * (f0 / 16 + 1) / groups; b < e; b += 64) _mm_prefetch(ahead + b, _MM_HINT_T0);
             const __mmask16 m = (__mmask16)((1u << fc) - 1);
             for (int g = 0; 16 * g < nr; g++) {
                 __m512 r[16];

@@ -442,12 +442,65 @@ int launch_leaf_idx_model(hipStream_t s, const uint32_t *nodes, const int64_t *o
     return EVT_OK;
 }
 
+// the leaf values of n trees for one row (tree t's at v + t * step) added to its running prediction in tree order, with predict!'s
+// clamps after each tree (src/predict.jl:1-84); values are read a few trees ahead of their use
+template <int KMAX, typename ADD>
+__device__ __forceinline__ void add_run(float *acc, const float *v, int step, int n, ADD add) {
+    int t = 0;
+    constexpr int U = KMAX <= 2 ? 8 : (KMAX <= 4 ? 4 : 2);
+    for (; t + U <= n; t += U) {
+        float lp[U][KMAX];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int k = 0; k < KMAX; k++) lp[u][k] = v[(t + u) * step + k];
+#pragma unroll
+        for (int u = 0; u < U; u++) add(acc, lp[u]);
+    }
+    for (; t < n; t++) {
+        float lp[KMAX];
+#pragma unroll
+        for (int k = 0; k < KMAX; k++) lp[k] = v[t * step + k];
+        add(acc, lp);
+    }
+}
+template <int KMAX>
+__device__ __forceinline__ void add_trees(float *acc, const float *v, int step, int n, int K, int loss) {
+    if (loss == EVT_LOSS_LOGLOSS) {
+        add_run<KMAX>(acc, v, step, n, [](float *a, const float *lp) {
+#pragma unroll
+            for (int k = 0; k < KMAX; k++) a[k] = fminf(fmaxf(a[k] + lp[k], -15.0f), 15.0f);
+        });
+    } else if (EVT_IS_MLE2P(loss)) {
+        add_run<KMAX>(acc, v, step, n, [](float *a, const float *lp) {
+#pragma unroll
+            for (int k = 0; k < KMAX; k++) a[k] = (k & 1) ? fmaxf(-15.0f, a[k] + lp[k]) : a[k] + lp[k];
+        });
+    } else if (loss == EVT_LOSS_MLOGLOSS) {
+        add_run<KMAX>(acc, v, step, n, [K](float *a, const float *lp) {
+            float m = -INFINITY;
+#pragma unroll
+            for (int k = 0; k < KMAX; k++) {
+                a[k] += lp[k];
+                m = k < K ? fmaxf(m, a[k]) : m;
+            }
+#pragma unroll
+            for (int k = 0; k < KMAX; k++) a[k] = fmaxf(-15.0f, a[k] - m);
+        });
+    } else {
+        add_run<KMAX>(acc, v, step, n, [](float *a, const float *lp) {
+#pragma unroll
+            for (int k = 0; k < KMAX; k++) a[k] += lp[k];
+        });
+    }
+}
+
 // Few rows, many trees: a block takes R rows and spreads the trees over its 256 / R lanes per row, so that a handful of rows still
 // occupies whole wavefronts (and a few thousand rows the chip), where a row per lane leaves a single chain of dependent reads.  A lane
 // walks WALK_U trees side by side over the completed trees (fixed depth, nodes from the caches: a model of 200 trees of
-// depth 8 is 100 KB); the leaf values of a run of trees meet in LDS, and one lane per row adds them in tree order with predict!'s
-// clamps, so the sum has the bits of the sequential one.  The bins may lie in pinned host memory, and so may the output.
-// Latency bound: three steps of a level (node, bin, next node) cost about 0.4 us from L2, whatever the number of rows in flight.
+// depth 8 is 100 KB); the leaf values of a run of trees meet in LDS, and one lane per row adds them in tree order,
+// so the sum has the bits of the sequential one.  The bins may lie in pinned host memory, and so may the output.
+// With a single row per block the nodes are first touched all at once: one trip to memory instead of one per level.
 // LEAF: the leaf's node id of every row and tree instead, tree by tree, in LB-byte words.
 #define WALK_U 4
 template <int KMAX, int R, bool LEAF, int LB>
@@ -456,11 +509,17 @@ __global__ __launch_bounds__(256) void k_walk_rows(const uint32_t *__restrict__ 
                                                   const uint8_t *__restrict__ x, int64_t ldx, int64_t n, int F, int wide, int K, int loss, int link,
                                                   float *__restrict__ out, void *__restrict__ leaf_out, int64_t leaf_ld) {
     constexpr int G = 256 / R;
-    extern __shared__ uint32_t smem[];
-    uint8_t *s_x = reinterpret_cast<uint8_t *>(smem);                      // [F][R]
-    float *s_v = reinterpret_cast<float *>(smem + ((size_t)F * R + 3) / 4); // [run][R][K]
+    extern __shared__ float4 smem4[];
+    float *s_v = reinterpret_cast<float *>(smem4);                                      // [run][R][KMAX]
+    uint8_t *s_x = reinterpret_cast<uint8_t *>(s_v + (LEAF ? 0 : (size_t)run * R * KMAX)); // [F][R]
     const int tid = threadIdx.x, r = tid % R, g = tid / R;
     const int64_t i0 = (int64_t)blockIdx.x * R;
+    if (R == 1) {
+        const int words = ntrees * stride < 8192 ? ntrees * stride : 8192;
+        uint32_t seen = 0;
+        for (int w = tid * 16; w < words; w += 256 * 16) seen |= cnodes[w];
+        asm volatile("" ::"v"(seen));
+    }
     for (int k = tid; k < F * R; k += 256) {
         const int64_t i = i0 + k % R;
         s_x[k] = x[(size_t)(k / R) * ldx + (i < n ? i : n - 1)];
@@ -472,58 +531,62 @@ __global__ __launch_bounds__(256) void k_walk_rows(const uint32_t *__restrict__ 
     for (int t0 = 0; t0 < ntrees; t0 += run) {
         const int t1 = t0 + run < ntrees ? t0 + run : ntrees;
         for (int tb = t0 + g; tb < t1; tb += G * WALK_U) {
-            uint32_t nid[WALK_U];
+            uint32_t nid[WALK_U], at[WALK_U];
             int levels[WALK_U], most = 0;
             const uint32_t *cn[WALK_U];
 #pragma unroll
             for (int u = 0; u < WALK_U; u++) {
-                const int t = tb + u * G;
+                const int t = tb + u * G < t1 ? tb + u * G : tb; // past the end: this lane's first tree again
+                const int4 m = *reinterpret_cast<const int4 *>(meta + t);
                 nid[u] = 1;
-                levels[u] = t < t1 ? meta[t].levels : 0;
-                cn[u] = cnodes + (size_t)(t < t1 ? t : t0) * stride;
-                most = levels[u] > most ? levels[u] : most;
+                cn[u] = cnodes + (size_t)(uint32_t)m.x;
+                at[u] = (uint32_t)m.y;
+                levels[u] = m.z;
+                most = m.z > most ? m.z : most;
             }
             for (int l = 0; l < most; l++) {
                 uint32_t nd[WALK_U];
 #pragma unroll
-                for (int u = 0; u < WALK_U; u++) nd[u] = l < levels[u] ? cn[u][nid[u] - 1] : 0u;
+                for (int u = 0; u < WALK_U; u++) nd[u] = cn[u][l < levels[u] ? nid[u] - 1 : 0];
 #pragma unroll
                 for (int u = 0; u < WALK_U; u++) {
-                    if (l >= levels[u]) continue;
                     const uint32_t f = wide ? nd[u] & 0xFFFFu : ((nd[u] >> 6) & 0x3FCu) | (nd[u] & 3u);
-                    nid[u] = step_node<false>(nid[u], nd[u], s_x[f * R + r]);
+                    const uint32_t next = step_node<false>(nid[u], nd[u], s_x[f * R + r]);
+                    nid[u] = l < levels[u] ? next : nid[u];
                 }
             }
 #pragma unroll
-            for (int u = 0; u < WALK_U; u++) {
-                const int t = tb + u * G;
-                if (t >= t1) continue;
-                const size_t at = (size_t)meta[t].leaf_off + (nid[u] - (1u << levels[u]));
-                if (LEAF) {
-                    const uint32_t id = cid[at];
+            for (int u = 0; u < WALK_U; u++) at[u] += nid[u] - (1u << levels[u]);
+            if (LEAF) {
+                uint32_t id[WALK_U];
+#pragma unroll
+                for (int u = 0; u < WALK_U; u++) id[u] = cid[at[u]];
+#pragma unroll
+                for (int u = 0; u < WALK_U; u++) {
+                    const int t = tb + u * G;
                     const size_t o = (size_t)t * leaf_ld + i0 + r;
-                    if (i0 + r < n) {
-                        if (LB == 1) static_cast<uint8_t *>(leaf_out)[o] = (uint8_t)id;
-                        else if (LB == 2) static_cast<uint16_t *>(leaf_out)[o] = (uint16_t)id;
-                        else static_cast<uint32_t *>(leaf_out)[o] = id;
+                    if (t < t1 && i0 + r < n) {
+                        if (LB == 1) static_cast<uint8_t *>(leaf_out)[o] = (uint8_t)id[u];
+                        else if (LB == 2) static_cast<uint16_t *>(leaf_out)[o] = (uint16_t)id[u];
+                        else static_cast<uint32_t *>(leaf_out)[o] = id[u];
                     }
-                } else {
-                    float *v = s_v + ((size_t)(t - t0) * R + r) * K;
-                    for (int k = 0; k < K; k++) v[k] = cleaf[at * K + k];
                 }
+            } else {
+                float lv[WALK_U][KMAX];
+#pragma unroll
+                for (int u = 0; u < WALK_U; u++)
+#pragma unroll
+                    for (int k = 0; k < KMAX; k++) lv[u][k] = cleaf[(size_t)at[u] * K + (k < K ? k : 0)];
+#pragma unroll
+                for (int u = 0; u < WALK_U; u++)
+                    if (tb + u * G < t1)
+#pragma unroll
+                        for (int k = 0; k < KMAX; k++) s_v[((size_t)(tb + u * G - t0) * R + r) * KMAX + k] = lv[u][k];
             }
         }
         if (LEAF) continue;
         __syncthreads();
-        if (tid < R) {
-#pragma unroll 4
-            for (int t = 0; t < t1 - t0; t++) {
-                float lp[KMAX];
-#pragma unroll
-                for (int k = 0; k < KMAX; k++) lp[k] = k < K ? s_v[((size_t)t * R + tid) * K + k] : 0.0f;
-                add_tree<KMAX>(acc, lp, K, loss);
-            }
-        }
+        if (tid < R) add_trees<KMAX>(acc, s_v + tid * KMAX, R * KMAX, t1 - t0, K, loss);
         __syncthreads();
     }
     if (!LEAF && tid < R && i0 + tid < n) {
@@ -544,8 +607,9 @@ static int launch_walk(hipStream_t s, const uint32_t *cnodes, int stride, const 
         once.mark(dev);
     }
     const int G = 256 / R;
-    const int run = LEAF ? ntrees : std::max(G, 8192 / (R * K) / G * G); // trees whose values fit 32 KB of LDS
-    const size_t lds = ((size_t)F * R + 3) / 4 * 4 + (LEAF ? 0 : (size_t)std::min(run, ntrees) * R * K * 4);
+    // trees whose values fit 32 KB of LDS
+    const int run = LEAF ? ntrees : std::min(ntrees, std::max(G, 8192 / (R * KMAX) / G * G));
+    const size_t lds = (size_t)F * R + (LEAF ? 0 : (size_t)run * R * KMAX * 4);
     hipLaunchKernelGGL((k_walk_rows<KMAX, R, LEAF, LB>), dim3((unsigned)((n + R - 1) / R)), dim3(256), lds, s, cnodes, stride,
                        static_cast<const ModelTree *>(meta), cleaf, cid, ntrees, run, x, ldx, n, F, wide, K, loss, link, out, leaf_out, leaf_ld);
     HIPCHK(hipGetLastError());
@@ -557,7 +621,8 @@ int launch_walk_rows(hipStream_t s, const uint32_t *cnodes, int stride, const vo
                      int64_t leaf_ld) {
     // rows per block: as few as fill the chip (1024 blocks of four wavefronts, eight of which share a compute unit), and no more than
     // 64 KB of bins
-    int R = n <= 1024 ? 1 : (n <= 8192 ? 4 : (n <= 65536 ? 16 : 64));
+    // (leaf ids go out R to a line: from 4096 rows on whole 64-byte ones)
+    int R = n <= 1024 ? 1 : (n <= (leaf_out ? 4096 : 8192) ? 4 : (n <= 32768 && !leaf_out ? 16 : 64));
     while (R > 1 && (size_t)R * F > 65536) R /= 4;
 #define EVT_WALK(KM_, LEAF_, LB_)                                                                                                                    \
     switch (R) {                                                                                                                                     \
@@ -571,7 +636,10 @@ int launch_walk_rows(hipStream_t s, const uint32_t *cnodes, int stride, const vo
         if (leaf_bytes == 2) { EVT_WALK(1, true, 2) }
         EVT_WALK(1, true, 4)
     }
+    if (K == 1) { EVT_WALK(1, false, 0) }
+    if (K == 2) { EVT_WALK(2, false, 0) }
     if (K <= 4) { EVT_WALK(4, false, 0) }
+    if (K <= 8) { EVT_WALK(8, false, 0) }
     EVT_WALK(EVT_MAX_K, false, 0)
 #undef EVT_WALK
 }

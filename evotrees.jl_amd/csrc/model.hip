@@ -223,8 +223,8 @@ int run(Model &m, const Request &q) {
     const int leaf_bytes = !q.leaf_out ? 0 : m.max_nodes <= 255 ? 1 : m.max_nodes <= 65535 ? 2 : 4;
     const int64_t back = q.leaf_out ? (int64_t)q.ntrees * leaf_bytes : (int64_t)m.K * 4; // bytes a row sends back
     const int64_t per_row = q.F + back;
-    // pieces of a sixth of the whole, so that binning, copies and kernels overlap; 256 KB at least, a buffer at most
-    const int64_t goal = std::min<int64_t>((int64_t)PINNED_BYTES - 4096, std::max<int64_t>(256 << 10, q.N * per_row / 6));
+    // pieces of a twelfth of the whole, so that binning, copies and kernels overlap; 256 KB at least, a buffer at most
+    const int64_t goal = std::min<int64_t>((int64_t)PINNED_BYTES - 4096, std::max<int64_t>(256 << 10, q.N * per_row / 12));
     ARGCHK(64 * per_row <= (int64_t)PINNED_BYTES - 4096, "too many trees for one piece");
     const int64_t rows_most = std::max<int64_t>(64, goal / per_row / 64 * 64);
     const bool rowwise = q.plan && q.src.rows_contiguous();

@@ -89,15 +89,12 @@ static int run_pieces(PinnedSlots &U, int NS, int64_t np, int tasks, int workers
             done[(size_t)p].fetch_add(1, std::memory_order_release);
         }
     };
-    struct Joined {
-        std::atomic<bool> &stop;
-        std::vector<std::thread> th;
-        ~Joined() {
-            stop.store(true);
-            for (auto &t : th) t.join();
-        }
-    } ws{stop, {}};
-    for (int w = 0; w < workers; w++) ws.th.emplace_back(work);
+    struct Stop { // whatever ends the call, workers that wait for a buffer stop waiting
+        std::atomic<bool> &flag;
+        ~Stop() { flag.store(true); }
+    };
+    HbWorkers ws(workers, work);
+    Stop on_return{stop};
     int64_t back = 0;
     for (int64_t p = 0; p < np; p++) {
         while (done[(size_t)p].load(std::memory_order_acquire) < tasks) {

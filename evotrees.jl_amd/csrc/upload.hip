@@ -68,8 +68,9 @@ BinPieces::BinPieces(int64_t N_, int F_, bool src_rows_contiguous, bool by_rows,
     }
     row_pieces = (N + rows - 1) / rows;
     np = row_pieces * ((F + cols - 1) / cols);
-    // a task is about 64k cells: 25 us of work, against 0.1 us to hand it out
-    block = rowwise ? std::max<int64_t>(64, 65536 / F / 64 * 64) : 65536;
+    // a task is 64k cells at most (25 us of work, against 0.1 us to hand it out), less when they would be few
+    const int64_t cells = std::max<int64_t>(4096, std::min<int64_t>(65536, rows * cols / 64));
+    block = std::max<int64_t>(64, (rowwise ? cells / F : std::min(cells, rows)) / 64 * 64);
     row_blocks = (int)((rows + block - 1) / block);
     per_piece = rowwise ? row_blocks : row_blocks * cols;
 }

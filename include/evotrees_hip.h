@@ -23,8 +23,9 @@
  *  - The library installs no signal handlers and never calls back into the caller's runtime.
  *    The calls that take a whole matrix or table from host memory (evt_binarize, evt_binarize_f64,
  *    evt_predict_f64, evt_model_predict, evt_bin_columns, evt_order_stats, and evt_set_xbin / evt_predict from 64 MB up)
- *    bin or copy it with worker threads of their own, up to one per core, which only read the
- *    caller's memory and are joined before the call returns; no other call starts a thread.
+ *    bin or copy it with worker threads of the library's own, up to one per core, which only touch
+ *    the caller's memory and have finished before the call returns (they stay asleep between
+ *    calls); no other call uses a thread.
  */
 #ifndef EVOTREES_HIP_H
 #define EVOTREES_HIP_H
