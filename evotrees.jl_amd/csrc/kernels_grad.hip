@@ -345,7 +345,7 @@ __global__ __launch_bounds__(256) void k_absmax(const float *__restrict__ grad, 
 // the row count in its low 16 bits ((q << 16) + 1) so that one 64-bit LDS add serves both.
 // Channel a reads gradient row a, except for mse whose channels are {g, w} = rows {0, 2}.
 __global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ grad, unsigned long long *__restrict__ gq, int64_t N,
-                                                 int NK, int NA, int mse, int pack, const uint32_t *__restrict__ absmax, uint32_t *absmax_next,
+                                                 int NK, int NA, int mse, int pack, int pack_wide, const uint32_t *__restrict__ absmax, uint32_t *absmax_next,
                                                  const int32_t *__restrict__ qbits, int32_t *qexp, double *qmul, double *qscale_g, int NAg,
                                                  int loss, int unit_w) {
     __shared__ double s_qmul[EVT_MC_MAX_NK];
@@ -394,6 +394,7 @@ __global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ grad
                 reinterpret_cast<int32_t *>(gq)[i] = (int32_t)q;
                 continue;
             }
+            if (a == 0 && pack_wide) q = (long long)(((unsigned long long)q << EVT_PACK_CNT_BITS) + 1ull); // the same word, for kernels that read every channel alike
             gq[(size_t)a * N + i] = (unsigned long long)q;
         }
     }
@@ -520,7 +521,7 @@ int launch_quantize(evt_ctx *c) {
     c->qscale = c->qscale_buf[c->q_cur];
     double *qmul = c->qscale + EVT_MC_MAX_NK; // decode scales per global channel first, then encode multipliers per gradient row
     hipLaunchKernelGGL(k_quantize, dim3((unsigned)std::min<int64_t>(4096, (c->N + 255) / 256)), dim3(256), 0, c->stream, c->grad, c->gq, c->N, c->NK, c->NA,
-                       EVT_TWO_CHAN(c->loss, c->K) ? 1 : 0, c->unit_w ? 1 : 0, absmax_set(c, c->absmax_cur), absmax_set(c, c->absmax_cur ^ 1),
+                       EVT_TWO_CHAN(c->loss, c->K) ? 1 : 0, (c->unit_w && c->NA <= EVT_MAX_NA) ? 1 : 0, (c->unit_w && c->NA > EVT_MAX_NA) ? 1 : 0, absmax_set(c, c->absmax_cur), absmax_set(c, c->absmax_cur ^ 1),
                        c->qbits, c->qexp, qmul, c->qscale, c->NAg, c->loss, c->unit_w ? 1 : 0);
     HIPCHK(hipGetLastError());
     c->absmax_cur ^= 1; // the next gradient pass raises the set this kernel cleared

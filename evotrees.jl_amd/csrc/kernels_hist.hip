@@ -41,7 +41,8 @@ struct HistArgs {
     int slots_per_tile;
     int min_rows;
     int seg_cost;
-    int a0; // first global channel of this launch (channels beyond EVT_HIST_GROUP take further launches)
+    int na_all; // accumulator channels of the loss: more than EVT_MAX_NA go EVT_HIST_GROUP to a block layer (blockIdx.z)
+    int pack;   // the channel groups' first channel carries the row count (as a 64-bit word, k_quantize)
     // level bookkeeping that rides along with the first launch of a level: the partition kernels' chunk descriptors
     const int32_t *act_node;
     const int64_t *cprefix;
@@ -75,13 +76,23 @@ __device__ __forceinline__ int first_node_of_span(const int64_t *__restrict__ bp
 // Chunk descriptors of the level (evt_fill_chunk_descriptors): they ride along with the first launch of a level, spread
 // over the wavefronts of its first block column; the work hides behind the histogram kernel's own set-up.
 __device__ __forceinline__ void fill_chunk_descriptors(const HistArgs &A) {
-    if (blockIdx.y != 0 || A.a0 != 0) return;
+    if (blockIdx.y != 0 || blockIdx.z != 0) return;
     const int wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
     evt_fill_chunk_descriptors(A.hdr, A.act_node, A.cprefix, A.seg_start, A.seg_len, A.cdesc, (int)blockIdx.x * nwaves + wave,
                                (int)gridDim.x * nwaves);
 }
 
-template <int NA, bool PACK>
+// Channel c of a block layer's group, for one row.  GRP: the layer's channels start at a0; past the last one it reads that again
+// (added to words the flush leaves out).
+template <bool PACK, bool GRP>
+__device__ __forceinline__ unsigned long long load_channel(const HistArgs &A, int a0, int c, uint32_t id) {
+    if constexpr (GRP) return A.gq[(size_t)(a0 + c < A.na_all ? a0 + c : A.na_all - 1) * A.N + id];
+    else return evt_load_gq<PACK>(A.gq, A.N, c, id);
+}
+
+// GRP: more channels than one block's LDS takes (multi-class, several targets).  A layer of blocks takes NA of them, all layers in one
+// launch: a level of 60k rows is 60 blocks per group, which fill a quarter of the chip one after the other.
+template <int NA, bool PACK, bool GRP>
 __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
     extern __shared__ unsigned long long H[]; // [NA][tile slots][B]
     const int tid = threadIdx.x, nthr = blockDim.x;
@@ -90,7 +101,9 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
     const int64_t total = A.hdr[LH_TOTAL_BUILD];
     fill_chunk_descriptors(A);
     if (n_build <= 0 || total <= 0) return;
-    if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0 && A.a0 == 0) A.stats[A.level] = total - (int64_t)n_build * A.seg_cost;
+    const int a0 = GRP ? (int)blockIdx.z * NA : 0;
+    const bool pk = GRP ? (A.pack && a0 == 0) : PACK; // channel 0 shares its word with the row count
+    if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && tid == 0) A.stats[A.level] = total - (int64_t)n_build * A.seg_cost;
 
     const int step = nwaves * A.RPW; // rows per block iteration
     // rows per block: an even share, but never so few that the flush of a whole LDS histogram
@@ -142,7 +155,7 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
             continue;
         }
         // the packed row counter holds 16 bits: a longer run of one node is flushed in several parts
-        const int64_t nend = (PACK && nend_all - start > EVT_HIST_MAX_ROWS_PER_BLOCK) ? start + EVT_HIST_MAX_ROWS_PER_BLOCK : nend_all;
+        const int64_t nend = (pk && nend_all - start > EVT_HIST_MAX_ROWS_PER_BLOCK) ? start + EVT_HIST_MAX_ROWS_PER_BLOCK : nend_all;
         const int64_t seg = A.bstart[i] - nbeg; // position in the row list = seg + p
         // software pipeline over U row groups per wave: the row ids of iteration k+2 and the records of
         // iteration k+1 are in flight while the LDS atomics of iteration k are issued
@@ -165,7 +178,7 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
                 if (rc[u] != INV) {
                     vc[u] = *reinterpret_cast<const uint4 *>(A.xrm + (size_t)rc[u] * A.RS + sub * 16);
 #pragma unroll
-                    for (int a = 0; a < NA; a++) gc[u][a] = evt_load_gq<PACK>(A.gq, A.N, a, rc[u]);
+                    for (int a = 0; a < NA; a++) gc[u][a] = load_channel<PACK, GRP>(A, a0, a, rc[u]);
                 }
             }
 #pragma unroll
@@ -180,7 +193,7 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
                     if (rn[u] != INV) {
                         vn[u] = *reinterpret_cast<const uint4 *>(A.xrm + (size_t)rn[u] * A.RS + sub * 16);
 #pragma unroll
-                        for (int a = 0; a < NA; a++) gn[u][a] = evt_load_gq<PACK>(A.gq, A.N, a, rn[u]);
+                        for (int a = 0; a < NA; a++) gn[u][a] = load_channel<PACK, GRP>(A, a0, a, rn[u]);
                     }
                 }
                 uint32_t rnn[U];
@@ -217,7 +230,7 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
         // flush this node's partial histogram: hist[node][slot][ag][bin].  A node whose rows all lie in
         // this block's span has a single writer: plain stores into its zero-initialised slice; a node
         // shared with other blocks is accumulated with 64-bit global atomics.
-        const bool sole = (nbeg >= blk_start) && (nrows_end <= blk_end) && !(PACK && nrows_end - nbeg > EVT_HIST_MAX_ROWS_PER_BLOCK);
+        const bool sole = (nbeg >= blk_start) && (nrows_end <= blk_end) && !(pk && nrows_end - nbeg > EVT_HIST_MAX_ROWS_PER_BLOCK);
         long long *hn = A.hist + (int64_t)(A.bnode[i] - 1) * A.node_stride;
         // blocks start at different words so that concurrent flushes of one node do not queue on the
         // same addresses
@@ -230,11 +243,12 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
             if (w != 0ull) {
                 H[idx] = 0ull;
                 const int a = idx / plane;
+                if (GRP && a0 + a >= A.na_all) continue;
                 const int rem = idx - a * plane;
                 const int s = rem / A.B;
                 const int bin = rem - s * A.B;
                 unsigned long long *base = reinterpret_cast<unsigned long long *>(hn) + ((int64_t)(slot0 + s) * A.NAg) * A.B + bin;
-                if (PACK && a == 0) {
+                if (pk && a == 0) {
                     const long long gsum = (long long)w >> EVT_PACK_CNT_BITS;
                     const unsigned long long cnt = w & ((1ull << EVT_PACK_CNT_BITS) - 1ull);
                     if (sole) {
@@ -245,9 +259,9 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
                         atomicAdd(base + (int64_t)(A.NAg - 1) * A.B, cnt);
                     }
                 } else if (sole) {
-                    base[(int64_t)(A.a0 + a) * A.B] = w;
+                    base[(int64_t)(a0 + a) * A.B] = w;
                 } else {
-                    atomicAdd(base + (int64_t)(A.a0 + a) * A.B, w);
+                    atomicAdd(base + (int64_t)(a0 + a) * A.B, w);
                 }
             }
         }
@@ -312,7 +326,7 @@ __device__ __forceinline__ uint32_t load_id(const uint32_t *p) {
     return NT ? __builtin_nontemporal_load(p) : *p;
 }
 
-template <int NA, bool PACK, int U, bool FULL, int PB, int PU, bool NT>
+template <int NA, bool PACK, bool GRP, int U, bool FULL, int PB, int PU, bool NT>
 __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
     extern __shared__ unsigned long long H[]; // [NA][PU][B][NS]
     const int tid = threadIdx.x, nthr = blockDim.x;
@@ -321,7 +335,9 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
     const int64_t total = A.hdr[LH_TOTAL_BUILD];
     fill_chunk_descriptors(A);
     if (n_build <= 0 || total <= 0) return;
-    if (blockIdx.x == 0 && tid == 0 && A.a0 == 0) A.stats[A.level] = total - (int64_t)n_build * A.seg_cost;
+    const int a0 = GRP ? (int)blockIdx.z * NA : 0;
+    const bool pk = GRP ? (A.pack && a0 == 0) : PACK; // channel 0 shares its word with the row count
+    if (blockIdx.x == 0 && blockIdx.z == 0 && tid == 0) A.stats[A.level] = total - (int64_t)n_build * A.seg_cost;
 
     static_assert(PB == 8 || PB == 4 || PB == 2, "a piece is 8, 4 or 2 bytes");
     static_assert(PU >= 1 && PU <= PB, "features per piece");
@@ -396,7 +412,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
             continue;
         }
         // the packed row counter holds 16 bits: a longer run of one node is flushed in several parts
-        const int64_t nend = (PACK && nend_all - start > EVT_HIST_MAX_ROWS_PER_BLOCK) ? start + EVT_HIST_MAX_ROWS_PER_BLOCK : nend_all;
+        const int64_t nend = (pk && nend_all - start > EVT_HIST_MAX_ROWS_PER_BLOCK) ? start + EVT_HIST_MAX_ROWS_PER_BLOCK : nend_all;
         const int64_t seg = bst - nbeg;
         // A wave takes SR = U * RPW consecutive positions of the run per iteration (U row groups of RPW rows).
         // Row ids and gradient words are fetched one position per lane (one load instruction per SR rows instead of
@@ -429,7 +445,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
                 idc = load_id<NT>(isp + ((fetcher && p < nend) ? p : lastp));
             }
 #pragma unroll
-            for (int a = 0; a < NA; a++) gc[a] = evt_load_gq<PACK>(A.gq, A.N, a, idc);
+            for (int a = 0; a < NA; a++) gc[a] = load_channel<PACK, GRP>(A, a0, a, idc);
             {
                 const int64_t p = pw + itstride + mypos;
                 idn = load_id<NT>(isp + ((fetcher && p < nend) ? p : lastp));
@@ -450,7 +466,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
                 const int rem = rem64 > 0x7fffffff ? 0x7fffffff : (int)rem64;
                 // next iteration's gradient words and the row ids of the one after: ahead of the records in issue order
 #pragma unroll
-                for (int a = 0; a < NA; a++) gn[a] = evt_load_gq<PACK>(A.gq, A.N, a, idn);
+                for (int a = 0; a < NA; a++) gn[a] = load_channel<PACK, GRP>(A, a0, a, idn);
                 uint32_t idnn;
                 {
                     const int64_t p = pw + 2 * itstride + mypos;
@@ -495,7 +511,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
         // flush: a wave covers 8 consecutive bins of 8 pieces `sub` (or of all NS pieces and 8 / NS bin chunks) of one
         // (channel, t): global accesses are whole 64-byte runs of one feature's bins, LDS reads spread over the bank
         // pairs.  Blocks start at different items so that concurrent flushes of one node do not queue on the same addresses.
-        const bool sole = (nbeg >= blk_start) && (nrows_end <= blk_end) && !(PACK && nrows_end - nbeg > EVT_HIST_MAX_ROWS_PER_BLOCK);
+        const bool sole = (nbeg >= blk_start) && (nrows_end <= blk_end) && !(pk && nrows_end - nbeg > EVT_HIST_MAX_ROWS_PER_BLOCK);
         long long *hn = A.hist + (int64_t)(A.bnode[i] - 1) * A.node_stride;
         const int nchunks = (B + 7) >> 3;
         const int nitems = NA * PU * nchunks * NS * 8; // (channel, t, bin chunk, piece, bin in chunk), the last fastest
@@ -550,9 +566,9 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
                 if (w == 0ull) continue;
                 *hwv[j] = 0ull;
                 const int slot = slotv[j], a = av[j], b = bv[j];
-                if (slot == 0xFFFF) continue;
+                if (slot == 0xFFFF || (GRP && a0 + a >= A.na_all)) continue;
                 unsigned long long *base = reinterpret_cast<unsigned long long *>(hn) + ((int64_t)slot * A.NAg) * B + b;
-                if (PACK && a == 0) {
+                if (pk && a == 0) {
                     const long long gsum = (long long)w >> EVT_PACK_CNT_BITS;
                     const unsigned long long cnt = w & ((1ull << EVT_PACK_CNT_BITS) - 1ull);
                     if (sole) {
@@ -563,9 +579,9 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
                         atomicAdd(base + (int64_t)(A.NAg - 1) * B, cnt);
                     }
                 } else if (sole) {
-                    base[(int64_t)(A.a0 + a) * B] = w;
+                    base[(int64_t)(a0 + a) * B] = w;
                 } else {
-                    atomicAdd(base + (int64_t)(A.a0 + a) * B, w);
+                    atomicAdd(base + (int64_t)(a0 + a) * B, w);
                 }
             }
         }
@@ -579,7 +595,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
     }
 }
 
-template <int NA, bool PACK, int U, int PB, int PU, bool NT>
+template <int NA, bool PACK, bool GRP, int U, int PB, int PU, bool NT>
 static int launch_hist16_q(evt_ctx *c, const HistArgs &A, dim3 grid, int threads, size_t lds) {
     // unpredicated atomics for every feature of the record pay off unless most features are left out: the words of
     // features outside the sample are simply not flushed
@@ -587,21 +603,21 @@ static int launch_hist16_q(evt_ctx *c, const HistArgs &A, dim3 grid, int threads
     if (lds > 64 * 1024) { // one block per CU may take most of its 160 KB
         static EvtDevOnce once;
         if (once.pending(c->device)) {
-            HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_hist_build16<NA, PACK, U, true, PB, PU, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-            HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_hist_build16<NA, PACK, U, false, PB, PU, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_hist_build16<NA, PACK, GRP, U, true, PB, PU, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_hist_build16<NA, PACK, GRP, U, false, PB, PU, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
             once.mark(c->device);
         }
     }
     // c->launch_e0 / launch_e1 (when profiling): the kernel's own dispatch records them
     if (full)
-        hipExtLaunchKernelGGL((k_hist_build16<NA, PACK, U, true, PB, PU, NT>), grid, dim3(threads), (uint32_t)lds, c->stream, c->launch_e0, c->launch_e1, 0, A);
+        hipExtLaunchKernelGGL((k_hist_build16<NA, PACK, GRP, U, true, PB, PU, NT>), grid, dim3(threads), (uint32_t)lds, c->stream, c->launch_e0, c->launch_e1, 0, A);
     else
-        hipExtLaunchKernelGGL((k_hist_build16<NA, PACK, U, false, PB, PU, NT>), grid, dim3(threads), (uint32_t)lds, c->stream, c->launch_e0, c->launch_e1, 0, A);
+        hipExtLaunchKernelGGL((k_hist_build16<NA, PACK, GRP, U, false, PB, PU, NT>), grid, dim3(threads), (uint32_t)lds, c->stream, c->launch_e0, c->launch_e1, 0, A);
     HIPCHK(hipGetLastError());
     return EVT_OK;
 }
 
-template <int NA, bool PACK>
+template <int NA, bool PACK, bool GRP>
 static int launch_hist16_t(evt_ctx *c, const HistArgs &A, dim3 grid, int threads, size_t lds) {
     // row groups (records) in flight per wave: as many as a DPP row can address, fewer when registers run out
     constexpr int U = (NA <= 2) ? 16 : 8;
@@ -612,21 +628,21 @@ static int launch_hist16_t(evt_ctx *c, const HistArgs &A, dim3 grid, int threads
     const int pu = c->PU < c->PBL ? c->PU : pb;
 #define H16Q(PB_, PU_)                                                                                                     \
     if (pb == PB_ && pu == PU_)                                                                                            \
-        return nt ? launch_hist16_q<NA, PACK, U, PB_, PU_, true>(c, A, grid, threads, lds) : launch_hist16_q<NA, PACK, U, PB_, PU_, false>(c, A, grid, threads, lds);
+        return nt ? launch_hist16_q<NA, PACK, GRP, U, PB_, PU_, true>(c, A, grid, threads, lds) : launch_hist16_q<NA, PACK, GRP, U, PB_, PU_, false>(c, A, grid, threads, lds);
     H16Q(8, 8) H16Q(8, 7) H16Q(8, 6) H16Q(8, 5) H16Q(4, 4) H16Q(4, 3) H16Q(2, 2)
 #undef H16Q
     evt_set_error("no histogram kernel for pieces of %d bytes holding %d features", pb, pu);
     return EVT_ERR_INTERNAL;
 }
 
-template <int NA, bool PACK>
+template <int NA, bool PACK, bool GRP>
 static int launch_hist_t(evt_ctx *c, const HistArgs &A, dim3 grid, int threads, size_t lds) {
     static EvtDevOnce once;
     if (lds > 64 * 1024 && once.pending(c->device)) {
-        HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_hist_build<NA, PACK>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_hist_build<NA, PACK, GRP>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         once.mark(c->device);
     }
-    hipExtLaunchKernelGGL((k_hist_build<NA, PACK>), grid, dim3(threads), (uint32_t)lds, c->stream, c->launch_e0, c->launch_e1, 0, A);
+    hipExtLaunchKernelGGL((k_hist_build<NA, PACK, GRP>), grid, dim3(threads), (uint32_t)lds, c->stream, c->launch_e0, c->launch_e1, 0, A);
     HIPCHK(hipGetLastError());
     return EVT_OK;
 }
@@ -664,85 +680,60 @@ int launch_hist_build(evt_ctx *c, int level, const uint32_t *is_cur) {
     A.seg_cost = c->hist_seg_cost;
     const int threads = c->hist_threads;
     const int64_t blocks = c->hist_blocks;
-    // accumulator channels are taken EVT_HIST_GROUP at a time (one launch each; the one- and two-output losses need
-    // a single launch); the packed row counter rides on channel 0, i.e. in the first group only
-    // timing events: one launch carries them itself; several launches (channel groups) are bracketed by event records
-    const bool one_launch = c->NA <= EVT_MAX_NA;
-    hipEvent_t ev0 = c->launch_e0, ev1 = c->launch_e1;
-    if (!one_launch) {
-        c->launch_e0 = c->launch_e1 = nullptr;
-        if (ev0) (void)hipEventRecord(ev0, c->stream);
+    // more accumulator channels than one launch's blocks take go EVT_HIST_GROUP to a layer of blocks (blockIdx.z)
+    const bool grouped = c->NA > EVT_MAX_NA;
+    const int na = grouped ? EVT_HIST_GROUP : c->NA;
+    const unsigned layers = grouped ? (unsigned)((c->NA + na - 1) / na) : 1u;
+    A.gq = c->gq;
+    A.na_all = c->NA;
+    A.pack = c->unit_w ? 1 : 0;
+    // feature tiling so that one block's LDS histogram stays within budget
+    const size_t budget = 64 * 1024;
+    const size_t per_slot = (size_t)na * c->B * 8;
+    int slots_per_tile = (int)(budget / per_slot);
+    if (slots_per_tile < 1) slots_per_tile = 1;
+    if (slots_per_tile > nfs) slots_per_tile = nfs;
+    const int ntiles = (nfs + slots_per_tile - 1) / slots_per_tile;
+    slots_per_tile = (nfs + ntiles - 1) / ntiles;
+    A.slots_per_tile = slots_per_tile;
+    const size_t lds = per_slot * slots_per_tile;
+    dim3 grid((unsigned)blocks, (unsigned)ntiles, layers);
+    // conflict-free variant: a block column takes a tile of TW bytes of every record - the whole record when its LDS
+    // histogram fits, else the widest power of two that does (down to 32 bytes) - with 16, 32 or 64 lanes per row;
+    // lanes past the record's last piece idle.  (16-byte records as 1-byte pieces were measured: no faster than the
+    // generic kernel.)
+    int tw = 32;
+    while (tw < c->RS && tw < 512) tw <<= 1;
+    const bool spread = c->PU < c->PBL; // features spread over all pieces: one tile takes the whole record (record_layout)
+    while (!spread && tw > 32 && (size_t)na * c->B * tw * 8 > 128 * 1024) tw >>= 1;
+    const int pb16 = tw >= 128 ? 8 : (tw == 64 ? 4 : 2);
+    A.TW = tw;
+    A.NSL = tw / pb16;
+    const int ntiles16 = (c->RS + tw - 1) / tw;
+    const size_t lds16 = (size_t)na * c->B * A.NSL * (spread ? c->PU : pb16) * 8; // channels x bins x feature bytes of a tile, words
+    const bool can16 = c->RS >= 32 && lds16 <= 128 * 1024 && (!spread || (pb16 == c->PBL && ntiles16 == 1));
+    const bool use16 = (c->hist_variant == 1) ? false : can16;
+    if (!use16 && c->LPR > 64) { // the generic kernel reads a record with one wavefront instruction: 64 lanes of 16 bytes
+        evt_set_error("%d accumulator channels x %d bins need the generic histogram kernel, which takes at most 1024 features", na, c->B);
+        return EVT_ERR_ARG;
     }
-    for (int a0 = 0; a0 < c->NA; a0 += (c->NA <= EVT_MAX_NA ? EVT_MAX_NA : EVT_HIST_GROUP)) {
-        const int na = (c->NA <= EVT_MAX_NA) ? c->NA : (c->NA - a0 < EVT_HIST_GROUP ? c->NA - a0 : EVT_HIST_GROUP);
-        A.a0 = a0;
-        A.gq = c->gq + (size_t)a0 * c->N;
-        const bool pack = c->unit_w && a0 == 0;
-        // feature tiling so that one block's LDS histogram stays within budget
-        const size_t budget = 64 * 1024;
-        const size_t per_slot = (size_t)na * c->B * 8;
-        int slots_per_tile = (int)(budget / per_slot);
-        if (slots_per_tile < 1) slots_per_tile = 1;
-        if (slots_per_tile > nfs) slots_per_tile = nfs;
-        const int ntiles = (nfs + slots_per_tile - 1) / slots_per_tile;
-        slots_per_tile = (nfs + ntiles - 1) / ntiles;
-        A.slots_per_tile = slots_per_tile;
-        const size_t lds = per_slot * slots_per_tile;
-        dim3 grid((unsigned)blocks, (unsigned)ntiles);
-        // conflict-free variant: a block column takes a tile of TW bytes of every record - the whole record when its LDS
-        // histogram fits, else the widest power of two that does (down to 32 bytes) - with 16, 32 or 64 lanes per row;
-        // lanes past the record's last piece idle.  (16-byte records as 1-byte pieces were measured: no faster than the
-        // generic kernel.)
-        int tw = 32;
-        while (tw < c->RS && tw < 512) tw <<= 1;
-        const bool spread = c->PU < c->PBL; // features spread over all pieces: one tile takes the whole record (record_layout)
-        while (!spread && tw > 32 && (size_t)na * c->B * tw * 8 > 128 * 1024) tw >>= 1;
-        const int pb16 = tw >= 128 ? 8 : (tw == 64 ? 4 : 2);
-        A.TW = tw;
-        A.NSL = tw / pb16;
-        const int ntiles16 = (c->RS + tw - 1) / tw;
-        const size_t lds16 = (size_t)na * c->B * A.NSL * (spread ? c->PU : pb16) * 8; // channels x bins x feature bytes of a tile, words
-        const bool can16 = c->RS >= 32 && lds16 <= 128 * 1024 && (!spread || (pb16 == c->PBL && ntiles16 == 1));
-        const bool use16 = (c->hist_variant == 1) ? false : can16;
-        if (!use16 && c->LPR > 64) { // the generic kernel reads a record with one wavefront instruction: 64 lanes of 16 bytes
-            evt_set_error("%d accumulator channels x %d bins need the generic histogram kernel, which takes at most 1024 features", na, c->B);
-            return EVT_ERR_ARG;
-        }
-        int r = EVT_ERR_ARG;
-        if (use16) {
-            // several block columns share the launch's blocks: the same number of LDS histograms is flushed per node
-            int64_t bx = blocks / ntiles16;
-            if (bx < 64) bx = blocks < 64 ? blocks : 64;
-            dim3 grid16((unsigned)bx, (unsigned)ntiles16);
-#define H16CASE(NA_) \
-    case NA_: r = pack ? launch_hist16_t<NA_, true>(c, A, grid16, threads, lds16) : launch_hist16_t<NA_, false>(c, A, grid16, threads, lds16); break;
-            switch (na) {
-                H16CASE(1)
-                H16CASE(2)
-                H16CASE(3)
-                H16CASE(4)
-                H16CASE(5)
-            }
-#undef H16CASE
-        } else {
-#define HCASE(NA_) \
-    case NA_: r = pack ? launch_hist_t<NA_, true>(c, A, grid, threads, lds) : launch_hist_t<NA_, false>(c, A, grid, threads, lds); break;
-            switch (na) {
-                HCASE(1)
-                HCASE(2)
-                HCASE(3)
-                HCASE(4)
-                HCASE(5)
-            }
+    // several block columns share the launch's blocks: the same number of LDS histograms is flushed per node
+    int64_t bx = blocks / ntiles16;
+    if (bx < 64) bx = blocks < 64 ? blocks : 64;
+    const dim3 grid16((unsigned)bx, (unsigned)ntiles16, layers);
+#define HCASE(NA_, PACK_, GRP_) \
+    return use16 ? launch_hist16_t<NA_, PACK_, GRP_>(c, A, grid16, threads, lds16) : launch_hist_t<NA_, PACK_, GRP_>(c, A, grid, threads, lds)
+    if (grouped) HCASE(EVT_HIST_GROUP, false, true);
+    // the channels of the one- and two-output losses, with unit weights (first channel packed) and with weights of their own
+    if (c->unit_w && na == 1) HCASE(1, true, false);
+    if (c->unit_w && na == 2) HCASE(2, true, false);
+    if (c->unit_w && na == 4) HCASE(4, true, false);
+    if (!c->unit_w && na == 2) HCASE(2, false, false);
+    if (!c->unit_w && na == 3) HCASE(3, false, false);
+    if (!c->unit_w && na == 5) HCASE(5, false, false);
 #undef HCASE
-        }
-        if (r != EVT_OK) {
-            if (r == EVT_ERR_ARG) evt_set_error("unsupported channel count %d", na);
-            return r;
-        }
-    }
-    if (!one_launch && ev1) (void)hipEventRecord(ev1, c->stream);
-    return EVT_OK;
+    evt_set_error("unsupported channel count %d", na);
+    return EVT_ERR_ARG;
 }
 
 // Reference-layout export for parity checks: out[k, bin, feat, node] Float64 (src/init.jl:204).
