@@ -405,7 +405,8 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     if (tree_type == EVT_TREE_OBLIVIOUS) ALLOC(c->ogains, (size_t)c->maxlvl * c->F * c->B);
     {
         uint8_t *sb = nullptr;
-        ALLOC(sb, (size_t)c->maxlvl * ((c->F + 3) / 4) * 64); // one 64-byte candidate (ScanBestQ, kernels_scan.hip) per node and group of 4 features
+        // one 64-byte candidate (ScanBestQ, kernels_scan.hip) per node and group of 4 features; oblivious: one of 16 bytes per block
+        ALLOC(sb, std::max((size_t)c->maxlvl * ((c->F + 3) / 4) * 64, (size_t)EVT_OBLIV_BLOCKS * 16));
         c->sbest = sb;
     }
     // pinned staging: tree read-back + small per-tree uploads

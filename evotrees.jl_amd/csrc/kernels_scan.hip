@@ -9,6 +9,7 @@
 // reference's "first maximum wins" (strict '>' at src/fit-utils.jl:447).
 #include "evt_internal.h"
 #include <float.h>
+#include <algorithm>
 
 #define NO_BIN 0x7fffffff
 
@@ -671,32 +672,39 @@ struct OblivArgs {
     const int32_t *act_node;
     double eta, lambda, L2, gamma;
     int bagging, nfs, B, K, NK, NAg, loss, level, zero_children;
+    ScanBest *best; // first maximum (gain, cell) of each block of k_obliv_max
+    int nbest;
 };
 
-__global__ __launch_bounds__(1024) void k_obliv_select(OblivArgs A) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
+// The level matrix and its first maximum: a block takes a share of the (feature position, bin) cells, a thread a cell at a time; the
+// nodes' gains are added in node order, eight requested ahead of their use.  One block of the whole level took 5 to 20 us per
+// level for this (50 features x 64 bins, up to 32 nodes), waiting for one load after the other.
+__global__ __launch_bounds__(256) void k_obliv_max(OblivArgs A) {
+    const int tid = threadIdx.x;
     const int n_act = (int)A.hdr[LH_N_ACT];
     if (n_act <= 0) return;
-    const int B = A.B, K = A.K, NK = A.NK, NAG = A.NAg;
     const int first = 1 << (A.level - 1);
-    __shared__ double s_g[1024];
-    __shared__ int s_i[1024];
-    __shared__ int s_dec[3];
-    __shared__ double s_gain;
-    __shared__ double s_sc[EVT_MC_MAX_NK];
-    if (tid < NAG) s_sc[tid] = A.qscale[tid];
-    // level matrix and its first maximum
+    const int cells = A.nfs * A.B;
+    __shared__ double s_g[256];
+    __shared__ int s_i[256];
     double bg = -INFINITY;
     int bi = NO_BIN;
-    const int cells = A.nfs * B;
-    for (int c = tid; c < cells; c += blockDim.x) {
+    for (int c = (int)blockIdx.x * 256 + tid; c < cells; c += (int)gridDim.x * 256) {
         double acc = 0.0;
         bool allpos = true;
-        for (int i = 0; i < n_act; i++) {
-            const int n = A.act_node[i];
-            const double g = A.ogains[(int64_t)(n - first) * cells + c];
-            acc += g;
-            if (n > 1) allpos = allpos && (g > 0.0);
+        for (int i0 = 0; i0 < n_act; i0 += 8) {
+            double g[8];
+            int n[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) n[j] = A.act_node[i0 + j < n_act ? i0 + j : n_act - 1];
+#pragma unroll
+            for (int j = 0; j < 8; j++) g[j] = A.ogains[(int64_t)(n[j] - first) * cells + c];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                if (i0 + j >= n_act) continue;
+                acc += g[j];
+                if (n[j] > 1) allpos = allpos && (g[j] > 0.0);
+            }
         }
         const double v = allpos ? acc : 0.0;
         if (v > bg) { bg = v; bi = c; } // c ascending per thread: first maximum kept
@@ -704,68 +712,96 @@ __global__ __launch_bounds__(1024) void k_obliv_select(OblivArgs A) {
     s_g[tid] = bg;
     s_i[tid] = bi;
     __syncthreads();
-    for (int o = blockDim.x >> 1; o > 0; o >>= 1) {
-        if (tid < o) {
-            if (s_g[tid + o] > s_g[tid] || (s_g[tid + o] == s_g[tid] && s_i[tid + o] < s_i[tid])) {
-                s_g[tid] = s_g[tid + o];
-                s_i[tid] = s_i[tid + o];
-            }
+    for (int o = 128; o > 0; o >>= 1) {
+        if (tid < o && (s_g[tid + o] > s_g[tid] || (s_g[tid + o] == s_g[tid] && s_i[tid + o] < s_i[tid]))) {
+            s_g[tid] = s_g[tid + o];
+            s_i[tid] = s_i[tid + o];
         }
         __syncthreads();
     }
     if (tid == 0) {
-        const int found = (s_i[0] != NO_BIN && s_g[0] > A.gamma) ? 1 : 0;
-        s_dec[0] = found;
-        s_dec[1] = found ? s_i[0] / B : 0;
-        s_dec[2] = found ? (s_i[0] % B) + 1 : 0;
-        s_gain = s_g[0];
+        A.best[blockIdx.x].gain = s_g[0];
+        A.best[blockIdx.x].jp = s_i[0];
     }
-    __syncthreads();
-    const int found = s_dec[0], bj = s_dec[1], bb = s_dec[2];
-    const double bgain = s_gain;
-    for (int i = wave; i < n_act; i += nwaves) {
-        const int n = A.act_node[i];
-        long long Sq[EVT_MC_MAX_NK];
-        double S[EVT_MC_MAX_NK];
-        for (int ag = 0; ag < NAG; ag++) Sq[ag] = A.node_sum[(int64_t)n * NAG + ag];
-        decode_vals(Sq, s_sc, A.loss, NK, S);
-        if (lane == 0) A.tree.w[n - 1] = (float)S[NK - 1];
-        if (!found) {
-            if (lane < K) A.tree.pred[(int64_t)K * (n - 1) + lane] = (float)leaf_value(A.loss, S, lane, K, A.eta, A.bagging, A.lambda, A.L2);
-            if (lane == 0) A.status[n] = ST_LEAF;
-            continue;
-        }
-        const int feat = (int)A.js[bj];
-        const bool numeric = A.feattypes[feat - 1] != 0;
-        const long long *hn = A.hist + (int64_t)(n - 1) * A.node_stride;
-        for (int ag = 0; ag < NAG; ag++) {
-            const int64_t o = ((int64_t)bj * NAG + ag) * B;
-            long long s = 0;
-            for (int b = lane; b < B; b += 64) {
-                const bool in = numeric ? (b + 1 <= bb) : (b + 1 == bb);
-                if (in) s += hn[o + b];
-            }
-            s = wave_sum_i64(s);
-            if (lane == 0) {
-                A.node_sum[(int64_t)(2 * n) * NAG + ag] = s;
-                A.node_sum[(int64_t)(2 * n + 1) * NAG + ag] = Sq[ag] - s;
-            }
-        }
-        if (lane == 0) {
-            A.tree.feat[n - 1] = feat;
-            A.tree.cond_bin[n - 1] = (uint8_t)bb;
-            A.tree.gain[n - 1] = (float)bgain;
-            A.tree.split[n - 1] = 1;
-            A.tree.packed[n - 1] = evt_pack_node(feat, bb, A.feattypes[feat - 1] != 0);
-            A.status[n] = ST_SPLIT;
-        }
-        if (!A.zero_children) continue;
+}
+
+// One node per block column (nodes of the level that are not active return): its first block takes the maximum of k_obliv_max's
+// blocks and writes the node's part of the level's decision, the others clear the children's histogram slices (whatever the
+// decision: the slices of a leaf are never read).
+__global__ __launch_bounds__(256) void k_obliv_apply(OblivArgs A) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = 4;
+    const int B = A.B, K = A.K, NK = A.NK, NAG = A.NAg;
+    const int n_act = (int)A.hdr[LH_N_ACT];
+    if ((int)blockIdx.x >= n_act) return;
+    const int n = A.act_node[blockIdx.x];
+    if (blockIdx.y > 0) {
         long long *hc = A.hist + (int64_t)(2 * n - 1) * A.node_stride;
         const int64_t used = (int64_t)A.nfs * NAG * B;
-        for (int64_t t = lane; t < used; t += 64) {
-            hc[t] = 0;
-            hc[A.node_stride + t] = 0;
+        const int64_t zb = gridDim.y - 1, per = (used + zb - 1) / zb;
+        const int64_t i0 = (int64_t)(blockIdx.y - 1) * per, i1 = i0 + per < used ? i0 + per : used;
+        for (int64_t i = i0 + tid; i < i1; i += 256) {
+            hc[i] = 0;
+            hc[A.node_stride + i] = 0;
         }
+        return;
+    }
+    __shared__ double s_g[256];
+    __shared__ int s_i[256];
+    __shared__ double s_sc[EVT_MC_MAX_NK], s_S[EVT_MC_MAX_NK];
+    __shared__ long long s_Sq[EVT_MC_MAX_NK];
+    double bg = -INFINITY;
+    int bi = NO_BIN;
+    for (int k = tid; k < A.nbest; k += 256) { // blocks' cells interleave: ties go to the lowest cell
+        const ScanBest r = A.best[k];
+        if (r.gain > bg || (r.gain == bg && r.jp < bi)) { bg = r.gain; bi = r.jp; }
+    }
+    s_g[tid] = bg;
+    s_i[tid] = bi;
+    if (tid < NAG) {
+        s_sc[tid] = A.qscale[tid];
+        s_Sq[tid] = A.node_sum[(int64_t)n * NAG + tid];
+    }
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if (tid < o && (s_g[tid + o] > s_g[tid] || (s_g[tid + o] == s_g[tid] && s_i[tid + o] < s_i[tid]))) {
+            s_g[tid] = s_g[tid + o];
+            s_i[tid] = s_i[tid + o];
+        }
+        __syncthreads();
+    }
+    if (tid == 0) decode_vals(s_Sq, s_sc, A.loss, NK, s_S);
+    __syncthreads();
+    const bool found = s_i[0] != NO_BIN && s_g[0] > A.gamma;
+    if (tid == 0) A.tree.w[n - 1] = (float)s_S[NK - 1];
+    if (!found) {
+        if (tid < K) A.tree.pred[(int64_t)K * (n - 1) + tid] = (float)leaf_value(A.loss, s_S, tid, K, A.eta, A.bagging, A.lambda, A.L2);
+        if (tid == 0) A.status[n] = ST_LEAF;
+        return;
+    }
+    const int bj = s_i[0] / B, bb = s_i[0] % B + 1;
+    const int feat = (int)A.js[bj];
+    const bool numeric = A.feattypes[feat - 1] != 0;
+    const long long *hn = A.hist + (int64_t)(n - 1) * A.node_stride;
+    for (int ag = wave; ag < NAG; ag += nwaves) {
+        const int64_t o = ((int64_t)bj * NAG + ag) * B;
+        long long s = 0;
+        for (int b = lane; b < B; b += 64) {
+            const bool in = numeric ? (b + 1 <= bb) : (b + 1 == bb);
+            if (in) s += hn[o + b];
+        }
+        s = wave_sum_i64(s);
+        if (lane == 0) {
+            A.node_sum[(int64_t)(2 * n) * NAG + ag] = s;
+            A.node_sum[(int64_t)(2 * n + 1) * NAG + ag] = s_Sq[ag] - s;
+        }
+    }
+    if (tid == 0) {
+        A.tree.feat[n - 1] = feat;
+        A.tree.cond_bin[n - 1] = (uint8_t)bb;
+        A.tree.gain[n - 1] = (float)s_g[0];
+        A.tree.split[n - 1] = 1;
+        A.tree.packed[n - 1] = evt_pack_node(feat, bb, numeric);
+        A.status[n] = ST_SPLIT;
     }
 }
 
@@ -796,33 +832,38 @@ __device__ __forceinline__ void node_totals_mc(const ScanArgs &A, int n, const l
     __syncthreads();
 }
 
-// left-side sums of one channel for this lane's BPL bins (numeric: inclusive prefix; categorical: the bin alone);
-// subtract nodes materialise h[n] = h[parent] - h[sibling] on the way
+// one channel's histogram words for this lane's BPL bins, requested (fetch) well before they are summed (left_sums): a node's own, or
+// its parent's and its sibling's
 template <int BPL>
-__device__ __forceinline__ void left_sums(const ScanArgs &A, long long *hn, const long long *hp, const long long *hs, int64_t o, bool is_sub,
-                                          bool numeric, int lane, long long *left) {
-    long long val[BPL];
-    long long run = 0;
+struct ChannelWords {
+    long long a[BPL], b[BPL];
+    __device__ __forceinline__ void fetch(const ScanArgs &A, const long long *hn, const long long *hp, const long long *hs, int64_t o, bool is_sub, int lane) {
 #pragma unroll
-    for (int t = 0; t < BPL; t++) {
-        const int b = lane * BPL + t;
-        long long v = 0;
-        if (b < A.B) {
-            if (is_sub) {
-                v = hp[o + b] - hs[o + b];
-                hn[o + b] = v;
-            } else {
-                v = hn[o + b];
-            }
+        for (int t = 0; t < BPL; t++) {
+            const int bin = lane * BPL + t < A.B ? lane * BPL + t : A.B - 1;
+            a[t] = is_sub ? hp[o + bin] : hn[o + bin];
+            b[t] = is_sub ? hs[o + bin] : 0;
         }
-        val[t] = v;
-        run += v;
-        left[t] = run;
     }
-    const long long excl = wave_incl_scan_i64(run) - run;
+    // left-side sums (numeric: inclusive prefix; categorical: the bin alone); subtract nodes materialise
+    // h[n] = h[parent] - h[sibling] on the way
+    __device__ __forceinline__ void left_sums(const ScanArgs &A, long long *hn, int64_t o, bool is_sub, bool numeric, int lane, long long *left) const {
+        long long val[BPL];
+        long long run = 0;
 #pragma unroll
-    for (int t = 0; t < BPL; t++) left[t] = numeric ? left[t] + excl : val[t];
-}
+        for (int t = 0; t < BPL; t++) {
+            const int bin = lane * BPL + t;
+            const long long v = bin < A.B ? a[t] - b[t] : 0;
+            if (is_sub && bin < A.B) hn[o + bin] = v;
+            val[t] = v;
+            run += v;
+            left[t] = run;
+        }
+        const long long excl = wave_incl_scan_i64(run) - run;
+#pragma unroll
+        for (int t = 0; t < BPL; t++) left[t] = numeric ? left[t] + excl : val[t];
+    }
+};
 
 template <int BPL>
 __global__ __launch_bounds__(256) void k_scan_mc(ScanArgs A) {
@@ -858,7 +899,16 @@ __global__ __launch_bounds__(256) void k_scan_mc(ScanArgs A) {
         long long lq[BPL];
         double w_l[BPL], w_r[BPL], sg[BPL];
         bool ok[BPL];
-        left_sums<BPL>(A, hn, hp, hs, ((int64_t)jp * NAG + (NAG - 1)) * B, is_sub, numeric, lane, lq);
+        const int64_t of = (int64_t)jp * NAG * B; // the feature's slice; the outputs' channel pairs are fetched two ahead
+        ChannelWords<BPL> cw, cg[2], ch[2];
+        cw.fetch(A, hn, hp, hs, of + (int64_t)(NAG - 1) * B, is_sub, lane);
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int k = j < K ? j : K - 1;
+            cg[j].fetch(A, hn, hp, hs, of + (int64_t)k * B, is_sub, lane);
+            ch[j].fetch(A, hn, hp, hs, of + (int64_t)(K + k) * B, is_sub, lane);
+        }
+        cw.left_sums(A, hn, of + (int64_t)(NAG - 1) * B, is_sub, numeric, lane, lq);
 #pragma unroll
         for (int t = 0; t < BPL; t++) {
             const int b = lane * BPL + t;
@@ -867,10 +917,17 @@ __global__ __launch_bounds__(256) void k_scan_mc(ScanArgs A) {
             ok[t] = (b < B) && (b + 1 <= bmax) && (w_l[t] > A.min_weight) && (w_r[t] > A.min_weight);
             sg[t] = 0.0;
         }
-        for (int k = 0; k < K; k++) {
+        for (int k0 = 0; k0 < K; k0 += 2)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int k = k0 + j;
+            if (k >= K) break;
             long long gq[BPL], hq[BPL];
-            left_sums<BPL>(A, hn, hp, hs, ((int64_t)jp * NAG + k) * B, is_sub, numeric, lane, gq);
-            left_sums<BPL>(A, hn, hp, hs, ((int64_t)jp * NAG + K + k) * B, is_sub, numeric, lane, hq);
+            cg[j].left_sums(A, hn, of + (int64_t)k * B, is_sub, numeric, lane, gq);
+            ch[j].left_sums(A, hn, of + (int64_t)(K + k) * B, is_sub, numeric, lane, hq);
+            const int kn = k + 2 < K ? k + 2 : K - 1;
+            cg[j].fetch(A, hn, hp, hs, of + (int64_t)kn * B, is_sub, lane);
+            ch[j].fetch(A, hn, hp, hs, of + (int64_t)(K + kn) * B, is_sub, lane);
             const double Sg = s_S[k], Sh = s_S[K + k];
 #pragma unroll
             for (int t = 0; t < BPL; t++) {
@@ -916,13 +973,25 @@ __global__ __launch_bounds__(256) void k_scan_mc(ScanArgs A) {
 __global__ __launch_bounds__(256) void k_scan_fin_mc(ScanArgs A, int ngroups) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = (1 << (A.level - 1)) + blockIdx.x;
+    const int B = A.B, NK = A.NK, K = A.K, NAG = A.NAg;
+    if (blockIdx.y > 0) { // the blocks beyond a node's first only clear the children's slices, whatever the decision (as in k_scan_fin)
+        if (A.status[n] == ST_INACTIVE) return;
+        long long *hc = A.hist + (int64_t)(2 * n - 1) * A.node_stride;
+        const int64_t used = (int64_t)A.nfs * NAG * B;
+        const int64_t zb = gridDim.y - 1, per = (used + zb - 1) / zb;
+        const int64_t i0 = (int64_t)(blockIdx.y - 1) * per, i1 = i0 + per < used ? i0 + per : used;
+        for (int64_t i = i0 + tid; i < i1; i += 256) {
+            hc[i] = 0;
+            hc[A.node_stride + i] = 0;
+        }
+        return;
+    }
     if (A.leaf_level) {
         if (n > 1 && A.status[n >> 1] != ST_SPLIT) return;
     } else {
         const int st = A.status[n];
         if (st != ST_BUILD && st != ST_SUBTRACT) return;
     }
-    const int B = A.B, NK = A.NK, K = A.K, NAG = A.NAg;
     long long *hn = A.hist + (int64_t)(n - 1) * A.node_stride;
     __shared__ long long s_Sq[EVT_MC_MAX_NK];
     __shared__ double s_S[EVT_MC_MAX_NK];
@@ -994,14 +1063,11 @@ __global__ __launch_bounds__(256) void k_scan_fin_mc(ScanArgs A, int ngroups) {
             }
         }
     }
-    if (!A.zero_children) return;
-    long long *hc = A.hist + (int64_t)(2 * n - 1) * A.node_stride;
-    const int64_t used = (int64_t)A.nfs * NAG * B;
-    for (int64_t i = tid; i < used; i += blockDim.x) {
-        hc[i] = 0;
-        hc[A.node_stride + i] = 0;
-    }
 }
+
+// Blocks per node that clear the children's histogram slices beside the block that decides: about 512 in all, so that neither a level
+// of one node nor one of wide slices (16 channels x 100 features: 1.6 MB per node) leaves them to few blocks.
+static unsigned zero_blocks_per_node(unsigned nodes) { return nodes >= 512 ? 1u : (512u / nodes < 64u ? 512u / nodes : 64u); }
 
 // The pass over the last split level also writes its children's leaf values (binary trees with the fixed channel layouts).
 bool scan_folds_leaves(const evt_ctx *c) { return !c->mc && c->tree_type != EVT_TREE_OBLIVIOUS && c->D > 1; }
@@ -1050,7 +1116,8 @@ int launch_scan(evt_ctx *c, int level, const evt_params *p, bool leaf_level) {
             else if (bpl == 2) hipLaunchKernelGGL((k_scan_mc<2>), grid, dim3(256), 0, c->stream, A);
             else hipLaunchKernelGGL((k_scan_mc<4>), grid, dim3(256), 0, c->stream, A);
         }
-        if (!A.oblivious || leaf_level) hipLaunchKernelGGL(k_scan_fin_mc, dim3(nodes), dim3(256), 0, c->stream, A, ngroups);
+        if (!A.oblivious || leaf_level)
+            hipLaunchKernelGGL(k_scan_fin_mc, dim3(nodes, !leaf_level && A.zero_children ? 1 + zero_blocks_per_node(nodes) : 1), dim3(256), 0, c->stream, A, ngroups);
         HIPCHK(hipGetLastError());
         return EVT_OK;
     }
@@ -1100,7 +1167,11 @@ int launch_obliv_select(evt_ctx *c, int level, const evt_params *p) {
     A.bagging = p->bagging_size;
     A.nfs = c->n_js_last; A.B = c->B; A.K = c->K; A.NK = c->NK; A.NAg = c->NAg; A.loss = c->loss; A.level = level;
     A.zero_children = (level + 1 < c->D) ? 1 : 0;
-    hipLaunchKernelGGL(k_obliv_select, dim3(1), dim3(1024), 0, c->stream, A);
+    A.best = reinterpret_cast<ScanBest *>(c->sbest);
+    A.nbest = (int)std::min<int64_t>(EVT_OBLIV_BLOCKS, ((int64_t)A.nfs * A.B + 255) / 256);
+    hipLaunchKernelGGL(k_obliv_max, dim3((unsigned)A.nbest), dim3(256), 0, c->stream, A);
+    const unsigned nodes = 1u << (level - 1);
+    hipLaunchKernelGGL(k_obliv_apply, dim3(nodes, A.zero_children ? 1 + zero_blocks_per_node(nodes) : 1), dim3(256), 0, c->stream, A);
     HIPCHK(hipGetLastError());
     return EVT_OK;
 }
