@@ -625,8 +625,9 @@ def fit(config, dtrain=None, x_train=None, y_train=None, w_train=None, offset_tr
             import warnings
             warnings.warn("To track eval metric in logger, both `x_eval` and `y_eval` must be provided.")
         for i in range(1, config.nrounds + 1):
-            # without an eval set nothing is read between two rounds: the device may start the next one early
-            grow_evotree(m, cache, config, more=(logger is None and i < config.nrounds))
+            # the device may start the next round early: between two rounds only the eval handle is read.  With early stopping
+            # that tree may turn out one too many; it is dropped with the handle, unless the caller keeps the handle
+            grow_evotree(m, cache, config, more=(i < config.nrounds and (logger is None or not return_cache)))
             if logger is not None:
                 cb(logger, i, m.trees[-1])  # as the reference: only the round's last tree reaches the eval prediction
                 if i % print_every_n == 0 and verbosity > 0:
