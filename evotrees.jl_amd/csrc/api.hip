@@ -191,6 +191,7 @@ extern "C" int evt_destroy(evt_handle c) {
     void *ptrs[] = {c->xcm, c->xrm, c->y, c->pred, c->grad, c->gq, c->is_a, c->is_b, c->nidx, c->mask, c->flagw, c->chunk_nleft, c->chunk_lpre,
                     c->hist, c->seg_start, c->seg_len, c->status, c->node_sum, c->tree_blob, c->tree.packed, c->js, c->jsmap, c->feattypes, c->mono, c->absmax, c->qexp_buf[0], c->qexp_buf[1], c->qbits,
                     c->qscale_buf[0], c->qscale_buf[1], c->planes, c->metric_partial, c->errflag, c->ogains, c->sbest, c->is_id, c->pt_nodes, c->pt_pred, c->mask_next,
+                    c->small_nid[0], c->small_nid[1], c->small_head[0], c->small_head[1], c->small_left[0], c->small_left[1],
                     c->alphas, c->alphas_f, c->qkeys_a, c->qkeys_b, c->qtemp};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -295,6 +296,12 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->hist_variant = 0;
     c->scan_fused = 1;
     c->hist_in_scatter = 1;
+    c->small_tree = 1;
+    for (int k = 0; k < 2; k++) {
+        c->small_nid[k] = nullptr;
+        c->small_head[k] = nullptr;
+        c->small_left[k] = nullptr;
+    }
     c->hist_seg_cost = 2048;
     c->record_nidx = false;
     c->nidx_valid = false;
@@ -428,6 +435,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     {
         std::vector<uint8_t> ft(c->F, 1);
         c->h_feattypes = ft;
+        c->h_mono.assign(c->F, 0);
         hipError_t e2 = hipMemcpy(c->feattypes, ft.data(), c->F, hipMemcpyHostToDevice);
         if (e2 == hipSuccess) e2 = hipMemset(c->mono, 0, sizeof(int32_t) * c->F);
         if (e2 == hipSuccess) e2 = hipMemset(c->absmax, 0, sizeof(uint32_t) * 2 * EVT_ABSMAX_STRIPES * EVT_MC_MAX_NK);
@@ -825,6 +833,7 @@ extern "C" int evt_set_feature_meta(evt_handle c, const uint8_t *feattypes, cons
     HIPCHK(hipMemcpy(c->feattypes, ft.data(), c->F, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(c->mono, mo.data(), sizeof(int32_t) * c->F, hipMemcpyHostToDevice));
     c->h_feattypes = ft;
+    c->h_mono = mo;
     return EVT_OK;
     });
 }
@@ -982,7 +991,8 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
     const bool fuse_pred = p->update_pred && all_rows && !defer;
     c->write_nidx = rec_nidx || defer;
 
-    int r = ensure_planes(c);
+    const bool small = !staged && small_tree_applies(c, n_js, all_rows);
+    int r = small ? EVT_OK : ensure_planes(c);
     if (r != EVT_OK) return r;
     if (EVT_IS_QUANTILE(c->loss)) {
         r = quantile_leaf_buffers(c);
@@ -1006,15 +1016,17 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
             HIPCHK(hipMemcpyAsync(c->mask, mask, c->N, hipMemcpyDefault, c->stream));
             HIPCHK(hipStreamSynchronize(c->stream)); // the caller may reuse its mask buffer as soon as this call returns
         }
-        r = launch_compact_mask(c, cond, draw, c->mask_seed);
+        if (!small) r = launch_compact_mask(c, cond, draw, c->mask_seed);
         if (r == EVT_OK && rec_nidx) r = launch_fill_u32(c, c->nidx, 0u, c->N);
     }
-    if (r == EVT_OK && all_rows) r = launch_tree_begin(c); // with a row sample the compaction above has set the tree up
+    if (r == EVT_OK && all_rows && !small) r = launch_tree_begin(c); // with a row sample the compaction above has set the tree up
     prof_end(c);
     if (r != EVT_OK) return r;
 
     c->step.all_rows = all_rows;
-    c->step.defer = defer;
+    c->step.defer = defer || (small && p->update_pred); // there rows outside the sample have a leaf too
+    c->step.small = small;
+    c->step.small_draw = draw;
     c->step.fuse_pred = fuse_pred;
     c->step.hist_fused = !staged && scatter_can_build_hist(c, c->n_js_last);
     c->step.blob_sent = false;
@@ -1111,7 +1123,7 @@ static int tree_close(evt_ctx *c) {
         prof_end(c);
         if (r != EVT_OK) return r;
     }
-    if (p->update_pred && !all_rows) {
+    if (p->update_pred && !all_rows && !c->step.small) {
         // rows outside the sample are predicted too (src/fit.jl:37): walk the new tree for all rows
         prof_begin(c, EVT_K_PREDICT, 0);
         r = launch_predict_tree_cache(c, true); // with the tree's transfer to the host in its last blocks
@@ -1121,7 +1133,7 @@ static int tree_close(evt_ctx *c) {
     }
     if (defer) {
         c->pend_pred = true;
-        c->nidx_valid = true;
+        c->nidx_valid = all_rows; // with a row sample the recorded leaves are those of all rows
     }
 
     // the tree (and the per-level row counts) comes back in one pinned transfer, queued behind the kernels
@@ -1152,6 +1164,10 @@ static int tree_fail(evt_ctx *c, int r) { // a failed stage leaves no tree open
 
 // every stage of an opened tree, then the close: what evt_grow_tree_begin queues
 static int tree_run_stages(evt_ctx *c, int r) {
+    if (r == EVT_OK && c->step.small) {
+        r = launch_small_tree(c, &c->step.p, c->step.small_draw);
+        c->step.phase = 4;
+    }
     while (r == EVT_OK && c->step.phase != 4) {
         r = tree_stage_hist(c);
         if (r == EVT_OK) r = tree_stage_scan(c);
@@ -1471,6 +1487,10 @@ extern "C" int evt_get_nidx(evt_handle c, uint32_t *out) {
         if (r != EVT_OK) return r;
     }
     if (!c->nidx_valid) { // not recorded while growing: walk the last tree (same decisions, row by row)
+        {
+            int r = launch_apply_pending(c); // the recorded leaves of all rows are about to be overwritten
+            if (r != EVT_OK) return r;
+        }
         int r = launch_nidx_from_tree(c, !c->last_all_rows, c->last_cond);
         if (r != EVT_OK) return r;
         c->nidx_valid = true;
@@ -1833,6 +1853,9 @@ extern "C" int evt_set_option(evt_handle c, const char *name, int64_t value) {
         if (!c->grads_ahead) c->grads_ready = false;
     } else if (strcmp(name, "record_nidx") == 0) {
         c->record_nidx = value != 0;
+    } else if (strcmp(name, "small_tree") == 0) {
+        ARGCHK(value >= 0 && value <= 2, "small_tree must be 0 (never), 1 (inputs of few rows) or 2 (wherever it can)");
+        c->small_tree = (int)value;
     } else if (strcmp(name, "scan_fused") == 0) {
         c->scan_fused = value != 0;
     } else if (strcmp(name, "hist_in_scatter") == 0) {

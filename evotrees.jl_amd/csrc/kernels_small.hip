@@ -1,0 +1,766 @@
+// Trees of small inputs (tens of thousands of rows): one kernel per level instead of a histogram, a search and a two-pass partition.
+//
+// At these sizes a level is a chain of short dependent kernels - 20 launches of 3 to 9 us for a tree of depth 6 on 2000 rows, whatever they
+// do.  Here a block owns one sampled feature and walks ALL rows: it takes the decisions of the level above (every block the same
+// ones, from the candidates all blocks left), moves every row's node id on, adds the rows into its feature's histograms in LDS - one
+// per active node, built outright: adding all rows costs less than subtracting siblings would save - searches them, and leaves its
+// best candidate per node.  The blocks meet only at the kernel boundary.  Rows keep their place: a node id per row stands for the row lists,
+// so rows outside the sample walk along (flagged) and the prediction needs no pass of its own over the tree.
+// The sums are the same integers and the gains the same expressions as in the kernels of larger inputs: same trees, bit for bit.
+#include "split_math.h"
+#include <algorithm>
+
+#define SMALL_OUT 0x80000000u // the row is not in the sample
+#define SMALL_MAX_NODES 256   // nodes of the deepest level that splits
+
+struct SmallHead { // a block's candidate for a node
+    double gain;
+    int bin;  // NO_BIN: none
+    int feat; // 1-based, negative when categorical
+    long long left[EVT_MAX_NA + 1]; // totals left of it; more channels go to SmallArgs::left_out
+};
+static_assert(sizeof(SmallHead) == 64, "one candidate per 64-byte line");
+
+struct SmallArgs {
+    const uint8_t *xcm;
+    const unsigned long long *gq;
+    uint8_t *mask;
+    const uint32_t *nid_in; // the rows' node ids as the level above left them
+    uint32_t *nid_out;
+    const SmallHead *head_in; // [node of the level above][block]
+    SmallHead *head_out;
+    const long long *left_in; // [node][block][NAg]: totals left of the candidate
+    long long *left_out;
+    long long *hist;
+    int64_t node_stride;
+    uint32_t *js;
+    const uint32_t *js_src; // the column sample where it is new (pinned host memory), or js
+    uint32_t *map_dst;
+    const uint32_t *map_src;
+    int map_words;
+    int32_t *status;
+    long long *node_sum;
+    const double *qscale;
+    TreeDev tree;
+    int64_t *stats;
+    const uint4 *blob_src; // final kernel: the tree's arrays and their pinned destination
+    uint4 *blob_dst;
+    int64_t blob_n;
+    uint32_t *nidx;
+    double eta, lambda, L2, gamma, min_weight;
+    unsigned long long seed;
+    int N, F, B, K, NK, NAg, NA, loss, level, D, nnodes, nfs, bagging;
+    int slots;     // histograms the block's LDS holds
+    int oblivious, sampled, draw, cond;
+    int wide;      // channel 0 staged as a 64-bit packed word (more channels than EVT_MAX_NA)
+    // the blocks' features, in the launch's arguments: a block need not wait for them.  0-based id | numeric << 16 | (constraint + 1) << 17
+    uint32_t feat[256];
+};
+#define SMALL_NUMERIC (1u << 16)
+
+__device__ __forceinline__ long long shfl_i64(long long v, int src) {
+    const int lo = __shfl((int)(v & 0xffffffffll), src), hi = __shfl((int)(v >> 32), src);
+    return ((long long)hi << 32) | (unsigned int)lo;
+}
+__device__ __forceinline__ double shfl_f64(double v, int src) { return __longlong_as_double(shfl_i64(__double_as_longlong(v), src)); }
+
+// lane i's statistic i (of 2K+1) from lane-held channel sums (decode_vals, a statistic per lane)
+__device__ __forceinline__ double lane_stat(const SmallArgs &A, long long q, int lane) {
+    const bool two = EVT_TWO_CHAN(A.loss, A.K);
+    const int src = two ? (lane == 0 ? 0 : 1) : (lane < A.NAg ? lane : 0);
+    double v = (double)shfl_i64(q, src) * A.qscale[src];
+    if (two && lane == 1) v = (A.loss == EVT_LOSS_MSE) ? 2.0 * v : 0.0;
+    return v;
+}
+// a node's weight and, for a leaf, its values (leaf_value, an output per lane)
+__device__ __forceinline__ void write_node(const SmallArgs &A, int n, long long q, int lane, bool leaf) {
+    const double S = lane_stat(A, q, lane);
+    double v[3] = {shfl_f64(S, lane < A.K ? lane : 0), shfl_f64(S, A.K + (lane < A.K ? lane : 0)), shfl_f64(S, 2 * A.K)};
+    if (lane == 0) A.tree.w[n - 1] = (float)v[2];
+    if (leaf && lane < A.K) A.tree.pred[(int64_t)A.K * (n - 1) + lane] = (float)leaf_value(A.loss, v, 0, 1, A.eta, A.bagging, A.lambda, A.L2);
+}
+
+// The decision for node p of the level above `A.level`, by one wavefront: the best of the blocks' candidates (highest gain, then
+// earliest feature; its bin is already the lowest).  Leaves the packed split in s_dec[p] (0: none) and the children's totals in
+// s_tot; the writer block also writes the Tree arrays and the children's state.
+__device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t *s_dec, long long *s_tot, bool writer, int lane) {
+    const int n = (1 << (A.level - 2)) + p, nag = A.NAg, nwg = A.nfs;
+    const int st = A.status[n];
+    const long long qn = lane < nag ? A.node_sum[(int64_t)n * nag + lane] : 0;
+    // every lane reads whole candidates (one line each), so that the winner's feature and totals are at hand
+    const SmallHead *hp = A.head_in + (int64_t)p * nwg;
+    union Words {
+        SmallHead h;
+        uint4 v[4];
+    } mine;
+    mine.h.gain = -INFINITY;
+    mine.h.bin = NO_BIN;
+    mine.h.feat = 0;
+    int bj = NO_BIN;
+    for (int w = lane; w < ((nwg + 63) & ~63); w += 64) {
+        Words c;
+        const uint4 *cp = reinterpret_cast<const uint4 *>(hp + (w < nwg ? w : nwg - 1));
+#pragma unroll
+        for (int k = 0; k < 4; k++) c.v[k] = cp[k];
+        if (w < nwg && c.h.gain > mine.h.gain) {
+            mine = c;
+            bj = w;
+        }
+    }
+    double bg = mine.h.gain;
+    int wj = bj;
+    wave_argmax(bg, wj);
+    // the writer block may have set the state to SPLIT or LEAF by now: anything but INACTIVE means the level reached the node
+    const bool active = st != ST_INACTIVE;
+    const bool found = active && wj != NO_BIN && bg > A.gamma;
+    uint32_t packed = 0;
+    long long ql = 0;
+    int feat = 0, bin = 0;
+    if (found) {
+        const int owner = wj & 63;
+        bin = __shfl(mine.h.bin, owner);
+        feat = __shfl(mine.h.feat, owner);
+        const bool numeric = feat > 0;
+        feat = numeric ? feat : -feat;
+        packed = evt_pack_node(feat, bin, numeric);
+        if (nag <= EVT_MAX_NA) {
+#pragma unroll
+            for (int ag = 0; ag < EVT_MAX_NA; ag++) {
+                const long long v = shfl_i64(mine.h.left[ag], owner);
+                ql = lane == ag ? v : ql;
+            }
+        } else {
+            ql = lane < nag ? A.left_in[((int64_t)p * nwg + wj) * nag + lane] : 0;
+        }
+    }
+    if (lane == 0) s_dec[p] = packed;
+    if (lane < nag) {
+        s_tot[(2 * p) * nag + lane] = ql;
+        s_tot[(2 * p + 1) * nag + lane] = qn - ql;
+    }
+    if (!writer || !active) return;
+    write_node(A, n, qn, lane, !found);
+    if (lane == 0) {
+        A.status[n] = found ? ST_SPLIT : ST_LEAF;
+        if (found) {
+            A.tree.feat[n - 1] = feat;
+            A.tree.cond_bin[n - 1] = (uint8_t)bin;
+            A.tree.gain[n - 1] = (float)bg;
+            A.tree.split[n - 1] = 1;
+            A.tree.packed[n - 1] = packed;
+        }
+    }
+    if (!found) return;
+    for (int child = 0; child < 2; child++) {
+        const int cn = 2 * n + child;
+        const long long qc = child ? qn - ql : ql;
+        if (lane < nag) A.node_sum[(int64_t)cn * nag + lane] = qc;
+        if (lane == 0) A.status[cn] = A.level < A.D ? ST_BUILD : ST_LEAF;
+        if (A.level == A.D) write_node(A, cn, qc, lane, true);
+    }
+}
+
+// where a row of the level above goes: the decision its node took (0: none, a leaf further up stays), the bin byte that decides, the
+// node it moves to
+__device__ __forceinline__ uint32_t row_decision(const SmallArgs &A, uint32_t nid, const uint32_t *s_dec) {
+    const int p = (int)(nid & ~SMALL_OUT) - (1 << (A.level - 2));
+    const uint32_t d = s_dec[p >= 0 ? p : 0];
+    return p >= 0 ? d : 0u;
+}
+__device__ __forceinline__ uint32_t decision_bin(const SmallArgs &A, uint32_t d, int row) {
+    const uint32_t f = d & 0xFFFFu;
+    return A.xcm[(size_t)(f ? f - 1 : 0) * A.N + row];
+}
+__device__ __forceinline__ uint32_t row_moves(uint32_t nid, uint32_t d, uint32_t xb) {
+    const uint32_t cb = (d >> 16) & 0xFFu;
+    const bool left = (d & EVT_NODE_NUMERIC) ? xb <= cb : xb == cb;
+    const uint32_t child = (nid & SMALL_OUT) | ((nid & ~SMALL_OUT) * 2 + (left ? 0u : 1u));
+    return (d & EVT_NODE_SPLIT) ? child : nid;
+}
+
+// 4 and 16 bytes from any 1-, or 4-byte aligned address
+__device__ __forceinline__ uint32_t load4(const uint8_t *p) {
+    uint32_t v;
+    __builtin_memcpy(&v, p, 4);
+    return v;
+}
+__device__ __forceinline__ uint4 load16(const uint32_t *p) {
+    uint4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+
+// a channel's value of one LDS histogram word: the first channel shares its word with the row count
+template <bool PACK>
+__device__ __forceinline__ long long channel_of(const unsigned long long *H, int B, int NAG, int ag, int b) {
+    if (!PACK) return (long long)H[ag * B + b];
+    if (ag == NAG - 1) return (long long)(H[b] & ((1ull << EVT_PACK_CNT_BITS) - 1ull));
+    const unsigned long long w = H[ag * B + b];
+    return ag == 0 ? (long long)w >> EVT_PACK_CNT_BITS : (long long)w;
+}
+
+// The search of one (node, feature) by one wavefront.  NAG: global channels (2, 3, 5), or 0 when their number is known at run time
+// only.  on_gain(b, ok, gain, left) is called for every bin of the lane; left: the totals left of it (NAG channels; NAG == 0: null).
+// Returns the node's totals in q (NAG != 0).
+template <int NAG, int BPL, bool PACK, typename GAIN>
+__device__ __forceinline__ void small_scan(const SmallArgs &A, const unsigned long long *H, const long long *tot, bool numeric, int constraint, int lane,
+                                           long long *hist_out, long long *q, GAIN on_gain) {
+    const int B = A.B, nag = NAG ? NAG : A.NAg;
+    const int bmax = numeric ? B - 1 : B;
+    if constexpr (NAG != 0) {
+        constexpr int K = NAG == 5 ? 2 : 1, NK = 2 * K + 1;
+        long long left[NAG][BPL];
+        double sc[NAG], S[NK];
+#pragma unroll
+        for (int ag = 0; ag < NAG; ag++) {
+            sc[ag] = A.qscale[ag];
+            long long val[BPL], run = 0;
+#pragma unroll
+            for (int t = 0; t < BPL; t++) {
+                const int b = lane * BPL + t;
+                val[t] = b < B ? channel_of<PACK>(H, B, NAG, ag, b) : 0;
+                if (b < B) hist_out[ag * B + b] = val[t];
+                run += val[t];
+                left[ag][t] = run;
+            }
+            const long long incl = wave_incl_scan_i64(run), excl = incl - run;
+            q[ag] = tot ? tot[ag] : shfl_i64(incl, 63); // the root's totals are the sums over any feature's bins
+#pragma unroll
+            for (int t = 0; t < BPL; t++) left[ag][t] = numeric ? left[ag][t] + excl : val[t];
+        }
+        decode_vals(q, sc, A.loss, NK, S);
+        double gain_p = 0.0;
+        for (int k = 0; k < K; k++) gain_p += node_gain_k(A.loss, S[k], S[K + k], S[2 * K], A.lambda, A.L2);
+        const double w_p = S[NK - 1];
+#pragma unroll
+        for (int t = 0; t < BPL; t++) {
+            const int b = lane * BPL + t;
+            long long ql[NAG];
+#pragma unroll
+            for (int ag = 0; ag < NAG; ag++) ql[ag] = left[ag][t];
+            double SL[NK];
+            decode_vals(ql, sc, A.loss, NK, SL);
+            const double w_l = SL[NK - 1], w_r = w_p - w_l;
+            bool ok = b < B && b + 1 <= bmax && w_l > A.min_weight && w_r > A.min_weight;
+            if (ok && constraint != 0) {
+                double SR[NK];
+                for (int k = 0; k < NK; k++) SR[k] = S[k] - SL[k];
+                const double predL = leaf_value(A.loss, SL, 0, K, A.eta, A.bagging, A.lambda, A.L2);
+                const double predR = leaf_value(A.loss, SR, 0, K, A.eta, A.bagging, A.lambda, A.L2);
+                ok = (constraint == -1 && predL > predR) || (constraint == 1 && predL < predR);
+            }
+            double gain = 0.0;
+            if (ok) {
+                double sg = 0.0;
+                for (int k = 0; k < K; k++) sg += split_gain_k(A.loss, S[k], S[K + k], w_p, SL[k], SL[K + k], w_l, w_r, A.lambda, A.L2);
+                gain = sg - gain_p;
+            }
+            on_gain(b, ok, gain, ql);
+        }
+    } else {
+        const int K = A.K;
+        auto lefts = [&](int ag, long long *left, long long &total) {
+            long long val[BPL], run = 0;
+#pragma unroll
+            for (int t = 0; t < BPL; t++) {
+                const int b = lane * BPL + t;
+                val[t] = b < B ? channel_of<PACK>(H, B, nag, ag, b) : 0;
+                if (b < B) hist_out[ag * B + b] = val[t];
+                run += val[t];
+                left[t] = run;
+            }
+            const long long incl = wave_incl_scan_i64(run), excl = incl - run;
+            total = tot ? tot[ag] : shfl_i64(incl, 63);
+#pragma unroll
+            for (int t = 0; t < BPL; t++) left[t] = numeric ? left[t] + excl : val[t];
+        };
+        long long lq[BPL], tq;
+        lefts(nag - 1, lq, tq);
+        const double w_p = (double)tq * A.qscale[nag - 1];
+        double w_l[BPL], w_r[BPL], sg[BPL], gain_p = 0.0;
+        bool ok[BPL];
+#pragma unroll
+        for (int t = 0; t < BPL; t++) {
+            const int b = lane * BPL + t;
+            w_l[t] = (double)lq[t] * A.qscale[nag - 1];
+            w_r[t] = w_p - w_l[t];
+            ok[t] = b < B && b + 1 <= bmax && w_l[t] > A.min_weight && w_r[t] > A.min_weight;
+            sg[t] = 0.0;
+        }
+        for (int k = 0; k < K; k++) {
+            long long gq[BPL], hq[BPL], tg, th;
+            lefts(k, gq, tg);
+            lefts(K + k, hq, th);
+            const double scg = A.qscale[k], sch = A.qscale[K + k];
+            const double Sg = (double)tg * scg, Sh = (double)th * sch;
+            gain_p += node_gain_k(A.loss, Sg, Sh, w_p, A.lambda, A.L2);
+#pragma unroll
+            for (int t = 0; t < BPL; t++)
+                sg[t] += split_gain_k(A.loss, Sg, Sh, w_p, (double)gq[t] * scg, (double)hq[t] * sch, w_l[t], w_r[t], A.lambda, A.L2);
+        }
+#pragma unroll
+        for (int t = 0; t < BPL; t++) on_gain(lane * BPL + t, ok[t], ok[t] ? sg[t] - gain_p : 0.0, static_cast<const long long *>(nullptr));
+    }
+}
+
+// totals left of bin lb (numeric: the bins up to it, categorical: it alone), a channel at a time
+template <bool PACK>
+__device__ __forceinline__ void small_left(const SmallArgs &A, const unsigned long long *Hs, int nag, bool numeric, int lb, int lane, SmallHead *out, long long *left) {
+    for (int ag = 0; ag < nag; ag++) {
+        long long t = 0;
+        for (int b = lane; b < lb && b < A.B; b += 64)
+            if (numeric || b + 1 == lb) t += channel_of<PACK>(Hs, A.B, nag, ag, b);
+        t = wave_sum_i64(t);
+        if (lane == 0) {
+            if (nag <= EVT_MAX_NA) out->left[ag] = t;
+            else left[ag] = t;
+        }
+    }
+}
+
+template <int NAG, int BPL, bool PACK>
+__global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
+    extern __shared__ unsigned long long s_dyn[];
+    __shared__ uint32_t s_dec[SMALL_MAX_NODES];
+    __shared__ uint16_t s_slot[SMALL_MAX_NODES];  // node of the level -> slot among the active ones (0xFFFF: not active)
+    __shared__ uint16_t s_node[SMALL_MAX_NODES];  // and back
+    __shared__ int s_nact, s_cnt, s_best;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int B = A.B, N = A.N, level = A.level;
+    const int nag = NAG ? NAG : A.NAg, na = NAG ? NAG - (PACK ? 1 : 0) : A.NA;
+    const bool writer = blockIdx.x == 0;
+    const int jp = blockIdx.x;
+    const int first = 1 << (level - 1), nlev = first;
+    long long *s_tot = reinterpret_cast<long long *>(s_dyn);                         // [nlev][nag]
+    double *s_gain = reinterpret_cast<double *>(s_tot + (level > 1 ? nlev * nag : 0)); // oblivious: [slots][B]
+    unsigned long long *H = reinterpret_cast<unsigned long long *>(s_gain + (A.oblivious ? A.slots * B : 0)); // [slots][na][B]
+    const uint32_t fw = A.feat[jp];
+    const int f = (int)(fw & 0xFFFFu), constraint = (int)(fw >> 17) - 1;
+    const bool numeric = (fw & SMALL_NUMERIC) != 0;
+    if (tid == 0) s_cnt = 0;
+    const uint8_t *col = A.xcm + (size_t)f * N;
+    // A thread takes U groups of 4 neighbouring rows at a time (the last group of all starts at N - 4 and leaves out what others
+    // have); what the first of them need is requested before the decisions.
+    constexpr int U = (NAG == 2 && PACK && BPL < 4) ? 2 : 1, GA = NAG ? NAG - (PACK ? 1 : 0) : 1;
+    const int ngroups = (N + 3) >> 2;
+    uint32_t nid[U][4], xb[U];
+    unsigned long long g[GA][U][4];
+    auto request = [&](int k0) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = k0 + u * 1024 < ngroups ? k0 + u * 1024 : ngroups - 1, r = 4 * k < N - 4 ? 4 * k : N - 4;
+            xb[u] = load4(col + r);
+            if (level > 1) {
+                const uint4 v = load16(A.nid_in + r);
+                nid[u][0] = v.x; nid[u][1] = v.y; nid[u][2] = v.z; nid[u][3] = v.w;
+            } else { // at the root: the rows' mask bytes
+                nid[u][0] = (A.sampled && !A.draw) ? load4(A.mask + r) : 0u;
+            }
+            if constexpr (NAG != 0) {
+#pragma unroll
+                for (int a = 0; a < GA; a++) {
+                    if (PACK && a == 0) {
+                        const uint4 v = load16(reinterpret_cast<const uint32_t *>(A.gq) + r);
+                        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                        for (int i = 0; i < 4; i++) g[a][u][i] = ((unsigned long long)(long long)(int32_t)w[i] << EVT_PACK_CNT_BITS) + 1ull;
+                    } else {
+                        const uint32_t *q = reinterpret_cast<const uint32_t *>(A.gq + (size_t)a * N + r);
+                        const uint4 v0 = load16(q), v1 = load16(q + 4);
+                        g[a][u][0] = ((unsigned long long)v0.y << 32) | v0.x;
+                        g[a][u][1] = ((unsigned long long)v0.w << 32) | v0.z;
+                        g[a][u][2] = ((unsigned long long)v1.y << 32) | v1.x;
+                        g[a][u][3] = ((unsigned long long)v1.w << 32) | v1.z;
+                    }
+                }
+            }
+        }
+    };
+    request(tid);
+    if (level > 1) {
+        const int np = nlev >> 1;
+        for (int p = wave; p < np; p += 16) small_decide(A, p, s_dec, s_tot, writer, lane);
+        __syncthreads();
+        if (wave == 0) { // the children of split nodes are the level's active nodes
+            int base = 0;
+            for (int p0 = 0; p0 < np; p0 += 64) {
+                const int p = p0 + lane;
+                const bool split = p < np && (s_dec[p] & EVT_NODE_SPLIT);
+                const unsigned long long m = __ballot(split);
+                const int at = base + 2 * __popcll(m & ((1ull << lane) - 1ull));
+                if (p < np) {
+                    s_slot[2 * p] = split ? (uint16_t)at : 0xFFFFu;
+                    s_slot[2 * p + 1] = split ? (uint16_t)(at + 1) : 0xFFFFu;
+                    if (split) {
+                        s_node[at] = (uint16_t)(2 * p);
+                        s_node[at + 1] = (uint16_t)(2 * p + 1);
+                    }
+                }
+                base += 2 * __popcll(m);
+            }
+            if (lane == 0) s_nact = base;
+        }
+    } else {
+        if (tid == 0) {
+            s_slot[0] = 0;
+            s_node[0] = 0;
+            s_nact = 1;
+        }
+        if (writer) { // a new tree
+            for (int n = tid; n < A.nnodes; n += 1024) {
+                A.tree.feat[n] = 0;
+                A.tree.cond_bin[n] = 0;
+                A.tree.w[n] = 0.0f;
+                A.tree.gain[n] = 0.0f;
+                A.tree.split[n] = 0;
+                A.tree.packed[n] = 0u;
+                for (int k = 0; k < A.K; k++) A.tree.pred[(int64_t)A.K * n + k] = 0.0f;
+            }
+            for (int n = tid; n < A.nnodes + 2; n += 1024) A.status[n] = n == 1 ? ST_BUILD : ST_INACTIVE;
+            for (int d = tid; d <= A.D; d += 1024) A.stats[d] = 0;
+            if (A.js_src != A.js)
+                for (int i = tid; i < A.nfs; i += 1024) A.js[i] = A.js_src[i];
+            for (int i = tid; i < A.map_words; i += 1024) A.map_dst[i] = A.map_src[i];
+        }
+    }
+    __syncthreads();
+    const int nact = s_nact;
+    int counted = 0;
+    auto take = [&](int k0, int base, int ns) { // the groups requested at k0, for the nodes in slots base .. base + ns
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int k = k0 + u * 1024, r = 4 * k < N - 4 ? 4 * k : N - 4;
+            if (k >= ngroups) continue;
+            if (level == 1) {
+                uint32_t mb = nid[u][0];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    uint32_t m = (mb >> (8 * i)) & 0xFFu;
+                    if (A.draw) {
+                        unsigned long long z = A.seed + (unsigned long long)(((r + i) >> 3) + 1) * 0x9E3779B97F4A7C15ull; // SplitMix64, as k_mask_count
+                        z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+                        z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+                        z ^= z >> 31;
+                        m = (uint32_t)(z >> (8 * ((r + i) & 7))) & 0xFFu;
+                        if (writer) A.mask[r + i] = (uint8_t)m;
+                    }
+                    nid[u][i] = (A.sampled && m > (uint32_t)A.cond) ? 1u | SMALL_OUT : 1u;
+                }
+            } else {
+                uint32_t d[4], b[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) d[i] = row_decision(A, nid[u][i], s_dec);
+#pragma unroll
+                for (int i = 0; i < 4; i++) b[i] = decision_bin(A, d[i], r + i);
+#pragma unroll
+                for (int i = 0; i < 4; i++) nid[u][i] = row_moves(nid[u][i], d[i], b[i]);
+            }
+            // every block has the same ids: each writes a share (a wavefront's 256 rows; rows of the last group twice, alike)
+            if (base == 0 && (k >> 6) % (int)gridDim.x == (int)blockIdx.x)
+#pragma unroll
+                for (int i = 0; i < 4; i++) A.nid_out[r + i] = nid[u][i];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int q = (int)(nid[u][i] & ~SMALL_OUT) - first;
+                if (r + i < 4 * k || (nid[u][i] & SMALL_OUT) || q < 0) continue;
+                const int slot = (int)s_slot[q] - base;
+                if (slot < 0 || slot >= ns) continue;
+                counted++;
+                unsigned long long *h = H + (size_t)slot * na * B + ((xb[u] >> (8 * i)) & 0xFFu) - 1;
+                if constexpr (NAG != 0) {
+#pragma unroll
+                    for (int a = 0; a < GA; a++) atomicAdd(h + a * B, g[a][u][i]);
+                } else {
+                    for (int a = 0; a < na; a++) {
+                        unsigned long long v;
+                        if (PACK && a == 0 && !A.wide) v = evt_load_gq<true>(A.gq, N, 0, (uint32_t)(r + i));
+                        else v = A.gq[(size_t)a * N + r + i];
+                        atomicAdd(h + a * B, v);
+                    }
+                }
+            }
+        }
+    };
+    int ns = nact < A.slots ? nact : A.slots;
+    for (int i = tid; i < ns * na * B; i += 1024) H[i] = 0ull;
+    __syncthreads();
+    take(tid, 0, ns);
+    for (int base = 0; base == 0 || base < nact; base += A.slots) {
+        if (base > 0) {
+            ns = nact - base < A.slots ? nact - base : A.slots;
+            for (int i = tid; i < ns * na * B; i += 1024) H[i] = 0ull;
+            __syncthreads();
+        }
+        for (int k0 = base > 0 ? tid : tid + 1024 * U; k0 < ngroups; k0 += 1024 * U) {
+            request(k0);
+            take(k0, base, ns);
+        }
+        __syncthreads();
+        for (int s = wave; s < ns; s += 16) {
+            const int q = s_node[base + s], n = first + q;
+            const unsigned long long *Hs = H + (size_t)s * na * B;
+            long long *hout = A.hist + (int64_t)(n - 1) * A.node_stride + (int64_t)jp * nag * B;
+            double lg = -INFINITY;
+            int lb = NO_BIN;
+            constexpr int QA = NAG ? NAG : 1;
+            long long tq[QA], lq[QA];
+#pragma unroll
+            for (int ag = 0; ag < QA; ag++) lq[ag] = 0;
+            small_scan<NAG, BPL, PACK>(A, Hs, level > 1 ? s_tot + q * nag : nullptr, numeric, constraint, lane, hout, tq,
+                                       [&](int b, bool ok, double gain, const long long *left) {
+                if (A.oblivious) {
+                    if (b < B) s_gain[s * B + b] = gain; // update_gains!
+                } else if (ok && gain > lg) {
+                    lg = gain;
+                    lb = b + 1;
+                    if constexpr (NAG != 0) {
+#pragma unroll
+                        for (int ag = 0; ag < QA; ag++) lq[ag] = left[ag];
+                    }
+                }
+            });
+            if (level == 1 && writer) { // the root's totals, for the kernels below
+                if constexpr (NAG != 0) {
+                    if (lane == 0)
+#pragma unroll
+                        for (int ag = 0; ag < QA; ag++) A.node_sum[(int64_t)n * nag + ag] = tq[ag];
+                } else {
+                    for (int ag = 0; ag < nag; ag++) {
+                        long long t = 0;
+                        for (int b = lane; b < B; b += 64) t += channel_of<PACK>(Hs, B, nag, ag, b);
+                        t = wave_sum_i64(t);
+                        if (lane == 0) A.node_sum[(int64_t)n * nag + ag] = t;
+                    }
+                }
+            }
+            if (A.oblivious) continue;
+            wave_argmax(lg, lb);
+            SmallHead *out = A.head_out + (int64_t)q * gridDim.x + jp;
+            if constexpr (NAG != 0) { // the lane that holds the winning bin has the totals left of it
+                if (lane == (lb != NO_BIN ? (lb - 1) / BPL : 0)) {
+                    SmallHead h;
+                    h.gain = lg;
+                    h.bin = lb;
+                    h.feat = numeric ? f + 1 : -(f + 1);
+#pragma unroll
+                    for (int ag = 0; ag < EVT_MAX_NA + 1; ag++) h.left[ag] = ag < QA ? lq[ag < QA ? ag : 0] : 0;
+                    *out = h;
+                }
+            } else {
+                if (lane == 0) {
+                    out->gain = lg;
+                    out->bin = lb;
+                    out->feat = numeric ? f + 1 : -(f + 1);
+                }
+                if (lb == NO_BIN) continue;
+                small_left<PACK>(A, Hs, nag, numeric, lb, lane, out, A.left_out + ((int64_t)q * gridDim.x + jp) * nag);
+            }
+        }
+        __syncthreads();
+    }
+    if (A.oblivious) { // all active nodes are in LDS: the feature's row of the level matrix, then its first maximum (grow_otree!, src/fit.jl:190-217)
+        if (wave == 0) {
+            double bg = -INFINITY;
+            int bb = NO_BIN;
+            for (int b = lane; b < B; b += 64) {
+                double acc = 0.0;
+                bool allpos = true;
+                for (int s = 0; s < nact; s++) {
+                    const double g = s_gain[s * B + b];
+                    acc += g;
+                    if (level > 1) allpos = allpos && g > 0.0;
+                }
+                const double v = allpos ? acc : 0.0;
+                if (v > bg) {
+                    bg = v;
+                    bb = b + 1;
+                }
+            }
+            wave_argmax(bg, bb);
+            if (lane == 0) s_best = bb;
+            for (int s = lane; s < nact; s += 64) {
+                SmallHead *out = A.head_out + (int64_t)s_node[s] * gridDim.x + jp;
+                out->gain = bg;
+                out->bin = bb;
+                out->feat = numeric ? f + 1 : -(f + 1);
+            }
+        }
+        __syncthreads();
+        const int lb = s_best;
+        for (int s = wave; s < nact; s += 16) {
+            const int64_t at = (int64_t)s_node[s] * gridDim.x + jp;
+            small_left<PACK>(A, H + (size_t)s * na * B, nag, numeric, lb, lane, A.head_out + at, A.left_out + at * nag);
+        }
+    }
+    if (writer) { // rows of the level: the root's is the size of the sample
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) counted += __shfl_xor(counted, o);
+        if (lane == 0) atomicAdd(&s_cnt, counted);
+        __syncthreads();
+        if (tid == 0) {
+            A.stats[level] = s_cnt;
+            if (level == 1) A.stats[0] = s_cnt;
+        }
+    }
+}
+
+// The last decisions, the leaves, and every row's leaf (added to the predictions by the next pass over the rows, as for larger
+// inputs).  The first block also sends the finished tree to the host's pinned buffer.
+__global__ __launch_bounds__(1024) void k_small_final(SmallArgs A) {
+    extern __shared__ unsigned long long s_dyn[];
+    __shared__ uint32_t s_dec[SMALL_MAX_NODES];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const bool writer = blockIdx.x == 0;
+    const int np = 1 << (A.level - 2);
+    long long *s_tot = reinterpret_cast<long long *>(s_dyn);
+    const int r = (int)blockIdx.x * 1024 + tid;
+    uint32_t nid = r < A.N ? A.nid_in[r] : 0u;
+    asm volatile("" : "+v"(nid));
+    for (int p = wave; p < np; p += 16) small_decide(A, p, s_dec, s_tot, writer, lane);
+    __syncthreads();
+    if (r < A.N) {
+        const uint32_t d = row_decision(A, nid, s_dec);
+        A.nidx[r] = row_moves(nid, d, decision_bin(A, d, r)) & ~SMALL_OUT;
+    }
+    if (writer)
+        for (int64_t i = tid; i < A.blob_n; i += 1024) A.blob_dst[i] = A.blob_src[i];
+}
+
+static size_t small_lds(const evt_ctx *c, int level, int slots) {
+    const size_t tot = level > 1 ? (size_t)(1 << (level - 1)) * c->NAg * 8 : 0;
+    const size_t gain = c->tree_type == EVT_TREE_OBLIVIOUS ? (size_t)slots * c->B * 8 : 0;
+    return tot + gain + (size_t)slots * c->NA * c->B * 8;
+}
+// histograms a block's LDS holds at the deepest level that splits
+static int small_slots(const evt_ctx *c) {
+    const int nodes = 1 << std::max(0, c->D - 2);
+    const size_t fixed = small_lds(c, c->D - 1, 0), one = small_lds(c, c->D - 1, 1) - fixed;
+    const size_t budget = 144 * 1024;
+    if (fixed > 32 * 1024) return 0;
+    return (int)std::min<size_t>((size_t)nodes, (budget - fixed) / one);
+}
+
+int small_tree_buffers(evt_ctx *c) {
+    if (c->small_nid[0]) return EVT_OK;
+    const size_t cand = (size_t)(1 << (c->D - 2)) * std::min(c->F, 256);
+    for (int k = 0; k < 2; k++) {
+        HIPCHK(hipMalloc((void **)&c->small_nid[k], sizeof(uint32_t) * (size_t)c->N));
+        HIPCHK(hipMalloc((void **)&c->small_head[k], sizeof(SmallHead) * cand));
+        if (c->NK > EVT_MAX_NA) HIPCHK(hipMalloc((void **)&c->small_left[k], sizeof(long long) * cand * c->NK));
+    }
+    return EVT_OK;
+}
+
+// Inputs that take this path.  A block walks all rows once per level (and once more for every `slots` nodes), so a level grows with the
+// rows, the channels and - through the candidates every block reads and the searches its 16 wavefronts share - the nodes, where the
+// other path spreads the rows over the chip and pays for its launches.  Estimates in microseconds, fitted to rounds of 1k to 65k rows,
+// 10 and 60 features, depths 5 to 9, 1 to 14 channels, that both paths grew: mse of depth 6 on 10 features 109 against 61 us per round at
+// 4k rows, 125 against 118 at 32k; 60 features 160 against 62 and 165 against 118; 7 classes of depth 5 182 against 143 at 4k, 201 against 255 at 16k.
+bool small_tree_applies(const evt_ctx *c, int nfs, bool all_rows) {
+    if (!c->small_tree || c->D < 2 || c->D > 10 || nfs > 256 || c->N < 4 || c->N > 65535 || !c->defer_pred || EVT_IS_QUANTILE(c->loss)) return false;
+    if (c->record_nidx && !all_rows) return false;
+    const bool obliv = c->tree_type == EVT_TREE_OBLIVIOUS;
+    const int nodes = 1 << (c->D - 2), slots = small_slots(c);
+    if (slots < 1 || (obliv && slots < nodes)) return false;
+    if (c->small_tree > 1) return true;
+    const double per_1k_rows = c->mc ? 0.3 + 0.2 * c->NA : 0.33 + 0.065 * c->NA;
+    double here = 0.0;
+    for (int l = 1; l < c->D; l++) {
+        const int n = (int)std::min<int64_t>(1 << (l - 1), c->N);
+        here += 5.0 + 3.5 * ((n + 15) / 16) + per_1k_rows * 1e-3 * c->N * ((n + slots - 1) / slots);
+    }
+    return here < (c->D - 1) * (18.0 + (nfs > 16 ? 9.0 : 0.0) + 3.0 * std::min(c->NA, 8) + (obliv ? 5.0 : 0.0));
+}
+
+int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw) {
+    int r = small_tree_buffers(c);
+    if (r != EVT_OK) return r;
+    SmallArgs A;
+    memset((void *)&A, 0, sizeof(A));
+    A.xcm = c->xcm;
+    A.gq = c->gq;
+    A.mask = c->mask;
+    A.hist = c->hist;
+    A.node_stride = (int64_t)c->F * c->NAg * c->B;
+    A.js = c->js;
+    A.js_src = c->js;
+    if (c->js_staged) { // read from the pinned buffer by the first kernel
+        A.js_src = reinterpret_cast<const uint32_t *>(c->h_stage_dev + c->blob_bytes);
+        A.map_src = reinterpret_cast<const uint32_t *>(c->h_stage_dev + c->blob_bytes + (size_t)c->F * 4);
+        A.map_dst = reinterpret_cast<uint32_t *>(c->jsmap);
+        A.map_words = c->RS / 2;
+        c->js_staged = false;
+    }
+    A.status = c->status;
+    A.node_sum = c->node_sum;
+    A.qscale = c->qscale;
+    A.tree = c->tree;
+    A.stats = c->stats;
+    A.nidx = c->nidx;
+    A.eta = p->eta; A.lambda = p->lambda; A.L2 = p->L2; A.gamma = p->gamma; A.min_weight = p->min_weight;
+    A.bagging = p->bagging_size;
+    A.seed = c->mask_seed;
+    A.N = (int)c->N; A.F = c->F; A.B = c->B; A.K = c->K; A.NK = c->NK; A.NAg = c->NAg; A.NA = c->NA; A.loss = c->loss; A.D = c->D; A.nnodes = c->nnodes;
+    A.nfs = c->n_js_last;
+    A.slots = small_slots(c);
+    A.oblivious = c->tree_type == EVT_TREE_OBLIVIOUS ? 1 : 0;
+    A.sampled = c->step.all_rows ? 0 : 1;
+    A.draw = draw ? 1 : 0;
+    A.cond = c->last_cond;
+    A.wide = c->NA > EVT_MAX_NA ? 1 : 0;
+    for (int j = 0; j < A.nfs; j++) {
+        const int f = (int)c->js_last[j] - 1;
+        A.feat[j] = (uint32_t)f | (c->h_feattypes[f] ? SMALL_NUMERIC : 0u) | ((uint32_t)(c->h_mono[f] + 1) << 17);
+    }
+    const int bpl = (c->B + 63) / 64;
+    for (int level = 1; level <= c->D; level++) {
+        A.level = level;
+        const int in = (level & 1) ^ 1, out = level & 1;
+        A.nid_in = c->small_nid[in]; A.nid_out = c->small_nid[out];
+        A.head_in = static_cast<const SmallHead *>(c->small_head[in]); A.head_out = static_cast<SmallHead *>(c->small_head[out]);
+        A.left_in = c->small_left[in]; A.left_out = c->small_left[out];
+        if (level == c->D) {
+            prof_begin(c, EVT_K_PARTITION, level);
+            A.blob_src = reinterpret_cast<const uint4 *>(c->tree_blob);
+            A.blob_dst = reinterpret_cast<uint4 *>(c->h_stage_dev);
+            A.blob_n = (int64_t)(c->blob_bytes / 16);
+            hipLaunchKernelGGL(k_small_final, dim3((unsigned)((c->N + 1023) / 1024)), dim3(1024), (size_t)(1 << (level - 1)) * c->NAg * 8, c->stream, A);
+            prof_end(c);
+            break;
+        }
+        const int nodes = 1 << (level - 1), slots = std::min(A.slots, nodes);
+        const int most = A.slots;
+        A.slots = slots;
+        const size_t lds = small_lds(c, level, slots);
+        prof_begin(c, level == 1 ? EVT_K_HIST : EVT_K_PARTITION, level); // below the root it moves rows, builds and searches at once
+#define SMALL3(NAG_, BPL_, PACK_)                                                                                                                  \
+    {                                                                                                                                              \
+        static EvtDevOnce once;                                                                                                                    \
+        if (once.pending(c->device)) {                                                                                                             \
+            HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_small_level<NAG_, BPL_, PACK_>), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024)); \
+            once.mark(c->device);                                                                                                                  \
+        }                                                                                                                                          \
+        hipLaunchKernelGGL((k_small_level<NAG_, BPL_, PACK_>), dim3((unsigned)c->n_js_last), dim3(1024), lds, c->stream, A);                       \
+    }
+#define SMALL2(NAG_, PACK_)             \
+    if (bpl == 1) SMALL3(NAG_, 1, PACK_) \
+    else if (bpl == 2) SMALL3(NAG_, 2, PACK_) \
+    else SMALL3(NAG_, 4, PACK_)
+#define SMALL1(NAG_)            \
+    if (c->unit_w) { SMALL2(NAG_, true) } \
+    else { SMALL2(NAG_, false) }
+        if (c->mc) { SMALL1(0) }
+        else if (c->NAg == 2) { SMALL1(2) }
+        else if (c->NAg == 3) { SMALL1(3) }
+        else { SMALL1(5) }
+#undef SMALL1
+#undef SMALL2
+#undef SMALL3
+        A.slots = most;
+        prof_end(c);
+        HIPCHK(hipGetLastError());
+    }
+    HIPCHK(hipGetLastError());
+    c->step.blob_sent = true;
+    return EVT_OK;
+}

@@ -1,0 +1,129 @@
+// What the split-search kernels share: wavefront primitives and the Float64 gain algebra (src/split.jl:1-141; src/predict.jl:198-262).
+#pragma once
+#include "evt_internal.h"
+#include <float.h>
+
+#define NO_BIN 0x7fffffff
+
+// ---- wavefront primitives -----------------------------------------------------------------
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ long long dpp_move_i64(long long x) {
+    int lo = (int)(x & 0xffffffffll), hi = (int)(x >> 32);
+    lo = __builtin_amdgcn_update_dpp(0, lo, CTRL, ROW_MASK, 0xf, false);
+    hi = __builtin_amdgcn_update_dpp(0, hi, CTRL, ROW_MASK, 0xf, false);
+    return ((long long)hi << 32) | (unsigned int)lo;
+}
+
+// Inclusive prefix sum over the 64 lanes of a wavefront.
+// row_shr:1,2,4,8 scan each row of 16 lanes; row_bcast:15 then row_bcast:31 carry row totals forward.
+__device__ __forceinline__ long long wave_incl_scan_i64(long long x) {
+    x += dpp_move_i64<0x111, 0xf>(x); // row_shr:1
+    x += dpp_move_i64<0x112, 0xf>(x); // row_shr:2
+    x += dpp_move_i64<0x114, 0xf>(x); // row_shr:4
+    x += dpp_move_i64<0x118, 0xf>(x); // row_shr:8
+    x += dpp_move_i64<0x142, 0xa>(x); // row_bcast:15 into rows 1 and 3
+    x += dpp_move_i64<0x143, 0xc>(x); // row_bcast:31 into rows 2 and 3
+    return x;
+}
+
+__device__ __forceinline__ long long wave_sum_i64(long long x) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        int lo = __shfl_xor((int)(x & 0xffffffffll), o), hi = __shfl_xor((int)(x >> 32), o);
+        x += ((long long)hi << 32) | (unsigned int)lo;
+    }
+    return x;
+}
+
+// Arg-max over the 64 lanes of a wavefront: highest gain, of equal gains the lowest bin; every lane gets the result.
+// Same data movement as the prefix scan above (row shifts, then row broadcasts; a lane without a source combines with
+// the identity), so the reduction ends in lane 63 - VALU moves only, where a butterfly of cross-lane shuffles goes
+// through the LDS crossbar eighteen times, each a dependent round trip.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ void argmax_step(double &g, int &b) {
+    const long long gb = __double_as_longlong(g);
+    const int olo = __builtin_amdgcn_update_dpp(0, (int)(gb & 0xffffffffll), CTRL, ROW_MASK, 0xf, false);
+    const int ohi = __builtin_amdgcn_update_dpp((int)0xFFF00000, (int)(gb >> 32), CTRL, ROW_MASK, 0xf, false); // -inf
+    const int ob = __builtin_amdgcn_update_dpp(NO_BIN, b, CTRL, ROW_MASK, 0xf, false);
+    const double og = __longlong_as_double(((long long)ohi << 32) | (unsigned int)olo);
+    if (og > g || (og == g && ob < b)) { g = og; b = ob; }
+}
+__device__ __forceinline__ void wave_argmax(double &g, int &b) {
+    argmax_step<0x111, 0xf>(g, b); // row_shr:1
+    argmax_step<0x112, 0xf>(g, b); // row_shr:2
+    argmax_step<0x114, 0xf>(g, b); // row_shr:4
+    argmax_step<0x118, 0xf>(g, b); // row_shr:8
+    argmax_step<0x142, 0xa>(g, b); // row_bcast:15 into rows 1 and 3
+    argmax_step<0x143, 0xc>(g, b); // row_bcast:31 into rows 2 and 3
+    const long long gb = __double_as_longlong(g);
+    const int lo = __builtin_amdgcn_readlane((int)(gb & 0xffffffffll), 63), hi = __builtin_amdgcn_readlane((int)(gb >> 32), 63);
+    g = __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+    b = __builtin_amdgcn_readlane(b, 63);
+}
+
+
+// ---- Float64 gain algebra, expression order as in the reference ------------------------------
+__device__ __forceinline__ double term_gh(double g, double h, double w, double lambda, double L2) {
+    double d = h + lambda * w + L2;
+    if (!(d > DBL_EPSILON)) d = DBL_EPSILON;
+    return g * g / d / 2.0;
+}
+
+// fixed-point channel sums -> the 2K+1 Float64 statistics [g.., h.., w]
+__device__ __forceinline__ void decode_vals(const long long *q, const double *sc, int loss, int NK, double *out) {
+    if (EVT_TWO_CHAN(loss, (NK - 1) / 2)) { // one-target mse / mae: channels {g, w}; h = 2w (mse), 0 (mae)
+        double w = (double)q[1] * sc[1];
+        out[0] = (double)q[0] * sc[0];
+        out[1] = (loss == EVT_LOSS_MSE) ? 2.0 * w : 0.0;
+        out[2] = w;
+    } else {
+        for (int k = 0; k < NK; k++) out[k] = (double)q[k] * sc[k];
+    }
+}
+
+// _term_cred with _cred_Z (src/split.jl:3-4, src/loss.jl:275-290): Z |m1| / (1 + L2 / w), Z = VHM / (VHM + EVPV) for
+// cred_var and the same ratio of square roots for cred_std, VHM = (m1 / w)^2, EVPV = max(eps, m2 / w - VHM)
+__device__ __forceinline__ double term_cred(int loss, double m1, double m2, double w, double L2) {
+    const double mean = m1 / w;
+    const double VHM = mean * mean;
+    double EVPV = m2 / w - VHM;
+    if (!(EVPV > DBL_EPSILON)) EVPV = DBL_EPSILON;
+    const double Z = (loss == EVT_LOSS_CRED_VAR) ? VHM / (VHM + EVPV) : sqrt(VHM) / (sqrt(VHM) + sqrt(EVPV));
+    return Z * fabs(m1) / (1.0 + L2 / w);
+}
+
+// One output's term of node_gain (src/split.jl:58-78): zero for mae.
+__device__ __forceinline__ double node_gain_k(int loss, double g, double h, double w, double lambda, double L2) {
+    if (EVT_IS_SHIFT(loss)) return 0.0;
+    if (EVT_IS_CRED(loss)) return term_cred(loss, g, h, w, L2);
+    return term_gh(g, h, w, lambda, L2);
+}
+
+// One output's term of split_gain (src/split.jl:108-141): left + right.  (Sg, Sh, w_p) are the node's totals.  mae:
+// _term_shift (src/split.jl:2), |g / w - mu_p| w / d on either side with d = max(eps, 1 + lambda + L2 / w).
+__device__ __forceinline__ double split_gain_k(int loss, double Sg, double Sh, double w_p, double g_l, double h_l, double w_l, double w_r,
+                                               double lambda, double L2) {
+    if (EVT_IS_SHIFT(loss)) {
+        double d_l = 1.0 + lambda + L2 / w_l, d_r = 1.0 + lambda + L2 / w_r;
+        if (!(d_l > DBL_EPSILON)) d_l = DBL_EPSILON;
+        if (!(d_r > DBL_EPSILON)) d_r = DBL_EPSILON;
+        const double mu_p = Sg / w_p;
+        return fabs(g_l / w_l - mu_p) * w_l / d_l + fabs((Sg - g_l) / w_r - mu_p) * w_r / d_r;
+    }
+    if (EVT_IS_CRED(loss)) return term_cred(loss, g_l, h_l, w_l, L2) + term_cred(loss, Sg - g_l, Sh - h_l, w_r, L2);
+    return term_gh(g_l, h_l, w_l, lambda, L2) + term_gh(Sg - g_l, Sh - h_l, w_r, lambda, L2);
+}
+
+// pred_leaf_cpu! / pred_scalar (src/predict.jl:198-262) for output k
+__device__ __forceinline__ double leaf_value(int loss, const double *S, int k, int K, double eta, int bagging, double lambda, double L2) {
+    if (EVT_IS_QUANTILE(loss)) return 0.0; // valued from the leaf's rows once the tree is complete (launch_quantile_leaves)
+    if (EVT_IS_CRED(loss)) return eta / (double)bagging * S[k] / (S[2 * K] + L2);
+    if (loss == EVT_LOSS_MAE) {
+        double d = S[2 * K] + lambda * S[2 * K] + L2;
+        if (!(d > DBL_EPSILON)) d = DBL_EPSILON;
+        return eta / (double)bagging * S[k] / d;
+    }
+    double d = S[K + k] + lambda * S[2 * K] + L2;
+    if (!(d > DBL_EPSILON)) d = DBL_EPSILON;
+    return -eta / (double)bagging * S[k] / d;
+}

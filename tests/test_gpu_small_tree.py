@@ -1,0 +1,77 @@
+"""One kernel per level (option "small_tree" = 2) against the histogram / search / partition kernels (= 0): trees, histograms, node ids,
+gradients and predictions over free-running rounds, bit for bit, at the edges of what that path takes."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import assert_tree_bits, make_data
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("N,F,B,D,loss,more", [
+    (4, 1, 2, 2, "mse", {}),
+    (5, 3, 16, 3, "mse", dict(weights=True)),
+    (1023, 7, 64, 6, "logloss", dict(sub="drawn")),
+    (4099, 10, 64, 10, "mse", {}),                                   # 256 nodes, several to a wavefront
+    (3001, 5, 255, 9, "logloss", dict(weights=True)),                # more nodes than LDS histograms: several passes over the rows
+    (8197, 17, 129, 5, "gaussian_mle", dict(weights=True, sub="mask")),
+    (65_535, 4, 33, 4, "mse", dict(sub="drawn")),
+    (2002, 256, 8, 5, "mse", {}),
+    (2500, 300, 8, 4, "poisson", dict(colsample=0.4)),
+    (6001, 9, 32, 6, "gaussian_mle", dict(cat=True, mono=True)),
+    (6001, 9, 100, 6, "mse", dict(cat=True, mono=True, sub="mask")),
+    (5003, 12, 64, 7, "gaussian_mle", dict(oblivious=True)),
+    (777, 6, 200, 4, "logloss", dict(oblivious=True, weights=True, cat=True, sub="drawn")),
+    (4001, 8, 32, 5, "mlogloss", dict(K=7)),
+    (2047, 8, 200, 6, "mlogloss", dict(K=3, weights=True, sub="mask", cat=True)),
+    (1500, 5, 64, 4, "mlogloss", dict(K=16, oblivious=True)),
+    (1200, 6, 64, 5, "mlogloss", dict(K=2)),
+])
+def test_one_kernel_per_level_changes_nothing(evt, N, F, B, D, loss, more):
+    rng = np.random.default_rng(N)
+    K = more.get("K")
+    if K:
+        x_bin = rng.integers(1, B + 1, size=(F, N), dtype=np.uint8)
+        y = (1 + (x_bin[0].astype(int) * K // (B + 1) + rng.integers(0, 2, N)) % K).astype(np.float32)
+        mu = np.zeros(K, np.float32)
+        w = (rng.random(N) + 0.5).astype(np.float32) if more.get("weights") else None
+    else:
+        x_bin, y, w, mu = make_data(N, N, F, B, loss, more.get("weights", False))
+    ft = (rng.random(F) > 0.4).astype(np.uint8) if more.get("cat") else None
+    mono = rng.integers(-1, 2, F).astype(np.int32) if more.get("mono") else None
+    nfs = max(1, int(F * more.get("colsample", 1.0)))
+    R = 4
+    jss = [np.sort(rng.choice(F, nfs, replace=False)).astype(np.uint32) + 1 for _ in range(R)]
+    masks = [rng.integers(0, 256, N, dtype=np.uint8) for _ in range(R)]
+    gp = evt.make_params(eta=0.4, min_weight=0.0 if N < 10 else 2.0, L2=1.0)
+    out = []
+    for small in (2, 0):
+        h = evt.Handle(N, F, B, len(mu), D, loss, "oblivious" if more.get("oblivious") else "binary")
+        h.set_option("small_tree", small)
+        h.set_xbin(x_bin)
+        h.set_feature_meta(ft, mono)
+        h.set_target(y, w, mu)
+        rec = []
+        for r in range(R):
+            h.update_grads()
+            if more.get("sub") == "drawn":
+                h.draw_mask(r + 5)
+                h.grow_tree_begin_staged(jss[r], gp, 140)
+                rec.append(h.grow_tree_end())
+            else:
+                rec.append(h.grow_tree(jss[r], gp, mask=masks[r] if more.get("sub") else None, cond=140))
+            rec += [h.get_hist(), h.get_nidx()]
+            if r != 1:  # with and without the predictions read between two rounds
+                rec.append(h.get_pred())
+        h.update_grads()
+        rec += [h.get_grads(), h.get_pred()]
+        h.close()
+        out.append(rec)
+    splits = 0
+    for a, b in zip(*out):
+        if isinstance(a, np.ndarray):
+            assert a.tobytes() == b.tobytes()
+        else:
+            assert_tree_bits(a, b)
+            splits += int(a.split.sum())
+    assert splits > 0 or N < 10
