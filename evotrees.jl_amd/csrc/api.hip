@@ -133,14 +133,8 @@ static void prof_collect(evt_ctx *c, const int64_t *stats_host, int64_t upto_seq
 
 template <typename T>
 static int dev_alloc(T **p, size_t n) {
-    *p = nullptr;
-    if (n == 0) n = 1;
-    hipError_t e = hipMalloc((void **)p, n * sizeof(T));
-    if (e != hipSuccess) {
-        evt_set_error("hipMalloc of %zu bytes failed: %s", n * sizeof(T), hipGetErrorString(e));
-        return EVT_ERR_NOMEM;
-    }
-    return EVT_OK;
+    *p = static_cast<T *>(dev_take(n * sizeof(T)));
+    return *p ? EVT_OK : EVT_ERR_NOMEM;
 }
 #define ALLOC(ptr, n)                         \
     do {                                      \
@@ -193,15 +187,14 @@ extern "C" int evt_destroy(evt_handle c) {
                     c->qscale_buf[0], c->qscale_buf[1], c->planes, c->metric_partial, c->errflag, c->ogains, c->sbest, c->is_id, c->pt_nodes, c->pt_pred, c->mask_next,
                     c->small_nid[0], c->small_nid[1], c->small_head[0], c->small_head[1], c->small_left[0], c->small_left[1],
                     c->alphas, c->alphas_f, c->qkeys_a, c->qkeys_b, c->qtemp};
-    for (void *p : ptrs)
-        if (p) (void)hipFree(p);
+    if (c->copy_stream) (void)hipStreamSynchronize(c->copy_stream);
+    for (void *p : ptrs) dev_give(p);
     for (int l = 0; l < 2; l++) {
         LevelTab &L = c->lvl[l];
         void *lp[] = {L.hdr, L.act_node, L.cprefix, L.bnode, L.bstart, L.bprefix, L.cdesc};
-        for (void *p : lp)
-            if (p) (void)hipFree(p);
+        for (void *p : lp) dev_give(p);
     }
-    if (c->h_stage_base) (void)hipHostFree(c->h_stage_base);
+    pinned_give(c->h_stage_base);
     for (auto &r : c->recs) {
         (void)hipEventDestroy(r.e0);
         (void)hipEventDestroy(r.e1);
@@ -209,22 +202,25 @@ extern "C" int evt_destroy(evt_handle c) {
     for (auto e : c->free_events) (void)hipEventDestroy(e);
     for (hipEvent_t e : c->tree_evs)
         if (e) (void)hipEventDestroy(e);
-    if (c->pt_stage) (void)hipHostFree(c->pt_stage);
-    if (c->copy_stream) {
-        (void)hipStreamSynchronize(c->copy_stream);
-        (void)hipStreamDestroy(c->copy_stream);
-    }
-    if (c->stream) (void)hipStreamDestroy(c->stream);
+    pinned_give(c->pt_stage);
+    if (c->copy_stream) stream_give(c->copy_stream, true);
+    if (c->stream) stream_give(c->stream, false);
     delete c;
     return EVT_OK;
     });
 }
 
+// by way of the end of the pinned staging buffer, past what trees stage there
 static hipError_t upload_alphas(evt_ctx *c) {
-    float af[EVT_MAX_K];
-    for (int k = 0; k < EVT_MAX_K; k++) af[k] = (float)c->h_alphas[k];
-    hipError_t e = hipMemcpy(c->alphas, c->h_alphas, sizeof(double) * EVT_MAX_K, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(c->alphas_f, af, sizeof(float) * EVT_MAX_K, hipMemcpyHostToDevice);
+    double *ad = reinterpret_cast<double *>(c->h_stage_base + c->h_stage_bytes - 512);
+    static_assert((sizeof(double) + sizeof(float)) * EVT_MAX_K <= 512, "the levels fit the slack of h_stage_bytes");
+    float *af = reinterpret_cast<float *>(ad + EVT_MAX_K);
+    for (int k = 0; k < EVT_MAX_K; k++) {
+        ad[k] = c->h_alphas[k];
+        af[k] = (float)c->h_alphas[k];
+    }
+    hipError_t e = hipMemcpyAsync(c->alphas, ad, sizeof(double) * EVT_MAX_K, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(c->alphas_f, af, sizeof(float) * EVT_MAX_K, hipMemcpyHostToDevice, c->stream);
     return e;
 }
 
@@ -331,12 +327,12 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     memset(c->prof_ms, 0, sizeof(c->prof_ms));
     memset(c->prof_units, 0, sizeof(c->prof_units));
     hipError_t e = hipGetDevice(&c->device);
-    if (e == hipSuccess) e = hipStreamCreate(&c->stream);
+    if (e == hipSuccess) e = stream_take(&c->stream, false);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&c->tree_evs[0], hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&c->tree_evs[1], hipEventDisableTiming);
     if (e != hipSuccess) {
         evt_set_error("stream creation failed: %s", hipGetErrorString(e));
-        if (c->stream) (void)hipStreamDestroy(c->stream);
+        if (c->stream) stream_give(c->stream, false);
         delete c;
         return EVT_ERR_HIP;
     }
@@ -419,43 +415,28 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     // pinned staging: tree read-back + small per-tree uploads
     c->h_stage_bytes = c->blob_bytes + (size_t)c->F * 4 + (size_t)c->RS * 2 + 1024;
     c->h_stage_bytes = (c->h_stage_bytes + 255) / 256 * 256;
-    if (hipHostMalloc((void **)&c->h_stage_base, 2 * c->h_stage_bytes, hipHostMallocDefault) != hipSuccess) {
-        evt_set_error("hipHostMalloc failed");
+    c->h_stage_base = c->h_stage_dev_base = static_cast<uint8_t *>(pinned_take(2 * c->h_stage_bytes));
+    if (!c->h_stage_base) {
         evt_destroy(c);
         return EVT_ERR_NOMEM;
     }
-    if (hipHostGetDevicePointer((void **)&c->h_stage_dev_base, c->h_stage_base, 0) != hipSuccess) {
-        evt_set_error("pinned staging buffer is not addressable from the device");
-        evt_destroy(c);
-        return EVT_ERR_HIP;
-    }
     c->h_stage = c->h_stage_base;
     c->h_stage_dev = c->h_stage_dev_base;
-    // defaults: all numeric, no monotone constraint
-    {
-        std::vector<uint8_t> ft(c->F, 1);
-        c->h_feattypes = ft;
-        c->h_mono.assign(c->F, 0);
-        hipError_t e2 = hipMemcpy(c->feattypes, ft.data(), c->F, hipMemcpyHostToDevice);
-        if (e2 == hipSuccess) e2 = hipMemset(c->mono, 0, sizeof(int32_t) * c->F);
-        if (e2 == hipSuccess) e2 = hipMemset(c->absmax, 0, sizeof(uint32_t) * 2 * EVT_ABSMAX_STRIPES * EVT_MC_MAX_NK);
-        if (e2 == hipSuccess) e2 = hipMemset(c->nidx, 0, sizeof(uint32_t) * N);
-        if (e2 == hipSuccess) e2 = hipMemset(c->errflag, 0, sizeof(int32_t));
-        if (e2 == hipSuccess) e2 = upload_alphas(c);
-        if (e2 != hipSuccess) {
-            evt_set_error("initial fills failed: %s", hipGetErrorString(e2));
-            evt_destroy(c);
-            return EVT_ERR_HIP;
-        }
-    }
-    {
-        int r = launch_iota(c, c->is_id, N);
-        hipError_t e3 = hipStreamSynchronize(c->stream);
-        if (r != EVT_OK || e3 != hipSuccess) {
-            if (r == EVT_OK) evt_set_error("initial fills failed: %s", hipGetErrorString(e3));
-            evt_destroy(c);
-            return r != EVT_OK ? r : EVT_ERR_HIP;
-        }
+    // defaults: all numeric, no monotone constraint; queued in stream order ahead of whatever reads them
+    c->h_feattypes.assign(c->F, 1);
+    c->h_mono.assign(c->F, 0);
+    hipError_t e2 = hipMemsetAsync(c->feattypes, 1, c->F, c->stream);
+    if (e2 == hipSuccess) e2 = hipMemsetAsync(c->mono, 0, sizeof(int32_t) * c->F, c->stream);
+    if (e2 == hipSuccess) e2 = hipMemsetAsync(c->absmax, 0, sizeof(uint32_t) * 2 * EVT_ABSMAX_STRIPES * EVT_MC_MAX_NK, c->stream);
+    if (e2 == hipSuccess) e2 = hipMemsetAsync(c->nidx, 0, sizeof(uint32_t) * N, c->stream);
+    if (e2 == hipSuccess) e2 = hipMemsetAsync(c->errflag, 0, sizeof(int32_t), c->stream);
+    if (e2 == hipSuccess) e2 = upload_alphas(c);
+    int r = EVT_OK;
+    if (e2 == hipSuccess) r = launch_iota(c, c->is_id, N);
+    if (r != EVT_OK || e2 != hipSuccess) {
+        if (r == EVT_OK) evt_set_error("initial fills failed: %s", hipGetErrorString(e2));
+        evt_destroy(c);
+        return r != EVT_OK ? r : EVT_ERR_HIP;
     }
     *out = c;
     return EVT_OK;
@@ -807,6 +788,7 @@ extern "C" int evt_set_alphas(evt_handle c, const double *alphas, int32_t n) {
     for (int k = 0; k < EVT_MAX_K; k++) c->h_alphas[k] = (k < n) ? a[k] : a[n - 1];
     c->n_alphas = n;
     HIPCHK(upload_alphas(c));
+    HIPCHK(hipStreamSynchronize(c->stream));
     c->have_grads = false; // the gradients of the quantile losses depend on the levels
     c->grads_ready = false;
     return EVT_OK;
@@ -850,7 +832,8 @@ static int ensure_planes(evt_ctx *c) {
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
         (void)hipGetLastError();
-        if (bytes > ((size_t)16 << 30) || bytes > free_b / 3 || hipMalloc((void **)&c->planes, bytes) != hipSuccess) {
+        if (bytes <= ((size_t)16 << 30) && bytes <= free_b / 3) c->planes = static_cast<uint32_t *>(dev_take(bytes));
+        if (!c->planes) {
             (void)hipGetLastError();
             c->planes = nullptr;
             c->use_planes = -1;
@@ -1200,7 +1183,7 @@ extern "C" int evt_stage_mask(evt_handle c, const uint8_t *mask) {
         evt_set_error("evt_stage_mask with two trees in flight: collect the older one first (evt_grow_tree_end)");
         return EVT_ERR_STATE;
     }
-    if (!c->copy_stream) HIPCHK(hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
+    if (!c->copy_stream) HIPCHK(stream_take(&c->copy_stream, true));
     if (!c->mask_next) {
         int r = dev_alloc(&c->mask_next, (size_t)c->N);
         if (r != EVT_OK) return r;
@@ -1404,19 +1387,15 @@ extern "C" int evt_predict_tree(evt_handle c, int32_t nnodes_tree, const int64_t
     }
     if (c->pt_cap < nn) { // device copies and upload buffer are kept between calls and grown on demand
         HIPCHK(hipStreamSynchronize(c->stream));
-        if (c->pt_nodes) (void)hipFree(c->pt_nodes);
-        if (c->pt_pred) (void)hipFree(c->pt_pred);
-        if (c->pt_stage) (void)hipHostFree(c->pt_stage);
+        dev_give(c->pt_nodes);
+        dev_give(c->pt_pred);
+        pinned_give(c->pt_stage);
         c->pt_nodes = nullptr; c->pt_pred = nullptr; c->pt_stage = nullptr; c->pt_stage_dev = nullptr; c->pt_cap = 0;
         const size_t cap = std::max(nn, (size_t)2047);
-        hipError_t e = hipMalloc((void **)&c->pt_nodes, sizeof(uint32_t) * cap);
-        if (e == hipSuccess) e = hipMalloc((void **)&c->pt_pred, sizeof(float) * cap * c->K);
-        if (e == hipSuccess) e = hipHostMalloc((void **)&c->pt_stage, sizeof(uint32_t) * cap * (1 + c->K), hipHostMallocDefault);
-        if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&c->pt_stage_dev, c->pt_stage, 0);
-        if (e != hipSuccess) {
-            evt_set_error("predict_tree buffers: %s", hipGetErrorString(e));
-            return EVT_ERR_NOMEM;
-        }
+        c->pt_nodes = static_cast<uint32_t *>(dev_take(sizeof(uint32_t) * cap));
+        c->pt_pred = static_cast<float *>(dev_take(sizeof(float) * cap * c->K));
+        c->pt_stage = c->pt_stage_dev = static_cast<uint8_t *>(pinned_take(sizeof(uint32_t) * cap * (1 + c->K)));
+        if (!c->pt_nodes || !c->pt_pred || !c->pt_stage) return EVT_ERR_NOMEM;
         c->pt_cap = cap;
     }
     memcpy(c->pt_stage, nodes.data(), sizeof(uint32_t) * nn);

@@ -7,6 +7,7 @@
 // best candidate per node.  The blocks meet only at the kernel boundary.  Rows keep their place: a node id per row stands for the row lists,
 // so rows outside the sample walk along (flagged) and the prediction needs no pass of its own over the tree.
 // The sums are the same integers and the gains the same expressions as in the kernels of larger inputs: same trees, bit for bit.
+#include "pool.h"
 #include "split_math.h"
 #include <algorithm>
 
@@ -640,13 +641,14 @@ static int small_slots(const evt_ctx *c) {
     return (int)std::min<size_t>((size_t)nodes, (budget - fixed) / one);
 }
 
-int small_tree_buffers(evt_ctx *c) {
-    if (c->small_nid[0]) return EVT_OK;
+static int small_tree_buffers(evt_ctx *c) {
+    if (c->small_nid[1]) return EVT_OK;
     const size_t cand = (size_t)(1 << (c->D - 2)) * std::min(c->F, 256);
     for (int k = 0; k < 2; k++) {
-        HIPCHK(hipMalloc((void **)&c->small_nid[k], sizeof(uint32_t) * (size_t)c->N));
-        HIPCHK(hipMalloc((void **)&c->small_head[k], sizeof(SmallHead) * cand));
-        if (c->NK > EVT_MAX_NA) HIPCHK(hipMalloc((void **)&c->small_left[k], sizeof(long long) * cand * c->NK));
+        c->small_head[k] = dev_take(sizeof(SmallHead) * cand);
+        if (c->NK > EVT_MAX_NA) c->small_left[k] = static_cast<long long *>(dev_take(sizeof(long long) * cand * c->NK));
+        c->small_nid[k] = static_cast<uint32_t *>(dev_take(sizeof(uint32_t) * (size_t)c->N));
+        if (!c->small_head[k] || !c->small_nid[k] || (c->NK > EVT_MAX_NA && !c->small_left[k])) return EVT_ERR_NOMEM;
     }
     return EVT_OK;
 }

@@ -41,7 +41,8 @@ struct Model {
     uint32_t *d_nodes = nullptr, *d_cid = nullptr;
     float *d_leaf = nullptr;
     CompletedTree *d_meta = nullptr;
-    size_t cap_nodes = 0, cap_leaf = 0, cap_cid = 0, cap_meta = 0;
+    uint8_t *d_form = nullptr; // the four of them, one after the other
+    size_t cap_form = 0;
     std::vector<CompletedTree> meta;
     std::unique_ptr<HbPlan> plan[2]; // by source type
     uint8_t *d_x = nullptr;          // bins of the pieces in flight
@@ -50,24 +51,18 @@ struct Model {
     ~Model() {
         (void)hipSetDevice(device);
         if (s) (void)hipStreamSynchronize(s);
-        void *p[] = {d_nodes, d_cid, d_leaf, d_meta, d_x};
-        for (void *q : p)
-            if (q) (void)hipFree(q);
-        if (s) (void)hipStreamDestroy(s);
+        void *p[] = {d_form, d_x};
+        for (void *q : p) dev_give(q);
+        if (s) stream_give(s, true);
     }
 };
 
-template <typename T>
-int grow(T **p, size_t *cap, size_t n) {
+int grow(uint8_t **p, size_t *cap, size_t n) {
     if (*cap >= n) return EVT_OK;
-    if (*p) (void)hipFree(*p);
-    *p = nullptr;
+    dev_give(*p);
     *cap = 0;
-    const hipError_t e = hipMalloc((void **)p, n * sizeof(T));
-    if (e != hipSuccess) {
-        evt_set_error("hipMalloc of %zu bytes failed: %s", n * sizeof(T), hipGetErrorString(e));
-        return EVT_ERR_NOMEM;
-    }
+    *p = static_cast<uint8_t *>(dev_take(n));
+    if (!*p) return EVT_ERR_NOMEM;
     *cap = n;
     return EVT_OK;
 }
@@ -173,17 +168,31 @@ int build(Model &m, const TreePtrs &t, const uint8_t *feattypes, int nft) {
         o += (size_t)n;
     }
     ARGCHK(leaf.size() < ((size_t)1 << 31), "the leaves of a kept model exceed 2^31 values");
+    // one block on the device, one copy: meta | nodes | leaf ids | leaf values, each from a 256-byte boundary on
+    auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+    const size_t o_nodes = up(sizeof(CompletedTree) * m.meta.size()), o_cid = o_nodes + up(4 * nodes.size()), o_leaf = o_cid + up(4 * cid.size());
+    const size_t bytes = o_leaf + up(4 * leaf.size());
     HIPCHK(hipStreamSynchronize(m.s));
-    int r = grow(&m.d_nodes, &m.cap_nodes, nodes.size());
-    if (r == EVT_OK) r = grow(&m.d_leaf, &m.cap_leaf, leaf.size());
-    if (r == EVT_OK) r = grow(&m.d_cid, &m.cap_cid, cid.size());
-    if (r == EVT_OK) r = grow(&m.d_meta, &m.cap_meta, m.meta.size());
+    const int r = grow(&m.d_form, &m.cap_form, bytes);
     if (r != EVT_OK) return r;
-    HIPCHK(hipMemcpyAsync(m.d_nodes, nodes.data(), 4 * nodes.size(), hipMemcpyHostToDevice, m.s));
-    HIPCHK(hipMemcpyAsync(m.d_leaf, leaf.data(), 4 * leaf.size(), hipMemcpyHostToDevice, m.s));
-    HIPCHK(hipMemcpyAsync(m.d_cid, cid.data(), 4 * cid.size(), hipMemcpyHostToDevice, m.s));
-    HIPCHK(hipMemcpyAsync(m.d_meta, m.meta.data(), sizeof(CompletedTree) * m.meta.size(), hipMemcpyHostToDevice, m.s));
-    HIPCHK(hipStreamSynchronize(m.s));
+    struct Staged { // pinned, and given back whichever way the call ends
+        void *p;
+        ~Staged() { pinned_give(p); }
+    } stage{bytes <= PINNED_BYTES ? pinned_take(PINNED_BYTES) : nullptr};
+    std::vector<uint8_t> plain(stage.p ? 0 : bytes);
+    uint8_t *h = stage.p ? static_cast<uint8_t *>(stage.p) : plain.data();
+    memcpy(h, m.meta.data(), sizeof(CompletedTree) * m.meta.size());
+    memcpy(h + o_nodes, nodes.data(), 4 * nodes.size());
+    memcpy(h + o_cid, cid.data(), 4 * cid.size());
+    memcpy(h + o_leaf, leaf.data(), 4 * leaf.size());
+    const hipError_t e = hipMemcpyAsync(m.d_form, h, bytes, hipMemcpyHostToDevice, m.s);
+    const hipError_t e2 = hipStreamSynchronize(m.s);
+    HIPCHK(e);
+    HIPCHK(e2);
+    m.d_meta = reinterpret_cast<CompletedTree *>(m.d_form);
+    m.d_nodes = reinterpret_cast<uint32_t *>(m.d_form + o_nodes);
+    m.d_cid = reinterpret_cast<uint32_t *>(m.d_form + o_cid);
+    m.d_leaf = reinterpret_cast<float *>(m.d_form + o_leaf);
     m.built = true;
     return EVT_OK;
 }
@@ -311,7 +320,7 @@ extern "C" int evt_model_create(int32_t loss, int32_t K, void **out) {
     m->loss = loss;
     m->K = K;
     HIPCHK(hipGetDevice(&m->device));
-    HIPCHK(hipStreamCreateWithFlags(&m->s, hipStreamNonBlocking));
+    HIPCHK(stream_take(&m->s, true));
     *out = m.release();
     return EVT_OK;
     });

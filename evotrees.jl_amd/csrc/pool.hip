@@ -1,0 +1,147 @@
+#include "pool.h"
+
+#include <map>
+#include <mutex>
+#include <unordered_map>
+
+namespace {
+
+std::mutex g_mu;
+struct Block {
+    size_t size;
+    int device;
+};
+std::unordered_map<void *, Block> g_out[2];                            // blocks in use: device, pinned
+std::multimap<std::pair<int, size_t>, void *> g_idle[2];               // by (device, size); pinned blocks under device 0
+std::map<int, size_t> g_kept[2];                                       // idle bytes by device
+std::multimap<int, hipStream_t> g_streams[2];                          // blocking, non-blocking
+const size_t STREAMS_KEPT = 4;
+
+// sizes are rounded up by an eighth at most, so that inputs of about the same size find each other's blocks
+size_t size_class(size_t n) {
+    size_t step = 4096;
+    while (step * 16 <= n) step <<= 1;
+    return (n + step - 1) / step * step;
+}
+int current_device() {
+    int d = 0;
+    return hipGetDevice(&d) == hipSuccess ? d : 0;
+}
+void release(int kind, void *p) {
+    if (kind == 0) (void)hipFree(p);
+    else (void)hipHostFree(p);
+}
+void trim(int kind) {
+    std::vector<void *> idle;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        for (auto &e : g_idle[kind]) idle.push_back(e.second);
+        g_idle[kind].clear();
+        g_kept[kind].clear();
+    }
+    for (void *p : idle) release(kind, p);
+}
+void *take(int kind, size_t bytes) {
+    const int dev = kind == 0 ? current_device() : 0;
+    const size_t n = size_class(bytes ? bytes : 1);
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        auto it = g_idle[kind].find({dev, n});
+        if (it != g_idle[kind].end()) {
+            void *p = it->second;
+            g_idle[kind].erase(it);
+            g_kept[kind][dev] -= n;
+            g_out[kind][p] = {n, dev};
+            return p;
+        }
+    }
+    void *p = nullptr;
+    hipError_t e = hipSuccess;
+    for (int attempt = 0; attempt < 2; attempt++) {
+        e = kind == 0 ? hipMalloc(&p, n) : hipHostMalloc(&p, n, hipHostMallocPortable);
+        if (e == hipSuccess) break;
+        (void)hipGetLastError();
+        trim(kind); // idle blocks of other sizes make room
+    }
+    if (e != hipSuccess) {
+        evt_set_error("%s of %zu bytes failed: %s", kind == 0 ? "hipMalloc" : "hipHostMalloc", n, hipGetErrorString(e));
+        return nullptr;
+    }
+    if (kind == 1) {
+        void *d = nullptr;
+        if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess || d != p) {
+            evt_set_error("pinned memory is not addressable from the device");
+            release(1, p);
+            return nullptr;
+        }
+    }
+    std::lock_guard<std::mutex> lk(g_mu);
+    g_out[kind][p] = {n, dev};
+    return p;
+}
+void give(int kind, void *p) {
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        auto it = g_out[kind].find(p);
+        if (it != g_out[kind].end()) {
+            const Block b = it->second;
+            g_out[kind].erase(it);
+            if (b.size <= POOL_BLOCK_KEPT && g_kept[kind][b.device] + b.size <= (kind == 0 ? POOL_DEVICE_KEPT : POOL_PINNED_KEPT)) {
+                g_idle[kind].insert({{b.device, b.size}, p});
+                g_kept[kind][b.device] += b.size;
+                return;
+            }
+        }
+    }
+    release(kind, p);
+}
+
+} // namespace
+
+void *dev_take(size_t bytes) { return take(0, bytes); }
+void dev_give(void *p) { give(0, p); }
+void *pinned_take(size_t bytes) { return take(1, bytes); }
+void pinned_give(void *p) { give(1, p); }
+
+hipError_t stream_take(hipStream_t *s, bool non_blocking) {
+    const int dev = current_device();
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        auto it = g_streams[non_blocking].find(dev);
+        if (it != g_streams[non_blocking].end()) {
+            *s = it->second;
+            g_streams[non_blocking].erase(it);
+            return hipSuccess;
+        }
+    }
+    return hipStreamCreateWithFlags(s, non_blocking ? hipStreamNonBlocking : hipStreamDefault);
+}
+void stream_give(hipStream_t s, bool non_blocking) {
+    const int dev = current_device();
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        if (g_streams[non_blocking].count(dev) < STREAMS_KEPT) {
+            g_streams[non_blocking].insert({dev, s});
+            return;
+        }
+    }
+    (void)hipStreamDestroy(s);
+}
+
+extern "C" int evt_trim(void) {
+    return guarded([&]() -> int {
+    trim(0);
+    trim(1);
+    std::vector<hipStream_t> idle;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        for (auto &q : g_streams) {
+            for (auto &e : q) idle.push_back(e.second);
+            q.clear();
+        }
+    }
+    for (hipStream_t s : idle) (void)hipStreamDestroy(s);
+    return EVT_OK;
+    });
+}

@@ -2,16 +2,12 @@
 #pragma once
 #include "evt_internal.h"
 #include "host_bin.h"
+#include "pool.h"
 
-// Pinned buffers of PINNED_BYTES each, kept between calls: pinning 8 MB costs the host more than filling them.  At most
-// PINNED_KEPT stay behind when nobody uses them (32 MB); evt_trim gives those back.  Any thread, any device (portable).
-static const size_t PINNED_BYTES = (size_t)8 << 20;
-static const int PINNED_KEPT = 4;
-void *pinned_take();          // nullptr: out of memory (the error is set); the device uses the same address
-void pinned_give(void *p);    // nothing on the device may still use it
+static const size_t PINNED_BYTES = (size_t)8 << 20; // a piece on its way up
 
 struct PinnedSlots { // NS of them, with an event each for the work that reads or writes them
-    static const int NS = PINNED_KEPT;
+    static const int NS = 4;
     void *host[NS] = {};
     hipEvent_t ev[NS] = {};
     hipStream_t s;
@@ -19,7 +15,7 @@ struct PinnedSlots { // NS of them, with an event each for the work that reads o
     explicit PinnedSlots(hipStream_t s_) : s(s_) {}
     int init(int n) {
         for (int k = 0; k < n; k++) {
-            host[k] = pinned_take();
+            host[k] = pinned_take(PINNED_BYTES);
             if (!host[k]) return EVT_ERR_NOMEM;
             HIPCHK(hipEventCreateWithFlags(&ev[k], hipEventDisableTiming));
         }

@@ -1,58 +1,7 @@
-// Pinned buffers, and the pipeline that bins a host matrix on its way to the device.
+// The pipeline that bins a host matrix on its way to the device.
 #include "upload.h"
 
 #include <algorithm>
-#include <mutex>
-
-namespace {
-std::mutex g_pin_m;
-std::vector<void *> g_pin_idle;
-} // namespace
-
-void *pinned_take() {
-    {
-        std::lock_guard<std::mutex> lk(g_pin_m);
-        if (!g_pin_idle.empty()) {
-            void *p = g_pin_idle.back();
-            g_pin_idle.pop_back();
-            return p;
-        }
-    }
-    void *p = nullptr;
-    const hipError_t e = hipHostMalloc(&p, PINNED_BYTES, hipHostMallocPortable);
-    if (e != hipSuccess) {
-        evt_set_error("hipHostMalloc failed: %s", hipGetErrorString(e));
-        return nullptr;
-    }
-    void *dev = nullptr;
-    if (hipHostGetDevicePointer(&dev, p, 0) != hipSuccess || dev != p) {
-        evt_set_error("pinned buffer is not addressable from the device");
-        (void)hipHostFree(p);
-        return nullptr;
-    }
-    return p;
-}
-void pinned_give(void *p) {
-    {
-        std::lock_guard<std::mutex> lk(g_pin_m);
-        if ((int)g_pin_idle.size() < PINNED_KEPT) {
-            g_pin_idle.push_back(p);
-            return;
-        }
-    }
-    (void)hipHostFree(p);
-}
-extern "C" int evt_trim(void) {
-    return guarded([&]() -> int {
-    std::vector<void *> idle;
-    {
-        std::lock_guard<std::mutex> lk(g_pin_m);
-        idle.swap(g_pin_idle);
-    }
-    for (void *p : idle) (void)hipHostFree(p);
-    return EVT_OK;
-    });
-}
 
 BinPieces::BinPieces(int64_t N_, int F_, bool src_rows_contiguous, bool by_rows, int64_t rows_most, int64_t cells_most)
     : N(N_), F(F_), rowwise(src_rows_contiguous) {

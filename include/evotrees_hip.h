@@ -128,7 +128,8 @@ const char *evt_last_error(void);
 /* Number of visible HIP devices; fails (EVT_ERR_HIP) when the runtime finds none. */
 int evt_device_count(int32_t *count);
 
-/* Gives back the pinned buffers that matrices go up through and that are kept between calls (at most 32 MB). */
+/* Gives back what the library keeps between calls for the next handle, model or matrix: device buffers (at most 1 GB per device),
+ * pinned ones (64 MB) and streams. */
 int evt_trim(void);
 
 /* ---- training cache ------------------------------------------------------------------
