@@ -76,12 +76,17 @@ struct TreePtrs {
     const float *const *pred;
 };
 
-bool same_trees(const Model &m, const TreePtrs &t) {
+bool same_shape(const Model &m, const TreePtrs &t) {
     if (!m.built || (size_t)t.n != m.nn.size()) return false;
+    for (int i = 0; i < t.n; i++)
+        if (m.nn[i] != t.nn[i]) return false;
+    return true;
+}
+bool same_trees(const Model &m, const TreePtrs &t) { // of trees of the same shape
     size_t o = 0;
     for (int i = 0; i < t.n; i++) {
         const size_t n = (size_t)m.nn[i];
-        if ((int64_t)n != t.nn[i] || memcmp(m.feat.data() + o, t.feat[i], 8 * n) || memcmp(m.cond_bin.data() + o, t.cond_bin[i], n) ||
+        if (memcmp(m.feat.data() + o, t.feat[i], 8 * n) || memcmp(m.cond_bin.data() + o, t.cond_bin[i], n) ||
             memcmp(m.split.data() + o, t.split[i], n) || memcmp(m.pred.data() + o * m.K, t.pred[i], 4 * n * m.K))
             return false;
         o += n;
@@ -209,6 +214,8 @@ struct Request {
     int F, ntrees, link;
     float *out;
     uint32_t *leaf_out;
+    const TreePtrs *check; // compare the caller's trees with the device form once the device is at work (null: known to be the same)
+    bool differ;           // they are not the same: the results are those of the old trees
 };
 
 int walk(Model &m, const Request &q, const uint8_t *x, int64_t n, void *out, int leaf_bytes) {
@@ -228,12 +235,13 @@ void widen(const T *src, uint32_t *dst, int64_t n) {
     for (int64_t i = 0; i < n; i++) dst[i] = src[i];
 }
 
-int run(Model &m, const Request &q) {
+int run(Model &m, Request &q) {
     const int leaf_bytes = !q.leaf_out ? 0 : m.max_nodes <= 255 ? 1 : m.max_nodes <= 65535 ? 2 : 4;
     const int64_t back = q.leaf_out ? (int64_t)q.ntrees * leaf_bytes : (int64_t)m.K * 4; // bytes a row sends back
     const int64_t per_row = q.F + back;
-    // pieces of a twelfth of the whole, so that binning, copies and kernels overlap; 256 KB at least, a buffer at most
-    const int64_t goal = std::min<int64_t>((int64_t)PINNED_BYTES - 4096, std::max<int64_t>(256 << 10, q.N * per_row / 12));
+    // pieces of a twelfth of the whole, so that binning, copies and kernels overlap; 256 KB at least, a buffer at most.  Leaf ids: of a
+    // fourth, so that as many as fit the buffers are spread out into the caller's words (most of the work) together at the end
+    const int64_t goal = std::min<int64_t>((int64_t)PINNED_BYTES - 4096, std::max<int64_t>(256 << 10, q.N * per_row / (q.leaf_out ? 4 : 12)));
     ARGCHK(64 * per_row <= (int64_t)PINNED_BYTES - 4096, "too many trees for one piece");
     const int64_t rows_most = std::max<int64_t>(64, goal / per_row / 64 * 64);
     const bool rowwise = q.plan && q.src.rows_contiguous();
@@ -276,6 +284,7 @@ int run(Model &m, const Request &q) {
         const int rw = walk(m, q, x, n, h + xs, leaf_bytes); // the kernel writes what comes back over the bus itself
         if (rw != EVT_OK) return rw;
         if (!direct) HIPCHK(hipEventRecord(U.ev[p % NS], m.s));
+        if (p == 0 && q.check) q.differ = !same_trees(m, *q.check);
         return EVT_OK;
     };
     auto retire = [&](int64_t p) {
@@ -283,7 +292,7 @@ int run(Model &m, const Request &q) {
         piece(p, &r0, &n);
         const uint8_t *h = static_cast<const uint8_t *>(U.host[p % NS]) + xs;
         if (q.leaf_out) {
-            hb_parallel(q.ntrees, (int)std::min<int64_t>(hb_workers(n * q.ntrees / 2), 8), [&](int t) {
+            hb_parallel(q.ntrees, hb_workers(n * q.ntrees / 2), [&](int t) {
                 uint32_t *d = q.leaf_out + (size_t)t * q.N + r0;
                 const size_t at = (size_t)t * n;
                 if (leaf_bytes == 1) widen(h + at, d, n);
@@ -345,16 +354,30 @@ extern "C" int evt_model_predict(void *model, int32_t n_model, const int64_t *nn
     HIPCHK(hipSetDevice(m.device));
     const TreePtrs t{n_model, nnodes, feat, cond_bin, split, pred};
     const size_t nft = feattypes ? (size_t)nfeattypes : 0;
-    if (m.feattypes.size() != nft || (nft && memcmp(m.feattypes.data(), feattypes, nft)) || !same_trees(m, t)) {
+    // The trees are compared with the device form while the device already walks it (20 us for 700 KB of trees); if they turn out to
+    // have changed, the new ones are packed and the call runs again.
+    bool known = m.feattypes.size() == nft && (!nft || !memcmp(m.feattypes.data(), feattypes, nft)) && same_shape(m, t) && m.max_feat <= nfeats;
+    if (!known) {
         const int r = build(m, t, feattypes, nfeattypes);
         if (r != EVT_OK) return r;
     }
+    auto walk_all = [&](Request &q) -> int {
+        q.check = known ? &t : nullptr;
+        q.differ = false;
+        int r = run(m, q);
+        if (r != EVT_OK || !q.differ) return r;
+        r = build(m, t, feattypes, nfeattypes);
+        if (r != EVT_OK) return r;
+        ARGCHK(m.max_feat <= nfeats, "tree feature id outside 1..nfeats");
+        q.check = nullptr;
+        return run(m, q);
+    };
     ARGCHK(m.max_feat <= nfeats, "tree feature id outside 1..nfeats");
-    Request q{nullptr, {}, nullptr, nobs, nfeats, ntrees, apply_link, out, leaf_out};
+    Request q{nullptr, {}, nullptr, nobs, nfeats, ntrees, apply_link, out, leaf_out, nullptr, false};
     if (!edges) {
         ARGCHK(dtype == EVT_U8, "a matrix of bins is EVT_U8");
         q.bins = static_cast<const uint8_t *>(x);
-        return run(m, q);
+        return walk_all(q);
     }
     ARGCHK((dtype == EVT_F32 || dtype == EVT_F64) && (row_stride == 1 || col_stride == 1), "dtype must be EVT_F32 or EVT_F64 and one of the two strides 1");
     bool same = m.edge_off.size() == (size_t)nfeats + 1;
@@ -379,6 +402,6 @@ extern "C" int evt_model_predict(void *model, int32_t n_model, const int64_t *nn
     }
     q.plan = plan.get();
     q.src = HbSource{x, dtype, row_stride, col_stride};
-    return run(m, q);
+    return walk_all(q);
     });
 }

@@ -94,7 +94,7 @@ static int run_pieces(PinnedSlots &U, int NS, int64_t np, int tasks, int workers
     int64_t back = 0;
     for (int64_t p = 0; p < np; p++) {
         while (done[(size_t)p].load(std::memory_order_acquire) < tasks) {
-            if (back < p) { // the oldest piece sent that has not been retired
+            if (back < p && back + NS < np) { // the oldest piece sent that has not been retired, while a piece needs its buffer
                 const hipError_t q = hipEventQuery(U.ev[back % NS]);
                 if (q == hipSuccess) {
                     retire(back++);
@@ -110,6 +110,7 @@ static int run_pieces(PinnedSlots &U, int NS, int64_t np, int tasks, int workers
         const int r = send(p);
         if (r != EVT_OK) return r;
     }
+    ws.join(); // the workers are free for what retire() shares out
     for (; back < np; back++) {
         HIPCHK(hipEventSynchronize(U.ev[back % NS]));
         retire(back);
