@@ -185,7 +185,7 @@ extern "C" int evt_destroy(evt_handle c) {
     void *ptrs[] = {c->xcm, c->xrm, c->y, c->pred, c->grad, c->gq, c->is_a, c->is_b, c->nidx, c->mask, c->flagw, c->chunk_nleft, c->chunk_lpre,
                     c->hist, c->seg_start, c->seg_len, c->status, c->node_sum, c->tree_blob, c->tree.packed, c->js, c->jsmap, c->feattypes, c->mono, c->absmax, c->qexp_buf[0], c->qexp_buf[1], c->qbits,
                     c->qscale_buf[0], c->qscale_buf[1], c->planes, c->metric_partial, c->errflag, c->ogains, c->sbest, c->is_id, c->pt_nodes, c->pt_pred, c->mask_next,
-                    c->small_nid[0], c->small_nid[1], c->small_head[0], c->small_head[1], c->small_left[0], c->small_left[1],
+                    c->small_nid[0], c->small_nid[1], c->small_head[0], c->small_head[1], c->small_left[0], c->small_left[1], c->small_acc,
                     c->alphas, c->alphas_f, c->qkeys_a, c->qkeys_b, c->qtemp};
     if (c->copy_stream) (void)hipStreamSynchronize(c->copy_stream);
     for (void *p : ptrs) dev_give(p);
@@ -293,6 +293,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->scan_fused = 1;
     c->hist_in_scatter = 1;
     c->small_tree = 1;
+    c->small_acc = nullptr;
     for (int k = 0; k < 2; k++) {
         c->small_nid[k] = nullptr;
         c->small_head[k] = nullptr;
@@ -974,7 +975,7 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
     const bool fuse_pred = p->update_pred && all_rows && !defer;
     c->write_nidx = rec_nidx || defer;
 
-    const bool small = !staged && small_tree_applies(c, n_js, all_rows);
+    const int small = staged ? 0 : small_tree_form(c, n_js, all_rows);
     int r = small ? EVT_OK : ensure_planes(c);
     if (r != EVT_OK) return r;
     if (EVT_IS_QUANTILE(c->loss)) {
@@ -1148,7 +1149,7 @@ static int tree_fail(evt_ctx *c, int r) { // a failed stage leaves no tree open
 // every stage of an opened tree, then the close: what evt_grow_tree_begin queues
 static int tree_run_stages(evt_ctx *c, int r) {
     if (r == EVT_OK && c->step.small) {
-        r = launch_small_tree(c, &c->step.p, c->step.small_draw);
+        r = launch_small_tree(c, &c->step.p, c->step.small_draw, c->step.small);
         c->step.phase = 4;
     }
     while (r == EVT_OK && c->step.phase != 4) {
@@ -1833,7 +1834,7 @@ extern "C" int evt_set_option(evt_handle c, const char *name, int64_t value) {
     } else if (strcmp(name, "record_nidx") == 0) {
         c->record_nidx = value != 0;
     } else if (strcmp(name, "small_tree") == 0) {
-        ARGCHK(value >= 0 && value <= 2, "small_tree must be 0 (never), 1 (inputs of few rows) or 2 (wherever it can)");
+        ARGCHK(value >= 0 && value <= 3, "small_tree must be 0 (never), 1 (inputs of few rows), 2 or 3 (one or two kernels per level wherever it can)");
         c->small_tree = (int)value;
     } else if (strcmp(name, "scan_fused") == 0) {
         c->scan_fused = value != 0;

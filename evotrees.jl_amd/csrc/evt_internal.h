@@ -185,12 +185,13 @@ struct evt_ctx {
     int hist_blocks, hist_threads, hist_min_rows, hist_seg_cost;
     int hist_variant;  // 0 auto, 1 generic 16-byte-piece kernel, 2 conflict-free 8-byte-piece kernel where it applies
     int scan_fused;    // option: the split search of a node with at most 16 sampled features runs in one kernel
-    int small_tree;    // option: one kernel per level (kernels_small.hip) - 0 never, 1 for inputs of few rows, 2 wherever it can
+    int small_tree;    // option: one kernel per level (kernels_small.hip) - 0 never, 1 for inputs of few rows, 2 wherever it can, 3 the form of two kernels per level wherever it can
     // its buffers, allocated with the first such tree: the rows' node ids, the blocks' candidates and the totals left of them, of
     // two levels each
     uint32_t *small_nid[2];
     void *small_head[2];
     long long *small_left[2];
+    uint8_t *small_acc; // where blocks share a feature's rows: their row counts, and the sums of their histograms (zero between levels)
     int hist_in_scatter; // option: with 16-byte records and few chunks the partition's scatter pass builds the next level's histograms
     bool record_nidx;  // leaf finalisation also writes the node id of every sampled row
     bool nidx_valid;   // nidx holds the last tree's node ids
@@ -209,7 +210,7 @@ struct evt_ctx {
         int level;
         bool all_rows, defer, fuse_pred;
         bool hist_fused; // levels below the root get their histograms from the scatter pass of the level above
-        bool small;      // one kernel per level (launch_small_tree)
+        int small;       // one kernel per level, or two and the blocks that share a feature's rows (small_tree_form)
         bool small_draw; // ... whose first draws the row mask
         bool blob_sent;  // the finished tree's transfer to the host rode along with the tree's last kernel
         uint32_t *is_cur, *is_next; // row-id lists of the current level and of the one below
@@ -377,8 +378,8 @@ int launch_obliv_select(evt_ctx *c, int level, const evt_params *p);
 int launch_part_count(evt_ctx *c, int level, const uint32_t *is_cur);
 int launch_part_scatter(evt_ctx *c, int level, const uint32_t *is_cur, uint32_t *is_next, bool fuse_pred);
 bool scatter_can_build_hist(const evt_ctx *c, int nfs);
-bool small_tree_applies(const evt_ctx *c, int nfs, bool all_rows);
-int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw);
+int small_tree_form(const evt_ctx *c, int nfs, bool all_rows);
+int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices);
 int launch_final_fused(evt_ctx *c, int level, const uint32_t *is_cur, bool fuse_pred, bool send_blob);
 int launch_nidx_from_segments(evt_ctx *c, int level, const uint32_t *is_cur);
 int launch_copy_to_host(evt_ctx *c, const void *src_dev, void *dst_host_dev, size_t nbytes);

@@ -1,4 +1,4 @@
-// Trees of small inputs (tens of thousands of rows): one kernel per level instead of a histogram, a search and a two-pass partition.
+// Trees of small inputs (thousands to a few hundred thousand rows): one or two kernels per level instead of a histogram, a search and a two-pass partition.
 //
 // At these sizes a level is a chain of short dependent kernels - 20 launches of 3 to 9 us for a tree of depth 6 on 2000 rows, whatever they
 // do.  Here a block owns one sampled feature and walks ALL rows: it takes the decisions of the level above (every block the same
@@ -52,6 +52,9 @@ struct SmallArgs {
     unsigned long long seed;
     int N, F, B, K, NK, NAg, NA, loss, level, D, nnodes, nfs, bagging;
     int slots;     // histograms the block's LDS holds
+    int slices;    // blocks that share a feature's rows
+    long long *acc; // slices > 1: [node][block][NAg][B], their histograms added up; zero between two levels
+    int *counts;    // ... and their rows, [level][slice]
     int oblivious, sampled, draw, cond;
     int wide;      // channel 0 staged as a 64-bit packed word (more channels than EVT_MAX_NA)
     // the blocks' features, in the launch's arguments: a block need not wait for them.  0-based id | numeric << 16 | (constraint + 1) << 17
@@ -319,7 +322,98 @@ __device__ __forceinline__ void small_left(const SmallArgs &A, const unsigned lo
     }
 }
 
+// The search of one (node, feature) and what it leaves: the node's histogram of the feature, the candidate - or, for an oblivious
+// level, the gains of all bins in s_gain - and at the root the node's totals.
 template <int NAG, int BPL, bool PACK>
+__device__ __forceinline__ void small_search(const SmallArgs &A, const unsigned long long *Hs, int q, int jp, int nwg, uint32_t fw, const long long *tot,
+                                             bool writer, double *s_gain, int lane) {
+    const int B = A.B, nag = NAG ? NAG : A.NAg, n = (1 << (A.level - 1)) + q;
+    const bool numeric = (fw & SMALL_NUMERIC) != 0;
+    const int feat = numeric ? (int)(fw & 0xFFFFu) + 1 : -((int)(fw & 0xFFFFu) + 1);
+    long long *hout = A.hist + (int64_t)(n - 1) * A.node_stride + (int64_t)jp * nag * B;
+    double lg = -INFINITY;
+    int lb = NO_BIN;
+    constexpr int QA = NAG ? NAG : 1;
+    long long tq[QA], lq[QA];
+#pragma unroll
+    for (int ag = 0; ag < QA; ag++) lq[ag] = 0;
+    small_scan<NAG, BPL, PACK>(A, Hs, tot, numeric, (int)(fw >> 17) - 1, lane, hout, tq, [&](int b, bool ok, double gain, const long long *left) {
+        if (A.oblivious) {
+            if (b < B) s_gain[b] = gain; // update_gains!
+        } else if (ok && gain > lg) {
+            lg = gain;
+            lb = b + 1;
+            if constexpr (NAG != 0) {
+#pragma unroll
+                for (int ag = 0; ag < QA; ag++) lq[ag] = left[ag];
+            }
+        }
+    });
+    if (A.level == 1 && writer) { // for the kernels below
+        if constexpr (NAG != 0) {
+            if (lane == 0)
+#pragma unroll
+                for (int ag = 0; ag < QA; ag++) A.node_sum[(int64_t)n * nag + ag] = tq[ag];
+        } else {
+            for (int ag = 0; ag < nag; ag++) {
+                long long t = 0;
+                for (int b = lane; b < B; b += 64) t += channel_of<PACK>(Hs, B, nag, ag, b);
+                t = wave_sum_i64(t);
+                if (lane == 0) A.node_sum[(int64_t)n * nag + ag] = t;
+            }
+        }
+    }
+    if (A.oblivious) return;
+    wave_argmax(lg, lb);
+    SmallHead *out = A.head_out + (int64_t)q * nwg + jp;
+    if constexpr (NAG != 0) { // the lane that holds the winning bin has the totals left of it
+        if (lane == (lb != NO_BIN ? (lb - 1) / BPL : 0)) {
+            SmallHead h;
+            h.gain = lg;
+            h.bin = lb;
+            h.feat = feat;
+#pragma unroll
+            for (int ag = 0; ag < EVT_MAX_NA + 1; ag++) h.left[ag] = ag < QA ? lq[ag < QA ? ag : 0] : 0;
+            *out = h;
+        }
+    } else {
+        if (lane == 0) {
+            out->gain = lg;
+            out->bin = lb;
+            out->feat = feat;
+        }
+        if (lb != NO_BIN) small_left<PACK>(A, Hs, nag, numeric, lb, lane, out, A.left_out + ((int64_t)q * nwg + jp) * nag);
+    }
+}
+
+// An oblivious level's row of one feature (grow_otree!, src/fit.jl:190-217), by one wavefront: the gains of the level's nodes added in
+// node order, zero where one of them is not positive, and the first maximum over the bins.
+__device__ __forceinline__ int small_obliv_best(const SmallArgs &A, const double *s_gain, int nact, int lane, double *gain) {
+    double bg = -INFINITY;
+    int bb = NO_BIN;
+    for (int b = lane; b < A.B; b += 64) {
+        double acc = 0.0;
+        bool allpos = true;
+        for (int s = 0; s < nact; s++) {
+            const double g = s_gain[s * A.B + b];
+            acc += g;
+            if (A.level > 1) allpos = allpos && g > 0.0;
+        }
+        const double v = allpos ? acc : 0.0;
+        if (v > bg) {
+            bg = v;
+            bb = b + 1;
+        }
+    }
+    wave_argmax(bg, bb);
+    *gain = bg;
+    return bb;
+}
+
+// SPLIT: a feature's rows are shared by `slices` blocks, which add their histograms into A.acc instead of searching them;
+// k_small_scan does that.  For inputs of few features, whose blocks would fill a part of the chip with long walks: 10 features in 25
+// slices take 0.4 us per 25k rows and channel pair where one block per feature takes 0.4 us per 1k, for 8 us more of launch and flush.
+template <int NAG, int BPL, bool PACK, bool SPLIT>
 __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
     extern __shared__ unsigned long long s_dyn[];
     __shared__ uint32_t s_dec[SMALL_MAX_NODES];
@@ -329,21 +423,28 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int B = A.B, N = A.N, level = A.level;
     const int nag = NAG ? NAG : A.NAg, na = NAG ? NAG - (PACK ? 1 : 0) : A.NA;
-    const bool writer = blockIdx.x == 0;
-    const int jp = blockIdx.x;
+    int jp = blockIdx.x, slice = 0;
+    if (SPLIT) { // blocks go to the 8 XCDs in turn: each takes a run of slices with all their features, whose rows' gradients then share its L2
+        const int L = (int)(blockIdx.y * gridDim.x + blockIdx.x), T = (int)(gridDim.x * gridDim.y), xcd = L & 7, rest = T & 7;
+        const int at = xcd * (T >> 3) + (xcd < rest ? xcd : rest) + (L >> 3);
+        slice = at / (int)gridDim.x;
+        jp = at - slice * (int)gridDim.x;
+    }
+    const bool writer = jp == 0 && slice == 0;
     const int first = 1 << (level - 1), nlev = first;
     long long *s_tot = reinterpret_cast<long long *>(s_dyn);                         // [nlev][nag]
     double *s_gain = reinterpret_cast<double *>(s_tot + (level > 1 ? nlev * nag : 0)); // oblivious: [slots][B]
-    unsigned long long *H = reinterpret_cast<unsigned long long *>(s_gain + (A.oblivious ? A.slots * B : 0)); // [slots][na][B]
+    unsigned long long *H = reinterpret_cast<unsigned long long *>(s_gain + (A.oblivious && !SPLIT ? A.slots * B : 0)); // [slots][na][B]
     const uint32_t fw = A.feat[jp];
-    const int f = (int)(fw & 0xFFFFu), constraint = (int)(fw >> 17) - 1;
+    const int f = (int)(fw & 0xFFFFu);
     const bool numeric = (fw & SMALL_NUMERIC) != 0;
     if (tid == 0) s_cnt = 0;
     const uint8_t *col = A.xcm + (size_t)f * N;
     // A thread takes U groups of 4 neighbouring rows at a time (the last group of all starts at N - 4 and leaves out what others
     // have); what the first of them need is requested before the decisions.
     constexpr int U = (NAG == 2 && PACK && BPL < 4) ? 2 : 1, GA = NAG ? NAG - (PACK ? 1 : 0) : 1;
-    const int ngroups = (N + 3) >> 2;
+    const int allgroups = (N + 3) >> 2, per = SPLIT ? (allgroups + A.slices - 1) / A.slices : allgroups;
+    const int gfirst = SPLIT ? slice * per : 0, ngroups = SPLIT && gfirst + per < allgroups ? gfirst + per : allgroups; // the block's: gfirst .. ngroups
     uint32_t nid[U][4], xb[U];
     unsigned long long g[GA][U][4];
     auto request = [&](int k0) {
@@ -377,7 +478,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
             }
         }
     };
-    request(tid);
+    request(gfirst + tid);
     if (level > 1) {
         const int np = nlev >> 1;
         for (int p = wave; p < np; p += 16) small_decide(A, p, s_dec, s_tot, writer, lane);
@@ -443,7 +544,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
                         z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
                         z ^= z >> 31;
                         m = (uint32_t)(z >> (8 * ((r + i) & 7))) & 0xFFu;
-                        if (writer) A.mask[r + i] = (uint8_t)m;
+                        if (jp == 0) A.mask[r + i] = (uint8_t)m;
                     }
                     nid[u][i] = (A.sampled && m > (uint32_t)A.cond) ? 1u | SMALL_OUT : 1u;
                 }
@@ -457,7 +558,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
                 for (int i = 0; i < 4; i++) nid[u][i] = row_moves(nid[u][i], d[i], b[i]);
             }
             // every block has the same ids: each writes a share (a wavefront's 256 rows; rows of the last group twice, alike)
-            if (base == 0 && (k >> 6) % (int)gridDim.x == (int)blockIdx.x)
+            if (base == 0 && (k >> 6) % (int)gridDim.x == jp)
 #pragma unroll
                 for (int i = 0; i < 4; i++) A.nid_out[r + i] = nid[u][i];
 #pragma unroll
@@ -485,99 +586,44 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
     int ns = nact < A.slots ? nact : A.slots;
     for (int i = tid; i < ns * na * B; i += 1024) H[i] = 0ull;
     __syncthreads();
-    take(tid, 0, ns);
+    take(gfirst + tid, 0, ns);
     for (int base = 0; base == 0 || base < nact; base += A.slots) {
         if (base > 0) {
             ns = nact - base < A.slots ? nact - base : A.slots;
             for (int i = tid; i < ns * na * B; i += 1024) H[i] = 0ull;
             __syncthreads();
         }
-        for (int k0 = base > 0 ? tid : tid + 1024 * U; k0 < ngroups; k0 += 1024 * U) {
+        for (int k0 = gfirst + tid + (base > 0 ? 0 : 1024 * U); k0 < ngroups; k0 += 1024 * U) {
             request(k0);
             take(k0, base, ns);
         }
         __syncthreads();
-        for (int s = wave; s < ns; s += 16) {
-            const int q = s_node[base + s], n = first + q;
-            const unsigned long long *Hs = H + (size_t)s * na * B;
-            long long *hout = A.hist + (int64_t)(n - 1) * A.node_stride + (int64_t)jp * nag * B;
-            double lg = -INFINITY;
-            int lb = NO_BIN;
-            constexpr int QA = NAG ? NAG : 1;
-            long long tq[QA], lq[QA];
-#pragma unroll
-            for (int ag = 0; ag < QA; ag++) lq[ag] = 0;
-            small_scan<NAG, BPL, PACK>(A, Hs, level > 1 ? s_tot + q * nag : nullptr, numeric, constraint, lane, hout, tq,
-                                       [&](int b, bool ok, double gain, const long long *left) {
-                if (A.oblivious) {
-                    if (b < B) s_gain[s * B + b] = gain; // update_gains!
-                } else if (ok && gain > lg) {
-                    lg = gain;
-                    lb = b + 1;
-                    if constexpr (NAG != 0) {
-#pragma unroll
-                        for (int ag = 0; ag < QA; ag++) lq[ag] = left[ag];
-                    }
-                }
-            });
-            if (level == 1 && writer) { // the root's totals, for the kernels below
-                if constexpr (NAG != 0) {
-                    if (lane == 0)
-#pragma unroll
-                        for (int ag = 0; ag < QA; ag++) A.node_sum[(int64_t)n * nag + ag] = tq[ag];
+        if constexpr (SPLIT) {
+            for (int i = tid; i < ns * na * B; i += 1024) {
+                const unsigned long long w = H[i];
+                if (w == 0ull) continue;
+                const int s = i / (na * B), rest = i - s * na * B, a = rest / B, b = rest - a * B;
+                unsigned long long *to = reinterpret_cast<unsigned long long *>(A.acc) + ((size_t)s_node[base + s] * A.nfs + jp) * nag * B + b;
+                if (PACK && a == 0) {
+                    const long long sum = (long long)w >> EVT_PACK_CNT_BITS;
+                    if (sum != 0) atomicAdd(to, (unsigned long long)sum);
+                    atomicAdd(to + (size_t)(nag - 1) * B, w & ((1ull << EVT_PACK_CNT_BITS) - 1ull));
                 } else {
-                    for (int ag = 0; ag < nag; ag++) {
-                        long long t = 0;
-                        for (int b = lane; b < B; b += 64) t += channel_of<PACK>(Hs, B, nag, ag, b);
-                        t = wave_sum_i64(t);
-                        if (lane == 0) A.node_sum[(int64_t)n * nag + ag] = t;
-                    }
+                    atomicAdd(to + (size_t)a * B, w);
                 }
             }
-            if (A.oblivious) continue;
-            wave_argmax(lg, lb);
-            SmallHead *out = A.head_out + (int64_t)q * gridDim.x + jp;
-            if constexpr (NAG != 0) { // the lane that holds the winning bin has the totals left of it
-                if (lane == (lb != NO_BIN ? (lb - 1) / BPL : 0)) {
-                    SmallHead h;
-                    h.gain = lg;
-                    h.bin = lb;
-                    h.feat = numeric ? f + 1 : -(f + 1);
-#pragma unroll
-                    for (int ag = 0; ag < EVT_MAX_NA + 1; ag++) h.left[ag] = ag < QA ? lq[ag < QA ? ag : 0] : 0;
-                    *out = h;
-                }
-            } else {
-                if (lane == 0) {
-                    out->gain = lg;
-                    out->bin = lb;
-                    out->feat = numeric ? f + 1 : -(f + 1);
-                }
-                if (lb == NO_BIN) continue;
-                small_left<PACK>(A, Hs, nag, numeric, lb, lane, out, A.left_out + ((int64_t)q * gridDim.x + jp) * nag);
-            }
+        } else
+        for (int s = wave; s < ns; s += 16) {
+            const int q = s_node[base + s];
+            small_search<NAG, BPL, PACK>(A, H + (size_t)s * na * B, q, jp, A.nfs, fw, level > 1 ? s_tot + q * nag : nullptr, writer,
+                                         A.oblivious ? s_gain + s * B : nullptr, lane);
         }
         __syncthreads();
     }
-    if (A.oblivious) { // all active nodes are in LDS: the feature's row of the level matrix, then its first maximum (grow_otree!, src/fit.jl:190-217)
+    if (A.oblivious && !SPLIT) { // all active nodes are in LDS: the feature's row of the level matrix, then its first maximum (grow_otree!, src/fit.jl:190-217)
         if (wave == 0) {
-            double bg = -INFINITY;
-            int bb = NO_BIN;
-            for (int b = lane; b < B; b += 64) {
-                double acc = 0.0;
-                bool allpos = true;
-                for (int s = 0; s < nact; s++) {
-                    const double g = s_gain[s * B + b];
-                    acc += g;
-                    if (level > 1) allpos = allpos && g > 0.0;
-                }
-                const double v = allpos ? acc : 0.0;
-                if (v > bg) {
-                    bg = v;
-                    bb = b + 1;
-                }
-            }
-            wave_argmax(bg, bb);
+            double bg;
+            const int bb = small_obliv_best(A, s_gain, nact, lane, &bg);
             if (lane == 0) s_best = bb;
             for (int s = lane; s < nact; s += 64) {
                 SmallHead *out = A.head_out + (int64_t)s_node[s] * gridDim.x + jp;
@@ -593,15 +639,77 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
             small_left<PACK>(A, H + (size_t)s * na * B, nag, numeric, lb, lane, A.head_out + at, A.left_out + at * nag);
         }
     }
-    if (writer) { // rows of the level: the root's is the size of the sample
+    if (jp == 0) { // rows of the level: the root's is the size of the sample
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) counted += __shfl_xor(counted, o);
         if (lane == 0) atomicAdd(&s_cnt, counted);
         __syncthreads();
-        if (tid == 0) {
+        if (tid == 0 && SPLIT) A.counts[level * 256 + slice] = s_cnt; // added up by k_small_final
+        if (tid == 0 && !SPLIT) {
             A.stats[level] = s_cnt;
             if (level == 1) A.stats[0] = s_cnt;
         }
+    }
+}
+
+// The searches of a level whose histograms the slices of k_small_level<SPLIT> left in A.acc: a wavefront per (node, feature), 16 nodes of one
+// feature to a block (all of them for an oblivious level, whose nodes' gains meet in LDS).
+template <int NAG, int BPL>
+__global__ __launch_bounds__(1024) void k_small_scan(SmallArgs A) {
+    extern __shared__ double s_gain[]; // oblivious: [active nodes][B]
+    __shared__ uint16_t s_node[SMALL_MAX_NODES];
+    __shared__ int s_nact, s_best;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int B = A.B, nag = NAG ? NAG : A.NAg, jp = blockIdx.x, first = 1 << (A.level - 1);
+    const uint32_t fw = A.feat[jp];
+    auto of = [&](int q) { return A.acc + ((size_t)q * A.nfs + jp) * nag * B; };
+    auto search = [&](int q, double *gain) {
+        small_search<NAG, BPL, false>(A, reinterpret_cast<const unsigned long long *>(of(q)), q, jp, A.nfs, fw,
+                                      A.level > 1 ? A.node_sum + (int64_t)(first + q) * nag : nullptr, jp == 0, gain, lane);
+    };
+    auto clear = [&](int q) {
+        for (int i = lane; i < nag * B; i += 64) of(q)[i] = 0;
+    };
+    if (!A.oblivious) {
+        const int q = (int)blockIdx.y * 16 + wave;
+        if (q >= first || A.status[first + q] != ST_BUILD) return;
+        search(q, nullptr);
+        clear(q);
+        return;
+    }
+    if (wave == 0) {
+        int base = 0;
+        for (int q0 = 0; q0 < first; q0 += 64) {
+            const bool on = q0 + lane < first && A.status[first + q0 + lane] == ST_BUILD;
+            const unsigned long long m = __ballot(on);
+            if (on) s_node[base + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)(q0 + lane);
+            base += __popcll(m);
+        }
+        if (lane == 0) s_nact = base;
+    }
+    __syncthreads();
+    const int nact = s_nact;
+    for (int s = wave; s < nact; s += 16) search(s_node[s], s_gain + s * B);
+    __syncthreads();
+    const bool numeric = (fw & SMALL_NUMERIC) != 0;
+    if (wave == 0) {
+        double bg;
+        const int bb = small_obliv_best(A, s_gain, nact, lane, &bg);
+        if (lane == 0) s_best = bb;
+        for (int s = lane; s < nact; s += 64) {
+            SmallHead *out = A.head_out + (int64_t)s_node[s] * A.nfs + jp;
+            out->gain = bg;
+            out->bin = bb;
+            out->feat = numeric ? (int)(fw & 0xFFFFu) + 1 : -((int)(fw & 0xFFFFu) + 1);
+        }
+    }
+    __syncthreads();
+    const int lb = s_best;
+    for (int s = wave; s < nact; s += 16) {
+        const int q = s_node[s];
+        const int64_t at = (int64_t)q * A.nfs + jp;
+        small_left<false>(A, reinterpret_cast<const unsigned long long *>(of(q)), nag, numeric, lb, lane, A.head_out + at, A.left_out + at * nag);
+        clear(q);
     }
 }
 
@@ -623,59 +731,93 @@ __global__ __launch_bounds__(1024) void k_small_final(SmallArgs A) {
         const uint32_t d = row_decision(A, nid, s_dec);
         A.nidx[r] = row_moves(nid, d, decision_bin(A, d, r)) & ~SMALL_OUT;
     }
-    if (writer)
-        for (int64_t i = tid; i < A.blob_n; i += 1024) A.blob_dst[i] = A.blob_src[i];
+    if (!writer) return;
+    if (A.slices > 1) {
+        for (int l = 1 + wave; l < A.level; l += 16) {
+            int t = 0;
+            for (int y = lane; y < A.slices; y += 64) t += A.counts[l * 256 + y];
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
+            if (lane == 0) {
+                A.stats[l] = t;
+                if (l == 1) A.stats[0] = t;
+            }
+        }
+        __syncthreads();
+    }
+    for (int64_t i = tid; i < A.blob_n; i += 1024) A.blob_dst[i] = A.blob_src[i];
 }
 
-static size_t small_lds(const evt_ctx *c, int level, int slots) {
+static size_t small_lds(const evt_ctx *c, int level, int slots, bool split) {
     const size_t tot = level > 1 ? (size_t)(1 << (level - 1)) * c->NAg * 8 : 0;
-    const size_t gain = c->tree_type == EVT_TREE_OBLIVIOUS ? (size_t)slots * c->B * 8 : 0;
+    const size_t gain = c->tree_type == EVT_TREE_OBLIVIOUS && !split ? (size_t)slots * c->B * 8 : 0;
     return tot + gain + (size_t)slots * c->NA * c->B * 8;
 }
 // histograms a block's LDS holds at the deepest level that splits
-static int small_slots(const evt_ctx *c) {
+static int small_slots(const evt_ctx *c, bool split) {
     const int nodes = 1 << std::max(0, c->D - 2);
-    const size_t fixed = small_lds(c, c->D - 1, 0), one = small_lds(c, c->D - 1, 1) - fixed;
+    const size_t fixed = small_lds(c, c->D - 1, 0, split), one = small_lds(c, c->D - 1, 1, split) - fixed;
     const size_t budget = 144 * 1024;
     if (fixed > 32 * 1024) return 0;
     return (int)std::min<size_t>((size_t)nodes, (budget - fixed) / one);
 }
 
-static int small_tree_buffers(evt_ctx *c) {
-    if (c->small_nid[1]) return EVT_OK;
+static size_t small_acc_bytes(const evt_ctx *c) { return (size_t)(1 << (c->D - 2)) * std::min(c->F, 256) * c->NAg * c->B * 8; }
+
+static int small_tree_buffers(evt_ctx *c, bool split) {
     const size_t cand = (size_t)(1 << (c->D - 2)) * std::min(c->F, 256);
-    for (int k = 0; k < 2; k++) {
+    for (int k = 0; k < 2 && !c->small_nid[1]; k++) {
         c->small_head[k] = dev_take(sizeof(SmallHead) * cand);
         if (c->NK > EVT_MAX_NA) c->small_left[k] = static_cast<long long *>(dev_take(sizeof(long long) * cand * c->NK));
         c->small_nid[k] = static_cast<uint32_t *>(dev_take(sizeof(uint32_t) * (size_t)c->N));
         if (!c->small_head[k] || !c->small_nid[k] || (c->NK > EVT_MAX_NA && !c->small_left[k])) return EVT_ERR_NOMEM;
     }
+    if (split && !c->small_acc) {
+        // the counts of the slices' rows, then the sums, for the larger of the weight modes
+        const size_t bytes = 16 * 256 * sizeof(int) + small_acc_bytes(c) / c->NAg * c->NK;
+        c->small_acc = static_cast<uint8_t *>(dev_take(bytes));
+        if (!c->small_acc) return EVT_ERR_NOMEM;
+        const int r = launch_fill_bytes(c, c->small_acc, (int64_t)bytes);
+        if (r != EVT_OK) return r;
+    }
     return EVT_OK;
 }
 
-// Inputs that take this path.  A block walks all rows once per level (and once more for every `slots` nodes), so a level grows with the
-// rows, the channels and - through the candidates every block reads and the searches its 16 wavefronts share - the nodes, where the
-// other path spreads the rows over the chip and pays for its launches.  Estimates in microseconds, fitted to rounds of 1k to 65k rows,
-// 10 and 60 features, depths 5 to 9, 1 to 14 channels, that both paths grew: mse of depth 6 on 10 features 109 against 61 us per round at
-// 4k rows, 125 against 118 at 32k; 60 features 160 against 62 and 165 against 118; 7 classes of depth 5 182 against 143 at 4k, 201 against 255 at 16k.
-bool small_tree_applies(const evt_ctx *c, int nfs, bool all_rows) {
-    if (!c->small_tree || c->D < 2 || c->D > 10 || nfs > 256 || c->N < 4 || c->N > 65535 || !c->defer_pred || EVT_IS_QUANTILE(c->loss)) return false;
-    if (c->record_nidx && !all_rows) return false;
+// Which form a tree takes: 0 the kernels of larger inputs, 1 one kernel per level, S > 1 two kernels per level with a feature's rows
+// shared by S blocks.  A block walks its rows once per level (and once more for every `slots` nodes), so a level grows with
+// rows / S, the channels and - through the candidates every block reads and the searches its 16 wavefronts share - the nodes; slices
+// add a launch and the words they flush.  The other path spreads rows of any number over the chip and pays for its launches.  Estimates
+// in microseconds, fitted to rounds that each of them grew (4k to 250k rows, 10 and 60 features, depths 5 to 9, 1 to 14 channels).
+// mse of depth 6, microseconds per round of the other path, S = 1 and S > 1: 10 features 119, 63, 74 at 4k rows, 126, 119, 77 at
+// 32k, 128, -, 83 at 120k, 133, -, 93 at 250k; 60 features 156, 63, 76 at 4k, 168, -, 133 at 120k, 181, -, 206 at 250k.
+// 7 classes of depth 5 on 10 features: 183, 145, 161 at 4k, 229, 902, 191 at 65k, 279, -, 331 at 250k.
+int small_tree_form(const evt_ctx *c, int nfs, bool all_rows) {
+    if (!c->small_tree || c->D < 2 || c->D > 10 || nfs > 256 || c->N < 4 || c->N > (1 << 24) || !c->defer_pred || EVT_IS_QUANTILE(c->loss)) return 0;
+    if (c->record_nidx && !all_rows) return 0;
     const bool obliv = c->tree_type == EVT_TREE_OBLIVIOUS;
-    const int nodes = 1 << (c->D - 2), slots = small_slots(c);
-    if (slots < 1 || (obliv && slots < nodes)) return false;
-    if (c->small_tree > 1) return true;
-    const double per_1k_rows = c->mc ? 0.3 + 0.2 * c->NA : 0.33 + 0.065 * c->NA;
-    double here = 0.0;
+    const int nodes = 1 << (c->D - 2), slots = small_slots(c, false), slots_split = small_slots(c, true);
+    const int S = std::max(2, 256 / nfs);
+    const bool can1 = c->N <= 65535 && slots >= 1 && (!obliv || slots == nodes);
+    const bool canS = slots_split >= 1 && c->N / S < 65000 && small_acc_bytes(c) <= ((size_t)64 << 20) && (!obliv || (size_t)nodes * c->B * 8 <= 144 * 1024);
+    if (c->small_tree == 2) return can1 ? 1 : 0;
+    if (c->small_tree == 3) return canS ? S : 0;
+    const double k = 1e-3 * c->N, per_1k = c->mc ? 0.3 + 0.2 * c->NA : 0.3 + 0.055 * c->NA;
+    double one = 0.0, split = 0.0;
     for (int l = 1; l < c->D; l++) {
-        const int n = (int)std::min<int64_t>(1 << (l - 1), c->N);
-        here += 5.0 + 3.5 * ((n + 15) / 16) + per_1k_rows * 1e-3 * c->N * ((n + slots - 1) / slots);
+        const int n = (int)std::min<int64_t>(1 << (l - 1), c->N), searches = (n + 15) / 16;
+        one += 5.0 + 3.5 * searches + per_1k * k * ((n + slots - 1) / std::max(1, slots));
+        split += (c->mc ? 18.0 : 11.0) + 2.5 * searches + per_1k * k / S * ((n + slots_split - 1) / std::max(1, slots_split)) +
+                 (double)std::min<int64_t>((int64_t)n * c->B, c->N / S) * c->NA * nfs * S / 141e3; // words flushed: no more than rows
     }
-    return here < (c->D - 1) * (18.0 + (nfs > 16 ? 9.0 : 0.0) + 3.0 * std::min(c->NA, 8) + (obliv ? 5.0 : 0.0));
+    const double launches = c->mc ? 16.0 + 0.8 * c->NA + (nfs > 16 ? 7.0 : 0.0) : 18.0 + 3.0 * std::min(c->NA, 8) + (nfs > 16 ? 9.0 : 0.0);
+    const double other = (c->D - 1) * (launches + (obliv ? 5.0 : 0.0) + 0.0068 * c->NA * k);
+    if (can1 && one < other && (!canS || one <= split)) return 1;
+    return canS && split < other ? S : 0;
 }
 
-int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw) {
-    int r = small_tree_buffers(c);
+int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
+    const bool split = slices > 1;
+    int r = small_tree_buffers(c, split);
     if (r != EVT_OK) return r;
     SmallArgs A;
     memset((void *)&A, 0, sizeof(A));
@@ -704,7 +846,10 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw) {
     A.seed = c->mask_seed;
     A.N = (int)c->N; A.F = c->F; A.B = c->B; A.K = c->K; A.NK = c->NK; A.NAg = c->NAg; A.NA = c->NA; A.loss = c->loss; A.D = c->D; A.nnodes = c->nnodes;
     A.nfs = c->n_js_last;
-    A.slots = small_slots(c);
+    A.slots = small_slots(c, split);
+    A.slices = slices;
+    A.counts = reinterpret_cast<int *>(c->small_acc);
+    A.acc = reinterpret_cast<long long *>(c->small_acc + 16 * 256 * sizeof(int));
     A.oblivious = c->tree_type == EVT_TREE_OBLIVIOUS ? 1 : 0;
     A.sampled = c->step.all_rows ? 0 : 1;
     A.draw = draw ? 1 : 0;
@@ -733,16 +878,26 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw) {
         const int nodes = 1 << (level - 1), slots = std::min(A.slots, nodes);
         const int most = A.slots;
         A.slots = slots;
-        const size_t lds = small_lds(c, level, slots);
+        const size_t lds = small_lds(c, level, slots, split), gain = A.oblivious ? (size_t)nodes * c->B * 8 : 0;
         prof_begin(c, level == 1 ? EVT_K_HIST : EVT_K_PARTITION, level); // below the root it moves rows, builds and searches at once
 #define SMALL3(NAG_, BPL_, PACK_)                                                                                                                  \
     {                                                                                                                                              \
         static EvtDevOnce once;                                                                                                                    \
         if (once.pending(c->device)) {                                                                                                             \
-            HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_small_level<NAG_, BPL_, PACK_>), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024)); \
+            for (const void *k : {reinterpret_cast<const void *>(k_small_level<NAG_, BPL_, PACK_, false>),                                         \
+                                  reinterpret_cast<const void *>(k_small_level<NAG_, BPL_, PACK_, true>), reinterpret_cast<const void *>(k_small_scan<NAG_, BPL_>)}) \
+                HIPCHK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));                                            \
             once.mark(c->device);                                                                                                                  \
         }                                                                                                                                          \
-        hipLaunchKernelGGL((k_small_level<NAG_, BPL_, PACK_>), dim3((unsigned)c->n_js_last), dim3(1024), lds, c->stream, A);                       \
+        const unsigned nf = (unsigned)c->n_js_last;                                                                                                \
+        if (!split) {                                                                                                                              \
+            hipLaunchKernelGGL((k_small_level<NAG_, BPL_, PACK_, false>), dim3(nf), dim3(1024), lds, c->stream, A);                                \
+        } else {                                                                                                                                   \
+            hipLaunchKernelGGL((k_small_level<NAG_, BPL_, PACK_, true>), dim3(nf, (unsigned)slices), dim3(1024), lds, c->stream, A);               \
+            prof_end(c);                                                                                                                           \
+            prof_begin(c, EVT_K_SCAN, level);                                                                                                      \
+            hipLaunchKernelGGL((k_small_scan<NAG_, BPL_>), dim3(nf, A.oblivious ? 1u : (unsigned)((nodes + 15) / 16)), dim3(1024), gain, c->stream, A); \
+        }                                                                                                                                          \
     }
 #define SMALL2(NAG_, PACK_)             \
     if (bpl == 1) SMALL3(NAG_, 1, PACK_) \

@@ -1,4 +1,4 @@
-"""One kernel per level (option "small_tree" = 2) against the histogram / search / partition kernels (= 0): trees, histograms, node ids,
+"""One and two kernels per level (option "small_tree" = 2 and 3) against the histogram / search / partition kernels (= 0): trees, histograms, node ids,
 gradients and predictions over free-running rounds, bit for bit, at the edges of what that path takes."""
 import numpy as np
 import pytest
@@ -26,6 +26,8 @@ pytestmark = pytest.mark.gpu
     (2047, 8, 200, 6, "mlogloss", dict(K=3, weights=True, sub="mask", cat=True)),
     (1500, 5, 64, 4, "mlogloss", dict(K=16, oblivious=True)),
     (1200, 6, 64, 5, "mlogloss", dict(K=2)),
+    (150_001, 3, 64, 6, "mse", dict(sub="drawn")),                   # more rows than one block per feature takes
+    (70_001, 12, 40, 5, "gaussian_mle", dict(oblivious=True, weights=True)),
 ])
 def test_one_kernel_per_level_changes_nothing(evt, N, F, B, D, loss, more):
     rng = np.random.default_rng(N)
@@ -45,7 +47,7 @@ def test_one_kernel_per_level_changes_nothing(evt, N, F, B, D, loss, more):
     masks = [rng.integers(0, 256, N, dtype=np.uint8) for _ in range(R)]
     gp = evt.make_params(eta=0.4, min_weight=0.0 if N < 10 else 2.0, L2=1.0)
     out = []
-    for small in (2, 0):
+    for small in (2, 3, 0):
         h = evt.Handle(N, F, B, len(mu), D, loss, "oblivious" if more.get("oblivious") else "binary")
         h.set_option("small_tree", small)
         h.set_xbin(x_bin)
@@ -68,10 +70,11 @@ def test_one_kernel_per_level_changes_nothing(evt, N, F, B, D, loss, more):
         h.close()
         out.append(rec)
     splits = 0
-    for a, b in zip(*out):
+    for a, a2, b in zip(*out):
         if isinstance(a, np.ndarray):
-            assert a.tobytes() == b.tobytes()
+            assert a.tobytes() == b.tobytes() and a2.tobytes() == b.tobytes()
         else:
             assert_tree_bits(a, b)
+            assert_tree_bits(a2, b)
             splits += int(a.split.sum())
     assert splits > 0 or N < 10
