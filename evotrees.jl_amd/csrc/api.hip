@@ -290,6 +290,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->hist_threads = 1024;
     c->hist_min_rows = 1024;
     c->hist_variant = 0;
+    c->hist_tile = 0;
     c->scan_fused = 1;
     c->hist_in_scatter = 1;
     c->small_tree = 1;
@@ -1824,6 +1825,9 @@ extern "C" int evt_set_option(evt_handle c, const char *name, int64_t value) {
         ARGCHK(value >= 0 && value <= 2, "hist_variant must be 0 (auto), 1 (generic) or 2 (conflict-free where it applies)");
         ARGCHK(value != 1 || c->LPR <= 64, "hist_variant 1: the generic histogram kernel takes records of up to 1024 bytes");
         c->hist_variant = (int)value;
+    } else if (strcmp(name, "hist_tile") == 0) {
+        ARGCHK(value == 0 || (value >= 16 && value <= 512 && (value & (value - 1)) == 0), "hist_tile must be 0 (auto) or a power of two in [16, 512]");
+        c->hist_tile = (int)value;
     } else if (strcmp(name, "bit_planes") == 0) {
         ARGCHK(value == 0 || value == 1, "bit_planes must be 0 or 1");
         c->use_planes = (int)value;

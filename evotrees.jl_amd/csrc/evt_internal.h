@@ -182,7 +182,7 @@ struct evt_ctx {
     bool last_all_rows;
 
     // tunables
-    int hist_blocks, hist_threads, hist_min_rows, hist_seg_cost;
+    int hist_blocks, hist_threads, hist_min_rows, hist_seg_cost, hist_tile;
     int hist_variant;  // 0 auto, 1 generic 16-byte-piece kernel, 2 conflict-free 8-byte-piece kernel where it applies
     int scan_fused;    // option: the split search of a node with at most 16 sampled features runs in one kernel
     int small_tree;    // option: one kernel per level (kernels_small.hip) - 0 never, 1 for inputs of few rows, 2 wherever it can, 3 the form of two kernels per level wherever it can

@@ -38,6 +38,7 @@ struct HistArgs {
     int RS, LPR, RPW, F, nfs, B, NAg, level;
     int NSL; // conflict-free kernel: lanes per row, the power of two >= 16 that covers a column tile's pieces
     int TW;  // conflict-free kernel: bytes of a record one block column (blockIdx.y) takes - a column tile
+    int lay_sh, lay_pu; // record layout: byte p holds feature (p >> lay_sh) * lay_pu + p % 2^lay_sh while the remainder is below lay_pu
     int slots_per_tile;
     int min_rows;
     int seg_cost;
@@ -316,9 +317,11 @@ __device__ __forceinline__ uint2 load_piece(const uint8_t *p) {
     } else if constexpr (PB == 4) {
         const uint32_t *q = reinterpret_cast<const uint32_t *>(p);
         return make_uint2(NT ? __builtin_nontemporal_load(q) : *q, 0u);
-    } else {
+    } else if constexpr (PB == 2) {
         const uint16_t *q = reinterpret_cast<const uint16_t *>(p);
         return make_uint2((uint32_t)(NT ? __builtin_nontemporal_load(q) : *q), 0u);
+    } else {
+        return make_uint2((uint32_t)(NT ? __builtin_nontemporal_load(p) : *p), 0u);
     }
 }
 template <bool NT>
@@ -339,7 +342,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
     const bool pk = GRP ? (A.pack && a0 == 0) : PACK; // channel 0 shares its word with the row count
     if (blockIdx.x == 0 && blockIdx.z == 0 && tid == 0) A.stats[A.level] = total - (int64_t)n_build * A.seg_cost;
 
-    static_assert(PB == 8 || PB == 4 || PB == 2, "a piece is 8, 4 or 2 bytes");
+    static_assert(PB == 8 || PB == 4 || PB == 2 || PB == 1, "a piece is 8, 4, 2 bytes or one");
     static_assert(PU >= 1 && PU <= PB, "features per piece");
     const int NS = A.NSL;         // lanes per row: one per piece of the record, idle ones beyond its last piece
     const int RPW = 64 / NS;      // rows per wave instruction
@@ -376,8 +379,10 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
             } else if constexpr (PB == 4) {
                 const uint2 q = *reinterpret_cast<const uint2 *>(A.jsmap + f0);
                 mw[0] = q.x; mw[1] = q.y;
-            } else {
+            } else if constexpr (PB == 2) {
                 mw[0] = *reinterpret_cast<const uint32_t *>(A.jsmap + f0);
+            } else {
+                mw[0] = A.jsmap[f0];
             }
         }
 #pragma unroll
@@ -520,7 +525,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
         // requested before the first is used, so a flush costs one LDS and one memory round trip, not FU of each
         constexpr int FU = 8;
         const bool all_feats = A.nfs == A.F; // slot of feature f is f itself
-        const int piece0 = tb / PB;          // first piece of this column tile
+        const int lay_sh = A.lay_sh, lay_pu = A.lay_pu, lay_mask = (1 << lay_sh) - 1;
         const bool pow2 = (nchunks & (nchunks - 1)) == 0; // decode with shifts
         const int ns_sh = __ffs(NS) - 1, nc_sh = __ffs(nchunks) - 1;
         for (int k0 = tid; k0 < nitems; k0 += FU * nthr) {
@@ -551,12 +556,13 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
                     const int t = rest % PU;
                     const int a = rest / PU;
                     const int b = chunk * 8 + bl;
-                    const int f = (piece0 + sidx) * PU + t; // the feature at byte t of the piece
+                    const int p = tb + sidx * PB + t;              // byte of the record
+                    const int f = (p >> lay_sh) * lay_pu + (p & lay_mask); // its feature, if it is no padding
                     if (b < B) {
                         hwv[j] = &H[(size_t)a * plane + ((size_t)t * B + b) * NS + sidx];
                         wv[j] = *hwv[j];
                         av[j] = a; bv[j] = b;
-                        if (f < A.F) slotv[j] = all_feats ? f : (int)A.jsmap[tb + sidx * PB + t]; // a padding byte's word has no slot
+                        if (f < A.F && (p & lay_mask) < lay_pu) slotv[j] = all_feats ? f : (int)A.jsmap[p]; // a padding byte's word has no slot
                     }
                 }
             }
@@ -595,6 +601,9 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
     }
 }
 
+// Bytes of a piece: 16 or more pieces cover a column tile of tw bytes.
+static int hist16_piece(int tw) { return tw >= 128 ? 8 : tw >> 4; }
+
 template <int NA, bool PACK, bool GRP, int U, int PB, int PU, bool NT>
 static int launch_hist16_q(evt_ctx *c, const HistArgs &A, dim3 grid, int threads, size_t lds) {
     // unpredicated atomics for every feature of the record pay off unless most features are left out: the words of
@@ -624,12 +633,12 @@ static int launch_hist16_t(evt_ctx *c, const HistArgs &A, dim3 grid, int threads
     // records larger in total than the last-level cache (256 MB) are streamed past it
     const bool nt = (size_t)c->N * c->RS > ((size_t)256 << 20);
     // (piece bytes, features per piece): a densely packed record has PU == PB, record_layout() picks the others
-    const int pb = A.TW >= 128 ? 8 : (A.TW == 64 ? 4 : 2);
-    const int pu = c->PU < c->PBL ? c->PU : pb;
+    const int pb = hist16_piece(A.TW);
+    const int pu = (c->PU < c->PBL && c->PU < pb) ? c->PU : pb;
 #define H16Q(PB_, PU_)                                                                                                     \
     if (pb == PB_ && pu == PU_)                                                                                            \
         return nt ? launch_hist16_q<NA, PACK, GRP, U, PB_, PU_, true>(c, A, grid, threads, lds) : launch_hist16_q<NA, PACK, GRP, U, PB_, PU_, false>(c, A, grid, threads, lds);
-    H16Q(8, 8) H16Q(8, 7) H16Q(8, 6) H16Q(8, 5) H16Q(4, 4) H16Q(4, 3) H16Q(2, 2)
+    H16Q(8, 8) H16Q(8, 7) H16Q(8, 6) H16Q(8, 5) H16Q(4, 4) H16Q(4, 3) H16Q(2, 2) H16Q(1, 1)
 #undef H16Q
     evt_set_error("no histogram kernel for pieces of %d bytes holding %d features", pb, pu);
     return EVT_ERR_INTERNAL;
@@ -645,6 +654,67 @@ static int launch_hist_t(evt_ctx *c, const HistArgs &A, dim3 grid, int threads, 
     hipExtLaunchKernelGGL((k_hist_build<NA, PACK, GRP>), grid, dim3(threads), (uint32_t)lds, c->stream, c->launch_e0, c->launch_e1, 0, A);
     HIPCHK(hipGetLastError());
     return EVT_OK;
+}
+
+// Launch shape of the conflict-free kernel: the bytes of a record that a block column takes (a tile) and the row spans.
+//
+// Every span adds a whole level's histogram into global memory, whatever the tile: the blocks' atomics drain at ~0.2 T/s, and with
+// one block per CU that takes whole records 256 spans flush (cfg2's features: 256 x 12 800 atomics, 16 of a launch's 33 us at 300k rows).
+// t tiles make 256 / t spans of the same 256 blocks: 1 / t of the atomics, against row ids and gradient words that
+// each tile reads again and narrower loads.  Few rows take narrow tiles, many rows whole records; a histogram of
+// many channels or bins takes fewer spans than there are CUs.  The estimate, in us, with the figures fitted to sweeps of 30k to 4M
+// rows a tree, 20 to 120 features, 1 to 15 channels, 32 to 255 bins and depths 5 to 11 (it picks the best or one within 8 % of it):
+//   8                                       launch, set-up, the first loads
+//   4.9e-6 * atomics of a span * spans      flush
+//   rows in millions * (max(3.2 * LDS adds of a row's 16 lanes, 18) + 3.5 * (tiles - 1)) * 256 / blocks of a layer
+// us per launch, whole records and 256 spans -> chosen: mse 100 features, 35k rows a launch 15.8 -> 10.4, 300k 33.5 -> 20.6, 600k 41.3 -> 29.7,
+// 2.2M 83 (whole records stay); logloss 28 features of 128 bins, 470k rows 30.2 -> 25.0; gaussian_mle 50 features, 140k rows
+// 32.8 -> 21.5; 7 classes, 30 features, 80k rows 36.4 -> 26.
+struct Hist16Shape {
+    int tw, pb, pu, ntiles;
+    size_t lds;
+    unsigned spans;
+};
+
+static bool choose_hist16(const evt_ctx *c, int level, int na, int layers, Hist16Shape *best) {
+    if (c->RS < 32 || c->hist_variant == 1) return false;
+    const bool spread = c->PU < c->PBL; // pieces of PBL bytes, PU features each (record_layout)
+    int tw = 32;
+    while (tw < c->RS && tw < 512) tw <<= 1;
+    // the root builds the sampled rows, a level below it the smaller children: at most half of them
+    const double sampled = c->last_all_rows ? 1.0 : (c->last_cond + 1) / 256.0;
+    const double rows = 1e-6 * (double)c->N * sampled * (level == 1 ? 1.0 : 0.4);
+    const double span_atomics = (double)c->n_js_last * c->B * c->NAg;
+    double least = 0;
+    bool found = false;
+    for (; tw >= 16; tw >>= 1) {
+        if (c->hist_tile > 0 && tw > c->hist_tile && tw > 16) continue;
+        if (found && (c->hist_tile > 0 || tw * 8 < c->RS)) break; // a set width, or more than eight tiles of a choice
+        Hist16Shape s;
+        s.tw = tw;
+        s.pb = hist16_piece(tw);
+        s.pu = (spread && c->PU < s.pb) ? c->PU : s.pb;
+        if (spread && s.pb > c->PBL) continue;
+        s.ntiles = (c->RS + tw - 1) / tw;
+        const int lanes = tw / s.pb;
+        s.lds = (size_t)na * c->B * lanes * s.pu * 8; // channels x bins x feature bytes of a tile, words
+        if (s.lds > 128 * 1024) continue;
+        if (tw == 16 && c->LPR > 64 && 2 * s.lds > 128 * 1024) break; // more than 1024 features whose 32-byte tiles do not fit are refused (launch_hist_build)
+        const double adds = 3.2 * s.pu * na * (lanes / 16) * s.ntiles;
+        const double per_row = (adds > 18 ? adds : 18) + 3.5 * (s.ntiles - 1);
+        int most = c->hist_blocks / (s.ntiles * layers);
+        if (most < 16) most = c->hist_blocks < 16 ? c->hist_blocks : 16;
+        for (int n = most; n >= 1 && (n == most || n >= 16) && 4 * n >= most; n >>= 1) {
+            const double us = 8 + 4.9e-6 * span_atomics * n + rows * per_row * 256 / ((double)n * s.ntiles);
+            if (!found || us < least) {
+                s.spans = (unsigned)n;
+                *best = s;
+                least = us;
+                found = true;
+            }
+        }
+    }
+    return found;
 }
 
 int launch_hist_build(evt_ctx *c, int level, const uint32_t *is_cur) {
@@ -698,29 +768,22 @@ int launch_hist_build(evt_ctx *c, int level, const uint32_t *is_cur) {
     A.slots_per_tile = slots_per_tile;
     const size_t lds = per_slot * slots_per_tile;
     dim3 grid((unsigned)blocks, (unsigned)ntiles, layers);
-    // conflict-free variant: a block column takes a tile of TW bytes of every record - the whole record when its LDS
-    // histogram fits, else the widest power of two that does (down to 32 bytes) - with 16, 32 or 64 lanes per row;
-    // lanes past the record's last piece idle.  (16-byte records as 1-byte pieces were measured: no faster than the
-    // generic kernel.)
-    int tw = 32;
-    while (tw < c->RS && tw < 512) tw <<= 1;
-    const bool spread = c->PU < c->PBL; // features spread over all pieces: one tile takes the whole record (record_layout)
-    while (!spread && tw > 32 && (size_t)na * c->B * tw * 8 > 128 * 1024) tw >>= 1;
-    const int pb16 = tw >= 128 ? 8 : (tw == 64 ? 4 : 2);
-    A.TW = tw;
-    A.NSL = tw / pb16;
-    const int ntiles16 = (c->RS + tw - 1) / tw;
-    const size_t lds16 = (size_t)na * c->B * A.NSL * (spread ? c->PU : pb16) * 8; // channels x bins x feature bytes of a tile, words
-    const bool can16 = c->RS >= 32 && lds16 <= 128 * 1024 && (!spread || (pb16 == c->PBL && ntiles16 == 1));
-    const bool use16 = (c->hist_variant == 1) ? false : can16;
+    // conflict-free variant: a block column takes a tile of TW bytes of every record, with 16, 32 or 64 lanes per row; lanes past the
+    // record's last piece idle.  (16-byte records as 1-byte pieces were measured: no faster than the generic kernel.)
+    Hist16Shape s16 = {};
+    const bool use16 = choose_hist16(c, level, na, (int)layers, &s16);
     if (!use16 && c->LPR > 64) { // the generic kernel reads a record with one wavefront instruction: 64 lanes of 16 bytes
         evt_set_error("%d accumulator channels x %d bins need the generic histogram kernel, which takes at most 1024 features", na, c->B);
         return EVT_ERR_ARG;
     }
-    // several block columns share the launch's blocks: the same number of LDS histograms is flushed per node
-    int64_t bx = blocks / ntiles16;
-    if (bx < 64) bx = blocks < 64 ? blocks : 64;
-    const dim3 grid16((unsigned)bx, (unsigned)ntiles16, layers);
+    const size_t lds16 = s16.lds;
+    if (use16) {
+        A.TW = s16.tw;
+        A.NSL = s16.tw / s16.pb;
+        A.lay_sh = __builtin_ctz((unsigned)c->PBL);
+        A.lay_pu = c->PU;
+    }
+    const dim3 grid16(use16 ? s16.spans : 1, use16 ? (unsigned)s16.ntiles : 1, layers);
 #define HCASE(NA_, PACK_, GRP_) \
     return use16 ? launch_hist16_t<NA_, PACK_, GRP_>(c, A, grid16, threads, lds16) : launch_hist_t<NA_, PACK_, GRP_>(c, A, grid, threads, lds)
     if (grouped) HCASE(EVT_HIST_GROUP, false, true);

@@ -396,6 +396,8 @@ int evt_get_profile(evt_handle h, int64_t *launches, double *ms, int64_t *units)
 int evt_reset_profile(evt_handle h);
 /* Options: "hist_blocks", "hist_threads", "hist_min_rows", "hist_seg_cost", "hist_variant" (launch shape,
  * work split and kernel variant of the histogram builder, for sweeps; results do not depend on them);
+ * "hist_tile" (bytes of a record that a block of the histogram kernel takes: 0, default: by an estimate on rows, features, channels and
+ * bins; 16 to 512, a power of two: that width or the next below it that fits; same trees and histograms, bit for bit);
  * "bit_planes" (1, default: before the first tree the library derives one bit plane per
  * (feature, bin threshold) from x_bin - F * (nbins - 1) * nobs / 8 bytes, taken only when that is at most 16 GiB and a third of the free
  * memory - and the row partition reads its decisions there; 0: it gathers bin bytes; same trees, bit for bit);
