@@ -184,7 +184,7 @@ extern "C" int evt_destroy(evt_handle c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     void *ptrs[] = {c->xcm, c->xrm, c->y, c->pred, c->grad, c->gq, c->is_a, c->is_b, c->nidx, c->mask, c->flagw, c->chunk_nleft, c->chunk_lpre,
                     c->hist, c->seg_start, c->seg_len, c->status, c->node_sum, c->tree_blob, c->tree.packed, c->js, c->jsmap, c->feattypes, c->mono, c->absmax, c->qexp_buf[0], c->qexp_buf[1], c->qbits,
-                    c->qscale_buf[0], c->qscale_buf[1], c->planes, c->metric_partial, c->errflag, c->ogains, c->sbest, c->is_id, c->pt_nodes, c->pt_pred, c->mask_next,
+                    c->qscale_buf[0], c->qscale_buf[1], c->planes, c->metric_partial, c->errflag, c->ogains, c->sbest, c->scan_count, c->is_id, c->pt_nodes, c->pt_pred, c->mask_next,
                     c->small_nid[0], c->small_nid[1], c->small_head[0], c->small_head[1], c->small_left[0], c->small_left[1], c->small_acc,
                     c->alphas, c->alphas_f, c->qkeys_a, c->qkeys_b, c->qtemp};
     if (c->copy_stream) (void)hipStreamSynchronize(c->copy_stream);
@@ -279,7 +279,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->n_alphas = 1;
     for (int k = 0; k < EVT_MAX_K; k++) c->h_alphas[k] = 0.5;
     c->qscale = nullptr; c->qexp_buf[0] = c->qexp_buf[1] = nullptr; c->qscale_buf[0] = c->qscale_buf[1] = nullptr; c->q_cur = c->q_tree = 0;
-    c->stats = nullptr; c->errflag = nullptr; c->ogains = nullptr; c->sbest = nullptr;
+    c->stats = nullptr; c->errflag = nullptr; c->ogains = nullptr; c->sbest = nullptr; c->scan_count = nullptr;
     c->h_stage = nullptr; c->h_stage_dev = nullptr; c->h_stage_bytes = 0; c->h_stage_base = nullptr; c->h_stage_dev_base = nullptr;
     c->n_js_last = 0;
     c->js_staged = false;
@@ -413,6 +413,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
         // one 64-byte candidate (ScanBestQ, kernels_scan.hip) per node and group of 4 features; oblivious: one of 16 bytes per block
         ALLOC(sb, std::max((size_t)c->maxlvl * ((c->F + 3) / 4) * 64, (size_t)EVT_OBLIV_BLOCKS * 16));
         c->sbest = sb;
+        ALLOC(c->scan_count, (size_t)c->maxlvl * EVT_SCAN_COUNT_STEP);
     }
     // pinned staging: tree read-back + small per-tree uploads
     c->h_stage_bytes = c->blob_bytes + (size_t)c->F * 4 + (size_t)c->RS * 2 + 1024;
@@ -432,6 +433,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->absmax, 0, sizeof(uint32_t) * 2 * EVT_ABSMAX_STRIPES * EVT_MC_MAX_NK, c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->nidx, 0, sizeof(uint32_t) * N, c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->errflag, 0, sizeof(int32_t), c->stream);
+    if (e2 == hipSuccess) e2 = hipMemsetAsync(c->scan_count, 0, sizeof(int32_t) * EVT_SCAN_COUNT_STEP * c->maxlvl, c->stream);
     if (e2 == hipSuccess) e2 = upload_alphas(c);
     int r = EVT_OK;
     if (e2 == hipSuccess) r = launch_iota(c, c->is_id, N);

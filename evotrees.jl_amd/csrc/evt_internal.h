@@ -45,6 +45,9 @@
 #define LH_TOTAL_BUILD 3 // build rows of the level + hist_seg_cost per build node
 #define LH_SIZE 8
 
+// split search: a node's block counter has a 128-byte line to itself (additions to one line follow each other, ~15 ns each)
+#define EVT_SCAN_COUNT_STEP 32
+
 struct LevelTab {
     int64_t *hdr;      // [LH_SIZE]
     int32_t *act_node; // active nodes in node (= position) order
@@ -158,6 +161,7 @@ struct evt_ctx {
     int64_t *stats;    // [D+1] rows built per level
     int32_t *errflag;  // device-side validation flag
     double *ogains;    // oblivious: [maxlvl][F][B]
+    int32_t *scan_count; // split search: blocks of a node that have handed in their candidate (kernels_scan.hip)
     void *sbest;       // split search: best candidate per (node of the level, feature group), 64 B each
 
     // host staging (pinned): two slots of h_stage_bytes each, so that a second tree can be queued before the first one

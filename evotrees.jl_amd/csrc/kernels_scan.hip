@@ -40,6 +40,8 @@ struct ScanArgs {
     double eta, lambda, L2, gamma, min_weight;
     int bagging;
     int nfs, B, F, K, NK, NAg, loss, level, leaf_level, oblivious, zero_children;
+    int32_t *counts; // last_decides: blocks of each node of the level that have handed in their candidate, zero between launches
+    int last_decides;
     int fold_leaves; // the level's children are leaves: their weight and values are written along with the split (no pass of their own)
     // the level's chunk descriptors, written here when no histogram kernel runs at this level (cdesc == nullptr: not here)
     const int64_t *hdr;
@@ -390,6 +392,71 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
             if (lane == b0 / BPL) write_children<NAG>(A, n, qL, s_Sq, s_sc);
         }
         if (A.zero_children) zero_children_slices<NAG>(A, n);
+    } else if (A.last_decides) {
+        // The node's blocks meet at a counter: each hands in its candidate with stores that go past its XCD's cache, and the one that
+        // comes last reads them all the same way and decides.  No block waits for another.  Bound by that chain (2 to 3 us: store, count,
+        // read) where a level has few nodes, by the histograms it reads and clears where it has many.  A second launch
+        // for the decision took 5 to 7 us and its gap: 100 features x 64 bins, two kernels -> one: 1 node 5.7 + 5.1 -> 7.4 us, 32 nodes
+        // 6.6 + 10.4 -> 9.4, 256 nodes 23.1 + 11.5 -> 28.7, 512 nodes 41.6 + 6.5 -> 46.1; 28 features x 128 bins 6.0 + 5.6 -> 7.8, 26.6 + 7.5 -> 31.0.
+        // (Counters side by side, 32 to a line: 500 features and 16 nodes 31 us, 14 with a line each.)
+        constexpr int CW = 3 + NAG; // words of a candidate: gain, position and bin, feature, totals
+        unsigned long long *cand = reinterpret_cast<unsigned long long *>(reinterpret_cast<ScanBestQ *>(A.sbest) + (int64_t)nodeidx * gridDim.y);
+        int last = 0;
+        if (tid == 0) {
+            unsigned long long w[CW];
+            w[0] = (unsigned long long)__double_as_longlong(bg);
+            w[1] = (unsigned int)bj | ((unsigned long long)(unsigned int)bb << 32);
+            w[2] = (unsigned int)s_wfeat[bw];
+#pragma unroll
+            for (int ag = 0; ag < NAG; ag++) w[3 + ag] = (unsigned long long)s_wq[bw][ag];
+#pragma unroll
+            for (int k = 0; k < CW; k++) __hip_atomic_store(cand + (size_t)blockIdx.y * 8 + k, w[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the candidate is in memory before it is counted
+            last = __hip_atomic_fetch_add(A.counts + (size_t)nodeidx * EVT_SCAN_COUNT_STEP, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.y - 1;
+        }
+        // the children's slices start from zero: a wave clears its feature's bins in both, whatever the node turns out to be
+        if (A.zero_children && have) {
+            long long *hc = A.hist + (int64_t)(2 * n - 1) * A.node_stride + o0;
+            for (int i = lane; i < NAG * B; i += 64) {
+                hc[i] = 0;
+                hc[A.node_stride + i] = 0;
+            }
+        }
+        if (wave != 0 || !__builtin_amdgcn_readfirstlane(last)) return;
+        asm volatile("" ::: "memory");
+        ScanBestQ mine;
+        mine.gain = -INFINITY; mine.jp = NO_BIN; mine.bin = NO_BIN; mine.feat = 1;
+        for (int g = lane; g < (int)gridDim.y; g += 64) { // ascending positions: only a strictly larger gain replaces an earlier one
+            unsigned long long w[CW];
+#pragma unroll
+            for (int k = 0; k < CW; k++) w[k] = __hip_atomic_load(cand + (size_t)g * 8 + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const double gg = __longlong_as_double((long long)w[0]);
+            if (gg > mine.gain) {
+                mine.gain = gg;
+                mine.jp = (int)(w[1] & 0xffffffffull);
+                mine.bin = (int)(w[1] >> 32);
+                mine.feat = (int)w[2];
+#pragma unroll
+                for (int ag = 0; ag < NAG; ag++) mine.qL[ag] = (long long)w[3 + ag];
+            }
+        }
+        double g = mine.gain;
+        int j = mine.jp;
+        wave_argmax(g, j); // highest gain, then the earliest feature, whose bin is already the lowest
+        const bool found = j != NO_BIN && g > A.gamma;
+        if (found ? (mine.jp == j) : (lane == 0)) {
+            A.counts[(size_t)nodeidx * EVT_SCAN_COUNT_STEP] = 0;
+            A.tree.w[n - 1] = (float)S[NK - 1];
+            const int feat = found ? (mine.feat < 0 ? -mine.feat : mine.feat) : 1;
+            scan_decide(A, n, S, s_dec, g, j, found ? mine.bin : NO_BIN, feat, found ? mine.feat > 0 : true);
+            if (found) {
+                if (A.level == 1) {
+#pragma unroll
+                    for (int ag = 0; ag < NAG; ag++) nsq[ag] = s_Sq[ag];
+                }
+                write_children<NAG>(A, n, mine.qL, nsq, sc);
+            }
+        }
     } else if (tid == 0) {
         ScanBestQ r;
         r.gain = bg; r.jp = bj; r.bin = bb;
@@ -400,7 +467,7 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
     }
 }
 
-// Pass 2: one block per node.  Leaf level: leaf value only.  Otherwise: arg-max over the feature
+// Pass 2 (leaf levels, and the search as two kernels): one block per node.  Leaf level: leaf value only.  Otherwise: arg-max over the feature
 // groups (first maximum: highest gain, then earliest feature, whose bin is already the lowest),
 // split iff gain > gamma; writes the Tree arrays, the children's totals (_child_sums!: left = bins
 // 1..bin of the parent histogram, or that bin alone for categorical features; right = parent - left,
@@ -967,6 +1034,8 @@ int launch_scan(evt_ctx *c, int level, const evt_params *p, bool leaf_level) {
     A.oblivious = (c->tree_type == EVT_TREE_OBLIVIOUS) ? 1 : 0;
     A.zero_children = (level + 1 < c->D) ? 1 : 0; // children at the last level never get a histogram
     A.fold_leaves = (!leaf_level && scan_folds_leaves(c) && level + 1 == c->D) ? 1 : 0;
+    A.counts = c->scan_count;
+    A.last_decides = 0;
     A.cdesc = nullptr;
     if (c->step.hist_fused && level > 1 && !leaf_level) {
         const LevelTab &L = c->lvl[level & 1];
@@ -997,6 +1066,7 @@ int launch_scan(evt_ctx *c, int level, const evt_params *p, bool leaf_level) {
     }
     // few sampled features: one block of 16 waves scans a node's features and finishes the node, no second launch
     const bool fused = !leaf_level && !A.oblivious && A.nfs <= 16 && c->scan_fused;
+    A.last_decides = !leaf_level && !A.oblivious && !fused && c->scan_fused ? 1 : 0;
 #define SCASE(NAG_)                                                                                     \
     case NAG_:                                                                                          \
         if (fused) {                                                                                    \
@@ -1010,7 +1080,7 @@ int launch_scan(evt_ctx *c, int level, const evt_params *p, bool leaf_level) {
             else if (bpl == 2) hipLaunchKernelGGL((k_scan<NAG_, 2, false>), grid, dim3(256), 0, c->stream, A); \
             else hipLaunchKernelGGL((k_scan<NAG_, 4, false>), grid, dim3(256), 0, c->stream, A);               \
         }                                                                                               \
-        if (!A.oblivious || leaf_level) hipLaunchKernelGGL(k_scan_fin<NAG_>, dim3(nodes, 1 + zero_blocks), dim3(256), 0, c->stream, A, ngroups); \
+        if (leaf_level || (!A.oblivious && !A.last_decides)) hipLaunchKernelGGL(k_scan_fin<NAG_>, dim3(nodes, 1 + zero_blocks), dim3(256), 0, c->stream, A, ngroups); \
         break;
     switch (c->NAg) {
         SCASE(2)
