@@ -823,6 +823,7 @@ __global__ __launch_bounds__(256) void k_scan_mc(ScanArgs A) {
     __shared__ double s_sc[EVT_MC_MAX_NK];
     __shared__ double s_wg[4];
     __shared__ int s_wjp[4], s_wbin[4];
+    __shared__ int s_last;
 
     node_totals_mc(A, n, hn, blockIdx.y == 0, s_Sq, s_S, s_sc);
     double gain_p = 0.0;
@@ -905,9 +906,77 @@ __global__ __launch_bounds__(256) void k_scan_mc(ScanArgs A) {
         for (int w = 0; w < nwaves; w++) {
             if (s_wg[w] > bg || (s_wg[w] == bg && s_wjp[w] < bj)) { bg = s_wg[w]; bj = s_wjp[w]; bb = s_wbin[w]; }
         }
-        ScanBest r;
-        r.gain = bg; r.jp = bj; r.bin = bb;
-        A.sbest[(int64_t)nodeidx * gridDim.y + blockIdx.y] = r;
+        if (!A.last_decides) {
+            ScanBest r;
+            r.gain = bg; r.jp = bj; r.bin = bb;
+            A.sbest[(int64_t)nodeidx * gridDim.y + blockIdx.y] = r;
+        } else { // the last of the node's blocks decides, as in k_scan
+            unsigned long long *mine = reinterpret_cast<unsigned long long *>(A.sbest + (int64_t)nodeidx * gridDim.y + blockIdx.y);
+            __hip_atomic_store(mine, (unsigned long long)__double_as_longlong(bg), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(mine + 1, (unsigned int)bj | ((unsigned long long)(unsigned int)bb << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the candidate is in memory before it is counted
+            s_last = __hip_atomic_fetch_add(A.counts + (size_t)nodeidx * EVT_SCAN_COUNT_STEP, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                     (int)gridDim.y - 1;
+        }
+    }
+    if (!A.last_decides) return;
+    if (A.zero_children && jp < A.nfs) { // the children's slices start from zero, whatever the node turns out to be
+        long long *hc = A.hist + (int64_t)(2 * n - 1) * A.node_stride + (int64_t)jp * NAG * B;
+        for (int i = lane; i < NAG * B; i += 64) {
+            hc[i] = 0;
+            hc[A.node_stride + i] = 0;
+        }
+    }
+    __syncthreads();
+    if (!s_last) return;
+    if (wave == 0) {
+        double g = -INFINITY;
+        int j = NO_BIN, b = NO_BIN;
+        const unsigned long long *cand = reinterpret_cast<const unsigned long long *>(A.sbest + (int64_t)nodeidx * gridDim.y);
+        for (int q = lane; q < (int)gridDim.y; q += 64) { // ascending positions: only a strictly larger gain replaces an earlier one
+            const double gg = __longlong_as_double((long long)__hip_atomic_load(cand + 2 * q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            const unsigned long long w = __hip_atomic_load(cand + 2 * q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (gg > g) { g = gg; j = (int)(w & 0xffffffffull); b = (int)(w >> 32); }
+        }
+        const int own = j;
+        wave_argmax(g, j);
+        const bool found = j != NO_BIN && g > A.gamma;
+        if (found ? own == j : lane == 0) {
+            A.counts[(size_t)nodeidx * EVT_SCAN_COUNT_STEP] = 0;
+            A.tree.w[n - 1] = (float)s_S[NK - 1];
+            s_wjp[0] = found ? j : NO_BIN;
+            s_wbin[0] = b;
+            if (found) {
+                const int feat = (int)A.js[j];
+                A.tree.feat[n - 1] = feat;
+                A.tree.cond_bin[n - 1] = (uint8_t)b;
+                A.tree.gain[n - 1] = (float)g;
+                A.tree.split[n - 1] = 1;
+                A.tree.packed[n - 1] = evt_pack_node(feat, b, A.feattypes[feat - 1] != 0);
+            }
+            A.status[n] = found ? ST_SPLIT : ST_LEAF;
+        }
+    }
+    __syncthreads();
+    const int bj = s_wjp[0], bb = s_wbin[0];
+    if (bj == NO_BIN) {
+        if (tid < K) A.tree.pred[(int64_t)K * (n - 1) + tid] = (float)leaf_value(A.loss, s_S, tid, K, A.eta, A.bagging, A.lambda, A.L2);
+        return;
+    }
+    // the children's totals; a subtract node's own slice was written by other blocks, so it is its parent's less its sibling's here too
+    const bool numeric = A.feattypes[A.js[bj] - 1] != 0;
+    for (int ag = wave; ag < NAG; ag += nwaves) {
+        const int64_t o = ((int64_t)bj * NAG + ag) * B;
+        long long s = 0;
+        for (int b = lane; b < B; b += 64) {
+            const bool in = numeric ? (b + 1 <= bb) : (b + 1 == bb);
+            if (in) s += is_sub ? hp[o + b] - hs[o + b] : hn[o + b];
+        }
+        s = wave_sum_i64(s);
+        if (lane == 0) {
+            A.node_sum[(int64_t)(2 * n) * NAG + ag] = s;
+            A.node_sum[(int64_t)(2 * n + 1) * NAG + ag] = s_Sq[ag] - s;
+        }
     }
 }
 
@@ -1053,20 +1122,21 @@ int launch_scan(evt_ctx *c, int level, const evt_params *p, bool leaf_level) {
     // extra blocks per node that only clear the children's histogram slices, while a level has few nodes
     unsigned zero_blocks = 0;
     if (!leaf_level && A.zero_children && !A.oblivious && nodes < 64) zero_blocks = 64 / nodes < 16 ? 64 / nodes : 16;
+    A.last_decides = !leaf_level && !A.oblivious && c->scan_fused ? 1 : 0;
     if (c->mc) { // any number of outputs: multi-class, several targets
         if (!leaf_level) {
             if (bpl == 1) hipLaunchKernelGGL((k_scan_mc<1>), grid, dim3(256), 0, c->stream, A);
             else if (bpl == 2) hipLaunchKernelGGL((k_scan_mc<2>), grid, dim3(256), 0, c->stream, A);
             else hipLaunchKernelGGL((k_scan_mc<4>), grid, dim3(256), 0, c->stream, A);
         }
-        if (!A.oblivious || leaf_level)
+        if (leaf_level || (!A.oblivious && !A.last_decides))
             hipLaunchKernelGGL(k_scan_fin_mc, dim3(nodes, !leaf_level && A.zero_children ? 1 + zero_blocks_per_node(nodes) : 1), dim3(256), 0, c->stream, A, ngroups);
         HIPCHK(hipGetLastError());
         return EVT_OK;
     }
     // few sampled features: one block of 16 waves scans a node's features and finishes the node, no second launch
     const bool fused = !leaf_level && !A.oblivious && A.nfs <= 16 && c->scan_fused;
-    A.last_decides = !leaf_level && !A.oblivious && !fused && c->scan_fused ? 1 : 0;
+    if (fused) A.last_decides = 0;
 #define SCASE(NAG_)                                                                                     \
     case NAG_:                                                                                          \
         if (fused) {                                                                                    \

@@ -411,7 +411,7 @@ int evt_reset_profile(evt_handle h);
  * while the host collects the tree, and that next call returns at once; meant for bagging_size 1 - with more
  * trees per round only the last one's work is used; 0, default; results do not depend on it); "scan_fused"
  * (1, default: one kernel searches and finishes a node's split - one block per node with at most 16 sampled features, else the last of a
- * node's blocks decides; losses of any number of outputs and oblivious trees take their own kernels -, 0: two kernels)
+ * node's blocks decides; oblivious trees take kernels of their own -, 0: two kernels)
  * and "hist_in_scatter" (1, default: with at most 16 features and a quarter of a million rows the levels below
  * the root get their histograms from the partition's scatter pass, one kernel less per level; 0: a histogram
  * kernel per level) - same trees and histograms, bit for bit, either way. */

@@ -19,13 +19,17 @@ pytestmark = pytest.mark.gpu
     ("mse", False, 5_001, 30, 32, 5, 30, dict(gamma=1e9)),                   # no candidate is good enough
     ("logloss", True, 900, 20, 32, 4, 20, dict(min_weight=1e6)),             # there is no candidate
     ("mse", True, 6_001, 50, 64, 6, 50, dict(cat=True, mono=True)),
+    ("mlogloss", False, 9_001, 3, 64, 6, 3, dict(K=7)),                      # any number of outputs: one block to a node
+    ("mlogloss", True, 9_001, 30, 255, 7, 26, dict(K=3, cat=True)),
+    ("mlogloss", False, 3_001, 280, 16, 4, 261, dict(K=5)),
+    ("mlogloss", False, 3_001, 20, 16, 4, 20, dict(K=16, gamma=1e9)),
 ])
 def test_last_block_decides(evt, loss, weights, N, F, B, D, n_js, more):
     more = dict(more)
     rng = np.random.default_rng(N)
     ft = (rng.random(F) > 0.4).astype(np.uint8) if more.pop("cat", False) else None
     mono = rng.integers(-1, 2, F).astype(np.int32) if more.pop("mono", False) else None
-    x_bin, y, w, mu = make_data(5, N, F, B, loss, weights)
+    x_bin, y, w, mu = make_data(5, N, F, B, loss, weights, K=more.pop("K", None))
     h, o, op, gp, pred0, grad = setup_pair(evt, loss, x_bin, y, w, mu, B, D, feattypes=ft, mono=mono, **more)
     orc.update_grads(op, pred0, y, grad)
     h.set_option("small_tree", 0)
