@@ -788,9 +788,9 @@ static int small_tree_buffers(evt_ctx *c, bool split) {
 // rows / S, the channels and - through the candidates every block reads and the searches its 16 wavefronts share - the nodes; slices
 // add a launch and the words they flush.  The other path spreads rows of any number over the chip and pays for its launches.  Estimates
 // in microseconds, fitted to rounds that each of them grew (4k to 250k rows, 10 and 60 features, depths 5 to 9, 1 to 14 channels).
-// mse of depth 6, microseconds per round of the other path, S = 1 and S > 1: 10 features 119, 63, 74 at 4k rows, 126, 119, 77 at
-// 32k, 128, -, 83 at 120k, 133, -, 93 at 250k; 60 features 156, 63, 76 at 4k, 168, -, 133 at 120k, 181, -, 206 at 250k.
-// 7 classes of depth 5 on 10 features: 183, 145, 161 at 4k, 229, 902, 191 at 65k, 279, -, 331 at 250k.
+// Whole calls of one round (host included, ~50 us) at depth 6, microseconds for the other path, S = 1 and S > 1: mse, 8 features 125, 81, 95 at 2k rows,
+// 139, 137, 96 at 30k, 148, -, 108 at 250k; mse, 100 features 150, 137, 120 at 30k; 3 classes, 8 features 195, 154, 149 at 8k,
+// 210, 543, 159 at 60k, 237, -, 215 at 250k; 7 classes, 8 features 213, 188, 226 at 2k, 275, -, 303 at 120k, 320, -, 396 at 250k.
 int small_tree_form(const evt_ctx *c, int nfs, bool all_rows) {
     if (!c->small_tree || c->D < 2 || c->D > 10 || nfs > 256 || c->N < 4 || c->N > (1 << 24) || !c->defer_pred || EVT_IS_QUANTILE(c->loss)) return 0;
     if (c->record_nidx && !all_rows) return 0;
@@ -801,15 +801,16 @@ int small_tree_form(const evt_ctx *c, int nfs, bool all_rows) {
     const bool canS = slots_split >= 1 && c->N / S < 65000 && small_acc_bytes(c) <= ((size_t)64 << 20) && (!obliv || (size_t)nodes * c->B * 8 <= 144 * 1024);
     if (c->small_tree == 2) return can1 ? 1 : 0;
     if (c->small_tree == 3) return canS ? S : 0;
-    const double k = 1e-3 * c->N, per_1k = c->mc ? 0.3 + 0.2 * c->NA : 0.3 + 0.055 * c->NA;
+    const double k = 1e-3 * c->N, per_1k = c->mc ? 0.3 + 0.2 * c->NA : 0.35 + 0.058 * c->NA, per_1k_s = c->mc ? 0.3 + 0.3 * c->NA : per_1k;
     double one = 0.0, split = 0.0;
     for (int l = 1; l < c->D; l++) {
         const int n = (int)std::min<int64_t>(1 << (l - 1), c->N), searches = (n + 15) / 16;
         one += 5.0 + 3.5 * searches + per_1k * k * ((n + slots - 1) / std::max(1, slots));
-        split += (c->mc ? 18.0 : 11.0) + 2.5 * searches + per_1k * k / S * ((n + slots_split - 1) / std::max(1, slots_split)) +
+        split += (c->mc ? 6.0 + 0.8 * c->NA : 11.0) + 2.5 * searches + per_1k_s * k / S * ((n + slots_split - 1) / std::max(1, slots_split)) +
                  (double)std::min<int64_t>((int64_t)n * c->B, c->N / S) * c->NA * nfs * S / 141e3; // words flushed: no more than rows
     }
-    const double launches = c->mc ? 16.0 + 0.8 * c->NA + (nfs > 16 ? 7.0 : 0.0) : 18.0 + 3.0 * std::min(c->NA, 8) + (nfs > 16 ? 9.0 : 0.0);
+    const double launches = c->mc ? 16.0 + 0.8 * c->NA + (nfs > 16 ? 2.0 + 0.008 * c->NA * std::max(0, nfs - 20) : std::max(0.0, 8.0 - 0.35 * c->NA))
+                                  : 18.0 + 3.0 * std::min(c->NA, 8) + (nfs > 16 ? 8.0 : 0.0);
     const double other = (c->D - 1) * (launches + (obliv ? 5.0 : 0.0) + 0.0068 * c->NA * k);
     if (can1 && one < other && (!canS || one <= split)) return 1;
     return canS && split < other ? S : 0;
