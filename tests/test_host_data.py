@@ -16,6 +16,12 @@ def _values(rng, kind, n):
         x = x * 1e300
     elif kind == "skewed":
         x = np.exp(9 * x)
+    elif kind == "denormal":  # of the smallest value there is and zero
+        x = np.where(x < 0, 0.0, 5e-324)
+    elif kind == "tiny":  # a range whose reciprocal overflows
+        x = x * 1e-310
+    elif kind == "far":  # almost all values share one of any number of equal slices, and are tiny there
+        x = np.where(rng.random(n) < 0.9, np.abs(x) * 1e-306, 1e-280)
     return x
 
 
@@ -45,7 +51,7 @@ def test_bins_of_every_layout(evt, kind, shape):
         assert np.array_equal(evt.binarize(lay, edges), bins)
 
 
-@pytest.mark.parametrize("kind", ["float32", "float64", "whole", "huge", "skewed"])
+@pytest.mark.parametrize("kind", ["float32", "float64", "whole", "huge", "skewed", "denormal", "tiny", "far"])
 @pytest.mark.parametrize("shape,nbins", [((1, 3), 4), ((64, 9), 2), ((65, 8), 255), ((3000, 17), 64), ((9000, 2), 8)])
 def test_edges_are_numpys_quantiles(evt, kind, shape, nbins):
     rng = np.random.default_rng(1)
