@@ -292,6 +292,17 @@ def _is_categorical(col):
     return hasattr(col, "categories") and hasattr(col, "codes")
 
 
+def _equal_columns(data, names):
+    """The columns of these names, each a vector of the first one's length: the library reads them by row number, without a check."""
+    cols = [_column(data, name) for name in names]
+    for name, col in zip(names, cols):
+        if not _is_categorical(col) and col.ndim != 1:
+            raise ValueError("feature %s is no vector" % name)
+        if len(col) != len(cols[0]):
+            raise ValueError("feature %s has %d rows, %s has %d" % (name, len(col), names[0], len(cols[0])))
+    return cols
+
+
 def _table_names(data):
     return [str(c) for c in (data.keys() if isinstance(data, dict) else data.columns)]
 
@@ -300,9 +311,8 @@ def get_edges_table(data, feature_names, nbins, rng):
     """get_edges for Tables input, src/fit-utils.jl:26-63: a Bool column is a two-level categorical feature, a
     categorical column is split on its levels (`==`, or `<=` when its levels are ordered), a Real column on the unique
     quantiles of the sampled rows."""
-    nrow = len(_column(data, feature_names[0]))
-    idx, nobs = _sample_rows(nrow, nbins, rng)
-    cols = [_column(data, name) for name in feature_names]
+    cols = _equal_columns(data, feature_names)
+    idx, nobs = _sample_rows(len(cols[0]), nbins, rng)
     real = [j for j, col in enumerate(cols) if not _is_categorical(col) and col.dtype.kind in "iuf"]
     q = _quantiles(_lib.table_columns([_real_column(cols[j]) for j in real]), idx, nobs, nbins) if real else None
     q = dict(zip(real, q)) if real else {}
@@ -338,10 +348,9 @@ def _real_column(col):
 
 def binarize_table(data, feature_names, edges):
     """binarize for Tables input, src/fit-utils.jl:74-92 -> (F, N) uint8 (the memory order of Julia's N x F matrix)."""
-    nrow = len(_column(data, feature_names[0]))
+    given = _equal_columns(data, feature_names)
     cols, search = [], []
-    for j, name in enumerate(feature_names):
-        col = _column(data, name)
+    for j, (name, col) in enumerate(zip(feature_names, given)):
         if _is_categorical(col):
             if list(col.categories) != list(edges[j]):  # levelcode refers to the training levels
                 col = col.set_categories(list(edges[j]))
@@ -358,9 +367,7 @@ def binarize_table(data, feature_names, edges):
             search.append(edges[j])
         else:
             raise RuntimeError("Invalid feature eltype: %s is %s" % (name, col.dtype))
-        if len(cols[j]) != nrow:
-            raise ValueError("feature %s has %d rows, %s has %d" % (name, len(cols[j]), feature_names[0], nrow))
-    return _lib.bin_columns(_lib.table_columns(cols), nrow, search)
+    return _lib.bin_columns(_lib.table_columns(cols), len(given[0]), search)
 
 
 def _table_features(data, target_names, weight_name, offset_name, feature_names):

@@ -56,3 +56,17 @@ def test_table_errors(evt):
     # default feature set: every Real / Bool / categorical column but the target, the weight and the offset
     from evotrees_jl_amd import _table_features
     assert _table_features(df, ["y"], "w", None, None) == ["num", "flag", "cat", "ord", "count"]
+
+
+@pytest.mark.parametrize("n,short", [(3000, 2999), (3000, 1), (200_000, 3000), (3000, 3001), (20_000, 0)])
+def test_ragged_tables_are_refused(evt, n, short):
+    """Columns of other lengths, and columns that are no vectors, before any of their rows is read."""
+    rng = np.random.default_rng(0)
+    good, bad = rng.random(n), rng.random(short)
+    edges, _, _ = evt.get_edges_table({"a": good}, ["a"], 16, np.random.default_rng(1))
+    for table in ({"a": good, "b": bad}, {"b": bad, "a": good}, {"a": good, "b": rng.random((n, 2))}, {"a": good, "b": bad > 0.5}):
+        names = list(table)
+        with pytest.raises(ValueError):
+            evt.get_edges_table(table, names, 16, np.random.default_rng(1))
+        with pytest.raises(ValueError):
+            evt.binarize_table(table, names, edges * 2)
