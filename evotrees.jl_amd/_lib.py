@@ -173,21 +173,28 @@ COLUMN = np.dtype([("data", np.uint64), ("stride", np.int64), ("dtype", np.int64
 DTYPE_IDS = {np.dtype(t): k for k, t in enumerate(("f4", "f8", "i1", "i2", "i4", "i8", "u1", "u2", "u4", "u8"))}
 
 
+class Columns:
+    """evt_column records and the array or arrays they point into, which live as long as the records do."""
+
+    def __init__(self, records, owner):
+        self.records, self.owner = records, owner
+
+
 def matrix_columns(x):
-    """The columns of a matrix (of a type in DTYPE_IDS) as evt_column records; they point into x."""
+    """The columns of a matrix of a type in DTYPE_IDS."""
     cols = np.empty(x.shape[1], COLUMN)
     cols["data"] = x.ctypes.data + x.strides[1] * np.arange(x.shape[1])
     cols["stride"] = x.strides[0]
     cols["dtype"] = DTYPE_IDS[x.dtype]
-    return cols
+    return Columns(cols, x)
 
 
 def table_columns(arrays):
-    """Vectors (Bool or of a type in DTYPE_IDS) as evt_column records; they point into the vectors."""
+    """Vectors, Bool or of a type in DTYPE_IDS, as columns."""
     cols = np.empty(len(arrays), COLUMN)
     for j, a in enumerate(arrays):
         cols[j] = (a.ctypes.data, a.strides[0], 6 if a.dtype == np.bool_ else DTYPE_IDS[a.dtype])
-    return cols
+    return Columns(cols, arrays)
 
 
 def strided_matrix(x):
@@ -216,8 +223,9 @@ def flat_edges(edges):
 def bin_columns(cols, nobs, edges):
     """Bins (F, nobs) of table columns, on the host: a column whose edges are empty gets value + 1."""
     flat, off = flat_edges(edges)
-    out = np.empty((len(cols), nobs), np.uint8)
-    check(load().evt_bin_columns(ptr(cols), len(cols), nobs, ptr(flat), ptr(off), ptr(out)))
+    n = len(cols.records)
+    out = np.empty((n, nobs), np.uint8)
+    check(load().evt_bin_columns(ptr(cols.records), n, nobs, ptr(flat), ptr(off), ptr(out)))
     return out
 
 
@@ -225,8 +233,8 @@ def order_stats(cols, idx, n, ranks):
     """(F, len(ranks)) order statistics of every column over the rows idx (None: the first n)."""
     ranks = np.ascontiguousarray(ranks, np.int64)
     idx = None if idx is None else np.ascontiguousarray(idx, np.int64)
-    out = np.empty((len(cols), len(ranks)), np.float64)
-    check(load().evt_order_stats(ptr(cols), len(cols), ptr(idx), n, ptr(ranks), len(ranks), ptr(out)))
+    out = np.empty((len(cols.records), len(ranks)), np.float64)
+    check(load().evt_order_stats(ptr(cols.records), len(cols.records), ptr(idx), n, ptr(ranks), len(ranks), ptr(out)))
     return out
 
 

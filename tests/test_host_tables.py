@@ -70,3 +70,17 @@ def test_ragged_tables_are_refused(evt, n, short):
             evt.get_edges_table(table, names, 16, np.random.default_rng(1))
         with pytest.raises(ValueError):
             evt.binarize_table(table, names, edges * 2)
+
+
+def test_columns_that_are_converted_live_as_long_as_they_are_read(evt):
+    """Real columns of types the library does not know are read from Float64 copies: large ones, whose memory is unmapped when freed."""
+    rng = np.random.default_rng(0)
+    n = 300_000
+    table = {"a": rng.random(n).astype(np.float16), "b": rng.random(n).astype(np.longdouble), "c": rng.random(n).astype(">f8")}
+    edges, _, _ = evt.get_edges_table(table, list(table), 16, np.random.default_rng(1))
+    rows = np.sort(np.random.default_rng(1).choice(n, 16_000, replace=False))
+    x_bin = evt.binarize_table(table, list(table), edges)
+    for j, col in enumerate(table.values()):
+        v = col.astype(np.float64)
+        assert np.array_equal(edges[j], np.unique(np.quantile(v[rows], np.arange(1, 16) / 16)))
+        assert np.array_equal(x_bin[j], np.searchsorted(edges[j], v, side="left") + 1)
