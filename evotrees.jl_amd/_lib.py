@@ -222,8 +222,10 @@ def flat_edges(edges):
 
 def bin_columns(cols, nobs, edges):
     """Bins (F, nobs) of table columns, on the host: a column whose edges are empty gets value + 1."""
-    flat, off = flat_edges(edges)
     n = len(cols.records)
+    if len(edges) < n:  # as the library reads them: one entry per column
+        raise IndexError("%d columns, but edges of %d" % (n, len(edges)))
+    flat, off = flat_edges(edges)
     out = np.empty((n, nobs), np.uint8)
     check(load().evt_bin_columns(ptr(cols.records), n, nobs, ptr(flat), ptr(off), ptr(out)))
     return out
@@ -294,6 +296,8 @@ class Handle:
     def binarize_matrix(self, x, edges):
         """x: (N, F) matrix as the program holds it, rows or columns contiguous; edges as for binarize."""
         assert x.shape == (self.N, self.F)
+        if len(edges) != self.F:
+            raise ValueError("%d columns, but edges of %d" % (self.F, len(edges)))
         x, rs, cs = strided_matrix(x)
         flat, off = flat_edges(edges)
         check(load().evt_binarize(self._h, ptr(x), DTYPE_IDS[x.dtype], rs, cs, ptr(flat), ptr(off)))

@@ -70,6 +70,20 @@ def test_edges_are_numpys_quantiles(evt, kind, shape, nbins):
             assert np.array_equal(edges[j], want, equal_nan=True)
 
 
+def test_more_columns_than_edges_are_refused(evt):
+    with pytest.raises(IndexError):
+        evt.binarize(np.zeros((50, 4)), [np.arange(3.0)] * 3)
+
+
+@pytest.mark.gpu
+def test_a_handle_takes_one_feature_for_each_of_its_columns(evt):
+    h = evt.Handle(50, 4, 16, 1, 3, "mse")
+    for n in (3, 5):
+        with pytest.raises(ValueError):
+            h.binarize_matrix(np.zeros((50, 4)), [np.arange(3.0)] * n)
+    h.close()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("order", ["C", "F"])
