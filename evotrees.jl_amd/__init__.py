@@ -358,10 +358,10 @@ def binarize_table(data, feature_names, edges):
             if (codes < 0).any():
                 raise RuntimeError("feature %s holds missing values or levels the model was not trained on" % name)
             cols.append(codes)
-            search.append(())  # code + 1
+            search.append(None)  # code + 1
         elif col.dtype == np.bool_:
             cols.append(col)
-            search.append(())
+            search.append(None)
         elif col.dtype.kind in "iuf":
             cols.append(_real_column(col))
             search.append(edges[j])
@@ -673,6 +673,8 @@ def update(config, m, cache, x_train=None, y_train=None, w_train=None):
 def binarize(x, edges):
     """binarize, src/fit-utils.jl:66-72 — host version used for inference inputs (searchsortedfirst, in the order of isless)."""
     x = np.asarray(x)
+    if x.ndim > 2:
+        raise ValueError("x must be a matrix")
     if x.dtype not in _lib.DTYPE_IDS:
         x = x.astype(np.float64)
     return _lib.bin_columns(_lib.matrix_columns(x), x.shape[0], edges)

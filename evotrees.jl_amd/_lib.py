@@ -214,19 +214,25 @@ def strided_matrix(x):
 
 def flat_edges(edges):
     """Edges of all features one after the other, and where each feature's start."""
+    edges = [np.asarray(e, np.float64) for e in edges]
+    if any(e.ndim != 1 for e in edges):
+        raise ValueError("the edges of a feature must be a vector")
     off = np.zeros(len(edges) + 1, np.int32)
     off[1:] = np.cumsum([len(e) for e in edges])
-    flat = np.concatenate([np.asarray(e, np.float64) for e in edges]) if len(edges) else np.zeros(0)
+    flat = np.concatenate(edges) if len(edges) else np.zeros(0)
     return np.ascontiguousarray(flat), off
 
 
 def bin_columns(cols, nobs, edges):
-    """Bins (F, nobs) of table columns, on the host: a column whose edges are empty gets value + 1."""
+    """Bins (F, nobs) of columns, on the host: 1 + the number of edges below a value, or the value + 1 where a column's edges are None."""
     n = len(cols.records)
     if len(edges) < n:  # as the library reads them: one entry per column
         raise IndexError("%d columns, but edges of %d" % (n, len(edges)))
-    flat, off = flat_edges(edges)
+    # the library takes a column without edges for one of codes; no value passes a NaN
+    flat, off = flat_edges([() if e is None else e if np.size(e) else [np.nan] for e in edges[:n]])
     out = np.empty((n, nobs), np.uint8)
+    if out.size == 0:
+        return out
     check(load().evt_bin_columns(ptr(cols.records), n, nobs, ptr(flat), ptr(off), ptr(out)))
     return out
 
@@ -234,8 +240,12 @@ def bin_columns(cols, nobs, edges):
 def order_stats(cols, idx, n, ranks):
     """(F, len(ranks)) order statistics of every column over the rows idx (None: the first n)."""
     ranks = np.ascontiguousarray(ranks, np.int64)
+    if n < 1 and len(ranks):
+        raise IndexError("order statistics of no rows")
     idx = None if idx is None else np.ascontiguousarray(idx, np.int64)
     out = np.empty((len(cols.records), len(ranks)), np.float64)
+    if out.size == 0:
+        return out
     check(load().evt_order_stats(ptr(cols.records), len(cols.records), ptr(idx), n, ptr(ranks), len(ranks), ptr(out)))
     return out
 

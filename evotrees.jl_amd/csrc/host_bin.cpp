@@ -152,7 +152,7 @@ void HbPlan::build(const double *edges_flat, const int32_t *off, int F_, int dty
         f.ne = off[j + 1] - off[j];
         f.e = edges.data() + off[j];
         f.levels = 4;
-        while ((1 << f.levels) - 1 < f.ne) f.levels++;
+        while ((1 << f.levels) - 1 < f.ne && f.levels < 8) f.levels++;
         f.heap = (int32_t)words;
         words += std::max(16, 1 << f.levels);
     }
@@ -162,7 +162,7 @@ void HbPlan::build(const double *edges_flat, const int32_t *off, int F_, int dty
     for (int j = 0; j < F; j++) {
         HbFeature &f = feat[j];
         key.resize(std::max(1, f.ne));
-        bool slow = false, all32 = true;
+        bool slow = f.ne > 254, all32 = true;
         for (int i = 0; i < f.ne; i++) {
             const double e = f.e[i];
             slow |= e != e || (e == 0.0 && signbit(e)) || (i > 0 && !(f.e[i - 1] <= e));

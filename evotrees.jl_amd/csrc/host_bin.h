@@ -19,12 +19,12 @@ struct HbSource {
     size_t esize() const { return dtype == EVT_F32 ? 4 : 8; }
 };
 
-#define HB_SLOW 1  // an edge is NaN or -0.0: compared by isless, value by value
+#define HB_SLOW 1  // an edge is NaN or -0.0, or there are more than 254: compared by isless, value by value
 #define HB_EXACT 2 // the Float32 search decides alone; otherwise a value that meets an edge there is compared in Float64
 
 // One feature's edges for a source type, laid out for the search.
 struct HbFeature {
-    int32_t levels; // steps of the search: 4 .. 8, 2^levels - 1 >= ne
+    int32_t levels; // steps of the search: 4 .. 8, 2^levels - 1 >= ne unless the feature is HB_SLOW
     int32_t flags;
     int32_t ne;
     int32_t heap;      // first word of the feature's search heap in HbPlan::heap

@@ -84,7 +84,7 @@ extern "C" int evt_bin_columns(const void *cols, int32_t ncols, int64_t nobs, co
     if (r != EVT_OK) return r;
     ARGCHK(nobs >= 1 && edge_off && out, "NULL argument");
     for (int j = 0; j < ncols; j++)
-        ARGCHK(edge_off[j] >= 0 && edge_off[j + 1] >= edge_off[j] && edge_off[j + 1] - edge_off[j] <= 254, "each feature has at most 254 edges");
+        ARGCHK(edge_off[j] >= 0 && edge_off[j + 1] >= edge_off[j], "edge offsets must ascend");
     ARGCHK(edges || edge_off[ncols] == 0, "NULL argument");
     hb_bin_columns(c.data(), ncols, nobs, edges, edge_off, out);
     return EVT_OK;

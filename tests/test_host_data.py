@@ -75,6 +75,29 @@ def test_more_columns_than_edges_are_refused(evt):
         evt.binarize(np.zeros((50, 4)), [np.arange(3.0)] * 3)
 
 
+def test_the_smallest_and_largest_calls(evt):
+    """No rows, no columns, no edges, more edges than a bin's byte counts (it wraps): what numpy's search gives."""
+    rng = np.random.default_rng(0)
+    assert evt.binarize(np.zeros((0, 3)), [np.arange(3.0)] * 3).shape == (3, 0)
+    assert evt.binarize(np.zeros((3, 0)), []).shape == (0, 3)
+    assert evt.binarize_table({"a": np.zeros(0)}, ["a"], [np.arange(3.0)]).shape == (1, 0)
+    assert np.array_equal(evt.binarize(np.arange(4)[:, None], [()]), np.ones((1, 4)))
+    for n in (254, 255, 256, 700):
+        e, x = np.sort(rng.random(n)), rng.random((77, 3))
+        want = np.stack([(np.searchsorted(e, x[:, j]) + 1).astype(np.uint8) for j in range(3)])
+        assert np.array_equal(evt.binarize(x, [e] * 3), want) and np.array_equal(evt.binarize(np.asfortranarray(x), [e] * 3), want)
+    for bad in (2.0, np.zeros((2, 2))):
+        with pytest.raises(ValueError):
+            evt.binarize(np.zeros((4, 1)), [bad])
+    with pytest.raises(ValueError):
+        evt.binarize(np.zeros((4, 2, 2)), [np.arange(3.0)] * 2)
+    assert evt.get_edges(np.zeros((3, 0)), 16, rng)[0] == []
+    assert [len(e) for e in evt.get_edges(np.zeros((3, 2)), 1, rng)[0]] == [0, 0]
+    for nbins in (2, 16):
+        with pytest.raises(IndexError):
+            evt.get_edges(np.zeros((0, 3)), nbins, rng)
+
+
 @pytest.mark.gpu
 def test_a_handle_takes_one_feature_for_each_of_its_columns(evt):
     h = evt.Handle(50, 4, 16, 1, 3, "mse")
