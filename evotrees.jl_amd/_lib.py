@@ -594,8 +594,8 @@ class KeptModel:
             return self._tree, self._edge if edges is not None else None
 
     def predict(self, x, trees, edges, feattypes, ntrees, leaf=False):
-        """(N, K) float32 with the link applied, or (N, ntrees) leaf ids, of the first ntrees trees; None when the trees cannot be kept.
-        x: an (N, F) matrix, or with edges=None (F, N) bins."""
+        """(N, K) float32 with the link applied, or (N, ntrees) leaf ids, of the first ntrees trees; None for what a kept model does not
+        take (trees too large, or invalid ones, also behind the first ntrees): the whole-model calls decide on it.  x: an (N, F) matrix, or with edges=None (F, N) bins."""
         held = self._take(trees, edges)
         if held is None:
             return None
@@ -606,7 +606,7 @@ class KeptModel:
         else:
             N, F = x.shape
             x, rs, cs = strided_matrix(x)
-            if F > len(edge[3]):
+            if F != len(edge[3]):
                 raise ValueError("the matrix has %d columns, the model %d features" % (F, len(edge[3])))
             args = edge[0] + (x.ctypes.data, DTYPE_IDS[x.dtype], rs, cs)
         ft = None if feattypes is None else np.ascontiguousarray(feattypes, np.uint8)
@@ -617,7 +617,10 @@ class KeptModel:
         else:
             out = np.empty((N, self.K), np.float32)
             outs = (out.ctypes.data, None)
-        check(load().evt_model_predict(self._h, *tree[0], *fta, *args, N, F, ntrees, 0 if leaf else 1, *outs))
+        rc = load().evt_model_predict(self._h, *tree[0], *fta, *args, N, F, ntrees, 0 if leaf else 1, *outs)
+        if rc in (EVT_ERR_ARG, EVT_ERR_NOMEM):
+            return None
+        check(rc)
         return out.T if leaf else out
 
 

@@ -72,3 +72,26 @@ def test_follows_changes_of_the_model(evt):
     m.trees[1].feat[-1] = 1
     with pytest.raises(evt.EvtError):
         evt.predict(m, x)
+
+
+def test_takes_what_the_whole_model_calls_take(evt):
+    rng = np.random.default_rng(4)
+    # leaf ids of so many trees that 64 rows of them do not fit a piece's buffer
+    m = _model(evt, rng, 3, 16, 1, "mse", [9] * 3)
+    m.trees = m.trees * 22_000
+    x = rng.random((3, 3))
+    assert np.array_equal(evt.predict_leaf_idx(m, x), np.tile(evt.predict_leaf_idx(m, x, ntree_limit=3), (1, 22_000)))
+    # trees behind the limit that the matrix is too narrow for, or that are none
+    m = _model(evt, rng, 3, 16, 1, "mse", [5] * 4)
+    wide = _model(evt, rng, 6, 16, 1, "mse", [5] * 4)
+    m.trees += wide.trees
+    x = rng.random((70, 3))
+    want = evt._lib.predict_model_f64(np.ascontiguousarray(x.T), m.info["edges"], m.info["feattypes"], "mse", 1, m.trees[:4])
+    assert np.array_equal(evt.predict(m, x, ntree_limit=4), want.reshape(-1))
+    with pytest.raises(evt.EvtError):
+        evt.predict(m, x)
+    m.trees[7].split[-1] = m.trees[7].feat[-1] = 1
+    assert np.array_equal(evt.predict(m, x, ntree_limit=4), want.reshape(-1))
+    for n in (2, 4):  # neither fewer columns than features nor more
+        with pytest.raises(ValueError):
+            evt.predict(m, rng.random((5, n)), ntree_limit=4)
