@@ -8,6 +8,8 @@
 #include <cmath>
 #include <condition_variable>
 #include <mutex>
+#include <system_error>
+#include <thread>
 
 bool hb_has_avx512() {
 #if defined(__x86_64__)
@@ -26,45 +28,72 @@ int hb_workers(int64_t cells) {
 }
 
 // The worker threads: started when first needed, kept asleep between calls (waking one costs about 5 us, starting one 15 and more), at
-// most one per core.  One parallel region uses them at a time; a region that finds them taken starts threads of its own.
+// most one per core less the caller's in the whole process.  Any number of regions use them at a time, each caller beside its own:
+// a worker that comes free joins the region with the fewest, and between two tasks leaves one that has more than its share while
+// another waits.
 namespace {
+struct Region {
+    const std::function<bool()> *step;
+    int wanted;                // workers that may still join; changed under Pool::m, as `active` is
+    std::atomic<int> active{0};
+    bool closed = false;
+};
 struct Pool {
     const pid_t pid = getpid();
-    std::mutex region; // held by the region that uses the workers
+    const int most = std::max(1, (int)std::thread::hardware_concurrency()) - 1;
     std::mutex m;
     std::condition_variable cv, cv_done;
     int threads = 0;
-    const std::function<void()> *job = nullptr; // null: nothing to join
-    uint64_t gen = 0;
-    int wanted = 0, active = 0;
+    std::vector<Region *> regions;
+    std::atomic<int> open{0}; // regions, for a look without the lock
+    Region *hungriest() {
+        Region *best = nullptr;
+        for (Region *r : regions)
+            if (r->wanted > 0 && (!best || r->active.load() < best->active.load())) best = r;
+        return best;
+    }
+    bool should_leave(const Region *r) { // one worker more there than here would still be no more than here now
+        if (open.load(std::memory_order_relaxed) < 2) return false;
+        std::lock_guard<std::mutex> lk(m);
+        for (const Region *o : regions)
+            if (o != r && o->wanted > 0 && o->active + 1 < r->active) return true;
+        return false;
+    }
     void loop() {
-        uint64_t seen = 0;
         std::unique_lock<std::mutex> lk(m);
         for (;;) {
-            cv.wait(lk, [&] { return job && gen != seen && wanted > 0; });
-            seen = gen;
-            wanted--;
-            active++;
-            const std::function<void()> *j = job;
+            Region *r;
+            cv.wait(lk, [&] { return (r = hungriest()) != nullptr; });
+            r->wanted--;
+            r->active++;
             lk.unlock();
-            (*j)();
+            bool more = true, leave = false;
+            while (!leave && (more = (*r->step)())) leave = should_leave(r);
             lk.lock();
-            if (--active == 0) cv_done.notify_all();
+            if (!more) r->wanted = 0; // nothing left to hand out
+            else if (!r->closed) r->wanted++;
+            if (--r->active == 0) cv_done.notify_all();
         }
     }
-    void start(int n, const std::function<void()> *j) {
+    void enter(Region *r) {
         std::lock_guard<std::mutex> lk(m);
-        for (; threads < n; threads++) std::thread([this] { loop(); }).detach();
-        job = j;
-        gen++;
-        wanted = n;
-        for (int i = 0; i < n; i++) cv.notify_one();
+        regions.push_back(r);
+        open.store((int)regions.size(), std::memory_order_relaxed);
+        int need = 0;
+        for (const Region *o : regions) need += o->wanted + o->active;
+        try {
+            for (; threads < std::min(need, most); threads++) std::thread([this] { loop(); }).detach();
+        } catch (const std::system_error &) { // no more threads to be had: the callers do their work themselves
+        }
+        for (int i = 0; i < r->wanted; i++) cv.notify_one();
     }
-    void finish() { // workers that have not joined by now do not; those that have are waited for
+    void leave(Region *r) { // workers that have not joined by now do not; those that have are waited for
         std::unique_lock<std::mutex> lk(m);
-        job = nullptr;
-        wanted = 0;
-        cv_done.wait(lk, [&] { return active == 0; });
+        r->closed = true;
+        r->wanted = 0;
+        cv_done.wait(lk, [&] { return r->active == 0; });
+        regions.erase(std::find(regions.begin(), regions.end(), r));
+        open.store((int)regions.size(), std::memory_order_relaxed);
     }
     static Pool &get() { // never destroyed: its threads outlive main.  After a fork the child has none of them and starts afresh
         static std::mutex gm;
@@ -76,44 +105,39 @@ struct Pool {
 };
 } // namespace
 
-HbWorkers::HbWorkers(int n, std::function<void()> f) : fn(std::move(f)) {
+struct HbWorkers::State {
+    std::function<bool()> step;
+    Pool &pool;
+    Region region;
+    State(int n, std::function<bool()> &&f) : step(std::move(f)), pool(Pool::get()) {
+        region.step = &step;
+        region.wanted = n;
+    }
+};
+HbWorkers::HbWorkers(int n, std::function<bool()> step) {
     if (n <= 0) return;
-    Pool &p = Pool::get();
-    if (p.region.try_lock()) {
-        pool = &p;
-        try {
-            p.start(n, &fn);
-        } catch (...) {
-            join();
-            throw;
-        }
-    } else {
-        try {
-            for (int w = 0; w < n; w++) own.emplace_back(fn);
-        } catch (...) {
-            join();
-            throw;
-        }
-    }
+    std::unique_ptr<State> s(new State(n, std::move(step)));
+    s->pool.enter(&s->region);
+    state = std::move(s);
 }
+bool HbWorkers::none() const { return !state || state->region.active.load(std::memory_order_relaxed) == 0; }
 void HbWorkers::join() {
-    if (pool) {
-        Pool *p = static_cast<Pool *>(pool);
-        p->finish();
-        p->region.unlock();
-        pool = nullptr;
-    }
-    for (auto &t : own) t.join();
-    own.clear();
+    if (state) state->pool.leave(&state->region);
+    state.reset();
 }
+HbWorkers::~HbWorkers() { join(); }
 
 void hb_parallel(int ntasks, int nworkers, const std::function<void(int)> &fn) {
     std::atomic<int> next{0};
-    auto loop = [&] {
-        for (int t; (t = next.fetch_add(1, std::memory_order_relaxed)) < ntasks;) fn(t);
+    auto step = [&]() -> bool {
+        const int t = next.fetch_add(1, std::memory_order_relaxed);
+        if (t >= ntasks) return false;
+        fn(t);
+        return true;
     };
-    HbWorkers ws(std::min(nworkers, ntasks - 1), loop);
-    loop();
+    HbWorkers ws(std::min(nworkers, ntasks - 1), step);
+    while (step()) {
+    }
 }
 
 // Float32 neighbours of a Float64 value: the largest not above it, the smallest not below it

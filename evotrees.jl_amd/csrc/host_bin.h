@@ -5,7 +5,7 @@
 
 #include <atomic>
 #include <functional>
-#include <thread>
+#include <memory>
 #include <vector>
 
 #include "../../include/evotrees_hip.h"
@@ -62,16 +62,18 @@ void hb_bin_columns(const HbColumn *cols, int nc, int64_t n, const double *edges
 // a column with a NaN among them gets NaN throughout
 void hb_order_stats(const HbColumn *cols, int nc, const int64_t *idx, int64_t n, const int64_t *ranks, int nr, double *out);
 
-// f() on up to n worker threads (fewer, or none, when they come too late to join) until join(), which waits for those that joined
+// step() again and again on up to n worker threads (fewer, or none, when others use them) until it returns false: no task is left.  A
+// task is short (tens of us): between two of them a worker may move to another caller's region, and come back.  join() waits for
+// the workers that are in a task; what no worker has taken by then is the caller's to do.
 class HbWorkers {
-    std::function<void()> fn;
-    void *pool = nullptr;
-    std::vector<std::thread> own;
+    struct State;
+    std::unique_ptr<State> state;
 
   public:
-    HbWorkers(int n, std::function<void()> f);
-    ~HbWorkers() { join(); }
+    HbWorkers(int n, std::function<bool()> step);
+    ~HbWorkers();
     HbWorkers(const HbWorkers &) = delete;
+    bool none() const; // no worker is at it now: the caller does its tasks itself
     void join();
 };
 // fn(0) .. fn(ntasks - 1) on the calling thread and up to nworkers more; all are done when it returns

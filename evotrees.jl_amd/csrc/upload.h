@@ -4,6 +4,8 @@
 #include "host_bin.h"
 #include "pool.h"
 
+#include <thread>
+
 static const size_t PINNED_BYTES = (size_t)8 << 20; // a piece on its way up
 
 struct PinnedSlots { // NS of them, with an event each for the work that reads or writes them
@@ -45,7 +47,7 @@ struct BinPieces {
     void bin(const HbPlan &P, const HbSource &S, int64_t p, int t, uint8_t *out) const; // the bin of (r, f) to out[(f - f0) * n + r - r0]
 };
 
-// The pieces 0 .. np - 1 through NS buffers: piece p is filled by its `tasks` calls of fill(p, t), on worker threads; then send(p) queues
+// The pieces 0 .. np - 1 through NS buffers: piece p is filled by its `tasks` calls of fill(p, t), on worker threads or this one; then send(p) queues
 // what the device does with it and records U.ev[p % NS]; when that event has come, retire(p), on the calling thread, and the buffer
 // is free for piece p + NS.  Everything has been retired when the call returns EVT_OK.
 template <typename Fill, typename Send, typename Retire>
@@ -74,22 +76,21 @@ static int run_pieces(PinnedSlots &U, int NS, int64_t np, int tasks, int workers
     std::vector<std::atomic<int>> done((size_t)np);
     for (auto &d : done) d.store(0, std::memory_order_relaxed);
     std::atomic<bool> stop{false};
-    auto work = [&] {
-        for (int64_t t; (t = next.fetch_add(1, std::memory_order_relaxed)) < total;) {
-            const int64_t p = t / tasks;
-            while (p >= released.load(std::memory_order_acquire)) {
-                if (stop.load(std::memory_order_relaxed)) return;
-                std::this_thread::yield();
-            }
-            fill(p, (int)(t % tasks));
-            done[(size_t)p].fetch_add(1, std::memory_order_release);
+    auto step = [&]() -> bool {
+        int64_t t = next.load(std::memory_order_relaxed);
+        if (t >= total || stop.load(std::memory_order_relaxed)) return false;
+        if (t / tasks >= released.load(std::memory_order_acquire)) std::this_thread::yield();
+        else if (next.compare_exchange_weak(t, t + 1, std::memory_order_relaxed)) {
+            fill(t / tasks, (int)(t % tasks));
+            done[(size_t)(t / tasks)].fetch_add(1, std::memory_order_release);
         }
+        return true;
     };
     struct Stop { // whatever ends the call, workers that wait for a buffer stop waiting
         std::atomic<bool> &flag;
         ~Stop() { flag.store(true); }
     };
-    HbWorkers ws(workers, work);
+    HbWorkers ws(workers, step);
     Stop on_return{stop};
     int64_t back = 0;
     for (int64_t p = 0; p < np; p++) {
@@ -105,7 +106,8 @@ static int run_pieces(PinnedSlots &U, int NS, int64_t np, int tasks, int workers
                     HIPCHK(q);
                 }
             }
-            std::this_thread::yield();
+            if (ws.none()) step();
+            else std::this_thread::yield();
         }
         const int r = send(p);
         if (r != EVT_OK) return r;

@@ -1,5 +1,8 @@
 """Features in host memory on their way in: binning by the host's cores and the quantile edges, for every layout and type a program
 may hold them in, against numpy's search in the order of isless and numpy's quantiles."""
+import os
+import threading
+
 import numpy as np
 import pytest
 
@@ -75,6 +78,44 @@ def test_more_columns_than_edges_are_refused(evt):
         evt.binarize(np.zeros((50, 4)), [np.arange(3.0)] * 3)
 
 
+class Threads:
+    """The most threads the process had at a look every half millisecond."""
+
+    def __enter__(self):
+        self.most, self._stop = 0, threading.Event()
+        self._t = threading.Thread(target=self._look)
+        self._t.start()
+        return self
+
+    def _look(self):
+        while not self._stop.wait(0.0005):
+            self.most = max(self.most, len(os.listdir("/proc/self/task")))
+
+    def __exit__(self, *_):
+        self._stop.set()
+        self._t.join()
+
+
+def test_callers_at_once_share_the_workers(evt):
+    """Any number of calls at a time: right results, and in all no more worker threads than cores."""
+    rng = np.random.default_rng(0)
+    x, e = rng.random((400_000, 6)), np.sort(rng.random(63))
+    want = evt.binarize(x, [e] * 6)
+    same = [False] * 8
+
+    def work(k):
+        same[k] = all(np.array_equal(evt.binarize(x, [e] * 6), want) for _ in range(6))
+    with Threads() as seen:
+        callers = [threading.Thread(target=work, args=(k,)) for k in range(8)]
+        before = len(os.listdir("/proc/self/task"))
+        for t in callers:
+            t.start()
+        for t in callers:
+            t.join()
+    assert all(same)
+    assert seen.most <= before + 8 + os.cpu_count() - 1
+
+
 def test_the_smallest_and_largest_calls(evt):
     """No rows, no columns, no edges, more edges than a bin's byte counts (it wraps): what numpy's search gives."""
     rng = np.random.default_rng(0)
@@ -121,3 +162,19 @@ def test_upload_of_a_matrix_as_it_lies(evt, dtype, order, shape):
     h.binarize_matrix(x, edges)
     assert np.array_equal(h.get_xbin(), evt.binarize(x, edges))
     h.close()
+
+
+@pytest.mark.gpu
+def test_leaf_ids_of_more_pieces_than_buffers(evt):
+    """The ids of a piece are spread out while later pieces are binned, by the same workers."""
+    from test_gpu_kept_model import _model
+    rng = np.random.default_rng(6)
+    m = _model(evt, rng, 4, 16, 1, "mse", [9] * 200)  # 2-byte ids, 404 bytes a row: ten pieces of 20k rows
+    x = rng.random((200_000, 4), np.float32)
+    want = evt._lib.predict_leaf_idx(evt.binarize(x, m.info["edges"]), m.info["feattypes"], m.trees)
+    evt.predict_leaf_idx(m, x)
+    before = len(os.listdir("/proc/self/task"))
+    with Threads() as seen:
+        got = evt.predict_leaf_idx(m, x)
+    assert np.array_equal(got, want)
+    assert seen.most <= before + 1
