@@ -7,8 +7,8 @@
 #include <algorithm>
 #include <cmath>
 #include <condition_variable>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 bool hb_has_avx512() {
@@ -37,6 +37,8 @@ struct Region {
     int wanted;                // workers that may still join; changed under Pool::m, as `active` is
     std::atomic<int> active{0};
     bool closed = false;
+    std::atomic<bool> failed{false};
+    std::exception_ptr error; // the first exception of a task; the caller's to throw
 };
 struct Pool {
     const pid_t pid = getpid();
@@ -68,8 +70,15 @@ struct Pool {
             r->active++;
             lk.unlock();
             bool more = true, leave = false;
-            while (!leave && (more = (*r->step)())) leave = should_leave(r);
+            std::exception_ptr error;
+            try {
+                while (!leave && (more = !r->failed.load(std::memory_order_relaxed) && (*r->step)())) leave = should_leave(r);
+            } catch (...) {
+                error = std::current_exception();
+                more = false;
+            }
             lk.lock();
+            if (error && !r->failed.exchange(true)) r->error = error;
             if (!more) r->wanted = 0; // nothing left to hand out
             else if (!r->closed) r->wanted++;
             if (--r->active == 0) cv_done.notify_all();
@@ -83,7 +92,7 @@ struct Pool {
         for (const Region *o : regions) need += o->wanted + o->active;
         try {
             for (; threads < std::min(need, most); threads++) std::thread([this] { loop(); }).detach();
-        } catch (const std::system_error &) { // no more threads to be had: the callers do their work themselves
+        } catch (const std::exception &) { // no more threads to be had: the callers do their work themselves
         }
         for (int i = 0; i < r->wanted; i++) cv.notify_one();
     }
@@ -121,11 +130,18 @@ HbWorkers::HbWorkers(int n, std::function<bool()> step) {
     state = std::move(s);
 }
 bool HbWorkers::none() const { return !state || state->region.active.load(std::memory_order_relaxed) == 0; }
+bool HbWorkers::failed() const { return state && state->region.failed.load(std::memory_order_relaxed); }
 void HbWorkers::join() {
-    if (state) state->pool.leave(&state->region);
-    state.reset();
+    if (!state) return;
+    const std::unique_ptr<State> s = std::move(state);
+    s->pool.leave(&s->region);
+    if (s->region.error) std::rethrow_exception(s->region.error);
 }
-HbWorkers::~HbWorkers() { join(); }
+HbWorkers::~HbWorkers() {
+    if (!state) return;
+    state->region.failed.store(true); // left by an exception or an error: no further task
+    state->pool.leave(&state->region);
+}
 
 void hb_parallel(int ntasks, int nworkers, const std::function<void(int)> &fn) {
     std::atomic<int> next{0};
@@ -136,8 +152,9 @@ void hb_parallel(int ntasks, int nworkers, const std::function<void(int)> &fn) {
         return true;
     };
     HbWorkers ws(std::min(nworkers, ntasks - 1), step);
-    while (step()) {
+    while (!ws.failed() && step()) {
     }
+    ws.join();
 }
 
 // Float32 neighbours of a Float64 value: the largest not above it, the smallest not below it

@@ -64,7 +64,8 @@ void hb_order_stats(const HbColumn *cols, int nc, const int64_t *idx, int64_t n,
 
 // step() again and again on up to n worker threads (fewer, or none, when others use them) until it returns false: no task is left.  A
 // task is short (tens of us): between two of them a worker may move to another caller's region, and come back.  join() waits for
-// the workers that are in a task; what no worker has taken by then is the caller's to do.
+// the workers that are in a task, and throws what a task threw first (failed(): no further one is begun); what no worker has taken
+// by then is the caller's to do.
 class HbWorkers {
     struct State;
     std::unique_ptr<State> state;
@@ -73,6 +74,7 @@ class HbWorkers {
     HbWorkers(int n, std::function<bool()> step);
     ~HbWorkers();
     HbWorkers(const HbWorkers &) = delete;
+    bool failed() const;
     bool none() const; // no worker is at it now: the caller does its tasks itself
     void join();
 };

@@ -106,6 +106,7 @@ static int run_pieces(PinnedSlots &U, int NS, int64_t np, int tasks, int workers
                     HIPCHK(q);
                 }
             }
+            if (ws.failed()) ws.join(); // throws
             if (ws.none()) step();
             else std::this_thread::yield();
         }

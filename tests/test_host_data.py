@@ -1,6 +1,7 @@
 """Features in host memory on their way in: binning by the host's cores and the quantile edges, for every layout and type a program
 may hold them in, against numpy's search in the order of isless and numpy's quantiles."""
 import os
+import subprocess
 import threading
 
 import numpy as np
@@ -114,6 +115,53 @@ def test_callers_at_once_share_the_workers(evt):
             t.join()
     assert all(same)
     assert seen.most <= before + 8 + os.cpu_count() - 1
+
+
+THROWING = r"""
+#include "host_bin.h"
+#include <cstdio>
+#include <new>
+#include <thread>
+#include <unistd.h>
+int main() {
+    for (int rep = 0; rep < 50; rep++) {
+        const std::thread::id caller = std::this_thread::get_id();
+        std::atomic<int> done{0}, on_worker{0};
+        bool caught = false;
+        try { // the caller's own tasks are slow: workers take most of the others, and throw
+            hb_parallel(64, 3, [&](int) {
+                usleep(500);
+                if (std::this_thread::get_id() != caller) {
+                    on_worker++;
+                    throw std::bad_alloc();
+                }
+                done++;
+            });
+        } catch (const std::bad_alloc &) {
+            caught = true;
+        }
+        if (caught != (on_worker > 0) || (!caught && done != 64)) return 1;
+        if (rep == 49 && !caught) return 2;
+        std::atomic<int> after{0};
+        hb_parallel(64, 3, [&](int) { after++; });
+        if (after != 64) return 3;
+    }
+    puts("ok");
+}
+"""
+
+
+def test_an_exception_of_a_worker_is_the_callers(evt, tmp_path):
+    """The worker threads as they are, in a program of their own: an exception there ended the process."""
+    if os.cpu_count() < 2:
+        pytest.skip("no worker beside the caller")
+    csrc = os.path.join(os.path.dirname(evt.__file__), "csrc")
+    (tmp_path / "main.cpp").write_text(THROWING)
+    exe = str(tmp_path / "main")
+    subprocess.run(["g++", "-x", "c++", "-O0", "-std=c++17", "-I", csrc, str(tmp_path / "main.cpp"), os.path.join(csrc, "host_bin.cpp"),
+                    os.path.join(csrc, "host_bin_avx512.cpp"), "-o", exe, "-pthread"], check=True)
+    run = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert (run.returncode, run.stdout) == (0, "ok\n"), run.stderr
 
 
 def test_the_smallest_and_largest_calls(evt):
