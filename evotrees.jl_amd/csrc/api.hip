@@ -585,7 +585,7 @@ static const int64_t UPLOAD_PIECE = (int64_t)32 << 20; // bytes
 // worker threads for an upload of this size: none below a few pieces, else up to six
 static int upload_workers(int64_t total_bytes) {
     if (total_bytes < 2 * UPLOAD_PIECE) return 0;
-    return (int)std::min<unsigned>(6, std::max(1u, std::thread::hardware_concurrency() / 2));
+    return (int)std::min(6, std::max(1, hb_cores() / 2));
 }
 // nbytes from the caller's memory to the device: large host buffers go through pinned buffers,
 // everything else is a plain copy.  The data has arrived when the call returns.

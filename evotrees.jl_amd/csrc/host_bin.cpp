@@ -1,6 +1,8 @@
 #include "host_bin.h"
 
 #include <math.h>
+#include <sched.h>
+#include <stdio.h>
 #include <string.h>
 #include <unistd.h>
 
@@ -21,10 +23,30 @@ bool hb_has_avx512() {
 #endif
 }
 
+// Cores that the container's CPU quota pays for (a process that runs on more is stopped for the rest of each period), or no limit.
+static int quota_cores(const char *cpu_max, const char *cfs_quota, const char *cfs_period) {
+    auto words = [](const char *path, long long *v, int most) { // the numbers a file starts with
+        int n = 0;
+        if (FILE *f = fopen(path, "r")) {
+            while (n < most && fscanf(f, "%lld", &v[n]) == 1) n++;
+            fclose(f);
+        }
+        return n;
+    };
+    long long v[2];
+    const bool have = words(cpu_max, v, 2) == 2 || (words(cfs_quota, v, 1) == 1 && words(cfs_period, v + 1, 1) == 1);
+    return have && v[0] > 0 && v[1] > 0 ? (int)std::max(1ll, std::min(1ll << 20, (v[0] + v[1] - 1) / v[1])) : 1 << 20;
+}
+int hb_cores() {
+    static const int quota = quota_cores("/sys/fs/cgroup/cpu.max", "/sys/fs/cgroup/cpu/cpu.cfs_quota_us", "/sys/fs/cgroup/cpu/cpu.cfs_period_us");
+    cpu_set_t set;
+    const int mine = sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : (int)std::thread::hardware_concurrency();
+    return std::max(1, std::min(mine, quota));
+}
 int hb_workers(int64_t cells) {
     // a worker takes about 5 us to wake, in which the calling thread bins 8k cells
-    static const int64_t most = std::max(1, (int)std::thread::hardware_concurrency()) - 1;
-    return (int)std::max<int64_t>(0, std::min<int64_t>(most, cells / 16384 - 1));
+    const int64_t worth = cells / 16384 - 1;
+    return worth <= 0 ? 0 : (int)std::min<int64_t>(hb_cores() - 1, worth);
 }
 
 // The worker threads: started when first needed, kept asleep between calls (waking one costs about 5 us, starting one 15 and more), at
@@ -42,7 +64,7 @@ struct Region {
 };
 struct Pool {
     const pid_t pid = getpid();
-    const int most = std::max(1, (int)std::thread::hardware_concurrency()) - 1;
+    int most = 0; // of the callers seen, each with its own affinity
     std::mutex m;
     std::condition_variable cv, cv_done;
     int threads = 0;
@@ -88,6 +110,7 @@ struct Pool {
         std::lock_guard<std::mutex> lk(m);
         regions.push_back(r);
         open.store((int)regions.size(), std::memory_order_relaxed);
+        most = std::max(most, hb_cores() - 1);
         int need = 0;
         for (const Region *o : regions) need += o->wanted + o->active;
         try {

@@ -41,6 +41,7 @@ struct HbPlan {
 // rows [r0, r0 + n) of features [f0, f1): the bin of (r, f) goes to out + (f - f0) * ldo + (r - r0)
 void hb_bin(const HbPlan &P, const HbSource &S, int64_t r0, int64_t n, int f0, int f1, uint8_t *out, int64_t ldo);
 bool hb_has_avx512();
+int hb_cores(); // that the calling thread may use: its affinity, within the container's CPU quota
 // worker threads worth starting for this much work, the calling thread not counted (0: none)
 int hb_workers(int64_t cells);
 

@@ -164,6 +164,34 @@ def test_an_exception_of_a_worker_is_the_callers(evt, tmp_path):
     assert (run.returncode, run.stdout) == (0, "ok\n"), run.stderr
 
 
+QUOTA = r"""
+#include "host_bin.cpp"
+int main(int, char **a) {
+    printf("%d %d\n", quota_cores(a[1], a[2], a[3]) >> 20 ? -1 : quota_cores(a[1], a[2], a[3]), hb_cores());
+}
+"""
+
+
+def test_cores_are_counted_within_affinity_and_quota(evt, tmp_path):
+    csrc = os.path.join(os.path.dirname(evt.__file__), "csrc")
+    (tmp_path / "main.cpp").write_text(QUOTA)
+    exe = str(tmp_path / "main")
+    subprocess.run(["g++", "-x", "c++", "-O0", "-std=c++17", "-I", csrc, str(tmp_path / "main.cpp"), os.path.join(csrc, "host_bin_avx512.cpp"), "-o", exe,
+                    "-pthread"], check=True)
+    for cpu_max, quota, period, want in (("max 100000", None, None, -1), ("1600000 100000", None, None, 16), ("150000 100000", None, None, 2),
+                                         (None, "-1", "100000", -1), (None, "50000", "100000", 1), (None, None, None, -1), ("", "200000", "100000", 2)):
+        files = []
+        for name, text in (("max", cpu_max), ("quota", quota), ("period", period)):
+            files.append(str(tmp_path / name))
+            if text is None and os.path.exists(files[-1]):
+                os.remove(files[-1])
+            elif text is not None:
+                open(files[-1], "w").write(text + "\n")
+        one = min(os.sched_getaffinity(0))
+        got = subprocess.run([exe] + files, capture_output=True, text=True, preexec_fn=lambda: os.sched_setaffinity(0, {one})).stdout
+        assert got == "%d 1\n" % want
+
+
 def test_the_smallest_and_largest_calls(evt):
     """No rows, no columns, no edges, more edges than a bin's byte counts (it wraps): what numpy's search gives."""
     rng = np.random.default_rng(0)
