@@ -64,7 +64,7 @@ struct Region {
 };
 struct Pool {
     const pid_t pid = getpid();
-    int most = 0; // of the callers seen, each with its own affinity
+    int most = 0; // threads: the most that a region has asked for, each caller's cores less one
     std::mutex m;
     std::condition_variable cv, cv_done;
     int threads = 0;
@@ -107,17 +107,20 @@ struct Pool {
         }
     }
     void enter(Region *r) {
-        std::lock_guard<std::mutex> lk(m);
-        regions.push_back(r);
-        open.store((int)regions.size(), std::memory_order_relaxed);
-        most = std::max(most, hb_cores() - 1);
-        int need = 0;
-        for (const Region *o : regions) need += o->wanted + o->active;
-        try {
-            for (; threads < std::min(need, most); threads++) std::thread([this] { loop(); }).detach();
-        } catch (const std::exception &) { // no more threads to be had: the callers do their work themselves
+        const int n = r->wanted;
+        {
+            std::lock_guard<std::mutex> lk(m);
+            regions.push_back(r);
+            open.store((int)regions.size(), std::memory_order_relaxed);
+            most = std::max(most, n);
+            int need = 0;
+            for (const Region *o : regions) need += o->wanted + o->active;
+            try {
+                for (; threads < std::min(need, most); threads++) std::thread([this] { loop(); }).detach();
+            } catch (const std::exception &) { // no more threads to be had: the callers do their work themselves
+            }
         }
-        for (int i = 0; i < r->wanted; i++) cv.notify_one();
+        for (int i = 0; i < n; i++) cv.notify_one(); // the lock is free: a worker that wakes does not wait for it
     }
     void leave(Region *r) { // workers that have not joined by now do not; those that have are waited for
         std::unique_lock<std::mutex> lk(m);
