@@ -203,8 +203,8 @@ extern "C" int evt_destroy(evt_handle c) {
     for (hipEvent_t e : c->tree_evs)
         if (e) (void)hipEventDestroy(e);
     pinned_give(c->pt_stage);
-    if (c->copy_stream) stream_give(c->copy_stream, true);
-    if (c->stream) stream_give(c->stream, false);
+    if (c->copy_stream) stream_give(c->copy_stream, true, c->device);
+    if (c->stream) stream_give(c->stream, false, c->device);
     delete c;
     return EVT_OK;
     });
@@ -334,7 +334,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     if (e == hipSuccess) e = hipEventCreateWithFlags(&c->tree_evs[1], hipEventDisableTiming);
     if (e != hipSuccess) {
         evt_set_error("stream creation failed: %s", hipGetErrorString(e));
-        if (c->stream) stream_give(c->stream, false);
+        if (c->stream) stream_give(c->stream, false, c->device);
         delete c;
         return EVT_ERR_HIP;
     }

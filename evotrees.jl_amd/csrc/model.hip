@@ -25,8 +25,7 @@ struct CompletedTree { // as k_predict_model_lds and k_walk_rows read it
 
 struct Model {
     std::mutex mu;
-    int device = 0, loss = 0, K = 0;
-    hipStream_t s = nullptr;
+    int loss = 0, K = 0;
     // the caller's arrays as they were when the device form was built
     std::vector<int32_t> nn;
     std::vector<int64_t> feat;
@@ -34,8 +33,11 @@ struct Model {
     std::vector<float> pred;
     std::vector<double> edges;
     std::vector<int32_t> edge_off;
-    // device form: trees completed to their depth, `stride` node words each, padded to a multiple of four trees
+    // device form: trees completed to their depth, `stride` node words each, padded to a multiple of four trees; on the device that
+    // was current in the call that built it
     bool built = false;
+    int device = -1;
+    hipStream_t s = nullptr; // idle between calls
     int ntrees = 0, max_int = 0, max_feat = 0, max_nodes = 0;
     bool all_numeric = true, wide = false;
     uint32_t *d_nodes = nullptr, *d_cid = nullptr;
@@ -48,13 +50,16 @@ struct Model {
     uint8_t *d_x = nullptr;          // bins of the pieces in flight
     size_t cap_x = 0;
 
-    ~Model() {
-        (void)hipSetDevice(device);
-        if (s) (void)hipStreamSynchronize(s);
-        void *p[] = {d_form, d_x};
-        for (void *q : p) dev_give(q);
-        if (s) stream_give(s, true);
+    void drop() { // what lies on the device: no call is running, and each has waited for its stream
+        built = false;
+        dev_give(d_form);
+        dev_give(d_x);
+        if (s) stream_give(s, true, device);
+        s = nullptr;
+        d_form = d_x = nullptr;
+        cap_form = cap_x = 0;
     }
+    ~Model() { drop(); }
 };
 
 int grow(uint8_t **p, size_t *cap, size_t n) {
@@ -177,7 +182,7 @@ int build(Model &m, const TreePtrs &t, const uint8_t *feattypes, int nft) {
     auto up = [](size_t n) { return (n + 255) / 256 * 256; };
     const size_t o_nodes = up(sizeof(CompletedTree) * m.meta.size()), o_cid = o_nodes + up(4 * nodes.size()), o_leaf = o_cid + up(4 * cid.size());
     const size_t bytes = o_leaf + up(4 * leaf.size());
-    HIPCHK(hipStreamSynchronize(m.s));
+    HIPCHK(hipStreamSynchronize(m.s)); // a walk of the old form
     const int r = grow(&m.d_form, &m.cap_form, bytes);
     if (r != EVT_OK) return r;
     struct Staged { // pinned, and given back whichever way the call ends
@@ -328,8 +333,6 @@ extern "C" int evt_model_create(int32_t loss, int32_t K, void **out) {
     std::unique_ptr<Model> m(new Model());
     m->loss = loss;
     m->K = K;
-    HIPCHK(hipGetDevice(&m->device));
-    HIPCHK(stream_take(&m->s, true));
     *out = m.release();
     return EVT_OK;
     });
@@ -351,7 +354,11 @@ extern "C" int evt_model_predict(void *model, int32_t n_model, const int64_t *nn
     ARGCHK((out != nullptr) != (leaf_out != nullptr), "one of out and leaf_out");
     Model &m = *static_cast<Model *>(model);
     std::lock_guard<std::mutex> lock(m.mu);
-    HIPCHK(hipSetDevice(m.device));
+    int device = 0; // the caller's, as for the whole-model calls
+    HIPCHK(hipGetDevice(&device));
+    if (m.device != device) m.drop();
+    m.device = device;
+    if (!m.s) HIPCHK(stream_take(&m.s, true));
     const TreePtrs t{n_model, nnodes, feat, cond_bin, split, pred};
     const size_t nft = feattypes ? (size_t)nfeattypes : 0;
     // The trees are compared with the device form while the device already walks it (20 us for 700 KB of trees); if they turn out to

@@ -14,4 +14,4 @@ void dev_give(void *p);
 void *pinned_take(size_t bytes); // portable, at the same address on host and device; nullptr: the error is set
 void pinned_give(void *p);
 hipError_t stream_take(hipStream_t *s, bool non_blocking); // on the current device
-void stream_give(hipStream_t s, bool non_blocking);        // idle
+void stream_give(hipStream_t s, bool non_blocking, int device); // idle; a stream of that device

@@ -14,8 +14,8 @@ struct Block {
 std::unordered_map<void *, Block> g_out[2];                            // blocks in use: device, pinned
 std::multimap<std::pair<int, size_t>, void *> g_idle[2];               // by (device, size); pinned blocks under device 0
 std::map<int, size_t> g_kept[2];                                       // idle bytes by device
-std::multimap<int, hipStream_t> g_streams[2];                          // blocking, non-blocking
-const size_t STREAMS_KEPT = 4;
+std::map<int, std::vector<hipStream_t>> g_streams[2];                  // idle ones by device, the last used at the end: blocking, non-blocking
+const size_t STREAMS_KEPT = 16; // per device and kind
 
 // sizes are rounded up by an eighth at most, so that inputs of about the same size find each other's blocks
 size_t size_class(size_t n) {
@@ -108,21 +108,21 @@ hipError_t stream_take(hipStream_t *s, bool non_blocking) {
     const int dev = current_device();
     {
         std::lock_guard<std::mutex> lk(g_mu);
-        auto it = g_streams[non_blocking].find(dev);
-        if (it != g_streams[non_blocking].end()) {
-            *s = it->second;
-            g_streams[non_blocking].erase(it);
+        std::vector<hipStream_t> &idle = g_streams[non_blocking][dev];
+        if (!idle.empty()) {
+            *s = idle.back();
+            idle.pop_back();
             return hipSuccess;
         }
     }
     return hipStreamCreateWithFlags(s, non_blocking ? hipStreamNonBlocking : hipStreamDefault);
 }
-void stream_give(hipStream_t s, bool non_blocking) {
-    const int dev = current_device();
+void stream_give(hipStream_t s, bool non_blocking, int dev) {
     {
         std::lock_guard<std::mutex> lk(g_mu);
-        if (g_streams[non_blocking].count(dev) < STREAMS_KEPT) {
-            g_streams[non_blocking].insert({dev, s});
+        std::vector<hipStream_t> &idle = g_streams[non_blocking][dev];
+        if (idle.size() < STREAMS_KEPT) {
+            idle.push_back(s);
             return;
         }
     }
@@ -137,7 +137,7 @@ extern "C" int evt_trim(void) {
     {
         std::lock_guard<std::mutex> lk(g_mu);
         for (auto &q : g_streams) {
-            for (auto &e : q) idle.push_back(e.second);
+            for (auto &e : q) idle.insert(idle.end(), e.second.begin(), e.second.end());
             q.clear();
         }
     }
