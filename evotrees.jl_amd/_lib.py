@@ -142,6 +142,11 @@ def device_count():
     return n.value
 
 
+def trim():
+    """Gives back the memory that the library keeps between calls, on the device and pinned, and what kept models hold."""
+    check(load().evt_trim())
+
+
 def copy_bandwidth(nbytes=1 << 30, iters=10):
     out = C.c_double(0.0)
     check(load().evt_copy_bandwidth(nbytes, iters, C.byref(out)))

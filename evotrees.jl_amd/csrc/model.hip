@@ -7,6 +7,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <list>
 #include <memory>
 #include <mutex>
 
@@ -37,7 +38,6 @@ struct Model {
     // was current in the call that built it
     bool built = false;
     int device = -1;
-    hipStream_t s = nullptr; // idle between calls
     int ntrees = 0, max_int = 0, max_feat = 0, max_nodes = 0;
     bool all_numeric = true, wide = false;
     uint32_t *d_nodes = nullptr, *d_cid = nullptr;
@@ -47,30 +47,91 @@ struct Model {
     size_t cap_form = 0;
     std::vector<CompletedTree> meta;
     std::unique_ptr<HbPlan> plan[2]; // by source type
-    uint8_t *d_x = nullptr;          // bins of the pieces in flight
-    size_t cap_x = 0;
+    size_t kept = 0;                 // bytes it is counted with in Kept; under Kept::mu, as the place in its list
+    std::list<Model *>::iterator at;
 
-    void drop() { // what lies on the device: no call is running, and each has waited for its stream
+    size_t bytes() const {
+        size_t n = cap_form + 4 * nn.capacity() + 8 * feat.capacity() + cond_bin.capacity() + split.capacity() + feattypes.capacity() +
+                   4 * pred.capacity() + 8 * edges.capacity() + 4 * edge_off.capacity() + sizeof(CompletedTree) * meta.capacity();
+        for (const auto &p : plan)
+            if (p) n += sizeof(HbFeature) * p->feat.capacity() + 8 * p->edges.capacity() + 4 * p->heap_store.capacity();
+        return n;
+    }
+    void drop() { // all that a call can make again; no call is running, and each has waited for its stream
         built = false;
         dev_give(d_form);
-        dev_give(d_x);
-        if (s) stream_give(s, true, device);
-        s = nullptr;
-        d_form = d_x = nullptr;
-        cap_form = cap_x = 0;
+        d_form = nullptr;
+        cap_form = 0;
+        std::vector<int32_t>().swap(nn);
+        std::vector<int64_t>().swap(feat);
+        std::vector<float>().swap(pred);
+        std::vector<double>().swap(edges);
+        std::vector<int32_t>().swap(edge_off);
+        std::vector<CompletedTree>().swap(meta);
+        for (auto *v : {&cond_bin, &split, &feattypes}) std::vector<uint8_t>().swap(*v);
+        for (auto &p : plan) p.reset();
     }
     ~Model() { drop(); }
 };
 
-int grow(uint8_t **p, size_t *cap, size_t n) {
-    if (*cap >= n) return EVT_OK;
-    dev_give(*p);
-    *cap = 0;
-    *p = static_cast<uint8_t *>(dev_take(n));
-    if (!*p) return EVT_ERR_NOMEM;
-    *cap = n;
-    return EVT_OK;
-}
+// All models, the last used first.  What they keep on the device and beside it is bounded together; beyond it those not used for longest
+// are packed anew by their next call (0.6 ms for 100 trees of depth 6, 1.3 ms for 200 of depth 8).
+struct Kept {
+    static const size_t MOST = (size_t)1 << 30; // bytes: some 800 models of 200 trees of depth 8
+    std::mutex mu;
+    std::list<Model *> models;
+    size_t bytes = 0;
+    static Kept &get() { // never destroyed: models outlive main
+        static Kept *k = new Kept();
+        return *k;
+    }
+    void count(Model *m, size_t n) {
+        bytes += n - m->kept;
+        m->kept = n;
+    }
+    void add(Model *m) {
+        std::lock_guard<std::mutex> lk(mu);
+        m->at = models.insert(models.end(), m);
+    }
+    void remove(Model *m) {
+        std::lock_guard<std::mutex> lk(mu);
+        count(m, 0);
+        models.erase(m->at);
+    }
+    void used(Model *m) { // by a call that holds its lock and is about to end
+        std::lock_guard<std::mutex> lk(mu);
+        count(m, m->bytes());
+        models.splice(models.begin(), models, m->at);
+        shrink(MOST, m);
+    }
+    void shrink(size_t most, Model *mine) {
+        for (auto it = models.rbegin(); it != models.rend() && bytes > most; ++it) {
+            Model *o = *it;
+            if (!o->kept) continue;
+            std::unique_lock<std::mutex> lk(o->mu, std::defer_lock);
+            if (o != mine && !lk.try_lock()) continue; // in a call: it comes by here at its end
+            o->drop();
+            count(o, 0);
+        }
+    }
+};
+
+// A stream for one call, on the current device.
+struct CallStream {
+    hipStream_t s = nullptr;
+    int device = 0;
+    bool idle = false; // the call has waited for all it queued
+    ~CallStream() {
+        if (!s) return;
+        if (!idle) (void)hipStreamSynchronize(s);
+        stream_give(s, true, device);
+    }
+};
+// Device memory for one call, given back when nothing uses it any more: declared before what waits for the stream.
+struct CallBuffer {
+    uint8_t *p = nullptr;
+    ~CallBuffer() { dev_give(p); }
+};
 
 struct TreePtrs {
     int32_t n;
@@ -100,7 +161,7 @@ bool same_trees(const Model &m, const TreePtrs &t) { // of trees of the same sha
 }
 
 // Copies the caller's arrays, checks them by the rules of evt_predict, completes the trees and uploads them.
-int build(Model &m, const TreePtrs &t, const uint8_t *feattypes, int nft) {
+int build(Model &m, const TreePtrs &t, const uint8_t *feattypes, int nft, hipStream_t s) {
     m.built = false;
     size_t total = 0;
     int levels_max = 0;
@@ -182,9 +243,13 @@ int build(Model &m, const TreePtrs &t, const uint8_t *feattypes, int nft) {
     auto up = [](size_t n) { return (n + 255) / 256 * 256; };
     const size_t o_nodes = up(sizeof(CompletedTree) * m.meta.size()), o_cid = o_nodes + up(4 * nodes.size()), o_leaf = o_cid + up(4 * cid.size());
     const size_t bytes = o_leaf + up(4 * leaf.size());
-    HIPCHK(hipStreamSynchronize(m.s)); // a walk of the old form
-    const int r = grow(&m.d_form, &m.cap_form, bytes);
-    if (r != EVT_OK) return r;
+    if (m.cap_form < bytes) { // no walk of the old form is running: each has been waited for
+        dev_give(m.d_form);
+        m.cap_form = 0;
+        m.d_form = static_cast<uint8_t *>(dev_take(bytes));
+        if (!m.d_form) return EVT_ERR_NOMEM;
+        m.cap_form = bytes;
+    }
     struct Staged { // pinned, and given back whichever way the call ends
         void *p;
         ~Staged() { pinned_give(p); }
@@ -195,8 +260,8 @@ int build(Model &m, const TreePtrs &t, const uint8_t *feattypes, int nft) {
     memcpy(h + o_nodes, nodes.data(), 4 * nodes.size());
     memcpy(h + o_cid, cid.data(), 4 * cid.size());
     memcpy(h + o_leaf, leaf.data(), 4 * leaf.size());
-    const hipError_t e = hipMemcpyAsync(m.d_form, h, bytes, hipMemcpyHostToDevice, m.s);
-    const hipError_t e2 = hipStreamSynchronize(m.s);
+    const hipError_t e = hipMemcpyAsync(m.d_form, h, bytes, hipMemcpyHostToDevice, s);
+    const hipError_t e2 = hipStreamSynchronize(s);
     HIPCHK(e);
     HIPCHK(e2);
     m.d_meta = reinterpret_cast<CompletedTree *>(m.d_form);
@@ -223,15 +288,15 @@ struct Request {
     bool differ;           // they are not the same: the results are those of the old trees
 };
 
-int walk(Model &m, const Request &q, const uint8_t *x, int64_t n, void *out, int leaf_bytes) {
+int walk(Model &m, hipStream_t s, const Request &q, const uint8_t *x, int64_t n, void *out, int leaf_bytes) {
     if (q.leaf_out)
-        return launch_walk_rows(m.s, m.d_nodes, std::max(1, m.max_int), m.d_meta, m.d_leaf, m.d_cid, q.ntrees, x, n, n, q.F, m.wide, m.K, m.loss, 0, nullptr, out,
+        return launch_walk_rows(s, m.d_nodes, std::max(1, m.max_int), m.d_meta, m.d_leaf, m.d_cid, q.ntrees, x, n, n, q.F, m.wide, m.K, m.loss, 0, nullptr, out,
                                 leaf_bytes, n);
     const int shape = n >= WALK_LDS_MIN_ROWS ? predict_lds_shape(q.F, m.max_int, m.K, 0) : 0;
     if (shape > 0)
-        return launch_predict_model_lds(m.s, m.d_nodes, m.d_leaf, m.d_meta, q.ntrees, x, n, q.F, m.max_int, m.K, m.loss, q.link, m.all_numeric ? 1 : 0, shape,
+        return launch_predict_model_lds(s, m.d_nodes, m.d_leaf, m.d_meta, q.ntrees, x, n, q.F, m.max_int, m.K, m.loss, q.link, m.all_numeric ? 1 : 0, shape,
                                         static_cast<float *>(out));
-    return launch_walk_rows(m.s, m.d_nodes, std::max(1, m.max_int), m.d_meta, m.d_leaf, m.d_cid, q.ntrees, x, n, n, q.F, m.wide, m.K, m.loss, q.link,
+    return launch_walk_rows(s, m.d_nodes, std::max(1, m.max_int), m.d_meta, m.d_leaf, m.d_cid, q.ntrees, x, n, n, q.F, m.wide, m.K, m.loss, q.link,
                             static_cast<float *>(out), nullptr, 0, 0);
 }
 
@@ -240,7 +305,7 @@ void widen(const T *src, uint32_t *dst, int64_t n) {
     for (int64_t i = 0; i < n; i++) dst[i] = src[i];
 }
 
-int run(Model &m, Request &q) {
+int run(Model &m, hipStream_t s, Request &q) {
     const int leaf_bytes = !q.leaf_out ? 0 : m.max_nodes <= 255 ? 1 : m.max_nodes <= 65535 ? 2 : 4;
     const int64_t back = q.leaf_out ? (int64_t)q.ntrees * leaf_bytes : (int64_t)m.K * 4; // bytes a row sends back
     const int64_t per_row = q.F + back;
@@ -253,13 +318,14 @@ int run(Model &m, Request &q) {
     const BinPieces B(q.N, q.F, rowwise, true, rows_most, 0);
     const int NS = (int)std::min<int64_t>(PinnedSlots::NS, B.np);
     const size_t xs = ((size_t)B.rows * q.F + 255) / 256 * 256; // a buffer holds a piece's bins, then what comes back
-    PinnedSlots U(m.s);
+    CallBuffer d_x; // bins of the pieces in flight
+    PinnedSlots U(s);
     int r = U.init(NS);
     if (r != EVT_OK) return r;
     const bool direct = B.np == 1 && (int64_t)q.N * q.F <= 65536; // a few bins are read over the bus by the kernel itself
     if (!direct) {
-        r = grow(&m.d_x, &m.cap_x, xs * NS);
-        if (r != EVT_OK) return r;
+        d_x.p = static_cast<uint8_t *>(dev_take(xs * NS));
+        if (!d_x.p) return EVT_ERR_NOMEM;
     }
     auto piece = [&](int64_t p, int64_t *r0, int64_t *n) {
         int f0, f1;
@@ -283,12 +349,12 @@ int run(Model &m, Request &q) {
         uint8_t *h = static_cast<uint8_t *>(U.host[p % NS]);
         const uint8_t *x = h;
         if (!direct) {
-            HIPCHK(hipMemcpyAsync(m.d_x + (p % NS) * xs, h, (size_t)n * q.F, hipMemcpyHostToDevice, m.s));
-            x = m.d_x + (p % NS) * xs;
+            HIPCHK(hipMemcpyAsync(d_x.p + (p % NS) * xs, h, (size_t)n * q.F, hipMemcpyHostToDevice, s));
+            x = d_x.p + (p % NS) * xs;
         }
-        const int rw = walk(m, q, x, n, h + xs, leaf_bytes); // the kernel writes what comes back over the bus itself
+        const int rw = walk(m, s, q, x, n, h + xs, leaf_bytes); // the kernel writes what comes back over the bus itself
         if (rw != EVT_OK) return rw;
-        if (!direct) HIPCHK(hipEventRecord(U.ev[p % NS], m.s));
+        if (!direct) HIPCHK(hipEventRecord(U.ev[p % NS], s));
         if (p == 0 && q.check) q.differ = !same_trees(m, *q.check);
         return EVT_OK;
     };
@@ -312,7 +378,7 @@ int run(Model &m, Request &q) {
         for (int t = 0; t < B.per_piece; t++) fill(0, t);
         r = send(0);
         if (r != EVT_OK) return r;
-        HIPCHK(hipStreamSynchronize(m.s));
+        HIPCHK(hipStreamSynchronize(s));
         U.idle = true;
         retire(0);
         return EVT_OK;
@@ -333,15 +399,24 @@ extern "C" int evt_model_create(int32_t loss, int32_t K, void **out) {
     std::unique_ptr<Model> m(new Model());
     m->loss = loss;
     m->K = K;
+    Kept::get().add(m.get());
     *out = m.release();
     return EVT_OK;
     });
 }
 extern "C" int evt_model_destroy(void *model) {
     return guarded([&]() -> int {
+    if (!model) return EVT_OK;
+    Kept::get().remove(static_cast<Model *>(model));
     delete static_cast<Model *>(model);
     return EVT_OK;
     });
+}
+
+void models_trim() {
+    Kept &k = Kept::get();
+    std::lock_guard<std::mutex> lk(k.mu);
+    k.shrink(0, nullptr);
 }
 
 extern "C" int evt_model_predict(void *model, int32_t n_model, const int64_t *nnodes, const int64_t *const *feat, const uint8_t *const *cond_bin,
@@ -354,30 +429,38 @@ extern "C" int evt_model_predict(void *model, int32_t n_model, const int64_t *nn
     ARGCHK((out != nullptr) != (leaf_out != nullptr), "one of out and leaf_out");
     Model &m = *static_cast<Model *>(model);
     std::lock_guard<std::mutex> lock(m.mu);
-    int device = 0; // the caller's, as for the whole-model calls
-    HIPCHK(hipGetDevice(&device));
-    if (m.device != device) m.drop();
-    m.device = device;
-    if (!m.s) HIPCHK(stream_take(&m.s, true));
+    struct Used {
+        Model *m;
+        ~Used() { Kept::get().used(m); }
+    } on_return{&m};
+    CallStream call;
+    HIPCHK(hipGetDevice(&call.device)); // the caller's, as for the whole-model calls
+    if (m.device != call.device) m.drop();
+    m.device = call.device;
+    HIPCHK(stream_take(&call.s, true));
+    const hipStream_t s = call.s;
     const TreePtrs t{n_model, nnodes, feat, cond_bin, split, pred};
     const size_t nft = feattypes ? (size_t)nfeattypes : 0;
     // The trees are compared with the device form while the device already walks it (20 us for 700 KB of trees); if they turn out to
     // have changed, the new ones are packed and the call runs again.
     bool known = m.feattypes.size() == nft && (!nft || !memcmp(m.feattypes.data(), feattypes, nft)) && same_shape(m, t) && m.max_feat <= nfeats;
     if (!known) {
-        const int r = build(m, t, feattypes, nfeattypes);
+        const int r = build(m, t, feattypes, nfeattypes, s);
         if (r != EVT_OK) return r;
     }
     auto walk_all = [&](Request &q) -> int {
         q.check = known ? &t : nullptr;
         q.differ = false;
-        int r = run(m, q);
-        if (r != EVT_OK || !q.differ) return r;
-        r = build(m, t, feattypes, nfeattypes);
-        if (r != EVT_OK) return r;
-        ARGCHK(m.max_feat <= nfeats, "tree feature id outside 1..nfeats");
-        q.check = nullptr;
-        return run(m, q);
+        int r = run(m, s, q);
+        if (r == EVT_OK && q.differ) {
+            r = build(m, t, feattypes, nfeattypes, s);
+            if (r != EVT_OK) return r;
+            ARGCHK(m.max_feat <= nfeats, "tree feature id outside 1..nfeats");
+            q.check = nullptr;
+            r = run(m, s, q);
+        }
+        call.idle = r == EVT_OK;
+        return r;
     };
     ARGCHK(m.max_feat <= nfeats, "tree feature id outside 1..nfeats");
     Request q{nullptr, {}, nullptr, nobs, nfeats, ntrees, apply_link, out, leaf_out, nullptr, false};

@@ -15,3 +15,5 @@ void *pinned_take(size_t bytes); // portable, at the same address on host and de
 void pinned_give(void *p);
 hipError_t stream_take(hipStream_t *s, bool non_blocking); // on the current device
 void stream_give(hipStream_t s, bool non_blocking, int device); // idle; a stream of that device
+
+void models_trim(); // what models keep between their calls, but for those in one (model.hip)

@@ -131,6 +131,7 @@ void stream_give(hipStream_t s, bool non_blocking, int dev) {
 
 extern "C" int evt_trim(void) {
     return guarded([&]() -> int {
+    models_trim();
     trim(0);
     trim(1);
     std::vector<hipStream_t> idle;

@@ -128,8 +128,8 @@ const char *evt_last_error(void);
 /* Number of visible HIP devices; fails (EVT_ERR_HIP) when the runtime finds none. */
 int evt_device_count(int32_t *count);
 
-/* Gives back what the library keeps between calls for the next handle, model or matrix: device buffers (at most 1 GB per device),
- * pinned ones (64 MB) and streams. */
+/* Gives back what the library keeps between calls: device buffers (at most 1 GB per device), pinned ones (64 MB) and streams for the next
+ * handle, model or matrix, and what models keep for their next call (1 GB in all; evt_model_predict). */
 int evt_trim(void);
 
 /* ---- training cache ------------------------------------------------------------------
@@ -345,7 +345,10 @@ int evt_predict_leaf_idx(int64_t nobs, int32_t nfeats, const uint8_t *x_bin_colm
  * of the n_model trees are walked.  edges: nfeats pointers to ascending Float64 arrays of n_edges entries, and x is a matrix in
  * host memory as evt_binarize takes it; edges == NULL: x holds nobs x nfeats column-major bins (EVT_U8).  Exactly one of out
  * (K x nobs, link applied when apply_link != 0) and leaf_out (nobs x ntrees column-major) is not NULL; both are host memory.
- * Results equal evt_predict's and evt_predict_leaf_idx's, bit for bit.  Calls on one model from several threads take turns. */
+ * Results equal evt_predict's and evt_predict_leaf_idx's, bit for bit.  Calls on one model from several threads take turns.  The
+ * packed form lies on the device that is current in the call (packed again when that has changed).  All models together keep at most
+ * 1 GB between calls, on the device and beside it; beyond that, and after evt_trim, those not used for longest are packed again by
+ * their next call. */
 int evt_model_create(int32_t loss, int32_t K, void **out);
 int evt_model_destroy(void *model);
 int evt_model_predict(void *model, int32_t n_model, const int64_t *nnodes, const int64_t *const *feat, const uint8_t *const *cond_bin,

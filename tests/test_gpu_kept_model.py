@@ -3,6 +3,7 @@ rows-per-block of the row kernel and the hand-over to the 1024-row kernel, outpu
 import numpy as np
 import pytest
 
+from test_gpu_lifecycle import _free_bytes
 from test_gpu_parity import _random_tree
 
 pytestmark = pytest.mark.gpu
@@ -95,3 +96,45 @@ def test_takes_what_the_whole_model_calls_take(evt):
     for n in (2, 4):  # neither fewer columns than features nor more
         with pytest.raises(ValueError):
             evt.predict(m, rng.random((5, n)), ntree_limit=4)
+
+
+def test_what_models_keep_is_bounded_and_given_back(evt):
+    """Twelve models that would keep 860 MB on the device and 1.8 GB beside it: 1 GB at most stays, and nothing after a trim."""
+    rng = np.random.default_rng(5)
+    x = rng.random((3, 4), np.float32)
+    models = []
+    for _ in range(12):
+        m = _model(evt, rng, 4, 16, 16, "mse", [11])
+        m.trees = m.trees * 1000
+        models.append(m)
+    evt.predict(models[0], x)
+    evt._lib.trim()
+    free = _free_bytes()
+    want = [evt.predict(m, x) for m in models]
+    assert 0 < free - _free_bytes() < 500 << 20
+    for m, w in zip(models, want):  # those that went are packed again
+        assert np.array_equal(evt.predict(m, x), w)
+    evt._lib.trim()
+    assert _free_bytes() >= free
+    for m, w in zip(models[:2], want):
+        assert np.array_equal(evt.predict(m, x), w)
+
+
+def test_calls_of_several_threads_on_several_models(evt):
+    import threading
+    rng = np.random.default_rng(8)
+    x = rng.random((700, 6))
+    models = [_model(evt, rng, 6, 32, 1, "mse", [5] * 8) for _ in range(3)]
+    want = [evt.predict(m, x) for m in models]
+    same = [False] * 6
+
+    def work(k):
+        same[k] = all(np.array_equal(evt.predict(models[(k + i) % 3], x), want[(k + i) % 3]) for i in range(40))
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(6)]
+    for t in threads:
+        t.start()
+    for _ in range(10):
+        evt._lib.trim()  # beside them
+    for t in threads:
+        t.join()
+    assert all(same)
