@@ -130,8 +130,8 @@ class Tree(TreeArrays):
     """Tree{L,K} (src/structs.jl:77-106)."""
 
     @staticmethod
-    def bias(mu):
-        t = Tree(len(mu), 1)
+    def bias(mu, cell=None):
+        t = Tree(len(mu), 1, cell)
         t.pred[0, :] = mu
         return t
 
@@ -401,6 +401,7 @@ class Cache:
 
     def __init__(self, handle, rng, nfs, params, N, F, config=None):
         self.handle, self.rng, self.nfs, self.params, self.N, self.F, self.config = handle, rng, nfs, params, N, F, config
+        self.cell = [object()]  # of all trees of the fit (TreeArrays)
         self.pending = []  # trees queued on the device and not yet collected, oldest first (at most two)
 
 
@@ -455,12 +456,12 @@ def init(config, x_train, y_train=None, w_train=None, offset_train=None, feature
     h.set_target(y32, w, mu, offset)
     info = dict(nrounds=0, feature_names=feature_names, target_levels=target_levels, target_isordered=False, edges=edges, featbins=featbins,
                 feattypes=feattypes)
-    m = EvoTree(config.loss, K, [Tree.bias(mu)], info)
     nfs = int(np.ceil(config.colsample * F))
     params = make_params(config.eta, config.L2, config.lambda_, config.gamma, config.min_weight, config.bagging_size, True)
     if config.bagging_size == 1:
         h.set_option("grads_ahead", 1)  # the next round's gradient update runs while the host collects the tree
-    return m, Cache(h, rng, nfs, params, N, F, config)
+    cache = Cache(h, rng, nfs, params, N, F, config)
+    return EvoTree(config.loss, K, [Tree.bias(mu, cache.cell)], info), cache
 
 
 def _begin_tree(cache, config, first_of_round):
@@ -481,7 +482,7 @@ def _begin_tree(cache, config, first_of_round):
         _lib.check(_lib.load().evt_grow_tree_begin_staged(h._h, cond, _lib.ptr(js), js.shape[0], cache.params))
     else:
         _lib.check(_lib.load().evt_grow_tree_begin(h._h, None, cond, _lib.ptr(js), js.shape[0], cache.params))
-    cache.pending.append(Tree(h.K, h.nnodes))
+    cache.pending.append(Tree(h.K, h.nnodes, cache.cell))
 
 
 def grow_evotree(m, cache, config, more=False):

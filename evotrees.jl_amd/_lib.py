@@ -258,16 +258,19 @@ def order_stats(cols, idx, n, ranks):
 class TreeArrays:
     """Host arrays in the layout of Tree{L,K} (src/structs.jl:77-106)."""
 
-    replaced = 0  # how often an array of any tree has been replaced by another: KeptModel looks at the trees again then
-
-    def __init__(self, K, nnodes):
+    def __init__(self, K, nnodes, cell=None):
+        # the cell holds another object after every replacement of an array by another: KeptModel looks at its trees again then.  The trees
+        # of one fit share theirs, so that one look tells of all of them
         self.__dict__.update(feat=np.zeros(nnodes, np.int64), cond_bin=np.zeros(nnodes, np.uint8), w=np.zeros(nnodes, np.float32),
                              gain=np.zeros(nnodes, np.float32), pred=np.zeros((nnodes, K), np.float32),  # memory order of Julia's K x nnodes matrix
-                             split=np.zeros(nnodes, np.uint8))
+                             split=np.zeros(nnodes, np.uint8), _cell=[object()] if cell is None else cell)
 
     def __setattr__(self, name, value):
         self.__dict__[name] = value
-        TreeArrays.replaced += 1
+        self._cell[0] = object()
+
+    def __setstate__(self, state):
+        self.__dict__.update({"_cell": [object()]}, **state)
 
     def as_out(self):
         return EvtTreeOut(ptr(self.feat), ptr(self.cond_bin), ptr(self.w), ptr(self.gain), ptr(self.pred), ptr(self.split))
@@ -557,6 +560,9 @@ class KeptModel:
             pass
 
     def _take_trees(self, trees):
+        cells = {id(c): c for c in (getattr(t, "_cell", None) for t in trees)}.values()
+        # read before the arrays are: a replacement beside this call is seen by the next.  Trees that tell of none are looked at every time
+        seen = None if None in cells else [(c, c[0]) for c in cells]
         arrays = []
         for t in trees:
             a = (t.feat, t.cond_bin, t.pred, t.split)
@@ -573,7 +579,7 @@ class KeptModel:
         if len(arrays) * max(1, int(nn.max())) > 1 << 28:
             return False
         self._tree = ((len(trees), nn.ctypes.data) + tuple(at[k].ctypes.data for k in range(4)), at, nn, arrays)
-        self.trees = list(trees)
+        self.trees, self._seen = list(trees), seen
         return True
 
     def _take_edges(self, edges):
@@ -588,12 +594,11 @@ class KeptModel:
         """The addresses of the trees' arrays and of the edges, with the objects that keep them valid; None when the arrays are of
         types that are not kept."""
         with self._lock:
-            seen = TreeArrays.replaced
-            if self.trees is None or self._seen != seen or len(self.trees) != len(trees) or not all(map(operator.is_, self.trees, trees)):
+            if (self.trees is None or self._seen is None or not all([c[0] is s for c, s in self._seen]) or len(self.trees) != len(trees)
+                    or not all(map(operator.is_, self.trees, trees))):
                 self.trees = None
                 if not self._take_trees(trees):
                     return None
-                self._seen = seen
             if edges is not None and (self.edges is None or len(self.edges) != len(edges) or not all(map(operator.is_, self.edges, edges))):
                 self._take_edges(edges)
             return self._tree, self._edge if edges is not None else None

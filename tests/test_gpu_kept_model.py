@@ -138,3 +138,40 @@ def test_calls_of_several_threads_on_several_models(evt):
     for t in threads:
         t.join()
     assert all(same)
+
+
+def test_replaced_arrays_are_noticed_whatever_other_trees_do(evt):
+    """Replacements beside each other on many threads, on this model's trees and on others'; copies of a model; trees of a fit."""
+    import copy
+    import pickle
+    import threading
+    rng = np.random.default_rng(10)
+    x, y = rng.random((300, 5)), rng.random(300)
+    m = evt.fit(evt.EvoTreeRegressor(nrounds=6, max_depth=4), x_train=x, y_train=y, verbosity=0)
+    _check(evt, m, x)
+    for c in (copy.deepcopy(m), pickle.loads(pickle.dumps(m))):
+        _check(evt, c, x)
+        c.trees[3].pred = c.trees[3].pred * 2
+        _check(evt, c, x)
+    _check(evt, m, x)
+    # an assignment to another model's tree leaves this one's addresses as they are
+    kept = evt._kept[m]
+    before = kept._tree
+    evt.Tree(1, 3).pred = np.zeros((3, 1), np.float32)
+    c.trees[0].pred = c.trees[0].pred + 1
+    evt.predict(m, x)
+    assert kept._tree is before
+    stop = threading.Event()
+
+    def replace(k):
+        while not stop.is_set():
+            m.trees[1 + k].pred = m.trees[1 + k].pred * np.float32(1)
+    threads = [threading.Thread(target=replace, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for _ in range(40):
+        m.trees[6].pred = m.trees[6].pred + np.float32(0.5)
+        _check(evt, m, x[:20])
+    stop.set()
+    for t in threads:
+        t.join()
