@@ -17,8 +17,10 @@ std::map<int, size_t> g_kept[2];                                       // idle b
 std::map<int, std::vector<hipStream_t>> g_streams[2];                  // idle ones by device, the last used at the end: blocking, non-blocking
 const size_t STREAMS_KEPT = 16; // per device and kind
 
-// sizes are rounded up by an eighth at most, so that inputs of about the same size find each other's blocks
+// sizes are rounded up by an eighth at most, so that inputs of about the same size find each other's blocks; those of blocks that are
+// never kept only to whole pages
 size_t size_class(size_t n) {
+    if (n > POOL_BLOCK_KEPT) return (n + 4095) / 4096 * 4096;
     size_t step = 4096;
     while (step * 16 <= n) step <<= 1;
     return (n + step - 1) / step * step;
