@@ -693,7 +693,7 @@ extern "C" int evt_binarize_f64(evt_handle c, const double *x_colmajor, const do
     if (e == hipSuccess) e = hipMemcpyAsync(d_off, off.data(), sizeof(int32_t) * (c->F + 1), hipMemcpyHostToDevice, c->stream);
     int r = EVT_OK;
     if (e == hipSuccess) {
-        r = launch_binarize(c, x_colmajor, d_edges, d_off);
+        r = launch_binarize(c->stream, x_colmajor, EVT_F64, 1, c->N, d_edges, d_off, c->B - 1, c->xcm, c->N, c->F, c->N);
         e = hipStreamSynchronize(c->stream);
     }
     if (d_off) (void)hipFree(d_off);
@@ -1629,11 +1629,14 @@ static int predict_common(int64_t nobs, int32_t nfeats, const uint8_t *x_bin, co
     ARGCHK((x_bin || x_f64) && tree_off && feat && cond_bin && split, "NULL argument");
     ARGCHK(leaf_out || (pred && out && K >= 1 && K <= EVT_MAX_K && loss >= 0 && loss <= EVT_LOSS_LAST), "invalid prediction arguments");
     std::vector<int32_t> eoff;
+    int max_edges = 0;
     if (x_f64) {
         ARGCHK(edges && edge_off, "NULL argument");
         eoff.assign(edge_off, edge_off + nfeats + 1);
-        for (int j = 0; j < nfeats; j++)
+        for (int j = 0; j < nfeats; j++) {
             ARGCHK(eoff[j] >= 0 && eoff[j + 1] - eoff[j] >= 1 && eoff[j + 1] - eoff[j] <= 254, "each feature needs 1..254 edges");
+            max_edges = std::max(max_edges, eoff[j + 1] - eoff[j]);
+        }
     }
     int ndev = 0;
     int r = evt_device_count(&ndev);
@@ -1715,7 +1718,7 @@ static int predict_common(int64_t nobs, int32_t nfeats, const uint8_t *x_bin, co
         if (e == hipSuccess) e = hipMemcpy(d_edges, edges, sizeof(double) * eoff[nfeats], hipMemcpyDefault);
         if (e == hipSuccess) e = hipMemcpy(d_eoff, eoff.data(), sizeof(int32_t) * (nfeats + 1), hipMemcpyHostToDevice);
         if (e == hipSuccess) {
-            r = launch_binarize_cols(s, x_f64, d_edges, d_eoff, d_x, nobs, nfeats, nobs, nobs);
+            r = launch_binarize(s, x_f64, EVT_F64, 1, nobs, d_edges, d_eoff, max_edges, d_x, nobs, nfeats, nobs);
             if (r == EVT_OK) e = hipStreamSynchronize(s);
         }
         void *tmp[] = {d_edges, d_eoff};

@@ -364,10 +364,9 @@ int launch_validate_classes(evt_ctx *c);
 int launch_init_pred(evt_ctx *c, const float *mu_dev, const float *offset_dev);
 // data layout
 int launch_transpose_validate(evt_ctx *c);
-int launch_binarize(evt_ctx *c, const double *x_dev, const double *edges_dev, const int32_t *edge_off_dev);
 int launch_build_planes(evt_ctx *c);
-int launch_binarize_cols(hipStream_t s, const double *x_dev, const double *edges_dev, const int32_t *edge_off_dev, uint8_t *xcm, int64_t n,
-                         int F, int64_t ldx, int64_t ldo);
+int launch_binarize(hipStream_t s, const void *x_dev, int dtype, int64_t rs, int64_t cs, const double *edges_dev, const int32_t *edge_off_dev, int max_edges,
+                    uint8_t *xcm, int64_t n, int F, int64_t ldo);
 int launch_eval_metric(evt_ctx *c, int metric, double *partial);
 // tree
 int launch_tree_begin(evt_ctx *c);

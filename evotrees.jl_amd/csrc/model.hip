@@ -308,7 +308,8 @@ void widen(const T *src, uint32_t *dst, int64_t n) {
 int run(Model &m, hipStream_t s, Request &q) {
     const int leaf_bytes = !q.leaf_out ? 0 : m.max_nodes <= 255 ? 1 : m.max_nodes <= 65535 ? 2 : 4;
     const int64_t back = q.leaf_out ? (int64_t)q.ntrees * leaf_bytes : (int64_t)m.K * 4; // bytes a row sends back
-    const int64_t per_row = q.F + back;
+    const bool raw = q.plan && 64 * ((int64_t)q.src.esize() * q.F + back) <= (int64_t)PINNED_BYTES - 4096 && bins_by_device(q.src.dtype, q.N * q.F);
+    const int64_t cell = raw ? (int64_t)q.src.esize() : 1, per_row = q.F * cell + back;
     // pieces of a twelfth of the whole, so that binning, copies and kernels overlap; 256 KB at least, a buffer at most.  Leaf ids: of a
     // fourth, so that as many as fit the buffers are spread out into the caller's words (most of the work) together at the end
     const int64_t goal = std::min<int64_t>((int64_t)PINNED_BYTES - 4096, std::max<int64_t>(256 << 10, q.N * per_row / (q.leaf_out ? 4 : 12)));
@@ -317,15 +318,19 @@ int run(Model &m, hipStream_t s, Request &q) {
     const bool rowwise = q.plan && q.src.rows_contiguous();
     const BinPieces B(q.N, q.F, rowwise, true, rows_most, 0);
     const int NS = (int)std::min<int64_t>(PinnedSlots::NS, B.np);
-    const size_t xs = ((size_t)B.rows * q.F + 255) / 256 * 256; // a buffer holds a piece's bins, then what comes back
+    const size_t xd = ((size_t)B.rows * q.F + 255) / 256 * 256;        // a piece's bins on the device
+    const size_t xs = ((size_t)B.rows * q.F * cell + 255) / 256 * 256; // a pinned buffer holds them (or the values), then what comes back
     CallBuffer d_x; // bins of the pieces in flight
+    DeviceBins D;
     PinnedSlots U(s);
     int r = U.init(NS);
     if (r != EVT_OK) return r;
-    const bool direct = B.np == 1 && (int64_t)q.N * q.F <= 65536; // a few bins are read over the bus by the kernel itself
+    const bool direct = !raw && B.np == 1 && (int64_t)q.N * q.F <= 65536; // a few bins are read over the bus by the kernel itself
     if (!direct) {
-        d_x.p = static_cast<uint8_t *>(dev_take(xs * NS));
+        d_x.p = static_cast<uint8_t *>(dev_take(xd * NS));
         if (!d_x.p) return EVT_ERR_NOMEM;
+        if (raw) r = D.init(s, *q.plan, xs, NS);
+        if (r != EVT_OK) return r;
     }
     auto piece = [&](int64_t p, int64_t *r0, int64_t *n) {
         int f0, f1;
@@ -333,7 +338,9 @@ int run(Model &m, hipStream_t s, Request &q) {
     };
     auto fill = [&](int64_t p, int t) {
         uint8_t *h = static_cast<uint8_t *>(U.host[p % NS]);
-        if (q.plan) {
+        if (raw) {
+            B.copy(q.src, p, t, h);
+        } else if (q.plan) {
             B.bin(*q.plan, q.src, p, t, h);
         } else {
             int64_t r0, n;
@@ -349,8 +356,14 @@ int run(Model &m, hipStream_t s, Request &q) {
         uint8_t *h = static_cast<uint8_t *>(U.host[p % NS]);
         const uint8_t *x = h;
         if (!direct) {
-            HIPCHK(hipMemcpyAsync(d_x.p + (p % NS) * xs, h, (size_t)n * q.F, hipMemcpyHostToDevice, s));
-            x = d_x.p + (p % NS) * xs;
+            uint8_t *d = d_x.p + (p % NS) * xd;
+            if (raw) {
+                const int rb = D.send(s, (int)(p % NS), h, q.src, n, 0, q.F, d, n);
+                if (rb != EVT_OK) return rb;
+            } else {
+                HIPCHK(hipMemcpyAsync(d, h, (size_t)n * q.F, hipMemcpyHostToDevice, s));
+            }
+            x = d;
         }
         const int rw = walk(m, s, q, x, n, h + xs, leaf_bytes); // the kernel writes what comes back over the bus itself
         if (rw != EVT_OK) return rw;

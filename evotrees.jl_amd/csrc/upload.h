@@ -45,6 +45,24 @@ struct BinPieces {
     BinPieces(int64_t N_, int F_, bool src_rows_contiguous, bool by_rows, int64_t rows_most, int64_t cells_most);
     void at(int64_t p, int64_t *r0, int64_t *n, int *f0, int *f1) const;
     void bin(const HbPlan &P, const HbSource &S, int64_t p, int t, uint8_t *out) const; // the bin of (r, f) to out[(f - f0) * n + r - r0]
+    void copy(const HbSource &S, int64_t p, int t, void *out) const; // its value there, or to out[(r - r0) * cols + f] when rowwise
+};
+
+// Pieces that go up as they lie and are binned by a kernel: for hosts whose cores are slower at it than the bus.
+bool bins_by_device(int dtype, int64_t cells);
+class DeviceBins {
+    uint8_t *edges = nullptr, *stage = nullptr;
+    size_t off_at = 0, slot = 0;
+    int max_edges = 0;
+
+  public: // declared before the pinned buffers: they wait for the stream
+    int init(hipStream_t s, const HbPlan &P, size_t slot_bytes, int slots);
+    // queues piece data of n rows and features [f0, f1) from h, by way of buffer k; its bins go to out + (f - f0) * ldo
+    int send(hipStream_t s, int k, const void *h, const HbSource &S, int64_t n, int f0, int f1, uint8_t *out, int64_t ldo);
+    ~DeviceBins() {
+        dev_give(edges);
+        dev_give(stage);
+    }
 };
 
 // The pieces 0 .. np - 1 through NS buffers: piece p is filled by its `tasks` calls of fill(p, t), on worker threads or this one; then send(p) queues

@@ -155,12 +155,13 @@ int evt_set_xbin(evt_handle h, const uint8_t *x_bin_colmajor);
 /* Device binarize: searchsortedfirst(edges[j], x[i,j]) for every cell (src/fit-utils.jl:66-72),
  * written straight into the cache's x_bin.  x is nobs x nfeats column-major Float64; edges are
  * concatenated per feature, edge_off has nfeats+1 entries.  A matrix in device memory is binned there,
- * one in host memory by the host's cores (evt_binarize). */
+ * one in host memory as evt_binarize does it. */
 int evt_binarize_f64(evt_handle h, const double *x_colmajor, const double *edges, const int32_t *edge_off);
 
 /* The same for a matrix in host memory as the program holds it: element (i, j) at x + i * row_stride + j * col_stride
  * elements of dtype (EVT_F32 or EVT_F64), one of the two strides being 1 (rows, or columns, one after the other); values are
- * compared as the Float64 they convert to.  Binned by the host's cores and sent as bytes. */
+ * compared as the Float64 they convert to.  Binned by the host's cores and sent as bytes, or, where these are few or without AVX-512, sent
+ * as it lies and binned on the device: the same bins. */
 int evt_binarize(evt_handle h, const void *x, int32_t dtype, int64_t row_stride, int64_t col_stride, const double *edges, const int32_t *edge_off);
 
 /* Host only, no device needed.  binarize for Tables input (src/fit-utils.jl:74-92): column j's bins go to x_bin_out + j * nobs;

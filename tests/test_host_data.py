@@ -79,6 +79,17 @@ def test_more_columns_than_edges_are_refused(evt):
         evt.binarize(np.zeros((50, 4)), [np.arange(3.0)] * 3)
 
 
+class OneCore:
+    """The calling thread on one core: there a large matrix goes up as it lies and is binned by the device."""
+
+    def __enter__(self):
+        self._was = os.sched_getaffinity(0)
+        os.sched_setaffinity(0, {min(self._was)})
+
+    def __exit__(self, *_):
+        os.sched_setaffinity(0, self._was)
+
+
 class Threads:
     """The most threads the process had at a look every half millisecond."""
 
@@ -254,3 +265,40 @@ def test_leaf_ids_of_more_pieces_than_buffers(evt):
         got = evt.predict_leaf_idx(m, x)
     assert np.array_equal(got, want)
     assert seen.most <= before + 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("order", ["C", "F", "wide C", "wide F"])
+@pytest.mark.parametrize("shape", [(70_001, 24), (1_000_003, 2), (400_003, 50), (17, 40_000), (300, 1030), (9_000_001, 2)])
+def test_a_matrix_binned_by_the_device(evt, dtype, order, shape):
+    """One piece, several, more than buffers; rows and columns contiguous, with gaps between them; edges that only isless tells apart."""
+    rng = np.random.default_rng(3)
+    N, F = shape
+    x = np.asarray(rng.random((N + 3, F + 5), np.float32), dtype, order=order[-1])
+    x = x[:N, :F] if "wide" in order else np.asarray(x[:N, :F], order=order)
+    edges = [np.sort(np.float32(rng.random(rng.choice([1, 7, 15])))).astype(np.float64) for _ in range(F)]
+    edges[0] = np.array([-0.0, 0.5, np.nan])
+    edges[1] = np.sort(rng.random(254))
+    for v in (np.nan, np.inf, -np.inf, 0.0, -0.0, 0.5):
+        for j in (0, F - 1):
+            x[rng.integers(N), j] = v
+    h = evt.Handle(N, F, 255, 1, 3, "mse")
+    with OneCore():
+        h.binarize_matrix(x, edges)
+    assert np.array_equal(h.get_xbin(), evt.binarize(x, edges))
+    h.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,F,K,loss,depths", [(70_001, 24, 1, "mse", [6] * 9), (400_003, 5, 3, "mlogloss", [5] * 6), (40_000, 100, 2, "gaussian_mle", [4] * 300)])
+def test_predictions_binned_by_the_device(evt, N, F, K, loss, depths):
+    from test_gpu_kept_model import _check, _model
+    rng = np.random.default_rng(N)
+    m = _model(evt, rng, F, 64, K, loss, depths)
+    x = rng.random((N, F), np.float32)
+    want, leaf = evt.predict(m, x), evt.predict_leaf_idx(m, x)
+    with OneCore():
+        for lay in (x, np.asfortranarray(x), x.astype(np.float64), np.repeat(x, 2, axis=1)[:, ::2]):
+            assert np.array_equal(evt.predict(m, lay), want) and np.array_equal(evt.predict_leaf_idx(m, lay), leaf)
+        _check(evt, m, x)  # the whole-model calls too
