@@ -61,6 +61,7 @@ struct Region {
     bool closed = false;
     std::atomic<bool> failed{false};
     std::exception_ptr error; // the first exception of a task; the caller's to throw
+    cpu_set_t cpus;           // the caller's: its workers run there too
 };
 struct Pool {
     const pid_t pid = getpid();
@@ -84,6 +85,8 @@ struct Pool {
         return false;
     }
     void loop() {
+        cpu_set_t cpus;
+        CPU_ZERO(&cpus);
         std::unique_lock<std::mutex> lk(m);
         for (;;) {
             Region *r;
@@ -91,6 +94,10 @@ struct Pool {
             r->wanted--;
             r->active++;
             lk.unlock();
+            if (!CPU_EQUAL(&cpus, &r->cpus)) {
+                cpus = r->cpus;
+                (void)sched_setaffinity(0, sizeof(cpus), &cpus); // of this thread
+            }
             bool more = true, leave = false;
             std::exception_ptr error;
             try {
@@ -147,6 +154,8 @@ struct HbWorkers::State {
     State(int n, std::function<bool()> &&f) : step(std::move(f)), pool(Pool::get()) {
         region.step = &step;
         region.wanted = n;
+        CPU_ZERO(&region.cpus);
+        (void)sched_getaffinity(0, sizeof(region.cpus), &region.cpus);
     }
 };
 HbWorkers::HbWorkers(int n, std::function<bool()> step) {

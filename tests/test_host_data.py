@@ -175,6 +175,43 @@ def test_an_exception_of_a_worker_is_the_callers(evt, tmp_path):
     assert (run.returncode, run.stdout) == (0, "ok\n"), run.stderr
 
 
+AFFINITY = r"""
+#include "host_bin.h"
+#include <cstdio>
+#include <sched.h>
+#include <unistd.h>
+int main() { // workers of a caller with few cores, then of one with all: each runs where its caller may
+    cpu_set_t all, few, got;
+    sched_getaffinity(0, sizeof(all), &all);
+    CPU_ZERO(&few);
+    for (int c = 0, n = 0; c < CPU_SETSIZE && n < 2; c++)
+        if (CPU_ISSET(c, &all)) CPU_SET(c, &few), n++;
+    for (const cpu_set_t *mine : {&few, &all, &few}) {
+        sched_setaffinity(0, sizeof(*mine), mine);
+        std::atomic<int> bad{0};
+        hb_parallel(64, 3, [&](int) {
+            usleep(300);
+            cpu_set_t here;
+            sched_getaffinity(0, sizeof(here), &here);
+            if (!CPU_EQUAL(&here, mine)) bad++;
+        });
+        if (bad) return 1;
+    }
+    puts("ok");
+}
+"""
+
+
+def test_workers_run_on_their_callers_cores(evt, tmp_path):
+    csrc = os.path.join(os.path.dirname(evt.__file__), "csrc")
+    (tmp_path / "main.cpp").write_text(AFFINITY)
+    exe = str(tmp_path / "main")
+    subprocess.run(["g++", "-x", "c++", "-O0", "-std=c++17", "-I", csrc, str(tmp_path / "main.cpp"), os.path.join(csrc, "host_bin.cpp"),
+                    os.path.join(csrc, "host_bin_avx512.cpp"), "-o", exe, "-pthread"], check=True)
+    run = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert (run.returncode, run.stdout) == (0, "ok\n"), run.stderr
+
+
 QUOTA = r"""
 #include "host_bin.cpp"
 int main(int, char **a) {
