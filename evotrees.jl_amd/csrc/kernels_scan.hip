@@ -399,6 +399,11 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
         // for the decision took 5 to 7 us and its gap: 100 features x 64 bins, two kernels -> one: 1 node 5.7 + 5.1 -> 7.4 us, 32 nodes
         // 6.6 + 10.4 -> 9.4, 256 nodes 23.1 + 11.5 -> 28.7, 512 nodes 41.6 + 6.5 -> 46.1; 28 features x 128 bins 6.0 + 5.6 -> 7.8, 26.6 + 7.5 -> 31.0.
         // (Counters side by side, 32 to a line: 500 features and 16 nodes 31 us, 14 with a line each.)
+        // Order: every word handed over is stored and loaded by agent-scope atomics, which go past the caches that are not shared, so that
+        // what a release adds to them is only the wait for the stores' completion, written out here, and what an acquire adds is only
+        // that the loads come behind the count, which the branch on it and the barrier for the compiler see to.  The language's own
+        // release also writes back the histograms that lie dirty in L2, and an acquire throws L2 away: a count with both 1318 us a tree, with
+        // the release and an acquire by the last block alone 1175, as it is 648 (100 features x 64 bins, 1M rows, depth 11).
         constexpr int CW = 3 + NAG; // words of a candidate: gain, position and bin, feature, totals
         unsigned long long *cand = reinterpret_cast<unsigned long long *>(reinterpret_cast<ScanBestQ *>(A.sbest) + (int64_t)nodeidx * gridDim.y);
         int last = 0;
