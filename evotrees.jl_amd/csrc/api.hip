@@ -7,11 +7,8 @@
 #include <string.h>
 
 #include <algorithm>
-#include <condition_variable>
 #include <memory>
-#include <mutex>
 #include <new>
-#include <thread>
 
 int launch_absmax_rows(evt_ctx *c, int k0, int k1);
 int launch_check_unit_weight(evt_ctx *c);
@@ -498,123 +495,6 @@ static int check_errflag(evt_ctx *c, const char *what) {
         evt_set_error("%s", what);
         return EVT_ERR_ARG;
     }
-    return EVT_OK;
-}
-
-// Large host buffers go up in pieces through three pinned buffers: a few worker threads copy piece k + 1 into its buffer while
-// the DMA engine moves piece k.  A copy straight from the caller's pageable memory is staged by the runtime
-// at about half the rate the bus gives pinned memory (31 against 57 GB/s on the box this was measured on), and one thread's
-// memcpy is no faster than that either.  The workers only copy memory, never call back into the caller's runtime, and are
-// joined before the call returns.
-struct CopyJob {
-    const char *src;
-    char *dst;
-    size_t n;
-};
-class CopyPool {
-    std::vector<std::thread> th;
-    std::mutex m;
-    std::condition_variable cv_go, cv_done;
-    const std::vector<CopyJob> *jobs = nullptr;
-    size_t gen = 0;
-    int pending = 0;
-    bool stop = false;
-    const int nt;
-    void run(int w) {
-        size_t seen = 0;
-        for (;;) {
-            std::unique_lock<std::mutex> lk(m);
-            cv_go.wait(lk, [&] { return stop || gen != seen; });
-            if (stop) return;
-            seen = gen;
-            const std::vector<CopyJob> *j = jobs;
-            lk.unlock();
-            for (const CopyJob &job : *j) { // worker w takes the w-th of nt slices of every job (cut at 64-byte multiples)
-                const size_t lo = (job.n * (size_t)w / nt) & ~(size_t)63;
-                const size_t hi = (w + 1 == nt) ? job.n : ((job.n * (size_t)(w + 1) / nt) & ~(size_t)63);
-                if (hi > lo) memcpy(job.dst + lo, job.src + lo, hi - lo);
-            }
-            lk.lock();
-            if (--pending == 0) cv_done.notify_one();
-        }
-    }
-
-  public:
-    explicit CopyPool(int n) : nt(n) {
-        for (int w = 0; w < n; w++) th.emplace_back([this, w] { run(w); });
-    }
-    ~CopyPool() {
-        {
-            std::lock_guard<std::mutex> lk(m);
-            stop = true;
-        }
-        cv_go.notify_all();
-        for (auto &t : th) t.join();
-    }
-    void copy(const std::vector<CopyJob> &j) { // returns when every job has been copied
-        std::unique_lock<std::mutex> lk(m);
-        jobs = &j;
-        pending = nt;
-        gen++;
-        cv_go.notify_all();
-        cv_done.wait(lk, [&] { return pending == 0; });
-    }
-};
-struct UploadSlots {
-    static const int NS = 3;
-    void *host[NS] = {nullptr, nullptr, nullptr};
-    double *dev[NS] = {nullptr, nullptr, nullptr};
-    hipEvent_t ev[NS] = {nullptr, nullptr, nullptr};
-    ~UploadSlots() {
-        for (int k = 0; k < NS; k++) {
-            if (ev[k]) (void)hipEventDestroy(ev[k]);
-            if (dev[k]) (void)hipFree(dev[k]);
-            if (host[k]) (void)hipHostFree(host[k]);
-        }
-    }
-    int init(size_t bytes, bool with_dev) {
-        for (int k = 0; k < NS; k++) {
-            HIPCHK(hipHostMalloc(&host[k], bytes, hipHostMallocDefault));
-            if (with_dev) HIPCHK(hipMalloc((void **)&dev[k], bytes));
-            HIPCHK(hipEventCreateWithFlags(&ev[k], hipEventDisableTiming));
-        }
-        return EVT_OK;
-    }
-};
-static const int64_t UPLOAD_PIECE = (int64_t)32 << 20; // bytes
-// worker threads for an upload of this size: none below a few pieces, else up to six
-static int upload_workers(int64_t total_bytes) {
-    if (total_bytes < 2 * UPLOAD_PIECE) return 0;
-    return (int)std::min(6, std::max(1, hb_cores() / 2));
-}
-// nbytes from the caller's memory to the device: large host buffers go through pinned buffers,
-// everything else is a plain copy.  The data has arrived when the call returns.
-static int upload_bytes(hipStream_t s, const void *src, void *dst, size_t nbytes) {
-    hipPointerAttribute_t attr;
-    const bool on_dev = (hipPointerGetAttributes(&attr, src) == hipSuccess) && attr.type == hipMemoryTypeDevice;
-    (void)hipGetLastError();
-    const int nworkers = on_dev ? 0 : upload_workers((int64_t)nbytes);
-    if (nworkers <= 1) {
-        HIPCHK(hipMemcpyAsync(dst, src, nbytes, hipMemcpyDefault, s));
-        HIPCHK(hipStreamSynchronize(s));
-        return EVT_OK;
-    }
-    UploadSlots U;
-    int r = U.init((size_t)UPLOAD_PIECE, false);
-    if (r != EVT_OK) return r;
-    CopyPool pool(nworkers);
-    std::vector<CopyJob> jobs(1);
-    int64_t piece = 0;
-    for (size_t o = 0; o < nbytes; o += (size_t)UPLOAD_PIECE, piece++) {
-        const size_t n = std::min((size_t)UPLOAD_PIECE, nbytes - o);
-        const int k = (int)(piece % UploadSlots::NS);
-        if (piece >= UploadSlots::NS) HIPCHK(hipEventSynchronize(U.ev[k]));
-        jobs[0] = {static_cast<const char *>(src) + o, static_cast<char *>(U.host[k]), n};
-        pool.copy(jobs);
-        HIPCHK(hipMemcpyAsync(static_cast<char *>(dst) + o, U.host[k], n, hipMemcpyHostToDevice, s));
-        HIPCHK(hipEventRecord(U.ev[k], s));
-    }
-    HIPCHK(hipStreamSynchronize(s));
     return EVT_OK;
 }
 

@@ -140,5 +140,7 @@ static int run_pieces(PinnedSlots &U, int NS, int64_t np, int tasks, int workers
     return EVT_OK;
 }
 
+// nbytes from the caller's memory, on the host or the device, to the device.  The data has arrived when the call returns.
+int upload_bytes(hipStream_t s, const void *src, void *dst, size_t nbytes);
 // Binned matrix -> device, column j to xcm + j * ldo.  The data has arrived when the call returns.
 int upload_bins(hipStream_t s, const HbPlan &P, const HbSource &S, int64_t N, uint8_t *xcm, int64_t ldo);

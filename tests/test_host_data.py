@@ -339,3 +339,14 @@ def test_predictions_binned_by_the_device(evt, N, F, K, loss, depths):
         for lay in (x, np.asfortranarray(x), x.astype(np.float64), np.repeat(x, 2, axis=1)[:, ::2]):
             assert np.array_equal(evt.predict(m, lay), want) and np.array_equal(evt.predict_leaf_idx(m, lay), leaf)
         _check(evt, m, x)  # the whole-model calls too
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [(64 << 20) - 1, 64 << 20, (64 << 20) + 1, (72 << 20) - 1, (72 << 20) + (1 << 19) + 1])
+def test_bins_of_more_than_a_buffer(evt, N):
+    """Around the size from which pinned pieces are taken, whole pieces, a piece and a task more, a byte more and less."""
+    x = np.random.default_rng(0).integers(1, 17, (1, N), dtype=np.uint8)
+    h = evt.Handle(N, 1, 16, 1, 1, "mse")
+    h.set_xbin(x)
+    assert np.array_equal(h.get_xbin(), x)
+    h.close()
