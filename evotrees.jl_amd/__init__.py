@@ -296,7 +296,7 @@ def _equal_columns(data, names):
     """The columns of these names, each a vector of the first one's length: the library reads them by row number, without a check."""
     cols = [_column(data, name) for name in names]
     for name, col in zip(names, cols):
-        if not _is_categorical(col) and col.ndim != 1:
+        if getattr(col, "ndim", 1) != 1:
             raise ValueError("feature %s is no vector" % name)
         if len(col) != len(cols[0]):
             raise ValueError("feature %s has %d rows, %s has %d" % (name, len(col), names[0], len(cols[0])))

@@ -220,11 +220,11 @@ def strided_matrix(x):
 def flat_edges(edges):
     """Edges of all features one after the other, and where each feature's start."""
     edges = [np.asarray(e, np.float64) for e in edges]
-    if any(e.ndim != 1 for e in edges):
+    flat = np.concatenate(edges) if edges else np.zeros(0)  # not of scalars, nor of vectors and matrices
+    if flat.ndim != 1:
         raise ValueError("the edges of a feature must be a vector")
     off = np.zeros(len(edges) + 1, np.int32)
-    off[1:] = np.cumsum([len(e) for e in edges])
-    flat = np.concatenate(edges) if len(edges) else np.zeros(0)
+    off[1:] = np.cumsum([e.size for e in edges])
     return np.ascontiguousarray(flat), off
 
 
@@ -234,7 +234,7 @@ def bin_columns(cols, nobs, edges):
     if len(edges) < n:  # as the library reads them: one entry per column
         raise IndexError("%d columns, but edges of %d" % (n, len(edges)))
     # the library takes a column without edges for one of codes; no value passes a NaN
-    flat, off = flat_edges([() if e is None else e if np.size(e) else [np.nan] for e in edges[:n]])
+    flat, off = flat_edges([() if e is None else e if (e.size if type(e) is np.ndarray else np.size(e)) else [np.nan] for e in edges[:n]])
     out = np.empty((n, nobs), np.uint8)
     if out.size == 0:
         return out

@@ -1499,8 +1499,6 @@ static void complete_trees(int ntrees, const int64_t *tree_off, const int64_t *f
     }
 }
 
-// Rows binned per pass of evt_predict_f64: bounds the Float64 staging buffer to chunk * nfeats * 8 bytes.
-
 static int predict_common(int64_t nobs, int32_t nfeats, const uint8_t *x_bin, const uint8_t *feattypes, int32_t loss, int32_t K, int32_t ntrees,
                           const int64_t *tree_off, const int64_t *feat, const uint8_t *cond_bin, const float *pred, const uint8_t *split,
                           int32_t apply_link, float *out, uint32_t *leaf_out, const double *x_f64 = nullptr, const double *edges = nullptr,

@@ -27,7 +27,7 @@
 // raises the copy of stripe blockIdx % EVT_ABSMAX_STRIPES: same-address atomics queue up one behind the other
 #define EVT_ABSMAX_STRIPES 32
 #define EVT_MC_MAX_NK 40 // >= 2 * EVT_MAX_K + 1: sizes of the per-row quantisation tables and of the generic kernels' arrays
-#define EVT_HIST_GROUP 4 // accumulator channels one histogram launch handles; more channels take several launches
+#define EVT_HIST_GROUP 4 // accumulator channels one histogram block handles; more channels are layers of the launch
 #define EVT_OBLIV_BLOCKS 256 // blocks of the search for an oblivious level's best cell
 #define EVT_METRIC_BLOCKS 1024 // partial sums of the evaluation metric
 #define EVT_MAX_DEPTH 16

@@ -621,7 +621,9 @@ int launch_walk_rows(hipStream_t s, const uint32_t *cnodes, int stride, const vo
                      int64_t leaf_ld) {
     // rows per block: as few as fill the chip (1024 blocks of four wavefronts, eight of which share a compute unit), and no more than
     // 64 KB of bins
-    // (leaf ids go out R to a line: from 4096 rows on whole 64-byte ones)
+    // (leaf ids go out R to a line: from 4096 rows on whole 64-byte ones).  Whole calls on bins beside set values of R, 100 and 200 trees of depth 6 and 8:
+    // values of one output within 10 % of the best from 1 to 131 000 rows; of seven outputs R = 16 is up to 1.34 times faster from 1000 rows on,
+    // and leaf ids between 64 rows and 16 000 take 1.2 to 4.7 times what R = 16 would
     int R = n <= 1024 ? 1 : (n <= (leaf_out ? 4096 : 8192) ? 4 : (n <= 32768 && !leaf_out ? 16 : 64));
     while (R > 1 && (size_t)R * F > 65536) R /= 4;
 #define EVT_WALK(KM_, LEAF_, LB_)                                                                                                                    \

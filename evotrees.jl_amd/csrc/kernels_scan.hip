@@ -347,7 +347,7 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
             }
         }
     }
-    if (A.oblivious) return; // decision is taken for the whole level by k_obliv_select
+    if (A.oblivious) return; // decision is taken for the whole level by k_obliv_max and k_obliv_apply
 
     if (lane == 0) {
         s_wg[wave] = wbest; s_wjp[wave] = wjp; s_wbin[wave] = wbin;

@@ -787,7 +787,8 @@ static int small_tree_buffers(evt_ctx *c, bool split) {
 // shared by S blocks.  A block walks its rows once per level (and once more for every `slots` nodes), so a level grows with
 // rows / S, the channels and - through the candidates every block reads and the searches its 16 wavefronts share - the nodes; slices
 // add a launch and the words they flush.  The other path spreads rows of any number over the chip and pays for its launches.  Estimates
-// in microseconds, fitted to rounds that each of them grew (4k to 250k rows, 10 and 60 features, depths 5 to 9, 1 to 14 channels).
+// in microseconds, fitted to rounds that each of them grew (2k to 250k rows, 8 to 100 features, depths 4 to 9, 1 to 15 channels): of 150 shapes
+// all but four take a form within 4 % of the best, the worst one 9 % off it.
 // Whole calls of one round (host included, ~50 us) at depth 6, microseconds for the other path, S = 1 and S > 1: mse, 8 features 125, 81, 95 at 2k rows,
 // 139, 137, 96 at 30k, 148, -, 108 at 250k; mse, 100 features 150, 137, 120 at 30k; 3 classes, 8 features 195, 154, 149 at 8k,
 // 210, 543, 159 at 60k, 237, -, 215 at 250k; 7 classes, 8 features 213, 188, 226 at 2k, 275, -, 303 at 120k, 320, -, 396 at 250k.

@@ -327,8 +327,8 @@ int evt_predict(int64_t nobs, int32_t nfeats, const uint8_t *x_bin_colmajor, con
                 const uint8_t *cond_bin, const float *pred, const uint8_t *split, int32_t apply_link,
                 float *out);
 /* The same from raw features: binarize(data; edges) (src/fit-utils.jl:66-72, searchsortedfirst per
- * column) on the device, in row chunks, followed by the traversal above — the whole of
- * _predict(m, data, ::Type{<:GPU}).  x is nobs x nfeats column-major Float64; edges / edge_off as in
+ * column; a matrix in host memory as evt_binarize bins it, one in device memory there) followed by the traversal
+ * above — the whole of _predict(m, data, ::Type{<:GPU}).  x is nobs x nfeats column-major Float64; edges / edge_off as in
  * evt_binarize_f64 (at most 254 edges per feature). */
 int evt_predict_f64(int64_t nobs, int32_t nfeats, const double *x_colmajor, const double *edges,
                     const int32_t *edge_off, const uint8_t *feattypes, int32_t loss, int32_t K, int32_t ntrees,
