@@ -7,7 +7,6 @@
 #include <unistd.h>
 
 #include <algorithm>
-#include <cmath>
 #include <condition_variable>
 #include <exception>
 #include <mutex>
@@ -355,16 +354,16 @@ static void select_ranks(T *v, int64_t n, const int64_t *ranks, int nr, double *
         hi = v[i] > hi ? v[i] : hi;
     }
     const double width = (double)hi - (double)lo;
-    int nb = 64;
-    while (nb < n / 2 && nb < 32768) nb <<= 1;
-    const double l = (double)lo, scale = (double)nb / width;
     // sorted where the slices have no width that Float64 holds: all values equal (0), an infinity among them (inf), or so close that
-    // nb / width overflows (denormals, also those that a skewed column leaves in one slice)
-    if (n <= 64 || depth >= 8 || !(width > 0 && width < 1e300 && std::isfinite(scale))) {
+    // nb / width would overflow (denormals, also those that a skewed column leaves in one slice)
+    if (n <= 64 || depth >= 8 || !(width > 1e-300 && width < 1e300)) {
         if (hi > lo) std::sort(v, v + n);
         for (int i = 0; i < nr; i++) out[i] = (double)v[ranks[i]];
         return;
     }
+    int nb = 64;
+    while (nb < n / 2 && nb < 32768) nb <<= 1;
+    const double l = (double)lo, scale = (double)nb / width;
     // (v - lo) * scale lies in [0, nb] up to rounding and is monotone in v, in rounded arithmetic too: a bucket's values all lie
     // between its neighbours'
     std::vector<uint32_t> first((size_t)nb + 1, 0);
