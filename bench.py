@@ -129,7 +129,7 @@ def record_slot_fill(F, B, na_max):
 
 
 def prepare(evt, cfg, opts=None):
-    """Synthetic data of the configuration, quantile edges, handle creation, upload + device binarize, target.
+    """Synthetic data of the configuration, quantile edges, handle creation, binarize + upload, target.
     Returns the handle and the seconds spent in each part (data generation apart: it is not part of a fit)."""
     N, F, B, D, loss = cfg["N"], cfg["F"], cfg["nbins"], cfg["depth"], cfg["loss"]
     K = 2 if loss == "gaussian_mle" else 1
@@ -452,8 +452,8 @@ def main():
         "config": {"workload": "%s: %s %dx%d nbins=%d max_depth=%d eta=%g rowsample=%g colsample=%g tree_type=%s" % (
             args.workload, loss, N, F, B, D, cfg["eta"], cfg["rowsample"], cfg["colsample"], cfg["tree_type"])},
         "roofline": roofline, "kernels_breakdown_%d_extra_rounds" % extra: kernels, "setup_s": round(t_setup, 2),
-        # what a whole fit of this workload costs: quantile edges on the host, upload of the Float64 matrix, device
-        # binarize, target upload (init, once), then the 200 rounds; the synthetic data's generation is not part of a fit
+        # what a whole fit of this workload costs: quantile edges on the host, the Float64 matrix binned and uploaded,
+        # target upload (init, once), then the 200 rounds; the synthetic data's generation is not part of a fit
         "init_s": t_init, "fit_total_s": round(t_setup + value, 2),
     }
     # rows built per level of the last tree (unit weights: Tree.w holds row counts): the smaller child of every split
@@ -528,8 +528,8 @@ def main():
             out["predict_model"] = {"error": str(e)}
 
     # The reference's whole inference call m(x) from a raw Float64 matrix in host memory (binarize + 200 trees + link, its
-    # published "infer" figure; src/predict.jl:118-136): evt_predict_f64, everything included - the 8 GB upload through pinned
-    # buffers, device binarize, the traversal, the predictions' way back.  The matrix is generated again (it was dropped after
+    # published "infer" figure; src/predict.jl:118-136): evt_predict_f64, everything included - binning the 8 GB, the
+    # upload, the traversal, the predictions' way back.  The matrix is generated again (it was dropped after
     # the set-up to free host memory).
     if args.workload == "cfg3" and not args.rows and not args.depth and args.side_steps > 0:
         try:

@@ -3,8 +3,8 @@
 //
 // A feature's edges sit in vector registers as a search heap (node h at lane h & 15 of register h >> 4): a step of the search is
 // a register permute that fetches every lane's own node, a compare, and h = 2 h + passed.  63 edges take six steps, 22
-// instructions for 16 values: 0.40 ns per Float64 value on one core of the host this was measured on, and with 16 cores the memory's own
-// rate (287 GB/s of Float64 read and binned; the same matrix moved to the device as it lies: 50 GB/s).
+// instructions for 16 values: 0.59 ns per Float64 value read from memory on one core of the host this was measured on (a plain search: 21), and
+// 170 to 180 GB/s of Float64 read and binned on 16 (the same matrix moved to the device as it lies: 43 GB/s).
 #include "host_bin.h"
 
 #if defined(__AVX512F__)

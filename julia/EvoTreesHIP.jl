@@ -112,7 +112,7 @@ function create_handle(nobs, nfeats, nbins, K, max_depth, L, tree_type)
     return h[]
 end
 
-# x_bin for a handle: a Float64 matrix is binned on the device (binarize, src/fit-utils.jl:66-72); anything else
+# x_bin for a handle: a Float64 matrix is binned by the library (binarize, src/fit-utils.jl:66-72); anything else
 # (Tables input with Bool / categorical columns, other element types) goes through the reference's own host
 # `binarize` (src/fit-utils.jl:74-92) and is uploaded as UInt8.
 function upload_features!(h::Ptr{Cvoid}, data, feature_names, edges)
