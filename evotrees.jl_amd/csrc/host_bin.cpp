@@ -178,6 +178,11 @@ HbWorkers::~HbWorkers() {
 }
 
 void hb_parallel(int ntasks, int nworkers, const std::function<void(int)> &fn) {
+    const int n = std::min(nworkers, ntasks - 1);
+    if (n <= 0) {
+        for (int t = 0; t < ntasks; t++) fn(t);
+        return;
+    }
     std::atomic<int> next{0};
     auto step = [&]() -> bool {
         const int t = next.fetch_add(1, std::memory_order_relaxed);
@@ -185,7 +190,7 @@ void hb_parallel(int ntasks, int nworkers, const std::function<void(int)> &fn) {
         fn(t);
         return true;
     };
-    HbWorkers ws(std::min(nworkers, ntasks - 1), step);
+    HbWorkers ws(n, step);
     while (!ws.failed() && step()) {
     }
     ws.join();
