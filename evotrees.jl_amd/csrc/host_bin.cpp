@@ -179,7 +179,7 @@ HbWorkers::~HbWorkers() {
 
 void hb_parallel(int ntasks, int nworkers, const std::function<void(int)> &fn) {
     const int n = std::min(nworkers, ntasks - 1);
-    if (n <= 0) {
+    if (n <= 0) { // the leaf ids of one row, 62 trees: 0.8 us of 23 less than by way of a region
         for (int t = 0; t < ntasks; t++) fn(t);
         return;
     }
