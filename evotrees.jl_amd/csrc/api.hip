@@ -179,7 +179,7 @@ extern "C" int evt_destroy(evt_handle c) {
     if (!c) return EVT_OK;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    void *ptrs[] = {c->xcm, c->xrm, c->y, c->pred, c->grad, c->gq, c->is_a, c->is_b, c->nidx, c->mask, c->flagw, c->chunk_nleft, c->chunk_lpre,
+    void *ptrs[] = {c->xcm, c->xrm, c->y, c->pred, c->grad, c->gq, c->is_a, c->is_b, c->nidx, c->mask, c->flagw, c->chunk_nleft, c->chunk_lpre, c->cursor,
                     c->hist, c->seg_start, c->seg_len, c->status, c->node_sum, c->tree_blob, c->tree.packed, c->js, c->jsmap, c->feattypes, c->mono, c->absmax, c->qexp_buf[0], c->qexp_buf[1], c->qbits,
                     c->qscale_buf[0], c->qscale_buf[1], c->planes, c->metric_partial, c->errflag, c->ogains, c->sbest, c->scan_count, c->is_id, c->pt_nodes, c->pt_pred, c->mask_next,
                     c->small_nid[0], c->small_nid[1], c->small_head[0], c->small_head[1], c->small_left[0], c->small_left[1], c->small_acc,
@@ -266,7 +266,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->have_xbin = c->have_target = c->have_grads = false;
     c->planes = nullptr; c->plane_words = 0; c->planes_ready = false; c->use_planes = 1;
     c->xcm = nullptr; c->xrm = nullptr; c->y = nullptr; c->pred = nullptr; c->grad = nullptr; c->gq = nullptr;
-    c->is_a = c->is_b = nullptr; c->nidx = nullptr; c->mask = nullptr; c->flagw = nullptr; c->chunk_nleft = nullptr; c->chunk_lpre = nullptr;
+    c->is_a = c->is_b = nullptr; c->nidx = nullptr; c->mask = nullptr; c->flagw = nullptr; c->chunk_nleft = nullptr; c->chunk_lpre = nullptr; c->cursor = nullptr;
     c->hist = nullptr; c->seg_start = c->seg_len = nullptr; c->status = nullptr; c->node_sum = nullptr;
     memset(&c->tree, 0, sizeof(c->tree));
     c->tree_blob = nullptr;
@@ -290,6 +290,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->hist_tile = 0;
     c->scan_fused = 1;
     c->hist_in_scatter = 1;
+    c->part_one_pass = 1;
     c->small_tree = 1;
     c->small_acc = nullptr;
     for (int k = 0; k < 2; k++) {
@@ -352,6 +353,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     ALLOC(c->flagw, (size_t)c->max_chunks * EVT_CHUNK_WORDS);
     ALLOC(c->chunk_nleft, c->max_chunks + 1);
     ALLOC(c->chunk_lpre, c->max_chunks + 1);
+    ALLOC(c->cursor, EVT_CURSOR_WORDS(c->nnodes));
     ALLOC(c->hist, (size_t)c->nnodes * c->F * NAgmax * c->B);
     ALLOC(c->seg_start, c->nnodes + 2);
     ALLOC(c->seg_len, c->nnodes + 2);
@@ -859,6 +861,7 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
     c->write_nidx = rec_nidx || defer;
 
     const int small = staged ? 0 : small_tree_form(c, n_js, all_rows);
+    c->step.hist_fused = !staged && scatter_can_build_hist(c, n_js); // the set-up below cuts the root's chunks by it
     int r = small ? EVT_OK : ensure_planes(c);
     if (r != EVT_OK) return r;
     if (EVT_IS_QUANTILE(c->loss)) {
@@ -895,7 +898,6 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
     c->step.small = small;
     c->step.small_draw = draw;
     c->step.fuse_pred = fuse_pred;
-    c->step.hist_fused = !staged && scatter_can_build_hist(c, c->n_js_last);
     c->step.blob_sent = false;
     c->step.p = *p;
     // the root's list is the identity (kept, never written) or what the mask compaction left in is_a; the levels below
@@ -1727,6 +1729,8 @@ extern "C" int evt_set_option(evt_handle c, const char *name, int64_t value) {
         c->scan_fused = value != 0;
     } else if (strcmp(name, "hist_in_scatter") == 0) {
         c->hist_in_scatter = value != 0;
+    } else if (strcmp(name, "part_one_pass") == 0) {
+        c->part_one_pass = value != 0;
     } else if (strcmp(name, "defer_pred") == 0) {
         c->defer_pred = value != 0;
     } else if (strcmp(name, "hist_threads") == 0) {

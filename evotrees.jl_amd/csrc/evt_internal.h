@@ -18,7 +18,8 @@
 #define ST_SPLIT 3    // scanned, split found
 #define ST_LEAF 4     // scanned (or last level), leaf
 
-#define EVT_CHUNK 2048        // rows per partition chunk (8 per thread of a 256-thread block)
+#define EVT_CHUNK 2048        // rows per partition chunk (8 per thread of a 256-thread block); part_chunk_rows() gives the levels of the one-pass form up to
+#define EVT_CHUNK_MAX 8192    // this many
 #define EVT_CHUNK_WORDS 32    // 64-bit ballot words per chunk
 #define EVT_MAX_NK 5  // gradient rows of the one- and two-output losses (register arrays of the specialised kernels)
 #define EVT_MAX_NA 5
@@ -44,6 +45,11 @@
 #define LH_N_BUILD 2
 #define LH_TOTAL_BUILD 3 // build rows of the level + hist_seg_cost per build node
 #define LH_SIZE 8
+
+// one-pass partition: a node's cursor has a 128-byte line to itself (additions to one line follow each other); the nodes of very deep levels, of few
+// chunks each, share lines
+#define EVT_CURSOR_SLOT(n) ((n) < 1024 ? (size_t)(n) * 16 : (size_t)16384 - 1024 + (n))
+#define EVT_CURSOR_WORDS(nnodes) ((size_t)16384 + (nnodes) + 2)
 
 // split search: a node's block counter has a 128-byte line to itself (additions to one line follow each other, ~15 ns each)
 #define EVT_SCAN_COUNT_STEP 32
@@ -126,6 +132,8 @@ struct evt_ctx {
     int32_t *chunk_nleft;
     int64_t *chunk_lpre;
     int64_t max_chunks;
+    unsigned long long *cursor; // one-pass partition: rows a split node's chunks have placed, left | right << 32 (part_cursor_slot)
+    int part_one_pass; // option: the partition of a level runs in one kernel where the split search knows the children's sizes
     long long *hist; // [node][jp][ag][bin]
     int64_t *seg_start, *seg_len;
     int32_t *status;
@@ -321,7 +329,7 @@ __device__ __forceinline__ unsigned long long evt_load_gq(const unsigned long lo
 // stores); `w` of `nw` wavefronts share the level's nodes.
 __device__ __forceinline__ void evt_fill_chunk_descriptors(const int64_t *__restrict__ hdr, const int32_t *__restrict__ act_node,
                                                            const int64_t *__restrict__ cprefix, const int64_t *__restrict__ seg_start,
-                                                           const int64_t *__restrict__ seg_len, uint4 *cdesc, int w, int nw) {
+                                                           const int64_t *__restrict__ seg_len, uint4 *cdesc, int chunk, int w, int nw) {
     const int lane = threadIdx.x & 63;
     const int n_act = (int)hdr[LH_N_ACT];
     for (int i = w; i < n_act; i += nw) {
@@ -329,7 +337,7 @@ __device__ __forceinline__ void evt_fill_chunk_descriptors(const int64_t *__rest
         const int64_t c0 = cprefix[i], c1 = cprefix[i + 1];
         const int64_t seg = seg_start[n], len = seg_len[n];
         for (int64_t c = c0 + lane; c < c1; c += 64)
-            cdesc[c] = make_uint4((uint32_t)n, (uint32_t)(seg + (c - c0) * EVT_CHUNK), (uint32_t)(seg + len), (uint32_t)c0);
+            cdesc[c] = make_uint4((uint32_t)n, (uint32_t)(seg + (c - c0) * chunk), (uint32_t)(seg + len), (uint32_t)c0);
     }
 }
 
@@ -378,6 +386,7 @@ int launch_hist_build(evt_ctx *c, int level, const uint32_t *is_cur);
 int launch_scan(evt_ctx *c, int level, const evt_params *p, bool leaf_level);
 bool scan_folds_leaves(const evt_ctx *c);
 int launch_obliv_select(evt_ctx *c, int level, const evt_params *p);
+int part_chunk_rows(const evt_ctx *c, int level);
 int launch_part_count(evt_ctx *c, int level, const uint32_t *is_cur);
 int launch_part_scatter(evt_ctx *c, int level, const uint32_t *is_cur, uint32_t *is_next, bool fuse_pred);
 bool scatter_can_build_hist(const evt_ctx *c, int nfs);

@@ -50,6 +50,7 @@ struct HistArgs {
     const int64_t *seg_start;
     const int64_t *seg_len;
     uint4 *cdesc;
+    int chunk; // rows of a chunk of this level
 };
 
 // First node of a block's span: the largest i with bprefix[i] <= start.  bprefix ascends from 0, so that is the number
@@ -79,7 +80,7 @@ __device__ __forceinline__ int first_node_of_span(const int64_t *__restrict__ bp
 __device__ __forceinline__ void fill_chunk_descriptors(const HistArgs &A) {
     if (blockIdx.y != 0 || blockIdx.z != 0) return;
     const int wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
-    evt_fill_chunk_descriptors(A.hdr, A.act_node, A.cprefix, A.seg_start, A.seg_len, A.cdesc, (int)blockIdx.x * nwaves + wave,
+    evt_fill_chunk_descriptors(A.hdr, A.act_node, A.cprefix, A.seg_start, A.seg_len, A.cdesc, A.chunk, (int)blockIdx.x * nwaves + wave,
                                (int)gridDim.x * nwaves);
 }
 
@@ -733,6 +734,7 @@ int launch_hist_build(evt_ctx *c, int level, const uint32_t *is_cur) {
     A.seg_start = c->seg_start;
     A.seg_len = c->seg_len;
     A.cdesc = L.cdesc;
+    A.chunk = part_chunk_rows(c, level);
     A.jsmap = c->jsmap;
     A.hist = c->hist;
     A.stats = c->stats;

@@ -3,18 +3,18 @@
 // split_set! (src/fit-utils.jl:93-312) is a stable partition of each split node's row-id segment;
 // update_nodes_idx_kernel! (ext/EvoTreesKernelAbstractionsExt/fit-utils.jl:9-31) is the same
 // decision written per row.  Here every node owns a contiguous segment [seg_start, seg_start+seg_len)
-// of the row-id list; a split rewrites the segment in place order (lefts first, both sides keeping
-// ascending row ids) into the other list buffer, so children are again contiguous segments.
-// Segments are cut into chunks of EVT_CHUNK rows that never cross a node boundary:
+// of the row-id list; a split rewrites the segment (lefts first) into the other list buffer, so children are again
+// contiguous segments.  Segments are cut into chunks that never cross a node boundary.  Two forms:
+//  one pass (k_part_move, unit weights): the split search left the children's row counts in the count channel of their
+//  totals, so a block decides its chunk, claims places in both children with one atomic addition and moves the rows;
+//  two passes (weights, whose totals hold no counts, and histograms built on the way):
 //   count   : one block per chunk evaluates x_bin[row, feat] <= cond_bin, keeps the ballots,
 //             counts lefts;
-//   next    : one block scans the chunk counts, sets the children's segments, picks which child
-//             is built (fewer rows; tie -> left, src/fit.jl:123-129) and writes the next level's
-//             tables (active nodes, chunk prefix, build list); it is the last block of the scatter
-//             kernel, except that inputs with thousands of chunks scan the counts in a kernel of
-//             its own before the scatter;
-//   scatter : one block per chunk moves row ids to their stable destination; chunks of nodes that
-//             became leaves record the node id per row (and add the leaf value to the prediction).
+//   scatter : one block per chunk moves row ids to their stable destination (ascending ids on both sides).
+// In both, chunks of nodes that became leaves record the node id per row (and add the leaf value to the prediction), and one
+// block sets the children's segments, picks which child is built (fewer rows; tie -> left, src/fit.jl:123-129) and writes
+// the next level's tables (active nodes, chunk prefix, build list).  It rides in the kernel that moves the rows; two passes
+// over thousands of chunks scan the counts in a kernel of its own before the scatter.
 // No host round trip is needed between levels.
 #include "evt_internal.h"
 #include <algorithm>
@@ -72,6 +72,9 @@ struct PartArgs {
     uint4 *copy_dst;
     int64_t copy_n;
     int copy_blocks;
+    // one-pass form: rows the node's chunks have placed so far, and the nodes' totals, whose last channel counts rows
+    unsigned long long *cursor;
+    const long long *node_sum;
 };
 
 // The word of the decision source that holds row `rid`: its bin byte, or - for a numeric split with bit planes - the
@@ -188,6 +191,11 @@ struct NextArgs {
     int64_t *n_bprefix;
     int64_t *n_stats; // rows the next level builds (the level's slot of the per-tree counts; the histogram kernel writes the same figure when it runs)
     int64_t seg_cost; // cost units added per build node in the histogram kernel's span space
+    int n_chunk;      // rows of a chunk of the next level
+    // one-pass form: a child's rows are its count channel, and its cursor starts from zero
+    const long long *node_sum;
+    int NAg;
+    unsigned long long *cursor;
 };
 
 // Two exclusive prefixes in one pass (same shape as block_excl_scan); s_tmp holds 34 values.
@@ -277,7 +285,7 @@ __device__ void level_tables_block(const NextArgs &A, long long *s_tmp /* [34] *
         const int64_t cp0 = A.cprefix[i], cp1 = A.cprefix[i + 1];
         const int st = A.status[n];
         const int64_t len = A.seg_len[n], start = A.seg_start[n];
-        const int64_t nl = A.chunk_lpre[cp1] - A.chunk_lpre[cp0];
+        const int64_t nl = A.node_sum ? A.node_sum[(int64_t)(2 * n) * A.NAg + A.NAg - 1] : A.chunk_lpre[cp1] - A.chunk_lpre[cp0];
         if (st != ST_SPLIT) continue;
         const int64_t nr = len - nl;
         A.seg_start[2 * n] = start;
@@ -287,8 +295,12 @@ __device__ void level_tables_block(const NextArgs &A, long long *s_tmp /* [34] *
         const bool build_left = nr >= nl; // the smaller child is built, tie -> left (src/fit.jl:123-129)
         A.status[2 * n] = build_left ? ST_BUILD : ST_SUBTRACT;
         A.status[2 * n + 1] = build_left ? ST_SUBTRACT : ST_BUILD;
+        if (A.cursor) {
+            A.cursor[EVT_CURSOR_SLOT(2 * n)] = 0ull;
+            A.cursor[EVT_CURSOR_SLOT(2 * n + 1)] = 0ull;
+        }
         s_pos += 1;
-        s_chunks += (nl + EVT_CHUNK - 1) / EVT_CHUNK + (nr + EVT_CHUNK - 1) / EVT_CHUNK;
+        s_chunks += (nl + A.n_chunk - 1) / A.n_chunk + (nr + A.n_chunk - 1) / A.n_chunk;
         s_brows += (build_left ? nl : nr) + A.seg_cost;
     }
     // children count (low 24 bits) and chunk count share one scan; the build rows take the other
@@ -305,12 +317,12 @@ __device__ void level_tables_block(const NextArgs &A, long long *s_tmp /* [34] *
         A.n_act_node[2 * p_pos] = 2 * n;
         A.n_act_node[2 * p_pos + 1] = 2 * n + 1;
         A.n_cprefix[2 * p_pos] = p_chunks;
-        A.n_cprefix[2 * p_pos + 1] = p_chunks + (nl + EVT_CHUNK - 1) / EVT_CHUNK;
+        A.n_cprefix[2 * p_pos + 1] = p_chunks + (nl + A.n_chunk - 1) / A.n_chunk;
         A.n_bnode[p_pos] = build_left ? 2 * n : 2 * n + 1;
         A.n_bstart[p_pos] = build_left ? start : start + nl;
         A.n_bprefix[p_pos] = p_brows;
         p_pos += 1;
-        p_chunks += (nl + EVT_CHUNK - 1) / EVT_CHUNK + (nr + EVT_CHUNK - 1) / EVT_CHUNK;
+        p_chunks += (nl + A.n_chunk - 1) / A.n_chunk + (nr + A.n_chunk - 1) / A.n_chunk;
         p_brows += (build_left ? nl : nr) + A.seg_cost;
     }
     if (tid == 0) {
@@ -529,6 +541,92 @@ __global__ __launch_bounds__(256) void k_part_scatter(PartArgs A, NextArgs NX) {
     }
 }
 
+// The partition of a level in one pass: a block decides its chunk's rows, claims as many places of either child with one addition to the
+// node's cursor, and writes the row ids there.  A chunk's rows keep their order; the chunks of a node follow each other in the order of
+// their claims, which nothing depends on: sums are integers, leaves are recorded by row id.  A wavefront owns NI * 64 neighbouring
+// positions, so that one total per wavefront is all that is exchanged.
+// Bound by its chain of trips to memory (descriptor, row ids and node, decision words, claim, stores) below a million rows, by the lists
+// and, deeper, the decision words' lines above.  us a level, count + scan of the counts + scatter -> this: 800k rows x 28 features, depth 8
+// 5.2 + 6.5 -> 7.4; 500k of 100 4.7 + 5.9 -> 7.5; 10M x 100, depth 11, root 17 + 5 + 19 -> 32, level 5 18 + 5 + 18 -> 35, level 9 33 + 5 + 19 -> 46.
+template <bool NT, int T, int NI>
+__global__ __launch_bounds__(T) void k_part_move(PartArgs A, NextArgs NX) {
+    constexpr int W = T / 64, CHUNK = NI * T;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ long long s_tmp[34];
+    __shared__ int s_cnt[W];
+    __shared__ unsigned long long s_claim;
+    const int64_t G = (int64_t)gridDim.x - 1;
+    if (blockIdx.x == 0) { // the next level's tables, beside the blocks that move the rows
+        level_tables_block(NX, s_tmp);
+        return;
+    }
+    uint4 cd = A.cdesc[blockIdx.x - 1];
+    const int64_t n_chunks = A.hdr[LH_N_CHUNKS];
+    for (int64_t c = blockIdx.x - 1; c < n_chunks; c += G, cd = A.cdesc[c < n_chunks ? c : 0]) {
+        const int n = (int)cd.x;
+        const uint32_t p0 = cd.y, pend = cd.z, seg = p0 - (uint32_t)(c - cd.w) * CHUNK; // positions are 32-bit numbers, as the row ids
+        const uint32_t left_of = pend - p0, wofs = wave * (NI * 64) + lane;               // rows from the chunk's first on; this lane's first
+        const uint32_t *isp = A.is_cur + p0;
+        uint32_t rid[NI], xbv[NI];
+#pragma unroll
+        for (int it = 0; it < NI; it++) rid[it] = isp[wofs + it * 64 < left_of ? wofs + it * 64 : left_of - 1];
+        const int st = A.status[n];
+        uint32_t nd = A.t_packed[n - 1]; // requested with the state, not behind the branch on it
+        uint32_t nl = (uint32_t)A.node_sum[(int64_t)(2 * n) * A.NAg + A.NAg - 1];
+        asm volatile("" : "+v"(nd), "+v"(nl));
+        if (st == ST_SPLIT) {
+            const int f = (int)(nd & 0xFFFFu) - 1;
+            const uint32_t cb = (nd >> 16) & 0xFFu;
+            const bool numeric = (nd & EVT_NODE_NUMERIC) != 0;
+            const uint8_t *col = A.xcm + (size_t)f * A.N;
+            const uint32_t *plane = (A.planes && numeric && cb >= 1u && cb < (uint32_t)A.B) ? A.planes + ((size_t)f * (A.B - 1) + (cb - 1)) * A.plane_words : nullptr;
+            if (plane) {
+#pragma unroll
+                for (int it = 0; it < NI; it++) xbv[it] = load_decision<NT>(nullptr, plane, rid[it]);
+            } else {
+#pragma unroll
+                for (int it = 0; it < NI; it++) xbv[it] = load_decision<NT>(col, nullptr, rid[it]);
+            }
+            unsigned long long bal[NI];
+            int cnt = 0;
+#pragma unroll
+            for (int it = 0; it < NI; it++) {
+                bal[it] = __ballot(wofs + it * 64 < left_of && decide_left(xbv[it], plane != nullptr, rid[it], numeric, cb));
+                cnt += __popcll(bal[it]);
+            }
+            if (lane == 0) s_cnt[wave] = cnt;
+            __syncthreads();
+            int lefts = 0, before = 0; // of the chunk, of the wavefronts before this one
+#pragma unroll
+            for (int w = 0; w < W; w++) {
+                const int v = s_cnt[w];
+                lefts += v;
+                before += w < wave ? v : 0;
+            }
+            const int rows = (int)(left_of < (uint32_t)CHUNK ? left_of : (uint32_t)CHUNK);
+            if (tid == 0) s_claim = atomicAdd(A.cursor + EVT_CURSOR_SLOT(n), (unsigned long long)lefts | ((unsigned long long)(rows - lefts) << 32));
+            __syncthreads();
+            const unsigned long long claim = s_claim;
+            uint32_t dL = seg + (uint32_t)claim + before, dR = seg + nl + (uint32_t)(claim >> 32) + (wave * (NI * 64) - before);
+#pragma unroll
+            for (int it = 0; it < NI; it++) {
+                const int lrank = __popcll(bal[it] & ((1ull << lane) - 1ull));
+                const bool left = (bal[it] >> lane) & 1ull;
+                if (wofs + it * 64 < left_of) A.is_next[left ? dL + lrank : dR + (lane - lrank)] = rid[it];
+                const int k = __popcll(bal[it]);
+                dL += k;
+                dR += 64 - k;
+            }
+        } else if (st == ST_LEAF && (A.write_nidx || A.fuse_pred)) { // rows of a node that stops here, as in k_part_scatter
+            for (uint32_t k = tid; k < (uint32_t)CHUNK && k < left_of; k += T) {
+                const uint32_t row = isp[k];
+                if (A.write_nidx) A.nidx[row] = (uint32_t)n;
+                if (A.fuse_pred) evt_add_leaf(A.pred + (size_t)A.K * row, A.t_pred + (size_t)A.K * (n - 1), A.K, A.loss);
+            }
+        }
+    }
+}
+
 // Last pass of a tree: rows of the deepest split level go straight to their leaf.  For a node that split,
 // the child is decided from x_bin[row, feat] exactly as the partition would (left iff <= cond_bin, or ==
 // for a categorical feature) but the row list is not rewritten: nothing reads it afterwards.  Each row
@@ -628,6 +726,8 @@ struct BeginArgs {
     int64_t seg_cost;
     int64_t root_words;
     int nnodes, K, D;
+    int chunk; // rows of a chunk of the root
+    unsigned long long *cursor;
     // the tree's column sample and its inverse map, from the pinned staging buffer to the device copies (0 words: unchanged)
     const uint32_t *js_src, *map_src;
     uint32_t *js_dst, *map_dst;
@@ -661,12 +761,13 @@ __device__ void tree_begin_block(BeginArgs A) {
         A.seg_start[1] = 0;
         A.seg_len[1] = A.n_is;
         A.hdr[LH_N_ACT] = 1;
-        A.hdr[LH_N_CHUNKS] = (A.n_is + EVT_CHUNK - 1) / EVT_CHUNK;
+        A.hdr[LH_N_CHUNKS] = (A.n_is + A.chunk - 1) / A.chunk;
         A.hdr[LH_N_BUILD] = 1;
         A.hdr[LH_TOTAL_BUILD] = A.n_is + A.seg_cost;
         A.act_node[0] = 1;
         A.cprefix[0] = 0;
-        A.cprefix[1] = (A.n_is + EVT_CHUNK - 1) / EVT_CHUNK;
+        A.cprefix[1] = (A.n_is + A.chunk - 1) / A.chunk;
+        A.cursor[EVT_CURSOR_SLOT(1)] = 0ull;
         A.bnode[0] = 1;
         A.bstart[0] = 0;
         A.bprefix[0] = 0;
@@ -834,6 +935,8 @@ static void fill_begin_args(evt_ctx *c, bool all_rows, BeginArgs &A) {
     A.nnodes = c->nnodes;
     A.K = c->K;
     A.D = c->D;
+    A.chunk = part_chunk_rows(c, 1);
+    A.cursor = c->cursor;
     A.js_words = A.map_words = 0;
     A.js_src = A.map_src = nullptr;
     A.js_dst = A.map_dst = nullptr;
@@ -914,14 +1017,33 @@ static void fill_part_args(evt_ctx *c, int level, const uint32_t *is_cur, uint32
     A.jsmap = nullptr;
     A.hist = nullptr;
     A.node_stride = 0;
-    A.F = A.nfs = A.NAg = 0;
+    A.F = A.nfs = 0;
+    A.NAg = c->NAg;
     A.copy_src = nullptr;
     A.copy_dst = nullptr;
     A.copy_n = 0;
     A.copy_blocks = 0;
+    A.cursor = c->cursor;
+    A.node_sum = c->node_sum;
+}
+
+// One pass where the children's sizes are in the totals (unit weights) and no histogram is built on the way.
+static bool part_in_one_pass(const evt_ctx *c) { return c->part_one_pass && c->unit_w && !c->step.hist_fused; }
+
+// Rows of a chunk of the level.  A node's chunks queue at its cursor, ~20 ns each: where a node has more than 128 of them they grow (us a level of
+// 1M rows, 2048 | 4096 | 8192 rows a chunk: root 11.7 | 8.9 | 9.0, two nodes 9.0 | 7.6 | 8.4, eight 6.8 | 6.8 | 8.3; 10M: 67 | 39 | 28, 62 | 36 | 28,
+// 34 | 28 | 23).  They grow too where the level is more blocks than the chip holds at once and nodes are many chunks (10M rows, 64 nodes 44 | - | 40).
+int part_chunk_rows(const evt_ctx *c, int level) {
+    int rows = EVT_CHUNK;
+    if (!part_in_one_pass(c) || level >= c->D - 1) return rows;
+    const int64_t per_node = (c->last_all_rows ? c->N : c->N * (c->last_cond + 1) / 256) >> (level - 1);
+    const int64_t all = per_node << (level - 1);
+    while (rows < EVT_CHUNK_MAX && (per_node > (int64_t)rows * 128 || (all > (int64_t)rows * 2048 && per_node >= (int64_t)rows * 16))) rows *= 2;
+    return rows;
 }
 
 int launch_part_count(evt_ctx *c, int level, const uint32_t *is_cur) {
+    if (part_in_one_pass(c)) return EVT_OK;
     PartArgs A;
     fill_part_args(c, level, is_cur, nullptr, false, A);
     if (A.stream_hint) hipLaunchKernelGGL(k_part_count<true>, dim3(grid_for_chunks(c->max_chunks)), dim3(256), 0, c->stream, A);
@@ -949,6 +1071,10 @@ static void fill_next_args(evt_ctx *c, int level, NextArgs &A) {
     A.n_bprefix = Nx.bprefix;
     A.n_stats = (level + 1 <= c->D) ? c->stats + level + 1 : nullptr;
     A.seg_cost = c->hist_seg_cost;
+    A.n_chunk = part_chunk_rows(c, level + 1);
+    A.node_sum = nullptr;
+    A.NAg = c->NAg;
+    A.cursor = nullptr;
 }
 
 // Moves the rows of the level's split nodes to their children and, in one extra block, writes the next level's tables.
@@ -957,6 +1083,21 @@ int launch_part_scatter(evt_ctx *c, int level, const uint32_t *is_cur, uint32_t 
     fill_part_args(c, level, is_cur, is_next, fuse_pred, A);
     NextArgs NX;
     fill_next_args(c, level, NX);
+    if (part_in_one_pass(c)) {
+        NX.node_sum = c->node_sum;
+        NX.cursor = c->cursor;
+        const int chunk = part_chunk_rows(c, level);
+        const dim3 grid((unsigned)std::min<int64_t>(c->N / chunk + (1 << (level - 1)) + 1, 4096) + 1);
+#define PMCASE(T_, NI_)                                                                                              \
+    if (chunk == T_ * NI_) {                                                                                         \
+        if (A.stream_hint) hipLaunchKernelGGL((k_part_move<true, T_, NI_>), grid, dim3(T_), 0, c->stream, A, NX);    \
+        else hipLaunchKernelGGL((k_part_move<false, T_, NI_>), grid, dim3(T_), 0, c->stream, A, NX);                 \
+    }
+        PMCASE(256, 8) PMCASE(512, 8) PMCASE(512, 16)
+#undef PMCASE
+        HIPCHK(hipGetLastError());
+        return EVT_OK;
+    }
     // up to a thousand chunks per level the bookkeeping rides along in the scatter kernel (one launch less per level)
     A.fold = c->max_chunks <= 1024 + c->maxlvl ? 1 : 2;
     if (A.fold == 2) {
@@ -973,7 +1114,6 @@ int launch_part_scatter(evt_ctx *c, int level, const uint32_t *is_cur, uint32_t 
         A.node_stride = (int64_t)c->F * c->NAg * c->B;
         A.F = c->F;
         A.nfs = c->n_js_last;
-        A.NAg = c->NAg;
         const size_t lds = (size_t)c->NA * c->n_js_last * c->B * 8;
         if (A.fold != 1 || !scatter_can_build_hist(c, c->n_js_last)) {
             evt_set_error("internal: scatter pass cannot build histograms for this shape");

@@ -155,7 +155,7 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
         // the partition's chunk descriptors of this level, when the level's histograms came from the scatter pass above
         // and no histogram kernel wrote them: the highest wavefronts take them (idle unless 16 features are sampled)
         if (A.cdesc)
-            evt_fill_chunk_descriptors(A.hdr, A.act_node, A.cprefix, A.seg_start, A.seg_len, A.cdesc,
+            evt_fill_chunk_descriptors(A.hdr, A.act_node, A.cprefix, A.seg_start, A.seg_len, A.cdesc, EVT_CHUNK,
                                        (int)blockIdx.x * nwaves + (nwaves - 1 - wave), (int)gridDim.x * nwaves);
     }
     // The block's time is a chain of round trips to memory, so requests go out in as few dependent steps as the data
