@@ -751,6 +751,252 @@ __global__ __launch_bounds__(256) void k_obliv_apply(OblivArgs A) {
     }
 }
 
+// A whole oblivious level in one launch: a block owns a sampled feature and searches all nodes of the level, a wavefront one or two of them, as
+// k_scan; adds their gains in node order in LDS, and hands in its first maximum with the nodes' totals left of it; the last block to do
+// so takes the best and writes the level's decision, the children's totals and, on the last level that splits, their leaves.  The hand-over is
+// k_scan's.  Bound by that chain and, from 16 nodes on, by the divisions of a block's searches (nodes spread over several blocks need one
+// more hand-over, which cost more than it gave: 16 nodes 14.7 -> 16.2 us).  In three launches (k_scan, k_obliv_max, k_obliv_apply) and one for
+// the leaves the chain was cut by kernel boundaries: 500k rows x 50 features x 64 bins of two outputs, 1, 4, 16 and 32 nodes and the leaves,
+// 18.7, 15.5, 16.2 and 23.0 -> 8.8, 9.0, 12.5 and 15.6 us.
+struct OblivLevelArgs {
+    OblivArgs o;
+    const int32_t *mono;
+    int32_t *counts;
+    double min_weight;
+    int fold_leaves;
+    unsigned long long *lefts; // [feature][node][NAG]: totals left of the feature's candidate
+};
+#define OBLIV_LEVEL_NODES 32
+
+// NPW: nodes of a wavefront
+template <int NAG, int BPL, int NPW>
+__global__ __launch_bounds__(NAG * BPL > 12 ? 512 : 1024) void k_obliv_level(OblivLevelArgs L) {
+    extern __shared__ double s_gain[]; // [nodes][B]
+    __shared__ long long s_tot[OBLIV_LEVEL_NODES * NAG], s_left[OBLIV_LEVEL_NODES * NAG];
+    __shared__ int s_last, s_bin, s_cell;
+    __shared__ double s_best;
+    const OblivArgs &A = L.o;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
+    constexpr int K = (NAG == 5) ? 2 : 1, NK = 2 * K + 1;
+    const int B = A.B, jp = blockIdx.x;
+    // all nodes of a level split on the same feature or none does: the level's nodes are all active, or none is
+    const int first = 1 << (A.level - 1), nodes = first;
+    const bool any = A.hdr[LH_N_ACT] > 0;
+    const int f = (int)A.js[jp] - 1;
+    int st[NPW];
+#pragma unroll
+    for (int j = 0; j < NPW; j++) st[j] = A.status[first + (wave + j * nwaves < nodes ? wave + j * nwaves : 0)];
+    double sc[NAG];
+#pragma unroll
+    for (int ag = 0; ag < NAG; ag++) sc[ag] = A.qscale[ag];
+    if (!any) return; // every block alike
+    const bool numeric = A.feattypes[f] != 0;
+    const int constraint = L.mono[f];
+    const int64_t o0 = (int64_t)jp * NAG * B;
+    const int bmax = numeric ? B - 1 : B;
+
+    long long left[NPW][NAG][BPL]; // the words of the wavefront's nodes, requested together, then the sums left of every bin
+    {
+        long long vb[NPW][NAG][BPL], nsq[NPW][NAG];
+#pragma unroll
+        for (int j = 0; j < NPW; j++) {
+            const int n = first + (wave + j * nwaves < nodes ? wave + j * nwaves : 0);
+            const bool is_sub = st[j] == ST_SUBTRACT;
+            const long long *pa = A.hist + (int64_t)((is_sub ? n >> 1 : n) - 1) * A.node_stride + o0, *pb = A.hist + (int64_t)((n ^ 1) - 1) * A.node_stride + o0;
+#pragma unroll
+            for (int ag = 0; ag < NAG; ag++) {
+                nsq[j][ag] = A.node_sum[(int64_t)n * NAG + ag]; // not yet written at level 1, and not used there
+#pragma unroll
+                for (int t = 0; t < BPL; t++) {
+                    const int o = ag * B + (lane * BPL + t < B ? lane * BPL + t : B - 1);
+                    left[j][ag][t] = pa[o];
+                    vb[j][ag][t] = is_sub ? pb[o] : 0;
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NPW; j++) {
+            const int s = wave + j * nwaves, n = first + s;
+            if (s >= nodes) continue;
+            const bool is_sub = st[j] == ST_SUBTRACT;
+            long long *hn = A.hist + (int64_t)(n - 1) * A.node_stride + o0;
+#pragma unroll
+            for (int ag = 0; ag < NAG; ag++) {
+                long long run = 0, val[BPL];
+#pragma unroll
+                for (int t = 0; t < BPL; t++) {
+                    const int b = lane * BPL + t;
+                    val[t] = b < B ? left[j][ag][t] - vb[j][ag][t] : 0;
+                    if (is_sub && b < B) hn[ag * B + b] = val[t]; // subtract_hist!
+                    run += val[t];
+                    left[j][ag][t] = run;
+                }
+                const long long incl = wave_incl_scan_i64(run), excl = incl - run;
+                if (A.level == 1) { // the root's totals are any feature's sums over its bins
+                    nsq[j][ag] = readlane_i64(incl, 63);
+                    if (jp == 0 && lane == 0) A.node_sum[(int64_t)n * NAG + ag] = nsq[j][ag];
+                }
+                if (lane == 0) s_tot[s * NAG + ag] = nsq[j][ag];
+#pragma unroll
+                for (int t = 0; t < BPL; t++) left[j][ag][t] = numeric ? left[j][ag][t] + excl : val[t];
+            }
+            double S[NK];
+            decode_vals(nsq[j], sc, A.loss, NK, S);
+            double gain_p = 0.0;
+            for (int k = 0; k < K; k++) gain_p += node_gain_k(A.loss, S[k], S[K + k], S[2 * K], A.lambda, A.L2);
+            const double w_p = S[NK - 1];
+#pragma unroll
+            for (int t = 0; t < BPL; t++) {
+                const int b = lane * BPL + t;
+                long long q[NAG];
+#pragma unroll
+                for (int ag = 0; ag < NAG; ag++) q[ag] = left[j][ag][t];
+                double SL[NK];
+                decode_vals(q, sc, A.loss, NK, SL);
+                const double w_l = SL[NK - 1], w_r = w_p - w_l;
+                bool ok = b < B && b + 1 <= bmax && w_l > L.min_weight && w_r > L.min_weight;
+                if (ok && constraint != 0) {
+                    double SR[NK];
+                    for (int k = 0; k < NK; k++) SR[k] = S[k] - SL[k];
+                    const double predL = leaf_value(A.loss, SL, 0, K, A.eta, A.bagging, A.lambda, A.L2);
+                    const double predR = leaf_value(A.loss, SR, 0, K, A.eta, A.bagging, A.lambda, A.L2);
+                    ok = (constraint == -1 && predL > predR) || (constraint == 1 && predL < predR);
+                }
+                double gain = 0.0;
+                if (ok) {
+                    double sg = 0.0;
+                    for (int k = 0; k < K; k++) sg += split_gain_k(A.loss, S[k], S[K + k], w_p, SL[k], SL[K + k], w_l, w_r, A.lambda, A.L2);
+                    gain = sg - gain_p;
+                }
+                if (b < B) s_gain[s * B + b] = gain; // update_gains!
+            }
+        }
+    }
+    __syncthreads();
+    if (wave == 0) { // the feature's row of the level matrix and its first maximum
+        double bg = -INFINITY;
+        int bi = NO_BIN;
+        for (int b = lane; b < B; b += 64) {
+            double acc = 0.0;
+            bool allpos = true;
+#pragma unroll 8
+            for (int s = 0; s < nodes; s++) {
+                const double g = s_gain[s * B + b];
+                acc += g;
+                if (A.level > 1) allpos = allpos && g > 0.0;
+            }
+            const double v = allpos ? acc : 0.0;
+            if (v > bg) {
+                bg = v;
+                bi = b;
+            }
+        }
+        wave_argmax(bg, bi);
+        if (lane == 0) {
+            s_bin = bi;
+            s_best = bg;
+        }
+    }
+    __syncthreads();
+    const int bi = s_bin;
+    if (bi != NO_BIN) { // the totals left of it, from the lane that holds the bin
+#pragma unroll
+        for (int j = 0; j < NPW; j++) {
+            const int s = wave + j * nwaves;
+            if (s < nodes && lane == bi / BPL) {
+#pragma unroll
+                for (int ag = 0; ag < NAG; ag++) {
+                    long long v = left[j][ag][0];
+#pragma unroll
+                    for (int t = 1; t < BPL; t++) v = bi % BPL == t ? left[j][ag][t] : v;
+                    __hip_atomic_store(L.lefts + ((size_t)jp * nodes + s) * NAG + ag, (unsigned long long)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+        }
+    }
+    if (tid == 0) {
+        unsigned long long *mine = reinterpret_cast<unsigned long long *>(A.best + jp);
+        __hip_atomic_store(mine, (unsigned long long)__double_as_longlong(s_best), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(mine + 1, (unsigned long long)(unsigned int)bi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // every wavefront's part of the candidate is in memory before it is counted
+    __syncthreads();
+    if (tid == 0) s_last = __hip_atomic_fetch_add(L.counts, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+    if (A.zero_children && wave > 0) { // meanwhile, whatever the decision: the slices of a leaf are never read
+        for (int s = wave - 1; s < nodes; s += nwaves - 1) {
+            long long *hc = A.hist + (int64_t)(2 * (first + s) - 1) * A.node_stride + o0;
+            for (int i = lane; i < NAG * B; i += 64) {
+                hc[i] = 0;
+                hc[A.node_stride + i] = 0;
+            }
+        }
+    }
+    __syncthreads();
+    if (!s_last) return;
+    if (wave == 0) {
+        double g = -INFINITY;
+        int j = NO_BIN, b = 0;
+        const unsigned long long *cand = reinterpret_cast<const unsigned long long *>(A.best);
+        for (int q = lane; q < (int)gridDim.x; q += 64) { // ascending features: only a strictly larger gain replaces an earlier one
+            const double gg = __longlong_as_double((long long)__hip_atomic_load(cand + 2 * q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            const int c = (int)__hip_atomic_load(cand + 2 * q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (gg > g) {
+                g = gg;
+                j = q;
+                b = c;
+            }
+        }
+        const int own = j;
+        wave_argmax(g, j); // highest gain, then the earliest feature, whose bin is already the lowest
+        if (j != NO_BIN ? own == j : lane == 0) {
+            s_best = g;
+            s_cell = j != NO_BIN && g > A.gamma ? j : NO_BIN;
+            s_bin = b;
+            *L.counts = 0;
+        }
+    }
+    __syncthreads();
+    const bool found = s_cell != NO_BIN;
+    const int bj = found ? s_cell : 0, bb = s_bin + 1;
+    if (found && tid < nodes * NAG)
+        s_left[tid] = (long long)__hip_atomic_load(L.lefts + (size_t)bj * nodes * NAG + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int feat = (int)A.js[bj];
+    const bool num = A.feattypes[feat - 1] != 0;
+    __syncthreads();
+    // a thread writes a node, or a child
+    const int who = tid / nodes, s = tid % nodes, n = first + s;
+    double S[EVT_MAX_NK];
+    if (who == 0) {
+        decode_vals(s_tot + s * NAG, sc, A.loss, NK, S);
+        A.tree.w[n - 1] = (float)S[NK - 1];
+        A.status[n] = found ? ST_SPLIT : ST_LEAF;
+        if (found) {
+            A.tree.feat[n - 1] = feat;
+            A.tree.cond_bin[n - 1] = (uint8_t)bb;
+            A.tree.gain[n - 1] = (float)s_best;
+            A.tree.split[n - 1] = 1;
+            A.tree.packed[n - 1] = evt_pack_node(feat, bb, num);
+        } else {
+            for (int k = 0; k < K; k++) A.tree.pred[(int64_t)K * (n - 1) + k] = (float)leaf_value(A.loss, S, k, K, A.eta, A.bagging, A.lambda, A.L2);
+        }
+    } else if (found && who <= 2) {
+        const int cn = 2 * n + who - 1;
+        long long qc[NAG];
+#pragma unroll
+        for (int ag = 0; ag < NAG; ag++) {
+            const long long l = s_left[s * NAG + ag];
+            qc[ag] = who == 2 ? s_tot[s * NAG + ag] - l : l;
+            A.node_sum[(int64_t)cn * NAG + ag] = qc[ag];
+        }
+        if (L.fold_leaves) { // as the pass over the last level would (write_children)
+            decode_vals(qc, sc, A.loss, NK, S);
+            A.tree.w[cn - 1] = (float)S[NK - 1];
+            for (int k = 0; k < K; k++) A.tree.pred[(int64_t)K * (cn - 1) + k] = (float)leaf_value(A.loss, S, k, K, A.eta, A.bagging, A.lambda, A.L2);
+            A.status[cn] = ST_LEAF;
+        }
+    }
+}
+
 // ---- any number of outputs (multi-class log loss) ------------------------------------------------
 // Same search as k_scan / k_scan_fin with the channel count a run-time value: the node statistics live in shared
 // memory and the candidate gain is the sum of term(left_k) + term(right_k) over the outputs, added in the
@@ -808,8 +1054,7 @@ struct ChannelWords {
         const long long incl = wave_incl_scan_i64(run), excl = incl - run;
 #pragma unroll
         for (int t = 0; t < BPL; t++) left[t] = numeric ? left[t] + excl : val[t];
-        const int lo = __builtin_amdgcn_readlane((int)(incl & 0xffffffffll), 63), hi = __builtin_amdgcn_readlane((int)(incl >> 32), 63);
-        return ((long long)hi << 32) | (unsigned int)lo;
+        return readlane_i64(incl, 63);
     }
 };
 
@@ -1096,10 +1341,22 @@ __global__ __launch_bounds__(256) void k_scan_fin_mc(ScanArgs A, int ngroups) {
 // of one node nor one of wide slices (16 channels x 100 features: 1.6 MB per node) leaves them to few blocks.
 static unsigned zero_blocks_per_node(unsigned nodes) { return nodes >= 512 ? 1u : (512u / nodes < 64u ? 512u / nodes : 64u); }
 
-// The pass over the last split level also writes its children's leaf values (binary trees with the fixed channel layouts).
-bool scan_folds_leaves(const evt_ctx *c) { return !c->mc && c->tree_type != EVT_TREE_OBLIVIOUS && c->D > 1; }
+// An oblivious level in one launch: where a wavefront's words (nodes x channels x bins per lane) are few enough for its registers and the searches a
+// block's wavefronts share do not outlast the launches saved.  us of a level in three launches | one, event pairs included (60k rows; 20 to 120
+// features): mse 64 bins 4 nodes 14 | 8, 16 nodes 16 | 9, 32 nodes 19 | 14; mse 128 bins 32 nodes 21 | 19; mse 255 bins 16 nodes 20 | 18, 32 nodes 27 | 32;
+// logloss 128 bins 16 nodes 18 | 13, 32 nodes 21 | 21; two outputs 64 bins 16 nodes 14 | 13, 128 bins 16 nodes 17 | 17, 255 bins 8 nodes 25 | 20, 16 nodes 24 | 32.
+static bool obliv_one_launch(const evt_ctx *c, int level) {
+    const int nodes = 1 << (level - 1), words = c->NAg * ((c->B + 63) / 64);
+    return c->tree_type == EVT_TREE_OBLIVIOUS && !c->mc && c->scan_fused && c->B >= 4 && nodes <= OBLIV_LEVEL_NODES && nodes * words <= 192;
+}
+
+// The pass over the last split level also writes its children's leaf values (the fixed channel layouts).
+bool scan_folds_leaves(const evt_ctx *c) { return !c->mc && c->D > 1 && (c->tree_type != EVT_TREE_OBLIVIOUS || obliv_one_launch(c, c->D - 1)); }
+
+static int launch_obliv_level(evt_ctx *c, int level, const evt_params *p);
 
 int launch_scan(evt_ctx *c, int level, const evt_params *p, bool leaf_level) {
+    if (!leaf_level && obliv_one_launch(c, level)) return launch_obliv_level(c, level, p);
     ScanArgs A;
     A.sbest = reinterpret_cast<ScanBest *>(c->sbest);
     A.hist = c->hist;
@@ -1182,9 +1439,8 @@ int launch_scan(evt_ctx *c, int level, const evt_params *p, bool leaf_level) {
     return EVT_OK;
 }
 
-int launch_obliv_select(evt_ctx *c, int level, const evt_params *p) {
+static void fill_obliv_args(evt_ctx *c, int level, const evt_params *p, OblivArgs &A) {
     const LevelTab &L = c->lvl[level & 1];
-    OblivArgs A;
     A.hist = c->hist;
     A.node_stride = (int64_t)c->F * c->NAg * c->B;
     A.js = c->js;
@@ -1202,6 +1458,36 @@ int launch_obliv_select(evt_ctx *c, int level, const evt_params *p) {
     A.zero_children = (level + 1 < c->D) ? 1 : 0;
     A.best = reinterpret_cast<ScanBest *>(c->sbest);
     A.nbest = (int)std::min<int64_t>(EVT_OBLIV_BLOCKS, ((int64_t)A.nfs * A.B + 255) / 256);
+}
+
+static int launch_obliv_level(evt_ctx *c, int level, const evt_params *p) {
+    OblivLevelArgs A;
+    fill_obliv_args(c, level, p, A.o);
+    A.mono = c->mono;
+    A.counts = c->scan_count;
+    A.min_weight = p->min_weight;
+    A.fold_leaves = level + 1 == c->D ? 1 : 0;
+    A.lefts = reinterpret_cast<unsigned long long *>(c->ogains); // nodes x features x bins words, unused in this form
+    const int nodes = 1 << (level - 1), bpl = (c->B + 63) / 64;
+    const dim3 grid((unsigned)A.o.nfs), block(64u * std::min(16, std::max(4, nodes)));
+    const size_t lds = (size_t)nodes * c->B * sizeof(double);
+#define OLCASE(NAG_, BPL_, NPW_)                                                                         \
+    if (c->NAg == NAG_ && (bpl <= 2 ? bpl : 4) == BPL_ && (nodes > 16) == (NPW_ > 1)) {                  \
+        hipLaunchKernelGGL((k_obliv_level<NAG_, BPL_, NPW_>), grid, block, lds, c->stream, A);           \
+        HIPCHK(hipGetLastError());                                                                       \
+        return EVT_OK;                                                                                   \
+    }
+    OLCASE(2, 1, 1) OLCASE(2, 2, 1) OLCASE(2, 4, 1) OLCASE(3, 1, 1) OLCASE(3, 2, 1) OLCASE(3, 4, 1) OLCASE(5, 1, 1) OLCASE(5, 2, 1) OLCASE(5, 4, 1)
+    OLCASE(2, 1, 2) OLCASE(2, 2, 2) OLCASE(3, 1, 2) OLCASE(3, 2, 2) OLCASE(5, 1, 2)
+#undef OLCASE
+    evt_set_error("unsupported global channel count %d", c->NAg);
+    return EVT_ERR_ARG;
+}
+
+int launch_obliv_select(evt_ctx *c, int level, const evt_params *p) {
+    if (obliv_one_launch(c, level)) return EVT_OK; // decided by launch_obliv_level
+    OblivArgs A;
+    fill_obliv_args(c, level, p, A);
     hipLaunchKernelGGL(k_obliv_max, dim3((unsigned)A.nbest), dim3(256), 0, c->stream, A);
     const unsigned nodes = 1u << (level - 1);
     hipLaunchKernelGGL(k_obliv_apply, dim3(nodes, A.zero_children ? 1 + zero_blocks_per_node(nodes) : 1), dim3(256), 0, c->stream, A);

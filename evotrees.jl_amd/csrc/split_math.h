@@ -26,14 +26,13 @@ __device__ __forceinline__ long long wave_incl_scan_i64(long long x) {
     return x;
 }
 
-__device__ __forceinline__ long long wave_sum_i64(long long x) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        int lo = __shfl_xor((int)(x & 0xffffffffll), o), hi = __shfl_xor((int)(x >> 32), o);
-        x += ((long long)hi << 32) | (unsigned int)lo;
-    }
-    return x;
+__device__ __forceinline__ long long readlane_i64(long long x, int lane) {
+    const int lo = __builtin_amdgcn_readlane((int)(x & 0xffffffffll), lane), hi = __builtin_amdgcn_readlane((int)(x >> 32), lane);
+    return ((long long)hi << 32) | (unsigned int)lo;
 }
+
+// Sum over the wavefront, in every lane: the scan's last lane (VALU moves; twelve cross-lane shuffles are as many trips through the LDS crossbar)
+__device__ __forceinline__ long long wave_sum_i64(long long x) { return readlane_i64(wave_incl_scan_i64(x), 63); }
 
 // Arg-max over the 64 lanes of a wavefront: highest gain, of equal gains the lowest bin; every lane gets the result.
 // Same data movement as the prefix scan above (row shifts, then row broadcasts; a lane without a source combines with
