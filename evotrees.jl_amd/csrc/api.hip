@@ -1723,7 +1723,7 @@ extern "C" int evt_set_option(evt_handle c, const char *name, int64_t value) {
     } else if (strcmp(name, "record_nidx") == 0) {
         c->record_nidx = value != 0;
     } else if (strcmp(name, "small_tree") == 0) {
-        ARGCHK(value >= 0 && value <= 3, "small_tree must be 0 (never), 1 (inputs of few rows), 2 or 3 (one or two kernels per level wherever it can)");
+        ARGCHK(value >= 0 && value <= 3, "small_tree must be 0 (never), 1 (inputs of few rows), 2 or 3 (a block, or several, per feature and level wherever it can)");
         c->small_tree = (int)value;
     } else if (strcmp(name, "scan_fused") == 0) {
         c->scan_fused = value != 0;

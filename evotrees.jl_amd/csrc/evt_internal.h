@@ -197,7 +197,7 @@ struct evt_ctx {
     int hist_blocks, hist_threads, hist_min_rows, hist_seg_cost, hist_tile;
     int hist_variant;  // 0 auto, 1 generic 16-byte-piece kernel, 2 conflict-free 8-byte-piece kernel where it applies
     int scan_fused;    // option: the split search of a node with at most 16 sampled features runs in one kernel
-    int small_tree;    // option: one kernel per level (kernels_small.hip) - 0 never, 1 for inputs of few rows, 2 wherever it can, 3 the form of two kernels per level wherever it can
+    int small_tree;    // option: one kernel per level (kernels_small.hip) - 0 never, 1 for inputs of few rows, 2 wherever it can, 3 with several blocks to a feature wherever it can
     // its buffers, allocated with the first such tree: the rows' node ids, the blocks' candidates and the totals left of them, of
     // two levels each
     uint32_t *small_nid[2];
@@ -222,7 +222,7 @@ struct evt_ctx {
         int level;
         bool all_rows, defer, fuse_pred;
         bool hist_fused; // levels below the root get their histograms from the scatter pass of the level above
-        int small;       // one kernel per level, or two and the blocks that share a feature's rows (small_tree_form)
+        int small;       // one kernel per level: the blocks that share a feature's rows (small_tree_form)
         bool small_draw; // ... whose first draws the row mask
         bool blob_sent;  // the finished tree's transfer to the host rode along with the tree's last kernel
         uint32_t *is_cur, *is_next; // row-id lists of the current level and of the one below

@@ -1,4 +1,4 @@
-// Trees of small inputs (thousands to a few hundred thousand rows): one or two kernels per level instead of a histogram, a search and a two-pass partition.
+// Trees of small inputs (thousands to a few hundred thousand rows): one kernel per level instead of a histogram, a search and a partition.
 //
 // At these sizes a level is a chain of short dependent kernels - 20 launches of 3 to 9 us for a tree of depth 6 on 2000 rows, whatever they
 // do.  Here a block owns one sampled feature and walks ALL rows: it takes the decisions of the level above (every block the same
@@ -55,6 +55,8 @@ struct SmallArgs {
     int slices;    // blocks that share a feature's rows
     long long *acc; // slices > 1: [node][block][NAg][B], their histograms added up; zero between two levels
     int *counts;    // ... and their rows, [level][slice]
+    int *done;      // ... and how many of a feature's blocks have added theirs, zero between two levels
+    int batch;      // ... and the nodes whose sums its last block's LDS holds at a time
     int oblivious, sampled, draw, cond;
     int wide;      // channel 0 staged as a 64-bit packed word (more channels than EVT_MAX_NA)
     // the blocks' features, in the launch's arguments: a block need not wait for them.  0-based id | numeric << 16 | (constraint + 1) << 17
@@ -307,13 +309,17 @@ __device__ __forceinline__ void small_scan(const SmallArgs &A, const unsigned lo
     }
 }
 
-// totals left of bin lb (numeric: the bins up to it, categorical: it alone), a channel at a time
-template <bool PACK>
+// totals left of bin lb (numeric: the bins up to it, categorical: it alone), a channel at a time.  SUMS: Hs lies in memory, where other blocks
+// have added to it in this launch
+template <bool PACK, bool SUMS>
 __device__ __forceinline__ void small_left(const SmallArgs &A, const unsigned long long *Hs, int nag, bool numeric, int lb, int lane, SmallHead *out, long long *left) {
     for (int ag = 0; ag < nag; ag++) {
         long long t = 0;
         for (int b = lane; b < lb && b < A.B; b += 64)
-            if (numeric || b + 1 == lb) t += channel_of<PACK>(Hs, A.B, nag, ag, b);
+            if (numeric || b + 1 == lb) {
+                if (SUMS) t += (long long)__hip_atomic_load(Hs + ag * A.B + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                else t += channel_of<PACK>(Hs, A.B, nag, ag, b);
+            }
         t = wave_sum_i64(t);
         if (lane == 0) {
             if (nag <= EVT_MAX_NA) out->left[ag] = t;
@@ -382,7 +388,7 @@ __device__ __forceinline__ void small_search(const SmallArgs &A, const unsigned 
             out->bin = lb;
             out->feat = feat;
         }
-        if (lb != NO_BIN) small_left<PACK>(A, Hs, nag, numeric, lb, lane, out, A.left_out + ((int64_t)q * nwg + jp) * nag);
+        if (lb != NO_BIN) small_left<PACK, false>(A, Hs, nag, numeric, lb, lane, out, A.left_out + ((int64_t)q * nwg + jp) * nag);
     }
 }
 
@@ -410,9 +416,12 @@ __device__ __forceinline__ int small_obliv_best(const SmallArgs &A, const double
     return bb;
 }
 
-// SPLIT: a feature's rows are shared by `slices` blocks, which add their histograms into A.acc instead of searching them;
-// k_small_scan does that.  For inputs of few features, whose blocks would fill a part of the chip with long walks: 10 features in 25
-// slices take 0.4 us per 25k rows and channel pair where one block per feature takes 0.4 us per 1k, for 8 us more of launch and flush.
+// SPLIT: a feature's rows are shared by `slices` blocks, which add their histograms into A.acc; the last of them to do so reads the sums and
+// searches them (100k rows x 10 features: 8.3 us a level and 5.2 for a kernel of its own that searched -> 13.9, and a round of five levels
+// 101 -> 92 us).  What passes between the blocks goes by agent-scope atomics, past the caches that are not shared, and is complete before its
+// block is counted (as in k_scan).  For inputs of
+// few features, whose blocks would fill a part of the chip with long walks: 10 features in 25 slices take 0.4 us per 25k rows and channel pair
+// where one block per feature takes 0.4 us per 1k, for 5 us more of flush and hand-over.
 template <int NAG, int BPL, bool PACK, bool SPLIT>
 __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
     extern __shared__ unsigned long long s_dyn[];
@@ -636,7 +645,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
         const int lb = s_best;
         for (int s = wave; s < nact; s += 16) {
             const int64_t at = (int64_t)s_node[s] * gridDim.x + jp;
-            small_left<PACK>(A, H + (size_t)s * na * B, nag, numeric, lb, lane, A.head_out + at, A.left_out + at * nag);
+            small_left<PACK, false>(A, H + (size_t)s * na * B, nag, numeric, lb, lane, A.head_out + at, A.left_out + at * nag);
         }
     }
     if (jp == 0) { // rows of the level: the root's is the size of the sample
@@ -650,66 +659,55 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
             if (level == 1) A.stats[0] = s_cnt;
         }
     }
-}
-
-// The searches of a level whose histograms the slices of k_small_level<SPLIT> left in A.acc: a wavefront per (node, feature), 16 nodes of one
-// feature to a block (all of them for an oblivious level, whose nodes' gains meet in LDS).
-template <int NAG, int BPL>
-__global__ __launch_bounds__(1024) void k_small_scan(SmallArgs A) {
-    extern __shared__ double s_gain[]; // oblivious: [active nodes][B]
-    __shared__ uint16_t s_node[SMALL_MAX_NODES];
-    __shared__ int s_nact, s_best;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int B = A.B, nag = NAG ? NAG : A.NAg, jp = blockIdx.x, first = 1 << (A.level - 1);
-    const uint32_t fw = A.feat[jp];
-    auto of = [&](int q) { return A.acc + ((size_t)q * A.nfs + jp) * nag * B; };
-    auto search = [&](int q, double *gain) {
-        small_search<NAG, BPL, false>(A, reinterpret_cast<const unsigned long long *>(of(q)), q, jp, A.nfs, fw,
-                                      A.level > 1 ? A.node_sum + (int64_t)(first + q) * nag : nullptr, jp == 0, gain, lane);
-    };
-    auto clear = [&](int q) {
-        for (int i = lane; i < nag * B; i += 64) of(q)[i] = 0;
-    };
-    if (!A.oblivious) {
-        const int q = (int)blockIdx.y * 16 + wave;
-        if (q >= first || A.status[first + q] != ST_BUILD) return;
-        search(q, nullptr);
-        clear(q);
-        return;
-    }
-    if (wave == 0) {
-        int base = 0;
-        for (int q0 = 0; q0 < first; q0 += 64) {
-            const bool on = q0 + lane < first && A.status[first + q0 + lane] == ST_BUILD;
-            const unsigned long long m = __ballot(on);
-            if (on) s_node[base + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)(q0 + lane);
-            base += __popcll(m);
+    if constexpr (SPLIT) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the block's sums are in memory before it is counted
+        __syncthreads();
+        if (tid == 0) s_best = __hip_atomic_fetch_add(A.done + jp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == A.slices - 1;
+        __syncthreads();
+        if (!s_best) return;
+        if (tid == 0) A.done[jp] = 0;
+        double *gains = s_gain; // oblivious: [active nodes][B]
+        unsigned long long *S = reinterpret_cast<unsigned long long *>(s_gain + (A.oblivious ? nact * B : 0)); // [batch][nag][B]
+        const int words = nag * B;
+        auto sums = [&](int q) { return reinterpret_cast<unsigned long long *>(A.acc) + ((size_t)q * A.nfs + jp) * words; };
+        for (int base = 0; base < nact; base += A.batch) {
+            const int nb = nact - base < A.batch ? nact - base : A.batch;
+            for (int i = tid; i < nb * words; i += 1024) {
+                const int k = i / words;
+                S[i] = __hip_atomic_load(sums(s_node[base + k]) + (i - k * words), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            __syncthreads();
+            for (int k = wave; k < nb; k += 16) {
+                const int q = s_node[base + k];
+                small_search<NAG, BPL, false>(A, S + (size_t)k * words, q, jp, A.nfs, fw, level > 1 ? s_tot + q * nag : nullptr, jp == 0,
+                                              A.oblivious ? gains + (base + k) * B : nullptr, lane);
+            }
+            __syncthreads();
         }
-        if (lane == 0) s_nact = base;
-    }
-    __syncthreads();
-    const int nact = s_nact;
-    for (int s = wave; s < nact; s += 16) search(s_node[s], s_gain + s * B);
-    __syncthreads();
-    const bool numeric = (fw & SMALL_NUMERIC) != 0;
-    if (wave == 0) {
-        double bg;
-        const int bb = small_obliv_best(A, s_gain, nact, lane, &bg);
-        if (lane == 0) s_best = bb;
-        for (int s = lane; s < nact; s += 64) {
-            SmallHead *out = A.head_out + (int64_t)s_node[s] * A.nfs + jp;
-            out->gain = bg;
-            out->bin = bb;
-            out->feat = numeric ? (int)(fw & 0xFFFFu) + 1 : -((int)(fw & 0xFFFFu) + 1);
+        if (A.oblivious) {
+            if (wave == 0) {
+                double bg;
+                const int bb = small_obliv_best(A, gains, nact, lane, &bg);
+                if (lane == 0) s_best = bb;
+                for (int k = lane; k < nact; k += 64) {
+                    SmallHead *out = A.head_out + (int64_t)s_node[k] * A.nfs + jp;
+                    out->gain = bg;
+                    out->bin = bb;
+                    out->feat = numeric ? f + 1 : -(f + 1);
+                }
+            }
+            __syncthreads();
+            const int lb = s_best;
+            for (int k = wave; k < nact; k += 16) {
+                const int64_t at = (int64_t)s_node[k] * A.nfs + jp;
+                small_left<false, true>(A, sums(s_node[k]), nag, numeric, lb, lane, A.head_out + at, A.left_out + at * nag);
+            }
+            __syncthreads();
         }
-    }
-    __syncthreads();
-    const int lb = s_best;
-    for (int s = wave; s < nact; s += 16) {
-        const int q = s_node[s];
-        const int64_t at = (int64_t)q * A.nfs + jp;
-        small_left<false>(A, reinterpret_cast<const unsigned long long *>(of(q)), nag, numeric, lb, lane, A.head_out + at, A.left_out + at * nag);
-        clear(q);
+        for (int i = tid; i < nact * words; i += 1024) {
+            const int k = i / words;
+            sums(s_node[k])[i - k * words] = 0;
+        }
     }
 }
 
@@ -753,6 +751,11 @@ static size_t small_lds(const evt_ctx *c, int level, int slots, bool split) {
     const size_t gain = c->tree_type == EVT_TREE_OBLIVIOUS && !split ? (size_t)slots * c->B * 8 : 0;
     return tot + gain + (size_t)slots * c->NA * c->B * 8;
 }
+// of the last of a feature's blocks: the nodes' gains (oblivious) and the sums of `batch` nodes, in the place of its histograms
+static size_t small_lds_search(const evt_ctx *c, int level, int batch) {
+    const size_t nodes = (size_t)1 << (level - 1), tot = level > 1 ? nodes * c->NAg * 8 : 0;
+    return tot + (c->tree_type == EVT_TREE_OBLIVIOUS ? nodes * c->B * 8 : 0) + (size_t)batch * c->NAg * c->B * 8;
+}
 // histograms a block's LDS holds at the deepest level that splits
 static int small_slots(const evt_ctx *c, bool split) {
     const int nodes = 1 << std::max(0, c->D - 2);
@@ -774,7 +777,7 @@ static int small_tree_buffers(evt_ctx *c, bool split) {
     }
     if (split && !c->small_acc) {
         // the counts of the slices' rows, then the sums, for the larger of the weight modes
-        const size_t bytes = 16 * 256 * sizeof(int) + small_acc_bytes(c) / c->NAg * c->NK;
+        const size_t bytes = 17 * 256 * sizeof(int) + small_acc_bytes(c) / c->NAg * c->NK; // the blocks' counts behind the rows'
         c->small_acc = static_cast<uint8_t *>(dev_take(bytes));
         if (!c->small_acc) return EVT_ERR_NOMEM;
         const int r = launch_fill_bytes(c, c->small_acc, (int64_t)bytes);
@@ -783,7 +786,7 @@ static int small_tree_buffers(evt_ctx *c, bool split) {
     return EVT_OK;
 }
 
-// Which form a tree takes: 0 the kernels of larger inputs, 1 one kernel per level, S > 1 two kernels per level with a feature's rows
+// Which form a tree takes: 0 the kernels of larger inputs, 1 a block per feature, S > 1 a feature's rows
 // shared by S blocks.  A block walks its rows once per level (and once more for every `slots` nodes), so a level grows with
 // rows / S, the channels and - through the candidates every block reads and the searches its 16 wavefronts share - the nodes; slices
 // add a launch and the words they flush.  The other path spreads rows of any number over the chip and pays for its launches.  Estimates
@@ -799,7 +802,7 @@ int small_tree_form(const evt_ctx *c, int nfs, bool all_rows) {
     const int nodes = 1 << (c->D - 2), slots = small_slots(c, false), slots_split = small_slots(c, true);
     const int S = std::max(2, 256 / nfs);
     const bool can1 = c->N <= 65535 && slots >= 1 && (!obliv || slots == nodes);
-    const bool canS = slots_split >= 1 && c->N / S < 65000 && small_acc_bytes(c) <= ((size_t)64 << 20) && (!obliv || (size_t)nodes * c->B * 8 <= 144 * 1024);
+    const bool canS = slots_split >= 1 && c->N / S < 65000 && small_acc_bytes(c) <= ((size_t)64 << 20) && small_lds_search(c, c->D - 1, 1) <= 144 * 1024;
     if (c->small_tree == 2) return can1 ? 1 : 0;
     if (c->small_tree == 3) return canS ? S : 0;
     const double k = 1e-3 * c->N, per_1k = c->mc ? 0.3 + 0.2 * c->NA : 0.35 + 0.058 * c->NA, per_1k_s = c->mc ? 0.3 + 0.3 * c->NA : per_1k;
@@ -851,7 +854,8 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
     A.slots = small_slots(c, split);
     A.slices = slices;
     A.counts = reinterpret_cast<int *>(c->small_acc);
-    A.acc = reinterpret_cast<long long *>(c->small_acc + 16 * 256 * sizeof(int));
+    A.done = A.counts + 16 * 256;
+    A.acc = reinterpret_cast<long long *>(c->small_acc + 17 * 256 * sizeof(int));
     A.oblivious = c->tree_type == EVT_TREE_OBLIVIOUS ? 1 : 0;
     A.sampled = c->step.all_rows ? 0 : 1;
     A.draw = draw ? 1 : 0;
@@ -880,14 +884,19 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
         const int nodes = 1 << (level - 1), slots = std::min(A.slots, nodes);
         const int most = A.slots;
         A.slots = slots;
-        const size_t lds = small_lds(c, level, slots, split), gain = A.oblivious ? (size_t)nodes * c->B * 8 : 0;
+        size_t lds = small_lds(c, level, slots, split);
+        if (split) { // a wavefront per node at a time, as far as they fit
+            A.batch = std::min(16, nodes);
+            while (A.batch > 1 && small_lds_search(c, level, A.batch) > std::max<size_t>(lds, 72 * 1024)) A.batch >>= 1;
+            lds = std::max(lds, small_lds_search(c, level, A.batch));
+        }
         prof_begin(c, level == 1 ? EVT_K_HIST : EVT_K_PARTITION, level); // below the root it moves rows, builds and searches at once
 #define SMALL3(NAG_, BPL_, PACK_)                                                                                                                  \
     {                                                                                                                                              \
         static EvtDevOnce once;                                                                                                                    \
         if (once.pending(c->device)) {                                                                                                             \
             for (const void *k : {reinterpret_cast<const void *>(k_small_level<NAG_, BPL_, PACK_, false>),                                         \
-                                  reinterpret_cast<const void *>(k_small_level<NAG_, BPL_, PACK_, true>), reinterpret_cast<const void *>(k_small_scan<NAG_, BPL_>)}) \
+                                  reinterpret_cast<const void *>(k_small_level<NAG_, BPL_, PACK_, true>)})                                         \
                 HIPCHK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));                                            \
             once.mark(c->device);                                                                                                                  \
         }                                                                                                                                          \
@@ -896,9 +905,6 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
             hipLaunchKernelGGL((k_small_level<NAG_, BPL_, PACK_, false>), dim3(nf), dim3(1024), lds, c->stream, A);                                \
         } else {                                                                                                                                   \
             hipLaunchKernelGGL((k_small_level<NAG_, BPL_, PACK_, true>), dim3(nf, (unsigned)slices), dim3(1024), lds, c->stream, A);               \
-            prof_end(c);                                                                                                                           \
-            prof_begin(c, EVT_K_SCAN, level);                                                                                                      \
-            hipLaunchKernelGGL((k_small_scan<NAG_, BPL_>), dim3(nf, A.oblivious ? 1u : (unsigned)((nodes + 15) / 16)), dim3(1024), gain, c->stream, A); \
         }                                                                                                                                          \
     }
 #define SMALL2(NAG_, PACK_)             \

@@ -405,8 +405,8 @@ int evt_reset_profile(evt_handle h);
  * "bit_planes" (1, default: before the first tree the library derives one bit plane per
  * (feature, bin threshold) from x_bin - F * (nbins - 1) * nobs / 8 bytes, taken only when that is at most 16 GiB and a third of the free
  * memory - and the row partition reads its decisions there; 0: it gathers bin bytes; same trees, bit for bit);
- * "small_tree" (inputs of few rows and up to 256 sampled features and depth 10 may grow a tree with one kernel per level, or two: 1,
- * default: where that is estimated to be faster; 0: never; 2, 3: the one or the other wherever it can; same trees, bit for bit);
+ * "small_tree" (inputs of few rows and up to 256 sampled features and depth 10 may grow a tree with one kernel per level, a block or several
+ * to a feature: 1, default: where that is estimated to be faster; 0: never; 2, 3: one block or several wherever it can; same trees, bit for bit);
  * "record_nidx" (1: the partition also records every sampled row's final node while the tree grows;
  * 0, default: evt_get_nidx derives it afterwards by walking the finished tree); "defer_pred" (1, default:
  * leaf values of a tree grown on every row are added in row order by the next pass over the rows;
@@ -415,8 +415,9 @@ int evt_reset_profile(evt_handle h);
  * while the host collects the tree, and that next call returns at once; meant for bagging_size 1 - with more
  * trees per round only the last one's work is used; 0, default; results do not depend on it); "scan_fused"
  * (1, default: one kernel searches and finishes a node's split - one block per node with at most 16 sampled features, else the last of a
- * node's blocks decides; oblivious trees take kernels of their own -, 0: two kernels)
- * and "hist_in_scatter" (1, default: with at most 16 features and a quarter of a million rows the levels below
+ * node's blocks decides; an oblivious level of up to 32 nodes is decided by the last of the level's blocks -, 0: a kernel of its own decides),
+ * "part_one_pass" (1, default: without weights the rows of a level move to their children in one kernel; 0: a count and a
+ * scatter pass) and "hist_in_scatter" (1, default: with at most 16 features and a quarter of a million rows the levels below
  * the root get their histograms from the partition's scatter pass, one kernel less per level; 0: a histogram
  * kernel per level) - same trees and histograms, bit for bit, either way. */
 int evt_set_option(evt_handle h, const char *name, int64_t value);
