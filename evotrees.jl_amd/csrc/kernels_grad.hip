@@ -88,8 +88,10 @@ __device__ __forceinline__ void raise_maxima(const float *mx, int K, uint32_t *a
 // LOSS: 0 mse (src/loss.jl:52), 1 logloss (:54-57), 2 gaussian_mle (:194-203), 3 poisson (:59-62),
 // 4 gamma (:64-67), 5 tweedie with rho = 1.5 (:69-76), 8 mae (:78), 9 cred_var / cred_std (:80-83).
 // grad rows: [g_1..g_K, h_1..h_K, w]; every written value is multiplied by w (src/loss.jl:104-108, :223-233).
+// Blocks of 256 threads, or of 1024 where the grid fills the chip: the blocks of a whole generation raise their maxima at the same time, and a
+// quarter of them queue for a quarter as long (1M rows, blocks of 256 | 1024: 8.4 | 6.5 us).
 template <int LOSS>
-__global__ __launch_bounds__(256) void k_grads(float *__restrict__ pred, const float *__restrict__ y, float *__restrict__ grad, int64_t N,
+__global__ __launch_bounds__(1024) void k_grads(float *__restrict__ pred, const float *__restrict__ y, float *__restrict__ grad, int64_t N,
                                               uint32_t *absmax, const uint32_t *__restrict__ pend_nidx,
                                               const float *__restrict__ pend_leaf, int unit_w) {
     constexpr int K = (LOSS == 2 || LOSS == 7) ? 2 : 1;
@@ -97,7 +99,7 @@ __global__ __launch_bounds__(256) void k_grads(float *__restrict__ pred, const f
     float mx[2 * K];
 #pragma unroll
     for (int k = 0; k < 2 * K; k++) mx[k] = 0.0f;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < N; i += (int64_t)gridDim.x * 256) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += (int64_t)gridDim.x * blockDim.x) {
         float out[2 * K];
         float *g = grad + (size_t)NK * i;
         const float w = unit_w ? 1.0f : g[NK - 1]; // unit weights: the weight row (all ones) is not read
@@ -146,7 +148,7 @@ __global__ __launch_bounds__(256) void k_grads(float *__restrict__ pred, const f
     }
     // per gradient row max |v| -> exponent bound of the fixed-point histogram.
     // One atomic per block and row: contended same-address atomics serialise in L2.
-    __shared__ float s_m[4][2 * K];
+    __shared__ float s_m[16][2 * K];
 #pragma unroll
     for (int k = 0; k < 2 * K; k++) {
         const float m = wave_max_f32(mx[k]);
@@ -155,7 +157,8 @@ __global__ __launch_bounds__(256) void k_grads(float *__restrict__ pred, const f
     __syncthreads();
     if (threadIdx.x < 2 * K) {
         const int k = threadIdx.x;
-        const float m = fmaxf(fmaxf(s_m[0][k], s_m[1][k]), fmaxf(s_m[2][k], s_m[3][k]));
+        float m = s_m[0][k];
+        for (int w = 1; w < (int)blockDim.x >> 6; w++) m = fmaxf(m, s_m[w][k]);
         absmax_raise(absmax, k, m);
     }
 }
@@ -446,22 +449,24 @@ int launch_grads(evt_ctx *c) {
         HIPCHK(hipGetLastError());
         return EVT_OK;
     }
+    const bool wide = nb == 2048;
+    const dim3 grid1(wide ? 512u : (unsigned)nb), block1(wide ? 1024u : 256u);
     if (c->loss == EVT_LOSS_MSE)
-        hipLaunchKernelGGL(k_grads<0>, grid, dim3(256), 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
+        hipLaunchKernelGGL(k_grads<0>, grid1, block1, 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
     else if (c->loss == EVT_LOSS_LOGLOSS)
-        hipLaunchKernelGGL(k_grads<1>, grid, dim3(256), 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
+        hipLaunchKernelGGL(k_grads<1>, grid1, block1, 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
     else if (c->loss == EVT_LOSS_LOGISTIC_MLE)
-        hipLaunchKernelGGL(k_grads<7>, grid, dim3(256), 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
+        hipLaunchKernelGGL(k_grads<7>, grid1, block1, 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
     else if (c->loss == EVT_LOSS_GAUSSIAN_MLE)
-        hipLaunchKernelGGL(k_grads<2>, grid, dim3(256), 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
+        hipLaunchKernelGGL(k_grads<2>, grid1, block1, 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
     else if (c->loss == EVT_LOSS_POISSON)
-        hipLaunchKernelGGL(k_grads<3>, grid, dim3(256), 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
+        hipLaunchKernelGGL(k_grads<3>, grid1, block1, 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
     else if (c->loss == EVT_LOSS_GAMMA)
-        hipLaunchKernelGGL(k_grads<4>, grid, dim3(256), 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
+        hipLaunchKernelGGL(k_grads<4>, grid1, block1, 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
     else if (c->loss == EVT_LOSS_MAE)
-        hipLaunchKernelGGL(k_grads<8>, grid, dim3(256), 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
+        hipLaunchKernelGGL(k_grads<8>, grid1, block1, 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
     else if (EVT_IS_CRED(c->loss))
-        hipLaunchKernelGGL(k_grads<9>, grid, dim3(256), 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
+        hipLaunchKernelGGL(k_grads<9>, grid1, block1, 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
     else if (c->loss == EVT_LOSS_MLOGLOSS)
 #define ML(KM_) hipLaunchKernelGGL(k_grads_mlogloss<KM_>, grid, dim3(256), 0, c->stream, c->pred, c->y, c->grad, c->N, c->K, am, pn, c->tree.pred, c->unit_w ? 1 : 0)
         if (c->K <= 4) ML(4);
@@ -469,7 +474,7 @@ int launch_grads(evt_ctx *c) {
         else ML(16);
 #undef ML
     else
-        hipLaunchKernelGGL(k_grads<5>, grid, dim3(256), 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
+        hipLaunchKernelGGL(k_grads<5>, grid1, block1, 0, c->stream, c->pred, c->y, c->grad, c->N, am, pn, c->tree.pred, c->unit_w ? 1 : 0);
     HIPCHK(hipGetLastError());
     return EVT_OK;
 }
@@ -534,7 +539,10 @@ int launch_quantize(evt_ctx *c) {
     c->qexp = c->qexp_buf[c->q_cur];
     c->qscale = c->qscale_buf[c->q_cur];
     double *qmul = c->qscale + EVT_MC_MAX_NK; // decode scales per global channel first, then encode multipliers per gradient row
-    hipLaunchKernelGGL(k_quantize, dim3((unsigned)std::min<int64_t>(4096, (c->N + 255) / 256)), dim3(256), 0, c->stream, c->grad, c->gq, c->N, c->NK, c->NA,
+    // every block derives the multipliers first: fewer blocks where a row is one word (1M rows, at most 1024 | 4096 blocks: 5.4 | 6.5 us; four words
+    // a row at 500k rows 7.8 | 6.9, one word at 10M 27.6 | 25.5)
+    const int64_t blocks = c->NA == 1 && c->N <= (int64_t)4 << 20 ? 1024 : 4096;
+    hipLaunchKernelGGL(k_quantize, dim3((unsigned)std::min<int64_t>(blocks, (c->N + 255) / 256)), dim3(256), 0, c->stream, c->grad, c->gq, c->N, c->NK, c->NA,
                        EVT_TWO_CHAN(c->loss, c->K) ? 1 : 0, (c->unit_w && c->NA <= EVT_MAX_NA) ? 1 : 0, (c->unit_w && c->NA > EVT_MAX_NA) ? 1 : 0, absmax_set(c, c->absmax_cur), absmax_set(c, c->absmax_cur ^ 1),
                        c->qbits, c->qexp, qmul, c->qscale, c->NAg, c->loss, c->unit_w ? 1 : 0);
     HIPCHK(hipGetLastError());
