@@ -61,7 +61,7 @@ struct LevelTab {
     int32_t *bnode;    // build nodes
     int64_t *bstart;   // their segment starts
     int64_t *bprefix;  // exclusive prefix of their lengths, n_build+1 entries
-    uint4 *cdesc;      // per chunk of the level: {node, first position, end of the node's segment, first chunk of the node}
+    uint4 *cdesc;      // per chunk of the level: {node, first position, end of the node's segment, first chunk of the node}; written with the tables
 };
 
 struct TreeDev {
@@ -321,24 +321,6 @@ __device__ __forceinline__ unsigned long long evt_load_gq(const unsigned long lo
         return ((unsigned long long)q << EVT_PACK_CNT_BITS) + 1ull;
     }
     return gq[(size_t)a * N + id];
-}
-
-// Chunk descriptors of a level, for the partition kernels that run after the split search: chunk c of the level is
-// chunk c - c0 of node n, whose segment ends at `end`: {n, first position, end, c0}.  One wavefront per active node
-// writes the descriptors of that node's chunks, cprefix[i] .. cprefix[i + 1] (two dependent trips to memory, then
-// stores); `w` of `nw` wavefronts share the level's nodes.
-__device__ __forceinline__ void evt_fill_chunk_descriptors(const int64_t *__restrict__ hdr, const int32_t *__restrict__ act_node,
-                                                           const int64_t *__restrict__ cprefix, const int64_t *__restrict__ seg_start,
-                                                           const int64_t *__restrict__ seg_len, uint4 *cdesc, int chunk, int w, int nw) {
-    const int lane = threadIdx.x & 63;
-    const int n_act = (int)hdr[LH_N_ACT];
-    for (int i = w; i < n_act; i += nw) {
-        const int n = act_node[i];
-        const int64_t c0 = cprefix[i], c1 = cprefix[i + 1];
-        const int64_t seg = seg_start[n], len = seg_len[n];
-        for (int64_t c = c0 + lane; c < c1; c += 64)
-            cdesc[c] = make_uint4((uint32_t)n, (uint32_t)(seg + (c - c0) * chunk), (uint32_t)(seg + len), (uint32_t)c0);
-    }
 }
 
 __device__ __forceinline__ void evt_add_leaf(float *pr, const float *lp, int K, int loss) {

@@ -44,13 +44,7 @@ struct HistArgs {
     int seg_cost;
     int na_all; // accumulator channels of the loss: more than EVT_MAX_NA go EVT_HIST_GROUP to a block layer (blockIdx.z)
     int pack;   // the channel groups' first channel carries the row count (as a 64-bit word, k_quantize)
-    // level bookkeeping that rides along with the first launch of a level: the partition kernels' chunk descriptors
-    const int32_t *act_node;
-    const int64_t *cprefix;
-    const int64_t *seg_start;
-    const int64_t *seg_len;
-    uint4 *cdesc;
-    int chunk; // rows of a chunk of this level
+    int tab;    // entries of bprefix, bstart and bnode that may be read
 };
 
 // First node of a block's span: the largest i with bprefix[i] <= start.  bprefix ascends from 0, so that is the number
@@ -75,14 +69,47 @@ __device__ __forceinline__ int first_node_of_span(const int64_t *__restrict__ bp
     return cnt - 1;
 }
 
-// Chunk descriptors of the level (evt_fill_chunk_descriptors): they ride along with the first launch of a level, spread
-// over the wavefronts of its first block column; the work hides behind the histogram kernel's own set-up.
-__device__ __forceinline__ void fill_chunk_descriptors(const HistArgs &A) {
-    if (blockIdx.y != 0 || blockIdx.z != 0) return;
-    const int wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
-    evt_fill_chunk_descriptors(A.hdr, A.act_node, A.cprefix, A.seg_start, A.seg_len, A.cdesc, A.chunk, (int)blockIdx.x * nwaves + wave,
-                               (int)gridDim.x * nwaves);
-}
+// The level's build list in a wavefront's registers, a node to a lane: requested together with the level's header, so that a block's first
+// row ids are its second trip to memory (they were its fourth, behind the search for its first node and that node's bounds) and a
+// block that goes from node to node waits for no table.  More than 63 build nodes: read from memory.  (With the chunk descriptors moved out of
+// this kernel's start: 1M x 100 sampled by half 15.1 -> 14.0 us a level, 800k x 28 of 128 bins 19.9 -> 19.1.)
+struct BuildList {
+    int64_t prefix, start;
+    int node;
+    bool held;
+    __device__ __forceinline__ void request(const HistArgs &A) {
+        const int lane = threadIdx.x & 63, k = lane < A.tab ? lane : A.tab - 1;
+        prefix = A.bprefix[k];
+        start = A.bstart[k];
+        node = A.bnode[k];
+    }
+    static __device__ __forceinline__ int64_t lane_of(int64_t v, int i) {
+        const int lo = __builtin_amdgcn_readlane((int)(v & 0xffffffffll), i), hi = __builtin_amdgcn_readlane((int)(v >> 32), i);
+        return ((int64_t)hi << 32) | (unsigned int)lo;
+    }
+    __device__ __forceinline__ int first(const HistArgs &A, int n_build, int64_t at) {
+        held = n_build < 64;
+        if (!held) return first_node_of_span(A.bprefix, n_build, at);
+        return __popcll(__ballot((int)(threadIdx.x & 63) < n_build && prefix <= at)) - 1;
+    }
+    // node i occupies [beg, next) of the span space, its rows start at `row0` of the list
+    __device__ __forceinline__ void bounds(const HistArgs &A, int i, int64_t &beg, int64_t &next, int64_t &row0) const {
+        if (held) {
+            const int u = __builtin_amdgcn_readfirstlane(i);
+            beg = lane_of(prefix, u);
+            next = lane_of(prefix, u + 1);
+            row0 = lane_of(start, u);
+        } else {
+            beg = A.bprefix[i];
+            next = A.bprefix[i + 1];
+            row0 = A.bstart[i];
+            asm volatile("" : "+v"(row0)); // requested with the two above, not behind the branch that follows
+        }
+    }
+    __device__ __forceinline__ int id(const HistArgs &A, int i) const {
+        return held ? __builtin_amdgcn_readlane(node, __builtin_amdgcn_readfirstlane(i)) : A.bnode[i];
+    }
+};
 
 // Channel c of a block layer's group, for one row.  GRP: the layer's channels start at a0; past the last one it reads that again
 // (added to words the flush leaves out).
@@ -99,9 +126,10 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
     extern __shared__ unsigned long long H[]; // [NA][tile slots][B]
     const int tid = threadIdx.x, nthr = blockDim.x;
     const int lane = tid & 63, wave = tid >> 6, nwaves = nthr >> 6;
+    BuildList list;
+    list.request(A);
     const int n_build = (int)A.hdr[LH_N_BUILD];
     const int64_t total = A.hdr[LH_TOTAL_BUILD];
-    fill_chunk_descriptors(A);
     if (n_build <= 0 || total <= 0) return;
     const int a0 = GRP ? (int)blockIdx.z * NA : 0;
     const bool pk = GRP ? (A.pack && a0 == 0) : PACK; // channel 0 shares its word with the row count
@@ -139,15 +167,15 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
     const bool lane_on = (rloc < A.RPW) && vmask != 0;
     __syncthreads();
 
-    int i = first_node_of_span(A.bprefix, n_build, start);
+    int i = list.first(A, n_build, start);
     const int64_t blk_start = start, blk_end = end;
 
     while (start < end) {
         // spans are cut in a cost space where node i occupies [bprefix[i], bprefix[i+1]): its rows first,
         // then seg_cost units standing for the fixed cost of one flush, so that a span holding many tiny
         // nodes carries proportionally fewer rows
-        const int64_t nbeg = A.bprefix[i];
-        const int64_t nxt = A.bprefix[i + 1];
+        int64_t nbeg, nxt, bst;
+        list.bounds(A, i, nbeg, nxt, bst);
         const int64_t nrows_end = nxt - A.seg_cost;
         const int64_t cend = end < nxt ? end : nxt;
         const int64_t nend_all = cend < nrows_end ? cend : nrows_end;
@@ -158,7 +186,7 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
         }
         // the packed row counter holds 16 bits: a longer run of one node is flushed in several parts
         const int64_t nend = (pk && nend_all - start > EVT_HIST_MAX_ROWS_PER_BLOCK) ? start + EVT_HIST_MAX_ROWS_PER_BLOCK : nend_all;
-        const int64_t seg = A.bstart[i] - nbeg; // position in the row list = seg + p
+        const int64_t seg = bst - nbeg; // position in the row list = seg + p
         // software pipeline over U row groups per wave: the row ids of iteration k+2 and the records of
         // iteration k+1 are in flight while the LDS atomics of iteration k are issued
         {
@@ -233,7 +261,7 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
         // this block's span has a single writer: plain stores into its zero-initialised slice; a node
         // shared with other blocks is accumulated with 64-bit global atomics.
         const bool sole = (nbeg >= blk_start) && (nrows_end <= blk_end) && !(pk && nrows_end - nbeg > EVT_HIST_MAX_ROWS_PER_BLOCK);
-        long long *hn = A.hist + (int64_t)(A.bnode[i] - 1) * A.node_stride;
+        long long *hn = A.hist + (int64_t)(list.id(A, i) - 1) * A.node_stride;
         // blocks start at different words so that concurrent flushes of one node do not queue on the
         // same addresses
         const int nwords = NA * plane;
@@ -335,9 +363,10 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
     extern __shared__ unsigned long long H[]; // [NA][PU][B][NS]
     const int tid = threadIdx.x, nthr = blockDim.x;
     const int lane = tid & 63, wave = tid >> 6, nwaves = nthr >> 6;
+    BuildList list;
+    list.request(A);
     const int n_build = (int)A.hdr[LH_N_BUILD];
     const int64_t total = A.hdr[LH_TOTAL_BUILD];
-    fill_chunk_descriptors(A);
     if (n_build <= 0 || total <= 0) return;
     const int a0 = GRP ? (int)blockIdx.z * NA : 0;
     const bool pk = GRP ? (A.pack && a0 == 0) : PACK; // channel 0 shares its word with the row count
@@ -397,7 +426,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
     const bool lane_on = vmask != 0;
     __syncthreads();
 
-    int i = first_node_of_span(A.bprefix, n_build, start);
+    int i = list.first(A, n_build, start);
     const int64_t blk_start = start, blk_end = end;
     char *Hb = reinterpret_cast<char *>(H);
 
@@ -405,10 +434,8 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
         // spans are cut in a cost space where node i occupies [bprefix[i], bprefix[i+1]): its rows first,
         // then seg_cost units standing for the fixed cost of one flush, so that a span holding many tiny
         // nodes carries proportionally fewer rows
-        const int64_t nbeg = A.bprefix[i];
-        const int64_t nxt = A.bprefix[i + 1];
-        int64_t bst = A.bstart[i];
-        asm volatile("" : "+v"(bst)); // requested with the two above, not behind the branch below
+        int64_t nbeg, nxt, bst;
+        list.bounds(A, i, nbeg, nxt, bst);
         const int64_t nrows_end = nxt - A.seg_cost;
         const int64_t cend = end < nxt ? end : nxt;
         const int64_t nend_all = cend < nrows_end ? cend : nrows_end;
@@ -518,7 +545,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
         // (channel, t): global accesses are whole 64-byte runs of one feature's bins, LDS reads spread over the bank
         // pairs.  Blocks start at different items so that concurrent flushes of one node do not queue on the same addresses.
         const bool sole = (nbeg >= blk_start) && (nrows_end <= blk_end) && !(pk && nrows_end - nbeg > EVT_HIST_MAX_ROWS_PER_BLOCK);
-        long long *hn = A.hist + (int64_t)(A.bnode[i] - 1) * A.node_stride;
+        long long *hn = A.hist + (int64_t)(list.id(A, i) - 1) * A.node_stride;
         const int nchunks = (B + 7) >> 3;
         const int nitems = NA * PU * nchunks * NS * 8; // (channel, t, bin chunk, piece, bin in chunk), the last fastest
         const int rot = (int)(((int64_t)blockIdx.x * 1031) % (nitems >> 6)) << 6;
@@ -729,12 +756,7 @@ int launch_hist_build(evt_ctx *c, int level, const uint32_t *is_cur) {
     A.bnode = L.bnode;
     A.bstart = L.bstart;
     A.bprefix = L.bprefix;
-    A.act_node = L.act_node;
-    A.cprefix = L.cprefix;
-    A.seg_start = c->seg_start;
-    A.seg_len = c->seg_len;
-    A.cdesc = L.cdesc;
-    A.chunk = part_chunk_rows(c, level);
+    A.tab = c->maxlvl + 2;
     A.jsmap = c->jsmap;
     A.hist = c->hist;
     A.stats = c->stats;

@@ -191,6 +191,7 @@ struct NextArgs {
     int64_t *n_bprefix;
     int64_t *n_stats; // rows the next level builds (the level's slot of the per-tree counts; the histogram kernel writes the same figure when it runs)
     int64_t seg_cost; // cost units added per build node in the histogram kernel's span space
+    uint4 *n_cdesc;
     int n_chunk;      // rows of a chunk of the next level
     // one-pass form: a child's rows are its count channel, and its cursor starts from zero
     const long long *node_sum;
@@ -280,6 +281,8 @@ __device__ void level_tables_block(const NextArgs &A, long long *s_tmp /* [34] *
     const int span = (n_act + nthr - 1) / nthr;
     const int i0 = tid * span, i1 = (i0 + span < n_act) ? i0 + span : n_act;
     long long s_pos = 0, s_chunks = 0, s_brows = 0;
+    int n1 = 0; // a thread's only node, where no thread has more: what the second half needs of it stays in registers
+    int64_t nl1 = 0, nr1 = 0, start1 = 0;
     for (int i = i0; i < i1; i++) {
         const int n = A.act_node[i];
         const int64_t cp0 = A.cprefix[i], cp1 = A.cprefix[i + 1];
@@ -299,6 +302,10 @@ __device__ void level_tables_block(const NextArgs &A, long long *s_tmp /* [34] *
             A.cursor[EVT_CURSOR_SLOT(2 * n)] = 0ull;
             A.cursor[EVT_CURSOR_SLOT(2 * n + 1)] = 0ull;
         }
+        n1 = n;
+        nl1 = nl;
+        nr1 = nr;
+        start1 = start;
         s_pos += 1;
         s_chunks += (nl + A.n_chunk - 1) / A.n_chunk + (nr + A.n_chunk - 1) / A.n_chunk;
         s_brows += (build_left ? nl : nr) + A.seg_cost;
@@ -308,22 +315,48 @@ __device__ void level_tables_block(const NextArgs &A, long long *s_tmp /* [34] *
     block_excl_scan2((s_chunks << 24) | s_pos, s_brows, &p_pc, &p_brows, &t_pc, &t_brows, s_tmp);
     long long p_pos = p_pc & 0xFFFFFF, p_chunks = p_pc >> 24;
     const long long t_pos = t_pc & 0xFFFFFF, t_chunks = t_pc >> 24;
-    for (int i = i0; i < i1; i++) {
-        const int n = A.act_node[i];
-        if (A.status[n] != ST_SPLIT) continue;
-        const int64_t nl = A.seg_len[2 * n], nr = A.seg_len[2 * n + 1];
-        const int64_t start = A.seg_start[2 * n];
-        const bool build_left = nr >= nl;
-        A.n_act_node[2 * p_pos] = 2 * n;
-        A.n_act_node[2 * p_pos + 1] = 2 * n + 1;
-        A.n_cprefix[2 * p_pos] = p_chunks;
-        A.n_cprefix[2 * p_pos + 1] = p_chunks + (nl + A.n_chunk - 1) / A.n_chunk;
-        A.n_bnode[p_pos] = build_left ? 2 * n : 2 * n + 1;
-        A.n_bstart[p_pos] = build_left ? start : start + nl;
-        A.n_bprefix[p_pos] = p_brows;
-        p_pos += 1;
-        p_chunks += (nl + A.n_chunk - 1) / A.n_chunk + (nr + A.n_chunk - 1) / A.n_chunk;
-        p_brows += (build_left ? nl : nr) + A.seg_cost;
+    // the chunks' descriptors: LDS holds the children of 256 nodes at a time; a child's first few are written by its own thread, those of
+    // children with many by the thread's whole wavefront
+    __shared__ uint4 s_child[512];
+    const int lane = tid & 63;
+    int i = i0;
+    for (int base = 0; base < t_pos; base += 256) { // (positions ascend with the thread, and with i)
+        for (; i < i1 && p_pos < base + 256; i++) {
+            const bool one = span == 1;
+            const int n = one ? n1 : A.act_node[i];
+            if (one ? n1 == 0 : A.status[n] != ST_SPLIT) continue;
+            const int64_t nl = one ? nl1 : A.seg_len[2 * n], nr = one ? nr1 : A.seg_len[2 * n + 1], start = one ? start1 : A.seg_start[2 * n];
+            const bool build_left = nr >= nl;
+            const int64_t cl = (nl + A.n_chunk - 1) / A.n_chunk, cr = (nr + A.n_chunk - 1) / A.n_chunk;
+            A.n_act_node[2 * p_pos] = 2 * n;
+            A.n_act_node[2 * p_pos + 1] = 2 * n + 1;
+            A.n_cprefix[2 * p_pos] = p_chunks;
+            A.n_cprefix[2 * p_pos + 1] = p_chunks + cl;
+            A.n_bnode[p_pos] = build_left ? 2 * n : 2 * n + 1;
+            A.n_bstart[p_pos] = build_left ? start : start + nl;
+            A.n_bprefix[p_pos] = p_brows;
+            s_child[2 * (p_pos - base)] = make_uint4(2 * n, (uint32_t)start, (uint32_t)(start + nl), (uint32_t)p_chunks);
+            s_child[2 * (p_pos - base) + 1] = make_uint4(2 * n + 1, (uint32_t)(start + nl), (uint32_t)(start + nl + nr), (uint32_t)(p_chunks + cl));
+            p_pos += 1;
+            p_chunks += cl + cr;
+            p_brows += (build_left ? nl : nr) + A.seg_cost;
+        }
+        __syncthreads();
+        const int kids = t_pos - base < 256 ? 2 * (int)(t_pos - base) : 512;
+        for (int q0 = 0; q0 < kids; q0 += nthr) {
+            const int q = q0 + tid;
+            const uint4 d = q < kids ? s_child[q] : make_uint4(0, 0, 0, 0);
+            const uint32_t rows = d.z - d.y, chunk = (uint32_t)A.n_chunk;
+#pragma unroll
+            for (uint32_t c = 0; c < 4; c++)
+                if (c * chunk < rows) A.n_cdesc[d.w + c] = make_uint4(d.x, d.y + c * chunk, d.z, d.w);
+            for (unsigned long long many = __ballot(rows > 4 * chunk); many; many &= many - 1) {
+                const int l = __ffsll((long long)many) - 1;
+                const uint4 e = make_uint4(__builtin_amdgcn_readlane(d.x, l), __builtin_amdgcn_readlane(d.y, l), __builtin_amdgcn_readlane(d.z, l), __builtin_amdgcn_readlane(d.w, l));
+                for (uint32_t c = 4 + lane; (int64_t)c * chunk < (int64_t)(e.z - e.y); c += 64) A.n_cdesc[e.w + c] = make_uint4(e.x, e.y + c * chunk, e.z, e.w);
+            }
+        }
+        __syncthreads();
     }
     if (tid == 0) {
         A.n_cprefix[2 * t_pos] = t_chunks;
@@ -727,6 +760,7 @@ struct BeginArgs {
     int64_t root_words;
     int nnodes, K, D;
     int chunk; // rows of a chunk of the root
+    uint4 *cdesc;
     unsigned long long *cursor;
     // the tree's column sample and its inverse map, from the pinned staging buffer to the device copies (0 words: unchanged)
     const uint32_t *js_src, *map_src;
@@ -753,9 +787,10 @@ __device__ void tree_begin_block(BeginArgs A) {
     for (int d = tid; d <= A.D; d += nthr) A.stats[d] = 0;
     for (int i = tid; i < A.js_words; i += nthr) A.js_dst[i] = A.js_src[i];
     for (int i = tid; i < A.map_words; i += nthr) A.map_dst[i] = A.map_src[i];
+    if (A.n_is_dev) A.n_is = *A.n_is_dev;
+    for (int64_t c = tid; c * A.chunk < A.n_is; c += nthr) A.cdesc[c] = make_uint4(1, (uint32_t)(c * A.chunk), (uint32_t)A.n_is, 0);
     __syncthreads();
     if (tid == 0) {
-        if (A.n_is_dev) A.n_is = *A.n_is_dev;
         A.stats[0] = A.n_is; // read back with the tree: the host learns how many rows the mask kept
         A.status[1] = ST_BUILD;
         A.seg_start[1] = 0;
@@ -936,6 +971,7 @@ static void fill_begin_args(evt_ctx *c, bool all_rows, BeginArgs &A) {
     A.K = c->K;
     A.D = c->D;
     A.chunk = part_chunk_rows(c, 1);
+    A.cdesc = L.cdesc;
     A.cursor = c->cursor;
     A.js_words = A.map_words = 0;
     A.js_src = A.map_src = nullptr;
@@ -1069,6 +1105,7 @@ static void fill_next_args(evt_ctx *c, int level, NextArgs &A) {
     A.n_bnode = Nx.bnode;
     A.n_bstart = Nx.bstart;
     A.n_bprefix = Nx.bprefix;
+    A.n_cdesc = Nx.cdesc;
     A.n_stats = (level + 1 <= c->D) ? c->stats + level + 1 : nullptr;
     A.seg_cost = c->hist_seg_cost;
     A.n_chunk = part_chunk_rows(c, level + 1);
@@ -1141,8 +1178,7 @@ int launch_part_scatter(evt_ctx *c, int level, const uint32_t *is_cur, uint32_t 
 }
 
 // The scatter pass can build the next level's histograms: 16-byte records, one launch's worth of channels in at most
-// 32 KB of LDS, a split search that writes the chunk descriptors the histogram kernel otherwise leaves behind (one block
-// per node: k_scan's fused form) and at most 128 chunks per level (a quarter of a million rows), where a level is a chain of
+// 32 KB of LDS, the split search of one block per node (k_scan's fused form) and at most 128 chunks per level (a quarter of a million rows), where a level is a chain of
 // kernels of a few microseconds each and one of them less is worth more than the histogram kernel's better use of the
 // machine: at 100k rows x 10 features the pass takes 12 us against 5 + 10 us for the two kernels, at 1M rows 22 against 6 + 12.
 bool scatter_can_build_hist(const evt_ctx *c, int nfs) {
