@@ -17,7 +17,7 @@ int launch_predict_model(hipStream_t s, const uint32_t *nodes, const float *leaf
                          int K, int loss, int apply_link, float *out, const int32_t *skip_flag);
 int predict_lds_shape(int F, int max_int, int K, int hint);
 int launch_predict_model_lds(hipStream_t s, const uint32_t *cnodes, const float *cleaf, const void *meta, int ntrees, const uint8_t *xcm, int64_t N,
-                             int F, int max_int, int K, int loss, int apply_link, int all_numeric, int shape, float *out);
+                             int F, int max_int, int K, int ks, int loss, int apply_link, int all_numeric, int shape, float *out);
 int launch_leaf_idx_model(hipStream_t s, const uint32_t *nodes, const int64_t *off, int ntrees, const uint8_t *xcm, int64_t N, uint32_t *out);
 
 static thread_local char g_err[512] = "";
@@ -1616,7 +1616,7 @@ static int predict_common(int64_t nobs, int32_t nfeats, const uint8_t *x_bin, co
     }
     if (e == hipSuccess && r == EVT_OK) {
         if (leaf_out) r = launch_leaf_idx_model(s, d_nodes, d_off, ntrees, d_x, nobs, d_leaf);
-        else if (use_lds) r = launch_predict_model_lds(s, d_cn, d_cl, d_cm, ntrees, d_x, nobs, nfeats, max_int, K, loss, apply_link, all_numeric ? 1 : 0, shape, d_out);
+        else if (use_lds) r = launch_predict_model_lds(s, d_cn, d_cl, d_cm, ntrees, d_x, nobs, nfeats, max_int, K, K, loss, apply_link, all_numeric ? 1 : 0, shape, d_out);
         else r = launch_predict_model(s, d_nodes, d_lp, d_off, ntrees, d_x, nobs, K, loss, apply_link, d_out, nullptr);
         e = hipDeviceSynchronize();
     }

@@ -220,7 +220,7 @@ __device__ __forceinline__ uint32_t step_node(uint32_t nid, uint32_t nd, uint32_
 
 struct ModelTree {
     int32_t node_off; // first internal node in the node array
-    int32_t leaf_off; // first last-level value (K floats each) in the value array
+    int32_t leaf_off; // first last-level leaf in the value array
     int32_t levels;   // depth - 1: levels walked
     int32_t n_int;    // internal nodes: 2^levels - 1
 };
@@ -230,7 +230,7 @@ struct ModelTree {
 template <int KMAX, int RB, int NT, int PRE, bool ALLNUM>
 __global__ __launch_bounds__(RB) void k_predict_model_lds(const uint32_t *__restrict__ cnodes, const float *__restrict__ cleaf,
                                                          const ModelTree *__restrict__ meta, int ntrees, const uint8_t *__restrict__ xcm,
-                                                         int64_t N, int F, int S4, int max_int, int K, int loss, int link, float *out) {
+                                                         int64_t N, int F, int S4, int max_int, int K, int ks, int loss, int link, float *out) {
     extern __shared__ uint32_t smem[];
     uint32_t *T = smem;                                                        // [2][NT][max_int]
     uint8_t *R = reinterpret_cast<uint8_t *>(smem + 2 * (size_t)NT * max_int); // [RB / 64][S4][64] words
@@ -322,8 +322,8 @@ __global__ __launch_bounds__(RB) void k_predict_model_lds(const uint32_t *__rest
         nprev = ntrees - g * NT < NT ? ntrees - g * NT : NT;
 #pragma unroll
         for (int j = 0; j < NT; j++) {
-            const float *lp = cleaf + (size_t)K * (m[j].leaf_off + pos[j]);
-            if (KMAX > 4 && (K & 3) == 0) { // rows of 4 values: 16-byte loads (the value array starts on an allocation boundary)
+            const float *lp = cleaf + (size_t)ks * (m[j].leaf_off + pos[j]);
+            if (KMAX > 4 && (ks & 3) == 0) { // rows of 4 values: 16-byte loads (the value array starts on an allocation boundary)
 #pragma unroll
                 for (int k = 0; k < KMAX; k += 4) {
                     if (k < K) {
@@ -366,7 +366,7 @@ __global__ __launch_bounds__(256) void k_leaf_idx_model(const uint32_t *__restri
 
 template <int KMAX, int RB, int NT, int PRE, bool ALLNUM>
 static int launch_model_lds(hipStream_t s, const uint32_t *cnodes, const float *cleaf, const void *meta, int ntrees, const uint8_t *xcm, int64_t N,
-                            int F, int max_int, int K, int loss, int apply_link, float *out) {
+                            int F, int max_int, int K, int ks, int loss, int apply_link, float *out) {
     static EvtDevOnce once;
     const int dev = EvtDevOnce::current();
     if (once.pending(dev)) {
@@ -377,7 +377,7 @@ static int launch_model_lds(hipStream_t s, const uint32_t *cnodes, const float *
     const int S4 = (F + 3) >> 2;
     const size_t lds = (size_t)RB * S4 * 4 + 8 * (size_t)NT * max_int;
     hipLaunchKernelGGL((k_predict_model_lds<KMAX, RB, NT, PRE, ALLNUM>), dim3((unsigned)((N + RB - 1) / RB)), dim3(RB), lds, s, cnodes, cleaf,
-                       static_cast<const ModelTree *>(meta), ntrees, xcm, N, F, S4, max_int, K, loss, apply_link, out);
+                       static_cast<const ModelTree *>(meta), ntrees, xcm, N, F, S4, max_int, K, ks, loss, apply_link, out);
     HIPCHK(hipGetLastError());
     return EVT_OK;
 }
@@ -398,14 +398,14 @@ int predict_lds_shape(int F, int max_int, int K, int hint) {
     return 0;
 }
 
-// Completed trees (see k_predict_model_lds): cnodes / cleaf / meta as the host prepared them.
+// Completed trees (see k_predict_model_lds): cnodes / cleaf / meta as the host prepared them; a leaf's K values lie ks apart.
 int launch_predict_model_lds(hipStream_t s, const uint32_t *cnodes, const float *cleaf, const void *meta, int ntrees, const uint8_t *xcm, int64_t N,
-                             int F, int max_int, int K, int loss, int apply_link, int all_numeric, int shape, float *out) {
+                             int F, int max_int, int K, int ks, int loss, int apply_link, int all_numeric, int shape, float *out) {
     const int mi = max_int > 0 ? max_int : 1;
     shape = predict_lds_shape(F, max_int, K, shape);
 #define EVT_PM(KM_, RB_, NT_, PRE_)                                                                                                          \
-    return all_numeric ? launch_model_lds<KM_, RB_, NT_, PRE_, true>(s, cnodes, cleaf, meta, ntrees, xcm, N, F, mi, K, loss, apply_link, out) \
-                       : launch_model_lds<KM_, RB_, NT_, PRE_, false>(s, cnodes, cleaf, meta, ntrees, xcm, N, F, mi, K, loss, apply_link, out)
+    return all_numeric ? launch_model_lds<KM_, RB_, NT_, PRE_, true>(s, cnodes, cleaf, meta, ntrees, xcm, N, F, mi, K, ks, loss, apply_link, out) \
+                       : launch_model_lds<KM_, RB_, NT_, PRE_, false>(s, cnodes, cleaf, meta, ntrees, xcm, N, F, mi, K, ks, loss, apply_link, out)
     if (K <= 4) {
         if (shape == 1) { EVT_PM(4, 1024, 4, 8); }
         if (shape == 2) { EVT_PM(4, 512, 2, 8); }
@@ -464,6 +464,7 @@ __device__ __forceinline__ void add_run(float *acc, const float *v, int step, in
         add(acc, lp);
     }
 }
+// one or two outputs of a row, by one lane
 template <int KMAX>
 __device__ __forceinline__ void add_trees(float *acc, const float *v, int step, int n, int K, int loss) {
     if (loss == EVT_LOSS_LOGLOSS) {
@@ -495,14 +496,69 @@ __device__ __forceinline__ void add_trees(float *acc, const float *v, int step, 
     }
 }
 
+// The largest of the values of KMAX neighbouring lanes (4, 8 or 16 of a DPP row), in all of them.  Written out, since as a move and a maximum of
+// its own each step costs three dependent instructions; a DPP read waits two states for the write before it.
+#define EVT_MAX_DPP(CTRL_) asm("s_nop 1\n\tv_max_f32_dpp %0, %1, %1 " CTRL_ " row_mask:0xf bank_mask:0xf" : "=v"(x) : "v"(x))
+template <int KMAX>
+__device__ __forceinline__ float group_max(float x) {
+    EVT_MAX_DPP("quad_perm:[1,0,3,2]"); // the neighbour
+    EVT_MAX_DPP("quad_perm:[2,3,0,1]"); // the other pair of the quad
+    if (KMAX >= 8) EVT_MAX_DPP("row_half_mirror"); // the other quad of eight
+    if (KMAX >= 16) EVT_MAX_DPP("row_mirror");     // the other eight
+    return x;
+}
+#undef EVT_MAX_DPP
+// More outputs: a lane adds one output of one row (the row's outputs side by side), P rows at a time, with the clamps of add_trees; the
+// lanes of a row meet where classes are shifted by their maximum.
+template <int P, typename ADD>
+__device__ __forceinline__ void add_run_lane(float *acc, const float *v, int step, int per, int n, ADD add) {
+    constexpr int U = 8 / P > 0 ? 8 / P : 1; // trees read ahead of their use
+    int t = 0;
+    for (; t + U <= n; t += U) {
+        float lp[U][P];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int p = 0; p < P; p++) lp[u][p] = v[(t + u) * step + p * per];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int p = 0; p < P; p++) acc[p] = add(acc[p] + lp[u][p]);
+    }
+    for (; t < n; t++)
+#pragma unroll
+        for (int p = 0; p < P; p++) acc[p] = add(acc[p] + v[t * step + p * per]);
+}
+// k: the lane's output; lanes past the last one stay at minus infinity where classes are shifted, and are not written out
+template <int KMAX, int P>
+__device__ __forceinline__ void add_trees_lane(float *acc, const float *v, int step, int per, int n, int k, int K, int loss, bool first) {
+    if (loss == EVT_LOSS_MLOGLOSS) {
+        const float least = k < K ? -15.0f : -INFINITY;
+        if (first && k >= K)
+#pragma unroll
+            for (int p = 0; p < P; p++) acc[p] = -INFINITY;
+        add_run_lane<P>(acc, v, step, per, n, [least](float a) { return fmaxf(least, a - group_max<KMAX>(a)); });
+    } else if (loss == EVT_LOSS_LOGLOSS) {
+        add_run_lane<P>(acc, v, step, per, n, [](float a) { return fminf(fmaxf(a, -15.0f), 15.0f); });
+    } else if (EVT_IS_MLE2P(loss)) {
+        add_run_lane<P>(acc, v, step, per, n, [k](float a) { return (k & 1) ? fmaxf(-15.0f, a) : a; });
+    } else {
+        add_run_lane<P>(acc, v, step, per, n, [](float a) { return a; });
+    }
+}
+
 // Few rows, many trees: a block takes R rows and spreads the trees over its 256 / R lanes per row, so that a handful of rows still
 // occupies whole wavefronts (and a few thousand rows the chip), where a row per lane leaves a single chain of dependent reads.  A lane
 // walks WALK_U trees side by side over the completed trees (fixed depth, nodes from the caches: a model of 200 trees of
 // depth 8 is 100 KB); the leaf values of a run of trees meet in LDS, and one lane per row adds them in tree order,
-// so the sum has the bits of the sequential one.  The bins may lie in pinned host memory, and so may the output.
+// so the sum has the bits of the sequential one - or, of more than two outputs, a lane per row and output: one lane went through all outputs of
+// a row while most of its block waited (16 700 rows, 100 trees, 7 classes: 50.8 -> 33.5 us, one row 27.0 -> 11.1).  The bins may lie in pinned host memory, and so may the output.
 // With a single row per block the nodes are first touched all at once: one trip to memory instead of one per level.
 // LEAF: the leaf's node id of every row and tree instead, tree by tree, in LB-byte words.
+// A leaf's values lie KMAX apart, those past the last output zero, and move in pieces of up to 16 bytes (word by word a tree's values were more
+// requests than its walk).
 #define WALK_U 4
+int walk_leaf_stride(int K) { return K <= 2 ? K : K <= 4 ? 4 : K <= 8 ? 8 : EVT_MAX_K; }
 template <int KMAX, int R, bool LEAF, int LB>
 __global__ __launch_bounds__(256) void k_walk_rows(const uint32_t *__restrict__ cnodes, int stride, const ModelTree *__restrict__ meta,
                                                   const float *__restrict__ cleaf, const uint32_t *__restrict__ cid, int ntrees, int run,
@@ -525,9 +581,11 @@ __global__ __launch_bounds__(256) void k_walk_rows(const uint32_t *__restrict__ 
         s_x[k] = x[(size_t)(k / R) * ldx + (i < n ? i : n - 1)];
     }
     __syncthreads();
-    float acc[KMAX];
+    constexpr bool WIDE = KMAX > 2; // a lane per row and output
+    constexpr int L = R * KMAX < 256 ? R * KMAX : 256, P = R * KMAX / L; // lanes that add, and what each of them adds
+    float acc[WIDE ? P : KMAX];
 #pragma unroll
-    for (int k = 0; k < KMAX; k++) acc[k] = 0.0f;
+    for (int k = 0; k < (WIDE ? P : KMAX); k++) acc[k] = 0.0f;
     for (int t0 = 0; t0 < ntrees; t0 += run) {
         const int t1 = t0 + run < ntrees ? t0 + run : ntrees;
         for (int tb = t0 + g; tb < t1; tb += G * WALK_U) {
@@ -572,24 +630,60 @@ __global__ __launch_bounds__(256) void k_walk_rows(const uint32_t *__restrict__ 
                     }
                 }
             } else {
-                float lv[WALK_U][KMAX];
+                alignas(16) float lv[WALK_U][KMAX];
+                if constexpr (WIDE) {
 #pragma unroll
-                for (int u = 0; u < WALK_U; u++)
+                    for (int u = 0; u < WALK_U; u++)
 #pragma unroll
-                    for (int k = 0; k < KMAX; k++) lv[u][k] = cleaf[(size_t)at[u] * K + (k < K ? k : 0)];
+                        for (int k = 0; k < KMAX; k += 4) *reinterpret_cast<float4 *>(&lv[u][k]) = *reinterpret_cast<const float4 *>(cleaf + (size_t)at[u] * KMAX + k);
 #pragma unroll
-                for (int u = 0; u < WALK_U; u++)
-                    if (tb + u * G < t1)
+                    for (int u = 0; u < WALK_U; u++)
+                        if (tb + u * G < t1)
 #pragma unroll
-                        for (int k = 0; k < KMAX; k++) s_v[((size_t)(tb + u * G - t0) * R + r) * KMAX + k] = lv[u][k];
+                            for (int k = 0; k < KMAX; k += 4)
+                                *reinterpret_cast<float4 *>(&s_v[((size_t)(tb + u * G - t0) * R + r) * KMAX + k]) = *reinterpret_cast<const float4 *>(&lv[u][k]);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < WALK_U; u++)
+#pragma unroll
+                        for (int k = 0; k < KMAX; k++) lv[u][k] = cleaf[(size_t)at[u] * K + (k < K ? k : 0)];
+#pragma unroll
+                    for (int u = 0; u < WALK_U; u++)
+                        if (tb + u * G < t1)
+#pragma unroll
+                            for (int k = 0; k < KMAX; k++) s_v[((size_t)(tb + u * G - t0) * R + r) * KMAX + k] = lv[u][k];
+                }
             }
         }
         if (LEAF) continue;
         __syncthreads();
-        if (tid < R) add_trees<KMAX>(acc, s_v + tid * KMAX, R * KMAX, t1 - t0, K, loss);
+        if constexpr (WIDE) {
+            if (tid < L) add_trees_lane<KMAX, P>(acc, s_v + tid, R * KMAX, L, t1 - t0, tid % KMAX, K, loss, t0 == 0);
+        } else {
+            if (tid < R) add_trees<KMAX>(acc, s_v + tid * KMAX, R * KMAX, t1 - t0, K, loss);
+        }
         __syncthreads();
     }
-    if (!LEAF && tid < R && i0 + tid < n) {
+    if constexpr (WIDE && !LEAF) { // the row's outputs meet in one lane, for the link
+        if (tid < L)
+#pragma unroll
+            for (int p = 0; p < P; p++) s_v[tid + p * L] = acc[p];
+        __syncthreads();
+        if (link) {
+            if (tid < R) {
+                float o[KMAX];
+#pragma unroll
+                for (int k = 0; k < KMAX; k++) o[k] = s_v[tid * KMAX + k];
+                apply_link<KMAX>(o, K, loss);
+#pragma unroll
+                for (int k = 0; k < KMAX; k++) s_v[tid * KMAX + k] = o[k];
+            }
+            __syncthreads();
+        }
+        // over the bus in whole runs
+        const int rows = n - i0 < R ? (int)(n - i0) : R;
+        for (int e = tid; e < rows * K; e += 256) out[(size_t)K * i0 + e] = s_v[e / K * KMAX + e % K];
+    } else if (!LEAF && tid < R && i0 + tid < n) {
         if (link) apply_link<KMAX>(acc, K, loss);
 #pragma unroll
         for (int k = 0; k < KMAX; k++)
@@ -621,10 +715,10 @@ int launch_walk_rows(hipStream_t s, const uint32_t *cnodes, int stride, const vo
                      int64_t leaf_ld) {
     // rows per block: as few as fill the chip (1024 blocks of four wavefronts, eight of which share a compute unit), and no more than
     // 64 KB of bins
-    // (leaf ids go out R to a line: from 4096 rows on whole 64-byte ones).  Whole calls on bins beside set values of R, 100 and 200 trees of depth 6 and 8:
-    // values of one output within 10 % of the best from 1 to 131 000 rows; of seven outputs R = 16 is up to 1.34 times faster from 1000 rows on,
-    // and leaf ids between 64 rows and 16 000 take 1.2 to 4.7 times what R = 16 would
-    int R = n <= 1024 ? 1 : (n <= (leaf_out ? 4096 : 8192) ? 4 : (n <= 32768 && !leaf_out ? 16 : 64));
+    // (leaf ids go out R to a line, tree after tree: more rows a block for the same number of rows).  Whole calls on bins beside set values of R, 60 to
+    // 200 trees of depth 6 to 8, one to twelve outputs, 1 to 200 000 rows: within 12 % of the best, mostly within 5.
+    int R = n <= 1024 ? 1 : n <= 8192 ? 4 : n <= 32768 ? 16 : 64;
+    if (leaf_out) R = n <= 4 ? 1 : n <= 192 ? 4 : n <= 3072 ? 16 : 64; // us, 1 | 4 | 16 | 64 rows a block: 1024 rows 184 | 73 | 59 | 65, 4096 rows 622 | 185 | 113 | 119
     while (R > 1 && (size_t)R * F > 65536) R /= 4;
 #define EVT_WALK(KM_, LEAF_, LB_)                                                                                                                    \
     switch (R) {                                                                                                                                     \

@@ -13,7 +13,8 @@
 
 int predict_lds_shape(int F, int max_int, int K, int hint);
 int launch_predict_model_lds(hipStream_t s, const uint32_t *cnodes, const float *cleaf, const void *meta, int ntrees, const uint8_t *xcm, int64_t N,
-                             int F, int max_int, int K, int loss, int apply_link, int all_numeric, int shape, float *out);
+                             int F, int max_int, int K, int ks, int loss, int apply_link, int all_numeric, int shape, float *out);
+int walk_leaf_stride(int K);
 int launch_walk_rows(hipStream_t s, const uint32_t *cnodes, int stride, const void *meta, const float *cleaf, const uint32_t *cid, int ntrees,
                      const uint8_t *x, int64_t ldx, int64_t n, int F, int wide, int K, int loss, int apply_link, float *out, void *leaf_out, int leaf_bytes,
                      int64_t leaf_ld);
@@ -163,7 +164,7 @@ bool same_trees(const Model &m, const TreePtrs &t) { // of trees of the same sha
 // Copies the caller's arrays, checks them by the rules of evt_predict, completes the trees and uploads them.
 int build(Model &m, const TreePtrs &t, const uint8_t *feattypes, int nft, hipStream_t s) {
     m.built = false;
-    size_t total = 0;
+    size_t total = 0, leaves = 0;
     int levels_max = 0;
     for (int i = 0; i < t.n; i++) {
         ARGCHK(t.nn[i] >= 1 && t.nn[i] <= ((int64_t)1 << 20) - 1, "a kept model takes trees of up to 2^20 - 1 nodes");
@@ -171,6 +172,7 @@ int build(Model &m, const TreePtrs &t, const uint8_t *feattypes, int nft, hipStr
         int d = 0;
         while (((int64_t)1 << d) - 1 < t.nn[i]) d++;
         levels_max = std::max(levels_max, d - 1);
+        leaves += (size_t)1 << (d - 1);
     }
     const int npad = (t.n + 3) / 4 * 4;
     m.max_int = (1 << levels_max) - 1;
@@ -203,8 +205,11 @@ int build(Model &m, const TreePtrs &t, const uint8_t *feattypes, int nft, hipStr
     m.wide = m.max_feat > 1024;
     m.all_numeric = true;
     m.ntrees = t.n;
-    std::vector<uint32_t> nodes((size_t)npad * stride, 0u), cid;
-    std::vector<float> leaf;
+    const int ks = walk_leaf_stride(m.K);
+    ARGCHK(leaves * m.K < ((size_t)1 << 31), "the leaves of a kept model exceed 2^31 values");
+    std::vector<uint32_t> nodes((size_t)npad * stride, 0u), cid(leaves);
+    std::vector<float> leaf(leaves * ks, 0.0f); // (one by one they took a tenth of a small model's first call)
+    leaves = 0;
     m.meta.assign(npad, CompletedTree{0, 0, 0, 0});
     std::vector<int32_t> src; // 0: a split node of the tree; otherwise the leaf whose value the node carries
     const uint32_t always_left = (255u << 16) | EVT_NODE_NUMERIC; // feature 1, bin <= 255
@@ -214,7 +219,7 @@ int build(Model &m, const TreePtrs &t, const uint8_t *feattypes, int nft, hipStr
         int d = 0;
         while ((1 << d) - 1 < n) d++;
         const int full = (1 << d) - 1, n_int = full / 2, n_leaf = n_int + 1;
-        m.meta[i] = {(int32_t)((size_t)i * stride), (int32_t)(leaf.size() / m.K), d - 1, n_int};
+        m.meta[i] = {(int32_t)((size_t)i * stride), (int32_t)leaves, d - 1, n_int};
         src.assign(full + 1, 0);
         for (int k = 1; k <= full; k++) {
             const int32_t up = k == 1 ? 0 : src[k >> 1];
@@ -231,14 +236,13 @@ int build(Model &m, const TreePtrs &t, const uint8_t *feattypes, int nft, hipStr
             }
             cn[k - 1] = w;
         }
-        for (int q = 0; q < n_leaf; q++) {
+        for (int q = 0; q < n_leaf; q++, leaves++) {
             const int32_t at = src[n_int + 1 + q];
-            cid.push_back((uint32_t)at);
-            for (int k = 0; k < m.K; k++) leaf.push_back(m.pred[m.K * (o + at - 1) + k]);
+            cid[leaves] = (uint32_t)at;
+            for (int k = 0; k < m.K; k++) leaf[leaves * ks + k] = m.pred[m.K * (o + at - 1) + k];
         }
         o += (size_t)n;
     }
-    ARGCHK(leaf.size() < ((size_t)1 << 31), "the leaves of a kept model exceed 2^31 values");
     // one block on the device, one copy: meta | nodes | leaf ids | leaf values, each from a 256-byte boundary on
     auto up = [](size_t n) { return (n + 255) / 256 * 256; };
     const size_t o_nodes = up(sizeof(CompletedTree) * m.meta.size()), o_cid = o_nodes + up(4 * nodes.size()), o_leaf = o_cid + up(4 * cid.size());
@@ -294,8 +298,8 @@ int walk(Model &m, hipStream_t s, const Request &q, const uint8_t *x, int64_t n,
                                 leaf_bytes, n);
     const int shape = n >= WALK_LDS_MIN_ROWS ? predict_lds_shape(q.F, m.max_int, m.K, 0) : 0;
     if (shape > 0)
-        return launch_predict_model_lds(s, m.d_nodes, m.d_leaf, m.d_meta, q.ntrees, x, n, q.F, m.max_int, m.K, m.loss, q.link, m.all_numeric ? 1 : 0, shape,
-                                        static_cast<float *>(out));
+        return launch_predict_model_lds(s, m.d_nodes, m.d_leaf, m.d_meta, q.ntrees, x, n, q.F, m.max_int, m.K, walk_leaf_stride(m.K), m.loss, q.link,
+                                        m.all_numeric ? 1 : 0, shape, static_cast<float *>(out));
     return launch_walk_rows(s, m.d_nodes, std::max(1, m.max_int), m.d_meta, m.d_leaf, m.d_cid, q.ntrees, x, n, n, q.F, m.wide, m.K, m.loss, q.link,
                             static_cast<float *>(out), nullptr, 0, 0);
 }
