@@ -192,7 +192,7 @@ struct NextArgs {
     int64_t *n_stats; // rows the next level builds (the level's slot of the per-tree counts; the histogram kernel writes the same figure when it runs)
     int64_t seg_cost; // cost units added per build node in the histogram kernel's span space
     uint4 *n_cdesc;
-    int n_chunk;      // rows of a chunk of the next level
+    int n_chunk_sh;   // rows of a chunk of the next level, a power of two (64-bit divisions by a number of it took 1 us of the chain)
     // one-pass form: a child's rows are its count channel, and its cursor starts from zero
     const long long *node_sum;
     int NAg;
@@ -245,7 +245,7 @@ __device__ void chunk_scan_block(const NextArgs &A, long long *s_tmp /* [34] */)
     long long total;
     {
         constexpr int SP = 8;
-        const int64_t span = (n_chunks + nthr - 1) / nthr;
+        const int64_t span = (n_chunks + nthr - 1) >> __builtin_ctz(nthr);
         const int64_t c0 = (int64_t)tid * span, c1 = (c0 + span < n_chunks) ? c0 + span : n_chunks;
         if (span <= SP) {
             int v[SP];
@@ -275,21 +275,77 @@ __device__ void chunk_scan_block(const NextArgs &A, long long *s_tmp /* [34] */)
 }
 
 // B: children segments + three scans over the active nodes (children count, chunks, build rows) -> the next level's tables
-__device__ void level_tables_block(const NextArgs &A, long long *s_tmp /* [34] */) {
+// SCAN: half A as well.  Of up to LEVEL_LPRE chunks its sums stay in LDS, and the nodes are read while they are added up: both halves one after
+// the other were three more trips to memory, 2 us of a scatter kernel of 7 (500k rows, 64 nodes).
+#define LEVEL_LPRE 1024
+struct NextNode {
+    int n, st;
+    int64_t cp0, cp1, len, start;
+};
+template <bool SCAN>
+__device__ void level_tables_block(const NextArgs &A, long long *s_tmp /* [34] */, uint4 *s_child /* [512] */, int *s_lpre /* SCAN: [LEVEL_LPRE + 1] */) {
     const int tid = threadIdx.x, nthr = blockDim.x;
     const int n_act = (int)A.hdr[LH_N_ACT];
-    const int span = (n_act + nthr - 1) / nthr;
+    const int64_t n_chunks = SCAN ? A.hdr[LH_N_CHUNKS] : 0;
+    const int span = (n_act + nthr - 1) >> __builtin_ctz(nthr); // threads of a block: a power of two
+    const int64_t whole = ((int64_t)1 << A.n_chunk_sh) - 1;
     const int i0 = tid * span, i1 = (i0 + span < n_act) ? i0 + span : n_act;
     long long s_pos = 0, s_chunks = 0, s_brows = 0;
     int n1 = 0; // a thread's only node, where no thread has more: what the second half needs of it stays in registers
     int64_t nl1 = 0, nr1 = 0, start1 = 0;
+    NextNode first = {0, 0, 0, 0, 0, 0};
+    if (i0 < i1) {
+        first.n = A.act_node[i0];
+        first.cp0 = A.cprefix[i0];
+        first.cp1 = A.cprefix[i0 + 1];
+    }
+    const bool near = SCAN && n_chunks <= LEVEL_LPRE;
+    if constexpr (SCAN) {
+        if (near) {
+            constexpr int SP = LEVEL_LPRE / 256;
+            const int sp = ((int)n_chunks + nthr - 1) >> __builtin_ctz(nthr), c0 = tid * sp, c1 = min(c0 + sp, (int)n_chunks);
+            int v[SP], sum = 0;
+#pragma unroll
+            for (int k = 0; k < SP; k++) v[k] = A.chunk_nleft[c0 + k < c1 ? c0 + k : 0];
+            if (i0 < i1) {
+                first.st = A.status[first.n];
+                first.len = A.seg_len[first.n];
+                first.start = A.seg_start[first.n];
+            }
+#pragma unroll
+            for (int k = 0; k < SP; k++) sum += v[k] = c0 + k < c1 ? v[k] : 0;
+            long long total;
+            int pre = (int)block_excl_scan(sum, &total, s_tmp);
+#pragma unroll
+            for (int k = 0; k < SP; k++) {
+                if (c0 + k < c1) s_lpre[c0 + k] = pre;
+                pre += v[k];
+            }
+            if (tid == 0) s_lpre[n_chunks] = (int)total;
+        } else {
+            chunk_scan_block(A, s_tmp);
+        }
+        __syncthreads();
+    }
+    if (!near && i0 < i1) {
+        first.st = A.status[first.n];
+        first.len = A.seg_len[first.n];
+        first.start = A.seg_start[first.n];
+    }
     for (int i = i0; i < i1; i++) {
-        const int n = A.act_node[i];
-        const int64_t cp0 = A.cprefix[i], cp1 = A.cprefix[i + 1];
-        const int st = A.status[n];
-        const int64_t len = A.seg_len[n], start = A.seg_start[n];
-        const int64_t nl = A.node_sum ? A.node_sum[(int64_t)(2 * n) * A.NAg + A.NAg - 1] : A.chunk_lpre[cp1] - A.chunk_lpre[cp0];
-        if (st != ST_SPLIT) continue;
+        NextNode q = first;
+        if (i > i0) {
+            q.n = A.act_node[i];
+            q.cp0 = A.cprefix[i];
+            q.cp1 = A.cprefix[i + 1];
+            q.st = A.status[q.n];
+            q.len = A.seg_len[q.n];
+            q.start = A.seg_start[q.n];
+        }
+        const int n = q.n;
+        const int64_t len = q.len, start = q.start;
+        const int64_t nl = A.node_sum ? A.node_sum[(int64_t)(2 * n) * A.NAg + A.NAg - 1] : near ? s_lpre[q.cp1] - s_lpre[q.cp0] : A.chunk_lpre[q.cp1] - A.chunk_lpre[q.cp0];
+        if (q.st != ST_SPLIT) continue;
         const int64_t nr = len - nl;
         A.seg_start[2 * n] = start;
         A.seg_len[2 * n] = nl;
@@ -307,7 +363,7 @@ __device__ void level_tables_block(const NextArgs &A, long long *s_tmp /* [34] *
         nr1 = nr;
         start1 = start;
         s_pos += 1;
-        s_chunks += (nl + A.n_chunk - 1) / A.n_chunk + (nr + A.n_chunk - 1) / A.n_chunk;
+        s_chunks += ((nl + whole) >> A.n_chunk_sh) + ((nr + whole) >> A.n_chunk_sh);
         s_brows += (build_left ? nl : nr) + A.seg_cost;
     }
     // children count (low 24 bits) and chunk count share one scan; the build rows take the other
@@ -315,9 +371,8 @@ __device__ void level_tables_block(const NextArgs &A, long long *s_tmp /* [34] *
     block_excl_scan2((s_chunks << 24) | s_pos, s_brows, &p_pc, &p_brows, &t_pc, &t_brows, s_tmp);
     long long p_pos = p_pc & 0xFFFFFF, p_chunks = p_pc >> 24;
     const long long t_pos = t_pc & 0xFFFFFF, t_chunks = t_pc >> 24;
-    // the chunks' descriptors: LDS holds the children of 256 nodes at a time; a child's first few are written by its own thread, those of
-    // children with many by the thread's whole wavefront
-    __shared__ uint4 s_child[512];
+    // the chunks' descriptors: LDS holds the children of 256 nodes at a time, which share the block's lanes; what a child has beyond
+    // eight of each of its lanes is written by a whole wavefront (a wavefront for every child of more than four took 1.5 us at 32 children)
     const int lane = tid & 63;
     int i = i0;
     for (int base = 0; base < t_pos; base += 256) { // (positions ascend with the thread, and with i)
@@ -327,7 +382,7 @@ __device__ void level_tables_block(const NextArgs &A, long long *s_tmp /* [34] *
             if (one ? n1 == 0 : A.status[n] != ST_SPLIT) continue;
             const int64_t nl = one ? nl1 : A.seg_len[2 * n], nr = one ? nr1 : A.seg_len[2 * n + 1], start = one ? start1 : A.seg_start[2 * n];
             const bool build_left = nr >= nl;
-            const int64_t cl = (nl + A.n_chunk - 1) / A.n_chunk, cr = (nr + A.n_chunk - 1) / A.n_chunk;
+            const int64_t cl = (nl + whole) >> A.n_chunk_sh, cr = (nr + whole) >> A.n_chunk_sh;
             A.n_act_node[2 * p_pos] = 2 * n;
             A.n_act_node[2 * p_pos + 1] = 2 * n + 1;
             A.n_cprefix[2 * p_pos] = p_chunks;
@@ -343,17 +398,18 @@ __device__ void level_tables_block(const NextArgs &A, long long *s_tmp /* [34] *
         }
         __syncthreads();
         const int kids = t_pos - base < 256 ? 2 * (int)(t_pos - base) : 512;
-        for (int q0 = 0; q0 < kids; q0 += nthr) {
-            const int q = q0 + tid;
+        const uint32_t chunk = 1u << A.n_chunk_sh;
+        const int gs = kids < nthr ? __clz(kids - 1) - __clz(nthr - 1) : 0, g = 1 << gs, sub = tid & (g - 1); // g lanes to a child
+        for (int q0 = 0; q0 < kids; q0 += nthr >> gs) {
+            const int q = q0 + (tid >> gs);
             const uint4 d = q < kids ? s_child[q] : make_uint4(0, 0, 0, 0);
-            const uint32_t rows = d.z - d.y, chunk = (uint32_t)A.n_chunk;
-#pragma unroll
-            for (uint32_t c = 0; c < 4; c++)
-                if (c * chunk < rows) A.n_cdesc[d.w + c] = make_uint4(d.x, d.y + c * chunk, d.z, d.w);
-            for (unsigned long long many = __ballot(rows > 4 * chunk); many; many &= many - 1) {
+            const uint32_t chunks = (uint32_t)((d.z - d.y + (uint64_t)chunk - 1) >> A.n_chunk_sh);
+#pragma unroll 1
+            for (uint32_t c = sub; c < min(chunks, 8u * g); c += g) A.n_cdesc[d.w + c] = make_uint4(d.x, d.y + c * chunk, d.z, d.w);
+            for (unsigned long long many = __ballot(chunks > 8u * g && (lane & (g - 1)) == 0); many; many &= many - 1) {
                 const int l = __ffsll((long long)many) - 1;
                 const uint4 e = make_uint4(__builtin_amdgcn_readlane(d.x, l), __builtin_amdgcn_readlane(d.y, l), __builtin_amdgcn_readlane(d.z, l), __builtin_amdgcn_readlane(d.w, l));
-                for (uint32_t c = 4 + lane; (int64_t)c * chunk < (int64_t)(e.z - e.y); c += 64) A.n_cdesc[e.w + c] = make_uint4(e.x, e.y + c * chunk, e.z, e.w);
+                for (uint32_t c = 8 * g + lane; (int64_t)c * chunk < (int64_t)(e.z - e.y); c += 64) A.n_cdesc[e.w + c] = make_uint4(e.x, e.y + c * chunk, e.z, e.w);
             }
         }
         __syncthreads();
@@ -367,13 +423,6 @@ __device__ void level_tables_block(const NextArgs &A, long long *s_tmp /* [34] *
         A.n_hdr[LH_TOTAL_BUILD] = t_brows;
         if (A.n_stats) *A.n_stats = t_brows - t_pos * A.seg_cost;
     }
-}
-
-// both halves by one block: the form that rides along in the scatter kernel for inputs of up to a thousand chunks per level
-__device__ void level_next_block(const NextArgs &A, long long *s_tmp /* [34] */) {
-    chunk_scan_block(A, s_tmp);
-    __syncthreads();
-    level_tables_block(A, s_tmp);
 }
 
 // Inputs with thousands of chunks per level: the scan of the chunk counts is a kernel of its own (one block of 1024 threads)
@@ -399,8 +448,11 @@ __global__ __launch_bounds__(256) void k_part_scatter(PartArgs A, NextArgs NX) {
     // fold 2: the chunk counts were scanned by k_chunk_scan, only the next level's tables ride along
     const bool fold = A.fold == 1;
     if (blockIdx.x == gridDim.x - 1) { // the level's bookkeeping, beside the blocks that move the rows
-        if (fold) level_next_block(NX, s_tmp);
-        else level_tables_block(NX, s_tmp);
+        __shared__ uint4 s_child[512];
+        __shared__ int s_lpre[LEVEL_LPRE + 1];
+        // both halves for inputs of up to a thousand chunks per level
+        if (fold) level_tables_block<true>(NX, s_tmp, s_child, s_lpre);
+        else level_tables_block<false>(NX, s_tmp, s_child, nullptr);
         return;
     }
     // the 16 features of a record -> LDS word of their first bin (bins are 1-based); vmask bit t: feature t is sampled
@@ -590,7 +642,8 @@ __global__ __launch_bounds__(T) void k_part_move(PartArgs A, NextArgs NX) {
     __shared__ unsigned long long s_claim;
     const int64_t G = (int64_t)gridDim.x - 1;
     if (blockIdx.x == 0) { // the next level's tables, beside the blocks that move the rows
-        level_tables_block(NX, s_tmp);
+        __shared__ uint4 s_child[512];
+        level_tables_block<false>(NX, s_tmp, s_child, nullptr);
         return;
     }
     uint4 cd = A.cdesc[blockIdx.x - 1];
@@ -759,7 +812,7 @@ struct BeginArgs {
     int64_t seg_cost;
     int64_t root_words;
     int nnodes, K, D;
-    int chunk; // rows of a chunk of the root
+    int chunk_sh; // rows of a chunk of the root, a power of two
     uint4 *cdesc;
     unsigned long long *cursor;
     // the tree's column sample and its inverse map, from the pinned staging buffer to the device copies (0 words: unchanged)
@@ -788,7 +841,8 @@ __device__ void tree_begin_block(BeginArgs A) {
     for (int i = tid; i < A.js_words; i += nthr) A.js_dst[i] = A.js_src[i];
     for (int i = tid; i < A.map_words; i += nthr) A.map_dst[i] = A.map_src[i];
     if (A.n_is_dev) A.n_is = *A.n_is_dev;
-    for (int64_t c = tid; c * A.chunk < A.n_is; c += nthr) A.cdesc[c] = make_uint4(1, (uint32_t)(c * A.chunk), (uint32_t)A.n_is, 0);
+    const int64_t n_chunks = (A.n_is + ((int64_t)1 << A.chunk_sh) - 1) >> A.chunk_sh;
+    for (int64_t c = tid; c < n_chunks; c += nthr) A.cdesc[c] = make_uint4(1, (uint32_t)(c << A.chunk_sh), (uint32_t)A.n_is, 0);
     __syncthreads();
     if (tid == 0) {
         A.stats[0] = A.n_is; // read back with the tree: the host learns how many rows the mask kept
@@ -796,12 +850,12 @@ __device__ void tree_begin_block(BeginArgs A) {
         A.seg_start[1] = 0;
         A.seg_len[1] = A.n_is;
         A.hdr[LH_N_ACT] = 1;
-        A.hdr[LH_N_CHUNKS] = (A.n_is + A.chunk - 1) / A.chunk;
+        A.hdr[LH_N_CHUNKS] = n_chunks;
         A.hdr[LH_N_BUILD] = 1;
         A.hdr[LH_TOTAL_BUILD] = A.n_is + A.seg_cost;
         A.act_node[0] = 1;
         A.cprefix[0] = 0;
-        A.cprefix[1] = (A.n_is + A.chunk - 1) / A.chunk;
+        A.cprefix[1] = n_chunks;
         A.cursor[EVT_CURSOR_SLOT(1)] = 0ull;
         A.bnode[0] = 1;
         A.bstart[0] = 0;
@@ -970,7 +1024,7 @@ static void fill_begin_args(evt_ctx *c, bool all_rows, BeginArgs &A) {
     A.nnodes = c->nnodes;
     A.K = c->K;
     A.D = c->D;
-    A.chunk = part_chunk_rows(c, 1);
+    A.chunk_sh = __builtin_ctz(part_chunk_rows(c, 1));
     A.cdesc = L.cdesc;
     A.cursor = c->cursor;
     A.js_words = A.map_words = 0;
@@ -1108,7 +1162,7 @@ static void fill_next_args(evt_ctx *c, int level, NextArgs &A) {
     A.n_cdesc = Nx.cdesc;
     A.n_stats = (level + 1 <= c->D) ? c->stats + level + 1 : nullptr;
     A.seg_cost = c->hist_seg_cost;
-    A.n_chunk = part_chunk_rows(c, level + 1);
+    A.n_chunk_sh = __builtin_ctz(part_chunk_rows(c, level + 1));
     A.node_sum = nullptr;
     A.NAg = c->NAg;
     A.cursor = nullptr;
