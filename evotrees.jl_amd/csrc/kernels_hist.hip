@@ -726,7 +726,8 @@ static bool choose_hist16(const evt_ctx *c, int level, int na, int layers, Hist1
         s.ntiles = (c->RS + tw - 1) / tw;
         const int lanes = tw / s.pb;
         s.lds = (size_t)na * c->B * lanes * s.pu * 8; // channels x bins x feature bytes of a tile, words
-        if (s.lds > 128 * 1024) continue;
+        // five channels of more than 204 bins: the narrowest tile takes all of a CU (the generic kernel, 34k rows x 166 features: 138 us a level, this one 43)
+        if (s.lds > (tw == 16 && !found ? 160 : 128) * 1024) continue;
         if (tw == 16 && c->LPR > 64 && 2 * s.lds > 128 * 1024) break; // more than 1024 features whose 32-byte tiles do not fit are refused (launch_hist_build)
         const double adds = 3.2 * s.pu * na * (lanes / 16) * s.ntiles;
         const double per_row = (adds > 18 ? adds : 18) + 3.5 * (s.ntiles - 1);

@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
     ("logloss", True, None, 3_001, 17, 7, 4, 9),          # one feature in a record's second half, bins no multiple of 8
     ("mse", False, None, 5_003, 33, 100, 5, 33),          # 3 to a piece of 4 bytes
     ("gaussian_mle", False, None, 30_001, 50, 64, 5, 50),  # four channels, pieces of one byte
-    ("gaussian_mle", True, None, 8_009, 64, 255, 4, 50),  # five channels of 255 bins: no width fits one block's LDS
+    ("gaussian_mle", True, None, 8_009, 64, 255, 4, 50),  # five channels of 255 bins: the 16-byte tile fits alone
     ("mlogloss", False, 7, 12_007, 30, 64, 4, 30),        # block layers
     ("mlogloss", True, 3, 6_001, 60, 255, 4, 30),         # block layers of 16-byte tiles only
     ("mse", False, None, 4_001, 120, 2, 2, 120),          # the fewest bins there are
