@@ -275,7 +275,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->alphas = nullptr; c->alphas_f = nullptr; c->qkeys_a = c->qkeys_b = nullptr; c->qtemp = nullptr; c->qtemp_bytes = 0;
     c->n_alphas = 1;
     for (int k = 0; k < EVT_MAX_K; k++) c->h_alphas[k] = 0.5;
-    c->qscale = nullptr; c->qexp_buf[0] = c->qexp_buf[1] = nullptr; c->qscale_buf[0] = c->qscale_buf[1] = nullptr; c->q_cur = c->q_tree = 0;
+    c->qscale = nullptr; c->qexp_buf[0] = c->qexp_buf[1] = nullptr; c->qscale_buf[0] = c->qscale_buf[1] = nullptr; c->q_cur = c->q_tree = 0; c->quant_pending = false;
     c->stats = nullptr; c->errflag = nullptr; c->ogains = nullptr; c->sbest = nullptr; c->scan_count = nullptr;
     c->h_stage = nullptr; c->h_stage_dev = nullptr; c->h_stage_bytes = 0; c->h_stage_base = nullptr; c->h_stage_dev_base = nullptr;
     c->n_js_last = 0;
@@ -609,10 +609,15 @@ static void set_channels(evt_ctx *c) {
     for (int k = c->NK; k < EVT_MC_MAX_NK; k++) c->h_qbits[k] = 0;
 }
 
+// The gradients' fixed-point words, where they were left to a tree that has not come
+static int finish_quantize(evt_ctx *c) { return c->quant_pending ? launch_quantize(c) : EVT_OK; }
+
 extern "C" int evt_set_target(evt_handle c, const float *y, const float *w, const float *mu, const float *offset) {
     return guarded([&]() -> int {
     CTXCHK(c);
     ARGCHK(y && mu, "y and mu must not be NULL");
+    const int fin = finish_quantize(c); // as the channels stand
+    if (fin != EVT_OK) return fin;
     c->have_target = false;
     c->have_grads = false;
     c->pend_pred = false; // the predictions start again from mu
@@ -734,11 +739,16 @@ static int ensure_planes(evt_ctx *c) {
 }
 
 static int queue_grads(evt_ctx *c) {
+    int r = finish_quantize(c); // the pass raises the maxima that the quantisation before it clears
+    if (r != EVT_OK) return r;
     prof_begin(c, EVT_K_GRAD, 0);
-    int r = launch_grads(c);
+    r = launch_grads(c);
     prof_end(c);
     if (r != EVT_OK) return r;
     if (c->profiling) c->prof_units[EVT_K_GRAD] += c->N;
+    // a tree of the kernels for small inputs quantises on its way: the next one is taken to be like the last (tree_open knows)
+    c->quant_pending = true;
+    if (small_tree_form(c, c->n_js_last > 0 ? c->n_js_last : c->F, c->n_js_last == 0 || c->last_all_rows)) return EVT_OK;
     prof_begin(c, EVT_K_OTHER, 0);
     r = launch_quantize(c);
     prof_end(c);
@@ -774,8 +784,9 @@ extern "C" int evt_set_grads(evt_handle c, const float *grad) {
     }
     c->grads_ready = false;
     c->have_grads = false;
+    int r = finish_quantize(c);
+    if (r != EVT_OK) return r;
     HIPCHK(hipMemcpyAsync(c->grad, grad, sizeof(float) * (size_t)c->N * c->NK, hipMemcpyDefault, c->stream));
-    int r = EVT_OK;
     if (c->unit_w) { // the target was set without weights: the row count stands for the weight, the weight row must say so
         r = launch_check_unit_weight(c);
         if (r == EVT_OK) r = check_errflag(c, "evt_set_grads: the weight row must be all ones when evt_set_target was given no weights");
@@ -830,6 +841,13 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
     c->grads_ready = false; // this tree changes the predictions
     c->last_all_rows = all_rows;
     c->last_cond = cond;
+    const int small = staged ? 0 : small_tree_form(c, n_js, all_rows);
+    int r = EVT_OK;
+    if (c->quant_pending) {
+        if (small) quant_set(c); // by the tree's first kernel
+        else r = launch_quantize(c);
+        if (r != EVT_OK) return r;
+    }
     c->q_tree = c->q_cur; // this tree is grown on (and decoded with) the tables of the gradients quantised last
     // a tree grown in stages records the node of every row on the way, so that evt_get_nidx can show it after each stage
     // ... and so does a quantile loss: its leaves are valued from the rows they hold once the tree is complete
@@ -860,9 +878,8 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
     const bool fuse_pred = p->update_pred && all_rows && !defer;
     c->write_nidx = rec_nidx || defer;
 
-    const int small = staged ? 0 : small_tree_form(c, n_js, all_rows);
     c->step.hist_fused = !staged && scatter_can_build_hist(c, n_js); // the set-up below cuts the root's chunks by it
-    int r = small ? EVT_OK : ensure_planes(c);
+    r = small ? EVT_OK : ensure_planes(c);
     if (r != EVT_OK) return r;
     if (EVT_IS_QUANTILE(c->loss)) {
         r = quantile_leaf_buffers(c);
@@ -1394,6 +1411,8 @@ extern "C" int evt_get_quant(evt_handle c, int32_t *qbits, int32_t *qexp) {
     CTXCHK(c);
     ARGCHK(qbits && qexp, "NULL argument");
     int32_t e[EVT_MC_MAX_NK];
+    const int r = finish_quantize(c);
+    if (r != EVT_OK) return r;
     // the tables of the last tree's gradients, also when the next round's have been quantised behind it
     HIPCHK(hipMemcpyAsync(e, c->n_js_last > 0 ? c->qexp_buf[c->q_tree] : c->qexp, sizeof(int32_t) * EVT_MC_MAX_NK, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));

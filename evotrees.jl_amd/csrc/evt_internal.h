@@ -165,6 +165,7 @@ struct evt_ctx {
     int32_t *qexp_buf[2];
     double *qscale_buf[2];
     int q_cur, q_tree;
+    bool quant_pending;  // the gradients' fixed-point words are still to be made: by the first kernel of a small tree, or by k_quantize
     double *metric_partial; // [2 * EVT_METRIC_BLOCKS + 1] evaluation-metric partial sums, result last
     int64_t *stats;    // [D+1] rows built per level
     int32_t *errflag;  // device-side validation flag
@@ -348,6 +349,8 @@ __device__ __forceinline__ void evt_add_leaf(float *pr, const float *lp, int K, 
 // grad
 int launch_grads(evt_ctx *c);
 int launch_quantize(evt_ctx *c);
+void quant_set(evt_ctx *c);
+uint32_t *absmax_set(evt_ctx *c, int which);
 int launch_apply_pending(evt_ctx *c);
 int launch_set_weight_row(evt_ctx *c, const float *w_dev);
 int launch_validate_classes(evt_ctx *c);

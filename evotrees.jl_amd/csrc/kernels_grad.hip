@@ -7,65 +7,8 @@
 // the addition to the prediction (predict!, src/predict.jl:1-46) happens here, in row order, as the
 // first thing the next gradient pass does (4 B of node id read and 4K B written more per row) - or in
 // k_apply_leaf when something else needs the predictions first.
-#include "evt_internal.h"
+#include "grad_math.h"
 #include <algorithm>
-
-// Maximum of the 64 lanes' values, none of them negative or NaN (their bit patterns order as they do), by VALU moves as in split_math.h's prefix
-// scan: seven outputs' fourteen maxima as cross-lane shuffles were 84 trips through the LDS crossbar, one after the other (60k rows of 7 classes: the
-// gradient pass 13.2 -> 10.1 us).
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ uint32_t max_step(uint32_t v) {
-    const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROW_MASK, 0xf, false);
-    return o > v ? o : v;
-}
-__device__ __forceinline__ float wave_max_f32(float x) {
-    uint32_t v = __float_as_uint(x);
-    v = max_step<0x111, 0xf>(v); // row_shr:1
-    v = max_step<0x112, 0xf>(v); // row_shr:2
-    v = max_step<0x114, 0xf>(v); // row_shr:4
-    v = max_step<0x118, 0xf>(v); // row_shr:8
-    v = max_step<0x142, 0xa>(v); // row_bcast:15 into rows 1 and 3
-    v = max_step<0x143, 0xc>(v); // row_bcast:31 into rows 2 and 3
-    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)v, 63));
-}
-
-__device__ __forceinline__ float dev_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
-__device__ __forceinline__ float dev_softplus(float x) { return fmaxf(x, 0.0f) + log1pf(expf(-fabsf(x))); }
-
-// mle2p_grad_hess, src/loss.jl:194-217: GaussianMLE (LOSS 2) and LogisticMLE (LOSS 7); raw is the unconstrained scale.
-template <int LOSS>
-__device__ __forceinline__ void mle2p_grad_hess(float loc, float raw, float y, float &g_loc, float &g_scale, float &h_loc, float &h_scale) {
-    const float scale = dev_softplus(raw);
-    const float dscale = dev_sigmoid(raw);
-    const float ds = dscale / scale;
-    if (LOSS == 2) {
-        const float resid = loc - y;
-        const float s2 = scale * scale;
-        g_loc = resid / s2;
-        g_scale = (1.0f - (resid * resid) / s2) * dscale / scale;
-        h_loc = 1.0f / s2;
-        h_scale = 2.0f * (ds * ds);
-    } else {
-        const float z = (y - loc) / scale;
-        const float th = tanhf(z / 2.0f);
-        g_loc = -th / scale;
-        g_scale = (1.0f - z * th) * dscale / scale;
-        h_loc = 1.0f / (3.0f * (scale * scale));
-        h_scale = (3.14159274f * 3.14159274f + 3.0f) / 9.0f * (ds * ds); // oftype(scale, pi)^2
-    }
-}
-
-// Raises the running maximum of gradient row k.  Same-address atomics from thousands of blocks queue up one behind the
-// other (about 20 ns each - 40 us for the 2048 blocks of a gradient pass), so the maximum is kept in
-// EVT_ABSMAX_STRIPES copies on different cache lines, a block raises the copy its index selects, and the one reader
-// (the quantisation pass, k_quantize) takes the largest.  The value only grows while a pass runs: a block whose own maximum is already
-// covered by what a device-scope load shows skips the atomic.
-__device__ __forceinline__ void absmax_raise(uint32_t *absmax, int k, float m) {
-    if (!(m > 0.0f)) return;
-    uint32_t *p = absmax + (blockIdx.x % EVT_ABSMAX_STRIPES) * EVT_MC_MAX_NK + k;
-    const uint32_t u = __float_as_uint(m);
-    if (__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < u) atomicMax(p, u);
-}
 
 // Maxima of any number of outputs (mx[k] and mx[EVT_MAX_K + k]: gradient row k and K + k), by a whole block of 256 threads: a thread raises a
 // row, all rows side by side, where one thread raising them in turn took two barriers and a trip to memory for each (60k rows of 7 classes:
@@ -85,8 +28,6 @@ __device__ __forceinline__ void raise_maxima(const float *mx, int K, uint32_t *a
         absmax_raise(absmax, t < EVT_MAX_K ? k : K + k, fmaxf(fmaxf(s_m[0][t], s_m[1][t]), fmaxf(s_m[2][t], s_m[3][t])));
 }
 
-// LOSS: 0 mse (src/loss.jl:52), 1 logloss (:54-57), 2 gaussian_mle (:194-203), 3 poisson (:59-62),
-// 4 gamma (:64-67), 5 tweedie with rho = 1.5 (:69-76), 8 mae (:78), 9 cred_var / cred_std (:80-83).
 // grad rows: [g_1..g_K, h_1..h_K, w]; every written value is multiplied by w (src/loss.jl:104-108, :223-233).
 // Blocks of 256 threads, or of 1024 where the grid fills the chip: the blocks of a whole generation raise their maxima at the same time, and a
 // quarter of them queue for a quarter as long (1M rows, blocks of 256 | 1024: 8.4 | 6.5 us).
@@ -104,42 +45,7 @@ __global__ __launch_bounds__(1024) void k_grads(float *__restrict__ pred, const 
         float *g = grad + (size_t)NK * i;
         const float w = unit_w ? 1.0f : g[NK - 1]; // unit weights: the weight row (all ones) is not read
         if (pend_nidx) evt_add_leaf(pred + (size_t)K * i, pend_leaf + (size_t)K * (pend_nidx[i] - 1), K, LOSS);
-        if (LOSS == 0) {
-            const float gg = 2.0f * (pred[i] - y[i]);
-            out[0] = gg * w;
-            out[1] = 2.0f * w;
-        } else if (LOSS == 1) {
-            const float s = dev_sigmoid(pred[i]);
-            out[0] = (s - y[i]) * w;
-            out[1] = (s * (1.0f - s)) * w;
-        } else if (LOSS == 3) {
-            const float e = expf(pred[i]);
-            out[0] = (e - y[i]) * w;
-            out[1] = e * w;
-        } else if (LOSS == 4) {
-            const float e = expf(pred[i]);
-            out[0] = (2.0f * (1.0f - y[i] / e)) * w;
-            out[1] = (2.0f * y[i] / e) * w;
-        } else if (LOSS == 5) {
-            const float e = expf(pred[i]);
-            const float a = powf(e, 0.5f), b = powf(e, -0.5f);
-            out[0] = (2.0f * (a - y[i] * b)) * w;
-            out[1] = (2.0f * (0.5f * a - (-0.5f) * y[i] * b)) * w;
-        } else if (LOSS == 8) { // mae (src/loss.jl:78): the residual, no second-order row
-            out[0] = (y[i] - pred[i]) * w;
-            out[1] = 0.0f * w;
-        } else if (LOSS == 9) { // credibility losses (src/loss.jl:80-83): residual and its square
-            const float d = y[i] - pred[i];
-            out[0] = d * w;
-            out[1] = (d * d) * w;
-        } else {
-            float g1, g2, h1, h2;
-            mle2p_grad_hess<LOSS>(pred[2 * i], pred[2 * i + 1], y[i], g1, g2, h1, h2);
-            out[0] = g1 * w;
-            out[1] = g2 * w;
-            out[2] = h1 * w;
-            out[3] = h2 * w;
-        }
+        grad_row<LOSS>(pred + (size_t)K * i, y[i], w, out);
 #pragma unroll
         for (int k = 0; k < 2 * K; k++) {
             g[k] = out[k];
@@ -364,18 +270,7 @@ __global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ grad
     __shared__ int s_qexp[EVT_MC_MAX_NK], s_qbits[EVT_MC_MAX_NK];
     const int t = threadIdx.x;
     if (t < NK) {
-        uint32_t mu = 0u;
-        for (int st = 0; st < EVT_ABSMAX_STRIPES; st++) {
-            const uint32_t v = absmax[st * EVT_MC_MAX_NK + t]; // non-negative floats order as their bit patterns
-            mu = v > mu ? v : mu;
-        }
-        const float m = __uint_as_float(mu);
-        int e = 0;
-        if (m > 0.0f) {
-            e = ilogbf(m) + 1;
-            if (e > 128) e = 128;
-            if (e < -140) e = -140;
-        }
+        const int e = quant_exponent(absmax, t);
         const int qb = qbits[t];
         s_qexp[t] = e;
         s_qbits[t] = qb;
@@ -390,8 +285,7 @@ __global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ grad
                 for (int st = 0; st < EVT_ABSMAX_STRIPES; st++) absmax_next[st * EVT_MC_MAX_NK + t] = 0u;
         }
         if (t < NAg) {
-            // global channel ag -> gradient row: mse {g, w}; otherwise identity; last channel is w (or the row count)
-            const int kk = EVT_TWO_CHAN(loss, (NK - 1) / 2) ? (t == 0 ? 0 : 2) : t; // one-target mse / mae: channels {g, w}
+            const int kk = quant_row(loss, (NK - 1) / 2, t); // the last channel is w (or the row count)
             if (t == NAg - 1 && unit_w) qscale_g[t] = 1.0;
             else qscale_g[t] = scalbn(1.0, s_qexp[kk] - s_qbits[kk]);
         }
@@ -414,7 +308,7 @@ __global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ grad
 }
 
 // the set of striped maxima the next gradient pass raises (and the quantisation behind it reads)
-static uint32_t *absmax_set(evt_ctx *c, int which) { return c->absmax + (size_t)which * EVT_ABSMAX_STRIPES * EVT_MC_MAX_NK; }
+uint32_t *absmax_set(evt_ctx *c, int which) { return c->absmax + (size_t)which * EVT_ABSMAX_STRIPES * EVT_MC_MAX_NK; }
 
 int launch_grads(evt_ctx *c) {
     // the maxima of the rows this kernel writes start from zero (cleared at creation and by the quantisation pass before last)
@@ -533,11 +427,16 @@ int launch_absmax_rows(evt_ctx *c, int k0, int k1) {
     return EVT_OK;
 }
 
-int launch_quantize(evt_ctx *c) {
-    // write the set of tables the last grown tree does not use: its histogram stays decodable
+// The tables the gradients at hand are quantised with: the set the last grown tree does not use, whose histogram stays decodable
+void quant_set(evt_ctx *c) {
     c->q_cur = c->q_tree ^ 1;
     c->qexp = c->qexp_buf[c->q_cur];
     c->qscale = c->qscale_buf[c->q_cur];
+}
+
+int launch_quantize(evt_ctx *c) {
+    quant_set(c);
+    c->quant_pending = false;
     double *qmul = c->qscale + EVT_MC_MAX_NK; // decode scales per global channel first, then encode multipliers per gradient row
     // every block derives the multipliers first: fewer blocks where a row is one word (1M rows, at most 1024 | 4096 blocks: 5.4 | 6.5 us; four words
     // a row at 500k rows 7.8 | 6.9, one word at 10M 27.6 | 25.5)

@@ -7,6 +7,7 @@
 // best candidate per node.  The blocks meet only at the kernel boundary.  Rows keep their place: a node id per row stands for the row lists,
 // so rows outside the sample walk along (flagged) and the prediction needs no pass of its own over the tree.
 // The sums are the same integers and the gains the same expressions as in the kernels of larger inputs: same trees, bit for bit.
+#include "grad_math.h"
 #include "pool.h"
 #include "split_math.h"
 #include <algorithm>
@@ -24,7 +25,7 @@ static_assert(sizeof(SmallHead) == 64, "one candidate per 64-byte line");
 
 struct SmallArgs {
     const uint8_t *xcm;
-    const unsigned long long *gq;
+    unsigned long long *gq;
     uint8_t *mask;
     const uint32_t *nid_in; // the rows' node ids as the level above left them
     uint32_t *nid_out;
@@ -41,7 +42,14 @@ struct SmallArgs {
     int map_words;
     int32_t *status;
     long long *node_sum;
-    const double *qscale;
+    double *qscale;
+    // the root: the gradients; fresh ones are still to be quantised, of their maxima, and leave the tables
+    const float *raw;
+    int fresh;
+    const uint32_t *absmax;
+    uint32_t *absmax_next;
+    const int32_t *qbits;
+    int32_t *qexp;
     TreeDev tree;
     int64_t *stats;
     const uint4 *blob_src; // final kernel: the tree's arrays and their pinned destination
@@ -70,17 +78,19 @@ __device__ __forceinline__ long long shfl_i64(long long v, int src) {
 }
 __device__ __forceinline__ double shfl_f64(double v, int src) { return __longlong_as_double(shfl_i64(__double_as_longlong(v), src)); }
 
-// lane i's statistic i (of 2K+1) from lane-held channel sums (decode_vals, a statistic per lane)
-__device__ __forceinline__ double lane_stat(const SmallArgs &A, long long q, int lane) {
+// lane i's statistic i (of 2K+1) from lane-held channel sums (decode_vals, a statistic per lane); sc: the lane's scale
+__device__ __forceinline__ int lane_channel(const SmallArgs &A, int lane) {
+    return EVT_TWO_CHAN(A.loss, A.K) ? (lane == 0 ? 0 : 1) : (lane < A.NAg ? lane : 0);
+}
+__device__ __forceinline__ double lane_stat(const SmallArgs &A, long long q, double sc, int lane) {
     const bool two = EVT_TWO_CHAN(A.loss, A.K);
-    const int src = two ? (lane == 0 ? 0 : 1) : (lane < A.NAg ? lane : 0);
-    double v = (double)shfl_i64(q, src) * A.qscale[src];
+    double v = (double)shfl_i64(q, lane_channel(A, lane)) * sc;
     if (two && lane == 1) v = (A.loss == EVT_LOSS_MSE) ? 2.0 * v : 0.0;
     return v;
 }
 // a node's weight and, for a leaf, its values (leaf_value, an output per lane)
-__device__ __forceinline__ void write_node(const SmallArgs &A, int n, long long q, int lane, bool leaf) {
-    const double S = lane_stat(A, q, lane);
+__device__ __forceinline__ void write_node(const SmallArgs &A, int n, long long q, double sc, int lane, bool leaf) {
+    const double S = lane_stat(A, q, sc, lane);
     double v[3] = {shfl_f64(S, lane < A.K ? lane : 0), shfl_f64(S, A.K + (lane < A.K ? lane : 0)), shfl_f64(S, 2 * A.K)};
     if (lane == 0) A.tree.w[n - 1] = (float)v[2];
     if (leaf && lane < A.K) A.tree.pred[(int64_t)A.K * (n - 1) + lane] = (float)leaf_value(A.loss, v, 0, 1, A.eta, A.bagging, A.lambda, A.L2);
@@ -92,7 +102,8 @@ __device__ __forceinline__ void write_node(const SmallArgs &A, int n, long long 
 __device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t *s_dec, long long *s_tot, bool writer, int lane) {
     const int n = (1 << (A.level - 2)) + p, nag = A.NAg, nwg = A.nfs;
     const int st = A.status[n];
-    const long long qn = lane < nag ? A.node_sum[(int64_t)n * nag + lane] : 0;
+    const long long qn = A.node_sum[(int64_t)n * nag + (lane < nag ? lane : 0)];
+    const double sc = A.qscale[lane_channel(A, lane)];
     // every lane reads whole candidates (one line each), so that the winner's feature and totals are at hand
     const SmallHead *hp = A.head_in + (int64_t)p * nwg;
     union Words {
@@ -108,6 +119,9 @@ __device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t
         const uint4 *cp = reinterpret_cast<const uint4 *>(hp + (w < nwg ? w : nwg - 1));
 #pragma unroll
         for (int k = 0; k < 4; k++) c.v[k] = cp[k];
+#pragma unroll
+        for (int k = 0; k < 4; k++) // all of it now: the compiler fetches the totals behind the comparison of the gains, a second trip to memory
+            asm volatile("" : "+v"(c.v[k].x), "+v"(c.v[k].y), "+v"(c.v[k].z), "+v"(c.v[k].w));
         if (w < nwg && c.h.gain > mine.h.gain) {
             mine = c;
             bj = w;
@@ -145,7 +159,7 @@ __device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t
         s_tot[(2 * p + 1) * nag + lane] = qn - ql;
     }
     if (!writer || !active) return;
-    write_node(A, n, qn, lane, !found);
+    write_node(A, n, qn, sc, lane, !found);
     if (lane == 0) {
         A.status[n] = found ? ST_SPLIT : ST_LEAF;
         if (found) {
@@ -162,7 +176,7 @@ __device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t
         const long long qc = child ? qn - ql : ql;
         if (lane < nag) A.node_sum[(int64_t)cn * nag + lane] = qc;
         if (lane == 0) A.status[cn] = A.level < A.D ? ST_BUILD : ST_LEAF;
-        if (A.level == A.D) write_node(A, cn, qc, lane, true);
+        if (A.level == A.D) write_node(A, cn, qc, sc, lane, true);
     }
 }
 
@@ -209,7 +223,7 @@ __device__ __forceinline__ long long channel_of(const unsigned long long *H, int
 // only.  on_gain(b, ok, gain, left) is called for every bin of the lane; left: the totals left of it (NAG channels; NAG == 0: null).
 // Returns the node's totals in q (NAG != 0).
 template <int NAG, int BPL, bool PACK, typename GAIN>
-__device__ __forceinline__ void small_scan(const SmallArgs &A, const unsigned long long *H, const long long *tot, bool numeric, int constraint, int lane,
+__device__ __forceinline__ void small_scan(const SmallArgs &A, const double *qs, const unsigned long long *H, const long long *tot, bool numeric, int constraint, int lane,
                                            long long *hist_out, long long *q, GAIN on_gain) {
     const int B = A.B, nag = NAG ? NAG : A.NAg;
     const int bmax = numeric ? B - 1 : B;
@@ -219,7 +233,7 @@ __device__ __forceinline__ void small_scan(const SmallArgs &A, const unsigned lo
         double sc[NAG], S[NK];
 #pragma unroll
         for (int ag = 0; ag < NAG; ag++) {
-            sc[ag] = A.qscale[ag];
+            sc[ag] = qs[ag];
             long long val[BPL], run = 0;
 #pragma unroll
             for (int t = 0; t < BPL; t++) {
@@ -282,13 +296,13 @@ __device__ __forceinline__ void small_scan(const SmallArgs &A, const unsigned lo
         };
         long long lq[BPL], tq;
         lefts(nag - 1, lq, tq);
-        const double w_p = (double)tq * A.qscale[nag - 1];
+        const double w_p = (double)tq * qs[nag - 1];
         double w_l[BPL], w_r[BPL], sg[BPL], gain_p = 0.0;
         bool ok[BPL];
 #pragma unroll
         for (int t = 0; t < BPL; t++) {
             const int b = lane * BPL + t;
-            w_l[t] = (double)lq[t] * A.qscale[nag - 1];
+            w_l[t] = (double)lq[t] * qs[nag - 1];
             w_r[t] = w_p - w_l[t];
             ok[t] = b < B && b + 1 <= bmax && w_l[t] > A.min_weight && w_r[t] > A.min_weight;
             sg[t] = 0.0;
@@ -297,7 +311,7 @@ __device__ __forceinline__ void small_scan(const SmallArgs &A, const unsigned lo
             long long gq[BPL], hq[BPL], tg, th;
             lefts(k, gq, tg);
             lefts(K + k, hq, th);
-            const double scg = A.qscale[k], sch = A.qscale[K + k];
+            const double scg = qs[k], sch = qs[K + k];
             const double Sg = (double)tg * scg, Sh = (double)th * sch;
             gain_p += node_gain_k(A.loss, Sg, Sh, w_p, A.lambda, A.L2);
 #pragma unroll
@@ -331,7 +345,7 @@ __device__ __forceinline__ void small_left(const SmallArgs &A, const unsigned lo
 // The search of one (node, feature) and what it leaves: the node's histogram of the feature, the candidate - or, for an oblivious
 // level, the gains of all bins in s_gain - and at the root the node's totals.
 template <int NAG, int BPL, bool PACK>
-__device__ __forceinline__ void small_search(const SmallArgs &A, const unsigned long long *Hs, int q, int jp, int nwg, uint32_t fw, const long long *tot,
+__device__ __forceinline__ void small_search(const SmallArgs &A, const double *qs, const unsigned long long *Hs, int q, int jp, int nwg, uint32_t fw, const long long *tot,
                                              bool writer, double *s_gain, int lane) {
     const int B = A.B, nag = NAG ? NAG : A.NAg, n = (1 << (A.level - 1)) + q;
     const bool numeric = (fw & SMALL_NUMERIC) != 0;
@@ -343,7 +357,7 @@ __device__ __forceinline__ void small_search(const SmallArgs &A, const unsigned 
     long long tq[QA], lq[QA];
 #pragma unroll
     for (int ag = 0; ag < QA; ag++) lq[ag] = 0;
-    small_scan<NAG, BPL, PACK>(A, Hs, tot, numeric, (int)(fw >> 17) - 1, lane, hout, tq, [&](int b, bool ok, double gain, const long long *left) {
+    small_scan<NAG, BPL, PACK>(A, qs, Hs, tot, numeric, (int)(fw >> 17) - 1, lane, hout, tq, [&](int b, bool ok, double gain, const long long *left) {
         if (A.oblivious) {
             if (b < B) s_gain[b] = gain; // update_gains!
         } else if (ok && gain > lg) {
@@ -392,6 +406,11 @@ __device__ __forceinline__ void small_search(const SmallArgs &A, const unsigned 
     }
 }
 
+// Requests every 64-byte line of the arguments at once: read where each is needed, they were ten trips one after the other.
+__device__ __forceinline__ void touch_args(const SmallArgs &A) {
+    asm volatile("" ::"s"(A.xcm), "s"(A.left_in), "s"(A.js_src), "s"(A.qscale), "s"(A.qexp), "s"(A.stats), "s"(A.gamma), "s"(A.nfs), "s"(A.cond));
+}
+
 // An oblivious level's row of one feature (grow_otree!, src/fit.jl:190-217), by one wavefront: the gains of the level's nodes added in
 // node order, zero where one of them is not positive, and the first maximum over the bins.
 __device__ __forceinline__ int small_obliv_best(const SmallArgs &A, const double *s_gain, int nact, int lane, double *gain) {
@@ -416,21 +435,28 @@ __device__ __forceinline__ int small_obliv_best(const SmallArgs &A, const double
     return bb;
 }
 
+// ROOT: the tree's first level, which also quantises the gradients (no k_quantize: 3.1 us and a launch of a round of 60 at 2000 rows x 10).  A level is a
+// chain of trips to memory in few blocks (2000 rows: 9.7 us below the root with its loads behind branches and its arguments read one by one, 8.7
+// now; the root 6.5 with the quantisation beside it, 7.0 with it inside).  Whole fits: 2000 x 10, 100 rounds 7.5 -> 6.9 ms, 100k x 10, 200 rounds
+// with an eval set 21.1 -> 20.2.
 // SPLIT: a feature's rows are shared by `slices` blocks, which add their histograms into A.acc; the last of them to do so reads the sums and
 // searches them (100k rows x 10 features: 8.3 us a level and 5.2 for a kernel of its own that searched -> 13.9, and a round of five levels
 // 101 -> 92 us).  What passes between the blocks goes by agent-scope atomics, past the caches that are not shared, and is complete before its
 // block is counted (as in k_scan).  For inputs of
 // few features, whose blocks would fill a part of the chip with long walks: 10 features in 25 slices take 0.4 us per 25k rows and channel pair
 // where one block per feature takes 0.4 us per 1k, for 5 us more of flush and hand-over.
-template <int NAG, int BPL, bool PACK, bool SPLIT>
+template <int NAG, int BPL, bool PACK, bool SPLIT, bool ROOT>
 __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
     extern __shared__ unsigned long long s_dyn[];
     __shared__ uint32_t s_dec[SMALL_MAX_NODES];
     __shared__ uint16_t s_slot[SMALL_MAX_NODES];  // node of the level -> slot among the active ones (0xFFFF: not active)
     __shared__ uint16_t s_node[SMALL_MAX_NODES];  // and back
     __shared__ int s_nact, s_cnt, s_best;
+    __shared__ double s_qs[EVT_MC_MAX_NK], s_qmul[EVT_MC_MAX_NK]; // scales of the channels; multipliers of the gradient rows (raw)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int B = A.B, N = A.N, level = A.level;
+    touch_args(A);
+    const int B = A.B, N = A.N, level = ROOT ? 1 : A.level;
+    __builtin_assume(ROOT || level > 1);
     const int nag = NAG ? NAG : A.NAg, na = NAG ? NAG - (PACK ? 1 : 0) : A.NA;
     int jp = blockIdx.x, slice = 0;
     if (SPLIT) { // blocks go to the 8 XCDs in turn: each takes a run of slices with all their features, whose rows' gradients then share its L2
@@ -450,31 +476,37 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
     if (tid == 0) s_cnt = 0;
     const uint8_t *col = A.xcm + (size_t)f * N;
     // A thread takes U groups of 4 neighbouring rows at a time (the last group of all starts at N - 4 and leaves out what others
-    // have); what the first of them need is requested before the decisions.
+    // have); what the first of them need is requested before the decisions, in straight-line code: with the root's loads and the other levels' behind
+    // branches each load was waited for before the next (six trips to memory before the first decision).
     constexpr int U = (NAG == 2 && PACK && BPL < 4) ? 2 : 1, GA = NAG ? NAG - (PACK ? 1 : 0) : 1;
     const int allgroups = (N + 3) >> 2, per = SPLIT ? (allgroups + A.slices - 1) / A.slices : allgroups;
     const int gfirst = SPLIT ? slice * per : 0, ngroups = SPLIT && gfirst + per < allgroups ? gfirst + per : allgroups; // the block's: gfirst .. ngroups
-    uint32_t nid[U][4], xb[U];
+    // a row's channel is a word of A.gq, or at the root its gradient, quantised on the way (as k_quantize does, whose launch this saves: A.fresh)
+    uint32_t nid[U][4], xb[U], g0[U][4]; // g0: channel 0 where it is 32 bits wide, or at the root the gradient
     unsigned long long g[GA][U][4];
+    constexpr bool NARROW = NAG != 0 && PACK; // channel 0 is staged as a 32-bit word
+    const uint8_t *const mask = A.sampled && !A.draw ? A.mask : col;
     auto request = [&](int k0) {
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int k = k0 + u * 1024 < ngroups ? k0 + u * 1024 : ngroups - 1, r = 4 * k < N - 4 ? 4 * k : N - 4;
             xb[u] = load4(col + r);
-            if (level > 1) {
+            if constexpr (ROOT) {
+                nid[u][0] = load4(mask + r); // the rows' mask bytes
+            } else {
                 const uint4 v = load16(A.nid_in + r);
                 nid[u][0] = v.x; nid[u][1] = v.y; nid[u][2] = v.z; nid[u][3] = v.w;
-            } else { // at the root: the rows' mask bytes
-                nid[u][0] = (A.sampled && !A.draw) ? load4(A.mask + r) : 0u;
             }
             if constexpr (NAG != 0) {
 #pragma unroll
                 for (int a = 0; a < GA; a++) {
-                    if (PACK && a == 0) {
-                        const uint4 v = load16(reinterpret_cast<const uint32_t *>(A.gq) + r);
-                        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+                    if constexpr (ROOT) {
+                        const float *q = A.raw + (size_t)r * A.NK + (NAG == 2 && a == 1 ? 2 : a);
 #pragma unroll
-                        for (int i = 0; i < 4; i++) g[a][u][i] = ((unsigned long long)(long long)(int32_t)w[i] << EVT_PACK_CNT_BITS) + 1ull;
+                        for (int i = 0; i < 4; i++) g[a][u][i] = __float_as_uint(q[i * A.NK]);
+                    } else if (NARROW && a == 0) {
+                        const uint4 v = load16(reinterpret_cast<const uint32_t *>(A.gq) + r);
+                        g0[u][0] = v.x; g0[u][1] = v.y; g0[u][2] = v.z; g0[u][3] = v.w;
                     } else {
                         const uint32_t *q = reinterpret_cast<const uint32_t *>(A.gq + (size_t)a * N + r);
                         const uint4 v0 = load16(q), v1 = load16(q + 4);
@@ -487,10 +519,53 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
             }
         }
     };
+    // the word of a gradient v of channel a, left for the levels below by the block that has the row's share
+    auto quantise = [&](float v, int a, int row, bool keep) {
+        const long long w = __double2ll_rn((double)v * s_qmul[quant_row(A.loss, A.K, a)]);
+        const unsigned long long packed = ((unsigned long long)w << EVT_PACK_CNT_BITS) + 1ull;
+        if (PACK && a == 0 && !(NAG == 0 && A.wide)) {
+            if (keep) reinterpret_cast<int32_t *>(A.gq)[row] = (int32_t)w;
+            return packed;
+        }
+        const unsigned long long out = PACK && a == 0 ? packed : (unsigned long long)w;
+        if (keep) A.gq[(size_t)a * N + row] = out;
+        return out;
+    };
     request(gfirst + tid);
-    if (level > 1) {
+    if constexpr (ROOT) { // the tables: made here of fresh gradients, or those the words in A.gq were made with
+        if (tid < A.NK) {
+            const double *mul = A.qscale + EVT_MC_MAX_NK;
+            if (A.fresh) {
+                const int e = quant_exponent(A.absmax, tid), qb = A.qbits[tid];
+                const double m = scalbn(1.0, qb - e);
+                s_qmul[tid] = m;
+                for (int ag = 0; ag < nag; ag++)
+                    if (quant_row(A.loss, A.K, ag) == tid) {
+                        const double sc = PACK && ag == nag - 1 ? 1.0 : scalbn(1.0, e - qb);
+                        s_qs[ag] = sc;
+                        if (writer) A.qscale[ag] = sc;
+                    }
+                if (writer) {
+                    A.qexp[tid] = e;
+                    A.qscale[EVT_MC_MAX_NK + tid] = m;
+                    if (tid < A.NK - 1)
+                        for (int st = 0; st < EVT_ABSMAX_STRIPES; st++) A.absmax_next[st * EVT_MC_MAX_NK + tid] = 0u;
+                }
+            } else {
+                s_qmul[tid] = mul[tid];
+                if (tid < nag) s_qs[tid] = A.qscale[tid];
+            }
+        }
+    }
+    const double my_scale = A.qscale[tid < nag ? tid : 0];
+    // the histograms of the first nodes, cleared while the loads are under way
+    for (int i = tid; i < (nlev < A.slots ? nlev : A.slots) * na * B; i += 1024) H[i] = 0ull;
+    if constexpr (!ROOT) {
         const int np = nlev >> 1;
-        for (int p = wave; p < np; p += 16) small_decide(A, p, s_dec, s_tot, writer, lane);
+        // the first outside the loop: in front of a loop that reads memory the compiler waits for what is under way
+        if (wave < np) small_decide(A, wave, s_dec, s_tot, writer, lane);
+        for (int p = wave + 16; p < np; p += 16) small_decide(A, p, s_dec, s_tot, writer, lane);
+        if (tid < nag) s_qs[tid] = my_scale;
         __syncthreads();
         if (wave == 0) { // the children of split nodes are the level's active nodes
             int base = 0;
@@ -538,12 +613,23 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
     const int nact = s_nact;
     int counted = 0;
     auto take = [&](int k0, int base, int ns) { // the groups requested at k0, for the nodes in slots base .. base + ns
+        uint32_t d[U][4], b[U][4];
+        if constexpr (!ROOT) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int k = k0 + u * 1024 < ngroups ? k0 + u * 1024 : ngroups - 1, r = 4 * k < N - 4 ? 4 * k : N - 4;
+#pragma unroll
+                for (int i = 0; i < 4; i++) d[u][i] = row_decision(A, nid[u][i], s_dec);
+#pragma unroll
+                for (int i = 0; i < 4; i++) b[u][i] = decision_bin(A, d[u][i], r + i);
+            }
+        }
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int k = k0 + u * 1024, r = 4 * k < N - 4 ? 4 * k : N - 4;
             if (k >= ngroups) continue;
-            if (level == 1) {
-                uint32_t mb = nid[u][0];
+            if constexpr (ROOT) {
+                const uint32_t mb = nid[u][0];
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     uint32_t m = (mb >> (8 * i)) & 0xFFu;
@@ -558,18 +644,29 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
                     nid[u][i] = (A.sampled && m > (uint32_t)A.cond) ? 1u | SMALL_OUT : 1u;
                 }
             } else {
-                uint32_t d[4], b[4];
 #pragma unroll
-                for (int i = 0; i < 4; i++) d[i] = row_decision(A, nid[u][i], s_dec);
-#pragma unroll
-                for (int i = 0; i < 4; i++) b[i] = decision_bin(A, d[i], r + i);
-#pragma unroll
-                for (int i = 0; i < 4; i++) nid[u][i] = row_moves(nid[u][i], d[i], b[i]);
+                for (int i = 0; i < 4; i++) nid[u][i] = row_moves(nid[u][i], d[u][i], b[u][i]);
             }
             // every block has the same ids: each writes a share (a wavefront's 256 rows; rows of the last group twice, alike)
-            if (base == 0 && (k >> 6) % (int)gridDim.x == jp)
+            const bool share = base == 0 && (k >> 6) % (int)gridDim.x == jp;
+            if (share)
 #pragma unroll
                 for (int i = 0; i < 4; i++) A.nid_out[r + i] = nid[u][i];
+            if constexpr (ROOT) {
+                const bool keep = share && A.fresh;
+                if constexpr (NAG != 0) {
+#pragma unroll
+                    for (int a = 0; a < GA; a++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) g[a][u][i] = quantise(__uint_as_float((uint32_t)g[a][u][i]), a, r + i, keep);
+                } else if (keep) {
+                    for (int i = 0; i < 4; i++)
+                        for (int a = 0; a < na; a++) quantise(A.raw[(size_t)(r + i) * A.NK + a], a, r + i, true);
+                }
+            } else if constexpr (NARROW) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) g[0][u][i] = ((unsigned long long)(long long)(int32_t)g0[u][i] << EVT_PACK_CNT_BITS) + 1ull;
+            }
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int q = (int)(nid[u][i] & ~SMALL_OUT) - first;
@@ -584,7 +681,8 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
                 } else {
                     for (int a = 0; a < na; a++) {
                         unsigned long long v;
-                        if (PACK && a == 0 && !A.wide) v = evt_load_gq<true>(A.gq, N, 0, (uint32_t)(r + i));
+                        if (ROOT) v = quantise(A.raw[(size_t)(r + i) * A.NK + a], a, r + i, false);
+                        else if (PACK && a == 0 && !A.wide) v = evt_load_gq<true>(A.gq, N, 0, (uint32_t)(r + i));
                         else v = A.gq[(size_t)a * N + r + i];
                         atomicAdd(h + a * B, v);
                     }
@@ -593,8 +691,6 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
         }
     };
     int ns = nact < A.slots ? nact : A.slots;
-    for (int i = tid; i < ns * na * B; i += 1024) H[i] = 0ull;
-    __syncthreads();
     take(gfirst + tid, 0, ns);
     for (int base = 0; base == 0 || base < nact; base += A.slots) {
         if (base > 0) {
@@ -624,7 +720,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
         } else
         for (int s = wave; s < ns; s += 16) {
             const int q = s_node[base + s];
-            small_search<NAG, BPL, PACK>(A, H + (size_t)s * na * B, q, jp, A.nfs, fw, level > 1 ? s_tot + q * nag : nullptr, writer,
+            small_search<NAG, BPL, PACK>(A, s_qs, H + (size_t)s * na * B, q, jp, A.nfs, fw, level > 1 ? s_tot + q * nag : nullptr, writer,
                                          A.oblivious ? s_gain + s * B : nullptr, lane);
         }
         __syncthreads();
@@ -679,7 +775,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
             __syncthreads();
             for (int k = wave; k < nb; k += 16) {
                 const int q = s_node[base + k];
-                small_search<NAG, BPL, false>(A, S + (size_t)k * words, q, jp, A.nfs, fw, level > 1 ? s_tot + q * nag : nullptr, jp == 0,
+                small_search<NAG, BPL, false>(A, s_qs, S + (size_t)k * words, q, jp, A.nfs, fw, level > 1 ? s_tot + q * nag : nullptr, jp == 0,
                                               A.oblivious ? gains + (base + k) * B : nullptr, lane);
             }
             __syncthreads();
@@ -718,12 +814,14 @@ __global__ __launch_bounds__(1024) void k_small_final(SmallArgs A) {
     __shared__ uint32_t s_dec[SMALL_MAX_NODES];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const bool writer = blockIdx.x == 0;
+    touch_args(A);
     const int np = 1 << (A.level - 2);
     long long *s_tot = reinterpret_cast<long long *>(s_dyn);
     const int r = (int)blockIdx.x * 1024 + tid;
     uint32_t nid = r < A.N ? A.nid_in[r] : 0u;
     asm volatile("" : "+v"(nid));
-    for (int p = wave; p < np; p += 16) small_decide(A, p, s_dec, s_tot, writer, lane);
+    if (wave < np) small_decide(A, wave, s_dec, s_tot, writer, lane);
+    for (int p = wave + 16; p < np; p += 16) small_decide(A, p, s_dec, s_tot, writer, lane);
     __syncthreads();
     if (r < A.N) {
         const uint32_t d = row_decision(A, nid, s_dec);
@@ -866,6 +964,14 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
         A.feat[j] = (uint32_t)f | (c->h_feattypes[f] ? SMALL_NUMERIC : 0u) | ((uint32_t)(c->h_mono[f] + 1) << 17);
     }
     const int bpl = (c->B + 63) / 64;
+    A.raw = c->grad;
+    if (c->quant_pending) {
+        A.fresh = 1;
+        A.absmax = absmax_set(c, c->absmax_cur);
+        A.absmax_next = absmax_set(c, c->absmax_cur ^ 1);
+        A.qbits = c->qbits;
+        A.qexp = c->qexp;
+    }
     for (int level = 1; level <= c->D; level++) {
         A.level = level;
         const int in = (level & 1) ^ 1, out = level & 1;
@@ -891,26 +997,29 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
             lds = std::max(lds, small_lds_search(c, level, A.batch));
         }
         prof_begin(c, level == 1 ? EVT_K_HIST : EVT_K_PARTITION, level); // below the root it moves rows, builds and searches at once
-#define SMALL3(NAG_, BPL_, PACK_)                                                                                                                  \
-    {                                                                                                                                              \
-        static EvtDevOnce once;                                                                                                                    \
-        if (once.pending(c->device)) {                                                                                                             \
-            for (const void *k : {reinterpret_cast<const void *>(k_small_level<NAG_, BPL_, PACK_, false>),                                         \
-                                  reinterpret_cast<const void *>(k_small_level<NAG_, BPL_, PACK_, true>)})                                         \
-                HIPCHK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));                                            \
-            once.mark(c->device);                                                                                                                  \
-        }                                                                                                                                          \
-        const unsigned nf = (unsigned)c->n_js_last;                                                                                                \
-        if (!split) {                                                                                                                              \
-            hipLaunchKernelGGL((k_small_level<NAG_, BPL_, PACK_, false>), dim3(nf), dim3(1024), lds, c->stream, A);                                \
-        } else {                                                                                                                                   \
-            hipLaunchKernelGGL((k_small_level<NAG_, BPL_, PACK_, true>), dim3(nf, (unsigned)slices), dim3(1024), lds, c->stream, A);               \
-        }                                                                                                                                          \
+#define SMALL4(NAG_, BPL_, PACK_, SPLIT_, ROOT_)                                                                                          \
+    {                                                                                                                                     \
+        static EvtDevOnce once;                                                                                                           \
+        if (once.pending(c->device)) {                                                                                                    \
+            HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_small_level<NAG_, BPL_, PACK_, SPLIT_, ROOT_>),                    \
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));                                          \
+            once.mark(c->device);                                                                                                         \
+        }                                                                                                                                 \
+        hipLaunchKernelGGL((k_small_level<NAG_, BPL_, PACK_, SPLIT_, ROOT_>), dim3((unsigned)c->n_js_last, split ? (unsigned)slices : 1u), \
+                           dim3(1024), lds, c->stream, A);                                                                                \
+    }
+#define SMALL3(NAG_, BPL_, PACK_)                                    \
+    if (split) {                                                     \
+        if (level == 1) SMALL4(NAG_, BPL_, PACK_, true, true)        \
+        else SMALL4(NAG_, BPL_, PACK_, true, false)                  \
+    } else {                                                         \
+        if (level == 1) SMALL4(NAG_, BPL_, PACK_, false, true)       \
+        else SMALL4(NAG_, BPL_, PACK_, false, false)                 \
     }
 #define SMALL2(NAG_, PACK_)             \
-    if (bpl == 1) SMALL3(NAG_, 1, PACK_) \
-    else if (bpl == 2) SMALL3(NAG_, 2, PACK_) \
-    else SMALL3(NAG_, 4, PACK_)
+    if (bpl == 1) { SMALL3(NAG_, 1, PACK_) } \
+    else if (bpl == 2) { SMALL3(NAG_, 2, PACK_) } \
+    else { SMALL3(NAG_, 4, PACK_) }
 #define SMALL1(NAG_)            \
     if (c->unit_w) { SMALL2(NAG_, true) } \
     else { SMALL2(NAG_, false) }
@@ -921,9 +1030,14 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
 #undef SMALL1
 #undef SMALL2
 #undef SMALL3
+#undef SMALL4
         A.slots = most;
         prof_end(c);
         HIPCHK(hipGetLastError());
+        if (c->quant_pending) { // made by the root's kernel, which cleared the set that the next gradient pass raises
+            c->quant_pending = false;
+            c->absmax_cur ^= 1;
+        }
     }
     HIPCHK(hipGetLastError());
     c->step.blob_sent = true;

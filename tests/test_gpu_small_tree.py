@@ -78,3 +78,64 @@ def test_one_kernel_per_level_changes_nothing(evt, N, F, B, D, loss, more):
             assert_tree_bits(a2, b)
             splits += int(a.split.sum())
     assert splits > 0 or N < 10
+
+
+@pytest.mark.parametrize("N,B,loss,K", [(1030, 64, "mse", 1), (2501, 200, "logloss", 1), (1999, 33, "gaussian_mle", 2), (1500, 40, "mlogloss", 7)])
+def test_gradients_quantised_by_the_tree_or_not(evt, N, B, loss, K):
+    """The root's kernel quantises what evt_update_grads left; whatever comes in between (a second update, other targets, gradients from outside,
+    the other kernels, a second tree on the same gradients) sees what k_quantize would have left: same tables, trees and histograms."""
+    F, D = 6, 4
+    rng = np.random.default_rng(N)
+    x_bin = rng.integers(1, B + 1, size=(F, N), dtype=np.uint8)
+    if loss == "mlogloss":
+        y, mu = (1 + (x_bin[0].astype(int) + rng.integers(0, 3, N)) % K).astype(np.float32), np.zeros(K, np.float32)
+    else:
+        _, y, _, mu = make_data(N, N, F, B, loss, False)
+    small_y = y if loss in ("mlogloss", "logloss") else y * np.float32(2.0 ** -9)  # smaller maxima: none may be left of the first targets
+    small_mu = mu if small_y is y else mu * np.float32(2.0 ** -9)
+    w = (rng.random(N) + 0.5).astype(np.float32)
+    js = np.arange(1, F + 1, dtype=np.uint32)
+    gp = evt.make_params(eta=0.3, L2=1.0)
+    keep = evt.make_params(eta=0.3, L2=1.0, update_pred=0, bagging_size=2)
+    out = []
+    for small in (2, 3, 0):
+        h = evt.Handle(N, F, B, len(mu), D, loss)
+        h.set_option("small_tree", small)
+        h.set_xbin(x_bin)
+        rec = []
+
+        def note():
+            rec.extend([h.get_hist(), np.concatenate(h.get_quant()), h.get_pred(), h.get_grads()])
+
+        h.set_target(y, None, mu)
+        h.update_grads()
+        h.update_grads()
+        rec.append(np.concatenate(h.get_quant()))  # before any tree
+        rec.append(h.grow_tree(js, gp))
+        note()
+        h.update_grads()
+        h.set_target(small_y, w, small_mu)  # other channels, smaller gradients
+        h.update_grads()
+        rec.append(h.grow_tree(js, keep))
+        rec.append(h.grow_tree(js, keep))  # on the same gradients
+        note()
+        h.update_grads()
+        h.set_option("small_tree", 0)
+        rec.append(h.grow_tree(js, gp))
+        h.set_option("small_tree", small)
+        note()
+        h.update_grads()
+        h.set_grads(h.get_grads() * np.float32(0.25))
+        rec.append(h.grow_tree(js, gp))
+        note()
+        h.close()
+        out.append(rec)
+    splits = 0
+    for a, a2, b in zip(*out):
+        if isinstance(a, np.ndarray):
+            assert a.tobytes() == b.tobytes() and a2.tobytes() == b.tobytes()
+        else:
+            assert_tree_bits(a, b)
+            assert_tree_bits(a2, b)
+            splits += int(a.split.sum())
+    assert splits > 0
