@@ -181,7 +181,7 @@ extern "C" int evt_destroy(evt_handle c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     void *ptrs[] = {c->xcm, c->xrm, c->y, c->pred, c->grad, c->gq, c->is_a, c->is_b, c->nidx, c->mask, c->flagw, c->chunk_nleft, c->chunk_lpre, c->cursor,
                     c->hist, c->seg_start, c->seg_len, c->status, c->node_sum, c->tree_blob, c->tree.packed, c->js, c->jsmap, c->feattypes, c->mono, c->absmax, c->qexp_buf[0], c->qexp_buf[1], c->qbits,
-                    c->qscale_buf[0], c->qscale_buf[1], c->planes, c->metric_partial, c->errflag, c->ogains, c->sbest, c->scan_count, c->is_id, c->pt_nodes, c->pt_pred, c->mask_next,
+                    c->qscale_buf[0], c->qscale_buf[1], c->planes, c->metric_partial, c->errflag, c->ogains, c->sbest, c->scan_count, c->is_id, c->pt_nodes, c->mask_next,
                     c->small_nid[0], c->small_nid[1], c->small_head[0], c->small_head[1], c->small_left[0], c->small_left[1], c->small_acc,
                     c->alphas, c->alphas_f, c->qkeys_a, c->qkeys_b, c->qtemp};
     if (c->copy_stream) (void)hipStreamSynchronize(c->copy_stream);
@@ -310,7 +310,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->tree_seq = 0;
     c->slot_seq[0] = c->slot_seq[1] = 0;
     c->step.phase = 0;
-    c->pt_nodes = nullptr; c->pt_pred = nullptr; c->pt_stage = nullptr; c->pt_stage_dev = nullptr; c->pt_cap = 0; c->pt_busy = false;
+    c->pt_nodes = nullptr; c->pt_stage = nullptr; c->pt_stage_dev = nullptr; c->pt_cap = 0; c->pt_busy = false;
     c->tree_evs[0] = c->tree_evs[1] = nullptr;
     c->mask_next = nullptr;
     c->copy_stream = nullptr;
@@ -433,6 +433,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->nidx, 0, sizeof(uint32_t) * N, c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->errflag, 0, sizeof(int32_t), c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->scan_count, 0, sizeof(int32_t) * EVT_SCAN_COUNT_STEP * c->maxlvl, c->stream);
+    if (e2 == hipSuccess) e2 = hipMemsetAsync(c->metric_partial + 2 * EVT_METRIC_BLOCKS, 0, sizeof(double), c->stream);
     if (e2 == hipSuccess) e2 = upload_alphas(c);
     int r = EVT_OK;
     if (e2 == hipSuccess) r = launch_iota(c, c->is_id, N);
@@ -1291,24 +1292,21 @@ extern "C" int evt_predict_tree(evt_handle c, int32_t nnodes_tree, const int64_t
     if (c->pt_cap < nn) { // device copies and upload buffer are kept between calls and grown on demand
         HIPCHK(hipStreamSynchronize(c->stream));
         dev_give(c->pt_nodes);
-        dev_give(c->pt_pred);
         pinned_give(c->pt_stage);
-        c->pt_nodes = nullptr; c->pt_pred = nullptr; c->pt_stage = nullptr; c->pt_stage_dev = nullptr; c->pt_cap = 0;
+        c->pt_nodes = nullptr; c->pt_stage = nullptr; c->pt_stage_dev = nullptr; c->pt_cap = 0;
         const size_t cap = std::max(nn, (size_t)2047);
-        c->pt_nodes = static_cast<uint32_t *>(dev_take(sizeof(uint32_t) * cap));
-        c->pt_pred = static_cast<float *>(dev_take(sizeof(float) * cap * c->K));
+        c->pt_nodes = static_cast<uint32_t *>(dev_take(sizeof(uint32_t) * cap * (1 + c->K)));
         c->pt_stage = c->pt_stage_dev = static_cast<uint8_t *>(pinned_take(sizeof(uint32_t) * cap * (1 + c->K)));
-        if (!c->pt_nodes || !c->pt_pred || !c->pt_stage) return EVT_ERR_NOMEM;
+        if (!c->pt_nodes || !c->pt_stage) return EVT_ERR_NOMEM;
         c->pt_cap = cap;
     }
     memcpy(c->pt_stage, nodes.data(), sizeof(uint32_t) * nn);
     memcpy(c->pt_stage + sizeof(uint32_t) * nn, pred, sizeof(float) * nn * c->K);
-    r = launch_copy_words(c, c->pt_stage_dev, c->pt_nodes, sizeof(uint32_t) * nn);
-    if (r == EVT_OK) r = launch_copy_words(c, c->pt_stage_dev + sizeof(uint32_t) * nn, c->pt_pred, sizeof(float) * nn * c->K);
+    r = launch_copy_words(c, c->pt_stage_dev, c->pt_nodes, sizeof(uint32_t) * nn * (1 + c->K)); // the leaf values behind the nodes
     if (r != EVT_OK) return r;
     c->pt_busy = true;
     prof_begin(c, EVT_K_PREDICT, 0);
-    r = launch_predict_tree_nodes(c, c->pt_nodes, nnodes_tree, c->pt_pred);
+    r = launch_predict_tree_nodes(c, c->pt_nodes, nnodes_tree, reinterpret_cast<const float *>(c->pt_nodes + nn));
     prof_end(c);
     if (r != EVT_OK) return r;
     if (c->profiling) {
@@ -1443,10 +1441,8 @@ extern "C" int evt_eval_metric(evt_handle c, int32_t metric, double *value_out) 
     }
     prof_begin(c, EVT_K_OTHER, 0);
     int r = launch_apply_pending(c);
-    if (r == EVT_OK) r = launch_eval_metric(c, metric, c->metric_partial);
+    if (r == EVT_OK) r = launch_eval_metric(c, metric, reinterpret_cast<double *>(c->h_stage_dev));
     prof_end(c);
-    if (r != EVT_OK) return r;
-    r = launch_copy_words(c, c->metric_partial + 2 * EVT_METRIC_BLOCKS, c->h_stage_dev, sizeof(double)); // a kernel's store, not the copy engine
     if (r != EVT_OK) return r;
     HIPCHK(hipStreamSynchronize(c->stream));
     c->pt_busy = false;

@@ -166,7 +166,7 @@ struct evt_ctx {
     double *qscale_buf[2];
     int q_cur, q_tree;
     bool quant_pending;  // the gradients' fixed-point words are still to be made: by the first kernel of a small tree, or by k_quantize
-    double *metric_partial; // [2 * EVT_METRIC_BLOCKS + 1] evaluation-metric partial sums, result last
+    double *metric_partial; // [2 * EVT_METRIC_BLOCKS + 1] evaluation-metric partial sums, then how many blocks have left theirs (zero between launches)
     int64_t *stats;    // [D+1] rows built per level
     int32_t *errflag;  // device-side validation flag
     double *ogains;    // oblivious: [maxlvl][F][B]
@@ -179,8 +179,7 @@ struct evt_ctx {
     uint8_t *h_stage_base, *h_stage_dev_base;
     // evt_predict_tree: device copies of the tree handed in (packed nodes, leaf values) and the pinned buffer they are
     // uploaded through; kept between calls and grown on demand
-    uint32_t *pt_nodes;
-    float *pt_pred;
+    uint32_t *pt_nodes; // the nodes, then the leaf values
     uint8_t *pt_stage, *pt_stage_dev;
     size_t pt_cap; // nodes
     bool pt_busy;  // an upload from pt_stage has been queued since the stream was last drained here
@@ -360,7 +359,7 @@ int launch_transpose_validate(evt_ctx *c);
 int launch_build_planes(evt_ctx *c);
 int launch_binarize(hipStream_t s, const void *x_dev, int dtype, int64_t rs, int64_t cs, const double *edges_dev, const int32_t *edge_off_dev, int max_edges,
                     uint8_t *xcm, int64_t n, int F, int64_t ldo);
-int launch_eval_metric(evt_ctx *c, int metric, double *partial);
+int launch_eval_metric(evt_ctx *c, int metric, double *out);
 // tree
 int launch_tree_begin(evt_ctx *c);
 int launch_iota(evt_ctx *c, uint32_t *dst, int64_t n);

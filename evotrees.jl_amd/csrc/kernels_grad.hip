@@ -452,7 +452,7 @@ int launch_quantize(evt_ctx *c) {
 // ---- evaluation metric ------------------------------------------------------------------------
 // Per row value of src/metrics.jl:1-28 (:88-91 for gaussian_mle) in Float32, weighted as eval[i] = w * v / K
 // (:43, :111), accumulated in Float64.  Two stages with a fixed shape (EVT_METRIC_BLOCKS partial sums, then one
-// block) keep the summation order, hence the result, independent of scheduling.
+// block's) keep the summation order, hence the result, independent of scheduling.
 __device__ __forceinline__ float metric_value_one(int metric, float pk, float yk);
 // T: target columns of y (K, or 1 when every output is measured against the one target: _target(y::AbstractVector, k, i) = y[i],
 // src/loss.jl:49).  alphas: the levels of the quantile metrics as Float32 (src/callback.jl:62-66).
@@ -525,10 +525,13 @@ __device__ __forceinline__ double block_sum_f64(double v, double *s_red) {
     return (s_red[0] + s_red[1]) + (s_red[2] + s_red[3]);
 }
 
-__global__ __launch_bounds__(256) void k_metric_partial(const float *__restrict__ pred, const float *__restrict__ y,
+// The block that leaves its sums last adds them up and stores the metric in host memory: two launches fewer per round than with a kernel for that and one
+// for the store (and a tree goes up in one copy): 100k x 10 with 25k eval rows, 200 rounds 20.8 -> 19.9 ms.
+__global__ __launch_bounds__(256) void k_metric(const float *__restrict__ pred, const float *__restrict__ y,
                                                        const float *__restrict__ grad, int64_t N, int NK, int K, int T, int metric, float kdiv,
-                                                       const float *__restrict__ alphas, double *__restrict__ partial) {
+                                                       const float *__restrict__ alphas, double *partial, int *count, double *out) {
     __shared__ double s_red[4];
+    __shared__ int s_last;
     double num = 0.0, den = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < N; i += (int64_t)gridDim.x * 256) {
         const float w = grad[(size_t)NK * i + NK - 1];
@@ -538,39 +541,38 @@ __global__ __launch_bounds__(256) void k_metric_partial(const float *__restrict_
     }
     num = block_sum_f64(num, s_red);
     den = block_sum_f64(den, s_red);
-    if (threadIdx.x == 0) {
-        partial[2 * blockIdx.x] = num;
-        partial[2 * blockIdx.x + 1] = den;
+    if (threadIdx.x == 0) { // past the caches that are not shared, and in memory before the block is counted
+        __hip_atomic_store(partial + 2 * blockIdx.x, num, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(partial + 2 * blockIdx.x + 1, den, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        s_last = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
     }
-}
-
-__global__ __launch_bounds__(256) void k_metric_final(const double *__restrict__ partial, int nblocks, int metric, double *out) {
-    __shared__ double s_red[4];
-    double num = 0.0, den = 0.0;
-    for (int b = threadIdx.x; b < nblocks; b += 256) {
-        num += partial[2 * b];
-        den += partial[2 * b + 1];
+    __syncthreads();
+    if (!s_last) return;
+    num = den = 0.0;
+    for (int b = threadIdx.x; b < (int)gridDim.x; b += 256) {
+        num += __hip_atomic_load(partial + 2 * b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        den += __hip_atomic_load(partial + 2 * b + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     num = block_sum_f64(num, s_red);
     den = block_sum_f64(den, s_red);
     if (threadIdx.x == 0) {
         const double r = num / den;
         out[0] = (metric == EVT_METRIC_RMSE) ? sqrt(r) : r;
+        *count = 0; // for the next launch
     }
 }
 
-// partial: 2 * EVT_METRIC_BLOCKS + 1 doubles; the metric lands in the last one
-int launch_eval_metric(evt_ctx *c, int metric, double *partial) {
+// the metric lands in `out`, the caller's pinned buffer
+int launch_eval_metric(evt_ctx *c, int metric, double *out) {
     int64_t nb = (c->N + 255) / 256;
     if (nb > EVT_METRIC_BLOCKS) nb = EVT_METRIC_BLOCKS;
     const float kdiv = (metric == EVT_METRIC_MLOGLOSS) ? 1.0f : (float)((metric == EVT_METRIC_GAUSSIAN_MLE || metric == EVT_METRIC_LOGISTIC_MLE) ? c->K / 2 : c->K);
     // y has K columns for the losses whose outputs each have a target; the multi-class, two-parameter and multiquantile
     // metrics index their own layouts
     const int T = (c->loss == EVT_LOSS_MULTIQUANTILE) ? 1 : c->K;
-    hipLaunchKernelGGL(k_metric_partial, dim3((unsigned)nb), dim3(256), 0, c->stream, c->pred, c->y, c->grad, c->N, c->NK, c->K, T, metric, kdiv,
-                       c->alphas_f, partial);
-    HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_metric_final, dim3(1), dim3(256), 0, c->stream, partial, (int)nb, metric, partial + 2 * EVT_METRIC_BLOCKS);
+    hipLaunchKernelGGL(k_metric, dim3((unsigned)nb), dim3(256), 0, c->stream, c->pred, c->y, c->grad, c->N, c->NK, c->K, T, metric, kdiv,
+                       c->alphas_f, c->metric_partial, reinterpret_cast<int *>(c->metric_partial + 2 * EVT_METRIC_BLOCKS), out);
     HIPCHK(hipGetLastError());
     return EVT_OK;
 }

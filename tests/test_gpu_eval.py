@@ -23,6 +23,35 @@ METRICS_OF = {
 }
 
 
+@pytest.mark.parametrize("N", [2, 255, 257, 262_144, 262_145, 600_001])  # one block, a partial one, all 1024 of them, several rows a thread
+def test_metric_of_the_last_block(evt, N):
+    """The last block to leave its sums adds them up and stores the metric: call after call on one handle and after trees of several sizes handed in."""
+    rng = np.random.default_rng(N)
+    h = evt.Handle(N, 3, 8, 1, 1, "mse")
+    x_bin = rng.integers(1, 9, size=(3, N), dtype=np.uint8)
+    y, w = rng.random(N, dtype=np.float32), rng.random(N, dtype=np.float32) + np.float32(0.5)
+    h.set_xbin(x_bin)
+    h.set_target(y, w, np.zeros(1, np.float32))
+    pred = np.zeros(N, np.float32)
+    for depth in (1, 3, 2):  # leaves in full heaps of 1, 7 and 3 nodes
+        n = (1 << depth) - 1
+        t = evt.TreeArrays(1, n)
+        t.feat[:], t.cond_bin[:], t.split[:], t.pred[:] = 0, 0, 0, 0.0
+        inner = n // 2
+        t.feat[:inner], t.cond_bin[:inner], t.split[:inner] = 1 + np.arange(inner) % 3, 4, 1
+        t.pred.reshape(-1)[inner:] = rng.random(n - inner, dtype=np.float32)
+        h.predict_tree(t)
+        node = np.zeros(N, np.int64)
+        for _ in range(depth - 1):
+            node = 2 * node + 1 + (x_bin[node % 3, np.arange(N)] > 4)
+        pred = pred + t.pred.reshape(-1)[node]
+        assert np.array_equal(h.get_pred().reshape(-1), pred)
+        d = pred - y
+        for metric, rows in (("mse", w * (d * d)), ("mae", w * np.abs(d)), ("mse", w * (d * d))):  # Float32 rows, Float64 sums
+            np.testing.assert_allclose(h.eval_metric(metric), rows.astype(np.float64).sum() / w.astype(np.float64).sum(), rtol=1e-12)
+    h.close()
+
+
 @pytest.mark.parametrize("loss,weights", [("mse", True), ("logloss", False), ("gaussian_mle", True), ("poisson", True),
                                           ("gamma", False), ("tweedie", True), ("mlogloss", True), ("logistic_mle", True),
                                           ("quantile", True), ("multiquantile", False)])
