@@ -917,6 +917,7 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
     c->step.small_draw = draw;
     c->step.fuse_pred = fuse_pred;
     c->step.blob_sent = false;
+    c->step.grads_done = false;
     c->step.p = *p;
     // the root's list is the identity (kept, never written) or what the mask compaction left in is_a; the levels below
     // alternate between is_a and is_b
@@ -1019,7 +1020,7 @@ static int tree_close(evt_ctx *c) {
         if (c->profiling) c->prof_units[EVT_K_PREDICT] += c->N;
     }
     if (defer) {
-        c->pend_pred = true;
+        c->pend_pred = !c->step.grads_done; // the gradient pass adds them
         c->nidx_valid = all_rows; // with a row sample the recorded leaves are those of all rows
     }
 
@@ -1034,7 +1035,8 @@ static int tree_close(evt_ctx *c) {
         // the next round's gradient update runs while the host collects this tree and prepares the next call.  Not with
         // bagging: the trees of one round are all grown on the same gradients (src/fit.jl:9-11), and the library cannot
         // tell which call is the round's last.
-        r = queue_grads(c);
+        if (c->step.grads_done) c->quant_pending = true; // by the tree's last kernel
+        else r = queue_grads(c);
         if (r != EVT_OK) return r;
         c->grads_ready = true;
     }

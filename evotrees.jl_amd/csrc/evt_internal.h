@@ -224,6 +224,7 @@ struct evt_ctx {
         bool hist_fused; // levels below the root get their histograms from the scatter pass of the level above
         int small;       // one kernel per level: the blocks that share a feature's rows (small_tree_form)
         bool small_draw; // ... whose first draws the row mask
+        bool grads_done; // the tree's last kernel added the leaf values and computed the next round's gradients
         bool blob_sent;  // the finished tree's transfer to the host rode along with the tree's last kernel
         uint32_t *is_cur, *is_next; // row-id lists of the current level and of the one below
         evt_params p;

@@ -56,6 +56,11 @@ struct SmallArgs {
     uint4 *blob_dst;
     int64_t blob_n;
     uint32_t *nidx;
+    // final kernel, where it computes the next round's gradients (k_grads)
+    float *pred;
+    const float *y;
+    float *grad;
+    uint32_t *maxima;
     double eta, lambda, L2, gamma, min_weight;
     unsigned long long seed;
     int N, F, B, K, NK, NAg, NA, loss, level, D, nnodes, nfs, bagging;
@@ -66,6 +71,7 @@ struct SmallArgs {
     int *done;      // ... and how many of a feature's blocks have added theirs, zero between two levels
     int batch;      // ... and the nodes whose sums its last block's LDS holds at a time
     int oblivious, sampled, draw, cond;
+    int unit_w;
     int wide;      // channel 0 staged as a 64-bit packed word (more channels than EVT_MAX_NA)
     // the blocks' features, in the launch's arguments: a block need not wait for them.  0-based id | numeric << 16 | (constraint + 1) << 17
     uint32_t feat[256];
@@ -88,18 +94,23 @@ __device__ __forceinline__ double lane_stat(const SmallArgs &A, long long q, dou
     if (two && lane == 1) v = (A.loss == EVT_LOSS_MSE) ? 2.0 * v : 0.0;
     return v;
 }
-// a node's weight and, for a leaf, its values (leaf_value, an output per lane)
-__device__ __forceinline__ void write_node(const SmallArgs &A, int n, long long q, double sc, int lane, bool leaf) {
+// a node's weight and, for a leaf, its values (leaf_value, an output per lane), in the tree's arrays (writer) and in s_leaf where rows will ask for them
+__device__ __forceinline__ void write_node(const SmallArgs &A, int n, long long q, double sc, int lane, bool leaf, bool writer, float *s_leaf) {
     const double S = lane_stat(A, q, sc, lane);
     double v[3] = {shfl_f64(S, lane < A.K ? lane : 0), shfl_f64(S, A.K + (lane < A.K ? lane : 0)), shfl_f64(S, 2 * A.K)};
-    if (lane == 0) A.tree.w[n - 1] = (float)v[2];
-    if (leaf && lane < A.K) A.tree.pred[(int64_t)A.K * (n - 1) + lane] = (float)leaf_value(A.loss, v, 0, 1, A.eta, A.bagging, A.lambda, A.L2);
+    if (writer && lane == 0) A.tree.w[n - 1] = (float)v[2];
+    if (leaf && lane < A.K) {
+        const float val = (float)leaf_value(A.loss, v, 0, 1, A.eta, A.bagging, A.lambda, A.L2);
+        if (writer) A.tree.pred[(int64_t)A.K * (n - 1) + lane] = val;
+        if (s_leaf) s_leaf[lane] = val;
+    }
 }
 
 // The decision for node p of the level above `A.level`, by one wavefront: the best of the blocks' candidates (highest gain, then
 // earliest feature; its bin is already the lowest).  Leaves the packed split in s_dec[p] (0: none) and the children's totals in
-// s_tot; the writer block also writes the Tree arrays and the children's state.
-__device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t *s_dec, long long *s_tot, bool writer, int lane) {
+// s_tot; the writer block also writes the Tree arrays and the children's state.  s_leaf (last level): the values of the leaves among the
+// nodes of the level above, then among the level's own.
+__device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t *s_dec, long long *s_tot, bool writer, int lane, float *s_leaf = nullptr) {
     const int n = (1 << (A.level - 2)) + p, nag = A.NAg, nwg = A.nfs;
     const int st = A.status[n];
     const long long qn = A.node_sum[(int64_t)n * nag + (lane < nag ? lane : 0)];
@@ -158,9 +169,9 @@ __device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t
         s_tot[(2 * p) * nag + lane] = ql;
         s_tot[(2 * p + 1) * nag + lane] = qn - ql;
     }
-    if (!writer || !active) return;
-    write_node(A, n, qn, sc, lane, !found);
-    if (lane == 0) {
+    if (!active || !(writer || s_leaf)) return;
+    write_node(A, n, qn, sc, lane, !found, writer, s_leaf ? s_leaf + p * A.K : nullptr);
+    if (writer && lane == 0) {
         A.status[n] = found ? ST_SPLIT : ST_LEAF;
         if (found) {
             A.tree.feat[n - 1] = feat;
@@ -174,9 +185,11 @@ __device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t
     for (int child = 0; child < 2; child++) {
         const int cn = 2 * n + child;
         const long long qc = child ? qn - ql : ql;
-        if (lane < nag) A.node_sum[(int64_t)cn * nag + lane] = qc;
-        if (lane == 0) A.status[cn] = A.level < A.D ? ST_BUILD : ST_LEAF;
-        if (A.level == A.D) write_node(A, cn, qc, sc, lane, true);
+        if (writer) {
+            if (lane < nag) A.node_sum[(int64_t)cn * nag + lane] = qc;
+            if (lane == 0) A.status[cn] = A.level < A.D ? ST_BUILD : ST_LEAF;
+        }
+        if (A.level == A.D) write_node(A, cn, qc, sc, lane, true, writer, s_leaf ? s_leaf + ((1 << (A.level - 2)) + 2 * p + child) * A.K : nullptr);
     }
 }
 
@@ -807,25 +820,83 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
     }
 }
 
-// The last decisions, the leaves, and every row's leaf (added to the predictions by the next pass over the rows, as for larger
-// inputs).  The first block also sends the finished tree to the host's pinned buffer.
+// The last decisions, the leaves, and every row's leaf.  The first block also sends the finished tree to the host's pinned buffer.
+// LOSS >= 0: the rows' leaf values are added and the next round's gradients computed here, as k_grads<LOSS> would (whose launch and trip through
+// the node ids this saves); otherwise the next pass over the rows adds them, as for larger inputs.
+// 2000 rows x 10: 6.0 + 3.4 us and the gap between two launches -> 6.9; 308k rows of two outputs 11.2 + 7.7 -> 16.4.  Whole fits: 100 rounds of the first
+// 6.9 -> 6.6 ms, 200 rounds of 100k x 10 with an eval set 20.0 -> 19.3, 138 of the last 24.7 -> 24.1 (with more blocks than are resident at once 25.5).
+template <int LOSS>
 __global__ __launch_bounds__(1024) void k_small_final(SmallArgs A) {
     extern __shared__ unsigned long long s_dyn[];
     __shared__ uint32_t s_dec[SMALL_MAX_NODES];
+    constexpr bool GRADS = LOSS >= 0;
+    constexpr int K = LOSS == 2 || LOSS == 7 ? 2 : 1, NK = 2 * K + 1;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const bool writer = blockIdx.x == 0;
     touch_args(A);
     const int np = 1 << (A.level - 2);
     long long *s_tot = reinterpret_cast<long long *>(s_dyn);
-    const int r = (int)blockIdx.x * 1024 + tid;
-    uint32_t nid = r < A.N ? A.nid_in[r] : 0u;
-    asm volatile("" : "+v"(nid));
-    if (wave < np) small_decide(A, wave, s_dec, s_tot, writer, lane);
-    for (int p = wave + 16; p < np; p += 16) small_decide(A, p, s_dec, s_tot, writer, lane);
-    __syncthreads();
-    if (r < A.N) {
+    float *s_leaf = GRADS ? reinterpret_cast<float *>(s_tot + 2 * np * A.NAg) : nullptr;
+    // the block's first rows are requested before the decisions; a block has more where there are more than 256 x 1024 of them
+    uint32_t nid;
+    float pr[K], y = 0.0f, w = 1.0f, mx[2 * K];
+#pragma unroll
+    for (int k = 0; k < 2 * K; k++) mx[k] = 0.0f;
+    auto request = [&](int r) {
+        const int row = r < A.N ? r : A.N - 1;
+        nid = A.nid_in[row];
+        if constexpr (GRADS) {
+#pragma unroll
+            for (int k = 0; k < K; k++) pr[k] = A.pred[(size_t)K * row + k];
+            y = A.y[row];
+            if (!A.unit_w) w = A.grad[(size_t)NK * row + NK - 1];
+        }
+    };
+    auto finish = [&](int r) {
         const uint32_t d = row_decision(A, nid, s_dec);
-        A.nidx[r] = row_moves(nid, d, decision_bin(A, d, r)) & ~SMALL_OUT;
+        const uint32_t leaf = row_moves(nid, d, decision_bin(A, d, r < A.N ? r : A.N - 1)) & ~SMALL_OUT;
+        if (r < A.N) A.nidx[r] = leaf;
+        if constexpr (GRADS) {
+            float l[K], out[2 * K];
+            const int at = (int)leaf - np; // nodes of the last two levels; leaves above them were written by an earlier kernel
+#pragma unroll
+            for (int k = 0; k < K; k++) l[k] = at >= 0 ? s_leaf[K * at + k] : A.tree.pred[(size_t)K * (leaf - 1) + k];
+            evt_add_leaf(pr, l, K, LOSS);
+            grad_row<LOSS>(pr, y, w, out);
+            if (r < A.N) {
+#pragma unroll
+                for (int k = 0; k < K; k++) A.pred[(size_t)K * r + k] = pr[k];
+#pragma unroll
+                for (int k = 0; k < 2 * K; k++) {
+                    A.grad[(size_t)NK * r + k] = out[k];
+                    mx[k] = fmaxf(mx[k], fabsf(out[k]));
+                }
+            }
+        }
+    };
+    const int r0 = (int)blockIdx.x * 1024 + tid;
+    request(r0);
+    if (wave < np) small_decide(A, wave, s_dec, s_tot, writer, lane, s_leaf);
+    for (int p = wave + 16; p < np; p += 16) small_decide(A, p, s_dec, s_tot, writer, lane, s_leaf);
+    __syncthreads();
+    finish(r0);
+    for (int r = r0 + (int)gridDim.x * 1024; r < A.N; r += (int)gridDim.x * 1024) {
+        request(r);
+        finish(r);
+    }
+    if constexpr (GRADS) {
+        __shared__ float s_m[16][2 * K];
+#pragma unroll
+        for (int k = 0; k < 2 * K; k++) {
+            const float m = wave_max_f32(mx[k]);
+            if (lane == 0) s_m[wave][k] = m;
+        }
+        __syncthreads();
+        if (tid < 2 * K) {
+            float m = s_m[0][tid];
+            for (int v = 1; v < 16; v++) m = fmaxf(m, s_m[v][tid]);
+            absmax_raise(A.maxima, tid, m);
+        }
     }
     if (!writer) return;
     if (A.slices > 1) {
@@ -983,7 +1054,28 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
             A.blob_src = reinterpret_cast<const uint4 *>(c->tree_blob);
             A.blob_dst = reinterpret_cast<uint4 *>(c->h_stage_dev);
             A.blob_n = (int64_t)(c->blob_bytes / 16);
-            hipLaunchKernelGGL(k_small_final, dim3((unsigned)((c->N + 1023) / 1024)), dim3(1024), (size_t)(1 << (level - 1)) * c->NAg * 8, c->stream, A);
+            // the next round's gradients are queued behind the tree (tree_close): of one target they are computed here
+            c->step.grads_done = c->grads_ahead && p->update_pred && p->bagging_size == 1 && !EVT_IS_QUANTILE(c->loss) && c->loss != EVT_LOSS_MLOGLOSS &&
+                                 c->K == (EVT_IS_MLE2P(c->loss) ? 2 : 1);
+            A.pred = c->pred;
+            A.y = c->y;
+            A.grad = c->grad;
+            A.maxima = absmax_set(c, c->absmax_cur);
+            A.unit_w = c->unit_w ? 1 : 0;
+            const size_t lds = (size_t)(1 << (level - 1)) * c->NAg * 8 + (c->step.grads_done ? (size_t)3 * (1 << (level - 2)) * c->K * 4 : 0);
+            // no more blocks than are resident at once: a second generation would take the decisions again
+#define FINAL(L_) hipLaunchKernelGGL(k_small_final<L_>, dim3((unsigned)std::min<int64_t>(256, (c->N + 1023) / 1024)), dim3(1024), lds, c->stream, A)
+            if (!c->step.grads_done) FINAL(-1);
+            else if (c->loss == EVT_LOSS_MSE) FINAL(0);
+            else if (c->loss == EVT_LOSS_LOGLOSS) FINAL(1);
+            else if (c->loss == EVT_LOSS_GAUSSIAN_MLE) FINAL(2);
+            else if (c->loss == EVT_LOSS_POISSON) FINAL(3);
+            else if (c->loss == EVT_LOSS_GAMMA) FINAL(4);
+            else if (c->loss == EVT_LOSS_TWEEDIE) FINAL(5);
+            else if (c->loss == EVT_LOSS_LOGISTIC_MLE) FINAL(7);
+            else if (c->loss == EVT_LOSS_MAE) FINAL(8);
+            else FINAL(9); // the credibility losses
+#undef FINAL
             prof_end(c);
             break;
         }

@@ -139,3 +139,62 @@ def test_gradients_quantised_by_the_tree_or_not(evt, N, B, loss, K):
             assert_tree_bits(a2, b)
             splits += int(a.split.sum())
     assert splits > 0
+
+
+@pytest.mark.parametrize("N,D,loss,more", [
+    (4, 2, "mse", {}),
+    (1025, 3, "mse", dict(weights=True, sub=True)),
+    (2049, 5, "logloss", {}),                          # a last block of one row
+    (1024, 4, "gaussian_mle", dict(weights=True)),
+    (3000, 6, "gaussian_mle", dict(oblivious=True)),
+    (1999, 4, "logistic_mle", dict(sub=True)),
+    (1500, 4, "poisson", {}),
+    (1500, 4, "gamma", dict(weights=True)),
+    (1500, 4, "tweedie", {}),
+    (1500, 4, "mae", dict(weights=True)),
+    (1500, 4, "cred_var", {}),
+    (1500, 4, "cred_std", dict(sub=True)),
+    (1500, 4, "mlogloss", {}),                         # several outputs: the gradient kernels of their own
+    (262_145, 4, "mse", dict(weights=True)),           # one row more than the last kernel's blocks take at once
+    (530_001, 3, "gaussian_mle", {}),
+    (5003, 10, "mse", dict(min_weight=40.0)),          # most leaves above the last level
+])
+def test_gradients_behind_the_tree(evt, N, D, loss, more):
+    """With "grads_ahead" a small tree's last kernel adds the leaf values and computes the next gradients: the bits that the kernels of larger inputs
+    and strictly alternating calls leave, also after a tree that keeps the predictions."""
+    F, B, K = 5, 32, 3
+    rng = np.random.default_rng(N + D)
+    if loss == "mlogloss":
+        x_bin = rng.integers(1, B + 1, size=(F, N), dtype=np.uint8)
+        y, mu, w = (1 + (x_bin[0].astype(int) + rng.integers(0, 2, N)) % K).astype(np.float32), np.zeros(K, np.float32), None
+    else:
+        x_bin, y, w, mu = make_data(N, N, F, B, loss, more.get("weights", False))
+    js = np.arange(1, F + 1, dtype=np.uint32)
+    args = dict(eta=0.4, min_weight=more.get("min_weight", 0.0 if N < 10 else 2.0), L2=1.0)
+    masks = [rng.integers(0, 256, N, dtype=np.uint8) for _ in range(5)]
+    out = []
+    for small, ahead in ((2, 1), (3, 1), (2, 0), (3, 0), (0, 1)):  # 2 is not taken above 65 535 rows
+        h = evt.Handle(N, F, B, len(mu), D, loss, "oblivious" if more.get("oblivious") else "binary")
+        h.set_option("small_tree", small)
+        h.set_option("grads_ahead", ahead)
+        h.set_xbin(x_bin)
+        h.set_target(y, w, mu)
+        rec = []
+        for r in range(5):
+            h.update_grads()
+            gp = evt.make_params(update_pred=r != 3, **args)
+            rec.append(h.grow_tree(js, gp, mask=masks[r] if more.get("sub") else None, cond=150))
+            rec.append(h.get_hist())
+            if r % 2:
+                rec.append(h.get_pred())
+        h.update_grads()
+        rec += [h.get_grads(), np.concatenate(h.get_quant()), h.get_pred()]
+        h.close()
+        out.append(rec)
+    for a in out[1:]:
+        for one, other in zip(out[0], a):
+            if isinstance(one, np.ndarray):
+                assert one.tobytes() == other.tobytes()
+            else:
+                assert_tree_bits(one, other)
+    assert sum(int(t.split.sum()) for t in out[0] if not isinstance(t, np.ndarray)) > 0 or N < 10
