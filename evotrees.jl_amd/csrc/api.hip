@@ -747,9 +747,9 @@ static int queue_grads(evt_ctx *c) {
     prof_end(c);
     if (r != EVT_OK) return r;
     if (c->profiling) c->prof_units[EVT_K_GRAD] += c->N;
-    // a tree of the kernels for small inputs quantises on its way: the next one is taken to be like the last (tree_open knows)
+    // a tree quantises on its way: inside its first kernel, or beside its set-up
     c->quant_pending = true;
-    if (small_tree_form(c, c->n_js_last > 0 ? c->n_js_last : c->F, c->n_js_last == 0 || c->last_all_rows)) return EVT_OK;
+    if (c->N <= EVT_QUANT_LATER) return EVT_OK;
     prof_begin(c, EVT_K_OTHER, 0);
     r = launch_quantize(c);
     prof_end(c);
@@ -845,7 +845,7 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
     const int small = staged ? 0 : small_tree_form(c, n_js, all_rows);
     int r = EVT_OK;
     if (c->quant_pending) {
-        if (small) quant_set(c); // by the tree's first kernel
+        if (small || c->N <= EVT_QUANT_LATER) quant_set(c); // by the tree's first kernel
         else r = launch_quantize(c);
         if (r != EVT_OK) return r;
     }

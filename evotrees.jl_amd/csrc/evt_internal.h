@@ -30,6 +30,8 @@
 #define EVT_MC_MAX_NK 40 // >= 2 * EVT_MAX_K + 1: sizes of the per-row quantisation tables and of the generic kernels' arrays
 #define EVT_HIST_GROUP 4 // accumulator channels one histogram block handles; more channels are layers of the launch
 #define EVT_OBLIV_BLOCKS 256 // blocks of the search for an oblivious level's best cell
+// rows up to which the gradients are quantised by the next tree's first kernel; more are quantised at once, while the host collects the tree before
+#define EVT_QUANT_LATER ((int64_t)4 << 20)
 #define EVT_METRIC_BLOCKS 1024 // partial sums of the evaluation metric
 #define EVT_MAX_DEPTH 16
 #define EVT_MAX_FEATS 65534 // a feature's slot in the column sample is a 16-bit word, 0xFFFF = not sampled
@@ -165,7 +167,7 @@ struct evt_ctx {
     int32_t *qexp_buf[2];
     double *qscale_buf[2];
     int q_cur, q_tree;
-    bool quant_pending;  // the gradients' fixed-point words are still to be made: by the first kernel of a small tree, or by k_quantize
+    bool quant_pending;  // the gradients' fixed-point words are still to be made: by the next tree's first kernel, or by k_quantize
     double *metric_partial; // [2 * EVT_METRIC_BLOCKS + 1] evaluation-metric partial sums, then how many blocks have left theirs (zero between launches)
     int64_t *stats;    // [D+1] rows built per level
     int32_t *errflag;  // device-side validation flag

@@ -121,3 +121,76 @@ __device__ __forceinline__ int quant_exponent(const uint32_t *__restrict__ absma
 }
 // gradient row of global channel ag: one-target mse / mae have {g, w}, otherwise the rows as they are
 __device__ __forceinline__ int quant_row(int loss, int K, int ag) { return EVT_TWO_CHAN(loss, K) && ag == 1 ? 2 : ag; }
+
+// lanes that share a row's channels, as a power of two (60k rows of 14 channels, set-up and quantisation in one launch: one lane a row 11.7 us,
+// four 9.3)
+__host__ __device__ inline int quant_lanes_sh(int na) { return na > EVT_MAX_NA ? 2 : 0; }
+
+struct QuantArgs {
+    const float *grad;
+    unsigned long long *gq;
+    int64_t N;
+    int NK, NA, NAg, loss, two, unit_w, pack, pack_wide;
+    const uint32_t *absmax;
+    uint32_t *absmax_next;
+    const int32_t *qbits;
+    int32_t *qexp;
+    double *qscale; // decode scales per global channel, then EVT_MC_MAX_NK on the multipliers per gradient row
+};
+void quant_args(evt_ctx *c, QuantArgs &Q);             // behind quant_set
+unsigned quant_blocks(const evt_ctx *c, int threads);
+void quant_taken(evt_ctx *c);                          // behind the launch
+
+// Quantisation tables of a gradient pass and the fixed-point words the histogram kernel adds, in one pass.
+// qexp[k] = ilogb(max |row k|) + 1 (0 for an all-zero row); qmul[k] = 2^(qbits - qexp) encodes, qscale decodes.  Every block
+// derives the multipliers from the striped maxima itself (a few dozen cached loads: no kernel of its own in front of this one);
+// block 0 also writes the tables for the readers that follow (split search, read-back).  The maxima live in two sets: a
+// gradient pass raises one, this kernel reads it and clears the other - which nobody uses at that moment - for the next pass,
+// so no pass starts from maxima an earlier one left behind.  The weight row (last) is written once and keeps its maximum.
+// Plane a of gq holds, per row, q = rint(v * 2^(qbits - qexp)) of gradient row chan_k[a]; with unit weights plane 0 also carries
+// the row count in its low 16 bits ((q << 16) + 1) so that one 64-bit LDS add serves both.
+// Channel a reads gradient row a, except for mse whose channels are {g, w} = rows {0, 2}.
+// `block` of `blocks`: of a kernel of its own, or of one that sets a tree up meanwhile (kernels_part.hip).
+__device__ __forceinline__ void quant_rows(const QuantArgs &Q, int block, int blocks) {
+    __shared__ double s_qmul[EVT_MC_MAX_NK];
+    __shared__ int s_qexp[EVT_MC_MAX_NK], s_qbits[EVT_MC_MAX_NK];
+    const int t = threadIdx.x, nthr = blockDim.x, NK = Q.NK;
+    if (t < NK) {
+        const int e = quant_exponent(Q.absmax, t);
+        const int qb = Q.qbits[t];
+        s_qexp[t] = e;
+        s_qbits[t] = qb;
+        s_qmul[t] = scalbn(1.0, qb - e);
+    }
+    __syncthreads();
+    if (block == 0) {
+        if (t < NK) {
+            Q.qexp[t] = s_qexp[t];
+            Q.qscale[EVT_MC_MAX_NK + t] = s_qmul[t];
+            if (t < NK - 1)
+                for (int st = 0; st < EVT_ABSMAX_STRIPES; st++) Q.absmax_next[st * EVT_MC_MAX_NK + t] = 0u;
+        }
+        if (t < Q.NAg) {
+            const int kk = quant_row(Q.loss, (NK - 1) / 2, t); // the last channel is w (or the row count)
+            if (t == Q.NAg - 1 && Q.unit_w) Q.qscale[t] = 1.0;
+            else Q.qscale[t] = scalbn(1.0, s_qexp[kk] - s_qbits[kk]);
+        }
+    }
+    // a block takes many rows (grid-stride), so that the prologue above is paid a couple of thousand times, not once per 256 rows
+    const int sh = quant_lanes_sh(Q.NA), part = t & ((1 << sh) - 1);
+    for (int64_t w = (int64_t)block * nthr + t; w < Q.N << sh; w += (int64_t)blocks * nthr) {
+        const int64_t i = w >> sh;
+        const float *g = Q.grad + (size_t)NK * i;
+#pragma unroll 5
+        for (int a = part; a < Q.NA; a += 1 << sh) { // several channels' words in flight
+            const int k = (Q.two && a == 1) ? 2 : a;
+            long long q = __double2ll_rn((double)g[k] * s_qmul[k]);
+            if (a == 0 && Q.pack) { // 30 bits: staged as a 32-bit word, widened to (q << 16) + 1 (the row count) by the histogram kernel
+                reinterpret_cast<int32_t *>(Q.gq)[i] = (int32_t)q;
+                continue;
+            }
+            if (a == 0 && Q.pack_wide) q = (long long)(((unsigned long long)q << EVT_PACK_CNT_BITS) + 1ull); // the same word, for kernels that read every channel alike
+            Q.gq[(size_t)a * Q.N + i] = (unsigned long long)q;
+        }
+    }
+}

@@ -253,59 +253,8 @@ __global__ __launch_bounds__(256) void k_absmax(const float *__restrict__ grad, 
     }
 }
 
-// Quantisation tables of a gradient pass and the fixed-point words the histogram kernel adds, in one kernel.
-// qexp[k] = ilogb(max |row k|) + 1 (0 for an all-zero row); qmul[k] = 2^(qbits - qexp) encodes, qscale decodes.  Every block
-// derives the multipliers from the striped maxima itself (a few dozen cached loads: no kernel of its own in front of this one);
-// block 0 also writes the tables for the readers that follow (split search, read-back).  The maxima live in two sets: a
-// gradient pass raises one, this kernel reads it and clears the other - which nobody uses at that moment - for the next pass,
-// so no pass starts from maxima an earlier one left behind.  The weight row (last) is written once and keeps its maximum.
-// Plane a of gq holds, per row, q = rint(v * 2^(qbits - qexp)) of gradient row chan_k[a]; with unit weights plane 0 also carries
-// the row count in its low 16 bits ((q << 16) + 1) so that one 64-bit LDS add serves both.
-// Channel a reads gradient row a, except for mse whose channels are {g, w} = rows {0, 2}.
-__global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ grad, unsigned long long *__restrict__ gq, int64_t N,
-                                                 int NK, int NA, int mse, int pack, int pack_wide, const uint32_t *__restrict__ absmax, uint32_t *absmax_next,
-                                                 const int32_t *__restrict__ qbits, int32_t *qexp, double *qmul, double *qscale_g, int NAg,
-                                                 int loss, int unit_w) {
-    __shared__ double s_qmul[EVT_MC_MAX_NK];
-    __shared__ int s_qexp[EVT_MC_MAX_NK], s_qbits[EVT_MC_MAX_NK];
-    const int t = threadIdx.x;
-    if (t < NK) {
-        const int e = quant_exponent(absmax, t);
-        const int qb = qbits[t];
-        s_qexp[t] = e;
-        s_qbits[t] = qb;
-        s_qmul[t] = scalbn(1.0, qb - e);
-    }
-    __syncthreads();
-    if (blockIdx.x == 0) {
-        if (t < NK) {
-            qexp[t] = s_qexp[t];
-            qmul[t] = s_qmul[t];
-            if (t < NK - 1)
-                for (int st = 0; st < EVT_ABSMAX_STRIPES; st++) absmax_next[st * EVT_MC_MAX_NK + t] = 0u;
-        }
-        if (t < NAg) {
-            const int kk = quant_row(loss, (NK - 1) / 2, t); // the last channel is w (or the row count)
-            if (t == NAg - 1 && unit_w) qscale_g[t] = 1.0;
-            else qscale_g[t] = scalbn(1.0, s_qexp[kk] - s_qbits[kk]);
-        }
-    }
-    // a block takes many rows (grid-stride), so that the prologue above is paid a couple of thousand times, not once per 256 rows
-    for (int64_t i = (int64_t)blockIdx.x * 256 + t; i < N; i += (int64_t)gridDim.x * 256) {
-        const float *g = grad + (size_t)NK * i;
-#pragma unroll 5
-        for (int a = 0; a < NA; a++) { // several channels' words in flight
-            const int k = (mse && a == 1) ? 2 : a;
-            long long q = __double2ll_rn((double)g[k] * s_qmul[k]);
-            if (a == 0 && pack) { // 30 bits: staged as a 32-bit word, widened to (q << 16) + 1 (the row count) by the histogram kernel
-                reinterpret_cast<int32_t *>(gq)[i] = (int32_t)q;
-                continue;
-            }
-            if (a == 0 && pack_wide) q = (long long)(((unsigned long long)q << EVT_PACK_CNT_BITS) + 1ull); // the same word, for kernels that read every channel alike
-            gq[(size_t)a * N + i] = (unsigned long long)q;
-        }
-    }
-}
+// The quantisation as a kernel of its own (quant_rows)
+__global__ __launch_bounds__(256) void k_quantize(QuantArgs Q) { quant_rows(Q, blockIdx.x, gridDim.x); }
 
 // the set of striped maxima the next gradient pass raises (and the quantisation behind it reads)
 uint32_t *absmax_set(evt_ctx *c, int which) { return c->absmax + (size_t)which * EVT_ABSMAX_STRIPES * EVT_MC_MAX_NK; }
@@ -434,18 +383,41 @@ void quant_set(evt_ctx *c) {
     c->qscale = c->qscale_buf[c->q_cur];
 }
 
+void quant_args(evt_ctx *c, QuantArgs &Q) {
+    Q.grad = c->grad;
+    Q.gq = c->gq;
+    Q.N = c->N;
+    Q.NK = c->NK; Q.NA = c->NA; Q.NAg = c->NAg; Q.loss = c->loss;
+    Q.two = EVT_TWO_CHAN(c->loss, c->K) ? 1 : 0;
+    Q.unit_w = c->unit_w ? 1 : 0;
+    Q.pack = (c->unit_w && c->NA <= EVT_MAX_NA) ? 1 : 0;
+    Q.pack_wide = (c->unit_w && c->NA > EVT_MAX_NA) ? 1 : 0;
+    Q.absmax = absmax_set(c, c->absmax_cur);
+    Q.absmax_next = absmax_set(c, c->absmax_cur ^ 1);
+    Q.qbits = c->qbits;
+    Q.qexp = c->qexp;
+    Q.qscale = c->qscale;
+}
+
+// Blocks of `threads` that quantise.  Every block derives the multipliers first: fewer where a row is one word (1M rows, at most 1024 | 4096 blocks of
+// 256: 5.4 | 6.5 us; four words a row at 500k rows 7.8 | 6.9, one word at 10M 27.6 | 25.5)
+unsigned quant_blocks(const evt_ctx *c, int threads) {
+    const int64_t most = (c->NA == 1 && c->N <= (int64_t)4 << 20 ? 1024 : 4096) * 256 / threads;
+    return (unsigned)std::min<int64_t>(most, ((c->N << quant_lanes_sh(c->NA)) + threads - 1) / threads);
+}
+
+void quant_taken(evt_ctx *c) {
+    c->quant_pending = false;
+    c->absmax_cur ^= 1; // the next gradient pass raises the set that the quantisation cleared
+}
+
 int launch_quantize(evt_ctx *c) {
     quant_set(c);
-    c->quant_pending = false;
-    double *qmul = c->qscale + EVT_MC_MAX_NK; // decode scales per global channel first, then encode multipliers per gradient row
-    // every block derives the multipliers first: fewer blocks where a row is one word (1M rows, at most 1024 | 4096 blocks: 5.4 | 6.5 us; four words
-    // a row at 500k rows 7.8 | 6.9, one word at 10M 27.6 | 25.5)
-    const int64_t blocks = c->NA == 1 && c->N <= (int64_t)4 << 20 ? 1024 : 4096;
-    hipLaunchKernelGGL(k_quantize, dim3((unsigned)std::min<int64_t>(blocks, (c->N + 255) / 256)), dim3(256), 0, c->stream, c->grad, c->gq, c->N, c->NK, c->NA,
-                       EVT_TWO_CHAN(c->loss, c->K) ? 1 : 0, (c->unit_w && c->NA <= EVT_MAX_NA) ? 1 : 0, (c->unit_w && c->NA > EVT_MAX_NA) ? 1 : 0, absmax_set(c, c->absmax_cur), absmax_set(c, c->absmax_cur ^ 1),
-                       c->qbits, c->qexp, qmul, c->qscale, c->NAg, c->loss, c->unit_w ? 1 : 0);
+    QuantArgs Q;
+    quant_args(c, Q);
+    hipLaunchKernelGGL(k_quantize, dim3(quant_blocks(c, 256)), dim3(256), 0, c->stream, Q);
     HIPCHK(hipGetLastError());
-    c->absmax_cur ^= 1; // the next gradient pass raises the set this kernel cleared
+    quant_taken(c);
     return EVT_OK;
 }
 

@@ -16,7 +16,7 @@
 // the next level's tables (active nodes, chunk prefix, build list).  It rides in the kernel that moves the rows; two passes
 // over thousands of chunks scan the counts in a kernel of its own before the scatter.
 // No host round trip is needed between levels.
-#include "evt_internal.h"
+#include "grad_math.h"
 #include <algorithm>
 
 // largest i in [0, n) with pre[i] <= v   (pre ascending, pre[0] <= v): the number of such entries, less one.  Every
@@ -860,11 +860,18 @@ __device__ void tree_begin_block(BeginArgs A) {
 }
 
 // The root's slice, shared by the kernel's blocks: one block took 26 us for 212 000 words (166 features, five channels, 255 bins).
-__device__ void tree_begin_root(const BeginArgs &A) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < A.root_words; i += (int64_t)gridDim.x * blockDim.x) A.hist[i] = 0;
+__device__ void tree_begin_root(const BeginArgs &A, int blocks) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < A.root_words; i += (int64_t)blocks * blockDim.x) A.hist[i] = 0;
 }
-__global__ __launch_bounds__(1024) void k_tree_begin(BeginArgs A) {
-    tree_begin_root(A);
+// Blocks from `blocks` on quantise the gradients, which have nothing to do with the set-up: side by side in one launch where the gradients' words are
+// still to be made: set-up + quantisation, us, 500k rows of four channels 4.2 + 6.9 -> 7.0, 60k of 14 channels 3.0 + 7.9 -> 9.3; mask count +
+// quantisation, 1M rows 3.1 + 5.8 -> 6.3, of two channels 3.2 + 7.5 -> 8.7 - and a launch each.
+__global__ __launch_bounds__(1024) void k_tree_begin(BeginArgs A, QuantArgs Q, int blocks) {
+    if ((int)blockIdx.x >= blocks) {
+        quant_rows(Q, (int)blockIdx.x - blocks, (int)gridDim.x - blocks);
+        return;
+    }
+    tree_begin_root(A, blocks);
     if (blockIdx.x == 0) tree_begin_block(A);
 }
 
@@ -883,12 +890,16 @@ __device__ __forceinline__ int wave_sum_i32(int v) {
 // draw of its own generator per tree.
 template <bool DRAW>
 __global__ __launch_bounds__(256) void k_mask_count(uint8_t *mask, uint8_t cond, int64_t N, int64_t n_chunks,
-                                                   unsigned long long *flagw, int32_t *chunk_nleft, unsigned long long seed) {
+                                                   unsigned long long *flagw, int32_t *chunk_nleft, unsigned long long seed, QuantArgs Q, int blocks) {
+    if ((int)blockIdx.x >= blocks) { // as k_tree_begin
+        quant_rows(Q, (int)blockIdx.x - blocks, (int)gridDim.x - blocks);
+        return;
+    }
     static_assert(EVT_CHUNK == 2048 && EVT_CHUNK_WORDS == 32, "a chunk is 256 threads x 8 bytes");
     const int tid = threadIdx.x;
     __shared__ unsigned long long s_w[EVT_CHUNK_WORDS];
     uint8_t *s_b = reinterpret_cast<uint8_t *>(s_w);
-    for (int64_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
+    for (int64_t c = blockIdx.x; c < n_chunks; c += blocks) {
         const int64_t p0 = c * EVT_CHUNK + (int64_t)tid * 8;
         unsigned long long v = ~0ull; // bytes past the end read as 255
         if (DRAW) {
@@ -950,7 +961,7 @@ __global__ __launch_bounds__(256) void k_mask_scatter(int64_t N, int64_t n_chunk
     __shared__ int s_pre[EVT_CHUNK_WORDS];
     __shared__ int s_sum[4];
     const int64_t G = (int64_t)gridDim.x - 1;
-    tree_begin_root(B);
+    tree_begin_root(B, (int)gridDim.x);
     if ((int64_t)blockIdx.x == G) {
         int64_t kept;
         if (SELF) { // no scan has run: the chunk counts (a thousand at most) are added up here
@@ -1048,8 +1059,16 @@ static void fill_begin_args(evt_ctx *c, bool all_rows, BeginArgs &A) {
 int launch_tree_begin(evt_ctx *c) {
     BeginArgs A;
     fill_begin_args(c, true, A);
-    hipLaunchKernelGGL(k_tree_begin, dim3((unsigned)std::min<int64_t>(1 + A.root_words / 4096, 64)), dim3(1024), 0, c->stream, A);
+    QuantArgs Q = {};
+    const unsigned blocks = (unsigned)std::min<int64_t>(1 + A.root_words / 4096, 64);
+    unsigned quant = 0;
+    if (c->quant_pending) {
+        quant_args(c, Q);
+        quant = quant_blocks(c, 1024);
+    }
+    hipLaunchKernelGGL(k_tree_begin, dim3(blocks + quant), dim3(1024), 0, c->stream, A, Q, (int)blocks);
     HIPCHK(hipGetLastError());
+    if (quant) quant_taken(c);
     c->js_staged = false;
     return EVT_OK;
 }
@@ -1059,9 +1078,16 @@ int launch_tree_begin(evt_ctx *c) {
 int launch_compact_mask(evt_ctx *c, uint8_t cond, bool draw, unsigned long long seed) {
     const int64_t n_chunks = (c->N + EVT_CHUNK - 1) / EVT_CHUNK;
     unsigned g = grid_for_chunks(n_chunks);
-    if (draw) hipLaunchKernelGGL(k_mask_count<true>, dim3(g), dim3(256), 0, c->stream, c->mask, cond, c->N, n_chunks, c->flagw, c->chunk_nleft, seed);
-    else hipLaunchKernelGGL(k_mask_count<false>, dim3(g), dim3(256), 0, c->stream, c->mask, cond, c->N, n_chunks, c->flagw, c->chunk_nleft, 0ull);
+    QuantArgs Q = {};
+    unsigned quant = 0;
+    if (c->quant_pending) {
+        quant_args(c, Q);
+        quant = quant_blocks(c, 256);
+    }
+    if (draw) hipLaunchKernelGGL(k_mask_count<true>, dim3(g + quant), dim3(256), 0, c->stream, c->mask, cond, c->N, n_chunks, c->flagw, c->chunk_nleft, seed, Q, (int)g);
+    else hipLaunchKernelGGL(k_mask_count<false>, dim3(g + quant), dim3(256), 0, c->stream, c->mask, cond, c->N, n_chunks, c->flagw, c->chunk_nleft, 0ull, Q, (int)g);
     HIPCHK(hipGetLastError());
+    if (quant) quant_taken(c);
     BeginArgs B;
     fill_begin_args(c, false, B);
     if (n_chunks <= 1024) { // the scatter's blocks add up the counts before their chunk themselves

@@ -1127,8 +1127,7 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
         prof_end(c);
         HIPCHK(hipGetLastError());
         if (c->quant_pending) { // made by the root's kernel, which cleared the set that the next gradient pass raises
-            c->quant_pending = false;
-            c->absmax_cur ^= 1;
+            quant_taken(c);
         }
     }
     HIPCHK(hipGetLastError());

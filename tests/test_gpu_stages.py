@@ -163,3 +163,47 @@ def test_stage_order_is_enforced(evt):
     assert_tree_bits(t_steps, t_one)
     h.close()
     o.close()
+
+
+@pytest.mark.parametrize("N,loss,K,weights,sub", [
+    (3, "mse", 1, False, None), (255, "mse", 1, True, "mask"), (2049, "logloss", 1, False, "drawn"), (1023, "gaussian_mle", 2, True, None),
+    (70_001, "gaussian_mle", 2, False, "drawn"), (1021, "mlogloss", 7, True, "mask"), (4097, "mlogloss", 3, False, None), (5000, "mlogloss", 16, True, None),
+])
+def test_quantised_beside_the_tree_set_up(evt, N, loss, K, weights, sub):
+    """The gradients' words come from blocks of the kernel that sets the tree up, or from k_quantize where the tables are asked for first: same bits,
+    in the first tree and in one behind it."""
+    F, B, D = 5, 24, 4
+    rng = np.random.default_rng(N)
+    x_bin = rng.integers(1, B + 1, size=(F, N), dtype=np.uint8)
+    if loss == "mlogloss":
+        y = (1 + (x_bin[0].astype(int) + rng.integers(0, 2, N)) % K).astype(np.float32)
+    elif loss == "logloss":
+        y = (rng.random(N) < 0.4).astype(np.float32)
+    else:
+        y = (x_bin[0] / np.float32(B) + rng.random(N, dtype=np.float32)).astype(np.float32)
+    w = (rng.random(N) + 0.5).astype(np.float32) if weights else None
+    js = np.arange(1, F + 1, dtype=np.uint32)
+    gp = evt.make_params(eta=0.3, L2=1.0, min_weight=0.0)
+    mask = rng.integers(0, 256, N, dtype=np.uint8)
+    out = []
+    for first in (False, True):
+        h = evt.Handle(N, F, B, K, D, loss)
+        h.set_option("small_tree", 0)
+        h.set_xbin(x_bin)
+        h.set_target(y, w, np.zeros(K, np.float32))
+        rec = []
+        for r in range(2):
+            h.update_grads()
+            if first:
+                h.get_quant()
+            if sub == "drawn":
+                h.draw_mask(r + 1)
+                h.grow_tree_begin_staged(js, gp, 150)
+                t = h.grow_tree_end()
+            else:
+                t = h.grow_tree(js, gp, mask=mask if sub else None, cond=150)
+            rec += [t.feat, t.cond_bin, t.split, t.gain, t.pred, t.w, h.get_hist(), np.concatenate(h.get_quant()), h.get_pred(), h.get_grads()]
+        h.close()
+        out.append(rec)
+    for a, b in zip(*out):
+        assert a.tobytes() == b.tobytes()
