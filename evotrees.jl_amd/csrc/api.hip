@@ -1,5 +1,5 @@
 // C ABI of libevotrees_hip.so: handle lifecycle, uploads, the per-tree level loop, read-back.
-#include "evt_internal.h"
+#include "grad_math.h"
 #include "upload.h"
 
 #include <stdarg.h>
@@ -1014,7 +1014,7 @@ static int tree_close(evt_ctx *c) {
     if (p->update_pred && !all_rows && !c->step.small) {
         // rows outside the sample are predicted too (src/fit.jl:37): walk the new tree for all rows
         prof_begin(c, EVT_K_PREDICT, 0);
-        r = launch_predict_tree_cache(c, true); // with the tree's transfer to the host in its last blocks
+        r = launch_predict_tree_cache(c, true, grads_with_tree(c, p)); // with the tree's transfer to the host in its last blocks
         prof_end(c);
         if (r != EVT_OK) return r;
         if (c->profiling) c->prof_units[EVT_K_PREDICT] += c->N;
@@ -1035,8 +1035,12 @@ static int tree_close(evt_ctx *c) {
         // the next round's gradient update runs while the host collects this tree and prepares the next call.  Not with
         // bagging: the trees of one round are all grown on the same gradients (src/fit.jl:9-11), and the library cannot
         // tell which call is the round's last.
-        if (c->step.grads_done) c->quant_pending = true; // by the tree's last kernel
-        else r = queue_grads(c);
+        if (c->step.grads_done) { // by the tree's last kernel
+            c->quant_pending = true;
+            if (c->N > EVT_QUANT_LATER) r = launch_quantize(c);
+        } else {
+            r = queue_grads(c);
+        }
         if (r != EVT_OK) return r;
         c->grads_ready = true;
     }

@@ -386,7 +386,7 @@ int launch_copy_words(evt_ctx *c, const void *src, void *dst, size_t nbytes);
 int launch_fill_u32(evt_ctx *c, uint32_t *dst, uint32_t v, int64_t n);
 int launch_fill_bytes(evt_ctx *c, void *dst, int64_t nbytes);
 // predict
-int launch_predict_tree_cache(evt_ctx *c, bool send_blob);
+int launch_predict_tree_cache(evt_ctx *c, bool send_blob, bool grads);
 int launch_hist_export(evt_ctx *c, double *out_dev);
 int launch_nidx_from_tree(evt_ctx *c, bool use_mask, uint8_t cond);
 

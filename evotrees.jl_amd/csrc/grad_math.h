@@ -59,6 +59,23 @@ __device__ __forceinline__ void absmax_raise(uint32_t *absmax, int k, float m) {
     if (__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < u) atomicMax(p, u);
 }
 
+// Raises the maxima by those of a block, a thread's in mx; s_m: a row of the block's wavefronts (16 at most)
+template <int ROWS>
+__device__ __forceinline__ void absmax_raise_block(const float *mx, float (*s_m)[ROWS], uint32_t *absmax) {
+#pragma unroll
+    for (int k = 0; k < ROWS; k++) {
+        const float m = wave_max_f32(mx[k]);
+        if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6][k] = m;
+    }
+    __syncthreads();
+    if (threadIdx.x < ROWS) {
+        const int k = threadIdx.x;
+        float m = s_m[0][k];
+        for (int w = 1; w < (int)blockDim.x >> 6; w++) m = fmaxf(m, s_m[w][k]);
+        absmax_raise(absmax, k, m);
+    }
+}
+
 // LOSS: 0 mse (src/loss.jl:52), 1 logloss (:54-57), 2 gaussian_mle (:194-203), 3 poisson (:59-62),
 // 4 gamma (:64-67), 5 tweedie with rho = 1.5 (:69-76), 8 mae (:78), 9 cred_var / cred_std (:80-83).
 // pr: the row's outputs (two of an MLE loss); out: g, then h of each, times the row's weight.
@@ -101,6 +118,29 @@ __device__ __forceinline__ void grad_row(const float *pr, float y, float w, floa
         out[3] = h2 * w;
     }
 }
+
+// grad_row's LOSS for the gradients of a handle, -1 where they are not those of one target
+inline int grad_row_loss(const evt_ctx *c) {
+    if (EVT_IS_QUANTILE(c->loss) || c->loss == EVT_LOSS_MLOGLOSS || c->K != (EVT_IS_MLE2P(c->loss) ? 2 : 1)) return -1;
+    return EVT_IS_CRED(c->loss) ? 9 : c->loss;
+}
+// A tree's last kernel computes the next round's gradients: those that would be queued behind the tree (tree_close), of one target
+inline bool grads_with_tree(const evt_ctx *c, const evt_params *p) {
+    return c->grads_ahead && p->update_pred && p->bagging_size == 1 && grad_row_loss(c) >= 0;
+}
+// LAUNCH(LOSS) for the handle's loss
+#define EVT_GRAD_ROW_CASES(c, LAUNCH) \
+    switch (grad_row_loss(c)) {       \
+    case 0: LAUNCH(0); break;         \
+    case 1: LAUNCH(1); break;         \
+    case 2: LAUNCH(2); break;         \
+    case 3: LAUNCH(3); break;         \
+    case 4: LAUNCH(4); break;         \
+    case 5: LAUNCH(5); break;         \
+    case 7: LAUNCH(7); break;         \
+    case 8: LAUNCH(8); break;         \
+    default: LAUNCH(9); break;        \
+    }
 
 // Exponent of gradient row t for its fixed-point words: ilogb(max |row t|) + 1, 0 for an all-zero row, from the striped maxima of one pass.
 __device__ __forceinline__ int quant_exponent(const uint32_t *__restrict__ absmax, int t) {

@@ -55,18 +55,7 @@ __global__ __launch_bounds__(1024) void k_grads(float *__restrict__ pred, const 
     // per gradient row max |v| -> exponent bound of the fixed-point histogram.
     // One atomic per block and row: contended same-address atomics serialise in L2.
     __shared__ float s_m[16][2 * K];
-#pragma unroll
-    for (int k = 0; k < 2 * K; k++) {
-        const float m = wave_max_f32(mx[k]);
-        if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6][k] = m;
-    }
-    __syncthreads();
-    if (threadIdx.x < 2 * K) {
-        const int k = threadIdx.x;
-        float m = s_m[0][k];
-        for (int w = 1; w < (int)blockDim.x >> 6; w++) m = fmaxf(m, s_m[w][k]);
-        absmax_raise(absmax, k, m);
-    }
+    absmax_raise_block<2 * K>(mx, s_m, absmax);
 }
 
 // Several targets at once (y is T x N, one column per row of data; src/loss.jl:49-50, :100-111, :219-236): the same

@@ -4,7 +4,7 @@
 // visited node costs one 4-byte load and nothing else has to be looked up.  Rows are independent; per row the
 // walk reads one bin byte per level, from the column-major x_bin (neighbouring rows share 64-byte sectors of
 // a column) or, in the whole-model kernel, from a copy of the block's rows in LDS.
-#include "evt_internal.h"
+#include "grad_math.h"
 #include <algorithm>
 
 __device__ __forceinline__ int walk_packed(const uint32_t *__restrict__ nodes, const uint8_t *__restrict__ xcm, int64_t N, int64_t i) {
@@ -27,26 +27,49 @@ __device__ __forceinline__ int walk_packed(const uint32_t *__restrict__ nodes, c
 // the bytes it moves: the first n_lds node words (the upper levels of the heap, all of it for depths up to 13) are copied to
 // LDS, where a lookup costs a fraction of a trip to the caches, and a thread walks R rows side by side - R bin bytes are
 // requested before the first is used.  Rows of a thread are 256 apart: the threads of a wavefront read neighbouring bytes.
-template <int R>
-__global__ __launch_bounds__(256) void k_predict_tree(const uint32_t *__restrict__ nodes, int n_lds, const float *__restrict__ leaf_pred,
+// LOSS >= 0: the next round's gradients are computed as well, as k_grads<LOSS> would from the predictions it read again; what they need is requested
+// ahead of the walk (walk + gradients, us: 1M rows, depth 6 9.8 + 5.8 and a launch -> 11.8; 1M rows, depth 8 10.9 + 5.5 -> 14.2).
+struct GradOut {
+    const float *y;
+    float *grad;
+    uint32_t *absmax;
+    int unit_w;
+};
+template <int R, int LOSS>
+__global__ __launch_bounds__(LOSS < 0 ? 256 : 1024) void k_predict_tree(const uint32_t *__restrict__ nodes, int n_lds, const float *__restrict__ leaf_pred,
                                                      const uint8_t *__restrict__ xcm, int64_t N, int K, int loss, float *pred,
                                                      const uint4 *__restrict__ copy_src, uint4 *__restrict__ copy_dst, int64_t copy_n,
-                                                     int copy_blocks) {
+                                                     int copy_blocks, GradOut O) {
     extern __shared__ uint32_t s_nodes[];
+    constexpr bool GRADS = LOSS >= 0;
+    constexpr int KG = LOSS == 2 || LOSS == 7 ? 2 : 1, NKG = 2 * KG + 1;
+    const int nthr = GRADS ? (int)blockDim.x : 256;
     const int64_t G = (int64_t)gridDim.x - copy_blocks;
     if ((int64_t)blockIdx.x >= G) {
-        for (int64_t k = ((int64_t)blockIdx.x - G) * 256 + threadIdx.x; k < copy_n; k += (int64_t)copy_blocks * 256) copy_dst[k] = copy_src[k];
+        for (int64_t k = ((int64_t)blockIdx.x - G) * nthr + threadIdx.x; k < copy_n; k += (int64_t)copy_blocks * nthr) copy_dst[k] = copy_src[k];
         return;
     }
-    for (int k = threadIdx.x; k < n_lds; k += 256) s_nodes[k] = nodes[k];
+    const int64_t i0 = (int64_t)blockIdx.x * (nthr * R) + threadIdx.x;
+    float pr[R][KG], y[R], w[R];
+    if constexpr (GRADS) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int64_t i = i0 + nthr * r < N ? i0 + nthr * r : N - 1;
+#pragma unroll
+            for (int k = 0; k < KG; k++) pr[r][k] = pred[(size_t)KG * i + k];
+            y[r] = O.y[i];
+            w[r] = 1.0f;
+            if (!O.unit_w) w[r] = O.grad[(size_t)NKG * i + NKG - 1];
+        }
+    }
+    for (int k = threadIdx.x; k < n_lds; k += nthr) s_nodes[k] = nodes[k];
     __syncthreads();
-    const int64_t i0 = (int64_t)blockIdx.x * (256 * R) + threadIdx.x;
     int nid[R];
     uint32_t nd[R];
 #pragma unroll
     for (int r = 0; r < R; r++) {
         nid[r] = 1;
-        nd[r] = (i0 + 256 * r < N) ? s_nodes[0] : 0u; // a row past the end walks nothing
+        nd[r] = (i0 + nthr * r < N) ? s_nodes[0] : 0u; // a row past the end walks nothing
     }
     for (;;) {
         uint32_t xb[R];
@@ -55,7 +78,7 @@ __global__ __launch_bounds__(256) void k_predict_tree(const uint32_t *__restrict
         for (int r = 0; r < R; r++) {
             xb[r] = 0;
             if (nd[r] & EVT_NODE_SPLIT) {
-                xb[r] = xcm[(size_t)((nd[r] & 0xFFFFu) - 1) * N + (i0 + 256 * r)];
+                xb[r] = xcm[(size_t)((nd[r] & 0xFFFFu) - 1) * N + (i0 + nthr * r)];
                 any = true;
             }
         }
@@ -70,25 +93,68 @@ __global__ __launch_bounds__(256) void k_predict_tree(const uint32_t *__restrict
             }
         }
     }
+    if constexpr (GRADS) {
+        __shared__ float s_m[16][2 * KG];
+        float mx[2 * KG];
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int64_t i = i0 + 256 * r;
-        if (i < N) evt_add_leaf(pred + (size_t)K * i, leaf_pred + (size_t)K * (nid[r] - 1), K, loss);
+        for (int k = 0; k < 2 * KG; k++) mx[k] = 0.0f;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int64_t i = i0 + nthr * r;
+            float out[2 * KG];
+            evt_add_leaf(pr[r], leaf_pred + (size_t)KG * (nid[r] - 1), KG, LOSS);
+            grad_row<LOSS>(pr[r], y[r], w[r], out);
+            if (i < N) {
+#pragma unroll
+                for (int k = 0; k < KG; k++) pred[(size_t)KG * i + k] = pr[r][k];
+#pragma unroll
+                for (int k = 0; k < 2 * KG; k++) {
+                    O.grad[(size_t)NKG * i + k] = out[k];
+                    mx[k] = fmaxf(mx[k], fabsf(out[k]));
+                }
+            }
+        }
+        absmax_raise_block<2 * KG>(mx, s_m, O.absmax);
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int64_t i = i0 + nthr * r;
+            if (i < N) evt_add_leaf(pred + (size_t)K * i, leaf_pred + (size_t)K * (nid[r] - 1), K, loss);
+        }
     }
 }
 
 // rows per thread: four once the rows fill the device several times over, one for small inputs (more blocks)
+// grads: with the next round's gradients.  Blocks raise the maxima one after the other, so that those of large inputs are wide and walk two rows a thread (1M rows,
+// depth 6 | depth 8: blocks of 256 15.1 | 17.7 us, 512 14.1 | 16.3, 1024 13.1 | 15.3, 1024 and two rows 11.8 | 14.2).
 static int launch_predict_tree_any(evt_ctx *c, const uint32_t *nodes, int nnodes, const float *leaf_pred, const uint4 *copy_src, uint4 *copy_dst,
-                                   int64_t copy_n, int copy_blocks) {
+                                   int64_t copy_n, int copy_blocks, bool grads) {
     const int n_lds = nnodes < 8192 ? nnodes : 8192;
     const size_t lds = (size_t)n_lds * sizeof(uint32_t);
-    if (c->N >= ((int64_t)1 << 21)) {
-        hipLaunchKernelGGL(k_predict_tree<4>, dim3((unsigned)((c->N + 1023) / 1024) + (unsigned)copy_blocks), dim3(256), lds, c->stream, nodes, n_lds,
-                           leaf_pred, c->xcm, c->N, c->K, c->loss, c->pred, copy_src, copy_dst, copy_n, copy_blocks);
+    const GradOut O = {c->y, c->grad, absmax_set(c, c->absmax_cur), c->unit_w ? 1 : 0};
+    const bool wide = grads && c->N > 2047 * 256;
+    const int R = c->N >= ((int64_t)1 << 21) ? 4 : wide ? 2 : 1, threads = wide ? 1024 : 256;
+    const dim3 grid((unsigned)((c->N + threads * R - 1) / (threads * R)) + (unsigned)copy_blocks);
+#define PT(R_, LOSS_)                                                                                                                               \
+    hipLaunchKernelGGL((k_predict_tree<R_, LOSS_>), grid, dim3(threads), lds, c->stream, nodes, n_lds, leaf_pred, c->xcm, c->N, c->K, c->loss, c->pred, \
+                       copy_src, copy_dst, copy_n, copy_blocks, O)
+#define PT1(LOSS_) PT(1, LOSS_)
+#define PT2(LOSS_) PT(2, LOSS_)
+#define PT4(LOSS_) PT(4, LOSS_)
+    if (!grads) {
+        if (R == 4) PT4(-1);
+        else PT1(-1);
+    } else if (R == 4) {
+        EVT_GRAD_ROW_CASES(c, PT4)
+    } else if (R == 2) {
+        EVT_GRAD_ROW_CASES(c, PT2)
     } else {
-        hipLaunchKernelGGL(k_predict_tree<1>, dim3((unsigned)((c->N + 255) / 256) + (unsigned)copy_blocks), dim3(256), lds, c->stream, nodes, n_lds,
-                           leaf_pred, c->xcm, c->N, c->K, c->loss, c->pred, copy_src, copy_dst, copy_n, copy_blocks);
+        EVT_GRAD_ROW_CASES(c, PT1)
     }
+#undef PT4
+#undef PT2
+#undef PT1
+#undef PT
     HIPCHK(hipGetLastError());
     return EVT_OK;
 }
@@ -111,18 +177,19 @@ int launch_nidx_from_tree(evt_ctx *c, bool use_mask, uint8_t cond) {
     return EVT_OK;
 }
 
-int launch_predict_tree_cache(evt_ctx *c, bool send_blob) {
+int launch_predict_tree_cache(evt_ctx *c, bool send_blob, bool grads) {
     const int64_t copy_n = send_blob ? (int64_t)(c->blob_bytes / 16) : 0;
     const int copy_blocks = (int)std::min<int64_t>(64, (copy_n + 255) / 256);
     const int r = launch_predict_tree_any(c, c->tree.packed, c->nnodes, c->tree.pred, reinterpret_cast<const uint4 *>(c->tree_blob),
-                                          reinterpret_cast<uint4 *>(c->h_stage_dev), copy_n, copy_blocks);
+                                          reinterpret_cast<uint4 *>(c->h_stage_dev), copy_n, copy_blocks, grads);
     if (r != EVT_OK) return r;
     if (send_blob) c->step.blob_sent = true;
+    if (grads) c->step.grads_done = true;
     return EVT_OK;
 }
 
 int launch_predict_tree_nodes(evt_ctx *c, const uint32_t *nodes_dev, int nnodes, const float *leaf_pred_dev) {
-    return launch_predict_tree_any(c, nodes_dev, nnodes, leaf_pred_dev, static_cast<const uint4 *>(nullptr), static_cast<uint4 *>(nullptr), (int64_t)0, 0);
+    return launch_predict_tree_any(c, nodes_dev, nnodes, leaf_pred_dev, static_cast<const uint4 *>(nullptr), static_cast<uint4 *>(nullptr), (int64_t)0, 0, false);
 }
 
 // apply_prediction_link!, src/predict.jl:105-116 (softmax!: :187-195)

@@ -886,17 +886,7 @@ __global__ __launch_bounds__(1024) void k_small_final(SmallArgs A) {
     }
     if constexpr (GRADS) {
         __shared__ float s_m[16][2 * K];
-#pragma unroll
-        for (int k = 0; k < 2 * K; k++) {
-            const float m = wave_max_f32(mx[k]);
-            if (lane == 0) s_m[wave][k] = m;
-        }
-        __syncthreads();
-        if (tid < 2 * K) {
-            float m = s_m[0][tid];
-            for (int v = 1; v < 16; v++) m = fmaxf(m, s_m[v][tid]);
-            absmax_raise(A.maxima, tid, m);
-        }
+        absmax_raise_block<2 * K>(mx, s_m, A.maxima);
     }
     if (!writer) return;
     if (A.slices > 1) {
@@ -1054,9 +1044,7 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
             A.blob_src = reinterpret_cast<const uint4 *>(c->tree_blob);
             A.blob_dst = reinterpret_cast<uint4 *>(c->h_stage_dev);
             A.blob_n = (int64_t)(c->blob_bytes / 16);
-            // the next round's gradients are queued behind the tree (tree_close): of one target they are computed here
-            c->step.grads_done = c->grads_ahead && p->update_pred && p->bagging_size == 1 && !EVT_IS_QUANTILE(c->loss) && c->loss != EVT_LOSS_MLOGLOSS &&
-                                 c->K == (EVT_IS_MLE2P(c->loss) ? 2 : 1);
+            c->step.grads_done = grads_with_tree(c, p);
             A.pred = c->pred;
             A.y = c->y;
             A.grad = c->grad;
@@ -1066,15 +1054,7 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
             // no more blocks than are resident at once: a second generation would take the decisions again
 #define FINAL(L_) hipLaunchKernelGGL(k_small_final<L_>, dim3((unsigned)std::min<int64_t>(256, (c->N + 1023) / 1024)), dim3(1024), lds, c->stream, A)
             if (!c->step.grads_done) FINAL(-1);
-            else if (c->loss == EVT_LOSS_MSE) FINAL(0);
-            else if (c->loss == EVT_LOSS_LOGLOSS) FINAL(1);
-            else if (c->loss == EVT_LOSS_GAUSSIAN_MLE) FINAL(2);
-            else if (c->loss == EVT_LOSS_POISSON) FINAL(3);
-            else if (c->loss == EVT_LOSS_GAMMA) FINAL(4);
-            else if (c->loss == EVT_LOSS_TWEEDIE) FINAL(5);
-            else if (c->loss == EVT_LOSS_LOGISTIC_MLE) FINAL(7);
-            else if (c->loss == EVT_LOSS_MAE) FINAL(8);
-            else FINAL(9); // the credibility losses
+            else EVT_GRAD_ROW_CASES(c, FINAL)
 #undef FINAL
             prof_end(c);
             break;

@@ -157,6 +157,8 @@ def test_gradients_quantised_by_the_tree_or_not(evt, N, B, loss, K):
     (1500, 4, "mlogloss", {}),                         # several outputs: the gradient kernels of their own
     (262_145, 4, "mse", dict(weights=True)),           # one row more than the last kernel's blocks take at once
     (530_001, 3, "gaussian_mle", {}),
+    (530_001, 4, "logloss", dict(sub=True, weights=True)),  # the walk over all rows behind a sampled tree: wide blocks
+    (2_097_153, 3, "mse", dict(sub=True)),             # ... and four rows a thread
     (5003, 10, "mse", dict(min_weight=40.0)),          # most leaves above the last level
 ])
 def test_gradients_behind_the_tree(evt, N, D, loss, more):
