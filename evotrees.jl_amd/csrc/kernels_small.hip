@@ -1,4 +1,4 @@
-// Trees of small inputs (thousands to a few hundred thousand rows): one kernel per level instead of a histogram, a search and a partition.
+// Trees of small inputs (thousands to a few hundred thousand rows): one kernel per level, or two where nodes are many, instead of a histogram, a search and a partition.
 //
 // At these sizes a level is a chain of short dependent kernels - 20 launches of 3 to 9 us for a tree of depth 6 on 2000 rows, whatever they
 // do.  Here a block owns one sampled feature and walks ALL rows: it takes the decisions of the level above (every block the same
@@ -69,6 +69,7 @@ struct SmallArgs {
     long long *acc; // slices > 1: [node][block][NAg][B], their histograms added up; zero between two levels
     int *counts;    // ... and their rows, [level][slice]
     int *done;      // ... and how many of a feature's blocks have added theirs, zero between two levels
+    int apart;      // ... and whether k_small_scan searches their sums instead of the last of those blocks
     int batch;      // ... and the nodes whose sums its last block's LDS holds at a time
     int oblivious, sampled, draw, cond;
     int unit_w;
@@ -769,6 +770,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
         }
     }
     if constexpr (SPLIT) {
+        if (A.apart) return;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the block's sums are in memory before it is counted
         __syncthreads();
         if (tid == 0) s_best = __hip_atomic_fetch_add(A.done + jp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == A.slices - 1;
@@ -781,9 +783,16 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
         auto sums = [&](int q) { return reinterpret_cast<unsigned long long *>(A.acc) + ((size_t)q * A.nfs + jp) * words; };
         for (int base = 0; base < nact; base += A.batch) {
             const int nb = nact - base < A.batch ? nact - base : A.batch;
-            for (int i = tid; i < nb * words; i += 1024) {
-                const int k = i / words;
-                S[i] = __hip_atomic_load(sums(s_node[base + k]) + (i - k * words), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int i0 = tid; i0 < nb * words; i0 += 4096) { // four words of a thread under way at a time
+                unsigned long long v[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int i = i0 + 1024 * u < nb * words ? i0 + 1024 * u : i0, k = i / words;
+                    v[u] = __hip_atomic_load(sums(s_node[base + k]) + (i - k * words), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    if (i0 + 1024 * u < nb * words) S[i0 + 1024 * u] = v[u];
             }
             __syncthreads();
             for (int k = wave; k < nb; k += 16) {
@@ -818,6 +827,25 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
             sums(s_node[k])[i - k * words] = 0;
         }
     }
+}
+
+// The searches of a level whose nodes are too many for the last of a feature's blocks (small_scan_apart): a wavefront per (node, feature), 16 nodes of one
+// feature to a block.  Not for oblivious levels, whose nodes' gains meet in one block either way.
+template <int NAG, int BPL>
+__global__ __launch_bounds__(1024) void k_small_scan(SmallArgs A) {
+    __shared__ double s_qs[EVT_MC_MAX_NK];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    touch_args(A);
+    const int nag = NAG ? NAG : A.NAg, jp = blockIdx.x, first = 1 << (A.level - 1), words = nag * A.B;
+    const int q = (int)blockIdx.y * 16 + wave;
+    const int st = A.status[first + (q < first ? q : 0)];
+    if (tid < nag) s_qs[tid] = A.qscale[tid];
+    __syncthreads();
+    if (q >= first || st != ST_BUILD) return;
+    long long *sums = A.acc + ((size_t)q * A.nfs + jp) * words;
+    small_search<NAG, BPL, false>(A, s_qs, reinterpret_cast<const unsigned long long *>(sums), q, jp, A.nfs, A.feat[jp],
+                                  A.level > 1 ? A.node_sum + (int64_t)(first + q) * nag : nullptr, jp == 0, nullptr, lane);
+    for (int i = lane; i < words; i += 64) sums[i] = 0;
 }
 
 // The last decisions, the leaves, and every row's leaf.  The first block also sends the finished tree to the host's pinned buffer.
@@ -914,6 +942,13 @@ static size_t small_lds(const evt_ctx *c, int level, int slots, bool split) {
 static size_t small_lds_search(const evt_ctx *c, int level, int batch) {
     const size_t nodes = (size_t)1 << (level - 1), tot = level > 1 ? nodes * c->NAg * 8 : 0;
     return tot + (c->tree_type == EVT_TREE_OBLIVIOUS ? nodes * c->B * 8 : 0) + (size_t)batch * c->NAg * c->B * 8;
+}
+// Whether a level's searches take a kernel of their own.  The last of a feature's blocks reads its nodes' sums, 1024 words at a time, and its 16 wavefronts search
+// them, where that kernel spreads them over the chip for a launch more.  20k rows, us a level, the last block | apart with the gap between its
+// launches: one output of 64 bins 4 nodes 11 | 14, 16 nodes 16 | 16, 32 nodes 22 | 18, 64 nodes 31 | 21; of 255 bins 4 nodes 16 | 17, 8 nodes 20 | 18, 32
+// nodes 40 | 29; two outputs of 64 bins 8 nodes 16 | 16, 16 nodes 20 | 19, 128 nodes 45 | 25.
+static bool small_scan_apart(const evt_ctx *c, int nodes) {
+    return c->tree_type != EVT_TREE_OBLIVIOUS && (nodes > 16 || (int64_t)nodes * c->NAg * c->B > 5120);
 }
 // histograms a block's LDS holds at the deepest level that splits
 static int small_slots(const evt_ctx *c, bool split) {
@@ -1066,7 +1101,8 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
         if (split) { // a wavefront per node at a time, as far as they fit
             A.batch = std::min(16, nodes);
             while (A.batch > 1 && small_lds_search(c, level, A.batch) > std::max<size_t>(lds, 72 * 1024)) A.batch >>= 1;
-            lds = std::max(lds, small_lds_search(c, level, A.batch));
+            A.apart = small_scan_apart(c, nodes) ? 1 : 0;
+            if (!A.apart) lds = std::max(lds, small_lds_search(c, level, A.batch));
         }
         prof_begin(c, level == 1 ? EVT_K_HIST : EVT_K_PARTITION, level); // below the root it moves rows, builds and searches at once
 #define SMALL4(NAG_, BPL_, PACK_, SPLIT_, ROOT_)                                                                                          \
@@ -1084,6 +1120,11 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
     if (split) {                                                     \
         if (level == 1) SMALL4(NAG_, BPL_, PACK_, true, true)        \
         else SMALL4(NAG_, BPL_, PACK_, true, false)                  \
+        if (A.apart) {                                               \
+            prof_end(c);                                             \
+            prof_begin(c, EVT_K_SCAN, level);                        \
+            hipLaunchKernelGGL((k_small_scan<NAG_, BPL_>), dim3((unsigned)c->n_js_last, (unsigned)((nodes + 15) / 16)), dim3(1024), 0, c->stream, A); \
+        }                                                            \
     } else {                                                         \
         if (level == 1) SMALL4(NAG_, BPL_, PACK_, false, true)       \
         else SMALL4(NAG_, BPL_, PACK_, false, false)                 \
