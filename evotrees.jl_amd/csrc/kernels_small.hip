@@ -829,23 +829,70 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
     }
 }
 
-// The searches of a level whose nodes are too many for the last of a feature's blocks (small_scan_apart): a wavefront per (node, feature), 16 nodes of one
-// feature to a block.  Not for oblivious levels, whose nodes' gains meet in one block either way.
+// The searches of a level that the last of a feature's blocks does not take (small_scan_apart): a wavefront per (node, feature), 16 nodes of one
+// feature to a block - all of them for an oblivious level, whose nodes' gains meet in LDS.
 template <int NAG, int BPL>
 __global__ __launch_bounds__(1024) void k_small_scan(SmallArgs A) {
+    extern __shared__ double s_gain[]; // oblivious: [active nodes][B]
     __shared__ double s_qs[EVT_MC_MAX_NK];
+    __shared__ uint16_t s_node[SMALL_MAX_NODES];
+    __shared__ int s_nact, s_best;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     touch_args(A);
     const int nag = NAG ? NAG : A.NAg, jp = blockIdx.x, first = 1 << (A.level - 1), words = nag * A.B;
-    const int q = (int)blockIdx.y * 16 + wave;
-    const int st = A.status[first + (q < first ? q : 0)];
+    const int mine = (int)blockIdx.y * 16 + wave;
+    const int st = A.status[first + (mine < first ? mine : 0)];
+    const uint32_t fw = A.feat[jp];
     if (tid < nag) s_qs[tid] = A.qscale[tid];
+    auto sums = [&](int q) { return A.acc + ((size_t)q * A.nfs + jp) * words; };
+    auto search = [&](int q, double *gain) {
+        small_search<NAG, BPL, false>(A, s_qs, reinterpret_cast<const unsigned long long *>(sums(q)), q, jp, A.nfs, fw,
+                                      A.level > 1 ? A.node_sum + (int64_t)(first + q) * nag : nullptr, jp == 0, gain, lane);
+    };
+    auto clear = [&](int q) {
+        for (int i = lane; i < words; i += 64) sums(q)[i] = 0;
+    };
+    if (!A.oblivious) {
+        __syncthreads();
+        if (mine >= first || st != ST_BUILD) return;
+        search(mine, nullptr);
+        clear(mine);
+        return;
+    }
+    if (wave == 0) {
+        int base = 0;
+        for (int q0 = 0; q0 < first; q0 += 64) {
+            const bool on = q0 + lane < first && A.status[first + q0 + lane] == ST_BUILD;
+            const unsigned long long m = __ballot(on);
+            if (on) s_node[base + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)(q0 + lane);
+            base += __popcll(m);
+        }
+        if (lane == 0) s_nact = base;
+    }
     __syncthreads();
-    if (q >= first || st != ST_BUILD) return;
-    long long *sums = A.acc + ((size_t)q * A.nfs + jp) * words;
-    small_search<NAG, BPL, false>(A, s_qs, reinterpret_cast<const unsigned long long *>(sums), q, jp, A.nfs, A.feat[jp],
-                                  A.level > 1 ? A.node_sum + (int64_t)(first + q) * nag : nullptr, jp == 0, nullptr, lane);
-    for (int i = lane; i < words; i += 64) sums[i] = 0;
+    const int nact = s_nact;
+    for (int s = wave; s < nact; s += 16) search(s_node[s], s_gain + s * A.B);
+    __syncthreads();
+    const bool numeric = (fw & SMALL_NUMERIC) != 0;
+    if (wave == 0) {
+        double bg;
+        const int bb = small_obliv_best(A, s_gain, nact, lane, &bg);
+        if (lane == 0) s_best = bb;
+        for (int s = lane; s < nact; s += 64) {
+            SmallHead *out = A.head_out + (int64_t)s_node[s] * A.nfs + jp;
+            out->gain = bg;
+            out->bin = bb;
+            out->feat = numeric ? (int)(fw & 0xFFFFu) + 1 : -((int)(fw & 0xFFFFu) + 1);
+        }
+    }
+    __syncthreads();
+    const int lb = s_best;
+    for (int s = wave; s < nact; s += 16) {
+        const int q = s_node[s];
+        const int64_t at = (int64_t)q * A.nfs + jp;
+        small_left<false, false>(A, reinterpret_cast<const unsigned long long *>(sums(q)), nag, numeric, lb, lane, A.head_out + at, A.left_out + at * nag);
+        clear(q);
+    }
 }
 
 // The last decisions, the leaves, and every row's leaf.  The first block also sends the finished tree to the host's pinned buffer.
@@ -947,8 +994,13 @@ static size_t small_lds_search(const evt_ctx *c, int level, int batch) {
 // them, where that kernel spreads them over the chip for a launch more.  20k rows, us a level, the last block | apart with the gap between its
 // launches: one output of 64 bins 4 nodes 11 | 14, 16 nodes 16 | 16, 32 nodes 22 | 18, 64 nodes 31 | 21; of 255 bins 4 nodes 16 | 17, 8 nodes 20 | 18, 32
 // nodes 40 | 29; two outputs of 64 bins 8 nodes 16 | 16, 16 nodes 20 | 19, 128 nodes 45 | 25.
+// The search of two outputs of more than 64 bins holds too many registers to sit in the level's kernel (42k rows x 44, 255 bins, depth 5, 64 rounds: in it 13.4 ms,
+// apart 11.9; 4837 x 18, oblivious of depth 8, 133
+// rounds 35.5 | 27.1), and an oblivious level is taken apart where LDS holds the sums of fewer than 16 nodes.
 static bool small_scan_apart(const evt_ctx *c, int nodes) {
-    return c->tree_type != EVT_TREE_OBLIVIOUS && (nodes > 16 || (int64_t)nodes * c->NAg * c->B > 5120);
+    if (!c->mc && c->NAg * ((c->B + 63) / 64) >= 10) return true;
+    if (c->tree_type == EVT_TREE_OBLIVIOUS) return (size_t)std::min(16, nodes) * c->NAg * c->B * 8 > 72 * 1024;
+    return nodes > 16 || (int64_t)nodes * c->NAg * c->B > 5120;
 }
 // histograms a block's LDS holds at the deepest level that splits
 static int small_slots(const evt_ctx *c, bool split) {
@@ -1121,9 +1173,15 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
         if (level == 1) SMALL4(NAG_, BPL_, PACK_, true, true)        \
         else SMALL4(NAG_, BPL_, PACK_, true, false)                  \
         if (A.apart) {                                               \
+            static EvtDevOnce once;                                  \
+            if (once.pending(c->device)) {                           \
+                HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_small_scan<NAG_, BPL_>), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024)); \
+                once.mark(c->device);                                \
+            }                                                        \
+            const size_t gain = A.oblivious ? (size_t)nodes * c->B * 8 : 0; \
             prof_end(c);                                             \
             prof_begin(c, EVT_K_SCAN, level);                        \
-            hipLaunchKernelGGL((k_small_scan<NAG_, BPL_>), dim3((unsigned)c->n_js_last, (unsigned)((nodes + 15) / 16)), dim3(1024), 0, c->stream, A); \
+            hipLaunchKernelGGL((k_small_scan<NAG_, BPL_>), dim3((unsigned)c->n_js_last, A.oblivious ? 1u : (unsigned)((nodes + 15) / 16)), dim3(1024), gain, c->stream, A); \
         }                                                            \
     } else {                                                         \
         if (level == 1) SMALL4(NAG_, BPL_, PACK_, false, true)       \

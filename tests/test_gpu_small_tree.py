@@ -28,6 +28,14 @@ pytestmark = pytest.mark.gpu
     (1200, 6, 64, 5, "mlogloss", dict(K=2)),
     (150_001, 3, 64, 6, "mse", dict(sub="drawn")),                   # more rows than one block per feature takes
     (70_001, 12, 40, 5, "gaussian_mle", dict(oblivious=True, weights=True)),
+    # levels of shared rows on either side of the line where their searches take a kernel of their own
+    (3001, 5, 255, 8, "gaussian_mle", dict(oblivious=True, weights=True)),
+    (4001, 6, 255, 5, "gaussian_mle", dict(sub="mask")),
+    (5001, 4, 128, 7, "gaussian_mle", {}),
+    (6007, 3, 200, 8, "mse", dict(oblivious=True)),
+    (7001, 3, 160, 7, "mse", dict(weights=True)),                    # 16 nodes of 320 words: the last that stays
+    (2003, 4, 255, 5, "mlogloss", dict(K=16)),
+    (2503, 4, 255, 6, "mlogloss", dict(K=5, oblivious=True)),
 ])
 def test_one_kernel_per_level_changes_nothing(evt, N, F, B, D, loss, more):
     rng = np.random.default_rng(N)
