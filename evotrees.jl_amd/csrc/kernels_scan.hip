@@ -7,6 +7,7 @@
 // Float64 with the reference's expression order, and the best candidate is found with a
 // cross-lane arg-max whose ties go to the lowest bin, then the earliest feature of js — the
 // reference's "first maximum wins" (strict '>' at src/fit-utils.jl:447).
+#include "obliv_rule.h"
 #include "split_math.h"
 #include <algorithm>
 
@@ -752,7 +753,6 @@ struct OblivLevelArgs {
     int fold_leaves;
     unsigned long long *lefts; // [feature][node][NAG]: totals left of the feature's candidate
 };
-#define OBLIV_LEVEL_NODES 32
 
 // NPW: nodes of a wavefront
 template <int NAG, int BPL, int NPW>
@@ -1327,13 +1327,9 @@ __global__ __launch_bounds__(256) void k_scan_fin_mc(ScanArgs A, int ngroups) {
 // of one node nor one of wide slices (16 channels x 100 features: 1.6 MB per node) leaves them to few blocks.
 static unsigned zero_blocks_per_node(unsigned nodes) { return nodes >= 512 ? 1u : (512u / nodes < 64u ? 512u / nodes : 64u); }
 
-// An oblivious level in one launch: where a wavefront's words (nodes x channels x bins per lane) are few enough for its registers and the searches a
-// block's wavefronts share do not outlast the launches saved.  us of a level in three launches | one, event pairs included (60k rows; 20 to 120
-// features): mse 64 bins 4 nodes 14 | 8, 16 nodes 16 | 9, 32 nodes 19 | 14; mse 128 bins 32 nodes 21 | 19; mse 255 bins 16 nodes 20 | 18, 32 nodes 27 | 32;
-// logloss 128 bins 16 nodes 18 | 13, 32 nodes 21 | 21; two outputs 64 bins 16 nodes 14 | 13, 128 bins 16 nodes 17 | 17, 255 bins 8 nodes 25 | 20, 16 nodes 24 | 32.
+// An oblivious level in one launch
 static bool obliv_one_launch(const evt_ctx *c, int level) {
-    const int nodes = 1 << (level - 1), words = c->NAg * ((c->B + 63) / 64);
-    return c->tree_type == EVT_TREE_OBLIVIOUS && !c->mc && c->scan_fused && c->B >= 4 && nodes <= OBLIV_LEVEL_NODES && nodes * words <= 192;
+    return c->tree_type == EVT_TREE_OBLIVIOUS && !c->mc && c->scan_fused && obliv_level_fits(c->NAg, c->B, 1 << (level - 1));
 }
 
 // The pass over the last split level also writes its children's leaf values (the fixed channel layouts).
@@ -1444,19 +1440,18 @@ static int launch_obliv_level(evt_ctx *c, int level, const evt_params *p) {
     A.min_weight = p->min_weight;
     A.fold_leaves = level + 1 == c->D ? 1 : 0;
     A.lefts = reinterpret_cast<unsigned long long *>(c->ogains); // nodes x features x bins words, unused in this form
-    const int nodes = 1 << (level - 1), bpl = (c->B + 63) / 64;
+    const int nodes = 1 << (level - 1);
     const dim3 grid((unsigned)A.o.nfs), block(64u * std::min(16, std::max(4, nodes)));
     const size_t lds = (size_t)nodes * c->B * sizeof(double);
-#define OLCASE(NAG_, BPL_, NPW_)                                                                         \
-    if (c->NAg == NAG_ && (bpl <= 2 ? bpl : 4) == BPL_ && (nodes > 16) == (NPW_ > 1)) {                  \
-        hipLaunchKernelGGL((k_obliv_level<NAG_, BPL_, NPW_>), grid, block, lds, c->stream, A);           \
-        HIPCHK(hipGetLastError());                                                                       \
-        return EVT_OK;                                                                                   \
+#define OLCASE(NAG_, BPL_, NPW_)                                                                                     \
+    if (c->NAg == NAG_ && obliv_lane_bins(c->B) == BPL_ && obliv_wave_nodes(nodes) == NPW_) {                        \
+        hipLaunchKernelGGL((k_obliv_level<NAG_, BPL_, NPW_>), grid, block, lds, c->stream, A);                       \
+        HIPCHK(hipGetLastError());                                                                                   \
+        return EVT_OK;                                                                                               \
     }
-    OLCASE(2, 1, 1) OLCASE(2, 2, 1) OLCASE(2, 4, 1) OLCASE(3, 1, 1) OLCASE(3, 2, 1) OLCASE(3, 4, 1) OLCASE(5, 1, 1) OLCASE(5, 2, 1) OLCASE(5, 4, 1)
-    OLCASE(2, 1, 2) OLCASE(2, 2, 2) OLCASE(3, 1, 2) OLCASE(3, 2, 2) OLCASE(5, 1, 2)
+    EVT_OBLIV_LEVELS(OLCASE)
 #undef OLCASE
-    evt_set_error("unsupported global channel count %d", c->NAg);
+    evt_set_error("internal: no kernel for an oblivious level of %d nodes, %d channels, %d bins", nodes, c->NAg, c->B);
     return EVT_ERR_ARG;
 }
 

@@ -21,6 +21,13 @@ pytestmark = pytest.mark.gpu
     ("mse", False, 300, 20, 32, 7, 20, dict(min_weight=20.0)),           # levels without a split
     ("mse", False, 5_001, 20, 32, 4, 20, dict(gamma=1e9)),               # the root is a leaf
     ("mae", True, 5_001, 20, 32, 5, 20, {}),
+    # 129 to 192 bins are three pieces of 64 but four bins to a lane: two channels take 32 nodes in one launch, and 64 in three
+    ("mse", False, 20_001, 20, 129, 7, 20, {}),
+    ("mse", True, 20_001, 20, 160, 8, 17, dict(cat=True, mono=True)),
+    ("mae", False, 20_001, 66, 192, 8, 66, {}),
+    ("mse", False, 20_001, 20, 193, 7, 20, {}),                          # four pieces: 16 nodes in one, 32 in three
+    ("logloss", False, 20_001, 20, 160, 7, 20, {}),
+    ("gaussian_mle", True, 20_001, 18, 160, 6, 18, {}),
 ])
 def test_one_launch_decides_the_level(evt, loss, weights, N, F, B, D, n_js, more):
     more = dict(more)
