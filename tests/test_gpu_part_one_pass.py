@@ -21,13 +21,16 @@ pytestmark = pytest.mark.gpu
     (30_011, 18, 16, 5, "mlogloss", dict(K=5)),
     (30_011, 18, 16, 6, "mse", dict(tt="oblivious")),
     (70_001, 17, 8, 13, "mse", {}),                                   # cursors past the first thousand
+    # every node of the level of 8192 is split: more chunks than the 4096 blocks of a launch, each of which takes several in turn
+    (100_003, 17, 2, 16, "mse", dict(L2=0.0)),
+    (200_003, 18, 2, 16, "mse", dict(L2=0.0, sub=True)),
 ])
 def test_one_pass_changes_nothing(evt, N, F, B, D, loss, more):
     rng = np.random.default_rng(N)
     x_bin, y, _, mu = make_data(N, N, F, B, loss, False, K=more.get("K"))
     ft = (rng.random(F) > 0.5).astype(np.uint8) if more.get("cat") else None
     js = np.arange(1, F + 1, dtype=np.uint32)
-    gp = evt.make_params(eta=0.4, min_weight=0.0 if N < 3_000 else 1.0)
+    gp = evt.make_params(eta=0.4, L2=more.get("L2", 1.0), min_weight=0.0 if N < 3_000 else 1.0)
     out = []
     for one in (1, 0):
         h = evt.Handle(N, F, B, len(mu), D, loss, more.get("tt", "binary"))
@@ -51,3 +54,5 @@ def test_one_pass_changes_nothing(evt, N, F, B, D, loss, more):
         for u, v in zip(a[1:], b[1:]):
             assert u.tobytes() == v.tobytes()
     assert N == 1 or out[0][0][0].split.sum() >= 1
+    if D == 16:
+        assert (out[0][0][0].split[2**13 - 1 : 2**14 - 1]).sum() > 5_000
