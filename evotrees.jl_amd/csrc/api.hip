@@ -845,7 +845,7 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
     const int small = staged ? 0 : small_tree_form(c, n_js, all_rows);
     int r = EVT_OK;
     if (c->quant_pending) {
-        if (small || c->N <= EVT_QUANT_LATER) quant_set(c); // by the tree's first kernel
+        if (small ? small_root_quantises(c, small) : c->N <= EVT_QUANT_LATER) quant_set(c); // by the tree's first kernel
         else r = launch_quantize(c);
         if (r != EVT_OK) return r;
     }

@@ -378,6 +378,7 @@ int launch_part_count(evt_ctx *c, int level, const uint32_t *is_cur);
 int launch_part_scatter(evt_ctx *c, int level, const uint32_t *is_cur, uint32_t *is_next, bool fuse_pred);
 bool scatter_can_build_hist(const evt_ctx *c, int nfs);
 int small_tree_form(const evt_ctx *c, int nfs, bool all_rows);
+bool small_root_quantises(const evt_ctx *c, int form);
 int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices);
 int launch_final_fused(evt_ctx *c, int level, const uint32_t *is_cur, bool fuse_pred, bool send_blob);
 int launch_nidx_from_segments(evt_ctx *c, int level, const uint32_t *is_cur);

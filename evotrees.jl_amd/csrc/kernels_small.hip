@@ -458,13 +458,15 @@ __device__ __forceinline__ int small_obliv_best(const SmallArgs &A, const double
 // chain of trips to memory in few blocks (2000 rows: 9.7 us below the root with its loads behind branches and its arguments read one by one, 8.7
 // now; the root 6.5 with the quantisation beside it, 7.0 with it inside).  Whole fits: 2000 x 10, 100 rounds 7.5 -> 6.9 ms, 100k x 10, 200 rounds
 // with an eval set 21.1 -> 20.2.
+// SMALL_ROOT_WORDS: any number of outputs, quantised ahead (small_root_quantises).
 // SPLIT: a feature's rows are shared by `slices` blocks, which add their histograms into A.acc; the last of them to do so reads the sums and
 // searches them (100k rows x 10 features: 8.3 us a level and 5.2 for a kernel of its own that searched -> 13.9, and a round of five levels
 // 101 -> 92 us).  What passes between the blocks goes by agent-scope atomics, past the caches that are not shared, and is complete before its
 // block is counted (as in k_scan).  For inputs of
 // few features, whose blocks would fill a part of the chip with long walks: 10 features in 25 slices take 0.4 us per 25k rows and channel pair
 // where one block per feature takes 0.4 us per 1k, for 5 us more of flush and hand-over.
-template <int NAG, int BPL, bool PACK, bool SPLIT, bool ROOT>
+enum SmallForm { SMALL_BELOW, SMALL_ROOT, SMALL_ROOT_WORDS };
+template <int NAG, int BPL, bool PACK, bool SPLIT, SmallForm FORM>
 __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
     extern __shared__ unsigned long long s_dyn[];
     __shared__ uint32_t s_dec[SMALL_MAX_NODES];
@@ -474,6 +476,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
     __shared__ double s_qs[EVT_MC_MAX_NK], s_qmul[EVT_MC_MAX_NK]; // scales of the channels; multipliers of the gradient rows (raw)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     touch_args(A);
+    constexpr bool ROOT = FORM != SMALL_BELOW, QUANT = FORM == SMALL_ROOT;
     const int B = A.B, N = A.N, level = ROOT ? 1 : A.level;
     __builtin_assume(ROOT || level > 1);
     const int nag = NAG ? NAG : A.NAg, na = NAG ? NAG - (PACK ? 1 : 0) : A.NA;
@@ -552,7 +555,9 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
     };
     request(gfirst + tid);
     if constexpr (ROOT) { // the tables: made here of fresh gradients, or those the words in A.gq were made with
-        if (tid < A.NK) {
+        if constexpr (!QUANT) {
+            if (tid < nag) s_qs[tid] = A.qscale[tid];
+        } else if (tid < A.NK) {
             const double *mul = A.qscale + EVT_MC_MAX_NK;
             if (A.fresh) {
                 const int e = quant_exponent(A.absmax, tid), qb = A.qbits[tid];
@@ -671,7 +676,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
             if (share)
 #pragma unroll
                 for (int i = 0; i < 4; i++) A.nid_out[r + i] = nid[u][i];
-            if constexpr (ROOT) {
+            if constexpr (QUANT) {
                 const bool keep = share && A.fresh;
                 if constexpr (NAG != 0) {
 #pragma unroll
@@ -682,7 +687,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
                     for (int i = 0; i < 4; i++)
                         for (int a = 0; a < na; a++) quantise(A.raw[(size_t)(r + i) * A.NK + a], a, r + i, true);
                 }
-            } else if constexpr (NARROW) {
+            } else if constexpr (NARROW && !ROOT) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) g[0][u][i] = ((unsigned long long)(long long)(int32_t)g0[u][i] << EVT_PACK_CNT_BITS) + 1ull;
             }
@@ -700,7 +705,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
                 } else {
                     for (int a = 0; a < na; a++) {
                         unsigned long long v;
-                        if (ROOT) v = quantise(A.raw[(size_t)(r + i) * A.NK + a], a, r + i, false);
+                        if (QUANT) v = quantise(A.raw[(size_t)(r + i) * A.NK + a], a, r + i, false);
                         else if (PACK && a == 0 && !A.wide) v = evt_load_gq<true>(A.gq, N, 0, (uint32_t)(r + i));
                         else v = A.gq[(size_t)a * N + r + i];
                         atomicAdd(h + a * B, v);
@@ -1071,6 +1076,12 @@ int small_tree_form(const evt_ctx *c, int nfs, bool all_rows) {
     return canS && split < other ? S : 0;
 }
 
+// Whether the root's kernel of a tree of this form (small_tree_form) quantises the gradients, or k_quantize does ahead of it.  Of any number of
+// outputs every block converts all channels of its rows, where a word made ahead is one load: there only blocks of few rows save by it.  Rounds of depth 5,
+// 64 bins, us, in the root | ahead: one block a feature, 7 outputs x 6 features 400 rows 131 | 130, 3000 145 | 134, 12k 297 | 209; several, 3 outputs
+// x 6 features (42 blocks each) 6k rows 105 | 109, 25k 109 | 111, 50k 114 | 115, x 30 (8) 6k 108 | 110, 12k 113 | 111, 25k 127 | 118; 7 x 100 (2) 2k 164 | 163, 6k 184 | 175.
+bool small_root_quantises(const evt_ctx *c, int form) { return !c->mc || (form > 1 && c->N <= (int64_t)1500 * form); }
+
 int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
     const bool split = slices > 1;
     int r = small_tree_buffers(c, split);
@@ -1162,21 +1173,22 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
             if (!A.apart) lds = std::max(lds, small_lds_search(c, level, A.batch));
         }
         prof_begin(c, level == 1 ? EVT_K_HIST : EVT_K_PARTITION, level); // below the root it moves rows, builds and searches at once
-#define SMALL4(NAG_, BPL_, PACK_, SPLIT_, ROOT_)                                                                                          \
+#define SMALL4(NAG_, BPL_, PACK_, SPLIT_, FORM_)                                                                                          \
     {                                                                                                                                     \
         static EvtDevOnce once;                                                                                                           \
         if (once.pending(c->device)) {                                                                                                    \
-            HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_small_level<NAG_, BPL_, PACK_, SPLIT_, ROOT_>),                    \
+            HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_small_level<NAG_, BPL_, PACK_, SPLIT_, FORM_>),                    \
                                        hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));                                          \
             once.mark(c->device);                                                                                                         \
         }                                                                                                                                 \
-        hipLaunchKernelGGL((k_small_level<NAG_, BPL_, PACK_, SPLIT_, ROOT_>), dim3((unsigned)c->n_js_last, split ? (unsigned)slices : 1u), \
+        hipLaunchKernelGGL((k_small_level<NAG_, BPL_, PACK_, SPLIT_, FORM_>), dim3((unsigned)c->n_js_last, split ? (unsigned)slices : 1u), \
                            dim3(1024), lds, c->stream, A);                                                                                \
     }
 #define SMALL3(NAG_, BPL_, PACK_)                                    \
     if (split) {                                                     \
-        if (level == 1) SMALL4(NAG_, BPL_, PACK_, true, true)        \
-        else SMALL4(NAG_, BPL_, PACK_, true, false)                  \
+        if (level > 1) SMALL4(NAG_, BPL_, PACK_, true, SMALL_BELOW) \
+        else if (A.fresh) SMALL4(NAG_, BPL_, PACK_, true, SMALL_ROOT) \
+        else SMALL4(NAG_, BPL_, PACK_, true, (NAG_ ? SMALL_ROOT : SMALL_ROOT_WORDS)) \
         if (A.apart) {                                               \
             static EvtDevOnce once;                                  \
             if (once.pending(c->device)) {                           \
@@ -1189,8 +1201,8 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
             hipLaunchKernelGGL((k_small_scan<NAG_, BPL_>), dim3((unsigned)c->n_js_last, A.oblivious ? 1u : (unsigned)((nodes + 15) / 16)), dim3(1024), gain, c->stream, A); \
         }                                                            \
     } else {                                                         \
-        if (level == 1) SMALL4(NAG_, BPL_, PACK_, false, true)       \
-        else SMALL4(NAG_, BPL_, PACK_, false, false)                 \
+        if (level > 1) SMALL4(NAG_, BPL_, PACK_, false, SMALL_BELOW) \
+        else SMALL4(NAG_, BPL_, PACK_, false, (NAG_ ? SMALL_ROOT : SMALL_ROOT_WORDS)) \
     }
 #define SMALL2(NAG_, PACK_)             \
     if (bpl == 1) { SMALL3(NAG_, 1, PACK_) } \

@@ -88,7 +88,8 @@ def test_one_kernel_per_level_changes_nothing(evt, N, F, B, D, loss, more):
     assert splits > 0 or N < 10
 
 
-@pytest.mark.parametrize("N,B,loss,K", [(1030, 64, "mse", 1), (2501, 200, "logloss", 1), (1999, 33, "gaussian_mle", 2), (1500, 40, "mlogloss", 7)])
+@pytest.mark.parametrize("N,B,loss,K", [(1030, 64, "mse", 1), (2501, 200, "logloss", 1), (1999, 33, "gaussian_mle", 2), (1500, 40, "mlogloss", 7),
+                                        (63_000, 64, "mlogloss", 3), (63_001, 33, "mlogloss", 2)])  # 42 blocks a feature: quantised by the root, and ahead of it
 def test_gradients_quantised_by_the_tree_or_not(evt, N, B, loss, K):
     """The root's kernel quantises what evt_update_grads left; whatever comes in between (a second update, other targets, gradients from outside,
     the other kernels, a second tree on the same gradients) sees what k_quantize would have left: same tables, trees and histograms."""
