@@ -134,7 +134,7 @@ struct evt_ctx {
     int32_t *chunk_nleft;
     int64_t *chunk_lpre;
     int64_t max_chunks;
-    unsigned long long *cursor; // one-pass partition: rows a split node's chunks have placed, left | right << 32 (part_cursor_slot)
+    unsigned long long *cursor; // one-pass partition: rows a split node's chunks have placed, left | right << 32 (EVT_CURSOR_SLOT)
     int part_one_pass; // option: the partition of a level runs in one kernel where the split search knows the children's sizes
     long long *hist; // [node][jp][ag][bin]
     int64_t *seg_start, *seg_len;

@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256) void k_grads_mt(float *__restrict__ pred, cons
 }
 
 // Multi-class log loss (src/loss.jl:93-98, :113-128): prob_k = exp(p_k) / sum_j exp(p_j); g_k = (prob_k - [y == k]) w,
-// h_k = prob_k (1 - prob_k) w; y holds the 1-based class.  The row maxima are reduced one gradient row at a time.
+// h_k = prob_k (1 - prob_k) w; y holds the 1-based class.
 // KM: a bound of K, 4, 8 or 16; a row's words are requested together (those past the last class read it again), where a request per class behind a
 // branch each was a trip to memory per class.  60k rows of 7 classes 13.7 -> 13.2 us.
 template <int KM>
