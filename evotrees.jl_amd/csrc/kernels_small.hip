@@ -420,10 +420,11 @@ __device__ __forceinline__ void small_search(const SmallArgs &A, const double *q
     }
 }
 
-// Searches of this many channels (0: a run-time count) and 64-bin pieces hold too many registers to sit in a level's kernel (small_scan_apart).  Compiled
+// Searches of this many channels (0: a run-time count) and bins to a lane (1, 2 or 4) hold too many registers to sit in a level's kernel (small_scan_apart).  Compiled
 // into it and never run, they still spilt its registers (108 to 340 bytes a lane, now none; rounds of two outputs: 42k rows x 44 features, 255 bins,
 // depth 5 147.0 -> 145.0 us, 20k x 6, depth 9 332 -> 327).
-constexpr bool small_search_large(int channels, int pieces) { return channels * pieces >= 10; }
+constexpr bool small_search_large(int channels, int bins) { return channels * bins >= 10; }
+static int bins_per_lane(int B) { return B <= 64 ? 1 : B <= 128 ? 2 : 4; }
 
 // Requests every 64-byte line of the arguments at once: read where each is needed, they were ten trips one after the other.
 __device__ __forceinline__ void touch_args(const SmallArgs &A) {
@@ -779,7 +780,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
             if (level == 1) A.stats[0] = s_cnt;
         }
     }
-    if constexpr (SPLIT && !small_search_large(NAG, BPL < 4 ? BPL : 3)) { // instances whose levels are all searched apart end here
+    if constexpr (SPLIT && !small_search_large(NAG, BPL)) { // instances whose levels are all searched apart end here
         if (A.apart) return;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the block's sums are in memory before it is counted
         __syncthreads();
@@ -1004,11 +1005,12 @@ static size_t small_lds_search(const evt_ctx *c, int level, int batch) {
 // them, where that kernel spreads them over the chip for a launch more.  20k rows, us a level, the last block | apart with the gap between its
 // launches: one output of 64 bins 4 nodes 11 | 14, 16 nodes 16 | 16, 32 nodes 22 | 18, 64 nodes 31 | 21; of 255 bins 4 nodes 16 | 17, 8 nodes 20 | 18, 32
 // nodes 40 | 29; two outputs of 64 bins 8 nodes 16 | 16, 16 nodes 20 | 19, 128 nodes 45 | 25.
-// The search of two outputs of more than 64 bins holds too many registers to sit in the level's kernel (42k rows x 44, 255 bins, depth 5, 64 rounds: in it 13.4 ms,
-// apart 11.9; 4837 x 18, oblivious of depth 8, 133
-// rounds 35.5 | 27.1), and an oblivious level is taken apart where LDS holds the sums of fewer than 16 nodes.
+// The search of two outputs of more than 64 bins, or of one output of three channels and more than 128, holds too many registers to sit in the level's kernel
+// (42k rows x 44, 255 bins, depth 5, 64 rounds: in it 13.4 ms, apart 11.9; 4837 x 18, oblivious of depth 8, 133 rounds 35.5 | 27.1; a round of three
+// channels x 192 bins, 74k x 3, depth 5 105 | 88 us, of 160 bins, 11k x 206, oblivious of depth 8 310 | 224), and an oblivious level is taken apart where
+// LDS holds the sums of fewer than 16 nodes.
 static bool small_scan_apart(const evt_ctx *c, int nodes) {
-    if (!c->mc && small_search_large(c->NAg, (c->B + 63) / 64)) return true;
+    if (!c->mc && small_search_large(c->NAg, bins_per_lane(c->B))) return true;
     if (c->tree_type == EVT_TREE_OBLIVIOUS) return (size_t)std::min(16, nodes) * c->NAg * c->B * 8 > 72 * 1024;
     return nodes > 16 || (int64_t)nodes * c->NAg * c->B > 5120;
 }
@@ -1127,7 +1129,7 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
         const int f = (int)c->js_last[j] - 1;
         A.feat[j] = (uint32_t)f | (c->h_feattypes[f] ? SMALL_NUMERIC : 0u) | ((uint32_t)(c->h_mono[f] + 1) << 17);
     }
-    const int bpl = (c->B + 63) / 64;
+    const int bpl = bins_per_lane(c->B);
     A.raw = c->grad;
     if (c->quant_pending) {
         A.fresh = 1;

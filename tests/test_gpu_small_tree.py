@@ -34,6 +34,9 @@ pytestmark = pytest.mark.gpu
     (5001, 4, 128, 7, "gaussian_mle", {}),
     (6007, 3, 200, 8, "mse", dict(oblivious=True)),
     (7001, 3, 160, 7, "mse", dict(weights=True)),                    # 16 nodes of 320 words: the last that stays
+    (5001, 5, 192, 6, "logloss", dict(weights=True)),                # three channels, four bins to a lane: searched apart from the root on
+    (5001, 4, 160, 6, "cred_var", dict(oblivious=True)),
+    (5001, 4, 128, 6, "poisson", dict(oblivious=True, sub="drawn")),
     (2003, 4, 255, 5, "mlogloss", dict(K=16)),
     (2503, 4, 255, 6, "mlogloss", dict(K=5, oblivious=True)),
 ])
