@@ -78,6 +78,7 @@ struct SmallArgs {
     uint32_t feat[256];
 };
 #define SMALL_NUMERIC (1u << 16)
+#define SMALL_ABSENT 1u // no split
 
 __device__ __forceinline__ long long shfl_i64(long long v, int src) {
     const int lo = __shfl((int)(v & 0xffffffffll), src), hi = __shfl((int)(v >> 32), src);
@@ -95,23 +96,19 @@ __device__ __forceinline__ double lane_stat(const SmallArgs &A, long long q, dou
     if (two && lane == 1) v = (A.loss == EVT_LOSS_MSE) ? 2.0 * v : 0.0;
     return v;
 }
-// a node's weight and, for a leaf, its values (leaf_value, an output per lane), in the tree's arrays (writer) and in s_leaf where rows will ask for them
-__device__ __forceinline__ void write_node(const SmallArgs &A, int n, long long q, double sc, int lane, bool leaf, bool writer, float *s_leaf) {
+// a node's weight and, for a leaf, its values (leaf_value, an output per lane)
+__device__ __forceinline__ void write_node(const SmallArgs &A, int n, long long q, double sc, int lane, bool leaf) {
     const double S = lane_stat(A, q, sc, lane);
     double v[3] = {shfl_f64(S, lane < A.K ? lane : 0), shfl_f64(S, A.K + (lane < A.K ? lane : 0)), shfl_f64(S, 2 * A.K)};
-    if (writer && lane == 0) A.tree.w[n - 1] = (float)v[2];
-    if (leaf && lane < A.K) {
-        const float val = (float)leaf_value(A.loss, v, 0, 1, A.eta, A.bagging, A.lambda, A.L2);
-        if (writer) A.tree.pred[(int64_t)A.K * (n - 1) + lane] = val;
-        if (s_leaf) s_leaf[lane] = val;
-    }
+    if (lane == 0) A.tree.w[n - 1] = (float)v[2];
+    if (leaf && lane < A.K) A.tree.pred[(int64_t)A.K * (n - 1) + lane] = (float)leaf_value(A.loss, v, 0, 1, A.eta, A.bagging, A.lambda, A.L2);
 }
 
 // The decision for node p of the level above `A.level`, by one wavefront: the best of the blocks' candidates (highest gain, then
 // earliest feature; its bin is already the lowest).  Leaves the packed split in s_dec[p] (0: none) and the children's totals in
-// s_tot; the writer block also writes the Tree arrays and the children's state.  s_leaf (last level): the values of the leaves among the
-// nodes of the level above, then among the level's own.
-__device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t *s_dec, long long *s_tot, bool writer, int lane, float *s_leaf = nullptr) {
+// s_tot; the writer block also writes the Tree arrays and the children's state.  s_own: the nodes' own totals are left there instead of their
+// weight and values in the tree's arrays, and SMALL_ABSENT in s_dec[p] where the level did not reach the node (small_leaves).
+__device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t *s_dec, long long *s_tot, bool writer, int lane, long long *s_own = nullptr) {
     const int n = (1 << (A.level - 2)) + p, nag = A.NAg, nwg = A.nfs;
     const int st = A.status[n];
     const long long qn = A.node_sum[(int64_t)n * nag + (lane < nag ? lane : 0)];
@@ -165,14 +162,15 @@ __device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t
             ql = lane < nag ? A.left_in[((int64_t)p * nwg + wj) * nag + lane] : 0;
         }
     }
-    if (lane == 0) s_dec[p] = packed;
+    if (lane == 0) s_dec[p] = s_own && !active ? SMALL_ABSENT : packed;
     if (lane < nag) {
         s_tot[(2 * p) * nag + lane] = ql;
         s_tot[(2 * p + 1) * nag + lane] = qn - ql;
+        if (s_own) s_own[p * nag + lane] = qn;
     }
-    if (!active || !(writer || s_leaf)) return;
-    write_node(A, n, qn, sc, lane, !found, writer, s_leaf ? s_leaf + p * A.K : nullptr);
-    if (writer && lane == 0) {
+    if (!active || !writer) return;
+    if (!s_own) write_node(A, n, qn, sc, lane, !found);
+    if (lane == 0) {
         A.status[n] = found ? ST_SPLIT : ST_LEAF;
         if (found) {
             A.tree.feat[n - 1] = feat;
@@ -186,11 +184,33 @@ __device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t
     for (int child = 0; child < 2; child++) {
         const int cn = 2 * n + child;
         const long long qc = child ? qn - ql : ql;
-        if (writer) {
-            if (lane < nag) A.node_sum[(int64_t)cn * nag + lane] = qc;
-            if (lane == 0) A.status[cn] = A.level < A.D ? ST_BUILD : ST_LEAF;
+        if (lane < nag) A.node_sum[(int64_t)cn * nag + lane] = qc;
+        if (lane == 0) A.status[cn] = A.level < A.D ? ST_BUILD : ST_LEAF;
+        if (A.level == A.D && !s_own) write_node(A, cn, qc, sc, lane, true);
+    }
+}
+
+// Weights and leaf values of the last two levels, behind the decisions that left their totals in LDS: a thread per node, where a wavefront that wrote three
+// nodes behind each of its decisions paid their divisions one after the other in every block (rounds, us: 21k rows x 19 features, depth 10 196 -> 183, 9.5k x 7,
+// depth 8 174 -> 170, 27k x 65 of two outputs, depth 8 176 -> 172).  s_leaf: the leaves' values, from node np on.
+template <int K>
+__device__ __forceinline__ void small_leaves(const SmallArgs &A, const uint32_t *s_dec, const long long *s_own, const long long *s_tot, int np, bool writer, const double *sc, float *s_leaf) {
+    for (int i = threadIdx.x; i < 3 * np; i += 1024) {
+        const bool child = i >= np;
+        const uint32_t d = s_dec[child ? (i - np) >> 1 : i];
+        const bool split = (d & EVT_NODE_SPLIT) != 0;
+        if (child ? !split : d == SMALL_ABSENT) continue;
+        double S[2 * K + 1];
+        decode_vals(child ? s_tot + (i - np) * A.NAg : s_own + i * A.NAg, sc, A.loss, 2 * K + 1, S);
+        const int n = np + i;
+        if (writer) A.tree.w[n - 1] = (float)S[2 * K];
+        if (split && !child) continue;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const float v = (float)leaf_value(A.loss, S, k, K, A.eta, A.bagging, A.lambda, A.L2);
+            if (writer) A.tree.pred[(int64_t)K * (n - 1) + k] = v;
+            s_leaf[K * i + k] = v;
         }
-        if (A.level == A.D) write_node(A, cn, qc, sc, lane, true, writer, s_leaf ? s_leaf + ((1 << (A.level - 2)) + 2 * p + child) * A.K : nullptr);
     }
 }
 
@@ -922,7 +942,11 @@ __global__ __launch_bounds__(1024) void k_small_final(SmallArgs A) {
     touch_args(A);
     const int np = 1 << (A.level - 2);
     long long *s_tot = reinterpret_cast<long long *>(s_dyn);
-    float *s_leaf = GRADS ? reinterpret_cast<float *>(s_tot + 2 * np * A.NAg) : nullptr;
+    long long *s_own = GRADS ? s_tot + 2 * np * A.NAg : nullptr;
+    float *s_leaf = GRADS ? reinterpret_cast<float *>(s_own + np * A.NAg) : nullptr;
+    double sc[NK];
+#pragma unroll
+    for (int a = 0; a < NK; a++) sc[a] = A.qscale[a];
     // the block's first rows are requested before the decisions; a block has more where there are more than 256 x 1024 of them
     uint32_t nid;
     float pr[K], y = 0.0f, w = 1.0f, mx[2 * K];
@@ -962,9 +986,13 @@ __global__ __launch_bounds__(1024) void k_small_final(SmallArgs A) {
     };
     const int r0 = (int)blockIdx.x * 1024 + tid;
     request(r0);
-    if (wave < np) small_decide(A, wave, s_dec, s_tot, writer, lane, s_leaf);
-    for (int p = wave + 16; p < np; p += 16) small_decide(A, p, s_dec, s_tot, writer, lane, s_leaf);
+    if (wave < np) small_decide(A, wave, s_dec, s_tot, writer, lane, s_own);
+    for (int p = wave + 16; p < np; p += 16) small_decide(A, p, s_dec, s_tot, writer, lane, s_own);
     __syncthreads();
+    if constexpr (GRADS) {
+        small_leaves<K>(A, s_dec, s_own, s_tot, np, writer, sc, s_leaf);
+        __syncthreads();
+    }
     finish(r0);
     for (int r = r0 + (int)gridDim.x * 1024; r < A.N; r += (int)gridDim.x * 1024) {
         request(r);
@@ -1155,7 +1183,7 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
             A.grad = c->grad;
             A.maxima = absmax_set(c, c->absmax_cur);
             A.unit_w = c->unit_w ? 1 : 0;
-            const size_t lds = (size_t)(1 << (level - 1)) * c->NAg * 8 + (c->step.grads_done ? (size_t)3 * (1 << (level - 2)) * c->K * 4 : 0);
+            const size_t lds = (size_t)(1 << (level - 1)) * c->NAg * 8 + (c->step.grads_done ? (size_t)(1 << (level - 2)) * (c->NAg * 8 + 3 * c->K * 4) : 0);
             // no more blocks than are resident at once: a second generation would take the decisions again
 #define FINAL(L_) hipLaunchKernelGGL(k_small_final<L_>, dim3((unsigned)std::min<int64_t>(256, (c->N + 1023) / 1024)), dim3(1024), lds, c->stream, A)
             if (!c->step.grads_done) FINAL(-1);

@@ -172,6 +172,7 @@ def test_gradients_quantised_by_the_tree_or_not(evt, N, B, loss, K):
     (530_001, 4, "logloss", dict(sub=True, weights=True)),  # the walk over all rows behind a sampled tree: wide blocks
     (2_097_153, 3, "mse", dict(sub=True)),             # ... and four rows a thread
     (5003, 10, "mse", dict(min_weight=40.0)),          # most leaves above the last level
+    (4001, 10, "gaussian_mle", dict(weights=True, min_weight=9.0)),  # nodes of the last two levels that no level reached
 ])
 def test_gradients_behind_the_tree(evt, N, D, loss, more):
     """With "grads_ahead" a small tree's last kernel adds the leaf values and computes the next gradients: the bits that the kernels of larger inputs
