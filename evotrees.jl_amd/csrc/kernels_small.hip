@@ -113,7 +113,9 @@ __device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t
     const int st = A.status[n];
     const long long qn = A.node_sum[(int64_t)n * nag + (lane < nag ? lane : 0)];
     const double sc = A.qscale[lane_channel(A, lane)];
-    // every lane reads whole candidates (one line each), so that the winner's feature and totals are at hand
+    // Up to 64 candidates: every lane reads a whole one (one line), so that the winner's feature and totals are at hand.  More: their first 16 bytes, and the
+    // winner's totals in a second trip - every block of the launch reads all of a level's candidates, and whole ones are what its reads took longest for
+    // (rounds, us, whole | first bytes: 1350 rows x 229 features, depth 10 275 | 218, 13k x 156, oblivious of depth 9 173 | 151, 985 x 100 and 250, depth 5 42.4 | 41.8, 46.9 | 44.7).
     const SmallHead *hp = A.head_in + (int64_t)p * nwg;
     union Words {
         SmallHead h;
@@ -123,17 +125,30 @@ __device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t
     mine.h.bin = NO_BIN;
     mine.h.feat = 0;
     int bj = NO_BIN;
-    for (int w = lane; w < ((nwg + 63) & ~63); w += 64) {
+    const bool whole = nwg <= 64;
+    if (whole) {
         Words c;
-        const uint4 *cp = reinterpret_cast<const uint4 *>(hp + (w < nwg ? w : nwg - 1));
+        const uint4 *cp = reinterpret_cast<const uint4 *>(hp + (lane < nwg ? lane : nwg - 1));
 #pragma unroll
         for (int k = 0; k < 4; k++) c.v[k] = cp[k];
 #pragma unroll
         for (int k = 0; k < 4; k++) // all of it now: the compiler fetches the totals behind the comparison of the gains, a second trip to memory
             asm volatile("" : "+v"(c.v[k].x), "+v"(c.v[k].y), "+v"(c.v[k].z), "+v"(c.v[k].w));
-        if (w < nwg && c.h.gain > mine.h.gain) {
+        if (lane < nwg && c.h.gain > mine.h.gain) {
             mine = c;
-            bj = w;
+            bj = lane;
+        }
+    } else {
+        for (int w0 = lane; w0 < nwg; w0 += 128) { // two of a lane under way at a time
+            Words c[2];
+#pragma unroll
+            for (int u = 0; u < 2; u++) c[u].v[0] = *reinterpret_cast<const uint4 *>(hp + (w0 + 64 * u < nwg ? w0 + 64 * u : nwg - 1));
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+                if (w0 + 64 * u < nwg && c[u].h.gain > mine.h.gain) {
+                    mine.v[0] = c[u].v[0];
+                    bj = w0 + 64 * u;
+                }
         }
     }
     double bg = mine.h.gain;
@@ -147,12 +162,15 @@ __device__ __forceinline__ void small_decide(const SmallArgs &A, int p, uint32_t
     int feat = 0, bin = 0;
     if (found) {
         const int owner = wj & 63;
+        const long long own_left = !whole && nag <= EVT_MAX_NA && lane < nag ? hp[wj].left[lane] : 0;
         bin = __shfl(mine.h.bin, owner);
         feat = __shfl(mine.h.feat, owner);
         const bool numeric = feat > 0;
         feat = numeric ? feat : -feat;
         packed = evt_pack_node(feat, bin, numeric);
-        if (nag <= EVT_MAX_NA) {
+        if (!whole && nag <= EVT_MAX_NA) {
+            ql = own_left;
+        } else if (nag <= EVT_MAX_NA) {
 #pragma unroll
             for (int ag = 0; ag < EVT_MAX_NA; ag++) {
                 const long long v = shfl_i64(mine.h.left[ag], owner);
