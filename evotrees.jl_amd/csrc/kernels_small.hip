@@ -1054,8 +1054,11 @@ static size_t small_lds_search(const evt_ctx *c, int level, int batch) {
 // The search of two outputs of more than 64 bins, or of one output of three channels and more than 128, holds too many registers to sit in the level's kernel
 // (42k rows x 44, 255 bins, depth 5, 64 rounds: in it 13.4 ms, apart 11.9; 4837 x 18, oblivious of depth 8, 133 rounds 35.5 | 27.1; a round of three
 // channels x 192 bins, 74k x 3, depth 5 105 | 88 us, of 160 bins, 11k x 206, oblivious of depth 8 310 | 224), and an oblivious level is taken apart where
-// LDS holds the sums of fewer than 16 nodes.
-static bool small_scan_apart(const evt_ctx *c, int nodes) {
+// LDS holds the sums of fewer than 16 nodes.  More blocks than compute units (one to each): a block that searches holds back those that have yet to walk (20k rows
+// and fewer x 220 features, depth 9, every level in the last block | apart: two outputs of 32 bins 405 | 333 us a round, one of 64 bins 354 | 273, oblivious 215 | 190;
+// of 128 features, 256 blocks, oblivious 125 | 132).
+static bool small_scan_apart(const evt_ctx *c, int nodes, int blocks) {
+    if (blocks > 256) return true;
     if (!c->mc && small_search_large(c->NAg, bins_per_lane(c->B))) return true;
     if (c->tree_type == EVT_TREE_OBLIVIOUS) return (size_t)std::min(16, nodes) * c->NAg * c->B * 8 > 72 * 1024;
     return nodes > 16 || (int64_t)nodes * c->NAg * c->B > 5120;
@@ -1217,7 +1220,7 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
         if (split) { // a wavefront per node at a time, as far as they fit
             A.batch = std::min(16, nodes);
             while (A.batch > 1 && small_lds_search(c, level, A.batch) > std::max<size_t>(lds, 72 * 1024)) A.batch >>= 1;
-            A.apart = small_scan_apart(c, nodes) ? 1 : 0;
+            A.apart = small_scan_apart(c, nodes, c->n_js_last * slices) ? 1 : 0;
             if (!A.apart) lds = std::max(lds, small_lds_search(c, level, A.batch));
         }
         prof_begin(c, level == 1 ? EVT_K_HIST : EVT_K_PARTITION, level); // below the root it moves rows, builds and searches at once

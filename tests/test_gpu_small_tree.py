@@ -21,7 +21,8 @@ pytestmark = pytest.mark.gpu
     (1500, 64, 8, 5, "mse", {}),                                      # a candidate to a lane, and one more
     (1500, 65, 8, 5, "gaussian_mle", dict(weights=True)),
     (1700, 193, 8, 7, "logloss", dict(oblivious=True, cat=True)),
-    (1300, 129, 8, 5, "mlogloss", dict(K=3)),
+    (1300, 129, 8, 5, "mlogloss", dict(K=3)),                         # two blocks each are more than the chip has units: searched apart
+    (1300, 128, 8, 5, "mse", dict(oblivious=True)),
     (6001, 9, 32, 6, "gaussian_mle", dict(cat=True, mono=True)),
     (6001, 9, 100, 6, "mse", dict(cat=True, mono=True, sub="mask")),
     (5003, 12, 64, 7, "gaussian_mle", dict(oblivious=True)),
