@@ -232,6 +232,9 @@ __device__ __forceinline__ void small_leaves(const SmallArgs &A, const uint32_t 
     }
 }
 
+// a value that is the same in every lane, in scalar registers
+__device__ __forceinline__ double uniform_f64(double v) { return __longlong_as_double(readlane_i64(__double_as_longlong(v), 0)); }
+
 // where a row of the level above goes: the decision its node took (0: none, a leaf further up stays), the bin byte that decides, the
 // node it moves to
 __device__ __forceinline__ uint32_t row_decision(const SmallArgs &A, uint32_t nid, const uint32_t *s_dec) {
@@ -271,10 +274,19 @@ __device__ __forceinline__ long long channel_of(const unsigned long long *H, int
     return ag == 0 ? (long long)w >> EVT_PACK_CNT_BITS : (long long)w;
 }
 
+// Searches of this many channels (0: a run-time count) and bins to a lane (1, 2 or 4) hold too many registers to sit in a level's kernel (small_scan_apart).  Compiled
+// into it and never run, they still spilt its registers (108 to 340 bytes a lane, now none; rounds of two outputs: 42k rows x 44 features, 255 bins,
+// depth 5 147.0 -> 145.0 us, 20k x 6, depth 9 332 -> 327).
+constexpr bool small_search_large(int channels, int bins) { return channels * bins >= 10; }
+static int bins_per_lane(int B) { return B <= 64 ? 1 : B <= 128 ? 2 : 4; }
+
 // The search of one (node, feature) by one wavefront.  NAG: global channels (2, 3, 5), or 0 when their number is known at run time
 // only.  on_gain(b, ok, gain, left) is called for every bin of the lane; left: the totals left of it (NAG channels; NAG == 0: null).
 // Returns the node's totals in q (NAG != 0).
-template <int NAG, int BPL, bool PACK, typename GAIN>
+// FEW: the node's totals and the scales are kept in scalar registers.  In a level's kernel a large search (small_search_large) spills less by it; elsewhere the moves cost
+// more than they give (rounds, us, without | with: two outputs, 3005 rows x 41 features x 100 bins, depth 9 206 | 177, 955 x 93 x 255, depth 7 188 | 177; of 64 bins, 5306 x 36,
+// depth 10 236 | 241; in k_small_scan, 429 x 105 x 160 bins, oblivious of depth 9 188 | 200).
+template <int NAG, int BPL, bool PACK, bool FEW, typename GAIN>
 __device__ __forceinline__ void small_scan(const SmallArgs &A, const double *qs, const unsigned long long *H, const long long *tot, bool numeric, int constraint, int lane,
                                            long long *hist_out, long long *q, GAIN on_gain) {
     const int B = A.B, nag = NAG ? NAG : A.NAg;
@@ -285,7 +297,7 @@ __device__ __forceinline__ void small_scan(const SmallArgs &A, const double *qs,
         double sc[NAG], S[NK];
 #pragma unroll
         for (int ag = 0; ag < NAG; ag++) {
-            sc[ag] = qs[ag];
+            sc[ag] = FEW ? uniform_f64(qs[ag]) : qs[ag];
             long long val[BPL], run = 0;
 #pragma unroll
             for (int t = 0; t < BPL; t++) {
@@ -296,7 +308,9 @@ __device__ __forceinline__ void small_scan(const SmallArgs &A, const double *qs,
                 left[ag][t] = run;
             }
             const long long incl = wave_incl_scan_i64(run), excl = incl - run;
-            q[ag] = tot ? tot[ag] : shfl_i64(incl, 63); // the root's totals are the sums over any feature's bins
+            // the root's totals are the sums over any feature's bins
+            if (FEW) q[ag] = tot ? readlane_i64(tot[ag], 0) : readlane_i64(incl, 63);
+            else q[ag] = tot ? tot[ag] : shfl_i64(incl, 63);
 #pragma unroll
             for (int t = 0; t < BPL; t++) left[ag][t] = numeric ? left[ag][t] + excl : val[t];
         }
@@ -396,7 +410,7 @@ __device__ __forceinline__ void small_left(const SmallArgs &A, const unsigned lo
 
 // The search of one (node, feature) and what it leaves: the node's histogram of the feature, the candidate - or, for an oblivious
 // level, the gains of all bins in s_gain - and at the root the node's totals.
-template <int NAG, int BPL, bool PACK>
+template <int NAG, int BPL, bool PACK, bool FEW>
 __device__ __forceinline__ void small_search(const SmallArgs &A, const double *qs, const unsigned long long *Hs, int q, int jp, int nwg, uint32_t fw, const long long *tot,
                                              bool writer, double *s_gain, int lane) {
     const int B = A.B, nag = NAG ? NAG : A.NAg, n = (1 << (A.level - 1)) + q;
@@ -409,7 +423,7 @@ __device__ __forceinline__ void small_search(const SmallArgs &A, const double *q
     long long tq[QA], lq[QA];
 #pragma unroll
     for (int ag = 0; ag < QA; ag++) lq[ag] = 0;
-    small_scan<NAG, BPL, PACK>(A, qs, Hs, tot, numeric, (int)(fw >> 17) - 1, lane, hout, tq, [&](int b, bool ok, double gain, const long long *left) {
+    small_scan<NAG, BPL, PACK, FEW>(A, qs, Hs, tot, numeric, (int)(fw >> 17) - 1, lane, hout, tq, [&](int b, bool ok, double gain, const long long *left) {
         if (A.oblivious) {
             if (b < B) s_gain[b] = gain; // update_gains!
         } else if (ok && gain > lg) {
@@ -457,12 +471,6 @@ __device__ __forceinline__ void small_search(const SmallArgs &A, const double *q
         if (lb != NO_BIN) small_left<PACK, false>(A, Hs, nag, numeric, lb, lane, out, A.left_out + ((int64_t)q * nwg + jp) * nag);
     }
 }
-
-// Searches of this many channels (0: a run-time count) and bins to a lane (1, 2 or 4) hold too many registers to sit in a level's kernel (small_scan_apart).  Compiled
-// into it and never run, they still spilt its registers (108 to 340 bytes a lane, now none; rounds of two outputs: 42k rows x 44 features, 255 bins,
-// depth 5 147.0 -> 145.0 us, 20k x 6, depth 9 332 -> 327).
-constexpr bool small_search_large(int channels, int bins) { return channels * bins >= 10; }
-static int bins_per_lane(int B) { return B <= 64 ? 1 : B <= 128 ? 2 : 4; }
 
 // Requests every 64-byte line of the arguments at once: read where each is needed, they were ten trips one after the other.
 __device__ __forceinline__ void touch_args(const SmallArgs &A) {
@@ -783,7 +791,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
         } else
         for (int s = wave; s < ns; s += 16) {
             const int q = s_node[base + s];
-            small_search<NAG, BPL, PACK>(A, s_qs, H + (size_t)s * na * B, q, jp, A.nfs, fw, level > 1 ? s_tot + q * nag : nullptr, writer,
+            small_search<NAG, BPL, PACK, small_search_large(NAG, BPL)>(A, s_qs, H + (size_t)s * na * B, q, jp, A.nfs, fw, level > 1 ? s_tot + q * nag : nullptr, writer,
                                          A.oblivious ? s_gain + s * B : nullptr, lane);
         }
         __syncthreads();
@@ -846,7 +854,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
             __syncthreads();
             for (int k = wave; k < nb; k += 16) {
                 const int q = s_node[base + k];
-                small_search<NAG, BPL, false>(A, s_qs, S + (size_t)k * words, q, jp, A.nfs, fw, level > 1 ? s_tot + q * nag : nullptr, jp == 0,
+                small_search<NAG, BPL, false, false>(A, s_qs, S + (size_t)k * words, q, jp, A.nfs, fw, level > 1 ? s_tot + q * nag : nullptr, jp == 0,
                                               A.oblivious ? gains + (base + k) * B : nullptr, lane);
             }
             __syncthreads();
@@ -895,7 +903,7 @@ __global__ __launch_bounds__(1024) void k_small_scan(SmallArgs A) {
     if (tid < nag) s_qs[tid] = A.qscale[tid];
     auto sums = [&](int q) { return A.acc + ((size_t)q * A.nfs + jp) * words; };
     auto search = [&](int q, double *gain) {
-        small_search<NAG, BPL, false>(A, s_qs, reinterpret_cast<const unsigned long long *>(sums(q)), q, jp, A.nfs, fw,
+        small_search<NAG, BPL, false, false>(A, s_qs, reinterpret_cast<const unsigned long long *>(sums(q)), q, jp, A.nfs, fw,
                                       A.level > 1 ? A.node_sum + (int64_t)(first + q) * nag : nullptr, jp == 0, gain, lane);
     };
     auto clear = [&](int q) {
