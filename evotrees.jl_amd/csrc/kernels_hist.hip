@@ -715,6 +715,11 @@ static bool choose_hist16(const evt_ctx *c, int level, int na, int layers, Hist1
     const double span_atomics = (double)c->n_js_last * c->B * c->NAg;
     double least = 0;
     bool found = false;
+    // Five channels of more than 204 bins: the narrowest tile takes all of a CU.  Few sampled features of few rows are left to the generic kernel, which flushes
+    // those alone (rounds of depth 9, 255 bins, us, this kernel | generic: 17 features 80k rows 454 | 394, 300k 539 | 557; 16 of 33, 80k 599 | 534, 300k 651 | 669;
+    // 33 features 20k 472 | 445, 80k 506 | 558; 50 of 100, 5k 473 | 556; 166 features 5k 666 | 1329).
+    const double nfs = c->n_js_last;
+    const bool few = c->hist_variant == 0 && nfs <= 33 && (double)c->N * sampled * nfs * nfs < 5e7;
     for (; tw >= 16; tw >>= 1) {
         if (c->hist_tile > 0 && tw > c->hist_tile && tw > 16) continue;
         if (found && (c->hist_tile > 0 || tw * 8 < c->RS)) break; // a set width, or more than eight tiles of a choice
@@ -726,8 +731,7 @@ static bool choose_hist16(const evt_ctx *c, int level, int na, int layers, Hist1
         s.ntiles = (c->RS + tw - 1) / tw;
         const int lanes = tw / s.pb;
         s.lds = (size_t)na * c->B * lanes * s.pu * 8; // channels x bins x feature bytes of a tile, words
-        // five channels of more than 204 bins: the narrowest tile takes all of a CU (the generic kernel, 34k rows x 166 features: 138 us a level, this one 43)
-        if (s.lds > (tw == 16 && !found ? 160 : 128) * 1024) continue;
+        if (s.lds > (tw == 16 && !found && !few ? 160 : 128) * 1024) continue;
         if (tw == 16 && c->LPR > 64 && 2 * s.lds > 128 * 1024) break; // more than 1024 features whose 32-byte tiles do not fit are refused (launch_hist_build)
         const double adds = 3.2 * s.pu * na * (lanes / 16) * s.ntiles;
         const double per_row = (adds > 18 ? adds : 18) + 3.5 * (s.ntiles - 1);
