@@ -1048,7 +1048,8 @@ struct ChannelWords {
 // and leaves its outputs' terms of every bin's gain in LDS, where the first adds them in the outputs' order.  Bound by that chain - one
 // trip for all of a wavefront's channels, two scans' and two divisions' length - where one wavefront per feature went through the
 // outputs one pair after the other: 60k rows x 30 features x 64 bins of 7 classes 16.2 -> 10.2 us a level.
-template <int BPL>
+// LOOP: a wavefront takes one pair of outputs after the other.
+template <int BPL, bool LOOP>
 __global__ __launch_bounds__(64 * (EVT_MAX_K / 2)) void k_scan_mc(ScanArgs A) {
     extern __shared__ double s_term[]; // [K][B]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
@@ -1070,14 +1071,17 @@ __global__ __launch_bounds__(64 * (EVT_MAX_K / 2)) void k_scan_mc(ScanArgs A) {
     __shared__ int s_last, s_jp, s_bin;
 
     const int64_t of = (int64_t)jp * NAG * B, ow = of + (int64_t)(NAG - 1) * B; // the feature's slice; its weights
-    const int k0 = 2 * wave, k1 = k0 + 1 < K ? k0 + 1 : k0;
+    int k0 = 2 * wave, k1 = k0 + 1 < K ? k0 + 1 : k0;
     ChannelWords<BPL> cw, cg[2], ch[2];
     cw.fetch(A, hn, hp, hs, ow, is_sub, lane);
+    auto fetch = [&]() {
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        cg[j].fetch(A, hn, hp, hs, of + (int64_t)(j ? k1 : k0) * B, is_sub, lane);
-        ch[j].fetch(A, hn, hp, hs, of + (int64_t)(K + (j ? k1 : k0)) * B, is_sub, lane);
-    }
+        for (int j = 0; j < 2; j++) {
+            cg[j].fetch(A, hn, hp, hs, of + (int64_t)(j ? k1 : k0) * B, is_sub, lane);
+            ch[j].fetch(A, hn, hp, hs, of + (int64_t)(K + (j ? k1 : k0)) * B, is_sub, lane);
+        }
+    };
+    fetch();
     const bool numeric = A.feattypes[f] != 0;
     if (tid < NAG) {
         s_sc[tid] = A.qscale[tid];
@@ -1085,17 +1089,20 @@ __global__ __launch_bounds__(64 * (EVT_MAX_K / 2)) void k_scan_mc(ScanArgs A) {
     }
     long long lq[BPL], gq[2][BPL], hq[2][BPL];
     const long long tw = cw.left_sums(A, hn, ow, is_sub && wave == 0, numeric, lane, lq);
+    auto sums = [&]() {
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int k = j ? k1 : k0;
-        const long long tg = cg[j].left_sums(A, hn, of + (int64_t)k * B, is_sub, numeric, lane, gq[j]);
-        const long long th = ch[j].left_sums(A, hn, of + (int64_t)(K + k) * B, is_sub, numeric, lane, hq[j]);
-        if (A.level == 1 && lane == 0) { // the root's totals are any feature's sums over its bins
-            s_Sq[k] = tg;
-            s_Sq[K + k] = th;
-            s_Sq[2 * K] = tw; // every wavefront the same
+        for (int j = 0; j < 2; j++) {
+            const int k = j ? k1 : k0;
+            const long long tg = cg[j].left_sums(A, hn, of + (int64_t)k * B, is_sub, numeric, lane, gq[j]);
+            const long long th = ch[j].left_sums(A, hn, of + (int64_t)(K + k) * B, is_sub, numeric, lane, hq[j]);
+            if (!LOOP && A.level == 1 && lane == 0) { // the root's totals are any feature's sums over its bins
+                s_Sq[k] = tg;
+                s_Sq[K + k] = th;
+                s_Sq[2 * K] = tw; // every wavefront the same
+            }
         }
-    }
+    };
+    sums();
     __syncthreads();
     if (tid < NAG) {
         s_S[tid] = (double)s_Sq[tid] * s_sc[tid];
@@ -1103,17 +1110,25 @@ __global__ __launch_bounds__(64 * (EVT_MAX_K / 2)) void k_scan_mc(ScanArgs A) {
     }
     const double scw = s_sc[NAG - 1], w_p = (double)s_Sq[NAG - 1] * scw;
     if (tid < K) s_gp[tid] = node_gain_k(A.loss, (double)s_Sq[tid] * s_sc[tid], (double)s_Sq[K + tid] * s_sc[K + tid], w_p, A.lambda, A.L2);
+    for (;;) {
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int k = j ? k1 : k0;
-        const double scg = s_sc[k], sch = s_sc[K + k], Sg = (double)s_Sq[k] * scg, Sh = (double)s_Sq[K + k] * sch;
+        for (int j = 0; j < 2; j++) {
+            const int k = j ? k1 : k0;
+            const double scg = s_sc[k], sch = s_sc[K + k], Sg = (double)s_Sq[k] * scg, Sh = (double)s_Sq[K + k] * sch;
 #pragma unroll
-        for (int t = 0; t < BPL; t++) {
-            const int b = lane * BPL + t;
-            const double w_l = (double)lq[t] * scw;
-            const double term = split_gain_k(A.loss, Sg, Sh, w_p, (double)gq[j][t] * scg, (double)hq[j][t] * sch, w_l, w_p - w_l, A.lambda, A.L2);
-            if (b < B) s_term[k * B + b] = term;
+            for (int t = 0; t < BPL; t++) {
+                const int b = lane * BPL + t;
+                const double w_l = (double)lq[t] * scw;
+                const double term = split_gain_k(A.loss, Sg, Sh, w_p, (double)gq[j][t] * scg, (double)hq[j][t] * sch, w_l, w_p - w_l, A.lambda, A.L2);
+                if (b < B) s_term[k * B + b] = term;
+            }
         }
+        if (!LOOP) break;
+        k0 += 2 * nwaves;
+        if (k0 >= K) break;
+        k1 = k0 + 1 < K ? k0 + 1 : k0;
+        fetch();
+        sums();
     }
     __syncthreads();
     if (wave == 0) {
@@ -1202,29 +1217,32 @@ __global__ __launch_bounds__(64 * (EVT_MAX_K / 2)) void k_scan_mc(ScanArgs A) {
         if (tid < K) A.tree.pred[(int64_t)K * (n - 1) + tid] = (float)leaf_value(A.loss, s_S, tid, K, A.eta, A.bagging, A.lambda, A.L2);
         return;
     }
-    // the children's totals, all of a wavefront's channels (five at most) requested at once; a subtract node's own slice was written by
-    // other blocks, so it is its parent's less its sibling's here too
+    // the children's totals, five of a wavefront's channels (all of them where it has two outputs) requested at once; a subtract node's own slice was
+    // written by other blocks, so it is its parent's less its sibling's here too
     const bool num = A.feattypes[A.js[bj] - 1] != 0;
-    ChannelWords<BPL> cc[5];
+    for (int ag0 = wave; ag0 < NAG; ag0 += 5 * nwaves) {
+        ChannelWords<BPL> cc[5];
 #pragma unroll
-    for (int j = 0; j < 5; j++) {
-        const int ag = wave + j * nwaves < NAG ? wave + j * nwaves : NAG - 1;
-        cc[j].fetch(A, hn, hp, hs, ((int64_t)bj * NAG + ag) * B, is_sub, lane);
-    }
-#pragma unroll
-    for (int j = 0; j < 5; j++) {
-        const int ag = wave + j * nwaves;
-        long long s = 0;
-#pragma unroll
-        for (int t = 0; t < BPL; t++) {
-            const int b = lane * BPL + t;
-            if (b < B && (num ? b + 1 <= bb : b + 1 == bb)) s += cc[j].a[t] - cc[j].b[t];
+        for (int j = 0; j < 5; j++) {
+            const int ag = ag0 + j * nwaves < NAG ? ag0 + j * nwaves : NAG - 1;
+            cc[j].fetch(A, hn, hp, hs, ((int64_t)bj * NAG + ag) * B, is_sub, lane);
         }
-        s = wave_sum_i64(s);
-        if (lane == 0 && ag < NAG) {
-            A.node_sum[(int64_t)(2 * n) * NAG + ag] = s;
-            A.node_sum[(int64_t)(2 * n + 1) * NAG + ag] = s_Sq[ag] - s;
+#pragma unroll
+        for (int j = 0; j < 5; j++) {
+            const int ag = ag0 + j * nwaves;
+            long long s = 0;
+#pragma unroll
+            for (int t = 0; t < BPL; t++) {
+                const int b = lane * BPL + t;
+                if (b < B && (num ? b + 1 <= bb : b + 1 == bb)) s += cc[j].a[t] - cc[j].b[t];
+            }
+            s = wave_sum_i64(s);
+            if (lane == 0 && ag < NAG) {
+                A.node_sum[(int64_t)(2 * n) * NAG + ag] = s;
+                A.node_sum[(int64_t)(2 * n + 1) * NAG + ag] = s_Sq[ag] - s;
+            }
         }
+        if (!LOOP) break;
     }
 }
 
@@ -1337,6 +1355,12 @@ bool scan_folds_leaves(const evt_ctx *c) { return !c->mc && c->D > 1 && (c->tree
 
 static int launch_obliv_level(evt_ctx *c, int level, const evt_params *p);
 
+// Whether two wavefronts take a block's pairs of outputs one after the other: blocks of five to seven wavefronts leave a compute unit places for too few of them
+// when a level is generations of blocks (rounds of depth 9, 3000 rows x 250 features, us, a wavefront to each pair | two: 10 classes 64 bins 1121 | 1021, 128 1722 |
+// 1607, 160 2740 | 2477, 255 3499 | 3204, 13 classes 1457 | 1287, 2166 | 2087, 3224 | 3201, 4483 | 4279; 7 classes, four wavefronts, 753 | 753, 1183 | 1184,
+// 1782 | 1883; 16 classes, eight, 160 bins 3596 | 3660; levels of at most 2560 blocks, 13 classes x 160 bins, depth 9, 479 | 488).
+static bool scan_mc_loops(const evt_ctx *c, int level) { return level > 1 && c->K > 8 && c->K < 15 && ((int64_t)c->n_js_last << (level - 1)) >= 8192; }
+
 int launch_scan(evt_ctx *c, int level, const evt_params *p, bool leaf_level) {
     if (!leaf_level && obliv_one_launch(c, level)) return launch_obliv_level(c, level, p);
     ScanArgs A;
@@ -1371,11 +1395,17 @@ int launch_scan(evt_ctx *c, int level, const evt_params *p, bool leaf_level) {
     A.last_decides = !leaf_level && !A.oblivious && c->scan_fused ? 1 : 0;
     if (c->mc) { // any number of outputs: multi-class, several targets
         if (!leaf_level) { // a block per node and feature; two outputs to a wavefront
-            const dim3 per_feature(nodes, (unsigned)A.nfs), block(64u * (((unsigned)c->K + 1) / 2));
+            const unsigned pairs = ((unsigned)c->K + 1) / 2;
+            const bool loop = scan_mc_loops(c, level);
+            const dim3 per_feature(nodes, (unsigned)A.nfs), block(64u * (loop ? 2 : pairs));
             const size_t lds = (size_t)c->K * c->B * sizeof(double);
-            if (bpl == 1) hipLaunchKernelGGL((k_scan_mc<1>), per_feature, block, lds, c->stream, A);
-            else if (bpl == 2) hipLaunchKernelGGL((k_scan_mc<2>), per_feature, block, lds, c->stream, A);
-            else hipLaunchKernelGGL((k_scan_mc<4>), per_feature, block, lds, c->stream, A);
+#define MCCASE(BPL_)                                                                                             \
+    if (loop) hipLaunchKernelGGL((k_scan_mc<BPL_, true>), per_feature, block, lds, c->stream, A);                \
+    else hipLaunchKernelGGL((k_scan_mc<BPL_, false>), per_feature, block, lds, c->stream, A);
+            if (bpl == 1) { MCCASE(1) }
+            else if (bpl == 2) { MCCASE(2) }
+            else { MCCASE(4) }
+#undef MCCASE
         }
         if (leaf_level || (!A.oblivious && !A.last_decides))
             hipLaunchKernelGGL(k_scan_fin_mc, dim3(nodes, !leaf_level && A.zero_children ? 1 + zero_blocks_per_node(nodes) : 1), dim3(256), 0, c->stream, A, A.nfs);

@@ -39,6 +39,9 @@ def test_class_gradients_and_their_maxima(evt, N, K):
     (2_001, 5, 255, 4, 16, 5, "binary", False),    # the largest block
     (40, 4, 64, 6, 3, 4, "binary", True),          # empty nodes and leaves at every level
     (4_001, 6, 65, 5, 5, 6, "oblivious", False),
+    (6_001, 258, 16, 8, 9, 256, "binary", True),    # from 32 nodes of 256 features on two wavefronts take the pairs of 9 to 14 outputs in turn
+    (5_001, 129, 70, 8, 14, 128, "oblivious", False),
+    (3_001, 256, 129, 7, 10, 256, "binary", False),
 ])
 def test_search_of_many_outputs(evt, N, F, B, D, K, n_js, tt, cat):
     rng = np.random.default_rng(N)
