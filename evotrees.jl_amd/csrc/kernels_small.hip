@@ -1056,20 +1056,20 @@ static size_t small_lds_search(const evt_ctx *c, int level, int batch) {
     return tot + (c->tree_type == EVT_TREE_OBLIVIOUS ? nodes * c->B * 8 : 0) + (size_t)batch * c->NAg * c->B * 8;
 }
 // Whether a level's searches take a kernel of their own.  The last of a feature's blocks reads its nodes' sums, 1024 words at a time, and its 16 wavefronts search
-// them, where that kernel spreads them over the chip for a launch more.  20k rows, us a level, the last block | apart with the gap between its
-// launches: one output of 64 bins 4 nodes 11 | 14, 16 nodes 16 | 16, 32 nodes 22 | 18, 64 nodes 31 | 21; of 255 bins 4 nodes 16 | 17, 8 nodes 20 | 18, 32
-// nodes 40 | 29; two outputs of 64 bins 8 nodes 16 | 16, 16 nodes 20 | 19, 128 nodes 45 | 25.
+// them, where that kernel spreads them over the chip for a launch more: apart from the first level on whose sums are 1024 words, which is where rounds of 4 to 128
+// features are best as a fit queues them (in the last block up to 512 | 1023 | 5120 words, us: one output of 64 bins, 30k rows x 8, depth 9 156 | 157 | 160, 15k x 60,
+// depth 8 126 | 125 | 127; of 128 bins 30k x 10, depth 9 174 | 174 | 178; two outputs of 64 bins 30k x 14, depth 9 208 | 208 | 214, 15k x 20, depth 8 151 | 151 | 155).
+// A block searches the many channels of several outputs at once longer: there up to 5120 words (3 classes, 64 bins, 15k x 30, depth 6 in it to 1023 | 5120 words: 1.02 | 1.00).
 // The search of two outputs of more than 64 bins, or of one output of three channels and more than 128, holds too many registers to sit in the level's kernel
 // (42k rows x 44, 255 bins, depth 5, 64 rounds: in it 13.4 ms, apart 11.9; 4837 x 18, oblivious of depth 8, 133 rounds 35.5 | 27.1; a round of three
-// channels x 192 bins, 74k x 3, depth 5 105 | 88 us, of 160 bins, 11k x 206, oblivious of depth 8 310 | 224), and an oblivious level is taken apart where
-// LDS holds the sums of fewer than 16 nodes.  More blocks than compute units (one to each): a block that searches holds back those that have yet to walk (20k rows
-// and fewer x 220 features, depth 9, every level in the last block | apart: two outputs of 32 bins 405 | 333 us a round, one of 64 bins 354 | 273, oblivious 215 | 190;
-// of 128 features, 256 blocks, oblivious 125 | 132).
+// channels x 192 bins, 74k x 3, depth 5 105 | 88 us, of 160 bins, 11k x 206, oblivious of depth 8 310 | 224).  More blocks than compute units (one to each): a
+// block that searches holds back those that have yet to walk (20k rows and fewer x 220 features, depth 9, every level in the last block | apart: two outputs of
+// 32 bins 405 | 333 us a round, one of 64 bins 354 | 273, oblivious 215 | 190; of 128 features, 256 blocks, oblivious 125 | 132).
 static bool small_scan_apart(const evt_ctx *c, int nodes, int blocks) {
     if (blocks > 256) return true;
     if (!c->mc && small_search_large(c->NAg, bins_per_lane(c->B))) return true;
     if (c->tree_type == EVT_TREE_OBLIVIOUS) return (size_t)std::min(16, nodes) * c->NAg * c->B * 8 > 72 * 1024;
-    return nodes > 16 || (int64_t)nodes * c->NAg * c->B > 5120;
+    return nodes > 16 || (int64_t)nodes * c->NAg * c->B > (c->mc ? 5120 : 1023);
 }
 // histograms a block's LDS holds at the deepest level that splits
 static int small_slots(const evt_ctx *c, bool split) {

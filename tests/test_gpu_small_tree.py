@@ -38,7 +38,9 @@ pytestmark = pytest.mark.gpu
     (4001, 6, 255, 5, "gaussian_mle", dict(sub="mask")),
     (5001, 4, 128, 7, "gaussian_mle", {}),
     (6007, 3, 200, 8, "mse", dict(oblivious=True)),
-    (7001, 3, 160, 7, "mse", dict(weights=True)),                    # 16 nodes of 320 words: the last that stays
+    (7001, 3, 160, 7, "mse", dict(weights=True)),                    # two nodes of 320 words are the last that stay
+    (3001, 5, 64, 6, "mse", {}),                                      # eight nodes are 1024 words: apart; of 63 bins they stay
+    (3001, 5, 63, 6, "mse", {}),
     (5001, 5, 192, 6, "logloss", dict(weights=True)),                # three channels, four bins to a lane: searched apart from the root on
     (5001, 4, 160, 6, "cred_var", dict(oblivious=True)),
     (5001, 4, 128, 6, "poisson", dict(oblivious=True, sub="drawn")),
