@@ -1064,11 +1064,13 @@ static size_t small_lds_search(const evt_ctx *c, int level, int batch) {
 // (42k rows x 44, 255 bins, depth 5, 64 rounds: in it 13.4 ms, apart 11.9; 4837 x 18, oblivious of depth 8, 133 rounds 35.5 | 27.1; a round of three
 // channels x 192 bins, 74k x 3, depth 5 105 | 88 us, of 160 bins, 11k x 206, oblivious of depth 8 310 | 224).  More blocks than compute units (one to each): a
 // block that searches holds back those that have yet to walk (20k rows and fewer x 220 features, depth 9, every level in the last block | apart: two outputs of
-// 32 bins 405 | 333 us a round, one of 64 bins 354 | 273, oblivious 215 | 190; of 128 features, 256 blocks, oblivious 125 | 132).
+// 32 bins 405 | 333 us a round, one of 64 bins 354 | 273, oblivious 215 | 190; of 128 features, 256 blocks, oblivious 125 | 132).  An oblivious level is decided
+// over all its nodes, whose sums its block holds 16 nodes at a time: apart from two channels of more than 224 bins on (255 bins, depth 8, 20k x 60 175 | 155 us a
+// round, 30k x 8 145 | 136; 160 bins, 15k x 60 equal), of several outputs where LDS holds the sums of fewer than 16 nodes.
 static bool small_scan_apart(const evt_ctx *c, int nodes, int blocks) {
     if (blocks > 256) return true;
     if (!c->mc && small_search_large(c->NAg, bins_per_lane(c->B))) return true;
-    if (c->tree_type == EVT_TREE_OBLIVIOUS) return (size_t)std::min(16, nodes) * c->NAg * c->B * 8 > 72 * 1024;
+    if (c->tree_type == EVT_TREE_OBLIVIOUS) return (size_t)std::min(16, nodes) * c->NAg * c->B * 8 > (c->mc ? 72 : 56) * 1024;
     return nodes > 16 || (int64_t)nodes * c->NAg * c->B > (c->mc ? 5120 : 1023);
 }
 // histograms a block's LDS holds at the deepest level that splits

@@ -38,6 +38,8 @@ pytestmark = pytest.mark.gpu
     (4001, 6, 255, 5, "gaussian_mle", dict(sub="mask")),
     (5001, 4, 128, 7, "gaussian_mle", {}),
     (6007, 3, 200, 8, "mse", dict(oblivious=True)),
+    (3011, 4, 224, 7, "mse", dict(oblivious=True)),                  # 16 nodes of 448 words are the last that stay
+    (3011, 4, 225, 7, "mse", dict(oblivious=True, weights=True)),
     (7001, 3, 160, 7, "mse", dict(weights=True)),                    # two nodes of 320 words are the last that stay
     (3001, 5, 64, 6, "mse", {}),                                      # eight nodes are 1024 words: apart; of 63 bins they stay
     (3001, 5, 63, 6, "mse", {}),
