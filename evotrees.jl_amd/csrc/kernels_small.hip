@@ -1106,12 +1106,14 @@ static int small_tree_buffers(evt_ctx *c, bool split) {
 // Which form a tree takes: 0 the kernels of larger inputs, 1 a block per feature, S > 1 a feature's rows
 // shared by S blocks.  A block walks its rows once per level (and once more for every `slots` nodes), so a level grows with
 // rows / S, the channels and - through the candidates every block reads and the searches its 16 wavefronts share - the nodes; slices
-// add a launch and the words they flush.  The other path spreads rows of any number over the chip and pays for its launches.  Estimates
-// in microseconds, fitted to rounds that each of them grew (2k to 250k rows, 8 to 100 features, depths 4 to 9, 1 to 15 channels): of 150 shapes
-// all but four take a form within 4 % of the best, the worst one 9 % off it.
-// Whole calls of one round (host included, ~50 us) at depth 6, microseconds for the other path, S = 1 and S > 1: mse, 8 features 125, 81, 95 at 2k rows,
-// 139, 137, 96 at 30k, 148, -, 108 at 250k; mse, 100 features 150, 137, 120 at 30k; 3 classes, 8 features 195, 154, 149 at 8k,
-// 210, 543, 159 at 60k, 237, -, 215 at 250k; 7 classes, 8 features 213, 188, 226 at 2k, 275, -, 303 at 120k, 320, -, 396 at 250k.
+// add the words they flush and, where a level is searched apart, a launch.  The other path spreads rows of any number over the chip and pays for its launches.
+// Estimates in microseconds, fitted to rounds of an earlier state of these kernels and checked on the present ones (500 to 300k rows, 3 to 250 features, depths 3 to
+// 10): of 364 shapes of one or two outputs 328 take a form within 4 % of the best and 353 within 10, the worst 1.32 times the best; of 186 of several outputs 149
+// and 157, the worst 1.65, where the other path, which has since become faster than its estimate, is not taken (profiles/rule_small_tree.txt).
+// What a further walk of all channels costs whatever its rows was added for those: 16 classes, 192 bins, 893 rows x 3, depth 6 906 -> 244 us, 14 classes, 160 bins,
+// 1558 x 4, depth 9 1209 -> 337; of 1658 shapes one takes more than 3 % longer by it.
+// A round of depth 6, 64 bins and 8 features as a fit queues it, microseconds for the other path, S = 1 and S > 1: mse 103, 58, 75 at 2k rows, 115, 109, 77 at 30k,
+// 127, -, 91 at 250k; 3 classes 146, 132, 121 at 8k, 161, 501, 139 at 60k, 190, -, 197 at 250k; 7 classes 148, 157, 184 at 2k, 186, -, 225 at 120k, 223, -, 299 at 250k.
 int small_tree_form(const evt_ctx *c, int nfs, bool all_rows) {
     if (!c->small_tree || c->D < 2 || c->D > 10 || nfs > 256 || c->N < 4 || c->N > (1 << 24) || !c->defer_pred || EVT_IS_QUANTILE(c->loss)) return 0;
     if (c->record_nidx && !all_rows) return 0;
@@ -1126,8 +1128,10 @@ int small_tree_form(const evt_ctx *c, int nfs, bool all_rows) {
     double one = 0.0, split = 0.0;
     for (int l = 1; l < c->D; l++) {
         const int n = (int)std::min<int64_t>(1 << (l - 1), c->N), searches = (n + 15) / 16;
-        one += 5.0 + 3.5 * searches + per_1k * k * ((n + slots - 1) / std::max(1, slots));
-        split += (c->mc ? 6.0 + 0.8 * c->NA : 11.0) + 2.5 * searches + per_1k_s * k / S * ((n + slots_split - 1) / std::max(1, slots_split)) +
+        const int walks = (n + slots - 1) / std::max(1, slots), walks_split = (n + slots_split - 1) / std::max(1, slots_split);
+        const double again = c->mc ? 0.5 * c->NA : 0.0; // a walk more clears and flushes the histograms of all channels, however few its rows
+        one += 5.0 + 3.5 * searches + per_1k * k * walks + again * (walks - 1);
+        split += (c->mc ? 6.0 + 0.8 * c->NA : 11.0) + 2.5 * searches + per_1k_s * k / S * walks_split + again * (walks_split - 1) +
                  (double)std::min<int64_t>((int64_t)n * c->B, c->N / S) * c->NA * nfs * S / 141e3; // words flushed: no more than rows
     }
     const double launches = c->mc ? 16.0 + 0.8 * c->NA + (nfs > 16 ? 2.0 + 0.008 * c->NA * std::max(0, nfs - 20) : std::max(0.0, 8.0 - 0.35 * c->NA))
