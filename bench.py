@@ -2,13 +2,13 @@
 
 A step is one boosting round (gradients -> one tree: histograms, split search, row partition ->
 prediction update) over a synthetic matrix that is already binned and resident in HBM when the
-timed region starts.  Default workload: BASELINE.json configs[2], the configuration the metric is
+timed region starts.  Default workload: the configuration the metric is
 quoted on (mse, 10M x 100 Float64 iid U(0,1), y ~ U(0,1), nbins 64, max_depth 11, eta 0.1, full
 row and column sampling, 200 rounds).
 
 Prints one JSON line.  `value` = seconds per 200 rounds (lower is better), scaled from the K timed
 rounds.  `roofline` = histogram kernel: algorithmic bytes rows_built*(Fs + 4*(2K+1) + 4) over the
-HIP-event time of its launches inside the timed region, against 8 TB/s.  `workloads` = the other BASELINE
+HIP-event time of its launches inside the timed region, against 8 TB/s.  `workloads` = the other
 configurations (a few dozen rounds each), `fit_total_s` = init + 200 rounds of the headline workload (without the process's
 one-time device context creation, reported as init_s.device_context_s).  `cpu_baseline` = the CPU
 oracle (a restatement of the reference's CPU algorithm, OpenMP over node x feature tiles) timed
@@ -285,7 +285,7 @@ def hist_roofline(cfg, prof_hist, nfs, NK):
 
 
 def side_workload(evt, name, steps, h=None, y=None, mu=None, rng=None, host_mask=False):
-    """One of BASELINE.json's other configurations, a few dozen rounds: ms per round, seconds per 200 rounds and the
+    """One of the other configurations, a few dozen rounds: ms per round, seconds per 200 rounds and the
     histogram kernel's fraction of the HBM peak.  cfg3s runs on the headline workload's own handle (same matrix)."""
     cfg = dict(WORKLOADS[name])
     own = h is None
@@ -329,7 +329,7 @@ def main():
     ap.add_argument("--option", action="append", default=[], help="name=value passed to evt_set_option (sweeps)")
     ap.add_argument("--predict", action="store_true", help="also time model inference on the training rows")
     ap.add_argument("--no-model-predict", action="store_true", help="skip the resident whole-model prediction figure")
-    ap.add_argument("--side-steps", type=int, default=40, help="timed rounds of each of the other BASELINE configurations (0: skip them)")
+    ap.add_argument("--side-steps", type=int, default=40, help="timed rounds of each of the other configurations (0: skip them)")
     args = ap.parse_args()
     if args.gpus != 1:
         print("bench.py: this build runs on ONE GPU; --gpus %d is not supported (no multi-GPU path is built)" % args.gpus,
@@ -558,7 +558,7 @@ def main():
         evt._lib.predict_model(xb, None, loss, K, m_trees, apply_link=True)
         out["predict"] = {"rows_per_s_incl_transfers": round(N / (time.perf_counter() - tp), 1), "trees": len(m_trees)}
 
-    # BASELINE.json's other configurations, a few dozen rounds each (cfg3s = the headline matrix with the sampling the
+    # the other configurations, a few dozen rounds each (cfg3s = the headline matrix with the sampling the
     # reference's published 10M x 100 table was run with, on the same handle)
     if args.side_steps > 0 and args.workload == "cfg3" and not args.rows and not args.depth:
         side = {}
