@@ -322,7 +322,7 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
 // and never writes out; the per-feature test (FULL = false) only pays when most features are left out.
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_row_bcast(uint32_t x) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false);
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, true); // every lane has a source: no register for a default
 }
 // value held by lane u of this lane's DPP row: the fetcher of row group u
 template <int u>
@@ -358,7 +358,7 @@ __device__ __forceinline__ uint32_t load_id(const uint32_t *p) {
     return NT ? __builtin_nontemporal_load(p) : *p;
 }
 
-template <int NA, bool PACK, bool GRP, int U, bool FULL, int PB, int PU, bool NT>
+template <int NA, bool PACK, bool GRP, int U, bool FULL, int PB, int PU, bool NT, bool FAR>
 __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
     extern __shared__ unsigned long long H[]; // [NA][PU][B][NS]
     const int tid = threadIdx.x, nthr = blockDim.x;
@@ -379,7 +379,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
     const int step = nwaves * RPW;
     int64_t T = (total + gridDim.x - 1) / gridDim.x;
     if (T < A.min_rows) T = A.min_rows;
-    T = ((T + U * step - 1) / (U * step)) * (U * step);
+    T = ((T + step - 1) / step) * step; // not whole iterations: 1024 rows at a time left a fifth of the blocks without any at 1600 rows a block
     int64_t start = (int64_t)blockIdx.x * T;
     if (start >= total) return;
     int64_t end = start + T < total ? start + T : total;
@@ -461,7 +461,6 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
             const int SR = U * RPW; // positions per wave iteration (<= 64)
             const int64_t itstride = (int64_t)nwaves * SR;
             const uint32_t *isp = A.is + seg;
-            // a record's address: row id times record size as one 32 x 32 -> 64 bit multiply-add, plus the piece's byte offset
             const uint32_t rs32 = (uint32_t)A.RS, pofs = (uint32_t)(tb + subl * PB);
             const int64_t lastp = nend - 1;          // >= start
             int64_t pw = start + (int64_t)wave * SR; // first position of this wave's iteration
@@ -473,6 +472,13 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
             uint32_t idc, idn;
             unsigned long long gc[NA], gn[NA];
             uint2 v[U];
+            // What a lane hands to its row group: where the row's record begins, multiplied out by the lane that fetched the id, so that a group's
+            // address is one addition whose operand comes by way of the row broadcast; FAR (records past 4 GB): the id, multiplied by every lane
+            // into 64 bits.  With the broadcasts' defaults gone a group of two features costs 8 vector instructions where it took 11 and a
+            // multiplication at a quarter of their rate: 500k rows x 50 of four channels, 23.4 -> 19.0 us a level, 1M x 100 sampled by half 14.5 -> 13.4,
+            // 800k x 28 of 128 bins' root 28.1 -> 25.3, 10M x 100's 282 -> 275 (with shares of whole steps instead of whole iterations, below).
+            auto handed = [&](uint32_t id) { return FAR ? id : id * rs32; };
+            auto piece = [&](uint32_t h) { return load_piece<PB, NT>(FAR ? A.xrm + ((size_t)h * rs32 + pofs) : A.xrm + (h + pofs)); };
             {
                 const int64_t p = pw + mypos;
                 idc = load_id<NT>(isp + ((fetcher && p < nend) ? p : lastp));
@@ -483,11 +489,11 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
                 const int64_t p = pw + itstride + mypos;
                 idn = load_id<NT>(isp + ((fetcher && p < nend) ? p : lastp));
             }
+            const uint32_t hc = handed(idc);
             __builtin_amdgcn_sched_barrier(0);
 #define EVT_H16_PRO(u_)                                                                                               \
     if constexpr ((u_) < U) {                                                                                         \
-        const uint32_t row = grp_bcast<(u_) < U ? (u_) : 0>(idc);                                               \
-        v[(u_) < U ? (u_) : 0] = load_piece<PB, NT>(A.xrm + ((size_t)row * rs32 + pofs));                   \
+        v[(u_) < U ? (u_) : 0] = piece(grp_bcast<(u_) < U ? (u_) : 0>(hc));                                    \
         __builtin_amdgcn_sched_barrier(0);                                                                            \
     }
             EVT_H16_PRO(0) EVT_H16_PRO(1) EVT_H16_PRO(2) EVT_H16_PRO(3) EVT_H16_PRO(4) EVT_H16_PRO(5) EVT_H16_PRO(6) EVT_H16_PRO(7)
@@ -496,7 +502,8 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
             for (; pw < nend; pw += itstride) {
                 // positions of this lane's rows left in the run, as a 32-bit number: group u is inside while u * RPW < rem
                 const int64_t rem64 = nend - pw - rloc;
-                const int rem = rem64 > 0x7fffffff ? 0x7fffffff : (int)rem64;
+                const int rem = !lane_on ? 0 : rem64 > 0x7fffffff ? 0x7fffffff : (int)rem64;
+                const uint32_t hn = handed(idn);
                 // next iteration's gradient words and the row ids of the one after: ahead of the records in issue order
 #pragma unroll
                 for (int a = 0; a < NA; a++) gn[a] = load_channel<PACK, GRP>(A, a0, a, idn);
@@ -516,7 +523,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
                 const uint32_t ghi = grp_bcast<ui>((uint32_t)(gc[a] >> 32));                                    \
                 gg[a] = ((unsigned long long)ghi << 32) | glo;                                                         \
             }                                                                                                         \
-            if (lane_on && ((u_) * RPW < rem)) {                                                                       \
+            if ((u_) * RPW < rem) {                                                                                    \
                 const uint32_t wds[2] = {v[ui].x, v[ui].y};                                                            \
                 _Pragma("unroll") for (int t = 0; t < PU; t++) {                                                       \
                     if (FULL || (vmask & (1u << t))) {                                                                \
@@ -527,8 +534,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
                 }                                                                                                     \
             }                                                                                                         \
         }                                                                                                             \
-        const uint32_t row = grp_bcast<ui>(idn);                                                                \
-        v[ui] = load_piece<PB, NT>(A.xrm + ((size_t)row * rs32 + pofs));                                  \
+        v[ui] = piece(grp_bcast<ui>(hn));                                                                      \
         __builtin_amdgcn_sched_barrier(0);                                                                            \
     }
                 EVT_H16_STEP(0) EVT_H16_STEP(1) EVT_H16_STEP(2) EVT_H16_STEP(3) EVT_H16_STEP(4) EVT_H16_STEP(5) EVT_H16_STEP(6) EVT_H16_STEP(7)
@@ -632,26 +638,27 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
 // Bytes of a piece: 16 or more pieces cover a column tile of tw bytes.
 static int hist16_piece(int tw) { return tw >= 128 ? 8 : tw >> 4; }
 
-template <int NA, bool PACK, bool GRP, int U, int PB, int PU, bool NT>
-static int launch_hist16_q(evt_ctx *c, const HistArgs &A, dim3 grid, int threads, size_t lds) {
-    // unpredicated atomics for every feature of the record pay off unless most features are left out: the words of
-    // features outside the sample are simply not flushed
-    const bool full = 2 * c->n_js_last >= c->F;
+template <int NA, bool PACK, bool GRP, int U, bool FULL, int PB, int PU, bool NT, bool FAR>
+static int launch_hist16_k(evt_ctx *c, const HistArgs &A, dim3 grid, int threads, size_t lds) {
     if (lds > 64 * 1024) { // one block per CU may take most of its 160 KB
         static EvtDevOnce once;
         if (once.pending(c->device)) {
-            HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_hist_build16<NA, PACK, GRP, U, true, PB, PU, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-            HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_hist_build16<NA, PACK, GRP, U, false, PB, PU, NT>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void *>(k_hist_build16<NA, PACK, GRP, U, FULL, PB, PU, NT, FAR>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
             once.mark(c->device);
         }
     }
     // c->launch_e0 / launch_e1 (when profiling): the kernel's own dispatch records them
-    if (full)
-        hipExtLaunchKernelGGL((k_hist_build16<NA, PACK, GRP, U, true, PB, PU, NT>), grid, dim3(threads), (uint32_t)lds, c->stream, c->launch_e0, c->launch_e1, 0, A);
-    else
-        hipExtLaunchKernelGGL((k_hist_build16<NA, PACK, GRP, U, false, PB, PU, NT>), grid, dim3(threads), (uint32_t)lds, c->stream, c->launch_e0, c->launch_e1, 0, A);
+    hipExtLaunchKernelGGL((k_hist_build16<NA, PACK, GRP, U, FULL, PB, PU, NT, FAR>), grid, dim3(threads), (uint32_t)lds, c->stream, c->launch_e0, c->launch_e1, 0, A);
     HIPCHK(hipGetLastError());
     return EVT_OK;
+}
+
+template <int NA, bool PACK, bool GRP, int U, int PB, int PU, bool NT, bool FAR>
+static int launch_hist16_q(evt_ctx *c, const HistArgs &A, dim3 grid, int threads, size_t lds) {
+    // unpredicated atomics for every feature of the record pay off unless most features are left out: the words of
+    // features outside the sample are simply not flushed
+    return 2 * c->n_js_last >= c->F ? launch_hist16_k<NA, PACK, GRP, U, true, PB, PU, NT, FAR>(c, A, grid, threads, lds)
+                                    : launch_hist16_k<NA, PACK, GRP, U, false, PB, PU, NT, FAR>(c, A, grid, threads, lds);
 }
 
 template <int NA, bool PACK, bool GRP>
@@ -660,12 +667,15 @@ static int launch_hist16_t(evt_ctx *c, const HistArgs &A, dim3 grid, int threads
     constexpr int U = (NA <= 2) ? 16 : 8;
     // records larger in total than the last-level cache (256 MB) are streamed past it
     const bool nt = (size_t)c->N * c->RS > ((size_t)256 << 20);
+    const bool far = (size_t)c->N * c->RS > 0xffffffffull; // a record's place takes more than 32 bits
     // (piece bytes, features per piece): a densely packed record has PU == PB, record_layout() picks the others
     const int pb = hist16_piece(A.TW);
     const int pu = (c->PU < c->PBL && c->PU < pb) ? c->PU : pb;
 #define H16Q(PB_, PU_)                                                                                                     \
     if (pb == PB_ && pu == PU_)                                                                                            \
-        return nt ? launch_hist16_q<NA, PACK, GRP, U, PB_, PU_, true>(c, A, grid, threads, lds) : launch_hist16_q<NA, PACK, GRP, U, PB_, PU_, false>(c, A, grid, threads, lds);
+        return !nt  ? launch_hist16_q<NA, PACK, GRP, U, PB_, PU_, false, false>(c, A, grid, threads, lds)                  \
+               : far ? launch_hist16_q<NA, PACK, GRP, U, PB_, PU_, true, true>(c, A, grid, threads, lds)                   \
+                     : launch_hist16_q<NA, PACK, GRP, U, PB_, PU_, true, false>(c, A, grid, threads, lds);
     H16Q(8, 8) H16Q(8, 7) H16Q(8, 6) H16Q(8, 5) H16Q(4, 4) H16Q(4, 3) H16Q(2, 2) H16Q(1, 1)
 #undef H16Q
     evt_set_error("no histogram kernel for pieces of %d bytes holding %d features", pb, pu);

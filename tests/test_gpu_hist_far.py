@@ -1,0 +1,34 @@
+"""Records that lie further than 32 bits hold from the first one: the histograms and the tree of a sample of the last features are those of a handle
+that has these features alone."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import assert_tree_bits, make_data
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("loss", ["mse", "gaussian_mle"])
+def test_records_past_four_gigabytes(evt, loss):
+    N, F, B, D = 1_080_001, 4000, 8, 3
+    assert N * F > 1 << 32  # a byte a feature
+    x8, y, w, mu = make_data(5, N, 8, B, loss, False)
+    x8 = np.ascontiguousarray(x8)
+    got = []
+    for x in (np.tile(x8, (F // 8, 1)), x8):
+        feats = x.shape[0]
+        print("features", feats, flush=True)
+        h = evt.Handle(N, feats, B, mu.shape[0], D, loss)
+        h.set_option("small_tree", 0)
+        h.set_xbin(x)
+        h.set_feature_meta(None, None)
+        h.set_target(y, w, mu)
+        h.update_grads()
+        js = np.arange(feats - 7, feats + 1, dtype=np.uint32)
+        tree = h.grow_tree(js, evt.make_params())
+        tree.feat[tree.feat > 0] -= feats - 8
+        got.append((tree, np.ascontiguousarray(h.get_hist()[:, feats - 8:])))
+        h.close()
+    assert got[0][0].split.any()
+    assert_tree_bits(got[0][0], got[1][0])
+    assert got[0][1].tobytes() == got[1][1].tobytes()
