@@ -265,7 +265,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->unit_w = true;
     c->have_xbin = c->have_target = c->have_grads = false;
     c->planes = nullptr; c->plane_words = 0; c->planes_ready = false; c->use_planes = 1;
-    c->xcm = nullptr; c->xrm = nullptr; c->y = nullptr; c->pred = nullptr; c->grad = nullptr; c->gq = nullptr;
+    c->xcm = nullptr; c->xrm = nullptr; c->y = nullptr; c->pred = nullptr; c->grad = nullptr; c->gq = nullptr; c->gq_rows = false;
     c->is_a = c->is_b = nullptr; c->nidx = nullptr; c->mask = nullptr; c->flagw = nullptr; c->chunk_nleft = nullptr; c->chunk_lpre = nullptr; c->cursor = nullptr;
     c->hist = nullptr; c->seg_start = c->seg_len = nullptr; c->status = nullptr; c->node_sum = nullptr;
     memset(&c->tree, 0, sizeof(c->tree));
@@ -344,7 +344,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     ALLOC(c->y, N * c->T);
     ALLOC(c->pred, (size_t)N * K);
     ALLOC(c->grad, (size_t)N * c->NK);
-    ALLOC(c->gq, (size_t)N * c->NK);
+    ALLOC(c->gq, EVT_GQ_WORDS(N, c->NK));
     ALLOC(c->is_a, N);
     ALLOC(c->is_b, N);
     ALLOC(c->is_id, N);
@@ -601,6 +601,7 @@ static void set_channels(evt_ctx *c) {
         if (!c->unit_w) c->chan_k[na++] = c->NK - 1;
     }
     c->NA = na;
+    c->gq_rows = na > 1; // what the first tree most likely reads; no words are there yet
     for (int a = na; a < EVT_MC_MAX_NK; a++) c->chan_k[a] = 0;
     c->NAg = EVT_TWO_CHAN(c->loss, c->K) ? 2 : c->NK;
     int qbg = 62 - ceil_log2_i64(c->N);
@@ -843,7 +844,8 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
     c->last_all_rows = all_rows;
     c->last_cond = cond;
     const int small = staged ? 0 : small_tree_form(c, n_js, all_rows);
-    int r = EVT_OK;
+    int r = gq_layout(c, !small);
+    if (r != EVT_OK) return r;
     if (c->quant_pending) {
         if (small ? small_root_quantises(c, small) : c->N <= EVT_QUANT_LATER) quant_set(c); // by the tree's first kernel
         else r = launch_quantize(c);

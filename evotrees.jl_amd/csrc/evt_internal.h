@@ -119,7 +119,8 @@ struct evt_ctx {
     float *y;
     float *pred;    // K x N
     float *grad;    // NK x N
-    unsigned long long *gq; // NA planes of N packed fixed-point words
+    unsigned long long *gq; // fixed-point words of the rows: NA planes of N, or (gq_rows) EVT_GQ_STRIDE(NA) words a row
+    bool gq_rows;           // which: the kernels of small trees walk all rows and read planes, the others gather rows
     uint32_t *is_a, *is_b;
     uint32_t *is_id;   // [N] 0..N-1, written once: the root's row list when every row is in the tree
     uint32_t *nidx;
@@ -311,6 +312,10 @@ static int guarded(F &&f) {
 #define EVT_TWO_CHAN(loss, K) (((loss) == EVT_LOSS_MSE || EVT_IS_SHIFT(loss)) && (K) == 1)
 #define EVT_NODE_SPLIT (1u << 24)
 #define EVT_NODE_NUMERIC (1u << 25)
+// Words from one row to the next where a row's words lie side by side: whole 16 bytes.
+#define EVT_GQ_STRIDE(na) (((na) + 1) & ~1)
+// ... and words of the allocation for either layout: a histogram layer of four channels may read past the last row's
+#define EVT_GQ_WORDS(n, nk) ((size_t)(n) * ((nk) + 1) + EVT_HIST_GROUP)
 #ifdef __HIPCC__
 __host__ __device__ __forceinline__ uint32_t evt_pack_node(int feat, int cond_bin, bool numeric) {
     return (uint32_t)feat | ((uint32_t)cond_bin << 16) | EVT_NODE_SPLIT | (numeric ? EVT_NODE_NUMERIC : 0u);
@@ -324,6 +329,25 @@ __device__ __forceinline__ unsigned long long evt_load_gq(const unsigned long lo
         return ((unsigned long long)q << EVT_PACK_CNT_BITS) + 1ull;
     }
     return gq[(size_t)a * N + id];
+}
+
+// The words of channels a0 .. a0 + NA - 1 of one row, side by side in memory (stride: words from row to row, even; a0 even) - one request per 16 bytes,
+// all of one line, where planes of N words cost a line for each channel once a node's rows lie apart.  One channel alone is a plane of
+// 32-bit words in either layout.
+template <int NA, bool PACK>
+__device__ __forceinline__ void evt_load_words(const unsigned long long *__restrict__ gq, int stride, int a0, uint32_t id, unsigned long long (&g)[NA]) {
+    if constexpr (NA == 1 && PACK) {
+        g[0] = evt_load_gq<true>(gq, 0, 0, id);
+    } else {
+        const unsigned long long *p = gq + (size_t)id * stride + a0;
+#pragma unroll
+        for (int a = 0; a + 1 < NA; a += 2) {
+            const ulonglong2 v = *reinterpret_cast<const ulonglong2 *>(p + a);
+            g[a] = v.x;
+            g[a + 1] = v.y;
+        }
+        if (NA & 1) g[NA - 1] = p[NA - 1];
+    }
 }
 
 __device__ __forceinline__ void evt_add_leaf(float *pr, const float *lp, int K, int loss) {
@@ -351,6 +375,7 @@ __device__ __forceinline__ void evt_add_leaf(float *pr, const float *lp, int K, 
 // grad
 int launch_grads(evt_ctx *c);
 int launch_quantize(evt_ctx *c);
+int gq_layout(evt_ctx *c, bool rows);
 void quant_set(evt_ctx *c);
 uint32_t *absmax_set(evt_ctx *c, int which);
 int launch_apply_pending(evt_ctx *c);

@@ -171,6 +171,7 @@ struct QuantArgs {
     unsigned long long *gq;
     int64_t N;
     int NK, NA, NAg, loss, two, unit_w, pack, pack_wide;
+    int stride; // words from row to row of gq, 0: planes of N words
     const uint32_t *absmax;
     uint32_t *absmax_next;
     const int32_t *qbits;
@@ -187,8 +188,9 @@ void quant_taken(evt_ctx *c);                          // behind the launch
 // block 0 also writes the tables for the readers that follow (split search, read-back).  The maxima live in two sets: a
 // gradient pass raises one, this kernel reads it and clears the other - which nobody uses at that moment - for the next pass,
 // so no pass starts from maxima an earlier one left behind.  The weight row (last) is written once and keeps its maximum.
-// Plane a of gq holds, per row, q = rint(v * 2^(qbits - qexp)) of gradient row chan_k[a]; with unit weights plane 0 also carries
-// the row count in its low 16 bits ((q << 16) + 1) so that one 64-bit LDS add serves both.
+// Word a of a row is q = rint(v * 2^(qbits - qexp)) of gradient row chan_k[a]; with unit weights word 0 also carries
+// the row count in its low 16 bits ((q << 16) + 1) so that one 64-bit LDS add serves both.  A row's words go to planes, or side by side (gq_rows).
+// absmax == nullptr: the words are made again, in the other layout, with the tables there are.
 // Channel a reads gradient row a, except for mse whose channels are {g, w} = rows {0, 2}.
 // `block` of `blocks`: of a kernel of its own, or of one that sets a tree up meanwhile (kernels_part.hip).
 __device__ __forceinline__ void quant_rows(const QuantArgs &Q, int block, int blocks) {
@@ -196,14 +198,18 @@ __device__ __forceinline__ void quant_rows(const QuantArgs &Q, int block, int bl
     __shared__ int s_qexp[EVT_MC_MAX_NK], s_qbits[EVT_MC_MAX_NK];
     const int t = threadIdx.x, nthr = blockDim.x, NK = Q.NK;
     if (t < NK) {
-        const int e = quant_exponent(Q.absmax, t);
-        const int qb = Q.qbits[t];
-        s_qexp[t] = e;
-        s_qbits[t] = qb;
-        s_qmul[t] = scalbn(1.0, qb - e);
+        if (Q.absmax) {
+            const int e = quant_exponent(Q.absmax, t);
+            const int qb = Q.qbits[t];
+            s_qexp[t] = e;
+            s_qbits[t] = qb;
+            s_qmul[t] = scalbn(1.0, qb - e);
+        } else {
+            s_qmul[t] = Q.qscale[EVT_MC_MAX_NK + t];
+        }
     }
     __syncthreads();
-    if (block == 0) {
+    if (block == 0 && Q.absmax) {
         if (t < NK) {
             Q.qexp[t] = s_qexp[t];
             Q.qscale[EVT_MC_MAX_NK + t] = s_qmul[t];
@@ -221,6 +227,17 @@ __device__ __forceinline__ void quant_rows(const QuantArgs &Q, int block, int bl
     for (int64_t w = (int64_t)block * nthr + t; w < Q.N << sh; w += (int64_t)blocks * nthr) {
         const int64_t i = w >> sh;
         const float *g = Q.grad + (size_t)NK * i;
+        if (Q.stride) { // 16 bytes, two channels, at a time
+#pragma unroll 3
+            for (int a = 2 * part; a < Q.NA; a += 2 << sh) {
+                long long q0 = __double2ll_rn((double)g[a] * s_qmul[a]);
+                const int a1 = a + 1 < Q.NA ? a + 1 : a, k1 = (Q.two && a1 == 1) ? 2 : a1;
+                const long long q1 = __double2ll_rn((double)g[k1] * s_qmul[k1]);
+                if (a == 0 && Q.unit_w) q0 = (long long)(((unsigned long long)q0 << EVT_PACK_CNT_BITS) + 1ull);
+                *reinterpret_cast<ulonglong2 *>(Q.gq + (size_t)i * Q.stride + a) = make_ulonglong2((unsigned long long)q0, (unsigned long long)q1);
+            }
+            continue;
+        }
 #pragma unroll 5
         for (int a = part; a < Q.NA; a += 1 << sh) { // several channels' words in flight
             const int k = (Q.two && a == 1) ? 2 : a;

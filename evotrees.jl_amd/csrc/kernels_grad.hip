@@ -381,6 +381,7 @@ void quant_args(evt_ctx *c, QuantArgs &Q) {
     Q.unit_w = c->unit_w ? 1 : 0;
     Q.pack = (c->unit_w && c->NA <= EVT_MAX_NA) ? 1 : 0;
     Q.pack_wide = (c->unit_w && c->NA > EVT_MAX_NA) ? 1 : 0;
+    Q.stride = c->gq_rows ? EVT_GQ_STRIDE(c->NA) : 0;
     Q.absmax = absmax_set(c, c->absmax_cur);
     Q.absmax_next = absmax_set(c, c->absmax_cur ^ 1);
     Q.qbits = c->qbits;
@@ -407,6 +408,21 @@ int launch_quantize(evt_ctx *c) {
     hipLaunchKernelGGL(k_quantize, dim3(quant_blocks(c, 256)), dim3(256), 0, c->stream, Q);
     HIPCHK(hipGetLastError());
     quant_taken(c);
+    return EVT_OK;
+}
+
+// The layout that a tree's kernels read.  Words that are still to be made are made in it; words that an earlier tree has made in the other (a
+// tree of the other form on the same gradients) are made again.
+int gq_layout(evt_ctx *c, bool rows) {
+    rows = rows && c->NA > 1;
+    if (c->gq_rows == rows) return EVT_OK;
+    c->gq_rows = rows;
+    if (c->quant_pending) return EVT_OK;
+    QuantArgs Q;
+    quant_args(c, Q);
+    Q.absmax = nullptr;
+    hipLaunchKernelGGL(k_quantize, dim3(quant_blocks(c, 256)), dim3(256), 0, c->stream, Q);
+    HIPCHK(hipGetLastError());
     return EVT_OK;
 }
 

@@ -44,6 +44,7 @@ struct HistArgs {
     int seg_cost;
     int na_all; // accumulator channels of the loss: more than EVT_MAX_NA go EVT_HIST_GROUP to a block layer (blockIdx.z)
     int pack;   // the channel groups' first channel carries the row count (as a 64-bit word, k_quantize)
+    int gq_stride; // words from row to row of gq
     int tab;    // entries of bprefix, bstart and bnode that may be read
 };
 
@@ -110,14 +111,6 @@ struct BuildList {
         return held ? __builtin_amdgcn_readlane(node, __builtin_amdgcn_readfirstlane(i)) : A.bnode[i];
     }
 };
-
-// Channel c of a block layer's group, for one row.  GRP: the layer's channels start at a0; past the last one it reads that again
-// (added to words the flush leaves out).
-template <bool PACK, bool GRP>
-__device__ __forceinline__ unsigned long long load_channel(const HistArgs &A, int a0, int c, uint32_t id) {
-    if constexpr (GRP) return A.gq[(size_t)(a0 + c < A.na_all ? a0 + c : A.na_all - 1) * A.N + id];
-    else return evt_load_gq<PACK>(A.gq, A.N, c, id);
-}
 
 // GRP: more channels than one block's LDS takes (multi-class, several targets).  A layer of blocks takes NA of them, all layers in one
 // launch: a level of 60k rows is 60 blocks per group, which fill a quarter of the chip one after the other.
@@ -207,8 +200,7 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
                 vc[u] = make_uint4(0, 0, 0, 0);
                 if (rc[u] != INV) {
                     vc[u] = *reinterpret_cast<const uint4 *>(A.xrm + (size_t)rc[u] * A.RS + sub * 16);
-#pragma unroll
-                    for (int a = 0; a < NA; a++) gc[u][a] = load_channel<PACK, GRP>(A, a0, a, rc[u]);
+                    evt_load_words<NA, PACK>(A.gq, A.gq_stride, a0, rc[u], gc[u]); // a layer's channels past the last are added to words the flush leaves out
                 }
             }
 #pragma unroll
@@ -222,8 +214,7 @@ __global__ __launch_bounds__(1024) void k_hist_build(HistArgs A) {
                     vn[u] = make_uint4(0, 0, 0, 0);
                     if (rn[u] != INV) {
                         vn[u] = *reinterpret_cast<const uint4 *>(A.xrm + (size_t)rn[u] * A.RS + sub * 16);
-#pragma unroll
-                        for (int a = 0; a < NA; a++) gn[u][a] = load_channel<PACK, GRP>(A, a0, a, rn[u]);
+                        evt_load_words<NA, PACK>(A.gq, A.gq_stride, a0, rn[u], gn[u]);
                     }
                 }
                 uint32_t rnn[U];
@@ -483,8 +474,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
                 const int64_t p = pw + mypos;
                 idc = load_id<NT>(isp + ((fetcher && p < nend) ? p : lastp));
             }
-#pragma unroll
-            for (int a = 0; a < NA; a++) gc[a] = load_channel<PACK, GRP>(A, a0, a, idc);
+            evt_load_words<NA, PACK>(A.gq, A.gq_stride, a0, idc, gc);
             {
                 const int64_t p = pw + itstride + mypos;
                 idn = load_id<NT>(isp + ((fetcher && p < nend) ? p : lastp));
@@ -505,8 +495,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
                 const int rem = !lane_on ? 0 : rem64 > 0x7fffffff ? 0x7fffffff : (int)rem64;
                 const uint32_t hn = handed(idn);
                 // next iteration's gradient words and the row ids of the one after: ahead of the records in issue order
-#pragma unroll
-                for (int a = 0; a < NA; a++) gn[a] = load_channel<PACK, GRP>(A, a0, a, idn);
+                evt_load_words<NA, PACK>(A.gq, A.gq_stride, a0, idn, gn);
                 uint32_t idnn;
                 {
                     const int64_t p = pw + 2 * itstride + mypos;
@@ -794,6 +783,7 @@ int launch_hist_build(evt_ctx *c, int level, const uint32_t *is_cur) {
     const int na = grouped ? EVT_HIST_GROUP : c->NA;
     const unsigned layers = grouped ? (unsigned)((c->NA + na - 1) / na) : 1u;
     A.gq = c->gq;
+    A.gq_stride = EVT_GQ_STRIDE(c->NA);
     A.na_all = c->NA;
     A.pack = c->unit_w ? 1 : 0;
     // feature tiling so that one block's LDS histogram stays within budget

@@ -63,6 +63,7 @@ struct PartArgs {
     // scatter pass that also builds the next level's histograms (16-byte records)
     const uint8_t *xrm;
     const unsigned long long *gq;
+    int gq_stride;
     const uint16_t *jsmap;
     long long *hist;
     int64_t node_stride;
@@ -513,8 +514,7 @@ __global__ __launch_bounds__(256) void k_part_scatter(PartArgs A, NextArgs NX) {
 #pragma unroll
             for (int it = 0; it < NI; it++) {
                 rec[it] = *reinterpret_cast<const uint4 *>(A.xrm + (size_t)rid[it] * 16);
-#pragma unroll
-                for (int a = 0; a < HNA; a++) gw[it][a] = evt_load_gq<PACK>(A.gq, A.N, a, rid[it]);
+                evt_load_words<HNA, PACK>(A.gq, A.gq_stride, 0, rid[it], gw[it]);
             }
         }
         if (st == ST_SPLIT) {
@@ -1229,6 +1229,7 @@ int launch_part_scatter(evt_ctx *c, int level, const uint32_t *is_cur, uint32_t 
         // the next level's histograms are built here: no histogram kernel runs at that level
         A.xrm = c->xrm;
         A.gq = c->gq;
+        A.gq_stride = EVT_GQ_STRIDE(c->NA);
         A.jsmap = c->jsmap;
         A.hist = c->hist;
         A.node_stride = (int64_t)c->F * c->NAg * c->B;
