@@ -179,7 +179,7 @@ extern "C" int evt_destroy(evt_handle c) {
     if (!c) return EVT_OK;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    void *ptrs[] = {c->xcm, c->xrm, c->y, c->pred, c->grad, c->gq, c->is_a, c->is_b, c->nidx, c->mask, c->flagw, c->chunk_nleft, c->chunk_lpre, c->cursor,
+    void *ptrs[] = {c->xcm, c->xrm, c->y, c->pred, c->grad, c->gq, c->is_a, c->is_b, c->nidx, c->mask, c->flagw, c->sample_claims, c->chunk_nleft, c->chunk_lpre, c->cursor,
                     c->hist, c->seg_start, c->seg_len, c->status, c->node_sum, c->tree_blob, c->tree.packed, c->js, c->jsmap, c->feattypes, c->mono, c->absmax, c->qexp_buf[0], c->qexp_buf[1], c->qbits,
                     c->qscale_buf[0], c->qscale_buf[1], c->planes, c->metric_partial, c->errflag, c->ogains, c->sbest, c->scan_count, c->is_id, c->pt_nodes, c->mask_next,
                     c->small_nid[0], c->small_nid[1], c->small_head[0], c->small_head[1], c->small_left[0], c->small_left[1], c->small_acc,
@@ -266,7 +266,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->have_xbin = c->have_target = c->have_grads = false;
     c->planes = nullptr; c->plane_words = 0; c->planes_ready = false; c->use_planes = 1;
     c->xcm = nullptr; c->xrm = nullptr; c->y = nullptr; c->pred = nullptr; c->grad = nullptr; c->gq = nullptr; c->gq_rows = false;
-    c->is_a = c->is_b = nullptr; c->nidx = nullptr; c->mask = nullptr; c->flagw = nullptr; c->chunk_nleft = nullptr; c->chunk_lpre = nullptr; c->cursor = nullptr;
+    c->is_a = c->is_b = nullptr; c->nidx = nullptr; c->mask = nullptr; c->flagw = nullptr; c->sample_claims = nullptr; c->chunk_nleft = nullptr; c->chunk_lpre = nullptr; c->cursor = nullptr;
     c->hist = nullptr; c->seg_start = c->seg_len = nullptr; c->status = nullptr; c->node_sum = nullptr;
     memset(&c->tree, 0, sizeof(c->tree));
     c->tree_blob = nullptr;
@@ -350,6 +350,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     ALLOC(c->is_id, N);
     ALLOC(c->nidx, N);
     ALLOC(c->mask, N);
+    ALLOC(c->sample_claims, 1);
     ALLOC(c->flagw, (size_t)c->max_chunks * EVT_CHUNK_WORDS);
     ALLOC(c->chunk_nleft, c->max_chunks + 1);
     ALLOC(c->chunk_lpre, c->max_chunks + 1);
@@ -432,6 +433,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->absmax, 0, sizeof(uint32_t) * 2 * EVT_ABSMAX_STRIPES * EVT_MC_MAX_NK, c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->nidx, 0, sizeof(uint32_t) * N, c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->errflag, 0, sizeof(int32_t), c->stream);
+    if (e2 == hipSuccess) e2 = hipMemsetAsync(c->sample_claims, 0, sizeof(unsigned long long), c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->scan_count, 0, sizeof(int32_t) * EVT_SCAN_COUNT_STEP * c->maxlvl, c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->metric_partial + 2 * EVT_METRIC_BLOCKS, 0, sizeof(double), c->stream);
     if (e2 == hipSuccess) e2 = upload_alphas(c);

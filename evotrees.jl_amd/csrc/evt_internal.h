@@ -51,6 +51,9 @@
 // one-pass partition: a node's cursor has a 128-byte line to itself (additions to one line follow each other); the nodes of very deep levels, of few
 // chunks each, share lines
 #define EVT_CURSOR_SLOT(n) ((n) < 1024 ? (size_t)(n) * 16 : (size_t)16384 - 1024 + (n))
+// row sample in one kernel: rows of a block, and blocks (claims of one address, ~15 ns each: more of them take the count and the scatter)
+#define EVT_SAMPLE_ROWS 8192
+#define EVT_SAMPLE_BLOCKS 512
 #define EVT_CURSOR_WORDS(nnodes) ((size_t)16384 + (nnodes) + 2)
 
 // split search: a node's block counter has a 128-byte line to itself (additions to one line follow each other, ~15 ns each)
@@ -131,6 +134,7 @@ struct evt_ctx {
     bool mask_next_valid;
     bool mask_seed_valid;   // the next staged tree draws its mask on the device from mask_seed (evt_draw_mask) instead of using mask_next
     unsigned long long mask_seed;
+    unsigned long long *sample_claims; // k_mask_sample: rows and blocks that have claimed places (zero between launches)
     unsigned long long *flagw;
     int32_t *chunk_nleft;
     int64_t *chunk_lpre;
@@ -332,8 +336,9 @@ __device__ __forceinline__ unsigned long long evt_load_gq(const unsigned long lo
 }
 
 // The words of channels a0 .. a0 + NA - 1 of one row, side by side in memory (stride: words from row to row, even; a0 even) - one request per 16 bytes,
-// all of one line, where planes of N words cost a line for each channel once a node's rows lie apart.  One channel alone is a plane of
-// 32-bit words in either layout.
+// all of one line, where planes of N words cost a line for each channel once a node's rows lie apart, and again in every column tile.  One channel alone is a
+// plane of 32-bit words in either layout.  us a histogram level, planes -> side by side: 500k rows x 50 of four channels 17.9 to 19.1 -> 15.6 to 18.3, 60k x 30 of 14
+// channels 12.9 to 14.6 -> 12.8 to 13.3, 800k x 28 of two 16.2 to 18.4 -> 16.3 to 17.7; the quantisation of several channels writes more (8.1 -> 8.9, beside the mask's count).
 template <int NA, bool PACK>
 __device__ __forceinline__ void evt_load_words(const unsigned long long *__restrict__ gq, int stride, int a0, uint32_t id, unsigned long long (&g)[NA]) {
     if constexpr (NA == 1 && PACK) {

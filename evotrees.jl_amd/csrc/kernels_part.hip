@@ -807,8 +807,7 @@ struct BeginArgs {
     int64_t *bprefix;
     long long *hist;
     int64_t *stats;
-    int64_t n_is;
-    const int64_t *n_is_dev; // non-null: the number of sampled rows is the total the mask compaction left on the device
+    int64_t n_is; // rows of a tree on every row
     int64_t seg_cost;
     int64_t root_words;
     int nnodes, K, D;
@@ -821,9 +820,10 @@ struct BeginArgs {
     int js_words, map_words;
 };
 
-// One block prepares a tree: empty Tree arrays, node states, the first level's tables, the column sample.  A kernel of its own for a tree on every row; with a row sample it is the last block of the kernel that
-// compacts the sampled rows (k_mask_scatter), which hands it the number of rows kept.
-__device__ void tree_begin_block(BeginArgs A) {
+// One block prepares a tree: empty Tree arrays, node states, the column sample; and, once the number of its rows is known, the first level's tables.
+// A kernel of its own for a tree on every row; with a row sample they ride in the kernel that
+// compacts the sampled rows (k_mask_sample, k_mask_scatter), which counts them.
+__device__ void tree_begin_arrays(const BeginArgs &A) {
     const int tid = threadIdx.x, nthr = blockDim.x; // 256 or 1024; each of four wavefronts starts another of the short lists
     for (int n = tid; n < A.nnodes; n += nthr) {
         A.tree.feat[n] = 0;
@@ -835,19 +835,23 @@ __device__ void tree_begin_block(BeginArgs A) {
         for (int k = 0; k < A.K; k++) A.tree.pred[(int64_t)A.K * n + k] = 0.0f;
     }
     for (int n = tid ^ 64; n < A.nnodes + 2; n += nthr) A.status[n] = n == 1 ? ST_BUILD : ST_INACTIVE;
-    if (A.n_is_dev) A.n_is = *A.n_is_dev;
-    for (int d = tid ^ 128; d <= A.D; d += nthr) A.stats[d] = d ? 0 : A.n_is; // read back with the tree: the host learns how many rows the mask kept
+    for (int d = tid ^ 128; d <= A.D; d += nthr)
+        if (d) A.stats[d] = 0;
     for (int i = tid; i < A.js_words; i += nthr) A.js_dst[i] = A.js_src[i];
     for (int i = tid; i < A.map_words; i += nthr) A.map_dst[i] = A.map_src[i];
-    const int64_t n_chunks = (A.n_is + ((int64_t)1 << A.chunk_sh) - 1) >> A.chunk_sh;
-    for (int64_t c = tid ^ 192; c < n_chunks; c += nthr) A.cdesc[c] = make_uint4(1, (uint32_t)(c << A.chunk_sh), (uint32_t)A.n_is, 0);
+}
+__device__ void tree_begin_rows(const BeginArgs &A, int64_t n_is) {
+    const int tid = threadIdx.x, nthr = blockDim.x;
+    const int64_t n_chunks = (n_is + ((int64_t)1 << A.chunk_sh) - 1) >> A.chunk_sh;
+    for (int64_t c = tid ^ 192; c < n_chunks; c += nthr) A.cdesc[c] = make_uint4(1, (uint32_t)(c << A.chunk_sh), (uint32_t)n_is, 0);
     if (tid == 128) {
+        A.stats[0] = n_is; // read back with the tree: the host learns how many rows the mask kept
         A.seg_start[1] = 0;
-        A.seg_len[1] = A.n_is;
+        A.seg_len[1] = n_is;
         A.hdr[LH_N_ACT] = 1;
         A.hdr[LH_N_CHUNKS] = n_chunks;
         A.hdr[LH_N_BUILD] = 1;
-        A.hdr[LH_TOTAL_BUILD] = A.n_is + A.seg_cost;
+        A.hdr[LH_TOTAL_BUILD] = n_is + A.seg_cost;
         A.act_node[0] = 1;
         A.cprefix[0] = 0;
         A.cprefix[1] = n_chunks;
@@ -855,7 +859,7 @@ __device__ void tree_begin_block(BeginArgs A) {
         A.bnode[0] = 1;
         A.bstart[0] = 0;
         A.bprefix[0] = 0;
-        A.bprefix[1] = A.n_is + A.seg_cost;
+        A.bprefix[1] = n_is + A.seg_cost;
     }
 }
 
@@ -872,7 +876,10 @@ __global__ __launch_bounds__(1024) void k_tree_begin(BeginArgs A, QuantArgs Q, i
         return;
     }
     tree_begin_root(A, blocks);
-    if (blockIdx.x == 0) tree_begin_block(A);
+    if (blockIdx.x == 0) {
+        tree_begin_arrays(A);
+        tree_begin_rows(A, A.n_is);
+    }
 }
 
 // ---- row subsampling: is = rows with mask <= cond, ascending (src/subsample.jl:6-38) -----------
@@ -882,12 +889,98 @@ __device__ __forceinline__ int wave_sum_i32(int v) {
     return v;
 }
 
-// A thread takes 8 consecutive mask bytes (one load); the 8 flags of 8 neighbouring threads make one 64-row flag word.
+// Which of the rows p0 .. p0 + 7 (p0 a multiple of 8) the mask keeps, row p0 in the lowest bit.
 // DRAW: the bytes are not read but drawn here and written to `mask` on the way: the mask's 8-byte word w is output w of
 // SplitMix64 (Steele, Lea, Flood 2014: a Weyl sequence with increment 0x9E3779B97F4A7C15 passed through two
 // multiply-xorshift rounds) started at state `seed`, stored little end first - byte i of the mask is bits 8*(i%8).. of output
 // i/8.  Stands in for rand!(rng, mask) of src/subsample.jl:7 when the caller accepts a counter-based stream keyed by one 64-bit
 // draw of its own generator per tree.
+template <bool DRAW>
+__device__ __forceinline__ unsigned mask_flags(uint8_t *mask, uint8_t cond, int64_t N, int64_t p0, unsigned long long seed) {
+    unsigned long long v = ~0ull; // bytes past the end read as 255
+    if (DRAW) {
+        unsigned long long z = seed + (unsigned long long)((p0 >> 3) + 1) * 0x9E3779B97F4A7C15ull;
+        z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+        z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+        z ^= z >> 31;
+        v = z;
+        if (p0 + 8 <= N) {
+            *reinterpret_cast<unsigned long long *>(mask + p0) = z;
+        } else {
+            for (int j = 0; p0 + j < N; j++) mask[p0 + j] = (uint8_t)(z >> (8 * j));
+        }
+    } else if (p0 + 8 <= N) {
+        v = *reinterpret_cast<const unsigned long long *>(mask + p0);
+    } else {
+        for (int j = 0; j < 8; j++)
+            if (p0 + j < N) v = (v & ~(0xFFull << (8 * j))) | ((unsigned long long)mask[p0 + j] << (8 * j));
+    }
+    unsigned flags = 0;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const bool keep = (p0 + j < N) && ((uint8_t)(v >> (8 * j)) <= cond);
+        flags |= keep ? (1u << j) : 0u;
+    }
+    return flags;
+}
+
+// The sample of up to EVT_SAMPLE_BLOCKS blocks' rows, and the tree's set-up, in one kernel: a block flags its 8192 rows, claims as many places of the
+// list by one addition and writes their ids there.  A block's rows stay in order, the blocks follow each other in the order of their
+// claims, which nothing depends on (k_part_move's chunks do the same).  The block that claims last knows the number of rows and writes the first
+// level's tables; block 0 prepares the rest of the tree, blocks behind the sample's quantise.  Bound by its chain (draw, count, claim, stores) and the
+// quantisation beside it: 1M rows 7.9 us with one word a row, 10.0 with two (a block's rows by 1024 threads: 9.1, 12.4: quantisation gets its blocks later).  In two kernels, a
+// count and a scatter that added the counts up, 5.9 + 5.1 and 8.9 + 4.7.
+template <bool DRAW>
+__global__ __launch_bounds__(256) void k_mask_sample(uint8_t *mask, uint8_t cond, int64_t N, unsigned long long seed, uint32_t *is_out,
+                                                     unsigned long long *claims, BeginArgs B, QuantArgs Q, int blocks) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if ((int)blockIdx.x > blocks) { // as k_tree_begin
+        quant_rows(Q, (int)blockIdx.x - blocks - 1, (int)gridDim.x - blocks - 1);
+        return;
+    }
+    if (blockIdx.x == 0) {
+        tree_begin_arrays(B);
+        return;
+    }
+    static_assert(EVT_SAMPLE_ROWS == 256 * 32, "32 rows to a thread");
+    __shared__ uint16_t s_row[EVT_SAMPLE_ROWS]; // the rows kept, from the block's first
+    __shared__ int s_cnt[4];
+    __shared__ unsigned long long s_claim;
+    const int64_t b0 = ((int64_t)blockIdx.x - 1) * EVT_SAMPLE_ROWS;
+    uint32_t flags = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) flags |= mask_flags<DRAW>(mask, cond, N, b0 + tid * 32 + 8 * j, seed) << (8 * j);
+    const int own = __popc(flags);
+    int incl = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int x = __shfl_up(incl, o);
+        if (lane >= o) incl += x;
+    }
+    if (lane == 63) s_cnt[wave] = incl;
+    __syncthreads();
+    int total = 0, at = incl - own;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+        const int v = s_cnt[w];
+        total += v;
+        at += w < wave ? v : 0;
+    }
+    // rows claimed so far, blocks that have claimed in the upper half
+    if (tid == 0) s_claim = atomicAdd(claims, (unsigned long long)total | (1ull << 40));
+    for (uint32_t f = flags; f; f &= f - 1) s_row[at++] = (uint16_t)(tid * 32 + __ffs(f) - 1);
+    for (int64_t i = b0 / EVT_SAMPLE_ROWS * 256 + tid; i < B.root_words; i += (int64_t)blocks * 256) B.hist[i] = 0;
+    __syncthreads();
+    const unsigned long long claim = s_claim;
+    const int64_t base = (int64_t)(claim & ((1ull << 40) - 1));
+    for (int i = tid; i < total; i += 256) is_out[base + i] = (uint32_t)b0 + s_row[i];
+    if ((int)(claim >> 40) == blocks - 1) {
+        if (tid == 0) *claims = 0ull; // for the next launch
+        tree_begin_rows(B, base + total);
+    }
+}
+
+// A thread takes 8 consecutive mask bytes (one load); the 8 flags of 8 neighbouring threads make one 64-row flag word.
 template <bool DRAW>
 __global__ __launch_bounds__(256) void k_mask_count(uint8_t *mask, uint8_t cond, int64_t N, int64_t n_chunks,
                                                    unsigned long long *flagw, int32_t *chunk_nleft, unsigned long long seed, QuantArgs Q, int blocks) {
@@ -901,30 +994,7 @@ __global__ __launch_bounds__(256) void k_mask_count(uint8_t *mask, uint8_t cond,
     uint8_t *s_b = reinterpret_cast<uint8_t *>(s_w);
     for (int64_t c = blockIdx.x; c < n_chunks; c += blocks) {
         const int64_t p0 = c * EVT_CHUNK + (int64_t)tid * 8;
-        unsigned long long v = ~0ull; // bytes past the end read as 255
-        if (DRAW) {
-            unsigned long long z = seed + (unsigned long long)((p0 >> 3) + 1) * 0x9E3779B97F4A7C15ull;
-            z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-            z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-            z ^= z >> 31;
-            v = z;
-            if (p0 + 8 <= N) {
-                *reinterpret_cast<unsigned long long *>(mask + p0) = z;
-            } else {
-                for (int j = 0; p0 + j < N; j++) mask[p0 + j] = (uint8_t)(z >> (8 * j));
-            }
-        } else if (p0 + 8 <= N) {
-            v = *reinterpret_cast<const unsigned long long *>(mask + p0);
-        } else {
-            for (int j = 0; j < 8; j++)
-                if (p0 + j < N) v = (v & ~(0xFFull << (8 * j))) | ((unsigned long long)mask[p0 + j] << (8 * j));
-        }
-        unsigned flags = 0;
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const bool keep = (p0 + j < N) && ((uint8_t)(v >> (8 * j)) <= cond);
-            flags |= keep ? (1u << j) : 0u;
-        }
+        const unsigned flags = mask_flags<DRAW>(mask, cond, N, p0, seed);
         s_b[tid] = (uint8_t)flags; // little end first: byte t of the chunk's flag words covers rows 8t .. 8t+7
         __syncthreads();
         if (tid < 64) {
@@ -950,53 +1020,26 @@ __global__ __launch_bounds__(1024) void k_mask_scan(const int32_t *chunk_nleft, 
     if (tid == 0) chunk_lpre[n_chunks] = total;
 }
 
-// SELF: no k_mask_scan has run - every block adds up the counts of the chunks before its own (a few hundred values:
-// cheaper than the launch).
-// The last block of the grid prepares the tree that is grown on the sample (tree_begin_block), with the number of rows kept.
-template <bool SELF>
+// The last block of the grid prepares the tree that is grown on the sample, with the number of rows kept.
 __global__ __launch_bounds__(256) void k_mask_scatter(int64_t N, int64_t n_chunks, const unsigned long long *flagw,
-                                                     const int32_t *chunk_nleft, int64_t *chunk_lpre, uint32_t *is_out, BeginArgs B) {
+                                                     const int64_t *chunk_lpre, uint32_t *is_out, BeginArgs B) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     __shared__ unsigned long long s_w[EVT_CHUNK_WORDS];
     __shared__ int s_pre[EVT_CHUNK_WORDS];
-    __shared__ int s_sum[4];
     const int64_t G = (int64_t)gridDim.x - 1;
     tree_begin_root(B, (int)gridDim.x);
     if ((int64_t)blockIdx.x == G) {
-        int64_t kept;
-        if (SELF) { // no scan has run: the chunk counts (a thousand at most) are added up here
-            int part = 0;
-            for (int64_t k = tid; k < n_chunks; k += 256) part += chunk_nleft[k];
-            part = wave_sum_i32(part);
-            if (lane == 0) s_sum[wave] = part;
-            __syncthreads();
-            kept = (int64_t)s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
-        } else {
-            kept = chunk_lpre[n_chunks];
-        }
-        B.n_is = kept;
-        B.n_is_dev = nullptr;
-        tree_begin_block(B);
+        tree_begin_arrays(B);
+        tree_begin_rows(B, chunk_lpre[n_chunks]);
         return;
     }
     for (int64_t c = blockIdx.x; c < n_chunks; c += G) {
         if (tid < EVT_CHUNK_WORDS) s_w[tid] = flagw[c * EVT_CHUNK_WORDS + tid];
-        int64_t base;
-        if (SELF) {
-            int part = 0;
-            for (int64_t k = tid; k < c; k += 256) part += chunk_nleft[k];
-            part = wave_sum_i32(part);
-            if (lane == 0) s_sum[wave] = part;
-        }
+        const int64_t base = chunk_lpre[c];
         __syncthreads();
         if (tid == 0) {
             int run = 0;
             for (int t = 0; t < EVT_CHUNK_WORDS; t++) { s_pre[t] = run; run += __popcll(s_w[t]); }
-        }
-        if (SELF) {
-            base = (int64_t)s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
-        } else {
-            base = chunk_lpre[c];
         }
         __syncthreads();
 #pragma unroll
@@ -1017,7 +1060,7 @@ static unsigned grid_for_chunks(int64_t max_chunks) {
     return (unsigned)g;
 }
 
-static void fill_begin_args(evt_ctx *c, bool all_rows, BeginArgs &A) {
+static void fill_begin_args(evt_ctx *c, BeginArgs &A) {
     const LevelTab &L = c->lvl[1];
     A.tree = c->tree;
     A.status = c->status;
@@ -1032,7 +1075,6 @@ static void fill_begin_args(evt_ctx *c, bool all_rows, BeginArgs &A) {
     A.hist = c->hist;
     A.stats = c->stats;
     A.n_is = c->N;
-    A.n_is_dev = all_rows ? nullptr : c->chunk_lpre + (c->N + EVT_CHUNK - 1) / EVT_CHUNK;
     A.seg_cost = c->hist_seg_cost;
     A.root_words = (int64_t)c->n_js_last * c->NAg * c->B;
     A.nnodes = c->nnodes;
@@ -1058,7 +1100,7 @@ static void fill_begin_args(evt_ctx *c, bool all_rows, BeginArgs &A) {
 // a tree on every row: the set-up block as a kernel of its own
 int launch_tree_begin(evt_ctx *c) {
     BeginArgs A;
-    fill_begin_args(c, true, A);
+    fill_begin_args(c, A);
     QuantArgs Q = {};
     const unsigned blocks = (unsigned)std::min<int64_t>(1 + A.root_words / 4096, 64);
     unsigned quant = 0;
@@ -1073,31 +1115,37 @@ int launch_tree_begin(evt_ctx *c) {
     return EVT_OK;
 }
 
-// Subsampling of a tree and its set-up.  draw: the mask's bytes are drawn from `seed` by the count pass (and written to
-// c->mask) instead of read.  The tree's set-up block rides in the scatter pass.
+// Subsampling of a tree and its set-up.  draw: the mask's bytes are drawn from `seed` on the way (and written to
+// c->mask) instead of read.
 int launch_compact_mask(evt_ctx *c, uint8_t cond, bool draw, unsigned long long seed) {
-    const int64_t n_chunks = (c->N + EVT_CHUNK - 1) / EVT_CHUNK;
-    unsigned g = grid_for_chunks(n_chunks);
+    BeginArgs B;
+    fill_begin_args(c, B);
     QuantArgs Q = {};
     unsigned quant = 0;
+    const int64_t blocks = (c->N + EVT_SAMPLE_ROWS - 1) / EVT_SAMPLE_ROWS;
+    const bool one = blocks <= EVT_SAMPLE_BLOCKS;
     if (c->quant_pending) {
         quant_args(c, Q);
         quant = quant_blocks(c, 256);
     }
-    if (draw) hipLaunchKernelGGL(k_mask_count<true>, dim3(g + quant), dim3(256), 0, c->stream, c->mask, cond, c->N, n_chunks, c->flagw, c->chunk_nleft, seed, Q, (int)g);
-    else hipLaunchKernelGGL(k_mask_count<false>, dim3(g + quant), dim3(256), 0, c->stream, c->mask, cond, c->N, n_chunks, c->flagw, c->chunk_nleft, 0ull, Q, (int)g);
-    HIPCHK(hipGetLastError());
-    if (quant) quant_taken(c);
-    BeginArgs B;
-    fill_begin_args(c, false, B);
-    if (n_chunks <= 1024) { // the scatter's blocks add up the counts before their chunk themselves
-        hipLaunchKernelGGL(k_mask_scatter<true>, dim3(g + 1), dim3(256), 0, c->stream, c->N, n_chunks, c->flagw, c->chunk_nleft, c->chunk_lpre, c->is_a, B);
-    } else {
+    if (one) {
+        const dim3 grid((unsigned)blocks + 1 + quant);
+        if (draw) hipLaunchKernelGGL(k_mask_sample<true>, grid, dim3(256), 0, c->stream, c->mask, cond, c->N, seed, c->is_a, c->sample_claims, B, Q, (int)blocks);
+        else hipLaunchKernelGGL(k_mask_sample<false>, grid, dim3(256), 0, c->stream, c->mask, cond, c->N, 0ull, c->is_a, c->sample_claims, B, Q, (int)blocks);
+        HIPCHK(hipGetLastError());
+        if (quant) quant_taken(c);
+    } else { // counts, their scan, and the rows' places from it
+        const int64_t n_chunks = (c->N + EVT_CHUNK - 1) / EVT_CHUNK;
+        const unsigned g = grid_for_chunks(n_chunks);
+        if (draw) hipLaunchKernelGGL(k_mask_count<true>, dim3(g + quant), dim3(256), 0, c->stream, c->mask, cond, c->N, n_chunks, c->flagw, c->chunk_nleft, seed, Q, (int)g);
+        else hipLaunchKernelGGL(k_mask_count<false>, dim3(g + quant), dim3(256), 0, c->stream, c->mask, cond, c->N, n_chunks, c->flagw, c->chunk_nleft, 0ull, Q, (int)g);
+        HIPCHK(hipGetLastError());
+        if (quant) quant_taken(c);
         hipLaunchKernelGGL(k_mask_scan, dim3(1), dim3(1024), 0, c->stream, c->chunk_nleft, c->chunk_lpre, n_chunks);
         HIPCHK(hipGetLastError());
-        hipLaunchKernelGGL(k_mask_scatter<false>, dim3(g + 1), dim3(256), 0, c->stream, c->N, n_chunks, c->flagw, c->chunk_nleft, c->chunk_lpre, c->is_a, B);
+        hipLaunchKernelGGL(k_mask_scatter, dim3(g + 1), dim3(256), 0, c->stream, c->N, n_chunks, c->flagw, c->chunk_lpre, c->is_a, B);
+        HIPCHK(hipGetLastError());
     }
-    HIPCHK(hipGetLastError());
     c->js_staged = false;
     return EVT_OK;
 }
