@@ -51,9 +51,8 @@
 // one-pass partition: a node's cursor has a 128-byte line to itself (additions to one line follow each other); the nodes of very deep levels, of few
 // chunks each, share lines
 #define EVT_CURSOR_SLOT(n) ((n) < 1024 ? (size_t)(n) * 16 : (size_t)16384 - 1024 + (n))
-// row sample in one kernel: rows of a block, and blocks (claims of one address, ~15 ns each: more of them take the count and the scatter)
+// rows of a block of the row sample
 #define EVT_SAMPLE_ROWS 8192
-#define EVT_SAMPLE_BLOCKS 512
 #define EVT_CURSOR_WORDS(nnodes) ((size_t)16384 + (nnodes) + 2)
 
 // split search: a node's block counter has a 128-byte line to itself (additions to one line follow each other, ~15 ns each)

@@ -822,7 +822,7 @@ struct BeginArgs {
 
 // One block prepares a tree: empty Tree arrays, node states, the column sample; and, once the number of its rows is known, the first level's tables.
 // A kernel of its own for a tree on every row; with a row sample they ride in the kernel that
-// compacts the sampled rows (k_mask_sample, k_mask_scatter), which counts them.
+// lists the sampled rows (k_mask_sample), which counts them.
 __device__ void tree_begin_arrays(const BeginArgs &A) {
     const int tid = threadIdx.x, nthr = blockDim.x; // 256 or 1024; each of four wavefronts starts another of the short lists
     for (int n = tid; n < A.nnodes; n += nthr) {
@@ -882,13 +882,7 @@ __global__ __launch_bounds__(1024) void k_tree_begin(BeginArgs A, QuantArgs Q, i
     }
 }
 
-// ---- row subsampling: is = rows with mask <= cond, ascending (src/subsample.jl:6-38) -----------
-__device__ __forceinline__ int wave_sum_i32(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
-
+// ---- row subsampling: is = rows with mask <= cond (src/subsample.jl:6-38) -----------
 // Which of the rows p0 .. p0 + 7 (p0 a multiple of 8) the mask keeps, row p0 in the lowest bit.
 // DRAW: the bytes are not read but drawn here and written to `mask` on the way: the mask's 8-byte word w is output w of
 // SplitMix64 (Steele, Lea, Flood 2014: a Weyl sequence with increment 0x9E3779B97F4A7C15 passed through two
@@ -924,12 +918,13 @@ __device__ __forceinline__ unsigned mask_flags(uint8_t *mask, uint8_t cond, int6
     return flags;
 }
 
-// The sample of up to EVT_SAMPLE_BLOCKS blocks' rows, and the tree's set-up, in one kernel: a block flags its 8192 rows, claims as many places of the
+// The sample's rows, and the tree's set-up, in one kernel: a block flags its 8192 rows, claims as many places of the
 // list by one addition and writes their ids there.  A block's rows stay in order, the blocks follow each other in the order of their
 // claims, which nothing depends on (k_part_move's chunks do the same).  The block that claims last knows the number of rows and writes the first
 // level's tables; block 0 prepares the rest of the tree, blocks behind the sample's quantise.  Bound by its chain (draw, count, claim, stores) and the
 // quantisation beside it: 1M rows 7.9 us with one word a row, 10.0 with two (a block's rows by 1024 threads: 9.1, 12.4: quantisation gets its blocks later).  In two kernels, a
-// count and a scatter that added the counts up, 5.9 + 5.1 and 8.9 + 4.7.
+// count and a scatter that added the counts up, 5.9 + 5.1 and 8.9 + 4.7; with a scan between them, from 2M rows on,
+// 100 rounds of 6M x 20 46.2 ms for 45.5, of 10M 67.4 for 67.7.
 template <bool DRAW>
 __global__ __launch_bounds__(256) void k_mask_sample(uint8_t *mask, uint8_t cond, int64_t N, unsigned long long seed, uint32_t *is_out,
                                                      unsigned long long *claims, BeginArgs B, QuantArgs Q, int blocks) {
@@ -977,79 +972,6 @@ __global__ __launch_bounds__(256) void k_mask_sample(uint8_t *mask, uint8_t cond
     if ((int)(claim >> 40) == blocks - 1) {
         if (tid == 0) *claims = 0ull; // for the next launch
         tree_begin_rows(B, base + total);
-    }
-}
-
-// A thread takes 8 consecutive mask bytes (one load); the 8 flags of 8 neighbouring threads make one 64-row flag word.
-template <bool DRAW>
-__global__ __launch_bounds__(256) void k_mask_count(uint8_t *mask, uint8_t cond, int64_t N, int64_t n_chunks,
-                                                   unsigned long long *flagw, int32_t *chunk_nleft, unsigned long long seed, QuantArgs Q, int blocks) {
-    if ((int)blockIdx.x >= blocks) { // as k_tree_begin
-        quant_rows(Q, (int)blockIdx.x - blocks, (int)gridDim.x - blocks);
-        return;
-    }
-    static_assert(EVT_CHUNK == 2048 && EVT_CHUNK_WORDS == 32, "a chunk is 256 threads x 8 bytes");
-    const int tid = threadIdx.x;
-    __shared__ unsigned long long s_w[EVT_CHUNK_WORDS];
-    uint8_t *s_b = reinterpret_cast<uint8_t *>(s_w);
-    for (int64_t c = blockIdx.x; c < n_chunks; c += blocks) {
-        const int64_t p0 = c * EVT_CHUNK + (int64_t)tid * 8;
-        const unsigned flags = mask_flags<DRAW>(mask, cond, N, p0, seed);
-        s_b[tid] = (uint8_t)flags; // little end first: byte t of the chunk's flag words covers rows 8t .. 8t+7
-        __syncthreads();
-        if (tid < 64) {
-            const unsigned long long w = tid < EVT_CHUNK_WORDS ? s_w[tid] : 0ull;
-            if (tid < EVT_CHUNK_WORDS) flagw[c * EVT_CHUNK_WORDS + tid] = w;
-            int cnt = __popcll(w);
-            cnt = wave_sum_i32(cnt);
-            if (tid == 0) chunk_nleft[c] = cnt;
-        }
-        __syncthreads();
-    }
-}
-
-__global__ __launch_bounds__(1024) void k_mask_scan(const int32_t *chunk_nleft, int64_t *chunk_lpre, int64_t n_chunks) {
-    __shared__ long long s_tmp[17];
-    const int tid = threadIdx.x;
-    const int64_t span = (n_chunks + 1023) / 1024;
-    const int64_t c0 = (int64_t)tid * span, c1 = (c0 + span < n_chunks) ? c0 + span : n_chunks;
-    long long s = 0, total;
-    for (int64_t c = c0; c < c1; c++) s += chunk_nleft[c];
-    long long pre = block_excl_scan(s, &total, s_tmp);
-    for (int64_t c = c0; c < c1; c++) { chunk_lpre[c] = pre; pre += chunk_nleft[c]; }
-    if (tid == 0) chunk_lpre[n_chunks] = total;
-}
-
-// The last block of the grid prepares the tree that is grown on the sample, with the number of rows kept.
-__global__ __launch_bounds__(256) void k_mask_scatter(int64_t N, int64_t n_chunks, const unsigned long long *flagw,
-                                                     const int64_t *chunk_lpre, uint32_t *is_out, BeginArgs B) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    __shared__ unsigned long long s_w[EVT_CHUNK_WORDS];
-    __shared__ int s_pre[EVT_CHUNK_WORDS];
-    const int64_t G = (int64_t)gridDim.x - 1;
-    tree_begin_root(B, (int)gridDim.x);
-    if ((int64_t)blockIdx.x == G) {
-        tree_begin_arrays(B);
-        tree_begin_rows(B, chunk_lpre[n_chunks]);
-        return;
-    }
-    for (int64_t c = blockIdx.x; c < n_chunks; c += G) {
-        if (tid < EVT_CHUNK_WORDS) s_w[tid] = flagw[c * EVT_CHUNK_WORDS + tid];
-        const int64_t base = chunk_lpre[c];
-        __syncthreads();
-        if (tid == 0) {
-            int run = 0;
-            for (int t = 0; t < EVT_CHUNK_WORDS; t++) { s_pre[t] = run; run += __popcll(s_w[t]); }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int it = 0; it < EVT_CHUNK / 256; it++) {
-            const int64_t p = c * EVT_CHUNK + it * 256 + tid;
-            const int wi = it * 4 + wave;
-            const unsigned long long word = s_w[wi];
-            if ((word >> lane) & 1ull) is_out[base + s_pre[wi] + __popcll(word & ((1ull << lane) - 1ull))] = (uint32_t)p;
-        }
-        __syncthreads();
     }
 }
 
@@ -1123,29 +1045,15 @@ int launch_compact_mask(evt_ctx *c, uint8_t cond, bool draw, unsigned long long 
     QuantArgs Q = {};
     unsigned quant = 0;
     const int64_t blocks = (c->N + EVT_SAMPLE_ROWS - 1) / EVT_SAMPLE_ROWS;
-    const bool one = blocks <= EVT_SAMPLE_BLOCKS;
     if (c->quant_pending) {
         quant_args(c, Q);
         quant = quant_blocks(c, 256);
     }
-    if (one) {
-        const dim3 grid((unsigned)blocks + 1 + quant);
-        if (draw) hipLaunchKernelGGL(k_mask_sample<true>, grid, dim3(256), 0, c->stream, c->mask, cond, c->N, seed, c->is_a, c->sample_claims, B, Q, (int)blocks);
-        else hipLaunchKernelGGL(k_mask_sample<false>, grid, dim3(256), 0, c->stream, c->mask, cond, c->N, 0ull, c->is_a, c->sample_claims, B, Q, (int)blocks);
-        HIPCHK(hipGetLastError());
-        if (quant) quant_taken(c);
-    } else { // counts, their scan, and the rows' places from it
-        const int64_t n_chunks = (c->N + EVT_CHUNK - 1) / EVT_CHUNK;
-        const unsigned g = grid_for_chunks(n_chunks);
-        if (draw) hipLaunchKernelGGL(k_mask_count<true>, dim3(g + quant), dim3(256), 0, c->stream, c->mask, cond, c->N, n_chunks, c->flagw, c->chunk_nleft, seed, Q, (int)g);
-        else hipLaunchKernelGGL(k_mask_count<false>, dim3(g + quant), dim3(256), 0, c->stream, c->mask, cond, c->N, n_chunks, c->flagw, c->chunk_nleft, 0ull, Q, (int)g);
-        HIPCHK(hipGetLastError());
-        if (quant) quant_taken(c);
-        hipLaunchKernelGGL(k_mask_scan, dim3(1), dim3(1024), 0, c->stream, c->chunk_nleft, c->chunk_lpre, n_chunks);
-        HIPCHK(hipGetLastError());
-        hipLaunchKernelGGL(k_mask_scatter, dim3(g + 1), dim3(256), 0, c->stream, c->N, n_chunks, c->flagw, c->chunk_lpre, c->is_a, B);
-        HIPCHK(hipGetLastError());
-    }
+    const dim3 grid((unsigned)blocks + 1 + quant);
+    if (draw) hipLaunchKernelGGL(k_mask_sample<true>, grid, dim3(256), 0, c->stream, c->mask, cond, c->N, seed, c->is_a, c->sample_claims, B, Q, (int)blocks);
+    else hipLaunchKernelGGL(k_mask_sample<false>, grid, dim3(256), 0, c->stream, c->mask, cond, c->N, 0ull, c->is_a, c->sample_claims, B, Q, (int)blocks);
+    HIPCHK(hipGetLastError());
+    if (quant) quant_taken(c);
     c->js_staged = false;
     return EVT_OK;
 }

@@ -705,7 +705,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
                 for (int i = 0; i < 4; i++) {
                     uint32_t m = (mb >> (8 * i)) & 0xFFu;
                     if (A.draw) {
-                        unsigned long long z = A.seed + (unsigned long long)(((r + i) >> 3) + 1) * 0x9E3779B97F4A7C15ull; // SplitMix64, as k_mask_count
+                        unsigned long long z = A.seed + (unsigned long long)(((r + i) >> 3) + 1) * 0x9E3779B97F4A7C15ull; // SplitMix64, as mask_flags
                         z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
                         z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
                         z ^= z >> 31;
