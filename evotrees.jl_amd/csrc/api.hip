@@ -7,8 +7,10 @@
 #include <string.h>
 
 #include <algorithm>
+#include <chrono>
 #include <memory>
 #include <new>
+#include <thread>
 
 int launch_absmax_rows(evt_ctx *c, int k0, int k1);
 int launch_check_unit_weight(evt_ctx *c);
@@ -179,7 +181,7 @@ extern "C" int evt_destroy(evt_handle c) {
     if (!c) return EVT_OK;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    void *ptrs[] = {c->xcm, c->xrm, c->y, c->pred, c->grad, c->gq, c->is_a, c->is_b, c->nidx, c->mask, c->flagw, c->sample_claims, c->chunk_nleft, c->chunk_lpre, c->cursor,
+    void *ptrs[] = {c->xcm, c->xrm, c->y, c->pred, c->grad, c->gq, c->is_a, c->is_b, c->nidx, c->mask, c->flagw, c->sample_claims, c->blob_arrived, c->chunk_nleft, c->chunk_lpre, c->cursor,
                     c->hist, c->seg_start, c->seg_len, c->status, c->node_sum, c->tree_blob, c->tree.packed, c->js, c->jsmap, c->feattypes, c->mono, c->absmax, c->qexp_buf[0], c->qexp_buf[1], c->qbits,
                     c->qscale_buf[0], c->qscale_buf[1], c->planes, c->metric_partial, c->errflag, c->ogains, c->sbest, c->scan_count, c->is_id, c->pt_nodes, c->mask_next,
                     c->small_nid[0], c->small_nid[1], c->small_head[0], c->small_head[1], c->small_left[0], c->small_left[1], c->small_acc,
@@ -266,7 +268,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->have_xbin = c->have_target = c->have_grads = false;
     c->planes = nullptr; c->plane_words = 0; c->planes_ready = false; c->use_planes = 1;
     c->xcm = nullptr; c->xrm = nullptr; c->y = nullptr; c->pred = nullptr; c->grad = nullptr; c->gq = nullptr; c->gq_rows = false;
-    c->is_a = c->is_b = nullptr; c->nidx = nullptr; c->mask = nullptr; c->flagw = nullptr; c->sample_claims = nullptr; c->chunk_nleft = nullptr; c->chunk_lpre = nullptr; c->cursor = nullptr;
+    c->is_a = c->is_b = nullptr; c->nidx = nullptr; c->mask = nullptr; c->flagw = nullptr; c->sample_claims = nullptr; c->blob_arrived = nullptr; c->slot_ev[0] = c->slot_ev[1] = false; c->chunk_nleft = nullptr; c->chunk_lpre = nullptr; c->cursor = nullptr;
     c->hist = nullptr; c->seg_start = c->seg_len = nullptr; c->status = nullptr; c->node_sum = nullptr;
     memset(&c->tree, 0, sizeof(c->tree));
     c->tree_blob = nullptr;
@@ -351,6 +353,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     ALLOC(c->nidx, N);
     ALLOC(c->mask, N);
     ALLOC(c->sample_claims, 1);
+    ALLOC(c->blob_arrived, 1);
     ALLOC(c->flagw, (size_t)c->max_chunks * EVT_CHUNK_WORDS);
     ALLOC(c->chunk_nleft, c->max_chunks + 1);
     ALLOC(c->chunk_lpre, c->max_chunks + 1);
@@ -418,10 +421,14 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     // pinned staging: tree read-back + small per-tree uploads
     c->h_stage_bytes = c->blob_bytes + (size_t)c->F * 4 + (size_t)c->RS * 2 + 1024;
     c->h_stage_bytes = (c->h_stage_bytes + 255) / 256 * 256;
-    c->h_stage_base = c->h_stage_dev_base = static_cast<uint8_t *>(pinned_take(2 * c->h_stage_bytes));
+    c->h_stage_base = c->h_stage_dev_base = static_cast<uint8_t *>(pinned_take(2 * c->h_stage_bytes + 128));
     if (!c->h_stage_base) {
         evt_destroy(c);
         return EVT_ERR_NOMEM;
+    }
+    for (int k = 0; k < 2; k++) { // behind the slots, a line each; trees count from 1
+        c->slot_flag[k] = reinterpret_cast<unsigned long long *>(c->h_stage_base + 2 * c->h_stage_bytes + 64 * k);
+        *c->slot_flag[k] = 0;
     }
     c->h_stage = c->h_stage_base;
     c->h_stage_dev = c->h_stage_dev_base;
@@ -433,6 +440,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->absmax, 0, sizeof(uint32_t) * 2 * EVT_ABSMAX_STRIPES * EVT_MC_MAX_NK, c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->nidx, 0, sizeof(uint32_t) * N, c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->errflag, 0, sizeof(int32_t), c->stream);
+    if (e2 == hipSuccess) e2 = hipMemsetAsync(c->blob_arrived, 0, sizeof(int), c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->sample_claims, 0, sizeof(unsigned long long), c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->scan_count, 0, sizeof(int32_t) * EVT_SCAN_COUNT_STEP * c->maxlvl, c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->metric_partial + 2 * EVT_METRIC_BLOCKS, 0, sizeof(double), c->stream);
@@ -1030,10 +1038,11 @@ static int tree_close(evt_ctx *c) {
 
     // the tree (and the per-level row counts) comes back in one pinned transfer, queued behind the kernels
     if (!c->step.blob_sent) {
-        r = launch_copy_to_host(c, c->tree_blob, c->h_stage_dev, c->blob_bytes);
+        r = launch_copy_to_host(c, true);
         if (r != EVT_OK) return r;
     }
-    HIPCHK(hipEventRecord(c->tree_evs[c->slot_w], c->stream));
+    c->slot_ev[c->slot_w] = c->profiling != 0; // the times of all its kernels are read when it is collected
+    if (c->profiling) HIPCHK(hipEventRecord(c->tree_evs[c->slot_w], c->stream));
     c->slot_seq[c->slot_w] = c->tree_seq;
     if (c->grads_ahead && p->update_pred && p->bagging_size == 1) {
         // the next round's gradient update runs while the host collects this tree and prepares the next call.  Not with
@@ -1215,6 +1224,44 @@ static int fill_tree_out(evt_ctx *c, const uint8_t *hs, evt_tree_out *tree) {
     return EVT_OK;
 }
 
+static inline void spin_pause() {
+#if defined(__x86_64__)
+    __builtin_ia32_pause();
+#endif
+}
+
+// Until a slot's tree has arrived; work queued behind it, and what else its last kernel does, may still be running.  The device writes the tree's number
+// behind its arrays; a stream that has failed, or run dry without, is found out by asking it now and then.
+static int wait_for_tree(evt_ctx *c, int slot) {
+    if (c->slot_ev[slot]) {
+        HIPCHK(hipEventSynchronize(c->tree_evs[slot]));
+        return EVT_OK;
+    }
+    const unsigned long long seq = (unsigned long long)c->slot_seq[slot];
+    auto there = [&]() { return __atomic_load_n(c->slot_flag[slot], __ATOMIC_ACQUIRE) == seq; };
+    for (int k = 0; k < 4096; k++) {
+        if (there()) return EVT_OK;
+        spin_pause();
+    }
+    auto asked = std::chrono::steady_clock::now();
+    while (!there()) {
+        std::this_thread::yield();
+        const auto now = std::chrono::steady_clock::now();
+        if (now - asked < std::chrono::milliseconds(200)) continue;
+        asked = now;
+        const hipError_t q = hipStreamQuery(c->stream);
+        if (q == hipErrorNotReady) {
+            (void)hipGetLastError();
+        } else if (q != hipSuccess) {
+            HIPCHK(q);
+        } else if (!there()) {
+            evt_set_error("internal: a tree's kernels have ended without it");
+            return EVT_ERR_INTERNAL;
+        }
+    }
+    return EVT_OK;
+}
+
 extern "C" int evt_grow_tree_end(evt_handle c, evt_tree_out *tree) {
     return guarded([&]() -> int {
     ARGCHK(c != nullptr, "handle is NULL");
@@ -1229,7 +1276,8 @@ extern "C" int evt_grow_tree_end(evt_handle c, evt_tree_out *tree) {
     c->slot_r ^= 1;
     const uint8_t *hs = c->h_stage_base + (size_t)slot * c->h_stage_bytes;
     const size_t o_stats = c->blob_stats;
-    HIPCHK(hipEventSynchronize(c->tree_evs[slot])); // the tree has arrived; work queued behind it may still be running
+    const int arrived = wait_for_tree(c, slot);
+    if (arrived != EVT_OK) return arrived;
     const int64_t n_is = reinterpret_cast<const int64_t *>(hs + o_stats)[0];
     if (c->profiling || !c->recs.empty()) {
         if (c->profiling) c->prof_units[EVT_K_PARTITION] += n_is;
@@ -1249,7 +1297,7 @@ extern "C" int evt_peek_tree(evt_handle c, evt_tree_out *tree) {
     return guarded([&]() -> int {
     CTXCHK_STEP(c);
     ARGCHK(tree, "tree is NULL");
-    int r = launch_copy_to_host(c, c->tree_blob, c->h_stage_dev, c->blob_bytes);
+    int r = launch_copy_to_host(c, false);
     if (r != EVT_OK) return r;
     HIPCHK(hipStreamSynchronize(c->stream));
     return fill_tree_out(c, c->h_stage, tree);

@@ -217,7 +217,11 @@ struct evt_ctx {
     bool write_nidx;   // the tree being grown records the node id of every row it places
     bool grads_ahead;    // option: a tree with update_pred queues the next gradient update behind itself
     bool grads_ready;    // the gradients of the predictions as they stand were computed ahead: evt_update_grads has nothing to do
-    hipEvent_t tree_evs[2]; // per slot, recorded behind the tree's transfer to the host: evt_grow_tree_end waits for this, not for the stream
+    // per slot: the word that the tree's number is written to behind its arrays; with kernels being timed, an event behind them all (slot_ev)
+    unsigned long long *slot_flag[2];
+    int *blob_arrived;
+    hipEvent_t tree_evs[2];
+    bool slot_ev[2];
     int tree_in_flight;     // trees queued by evt_grow_tree_begin that evt_grow_tree_end has not collected (0..2)
     int slot_w, slot_r;     // staging slot of the next tree queued / of the oldest tree not yet collected
     int64_t tree_seq;       // trees opened so far; slot_seq: the tree each slot holds
@@ -334,6 +338,34 @@ __device__ __forceinline__ unsigned long long evt_load_gq(const unsigned long lo
     return gq[(size_t)a * N + id];
 }
 
+// The finished tree's arrays on their way to the host's pinned buffer, in `blocks` blocks of the tree's last kernel, and behind them the word the host
+// waits for.  An event recorded behind the kernel put a packet into the queue that the next tree's first kernel waited for: 5.5 us between two trees,
+// where kernels of one tree follow each other without a gap.
+// Order: the words go out as system-scope atomic stores, past the device's caches; each thread waits for its own to arrive; the block that
+// counts itself last stores the flag.
+struct BlobOut {
+    const uint4 *src;
+    uint4 *dst;
+    int64_t n; // 16-byte words
+    int blocks;
+    int *arrived; // blocks that have stored theirs, zero between trees
+    unsigned long long *flag, seq; // the slot's word in pinned memory (nullptr: nobody waits for it), and what it becomes
+};
+__device__ __forceinline__ void blob_send(const BlobOut &O, int block) {
+    const unsigned long long *s = reinterpret_cast<const unsigned long long *>(O.src);
+    unsigned long long *d = reinterpret_cast<unsigned long long *>(O.dst);
+    for (int64_t i = (int64_t)block * blockDim.x + threadIdx.x; i < 2 * O.n; i += (int64_t)O.blocks * blockDim.x)
+        __hip_atomic_store(d + i, s[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x != 0 || !O.flag) return;
+    if (O.blocks > 1) {
+        if (__hip_atomic_fetch_add(O.arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != O.blocks - 1) return;
+        *O.arrived = 0;
+    }
+    __hip_atomic_store(O.flag, O.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The words of channels a0 .. a0 + NA - 1 of one row, side by side in memory (stride: words from row to row, even; a0 even) - one request per 16 bytes,
 // all of one line, where planes of N words cost a line for each channel once a node's rows lie apart, and again in every column tile.  One channel alone is a
 // plane of 32-bit words in either layout.  us a histogram level, planes -> side by side: 500k rows x 50 of four channels 17.9 to 19.1 -> 15.6 to 18.3, 60k x 30 of 14
@@ -411,7 +443,9 @@ bool small_root_quantises(const evt_ctx *c, int form);
 int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices);
 int launch_final_fused(evt_ctx *c, int level, const uint32_t *is_cur, bool fuse_pred, bool send_blob);
 int launch_nidx_from_segments(evt_ctx *c, int level, const uint32_t *is_cur);
-int launch_copy_to_host(evt_ctx *c, const void *src_dev, void *dst_host_dev, size_t nbytes);
+struct BlobOut;
+void blob_out(evt_ctx *c, BlobOut &O);
+int launch_copy_to_host(evt_ctx *c, bool flag);
 int launch_copy_words(evt_ctx *c, const void *src, void *dst, size_t nbytes);
 int launch_fill_u32(evt_ctx *c, uint32_t *dst, uint32_t v, int64_t n);
 int launch_fill_bytes(evt_ctx *c, void *dst, int64_t nbytes);

@@ -68,11 +68,7 @@ struct PartArgs {
     long long *hist;
     int64_t node_stride;
     int F, nfs, NAg;
-    // last pass of a tree: the finished tree's arrays go to the host's pinned buffer in copy_blocks extra blocks
-    const uint4 *copy_src;
-    uint4 *copy_dst;
-    int64_t copy_n;
-    int copy_blocks;
+    BlobOut blob; // last pass of a tree: its arrays go to the host in blob.blocks extra blocks
     // one-pass form: rows the node's chunks have placed so far, and the nodes' totals, whose last channel counts rows
     unsigned long long *cursor;
     const long long *node_sum;
@@ -721,11 +717,11 @@ __global__ __launch_bounds__(T) void k_part_move(PartArgs A, NextArgs NX) {
 template <bool NT>
 __global__ __launch_bounds__(256) void k_final_fused(PartArgs A) {
     const int tid = threadIdx.x;
-    const int64_t G = (int64_t)gridDim.x - A.copy_blocks;
+    const int64_t G = (int64_t)gridDim.x - A.blob.blocks;
     if ((int64_t)blockIdx.x >= G) {
         // the tree's arrays are complete (this is the tree's last kernel and writes none of them): their way back to the
         // host rides along instead of taking a launch of its own
-        for (int64_t i = ((int64_t)blockIdx.x - G) * 256 + tid; i < A.copy_n; i += (int64_t)A.copy_blocks * 256) A.copy_dst[i] = A.copy_src[i];
+        blob_send(A.blob, (int)(blockIdx.x - G));
         return;
     }
     uint4 cd = A.cdesc[blockIdx.x];
@@ -1094,10 +1090,7 @@ static void fill_part_args(evt_ctx *c, int level, const uint32_t *is_cur, uint32
     A.node_stride = 0;
     A.F = A.nfs = 0;
     A.NAg = c->NAg;
-    A.copy_src = nullptr;
-    A.copy_dst = nullptr;
-    A.copy_n = 0;
-    A.copy_blocks = 0;
+    A.blob.blocks = 0;
     A.cursor = c->cursor;
     A.node_sum = c->node_sum;
 }
@@ -1231,13 +1224,10 @@ int launch_final_fused(evt_ctx *c, int level, const uint32_t *is_cur, bool fuse_
     PartArgs A;
     fill_part_args(c, level, is_cur, nullptr, fuse_pred, A);
     if (send_blob) {
-        A.copy_src = reinterpret_cast<const uint4 *>(c->tree_blob);
-        A.copy_dst = reinterpret_cast<uint4 *>(c->h_stage_dev);
-        A.copy_n = (int64_t)(c->blob_bytes / 16);
-        A.copy_blocks = (int)std::min<int64_t>(64, (A.copy_n + 255) / 256);
+        blob_out(c, A.blob);
         c->step.blob_sent = true;
     }
-    const dim3 grid(grid_for_chunks(c->max_chunks) + (unsigned)A.copy_blocks);
+    const dim3 grid(grid_for_chunks(c->max_chunks) + (unsigned)A.blob.blocks);
     if (A.stream_hint) hipLaunchKernelGGL(k_final_fused<true>, grid, dim3(256), 0, c->stream, A);
     else hipLaunchKernelGGL(k_final_fused<false>, grid, dim3(256), 0, c->stream, A);
     HIPCHK(hipGetLastError());

@@ -21,8 +21,7 @@ __device__ __forceinline__ int walk_packed(const uint32_t *__restrict__ nodes, c
     return nid;
 }
 
-// one tree added to pred (K x N), all rows.  copy_blocks extra blocks at the end of the grid carry copy_n 16-byte words
-// from copy_src to copy_dst: the finished tree's way back to the host's pinned buffer, when this is the tree's last kernel.
+// one tree added to pred (K x N), all rows.  blob.blocks extra blocks at the end of the grid send the finished tree to the host, when this is its last kernel.
 // A row's walk is a chain of dependent loads (node word, bin byte, node word, ...), so the kernel is paced by latency, not by
 // the bytes it moves: the first n_lds node words (the upper levels of the heap, all of it for depths up to 13) are copied to
 // LDS, where a lookup costs a fraction of a trip to the caches, and a thread walks R rows side by side - R bin bytes are
@@ -38,15 +37,14 @@ struct GradOut {
 template <int R, int LOSS>
 __global__ __launch_bounds__(LOSS < 0 ? 256 : 1024) void k_predict_tree(const uint32_t *__restrict__ nodes, int n_lds, const float *__restrict__ leaf_pred,
                                                      const uint8_t *__restrict__ xcm, int64_t N, int K, int loss, float *pred,
-                                                     const uint4 *__restrict__ copy_src, uint4 *__restrict__ copy_dst, int64_t copy_n,
-                                                     int copy_blocks, GradOut O) {
+                                                     BlobOut blob, GradOut O) {
     extern __shared__ uint32_t s_nodes[];
     constexpr bool GRADS = LOSS >= 0;
     constexpr int KG = LOSS == 2 || LOSS == 7 ? 2 : 1, NKG = 2 * KG + 1;
     const int nthr = GRADS ? (int)blockDim.x : 256;
-    const int64_t G = (int64_t)gridDim.x - copy_blocks;
+    const int64_t G = (int64_t)gridDim.x - blob.blocks;
     if ((int64_t)blockIdx.x >= G) {
-        for (int64_t k = ((int64_t)blockIdx.x - G) * nthr + threadIdx.x; k < copy_n; k += (int64_t)copy_blocks * nthr) copy_dst[k] = copy_src[k];
+        blob_send(blob, (int)(blockIdx.x - G));
         return;
     }
     const int64_t i0 = (int64_t)blockIdx.x * (nthr * R) + threadIdx.x;
@@ -127,17 +125,16 @@ __global__ __launch_bounds__(LOSS < 0 ? 256 : 1024) void k_predict_tree(const ui
 // rows per thread: four once the rows fill the device several times over, one for small inputs (more blocks)
 // grads: with the next round's gradients.  Blocks raise the maxima one after the other, so that those of large inputs are wide and walk two rows a thread (1M rows,
 // depth 6 | depth 8: blocks of 256 15.1 | 17.7 us, 512 14.1 | 16.3, 1024 13.1 | 15.3, 1024 and two rows 11.8 | 14.2).
-static int launch_predict_tree_any(evt_ctx *c, const uint32_t *nodes, int nnodes, const float *leaf_pred, const uint4 *copy_src, uint4 *copy_dst,
-                                   int64_t copy_n, int copy_blocks, bool grads) {
+static int launch_predict_tree_any(evt_ctx *c, const uint32_t *nodes, int nnodes, const float *leaf_pred, const BlobOut &blob, bool grads) {
     const int n_lds = nnodes < 8192 ? nnodes : 8192;
     const size_t lds = (size_t)n_lds * sizeof(uint32_t);
     const GradOut O = {c->y, c->grad, absmax_set(c, c->absmax_cur), c->unit_w ? 1 : 0};
     const bool wide = grads && c->N > 2047 * 256;
     const int R = c->N >= ((int64_t)1 << 21) ? 4 : wide ? 2 : 1, threads = wide ? 1024 : 256;
-    const dim3 grid((unsigned)((c->N + threads * R - 1) / (threads * R)) + (unsigned)copy_blocks);
+    const dim3 grid((unsigned)((c->N + threads * R - 1) / (threads * R)) + (unsigned)blob.blocks);
 #define PT(R_, LOSS_)                                                                                                                               \
     hipLaunchKernelGGL((k_predict_tree<R_, LOSS_>), grid, dim3(threads), lds, c->stream, nodes, n_lds, leaf_pred, c->xcm, c->N, c->K, c->loss, c->pred, \
-                       copy_src, copy_dst, copy_n, copy_blocks, O)
+                       blob, O)
 #define PT1(LOSS_) PT(1, LOSS_)
 #define PT2(LOSS_) PT(2, LOSS_)
 #define PT4(LOSS_) PT(4, LOSS_)
@@ -178,10 +175,9 @@ int launch_nidx_from_tree(evt_ctx *c, bool use_mask, uint8_t cond) {
 }
 
 int launch_predict_tree_cache(evt_ctx *c, bool send_blob, bool grads) {
-    const int64_t copy_n = send_blob ? (int64_t)(c->blob_bytes / 16) : 0;
-    const int copy_blocks = (int)std::min<int64_t>(64, (copy_n + 255) / 256);
-    const int r = launch_predict_tree_any(c, c->tree.packed, c->nnodes, c->tree.pred, reinterpret_cast<const uint4 *>(c->tree_blob),
-                                          reinterpret_cast<uint4 *>(c->h_stage_dev), copy_n, copy_blocks, grads);
+    BlobOut blob = {};
+    if (send_blob) blob_out(c, blob);
+    const int r = launch_predict_tree_any(c, c->tree.packed, c->nnodes, c->tree.pred, blob, grads);
     if (r != EVT_OK) return r;
     if (send_blob) c->step.blob_sent = true;
     if (grads) c->step.grads_done = true;
@@ -189,7 +185,7 @@ int launch_predict_tree_cache(evt_ctx *c, bool send_blob, bool grads) {
 }
 
 int launch_predict_tree_nodes(evt_ctx *c, const uint32_t *nodes_dev, int nnodes, const float *leaf_pred_dev) {
-    return launch_predict_tree_any(c, nodes_dev, nnodes, leaf_pred_dev, static_cast<const uint4 *>(nullptr), static_cast<uint4 *>(nullptr), (int64_t)0, 0, false);
+    return launch_predict_tree_any(c, nodes_dev, nnodes, leaf_pred_dev, BlobOut{}, false);
 }
 
 // apply_prediction_link!, src/predict.jl:105-116 (softmax!: :187-195)

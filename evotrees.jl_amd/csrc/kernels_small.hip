@@ -52,9 +52,7 @@ struct SmallArgs {
     int32_t *qexp;
     TreeDev tree;
     int64_t *stats;
-    const uint4 *blob_src; // final kernel: the tree's arrays and their pinned destination
-    uint4 *blob_dst;
-    int64_t blob_n;
+    BlobOut blob; // final kernel: the tree's arrays and their pinned destination
     uint32_t *nidx;
     // final kernel, where it computes the next round's gradients (k_grads)
     float *pred;
@@ -1042,7 +1040,7 @@ __global__ __launch_bounds__(1024) void k_small_final(SmallArgs A) {
         }
         __syncthreads();
     }
-    for (int64_t i = tid; i < A.blob_n; i += 1024) A.blob_dst[i] = A.blob_src[i];
+    blob_send(A.blob, 0);
 }
 
 static size_t small_lds(const evt_ctx *c, int level, int slots, bool split) {
@@ -1209,9 +1207,8 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
         A.left_in = c->small_left[in]; A.left_out = c->small_left[out];
         if (level == c->D) {
             prof_begin(c, EVT_K_PARTITION, level);
-            A.blob_src = reinterpret_cast<const uint4 *>(c->tree_blob);
-            A.blob_dst = reinterpret_cast<uint4 *>(c->h_stage_dev);
-            A.blob_n = (int64_t)(c->blob_bytes / 16);
+            blob_out(c, A.blob);
+            A.blob.blocks = 1; // the one that writes the tree
             c->step.grads_done = grads_with_tree(c, p);
             A.pred = c->pred;
             A.y = c->y;
