@@ -6,6 +6,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <math.h>
+
 #include <algorithm>
 #include <chrono>
 #include <memory>
@@ -303,7 +305,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->hist_seg_cost = 2048;
     c->record_nidx = false;
     c->nidx_valid = false;
-    c->defer_pred = true;
+    c->defer_pred = 1;
     c->write_nidx = false;
     c->pend_pred = false;
     c->is_id = nullptr;
@@ -814,6 +816,20 @@ extern "C" int evt_set_grads(evt_handle c, const float *grad) {
     });
 }
 
+// Whether the rows of a tree on every row are walked through it at the end, in row order and with the next gradients computed on the way (k_predict_tree), or
+// leave their leaf's number from its last level's lists, a scattered word each, for the gradient pass to look up.  The walk reads a line of a column
+// for 128 rows where any of them tests that feature: of 128 rows at most min(2^l, 128) nodes of level l.  It is one kernel for two and shorter
+// wherever the bins come from the caches, or fewer than about 88 bytes a row from memory; us a round, walk less than words: 60k to 1M rows of 20 to 100 features, depth 5 to 10, -1 to
+// -30; 4M x 20 -19 to -51; 10M x 100, depth 6 (27 bytes) -58, 8 (72) -131, 11 (99) +59; 4M x 100, depth 11 +11; 10M x 20, depth 11 -162;
+// 10M x 50 of two outputs, depth 11 (50) -121.
+static bool walk_pays(const evt_ctx *c) {
+    if ((size_t)c->N * c->F <= (size_t)256 << 20) return true; // what the last-level cache holds
+    const double feats = c->n_js_last;
+    double nodes = 0;
+    for (int l = 0; l + 1 < c->D; l++) nodes += std::min(1 << l, 128);
+    return feats * (1 - exp(-nodes / feats)) <= 88;
+}
+
 static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t cond, const uint32_t *js, int32_t n_js, const evt_params *p,
                      bool staged) {
     ARGCHK(js && p, "js and params must not be NULL");
@@ -887,8 +903,10 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
     // With every row in the tree the leaf of each row is recorded while growing and its value is added later, in row
     // order (fused into the next gradient pass): a scattered 4-byte write per row instead of a scattered read-modify-write.
     // (a quantile loss's leaf values do not exist before the tree is complete: always deferred)
-    const bool defer = p->update_pred && all_rows && (c->defer_pred || EVT_IS_QUANTILE(c->loss));
-    const bool fuse_pred = p->update_pred && all_rows && !defer;
+    // ... or, with the next gradients, by walking the tree
+    const bool walk = p->update_pred && all_rows && !small && !rec_nidx && (c->defer_pred == 2 || (c->defer_pred == 1 && walk_pays(c))) && grads_with_tree(c, p);
+    const bool defer = p->update_pred && all_rows && !walk && (c->defer_pred || EVT_IS_QUANTILE(c->loss));
+    const bool fuse_pred = p->update_pred && all_rows && !walk && !defer;
     c->write_nidx = rec_nidx || defer;
 
     c->step.hist_fused = !staged && scatter_can_build_hist(c, n_js); // the set-up below cuts the root's chunks by it
@@ -928,6 +946,7 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
     c->step.small = small;
     c->step.small_draw = draw;
     c->step.fuse_pred = fuse_pred;
+    c->step.walk = walk;
     c->step.blob_sent = false;
     c->step.grads_done = false;
     c->step.p = *p;
@@ -992,7 +1011,7 @@ static int tree_stage_partition(evt_ctx *c) {
     } else {
         // the tree's last kernel unless its leaves are still to be valued (quantile losses) or the rows outside the sample
         // are still to be predicted: the finished tree's transfer to the host rides along
-        const bool last_kernel = !EVT_IS_QUANTILE(c->loss) && !(c->step.p.update_pred && !c->step.all_rows);
+        const bool last_kernel = !EVT_IS_QUANTILE(c->loss) && !(c->step.p.update_pred && (!c->step.all_rows || c->step.walk));
         r = launch_final_fused(c, level, is_cur, c->step.fuse_pred, last_kernel);
     }
     prof_end(c);
@@ -1023,7 +1042,7 @@ static int tree_close(evt_ctx *c) {
         prof_end(c);
         if (r != EVT_OK) return r;
     }
-    if (p->update_pred && !all_rows && !c->step.small) {
+    if (p->update_pred && (!all_rows || c->step.walk) && !c->step.small) {
         // rows outside the sample are predicted too (src/fit.jl:37): walk the new tree for all rows
         prof_begin(c, EVT_K_PREDICT, 0);
         r = launch_predict_tree_cache(c, true, grads_with_tree(c, p)); // with the tree's transfer to the host in its last blocks
@@ -1805,7 +1824,8 @@ extern "C" int evt_set_option(evt_handle c, const char *name, int64_t value) {
     } else if (strcmp(name, "part_one_pass") == 0) {
         c->part_one_pass = value != 0;
     } else if (strcmp(name, "defer_pred") == 0) {
-        c->defer_pred = value != 0;
+        ARGCHK(value >= 0 && value <= 3, "defer_pred must be 0 (while the last level is partitioned), 1 (in row order), 2 or 3 (in row order, always or never by walking the tree)");
+        c->defer_pred = (int)value;
     } else if (strcmp(name, "hist_threads") == 0) {
         ARGCHK(value == 256 || value == 512 || value == 1024, "hist_threads must be 256, 512 or 1024");
         c->hist_threads = (int)value;

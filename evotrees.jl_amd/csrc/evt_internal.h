@@ -213,7 +213,7 @@ struct evt_ctx {
     int hist_in_scatter; // option: with 16-byte records and few chunks the partition's scatter pass builds the next level's histograms
     bool record_nidx;  // leaf finalisation also writes the node id of every sampled row
     bool nidx_valid;   // nidx holds the last tree's node ids
-    bool defer_pred;   // a tree grown on every row records leaf ids and leaves the addition to the next row-order pass
+    int defer_pred;    // a tree grown on every row records leaf ids and leaves the addition to the next row-order pass
     bool write_nidx;   // the tree being grown records the node id of every row it places
     bool grads_ahead;    // option: a tree with update_pred queues the next gradient update behind itself
     bool grads_ready;    // the gradients of the predictions as they stand were computed ahead: evt_update_grads has nothing to do
@@ -231,6 +231,7 @@ struct evt_ctx {
         int phase; // 0 no tree open, 1 histogram next, 2 split search next, 3 partition next, 4 levels done
         int level;
         bool all_rows, defer, fuse_pred;
+        bool walk;       // a tree on every row whose rows are walked through it at the end, as those of a sampled tree are (walk_pays)
         bool hist_fused; // levels below the root get their histograms from the scatter pass of the level above
         int small;       // one kernel per level: the blocks that share a feature's rows (small_tree_form)
         bool small_draw; // ... whose first draws the row mask

@@ -1,0 +1,41 @@
+"""Trees on every row whose rows are walked through them at the end give the predictions, gradients, node ids and following trees of those whose
+rows leave their leaf's number, and of those whose leaf values are added while the last level is partitioned, bit for bit."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import assert_tree_bits, make_data
+
+pytestmark = pytest.mark.gpu
+
+
+LOSSES = [("mse", False), ("mse", True), ("logloss", False), ("poisson", True), ("gamma", False), ("tweedie", False), ("mae", False), ("gaussian_mle", False),
+          ("logistic_mle", True)]
+
+
+@pytest.mark.parametrize("loss,weights,N,F,D,tt", [(*lw, *s) for lw in LOSSES for s in ((63, 5, 3, "binary"), (8_001, 20, 6, "oblivious"))] +
+                         [(*lw, *s) for lw in LOSSES if not lw[1] for s in ((600_007, 17, 5, "binary"), (2_100_001, 9, 4, "binary"))])
+def test_walk_equals_words(evt, loss, weights, N, F, D, tt):
+    x_bin, y, w, mu = make_data(N, N, F, 32, loss, weights)
+    js = np.arange(1, F + 1, dtype=np.uint32)
+    gp = evt.make_params(eta=0.3)
+    out = []
+    for defer in (2, 3, 0):
+        h = evt.Handle(N, F, 32, mu.shape[0], D, loss, tt)
+        h.set_option("small_tree", 0)
+        h.set_option("grads_ahead", 1)
+        h.set_option("defer_pred", defer)
+        h.set_xbin(x_bin)
+        h.set_target(y, w, mu)
+        rec = []
+        for _ in range(3):
+            h.update_grads()
+            t = h.grow_tree(js, gp)
+            rec.append((t, h.get_pred(), h.get_grads(), h.get_nidx()))
+        h.close()
+        out.append(rec)
+    for other in out[1:]:
+        for a, b in zip(out[0], other):
+            assert_tree_bits(a[0], b[0])
+            for u, v in zip(a[1:], b[1:]):
+                assert u.tobytes() == v.tobytes()
+    assert N < 100 or out[0][0][0].split.any()
