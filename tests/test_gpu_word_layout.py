@@ -30,5 +30,16 @@ def test_layouts_change_between_trees(evt, loss, weights, K, N, F):
     assert t_fx.split.any()
     for t in trees:
         assert_tree_bits(t, t_fx)
+    for first in (2, 3, 0):  # the words made by the root's kernel of a small tree, or beside the other form's set-up, of the device's own gradients
+        h.update_grads()
+        trees = []
+        for form in (first, 0, 3):
+            h.set_option("small_tree", form)
+            trees.append(h.grow_tree(js, gp))
+        own = h.get_grads()
+        o.set_quant(own, h.get_quant()[0])
+        t_fx, _ = o.grow_tree(own, np.arange(N, dtype=np.uint32), js, mode=1)
+        for t in trees:
+            assert_tree_bits(t, t_fx)
     h.close()
     o.close()
