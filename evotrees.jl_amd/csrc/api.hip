@@ -195,7 +195,7 @@ extern "C" int evt_destroy(evt_handle c) {
         void *lp[] = {L.hdr, L.act_node, L.cprefix, L.bnode, L.bstart, L.bprefix, L.cdesc};
         for (void *p : lp) dev_give(p);
     }
-    pinned_give(c->h_stage_base);
+    coherent_give(c->h_stage_base);
     for (auto &r : c->recs) {
         (void)hipEventDestroy(r.e0);
         (void)hipEventDestroy(r.e1);
@@ -420,10 +420,10 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
         c->sbest = sb;
         ALLOC(c->scan_count, (size_t)c->maxlvl * EVT_SCAN_COUNT_STEP);
     }
-    // pinned staging: tree read-back + small per-tree uploads
+    // pinned staging: tree read-back + small per-tree uploads; coherent: wait_for_tree reads it while the kernel that fills it runs
     c->h_stage_bytes = c->blob_bytes + (size_t)c->F * 4 + (size_t)c->RS * 2 + 1024;
     c->h_stage_bytes = (c->h_stage_bytes + 255) / 256 * 256;
-    c->h_stage_base = c->h_stage_dev_base = static_cast<uint8_t *>(pinned_take(2 * c->h_stage_bytes + 128));
+    c->h_stage_base = c->h_stage_dev_base = static_cast<uint8_t *>(coherent_take(2 * c->h_stage_bytes + 128));
     if (!c->h_stage_base) {
         evt_destroy(c);
         return EVT_ERR_NOMEM;

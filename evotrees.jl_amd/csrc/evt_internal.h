@@ -343,7 +343,8 @@ __device__ __forceinline__ unsigned long long evt_load_gq(const unsigned long lo
 // waits for.  An event recorded behind the kernel put a packet into the queue that the next tree's first kernel waited for: 5.5 us between two trees,
 // where kernels of one tree follow each other without a gap.
 // Order: the words go out as system-scope atomic stores, past the device's caches; each thread waits for its own to arrive; the block that
-// counts itself last stores the flag.
+// counts itself last stores the flag.  The kernel has not ended when the host reads them, so that dst and flag must lie in coherent
+// (fine-grained) memory, coherent_take's: in other pinned memory only the kernel's end makes stores visible, in no order before it.
 struct BlobOut {
     const uint4 *src;
     uint4 *dst;

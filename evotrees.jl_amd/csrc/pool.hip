@@ -11,9 +11,10 @@ struct Block {
     size_t size;
     int device;
 };
-std::unordered_map<void *, Block> g_out[2];                            // blocks in use: device, pinned
-std::multimap<std::pair<int, size_t>, void *> g_idle[2];               // by (device, size); pinned blocks under device 0
-std::map<int, size_t> g_kept[2];                                       // idle bytes by device
+enum { DEVICE, PINNED, COHERENT, KINDS };
+std::unordered_map<void *, Block> g_out[KINDS];                        // blocks in use
+std::multimap<std::pair<int, size_t>, void *> g_idle[KINDS];           // by (device, size); pinned blocks under device 0
+std::map<int, size_t> g_kept[KINDS];                                   // idle bytes by device
 std::map<int, std::vector<hipStream_t>> g_streams[2];                  // idle ones by device, the last used at the end: blocking, non-blocking
 const size_t STREAMS_KEPT = 16; // per device and kind
 
@@ -30,7 +31,7 @@ int current_device() {
     return hipGetDevice(&d) == hipSuccess ? d : 0;
 }
 void release(int kind, void *p) {
-    if (kind == 0) (void)hipFree(p);
+    if (kind == DEVICE) (void)hipFree(p);
     else (void)hipHostFree(p);
 }
 void trim(int kind) {
@@ -44,7 +45,7 @@ void trim(int kind) {
     for (void *p : idle) release(kind, p);
 }
 void *take(int kind, size_t bytes) {
-    const int dev = kind == 0 ? current_device() : 0;
+    const int dev = kind == DEVICE ? current_device() : 0;
     const size_t n = size_class(bytes ? bytes : 1);
     {
         std::lock_guard<std::mutex> lk(g_mu);
@@ -60,20 +61,22 @@ void *take(int kind, size_t bytes) {
     void *p = nullptr;
     hipError_t e = hipSuccess;
     for (int attempt = 0; attempt < 2; attempt++) {
-        e = kind == 0 ? hipMalloc(&p, n) : hipHostMalloc(&p, n, hipHostMallocPortable);
+        e = kind == DEVICE ? hipMalloc(&p, n) : hipHostMalloc(&p, n, hipHostMallocPortable | (kind == COHERENT ? hipHostMallocCoherent : 0u));
         if (e == hipSuccess) break;
         (void)hipGetLastError();
-        trim(kind); // idle blocks of other sizes make room
+        // idle blocks of other sizes make room
+        if (kind == DEVICE) trim(DEVICE);
+        else trim(PINNED), trim(COHERENT);
     }
     if (e != hipSuccess) {
-        evt_set_error("%s of %zu bytes failed: %s", kind == 0 ? "hipMalloc" : "hipHostMalloc", n, hipGetErrorString(e));
+        evt_set_error("%s of %zu bytes failed: %s", kind == DEVICE ? "hipMalloc" : "hipHostMalloc", n, hipGetErrorString(e));
         return nullptr;
     }
-    if (kind == 1) {
+    if (kind != DEVICE) {
         void *d = nullptr;
         if (hipHostGetDevicePointer(&d, p, 0) != hipSuccess || d != p) {
             evt_set_error("pinned memory is not addressable from the device");
-            release(1, p);
+            release(kind, p);
             return nullptr;
         }
     }
@@ -89,7 +92,7 @@ void give(int kind, void *p) {
         if (it != g_out[kind].end()) {
             const Block b = it->second;
             g_out[kind].erase(it);
-            if (b.size <= POOL_BLOCK_KEPT && g_kept[kind][b.device] + b.size <= (kind == 0 ? POOL_DEVICE_KEPT : POOL_PINNED_KEPT)) {
+            if (b.size <= POOL_BLOCK_KEPT && g_kept[kind][b.device] + b.size <= (kind == DEVICE ? POOL_DEVICE_KEPT : POOL_PINNED_KEPT)) {
                 g_idle[kind].insert({{b.device, b.size}, p});
                 g_kept[kind][b.device] += b.size;
                 return;
@@ -101,10 +104,12 @@ void give(int kind, void *p) {
 
 } // namespace
 
-void *dev_take(size_t bytes) { return take(0, bytes); }
-void dev_give(void *p) { give(0, p); }
-void *pinned_take(size_t bytes) { return take(1, bytes); }
-void pinned_give(void *p) { give(1, p); }
+void *dev_take(size_t bytes) { return take(DEVICE, bytes); }
+void dev_give(void *p) { give(DEVICE, p); }
+void *pinned_take(size_t bytes) { return take(PINNED, bytes); }
+void pinned_give(void *p) { give(PINNED, p); }
+void *coherent_take(size_t bytes) { return take(COHERENT, bytes); }
+void coherent_give(void *p) { give(COHERENT, p); }
 
 hipError_t stream_take(hipStream_t *s, bool non_blocking) {
     const int dev = current_device();
@@ -134,8 +139,7 @@ void stream_give(hipStream_t s, bool non_blocking, int dev) {
 extern "C" int evt_trim(void) {
     return guarded([&]() -> int {
     models_trim();
-    trim(0);
-    trim(1);
+    for (int k = 0; k < KINDS; k++) trim(k);
     std::vector<hipStream_t> idle;
     {
         std::lock_guard<std::mutex> lk(g_mu);
