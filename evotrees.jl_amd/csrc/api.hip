@@ -1824,8 +1824,7 @@ extern "C" int evt_set_option(evt_handle c, const char *name, int64_t value) {
     } else if (strcmp(name, "part_one_pass") == 0) {
         c->part_one_pass = value != 0;
     } else if (strcmp(name, "defer_pred") == 0) {
-        ARGCHK(value >= 0 && value <= 3, "defer_pred must be 0 (while the last level is partitioned), 1 (in row order), 2 or 3 (in row order, always or never by walking the tree)");
-        c->defer_pred = (int)value;
+        c->defer_pred = value == 2 || value == 3 ? (int)value : value != 0; // 2, 3: always or never by walking the tree
     } else if (strcmp(name, "hist_threads") == 0) {
         ARGCHK(value == 256 || value == 512 || value == 1024, "hist_threads must be 256, 512 or 1024");
         c->hist_threads = (int)value;

@@ -411,7 +411,7 @@ int evt_reset_profile(evt_handle h);
  * 0, default: evt_get_nidx derives it afterwards by walking the finished tree); "defer_pred" (1, default:
  * leaf values of a tree grown on every row are added in row order by the next pass over the rows, or, with "grads_ahead", by a walk of
  * all rows through the tree that computes the next gradients too, where that is estimated to be faster; 2, 3: the walk always or never;
- * 0: they are added while the tree's last level is partitioned; results do not depend on it); "grads_ahead"
+ * any other value but 0: as 1; 0: they are added while the tree's last level is partitioned; results do not depend on it); "grads_ahead"
  * (1: a tree grown with update_pred queues the next evt_update_grads behind itself, so the device computes it
  * while the host collects the tree, and that next call returns at once; meant for bagging_size 1 - with more
  * trees per round only the last one's work is used; 0, default; results do not depend on it); "scan_fused"

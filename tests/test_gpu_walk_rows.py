@@ -39,3 +39,21 @@ def test_walk_equals_words(evt, loss, weights, N, F, D, tt):
             for u, v in zip(a[1:], b[1:]):
                 assert u.tobytes() == v.tobytes()
     assert N < 100 or out[0][0][0].split.any()
+
+
+def test_any_integer_means_on_or_off(evt):
+    N, F = 4_001, 6
+    x_bin, y, w, mu = make_data(N, N, F, 32, "mse", False)
+    h = evt.Handle(N, F, 32, 1, 4, "mse")
+    h.set_option("small_tree", 0)
+    h.set_xbin(x_bin)
+    first = None
+    for value in (1, 4, 255, -1, -(1 << 40), 1 << 40, 0):
+        h.set_option("defer_pred", value)
+        h.set_target(y, w, mu)
+        h.update_grads()
+        got = (h.grow_tree(np.arange(1, F + 1, dtype=np.uint32), evt.make_params(eta=0.3)), h.get_pred())
+        first = first or got
+        assert_tree_bits(got[0], first[0])
+        assert got[1].tobytes() == first[1].tobytes()
+    h.close()
