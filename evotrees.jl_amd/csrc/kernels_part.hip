@@ -917,27 +917,36 @@ __device__ __forceinline__ unsigned mask_flags(uint8_t *mask, uint8_t cond, int6
 // The sample's rows, and the tree's set-up, in one kernel: a block flags its 8192 rows, claims as many places of the
 // list by one addition and writes their ids there.  A block's rows stay in order, the blocks follow each other in the order of their
 // claims, which nothing depends on (k_part_move's chunks do the same).  The block that claims last knows the number of rows and writes the first
-// level's tables; block 0 prepares the rest of the tree, blocks behind the sample's quantise.  Bound by its chain (draw, count, claim, stores) and the
+// level's tables; block 0 prepares the rest of the tree.  Blocks behind the sample's help it clear the root's slice where that has more words than the
+// sample's blocks write in a few stores each (30k rows x 120 features of 255 bins and 15 channels, 459k words: 6.8 us; 18.3 by the 4 blocks of the sample), those behind them quantise.  Bound by its chain (draw, count, claim, stores) and the
 // quantisation beside it: 1M rows 7.9 us with one word a row, 10.0 with two (a block's rows by 1024 threads: 9.1, 12.4: quantisation gets its blocks later).  In two kernels, a
 // count and a scatter that added the counts up, 5.9 + 5.1 and 8.9 + 4.7; with a scan between them, from 2M rows on,
 // 100 rounds of 6M x 20 46.2 ms for 45.5, of 10M 67.4 for 67.7.
 template <bool DRAW>
 __global__ __launch_bounds__(256) void k_mask_sample(uint8_t *mask, uint8_t cond, int64_t N, unsigned long long seed, uint32_t *is_out,
-                                                     unsigned long long *claims, BeginArgs B, QuantArgs Q, int blocks) {
+                                                     unsigned long long *claims, BeginArgs B, QuantArgs Q, int blocks, int clear) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if ((int)blockIdx.x > blocks) { // as k_tree_begin
-        quant_rows(Q, (int)blockIdx.x - blocks - 1, (int)gridDim.x - blocks - 1);
+    const int own_block = (int)blockIdx.x - 1, set_up = blocks + clear;
+    if (own_block >= set_up) { // as k_tree_begin
+        quant_rows(Q, own_block - set_up, (int)gridDim.x - 1 - set_up);
         return;
     }
-    if (blockIdx.x == 0) {
+    if (own_block < 0) {
         tree_begin_arrays(B);
+        return;
+    }
+    auto clear_root = [&]() {
+        for (int64_t i = (int64_t)own_block * 256 + tid; i < B.root_words; i += (int64_t)set_up * 256) B.hist[i] = 0;
+    };
+    if (own_block >= blocks) {
+        clear_root();
         return;
     }
     static_assert(EVT_SAMPLE_ROWS == 256 * 32, "32 rows to a thread");
     __shared__ uint16_t s_row[EVT_SAMPLE_ROWS]; // the rows kept, from the block's first
     __shared__ int s_cnt[4];
     __shared__ unsigned long long s_claim;
-    const int64_t b0 = ((int64_t)blockIdx.x - 1) * EVT_SAMPLE_ROWS;
+    const int64_t b0 = (int64_t)own_block * EVT_SAMPLE_ROWS;
     uint32_t flags = 0;
 #pragma unroll
     for (int j = 0; j < 4; j++) flags |= mask_flags<DRAW>(mask, cond, N, b0 + tid * 32 + 8 * j, seed) << (8 * j);
@@ -960,7 +969,7 @@ __global__ __launch_bounds__(256) void k_mask_sample(uint8_t *mask, uint8_t cond
     // rows claimed so far, blocks that have claimed in the upper half
     if (tid == 0) s_claim = atomicAdd(claims, (unsigned long long)total | (1ull << 40));
     for (uint32_t f = flags; f; f &= f - 1) s_row[at++] = (uint16_t)(tid * 32 + __ffs(f) - 1);
-    for (int64_t i = b0 / EVT_SAMPLE_ROWS * 256 + tid; i < B.root_words; i += (int64_t)blocks * 256) B.hist[i] = 0;
+    clear_root();
     __syncthreads();
     const unsigned long long claim = s_claim;
     const int64_t base = (int64_t)(claim & ((1ull << 40) - 1));
@@ -1045,9 +1054,10 @@ int launch_compact_mask(evt_ctx *c, uint8_t cond, bool draw, unsigned long long 
         quant_args(c, Q);
         quant = quant_blocks(c, 256);
     }
-    const dim3 grid((unsigned)blocks + 1 + quant);
-    if (draw) hipLaunchKernelGGL(k_mask_sample<true>, grid, dim3(256), 0, c->stream, c->mask, cond, c->N, seed, c->is_a, c->sample_claims, B, Q, (int)blocks);
-    else hipLaunchKernelGGL(k_mask_sample<false>, grid, dim3(256), 0, c->stream, c->mask, cond, c->N, 0ull, c->is_a, c->sample_claims, B, Q, (int)blocks);
+    const int64_t clear = std::max<int64_t>(0, std::min<int64_t>(256, B.root_words / 4096) - blocks); // 16 words a thread, up to a block to a compute unit
+    const dim3 grid((unsigned)(1 + blocks + clear) + quant);
+    if (draw) hipLaunchKernelGGL(k_mask_sample<true>, grid, dim3(256), 0, c->stream, c->mask, cond, c->N, seed, c->is_a, c->sample_claims, B, Q, (int)blocks, (int)clear);
+    else hipLaunchKernelGGL(k_mask_sample<false>, grid, dim3(256), 0, c->stream, c->mask, cond, c->N, 0ull, c->is_a, c->sample_claims, B, Q, (int)blocks, (int)clear);
     HIPCHK(hipGetLastError());
     if (quant) quant_taken(c);
     c->js_staged = false;

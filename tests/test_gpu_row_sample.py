@@ -38,3 +38,26 @@ def test_sampled_rows(evt, N, loss):
         assert not got[mask > 127].any() and np.array_equal(got[rows], np.asarray(nidx)[rows])
     h.close()
     o.close()
+
+
+@pytest.mark.parametrize("N", [1_003, 8_193, 30_011])
+def test_few_rows_of_a_large_root_slice(evt, N):
+    """Blocks of their own clear the root's slice: 306,000 words, which the trees before have filled."""
+    F, B, K = 80, 255, 7
+    x_bin, y, w, mu = make_data(N, N, F, B, "mlogloss", True, K=K)
+    h, o, op, gp, pred0, grad = setup_pair(evt, "mlogloss", x_bin, y, w, mu, B, 2)
+    orc.update_grads(op, pred0, y, grad)
+    h.set_option("small_tree", 0)
+    h.set_grads(grad)
+    js = np.arange(1, F + 1, dtype=np.uint32)
+    gp.update_pred = 0
+    o.set_quant(grad, h.get_quant()[0])
+    rng = np.random.default_rng(N)
+    for cond in (127, 255, 20, 200):
+        mask = rng.integers(0, 256, N).astype(np.uint8)
+        t = h.grow_tree(js, gp, mask=mask, cond=cond)
+        t_fx, _ = o.grow_tree(grad, np.flatnonzero(mask <= cond).astype(np.uint32), js, mode=1)
+        assert_tree_bits(t, t_fx)
+        assert t.split.any()
+    h.close()
+    o.close()
