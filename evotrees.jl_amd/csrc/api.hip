@@ -225,6 +225,9 @@ static hipError_t upload_alphas(evt_ctx *c) {
     return e;
 }
 
+// LDS channels: rows of the gradient matrix that need their own accumulator
+static int n_channels(const evt_ctx *c, bool unit_w) { return (EVT_TWO_CHAN(c->loss, c->K) ? 1 : c->NK - 1) + (unit_w ? 0 : 1); }
+
 extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K, int32_t max_depth, int32_t loss, int32_t tree_type,
                           evt_handle *out) {
     return guarded([&]() -> int {
@@ -269,7 +272,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->unit_w = true;
     c->have_xbin = c->have_target = c->have_grads = false;
     c->planes = nullptr; c->plane_words = 0; c->planes_ready = false; c->use_planes = 1;
-    c->xcm = nullptr; c->xrm = nullptr; c->y = nullptr; c->pred = nullptr; c->grad = nullptr; c->gq = nullptr; c->gq_rows = false;
+    c->xcm = nullptr; c->xrm = nullptr; c->y = nullptr; c->pred = nullptr; c->grad = nullptr; c->gq = nullptr; c->gq_words = 0; c->gq_rows = false;
     c->is_a = c->is_b = nullptr; c->nidx = nullptr; c->mask = nullptr; c->flagw = nullptr; c->sample_claims = nullptr; c->blob_arrived = nullptr; c->slot_ev[0] = c->slot_ev[1] = false; c->chunk_nleft = nullptr; c->chunk_lpre = nullptr; c->cursor = nullptr;
     c->hist = nullptr; c->seg_start = c->seg_len = nullptr; c->status = nullptr; c->node_sum = nullptr;
     memset(&c->tree, 0, sizeof(c->tree));
@@ -348,7 +351,8 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     ALLOC(c->y, N * c->T);
     ALLOC(c->pred, (size_t)N * K);
     ALLOC(c->grad, (size_t)N * c->NK);
-    ALLOC(c->gq, EVT_GQ_WORDS(N, c->NK));
+    c->gq_words = EVT_GQ_WORDS(N, n_channels(c, true)); // evt_set_target takes what weights need beside
+    ALLOC(c->gq, c->gq_words);
     ALLOC(c->is_a, N);
     ALLOC(c->is_b, N);
     ALLOC(c->is_id, N);
@@ -603,7 +607,6 @@ extern "C" int evt_binarize_f64(evt_handle c, const double *x_colmajor, const do
 }
 
 static void set_channels(evt_ctx *c) {
-    // LDS channels (rows of the gradient matrix that need their own accumulator)
     int na = 0;
     if (EVT_TWO_CHAN(c->loss, c->K)) {
         c->chan_k[na++] = 0;                   // g ; h is derived (mse: 2w, mae: 0)
@@ -638,6 +641,15 @@ extern "C" int evt_set_target(evt_handle c, const float *y, const float *w, cons
     c->grads_ready = false;
     c->unit_w = (w == nullptr);
     set_channels(c);
+    const size_t words = EVT_GQ_WORDS(c->N, c->NA);
+    if (words > c->gq_words) { // no target, no tree: nobody reads the words that were there
+        HIPCHK(hipStreamSynchronize(c->stream));
+        dev_give(c->gq);
+        c->gq_words = 0;
+        c->gq = static_cast<unsigned long long *>(dev_take(words * sizeof(*c->gq)));
+        if (!c->gq) return EVT_ERR_NOMEM;
+        c->gq_words = words;
+    }
     HIPCHK(hipMemcpyAsync(c->y, y, sizeof(float) * c->N * c->T, hipMemcpyDefault, c->stream));
     if (c->loss == EVT_LOSS_MLOGLOSS) {
         int r = launch_validate_classes(c);

@@ -122,6 +122,7 @@ struct evt_ctx {
     float *pred;    // K x N
     float *grad;    // NK x N
     unsigned long long *gq; // fixed-point words of the rows: NA planes of N, or (gq_rows) EVT_GQ_STRIDE(NA) words a row
+    size_t gq_words;        // of the allocation: the channels of the targets set so far, without weights or with them
     bool gq_rows;           // which: the kernels of small trees walk all rows and read planes, the others gather rows
     uint32_t *is_a, *is_b;
     uint32_t *is_id;   // [N] 0..N-1, written once: the root's row list when every row is in the tree
@@ -322,8 +323,8 @@ static int guarded(F &&f) {
 #define EVT_NODE_NUMERIC (1u << 25)
 // Words from one row to the next where a row's words lie side by side: whole 16 bytes.
 #define EVT_GQ_STRIDE(na) (((na) + 1) & ~1)
-// ... and words of the allocation for either layout: a histogram layer of four channels may read past the last row's
-#define EVT_GQ_WORDS(n, nk) ((size_t)(n) * ((nk) + 1) + EVT_HIST_GROUP)
+// ... and words of the allocation for either layout (one channel alone takes half of its): a histogram layer of four channels may read past the last row's
+#define EVT_GQ_WORDS(n, na) ((size_t)(n) * ((na) > 1 ? EVT_GQ_STRIDE(na) : 1) + EVT_HIST_GROUP)
 #ifdef __HIPCC__
 __host__ __device__ __forceinline__ uint32_t evt_pack_node(int feat, int cond_bin, bool numeric) {
     return (uint32_t)feat | ((uint32_t)cond_bin << 16) | EVT_NODE_SPLIT | (numeric ? EVT_NODE_NUMERIC : 0u);

@@ -606,3 +606,50 @@ def test_large_buffers_are_as_large_as_asked(evt):
         evt._lib.trim()
     print(used)
     assert used[1] < 1.01 * used[0] + (64 << 20)
+
+
+@pytest.mark.parametrize("loss,K,words", [("mse", 1, (1, 2)), ("logloss", 1, (2, 4)), ("mlogloss", 3, (6, 8))])
+def test_words_take_the_channels_there_are(evt, loss, K, words):
+    """The fixed-point words of a row: as many as the target's channels fill, in whole 16 bytes where there are several; those of weights from a target with weights on."""
+    evt._lib.trim()
+    N, F = 1 << 24, 1
+    # bins, records, target, predictions, gradients, row lists, node ids, mask, the partition's ballots
+    row = F + 16 + 4 + 4 * K + 4 * (2 * K + 1) + 3 * 4 + 4 + 1 + 0.125
+    y = (np.arange(N) % 2 + (1 if K > 1 else 0)).astype(np.float32)
+    free = _free_bytes()
+    h = evt.Handle(N, F, 16, K, 1, loss)
+    used = []
+    for w in (None, y + 1):
+        h.set_target(y, w, np.zeros(K, np.float32))
+        evt._lib.trim()  # the words of fewer channels, kept for another handle
+        used.append((free - _free_bytes()) / N - row)
+    h.close()
+    evt._lib.trim()
+    print(used)
+    for got, n in zip(used, words):
+        assert 8 * n - 1 < got < 8 * n + 4  # a bit of 64 MB for the rest: tables, staging, what the runtime takes
+
+
+@pytest.mark.parametrize("loss,K", [("mse", 1), ("gaussian_mle", 2), ("mlogloss", 3)])
+def test_targets_with_and_without_weights_on_one_handle(evt, loss, K):
+    N, F = 5_003, 9
+    js = np.arange(1, F + 1, dtype=np.uint32)
+    x_bin, y, w, mu = make_data(11, N, F, 32, loss, True, K=K)
+    one = evt.Handle(N, F, 32, K, 4, loss)
+    one.set_xbin(x_bin)
+    for weights, form in ((None, 0), (w, 0), (None, 2), (w, 3), (w, 0), (None, 0)):
+        fresh = evt.Handle(N, F, 32, K, 4, loss)
+        fresh.set_xbin(x_bin)
+        got = []
+        for h in (one, fresh):
+            h.set_option("small_tree", form)
+            h.set_target(y, weights, mu, np.tile(mu, (N, 1)) * 0.5 if form == 0 else None)
+            for _ in range(2):
+                h.update_grads()
+                t = h.grow_tree(js, evt.make_params(eta=0.3))
+            got.append((t, h.get_pred()))
+        fresh.close()
+        assert got[0][0].split.any()
+        assert_tree_bits(got[0][0], got[1][0])
+        assert got[0][1].tobytes() == got[1][1].tobytes()
+    one.close()
