@@ -1,12 +1,11 @@
 // C ABI of libevotrees_hip.so: handle lifecycle, uploads, the per-tree level loop, read-back.
 #include "grad_math.h"
 #include "upload.h"
+#include "walk_rule.h"
 
 #include <stdarg.h>
 #include <stdio.h>
 #include <string.h>
-
-#include <math.h>
 
 #include <algorithm>
 #include <chrono>
@@ -828,20 +827,6 @@ extern "C" int evt_set_grads(evt_handle c, const float *grad) {
     });
 }
 
-// Whether the rows of a tree on every row are walked through it at the end, in row order and with the next gradients computed on the way (k_predict_tree), or
-// leave their leaf's number from its last level's lists, a scattered word each, for the gradient pass to look up.  The walk reads a line of a column
-// for 128 rows where any of them tests that feature: of 128 rows at most min(2^l, 128) nodes of level l.  It is one kernel for two and shorter
-// wherever the bins come from the caches, or fewer than about 88 bytes a row from memory; us a round, walk less than words: 60k to 1M rows of 20 to 100 features, depth 5 to 10, -1 to
-// -30; 4M x 20 -19 to -51; 10M x 100, depth 6 (27 bytes) -58, 8 (72) -131, 11 (99) +59; 4M x 100, depth 11 +11; 10M x 20, depth 11 -162;
-// 10M x 50 of two outputs, depth 11 (50) -121.
-static bool walk_pays(const evt_ctx *c) {
-    if ((size_t)c->N * c->F <= (size_t)256 << 20) return true; // what the last-level cache holds
-    const double feats = c->n_js_last;
-    double nodes = 0;
-    for (int l = 0; l + 1 < c->D; l++) nodes += std::min(1 << l, 128);
-    return feats * (1 - exp(-nodes / feats)) <= 88;
-}
-
 static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t cond, const uint32_t *js, int32_t n_js, const evt_params *p,
                      bool staged) {
     ARGCHK(js && p, "js and params must not be NULL");
@@ -916,7 +901,7 @@ static int tree_open(evt_ctx *c, const uint8_t *mask, bool mask_staged, uint8_t 
     // order (fused into the next gradient pass): a scattered 4-byte write per row instead of a scattered read-modify-write.
     // (a quantile loss's leaf values do not exist before the tree is complete: always deferred)
     // ... or, with the next gradients, by walking the tree
-    const bool walk = p->update_pred && all_rows && !small && !rec_nidx && (c->defer_pred == 2 || (c->defer_pred == 1 && walk_pays(c))) && grads_with_tree(c, p);
+    const bool walk = p->update_pred && all_rows && !small && !rec_nidx && (c->defer_pred == 2 || (c->defer_pred == 1 && walk_pays(c->N, c->F, c->n_js_last, c->D, c->tree_type == EVT_TREE_OBLIVIOUS))) && grads_with_tree(c, p);
     const bool defer = p->update_pred && all_rows && !walk && (c->defer_pred || EVT_IS_QUANTILE(c->loss));
     const bool fuse_pred = p->update_pred && all_rows && !walk && !defer;
     c->write_nidx = rec_nidx || defer;
