@@ -45,6 +45,7 @@ struct HistArgs {
     int na_all; // accumulator channels of the loss: more than EVT_MAX_NA go EVT_HIST_GROUP to a block layer (blockIdx.z)
     int pack;   // the channel groups' first channel carries the row count (as a 64-bit word, k_quantize)
     int gq_stride; // words from row to row of gq
+    int whole;  // k_hist_build16: blocks take shares of whole iterations (choose_hist16)
     int tab;    // entries of bprefix, bstart and bnode that may be read
 };
 
@@ -370,7 +371,8 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
     const int step = nwaves * RPW;
     int64_t T = (total + gridDim.x - 1) / gridDim.x;
     if (T < A.min_rows) T = A.min_rows;
-    T = ((T + step - 1) / step) * step; // not whole iterations: 1024 rows at a time left a fifth of the blocks without any at 1600 rows a block
+    const int share = A.whole ? U * step : step;
+    T = ((T + share - 1) / share) * share;
     int64_t start = (int64_t)blockIdx.x * T;
     if (start >= total) return;
     int64_t end = start + T < total ? start + T : total;
@@ -467,7 +469,7 @@ __global__ __launch_bounds__(1024) void k_hist_build16(HistArgs A) {
             // address is one addition whose operand comes by way of the row broadcast; FAR (records past 4 GB): the id, multiplied by every lane
             // into 64 bits.  With the broadcasts' defaults gone a group of two features costs 8 vector instructions where it took 11 and a
             // multiplication at a quarter of their rate: 500k rows x 50 of four channels, 23.4 -> 19.0 us a level, 1M x 100 sampled by half 14.5 -> 13.4,
-            // 800k x 28 of 128 bins' root 28.1 -> 25.3, 10M x 100's 282 -> 275 (with shares of whole steps instead of whole iterations, below).
+            // 800k x 28 of 128 bins' root 28.1 -> 25.3, 10M x 100's 282 -> 275 (with shares of steps instead of whole iterations, which choose_hist16 tells apart).
             auto handed = [&](uint32_t id) { return FAR ? id : id * rs32; };
             auto piece = [&](uint32_t h) { return load_piece<PB, NT>(FAR ? A.xrm + ((size_t)h * rs32 + pofs) : A.xrm + (h + pofs)); };
             {
@@ -697,10 +699,14 @@ static int launch_hist_t(evt_ctx *c, const HistArgs &A, dim3 grid, int threads, 
 // us per launch, whole records and 256 spans -> chosen: mse 100 features, 35k rows a launch 15.8 -> 10.4, 300k 33.5 -> 20.6, 600k 41.3 -> 29.7,
 // 2.2M 83 (whole records stay); logloss 28 features of 128 bins, 470k rows 30.2 -> 25.0; gaussian_mle 50 features, 140k rows
 // 32.8 -> 21.5; 7 classes, 30 features, 80k rows 36.4 -> 26.
+// A span's share of the rows is rounded up to whole iterations (U steps), so that fewer spans are flushed, where the estimate has the flush above two thirds of the rows'
+// part, elsewhere to steps, so that every block has rows.  us a round, steps | iterations: 30k rows of 120 features, 255 bins and 15 channels sampled by half 426 | 398,
+// 1M x 28 of 128 bins, three channels, depth 8 250 | 247, 400k x 40 of 255 bins 245.4 | 242.8; 500k x 50 of four channels 231.2 | 233.7, 2M x 50 of 128 bins and three channels 401 | 405.
 struct Hist16Shape {
     int tw, pb, pu, ntiles;
     size_t lds;
     unsigned spans;
+    bool whole;
 };
 
 static bool choose_hist16(const evt_ctx *c, int level, int na, int layers, Hist16Shape *best) {
@@ -737,9 +743,10 @@ static bool choose_hist16(const evt_ctx *c, int level, int na, int layers, Hist1
         int most = c->hist_blocks / (s.ntiles * layers);
         if (most < 16) most = c->hist_blocks < 16 ? c->hist_blocks : 16;
         for (int n = most; n >= 1 && (n == most || n >= 16) && 4 * n >= most; n >>= 1) {
-            const double us = 8 + 4.9e-6 * span_atomics * n + rows * per_row * 256 / ((double)n * s.ntiles);
+            const double flush = 4.9e-6 * span_atomics * n, stream = rows * per_row * 256 / ((double)n * s.ntiles), us = 8 + flush + stream;
             if (!found || us < least) {
                 s.spans = (unsigned)n;
+                s.whole = 1.5 * flush > stream;
                 *best = s;
                 least = us;
                 found = true;
@@ -786,6 +793,7 @@ int launch_hist_build(evt_ctx *c, int level, const uint32_t *is_cur) {
     A.gq_stride = EVT_GQ_STRIDE(c->NA);
     A.na_all = c->NA;
     A.pack = c->unit_w ? 1 : 0;
+    A.whole = 0;
     // feature tiling so that one block's LDS histogram stays within budget
     const size_t budget = 64 * 1024;
     const size_t per_slot = (size_t)na * c->B * 8;
@@ -808,6 +816,7 @@ int launch_hist_build(evt_ctx *c, int level, const uint32_t *is_cur) {
     const size_t lds16 = s16.lds;
     if (use16) {
         A.TW = s16.tw;
+        A.whole = s16.whole;
         A.NSL = s16.tw / s16.pb;
         A.lay_sh = __builtin_ctz((unsigned)c->PBL);
         A.lay_pu = c->PU;

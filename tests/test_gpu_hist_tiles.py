@@ -48,3 +48,29 @@ def test_every_tile_width_gives_the_same_tree(evt, loss, weights, K, N, F, B, D,
     assert t_fx.split.any()
     h.close()
     o.close()
+
+
+@pytest.mark.parametrize("loss,weights,K,F,B", [("mse", False, None, 20, 16), ("mse", False, None, 100, 255), ("gaussian_mle", True, None, 33, 64)])
+def test_shares_of_steps_and_of_iterations(evt, loss, weights, K, F, B):
+    """Rows around the edges of a block's share, rounded up to steps (few spans, little to flush) and to whole iterations (many): the histograms
+    of the generic kernel."""
+    for N in (63, 64, 65, 1023, 1024, 1025, 4097, 31 * 1024 + 1, 131_073):
+        x_bin, y, w, mu = make_data(N, N, F, B, loss, weights, K=K)
+        h = evt.Handle(N, F, B, mu.shape[0], 3, loss)
+        h.set_option("small_tree", 0)
+        h.set_option("hist_in_scatter", 0)
+        h.set_xbin(x_bin)
+        h.set_target(y, w, mu)
+        h.update_grads()
+        gp = evt.make_params()
+        gp.update_pred = 0
+        js = np.arange(1, F + 1, dtype=np.uint32)
+        got = []
+        for variant, blocks in ((1, 256), (0, 256), (0, 31), (0, 2)):
+            h.set_option("hist_variant", variant)
+            h.set_option("hist_blocks", blocks)
+            got.append((h.grow_tree(js, gp), h.get_hist()))
+        h.close()
+        for t, hist in got[1:]:
+            assert_tree_bits(t, got[0][0])
+            assert hist.tobytes() == got[0][1].tobytes()
