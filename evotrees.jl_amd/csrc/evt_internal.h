@@ -329,15 +329,10 @@ static int guarded(F &&f) {
 __host__ __device__ __forceinline__ uint32_t evt_pack_node(int feat, int cond_bin, bool numeric) {
     return (uint32_t)feat | ((uint32_t)cond_bin << 16) | EVT_NODE_SPLIT | (numeric ? EVT_NODE_NUMERIC : 0u);
 }
-// The fixed-point word of channel a for one row.  The channel that shares its word with the row count holds 30 bits:
-// it is staged as a 32-bit word (half the plane to gather from) and widened here to (q << 16) + 1.
-template <bool PACK>
-__device__ __forceinline__ unsigned long long evt_load_gq(const unsigned long long *__restrict__ gq, int64_t N, int a, uint32_t id) {
-    if (PACK && a == 0) {
-        const long long q = (long long)reinterpret_cast<const int32_t *>(gq)[id];
-        return ((unsigned long long)q << EVT_PACK_CNT_BITS) + 1ull;
-    }
-    return gq[(size_t)a * N + id];
+// The word of a row whose one channel shares it with the row count, staged as 32 bits (30 of gradient, half the plane to gather from) and widened here to (q << 16) + 1.
+__device__ __forceinline__ unsigned long long evt_load_narrow(const unsigned long long *__restrict__ gq, uint32_t id) {
+    const long long q = (long long)reinterpret_cast<const int32_t *>(gq)[id];
+    return ((unsigned long long)q << EVT_PACK_CNT_BITS) + 1ull;
 }
 
 // The finished tree's arrays on their way to the host's pinned buffer, in `blocks` blocks of the tree's last kernel, and behind them the word the host
@@ -376,7 +371,7 @@ __device__ __forceinline__ void blob_send(const BlobOut &O, int block) {
 template <int NA, bool PACK>
 __device__ __forceinline__ void evt_load_words(const unsigned long long *__restrict__ gq, int stride, int a0, uint32_t id, unsigned long long (&g)[NA]) {
     if constexpr (NA == 1 && PACK) {
-        g[0] = evt_load_gq<true>(gq, 0, 0, id);
+        g[0] = evt_load_narrow(gq, id);
     } else {
         const unsigned long long *p = gq + (size_t)id * stride + a0;
 #pragma unroll

@@ -46,28 +46,22 @@ struct ScanArgs {
     int fold_leaves; // the level's children are leaves: their weight and values are written along with the split (no pass of their own)
 };
 
-// shared prologue: node totals -> Float64 statistics.  Root totals are the bin sums of its first
-// sampled feature (exact in integers: every feature's bins sum to the same total); other nodes carry
-// the totals their parent's split gave them.
+// The root's totals -> Float64 statistics: the bin sums of its first sampled feature (exact in integers: every feature's bins sum to the same total); other nodes
+// carry the totals their parent's split gave them.
 template <int NAG>
-__device__ __forceinline__ void node_totals(const ScanArgs &A, int n, const long long *hn, bool writer, long long *s_Sq, double *s_S,
-                                            double *s_sc) {
+__device__ __forceinline__ void root_totals(const ScanArgs &A, int n, const long long *hn, long long *s_Sq, double *s_S, double *s_sc) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (tid < NAG) s_sc[tid] = A.qscale[tid];
-    if (A.level == 1) {
-        if (wave == 0) {
-            for (int ag = 0; ag < NAG; ag++) {
-                long long s = 0;
-                for (int b = lane; b < A.B; b += 64) s += hn[(int64_t)ag * A.B + b];
-                s = wave_sum_i64(s);
-                if (lane == 0) {
-                    s_Sq[ag] = s;
-                    if (writer) A.node_sum[(int64_t)n * NAG + ag] = s;
-                }
+    if (wave == 0) {
+        for (int ag = 0; ag < NAG; ag++) {
+            long long s = 0;
+            for (int b = lane; b < A.B; b += 64) s += hn[(int64_t)ag * A.B + b];
+            s = wave_sum_i64(s);
+            if (lane == 0) {
+                s_Sq[ag] = s;
+                A.node_sum[(int64_t)n * NAG + ag] = s;
             }
         }
-    } else if (tid < NAG) {
-        s_Sq[tid] = A.node_sum[(int64_t)n * NAG + tid];
     }
     __syncthreads();
     if (tid == 0) {
@@ -520,7 +514,7 @@ __global__ __launch_bounds__(256) void k_scan_fin(ScanArgs A, int ngroups) {
     __shared__ int s_dec[3];
 
     if (A.level == 1) {
-        node_totals<NAG>(A, n, hn, true, s_Sq, s_S, s_sc);
+        root_totals<NAG>(A, n, hn, s_Sq, s_S, s_sc);
     } else {
         if (tid < NAG) {
             s_sc[tid] = qs;
@@ -987,8 +981,7 @@ __global__ __launch_bounds__(NAG * BPL > 12 ? 512 : 1024) void k_obliv_level(Obl
 // Same search as k_scan / k_scan_fin with the channel count a run-time value: the node statistics live in shared
 // memory and the candidate gain is the sum of term(left_k) + term(right_k) over the outputs, added in the
 // reference's order (split_gain, src/split.jl:108-117), from one prefix scan per channel.
-__device__ __forceinline__ void node_totals_mc(const ScanArgs &A, int n, const long long *hn, bool writer, long long *s_Sq, double *s_S,
-                                               double *s_sc) {
+__device__ __forceinline__ void node_totals_mc(const ScanArgs &A, int n, const long long *hn, long long *s_Sq, double *s_S, double *s_sc) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int NAG = A.NAg;
     if (tid < NAG) s_sc[tid] = A.qscale[tid];
@@ -999,7 +992,7 @@ __device__ __forceinline__ void node_totals_mc(const ScanArgs &A, int n, const l
             s = wave_sum_i64(s);
             if (lane == 0) {
                 s_Sq[ag] = s;
-                if (writer) A.node_sum[(int64_t)n * NAG + ag] = s;
+                A.node_sum[(int64_t)n * NAG + ag] = s;
             }
         }
     } else if (tid < NAG) {
@@ -1275,7 +1268,7 @@ __global__ __launch_bounds__(256) void k_scan_fin_mc(ScanArgs A, int ngroups) {
     __shared__ double s_g[256];
     __shared__ int s_j[256], s_b[256];
     __shared__ int s_dec[3];
-    node_totals_mc(A, n, hn, true, s_Sq, s_S, s_sc);
+    node_totals_mc(A, n, hn, s_Sq, s_S, s_sc);
     if (tid == 0) A.tree.w[n - 1] = (float)s_S[NK - 1];
     if (A.leaf_level) {
         if (tid < K) A.tree.pred[(int64_t)K * (n - 1) + tid] = (float)leaf_value(A.loss, s_S, tid, K, A.eta, A.bagging, A.lambda, A.L2);

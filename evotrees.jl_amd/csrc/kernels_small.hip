@@ -751,7 +751,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
                     for (int a = 0; a < na; a++) {
                         unsigned long long v;
                         if (QUANT) v = quantise(A.raw[(size_t)(r + i) * A.NK + a], a, r + i, false);
-                        else if (PACK && a == 0 && !A.wide) v = evt_load_gq<true>(A.gq, N, 0, (uint32_t)(r + i));
+                        else if (PACK && a == 0 && !A.wide) v = evt_load_narrow(A.gq, (uint32_t)(r + i));
                         else v = A.gq[(size_t)a * N + r + i];
                         atomicAdd(h + a * B, v);
                     }
