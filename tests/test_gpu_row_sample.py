@@ -61,3 +61,30 @@ def test_few_rows_of_a_large_root_slice(evt, N):
         assert t.split.any()
     h.close()
     o.close()
+
+
+@pytest.mark.parametrize("loss,weights,N", [("mse", False, 8_191), ("mse", False, 8_193), ("logloss", True, 16_389), ("gaussian_mle", False, 1_048_577),
+                                            ("mse", False, 2_100_003), ("mse", True, 2_100_003)])
+def test_drawn_rows_beside_the_quantisation(evt, loss, weights, N):
+    """The mask drawn on the way, its last bytes and blocks partly filled, while blocks of the same kernel quantise the device's own gradients."""
+    F, B, D = 6, 16, 3
+    x_bin, y, w, mu = make_data(N, N, F, B, loss, weights)
+    h, o, op, gp, pred0, grad = setup_pair(evt, loss, x_bin, y, w, mu, B, D)
+    h.set_option("small_tree", 0)
+    js = np.arange(1, F + 1, dtype=np.uint32)
+    for k, cond in enumerate((127, 204, 1)):
+        seed = 1_000_003 * N + k
+        h.update_grads()
+        grad = h.get_grads()
+        h.draw_mask(seed)
+        h.grow_tree_begin_staged(js, gp, cond)
+        t = h.grow_tree_end()
+        rows = np.flatnonzero(evt.splitmix_mask(seed, N) <= cond).astype(np.uint32)
+        o.set_quant(grad, h.get_quant()[0])
+        t_fx, nidx = o.grow_tree(grad, rows, js, mode=1)
+        assert_tree_bits(t, t_fx)
+        got, want = h.get_nidx(), np.zeros(N, np.uint32)
+        want[rows] = np.asarray(nidx)[rows]
+        assert np.array_equal(got, want)
+    h.close()
+    o.close()

@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("loss,weights,K,N,F", [
     ("mse", False, None, 2_003, 20), ("mse", True, None, 2_003, 20), ("logloss", False, None, 1_001, 17), ("logloss", True, None, 1_001, 9),
     ("gaussian_mle", False, None, 4_003, 33), ("gaussian_mle", True, None, 777, 33), ("mlogloss", False, 3, 1_501, 12), ("mlogloss", True, 8, 1_501, 30),
+    ("gaussian_mle", True, None, 60_013, 20), ("mse", True, None, 300_007, 8), ("mlogloss", True, 4, 40_009, 6),
 ])
 def test_layouts_change_between_trees(evt, loss, weights, K, N, F):
     B = 32
