@@ -138,7 +138,7 @@ int launch_iota(evt_ctx *c, uint32_t *dst, int64_t n) {
     return EVT_OK;
 }
 
-// Small device -> pinned host copies by a kernel (16-byte words; nbytes is a multiple of 16).  A stream-ordered
+// A tree's arrays to its pinned slot by a kernel (blob_send: system-scope stores of 8 bytes).  A stream-ordered
 // hipMemcpyAsync goes through the copy engine, and handing the stream over to it and back stalls the kernels queued
 // behind it for tens of microseconds; a kernel's stores over the bus do not.
 __global__ __launch_bounds__(256) void k_copy_to_host(BlobOut O) { blob_send(O, (int)blockIdx.x); }

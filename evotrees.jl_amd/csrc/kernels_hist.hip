@@ -692,7 +692,7 @@ static int launch_hist_t(evt_ctx *c, const HistArgs &A, dim3 grid, int threads, 
 // t tiles make 256 / t spans of the same 256 blocks: 1 / t of the atomics, against row ids and gradient words that
 // each tile reads again and narrower loads.  Few rows take narrow tiles, many rows whole records; a histogram of
 // many channels or bins takes fewer spans than there are CUs.  The estimate, in us, with the figures fitted to sweeps of 30k to 4M
-// rows a tree, 20 to 120 features, 1 to 15 channels, 32 to 255 bins and depths 5 to 11 (it picks the best or one within 8 % of it):
+// rows a tree, 20 to 120 features, 1 to 15 channels, 32 to 255 bins and depths 5 to 11 (it picks the best or, with the present kernel, one within 5 % of it):
 //   8                                       launch, set-up, the first loads
 //   4.9e-6 * atomics of a span * spans      flush
 //   rows in millions * (max(3.2 * LDS adds of a row's 16 lanes, 18) + 3.5 * (tiles - 1)) * 256 / blocks of a layer

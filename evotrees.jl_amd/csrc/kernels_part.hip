@@ -1,6 +1,6 @@
 // Row partitioning and level bookkeeping, all device resident.
 //
-// split_set! (src/fit-utils.jl:93-312) is a stable partition of each split node's row-id segment;
+// split_set! (src/fit-utils.jl:93-312) is a stable partition of each split node's row-id segment, whose order is free here (all sums are of integers);
 // update_nodes_idx_kernel! (ext/EvoTreesKernelAbstractionsExt/fit-utils.jl:9-31) is the same
 // decision written per row.  Here every node owns a contiguous segment [seg_start, seg_start+seg_len)
 // of the row-id list; a split rewrites the segment (lefts first) into the other list buffer, so children are again
@@ -10,7 +10,7 @@
 //  two passes (weights, whose totals hold no counts, and histograms built on the way):
 //   count   : one block per chunk evaluates x_bin[row, feat] <= cond_bin, keeps the ballots,
 //             counts lefts;
-//   scatter : one block per chunk moves row ids to their stable destination (ascending ids on both sides).
+//   scatter : one block per chunk moves row ids to their stable destination (ascending ids on both sides where the node's are: in a tree on every row).
 // In both, chunks of nodes that became leaves record the node id per row (and add the leaf value to the prediction), and one
 // block sets the children's segments, picks which child is built (fewer rows; tie -> left, src/fit.jl:123-129) and writes
 // the next level's tables (active nodes, chunk prefix, build list).  It rides in the kernel that moves the rows; two passes
@@ -864,8 +864,7 @@ __device__ void tree_begin_root(const BeginArgs &A, int blocks) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < A.root_words; i += (int64_t)blocks * blockDim.x) A.hist[i] = 0;
 }
 // Blocks from `blocks` on quantise the gradients, which have nothing to do with the set-up: side by side in one launch where the gradients' words are
-// still to be made: set-up + quantisation, us, 500k rows of four channels 4.2 + 6.9 -> 7.0, 60k of 14 channels 3.0 + 7.9 -> 9.3; mask count +
-// quantisation, 1M rows 3.1 + 5.8 -> 6.3, of two channels 3.2 + 7.5 -> 8.7 - and a launch each.
+// still to be made: set-up + quantisation, us, 500k rows of four channels 4.2 + 6.9 -> 7.0, 60k of 14 channels 3.0 + 7.9 -> 9.3 - and a launch each.
 __global__ __launch_bounds__(1024) void k_tree_begin(BeginArgs A, QuantArgs Q, int blocks) {
     if ((int)blockIdx.x >= blocks) {
         quant_rows(Q, (int)blockIdx.x - blocks, (int)gridDim.x - blocks);
@@ -920,8 +919,8 @@ __device__ __forceinline__ unsigned mask_flags(uint8_t *mask, uint8_t cond, int6
 // level's tables; block 0 prepares the rest of the tree.  Blocks behind the sample's help it clear the root's slice where that has more words than the
 // sample's blocks write in a few stores each (30k rows x 120 features of 255 bins and 15 channels, 459k words: 6.8 us; 18.3 by the 4 blocks of the sample), those behind them quantise.  Bound by its chain (draw, count, claim, stores) and the
 // quantisation beside it: 1M rows 7.9 us with one word a row, 10.0 with two (a block's rows by 1024 threads: 9.1, 12.4: quantisation gets its blocks later).  In two kernels, a
-// count and a scatter that added the counts up, 5.9 + 5.1 and 8.9 + 4.7; with a scan between them, from 2M rows on,
-// 100 rounds of 6M x 20 46.2 ms for 45.5, of 10M 67.4 for 67.7.
+// count and a scatter that added the counts up, 5.9 + 5.1 and 8.9 + 4.7; where a scan ran between them, from 2M rows on, and the quantisation is a kernel of its own, 6M rows
+// 15.8 us for 6.2 + 4.7 + 7.6, 10M 23.1 for 7.4 + 5.4 + 10.9.
 template <bool DRAW>
 __global__ __launch_bounds__(256) void k_mask_sample(uint8_t *mask, uint8_t cond, int64_t N, unsigned long long seed, uint32_t *is_out,
                                                      unsigned long long *claims, BeginArgs B, QuantArgs Q, int blocks, int clear) {
