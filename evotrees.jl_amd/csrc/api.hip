@@ -182,7 +182,7 @@ extern "C" int evt_destroy(evt_handle c) {
     if (!c) return EVT_OK;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    void *ptrs[] = {c->xcm, c->xrm, c->y, c->pred, c->grad, c->gq, c->is_a, c->is_b, c->nidx, c->mask, c->flagw, c->sample_claims, c->blob_arrived, c->chunk_nleft, c->chunk_lpre, c->cursor,
+    void *ptrs[] = {c->xcm, c->xrm, c->y, c->pred, c->grad, c->grad_next, c->gq, c->is_a, c->is_b, c->nidx, c->mask, c->flagw, c->sample_claims, c->blob_arrived, c->chunk_nleft, c->chunk_lpre, c->cursor,
                     c->hist, c->seg_start, c->seg_len, c->status, c->node_sum, c->tree_blob, c->tree.packed, c->js, c->jsmap, c->feattypes, c->mono, c->absmax, c->qexp_buf[0], c->qexp_buf[1], c->qbits,
                     c->qscale_buf[0], c->qscale_buf[1], c->planes, c->metric_partial, c->errflag, c->ogains, c->sbest, c->scan_count, c->is_id, c->pt_nodes, c->mask_next,
                     c->small_nid[0], c->small_nid[1], c->small_head[0], c->small_head[1], c->small_left[0], c->small_left[1], c->small_acc,
@@ -277,7 +277,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     memset(&c->tree, 0, sizeof(c->tree));
     c->tree_blob = nullptr;
     memset(c->lvl, 0, sizeof(c->lvl));
-    c->js = nullptr; c->jsmap = nullptr; c->feattypes = nullptr; c->mono = nullptr; c->absmax = nullptr; c->absmax_cur = 0; c->qexp = nullptr; c->qbits = nullptr;
+    c->js = nullptr; c->jsmap = nullptr; c->feattypes = nullptr; c->mono = nullptr; c->absmax = nullptr; c->absmax_cur = 0; c->absmax_other = 1; c->absmax_spare = 2; c->grad_next = nullptr; c->path_off = 0; c->slot_path[0] = c->slot_path[1] = false; c->qexp = nullptr; c->qbits = nullptr;
     c->alphas = nullptr; c->alphas_f = nullptr; c->qkeys_a = c->qkeys_b = nullptr; c->qtemp = nullptr; c->qtemp_bytes = 0;
     c->n_alphas = 1;
     for (int k = 0; k < EVT_MAX_K; k++) c->h_alphas[k] = 0.5;
@@ -403,7 +403,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     ALLOC(c->jsmap, c->RS);
     ALLOC(c->feattypes, c->F);
     ALLOC(c->mono, c->F);
-    ALLOC(c->absmax, 2 * EVT_ABSMAX_STRIPES * EVT_MC_MAX_NK);
+    ALLOC(c->absmax, 3 * EVT_ABSMAX_STRIPES * EVT_MC_MAX_NK);
     ALLOC(c->alphas, EVT_MAX_K);
     ALLOC(c->alphas_f, EVT_MAX_K);
     for (int s = 0; s < 2; s++) {
@@ -426,6 +426,10 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     // pinned staging: tree read-back + small per-tree uploads; coherent: wait_for_tree reads it while the kernel that fills it runs
     c->h_stage_bytes = c->blob_bytes + (size_t)c->F * 4 + (size_t)c->RS * 2 + 1024;
     c->h_stage_bytes = (c->h_stage_bytes + 255) / 256 * 256;
+    if (!c->mc && tree_type != EVT_TREE_OBLIVIOUS && c->D >= 2 && c->D <= 10) {
+        c->path_off = c->h_stage_bytes;
+        c->h_stage_bytes += ((size_t)c->nnodes * sizeof(PathNode) + 8 * EVT_PATH_BLOCKS + 255) / 256 * 256;
+    }
     c->h_stage_base = c->h_stage_dev_base = static_cast<uint8_t *>(coherent_take(2 * c->h_stage_bytes + 128));
     if (!c->h_stage_base) {
         evt_destroy(c);
@@ -434,6 +438,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     for (int k = 0; k < 2; k++) { // behind the slots, a line each; trees count from 1
         c->slot_flag[k] = reinterpret_cast<unsigned long long *>(c->h_stage_base + 2 * c->h_stage_bytes + 64 * k);
         *c->slot_flag[k] = 0;
+        if (c->path_off) memset(c->h_stage_base + k * c->h_stage_bytes + c->path_off + (size_t)c->nnodes * sizeof(PathNode), 0, 8 * EVT_PATH_BLOCKS);
     }
     c->h_stage = c->h_stage_base;
     c->h_stage_dev = c->h_stage_dev_base;
@@ -442,7 +447,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     c->h_mono.assign(c->F, 0);
     hipError_t e2 = hipMemsetAsync(c->feattypes, 1, c->F, c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->mono, 0, sizeof(int32_t) * c->F, c->stream);
-    if (e2 == hipSuccess) e2 = hipMemsetAsync(c->absmax, 0, sizeof(uint32_t) * 2 * EVT_ABSMAX_STRIPES * EVT_MC_MAX_NK, c->stream);
+    if (e2 == hipSuccess) e2 = hipMemsetAsync(c->absmax, 0, sizeof(uint32_t) * 3 * EVT_ABSMAX_STRIPES * EVT_MC_MAX_NK, c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->nidx, 0, sizeof(uint32_t) * N, c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->errflag, 0, sizeof(int32_t), c->stream);
     if (e2 == hipSuccess) e2 = hipMemsetAsync(c->blob_arrived, 0, sizeof(int), c->stream);
@@ -1057,6 +1062,7 @@ static int tree_close(evt_ctx *c) {
         r = launch_copy_to_host(c, true);
         if (r != EVT_OK) return r;
     }
+    c->slot_path[c->slot_w] = c->step.small == SMALL_PATH;
     c->slot_ev[c->slot_w] = c->profiling != 0; // the times of all its kernels are read when it is collected
     if (c->profiling) HIPCHK(hipEventRecord(c->tree_evs[c->slot_w], c->stream));
     c->slot_seq[c->slot_w] = c->tree_seq;
@@ -1087,7 +1093,7 @@ static int tree_fail(evt_ctx *c, int r) { // a failed stage leaves no tree open
 // every stage of an opened tree, then the close: what evt_grow_tree_begin queues
 static int tree_run_stages(evt_ctx *c, int r) {
     if (r == EVT_OK && c->step.small) {
-        r = launch_small_tree(c, &c->step.p, c->step.small_draw, c->step.small);
+        r = c->step.small == SMALL_PATH ? launch_small_path(c, &c->step.p, c->step.small_draw) : launch_small_tree(c, &c->step.p, c->step.small_draw, c->step.small);
         c->step.phase = 4;
     }
     while (r == EVT_OK && c->step.phase != 4) {
@@ -1240,6 +1246,21 @@ static int fill_tree_out(evt_ctx *c, const uint8_t *hs, evt_tree_out *tree) {
     return EVT_OK;
 }
 
+// ... and of a tree of one launch
+static int fill_tree_out(evt_ctx *c, const PathNode *nodes, evt_tree_out *tree) {
+    ARGCHK(tree->feat && tree->cond_bin && tree->w && tree->gain && tree->pred && tree->split, "tree output arrays must not be NULL");
+    for (int n = 0; n < c->nnodes; n++) {
+        const PathNode v = nodes[n];
+        tree->feat[n] = v.feat;
+        tree->cond_bin[n] = (uint8_t)v.cond_bin;
+        tree->w[n] = v.w;
+        tree->gain[n] = v.gain;
+        tree->split[n] = (uint8_t)v.split;
+        for (int k = 0; k < c->K; k++) tree->pred[(size_t)c->K * n + k] = v.pred[k];
+    }
+    return EVT_OK;
+}
+
 static inline void spin_pause() {
 #if defined(__x86_64__)
     __builtin_ia32_pause();
@@ -1254,7 +1275,15 @@ static int wait_for_tree(evt_ctx *c, int slot) {
         return EVT_OK;
     }
     const unsigned long long seq = (unsigned long long)c->slot_seq[slot];
-    auto there = [&]() { return __atomic_load_n(c->slot_flag[slot], __ATOMIC_ACQUIRE) == seq; };
+    const bool path = c->slot_path[slot];
+    const unsigned long long *flags =
+        path ? reinterpret_cast<const unsigned long long *>(c->h_stage_base + (size_t)slot * c->h_stage_bytes + c->path_off + (size_t)c->nnodes * sizeof(PathNode)) : c->slot_flag[slot];
+    int seen = 0;
+    const int words = path ? 1 << (c->D - 2) : 1;
+    auto there = [&]() {
+        while (seen < words && __atomic_load_n(flags + seen, __ATOMIC_ACQUIRE) == seq) seen++;
+        return seen == words;
+    };
     for (int k = 0; k < 4096; k++) {
         if (there()) return EVT_OK;
         spin_pause();
@@ -1294,16 +1323,20 @@ extern "C" int evt_grow_tree_end(evt_handle c, evt_tree_out *tree) {
     const size_t o_stats = c->blob_stats;
     const int arrived = wait_for_tree(c, slot);
     if (arrived != EVT_OK) return arrived;
-    const int64_t n_is = reinterpret_cast<const int64_t *>(hs + o_stats)[0];
+    const bool path = c->slot_path[slot];
+    const PathNode *nodes = reinterpret_cast<const PathNode *>(hs + c->path_off);
+    int64_t n_is = path ? nodes[0].rows : reinterpret_cast<const int64_t *>(hs + o_stats)[0];
     if (c->profiling || !c->recs.empty()) {
         if (c->profiling) c->prof_units[EVT_K_PARTITION] += n_is;
-        prof_collect(c, reinterpret_cast<const int64_t *>(hs + o_stats), c->slot_seq[slot]);
+        int64_t rows[EVT_MAX_DEPTH + 2] = {n_is}; // of the levels
+        for (int n = 1; path && n <= c->nnodes; n++) rows[32 - __builtin_clz((unsigned)n)] += nodes[n - 1].rows;
+        prof_collect(c, path ? rows : reinterpret_cast<const int64_t *>(hs + o_stats), c->slot_seq[slot]);
     }
     if (n_is == 0) { // the tree grown on no rows is a single zero leaf; report it as the reference does
         evt_set_error("no subsample observation - choose larger rowsample");
         return EVT_ERR_EMPTY;
     }
-    if (tree) return fill_tree_out(c, hs, tree);
+    if (tree) return path ? fill_tree_out(c, nodes, tree) : fill_tree_out(c, hs, tree);
     return EVT_OK;
     });
 }
@@ -1812,7 +1845,7 @@ extern "C" int evt_set_option(evt_handle c, const char *name, int64_t value) {
     } else if (strcmp(name, "record_nidx") == 0) {
         c->record_nidx = value != 0;
     } else if (strcmp(name, "small_tree") == 0) {
-        ARGCHK(value >= 0 && value <= 3, "small_tree must be 0 (never), 1 (inputs of few rows), 2 or 3 (a block, or several, per feature and level wherever it can)");
+        ARGCHK(value >= 0 && value <= 4, "small_tree must be 0 (never), 1 (inputs of few rows), 2 or 3 (a block, or several, per feature and level wherever it can) or 4 (one launch per tree wherever it can)");
         c->small_tree = (int)value;
     } else if (strcmp(name, "scan_fused") == 0) {
         c->scan_fused = value != 0;

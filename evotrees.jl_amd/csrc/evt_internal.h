@@ -68,6 +68,14 @@ struct LevelTab {
     uint4 *cdesc;      // per chunk of the level: {node, first position, end of the node's segment, first chunk of the node}; written with the tables
 };
 
+// a node in the pinned buffer
+struct PathNode {
+    uint32_t feat : 16, cond_bin : 8, split : 8;
+    uint32_t rows; // of the sample, of a node that was searched
+    float w, gain, pred[2];
+};
+#define EVT_PATH_BLOCKS 256
+
 struct TreeDev {
     int32_t *feat;    // 1-based, 0 none
     uint8_t *cond_bin;
@@ -121,6 +129,7 @@ struct evt_ctx {
     float *y;
     float *pred;    // K x N
     float *grad;    // NK x N
+    float *grad_next; // another: the next gradients where a kernel computes them beside those it reads (kernels_path.hip); allocated with the first such tree
     unsigned long long *gq; // fixed-point words of the rows: NA planes of N, or (gq_rows) EVT_GQ_STRIDE(NA) words a row
     size_t gq_words;        // of the allocation: the channels of the targets set so far, without weights or with them
     bool gq_rows;           // which: the kernels of small trees walk all rows and read planes, the others gather rows
@@ -153,8 +162,12 @@ struct evt_ctx {
     uint16_t *jsmap;   // [RS] slot of the feature at byte p of a record, 0xFFFF = not sampled / padding
     uint8_t *feattypes;
     int32_t *mono;
-    uint32_t *absmax;  // [2][EVT_ABSMAX_STRIPES][EVT_MC_MAX_NK] float bits: two sets, raised by alternate gradient passes
-    int absmax_cur;    // the set the next gradient pass raises
+    // [3][EVT_ABSMAX_STRIPES][EVT_MC_MAX_NK] float bits: two sets, raised by alternate gradient passes, and a third for a kernel that reads one,
+    // clears the second and raises the next gradients' (kernels_path.hip)
+    uint32_t *absmax;
+    int absmax_cur;    // the set the next gradient pass raises, and the quantisation behind it reads
+    int absmax_other;  // the one that quantisation clears
+    int absmax_spare;  // zero but for the weights' row
     // quantile losses: levels (Float64 for the gradients, Float32 for the metrics) and the sort buffers of the leaf pass
     double h_alphas[EVT_MAX_K];
     int32_t n_alphas;
@@ -204,7 +217,9 @@ struct evt_ctx {
     int hist_blocks, hist_threads, hist_min_rows, hist_seg_cost, hist_tile;
     int hist_variant;  // 0 auto, 1 generic 16-byte-piece kernel, 2 conflict-free 8-byte-piece kernel where it applies
     int scan_fused;    // option: the split search of a node with at most 16 sampled features runs in one kernel
-    int small_tree;    // option: one kernel per level (kernels_small.hip) - 0 never, 1 for inputs of few rows, 2 wherever it can, 3 with several blocks to a feature wherever it can
+    // option: one kernel per level (kernels_small.hip) or tree (kernels_path.hip) - 0 never, 1 for inputs of few rows, 2 one per level wherever it can, 3 with several blocks to a
+    // feature wherever it can, 4 one per tree wherever it can
+    int small_tree;
     // its buffers, allocated with the first such tree: the rows' node ids, the blocks' candidates and the totals left of them, of
     // two levels each
     uint32_t *small_nid[2];
@@ -223,6 +238,10 @@ struct evt_ctx {
     int *blob_arrived;
     hipEvent_t tree_evs[2];
     bool slot_ev[2];
+    // a tree of one launch (kernels_path.hip) leaves its nodes behind the slot's arrays, 24 bytes each (PathNode), and behind them a word per block
+    // that becomes the tree's number; path_off: where, 0 for a handle that grows none
+    size_t path_off;
+    bool slot_path[2];
     int tree_in_flight;     // trees queued by evt_grow_tree_begin that evt_grow_tree_end has not collected (0..2)
     int slot_w, slot_r;     // staging slot of the next tree queued / of the oldest tree not yet collected
     int64_t tree_seq;       // trees opened so far; slot_seq: the tree each slot holds
@@ -234,7 +253,7 @@ struct evt_ctx {
         bool all_rows, defer, fuse_pred;
         bool walk;       // a tree on every row whose rows are walked through it at the end, as those of a sampled tree are (walk_pays)
         bool hist_fused; // levels below the root get their histograms from the scatter pass of the level above
-        int small;       // one kernel per level: the blocks that share a feature's rows (small_tree_form)
+        int small;       // one kernel per level: the blocks that share a feature's rows; SMALL_PATH: one for the tree (small_tree_form)
         bool small_draw; // ... whose first draws the row mask
         bool grads_done; // the tree's last kernel added the leaf values and computed the next round's gradients
         bool blob_sent;  // the finished tree's transfer to the host rode along with the tree's last kernel
@@ -439,6 +458,9 @@ bool scatter_can_build_hist(const evt_ctx *c, int nfs);
 int small_tree_form(const evt_ctx *c, int nfs, bool all_rows);
 bool small_root_quantises(const evt_ctx *c, int form);
 int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices);
+#define SMALL_PATH (-1) // of small_tree_form: the whole tree in one launch
+bool small_path_takes(const evt_ctx *c, int nfs, bool whatever);
+int launch_small_path(evt_ctx *c, const evt_params *p, bool draw);
 int launch_final_fused(evt_ctx *c, int level, const uint32_t *is_cur, bool fuse_pred, bool send_blob);
 int launch_nidx_from_segments(evt_ctx *c, int level, const uint32_t *is_cur);
 struct BlobOut;

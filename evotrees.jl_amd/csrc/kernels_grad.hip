@@ -354,7 +354,7 @@ int launch_absmax_rows(evt_ctx *c, int k0, int k1) {
     int64_t nb = (c->N + 255) / 256;
     if (nb > 2048) nb = 2048;
     for (int pass = 0; pass < 2; pass++) {
-        uint32_t *am = absmax_set(c, pass == 0 ? c->absmax_cur : c->absmax_cur ^ 1);
+        uint32_t *am = absmax_set(c, pass == 0 ? c->absmax_cur : c->absmax_other);
         const int a0 = pass == 0 ? k0 : std::max(k0, c->NK - 1);
         if (a0 >= k1) continue;
         hipLaunchKernelGGL(k_absmax_clear, dim3(1), dim3(256), 0, c->stream, am, a0, k1);
@@ -383,7 +383,7 @@ void quant_args(evt_ctx *c, QuantArgs &Q) {
     Q.pack_wide = (c->unit_w && c->NA > EVT_MAX_NA) ? 1 : 0;
     Q.stride = c->gq_rows ? EVT_GQ_STRIDE(c->NA) : 0;
     Q.absmax = absmax_set(c, c->absmax_cur);
-    Q.absmax_next = absmax_set(c, c->absmax_cur ^ 1);
+    Q.absmax_next = absmax_set(c, c->absmax_other);
     Q.qbits = c->qbits;
     Q.qexp = c->qexp;
     Q.qscale = c->qscale;
@@ -398,7 +398,7 @@ unsigned quant_blocks(const evt_ctx *c, int threads) {
 
 void quant_taken(evt_ctx *c) {
     c->quant_pending = false;
-    c->absmax_cur ^= 1; // the next gradient pass raises the set that the quantisation cleared
+    std::swap(c->absmax_cur, c->absmax_other); // the next gradient pass raises the set that the quantisation cleared
 }
 
 int launch_quantize(evt_ctx *c) {

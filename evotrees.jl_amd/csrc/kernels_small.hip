@@ -1101,7 +1101,7 @@ static int small_tree_buffers(evt_ctx *c, bool split) {
     return EVT_OK;
 }
 
-// Which form a tree takes: 0 the kernels of larger inputs, 1 a block per feature, S > 1 a feature's rows
+// Which form a tree takes: 0 the kernels of larger inputs, SMALL_PATH one launch (small_path_takes), 1 a block per feature, S > 1 a feature's rows
 // shared by S blocks.  A block walks its rows once per level (and once more for every `slots` nodes), so a level grows with
 // rows / S, the channels and - through the candidates every block reads and the searches its 16 wavefronts share - the nodes; slices
 // add the words they flush and, where a level is searched apart, a launch.  The other path spreads rows of any number over the chip and pays for its launches.
@@ -1115,6 +1115,8 @@ static int small_tree_buffers(evt_ctx *c, bool split) {
 int small_tree_form(const evt_ctx *c, int nfs, bool all_rows) {
     if (!c->small_tree || c->D < 2 || c->D > 10 || nfs > 256 || c->N < 4 || c->N > (1 << 24) || !c->defer_pred || EVT_IS_QUANTILE(c->loss)) return 0;
     if (c->record_nidx && !all_rows) return 0;
+    if ((c->small_tree == 1 || c->small_tree == 4) && small_path_takes(c, nfs, c->small_tree == 4)) return SMALL_PATH;
+    if (c->small_tree == 4) return 0;
     const bool obliv = c->tree_type == EVT_TREE_OBLIVIOUS;
     const int nodes = 1 << (c->D - 2), slots = small_slots(c, false), slots_split = small_slots(c, true);
     const int S = std::max(2, 256 / nfs);
@@ -1195,7 +1197,7 @@ int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices) {
     if (c->quant_pending) {
         A.fresh = 1;
         A.absmax = absmax_set(c, c->absmax_cur);
-        A.absmax_next = absmax_set(c, c->absmax_cur ^ 1);
+        A.absmax_next = absmax_set(c, c->absmax_other);
         A.qbits = c->qbits;
         A.qexp = c->qexp;
     }

@@ -406,7 +406,7 @@ int evt_reset_profile(evt_handle h);
  * (feature, bin threshold) from x_bin - F * (nbins - 1) * nobs / 8 bytes, taken only when that is at most 16 GiB and a third of the free
  * memory - and the row partition reads its decisions there; 0: it gathers bin bytes; same trees, bit for bit);
  * "small_tree" (inputs of few rows and up to 256 sampled features and depth 10 may grow a tree with one kernel per level (two where
- * nodes are many), a block or several to a feature: 1, default: where that is estimated to be faster; 0: never; 2, 3: one block or several wherever it can; same trees, bit for bit);
+ * nodes are many), a block or several to a feature: 1, default: where that is estimated to be faster; 0: never; 2, 3: one block or several wherever it can; 4: the whole tree in one launch wherever it can; same trees, bit for bit);
  * "record_nidx" (1: the partition also records every sampled row's final node while the tree grows;
  * 0, default: evt_get_nidx derives it afterwards by walking the finished tree); "defer_pred" (1, default:
  * leaf values of a tree grown on every row are added in row order by the next pass over the rows, or, with "grads_ahead", by a walk of
