@@ -756,6 +756,7 @@ __global__ __launch_bounds__(NAG * BPL > 12 ? 512 : 1024) void k_obliv_level(Obl
     __shared__ int s_last, s_bin, s_cell;
     __shared__ double s_best;
     const OblivArgs &A = L.o;
+    touch_kernargs<sizeof(OblivLevelArgs)>();
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
     constexpr int K = (NAG == 5) ? 2 : 1, NK = 2 * K + 1;
     const int B = A.B, jp = blockIdx.x;
@@ -769,6 +770,8 @@ __global__ __launch_bounds__(NAG * BPL > 12 ? 512 : 1024) void k_obliv_level(Obl
     double sc[NAG];
 #pragma unroll
     for (int ag = 0; ag < NAG; ag++) sc[ag] = A.qscale[ag];
+#pragma unroll
+    for (int j = 0; j < NPW; j++) asm volatile("" : "+v"(st[j])); // requested ahead of the branch
     if (!any) return; // every block alike
     const bool numeric = A.feattypes[f] != 0;
     const int constraint = L.mono[f];
@@ -1046,6 +1049,7 @@ template <int BPL, bool LOOP>
 __global__ __launch_bounds__(64 * (EVT_MAX_K / 2)) void k_scan_mc(ScanArgs A) {
     extern __shared__ double s_term[]; // [K][B]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
+    touch_kernargs<sizeof(ScanArgs)>();
     const int nodeidx = blockIdx.x, n = (1 << (A.level - 1)) + nodeidx, jp = blockIdx.y;
     int f = (int)A.js[jp] - 1;
     const int st = A.status[n];
