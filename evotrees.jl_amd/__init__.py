@@ -402,6 +402,7 @@ class Cache:
     def __init__(self, handle, rng, nfs, params, N, F, config=None):
         self.handle, self.rng, self.nfs, self.params, self.N, self.F, self.config = handle, rng, nfs, params, N, F, config
         self.cell = [object()]  # of all trees of the fit (TreeArrays)
+        self.all_feats = np.arange(1, F + 1, dtype=np.uint32)
         self.pending = []  # trees queued on the device and not yet collected, oldest first (at most two)
 
 
@@ -474,7 +475,7 @@ def _begin_tree(cache, config, first_of_round):
     cond = int(np.rint(255 * config.rowsample))  # round(UInt8, 255*rowsample), src/subsample.jl:9
     seed = int(cache.rng.integers(0, 1 << 64, dtype=np.uint64)) if cond < 255 else None
     if cache.nfs >= cache.F:
-        js = np.arange(1, cache.F + 1, dtype=np.uint32)
+        js = cache.all_feats
     else:
         js = (np.sort(cache.rng.choice(cache.F, cache.nfs, replace=False)) + 1).astype(np.uint32)
     if seed is not None:
@@ -505,7 +506,7 @@ def grow_evotree(m, cache, config, more=False):
             _begin_tree(cache, config, b == 0)
         if b + 1 < n:
             _begin_tree(cache, config, False)
-        elif more:
+        elif more and len(cache.pending) < 2:  # fit may have queued it while the round before was evaluated
             _begin_tree(cache, config, True)
         t = cache.pending.pop(0)
         try:
@@ -567,8 +568,16 @@ class CallBack:
         self.handle = h
 
     def __call__(self, logger, it, tree):
+        self.start(tree)
+        self.finish(logger, it)
+
+    def start(self, tree):
+        """The call's device work, queued; finish() waits for it."""
         self.handle.predict_tree(tree)
-        update_logger(logger, it, self.handle.eval_metric(self.metric))
+        self.handle.eval_metric_begin(self.metric)
+
+    def finish(self, logger, it):
+        update_logger(logger, it, self.handle.eval_metric_end())
 
     def close(self):
         self.handle.close()
@@ -637,7 +646,13 @@ def fit(config, dtrain=None, x_train=None, y_train=None, w_train=None, offset_tr
             # that tree may turn out one too many; it is dropped with the handle, unless the caller keeps the handle
             grow_evotree(m, cache, config, more=(i < config.nrounds and (logger is None or not return_cache)))
             if logger is not None:
-                cb(logger, i, m.trees[-1])  # as the reference: only the round's last tree reaches the eval prediction
+                cb.start(m.trees[-1])  # as the reference: only the round's last tree reaches the eval prediction
+                # while the device evaluates the round and grows the tree behind it, the host queues the one after that (one more that early stopping may drop): of small
+                # fits the host is what a round waits for (2000 rows x 10 with 500 eval rows, 100 rounds 5.5 -> 4.5 ms together with cheaper addresses of arrays;
+                # 100k rows, where it is the device, level)
+                if i + 1 < config.nrounds and not return_cache and config.bagging_size == 1 and len(cache.pending) == 1:
+                    _begin_tree(cache, config, True)
+                cb.finish(logger, i)
                 if i % print_every_n == 0 and verbosity > 0:
                     print("iter %d: %s = %.6g" % (i, config.metric, logger["metrics"][-1]))
                 if logger["iter_since_best"] >= logger["early_stopping_rounds"]:

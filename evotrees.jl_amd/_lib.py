@@ -27,7 +27,7 @@ EXPORTS = [
     "evt_grow_tree_begin", "evt_grow_tree_end", "evt_stage_mask", "evt_grow_tree_begin_staged", "evt_draw_mask",
     "evt_tree_open", "evt_hist_build", "evt_split_scan", "evt_update_nodes_idx", "evt_tree_close", "evt_peek_tree",
     "evt_predict_tree", "evt_get_xbin", "evt_get_pred", "evt_get_grads", "evt_get_nidx", "evt_get_hist", "evt_get_quant",
-    "evt_predict", "evt_predict_f64", "evt_predict_leaf_idx", "evt_eval_metric", "evt_set_profiling", "evt_get_profile", "evt_reset_profile",
+    "evt_predict", "evt_predict_f64", "evt_predict_leaf_idx", "evt_eval_metric", "evt_eval_metric_begin", "evt_eval_metric_end", "evt_set_profiling", "evt_get_profile", "evt_reset_profile",
     "evt_set_option", "evt_synchronize", "evt_copy_bandwidth", "evt_read_bandwidth", "evt_predict_static",
     "evt_lds_atomic_rate", "evt_global_atomic_rate", "evt_trim", "evt_binarize", "evt_bin_columns", "evt_order_stats",
     "evt_model_create", "evt_model_destroy", "evt_model_predict",
@@ -106,6 +106,8 @@ def load():
         "evt_model_destroy": [vp],
         "evt_model_predict": [vp, i32, vp, vp, vp, vp, vp, vp, i32, vp, vp, vp, i32, i64, i64, i64, i32, i32, i32, vp, vp],
         "evt_eval_metric": [vp, i32, vp],
+        "evt_eval_metric_begin": [vp, i32],
+        "evt_eval_metric_end": [vp, vp],
         "evt_set_profiling": [vp, i32],
         "evt_get_profile": [vp, vp, vp, vp],
         "evt_reset_profile": [vp],
@@ -131,9 +133,22 @@ def check(rc):
 
 
 def ptr(a):
+    """An array's address as an argument of a call, which keeps the array alive: by way of its buffer (0.4 us; ndarray.ctypes 2.4, of which a round of a fit paid a
+    dozen), or as numpy gives it where that is refused (read-only, empty or strided arrays)."""
     if a is None:
         return None
-    return a.ctypes.data_as(C.c_void_p)
+    try:
+        return C.byref(C.c_char.from_buffer(a))
+    except (TypeError, ValueError, BufferError):
+        return a.ctypes.data_as(C.c_void_p)
+
+
+def address(a):
+    """An array's address as a number: the caller keeps the array alive."""
+    try:
+        return C.addressof(C.c_char.from_buffer(a))
+    except (TypeError, ValueError, BufferError):
+        return a.ctypes.data
 
 
 def device_count():
@@ -273,7 +288,7 @@ class TreeArrays:
         self.__dict__.update({"_cell": [object()]}, **state)
 
     def as_out(self):
-        return EvtTreeOut(ptr(self.feat), ptr(self.cond_bin), ptr(self.w), ptr(self.gain), ptr(self.pred), ptr(self.split))
+        return EvtTreeOut(address(self.feat), address(self.cond_bin), address(self.w), address(self.gain), address(self.pred), address(self.split))
 
 
 class Handle:
@@ -425,6 +440,15 @@ class Handle:
         """Metric of the handle's prediction against its target and weights (the eval CallBack's feval)."""
         v = C.c_double(0.0)
         check(load().evt_eval_metric(self._h, METRIC_IDS[metric], C.byref(v)))
+        return v.value
+
+    def eval_metric_begin(self, metric):
+        """Queues the metric; eval_metric_end waits for it."""
+        check(load().evt_eval_metric_begin(self._h, METRIC_IDS[metric]))
+
+    def eval_metric_end(self):
+        v = C.c_double(0.0)
+        check(load().evt_eval_metric_end(self._h, C.byref(v)))
         return v.value
 
     def get_xbin(self):

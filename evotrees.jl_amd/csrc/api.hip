@@ -277,7 +277,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     memset(&c->tree, 0, sizeof(c->tree));
     c->tree_blob = nullptr;
     memset(c->lvl, 0, sizeof(c->lvl));
-    c->js = nullptr; c->jsmap = nullptr; c->feattypes = nullptr; c->mono = nullptr; c->absmax = nullptr; c->absmax_cur = 0; c->absmax_other = 1; c->absmax_spare = 2; c->grad_next = nullptr; c->path_off = 0; c->slot_path[0] = c->slot_path[1] = false; c->qexp = nullptr; c->qbits = nullptr;
+    c->js = nullptr; c->jsmap = nullptr; c->feattypes = nullptr; c->mono = nullptr; c->absmax = nullptr; c->absmax_cur = 0; c->absmax_other = 1; c->absmax_spare = 2; c->grad_next = nullptr; c->path_off = 0; c->metric_host = nullptr; c->metric_queued = false; c->slot_path[0] = c->slot_path[1] = false; c->qexp = nullptr; c->qbits = nullptr;
     c->alphas = nullptr; c->alphas_f = nullptr; c->qkeys_a = c->qkeys_b = nullptr; c->qtemp = nullptr; c->qtemp_bytes = 0;
     c->n_alphas = 1;
     for (int k = 0; k < EVT_MAX_K; k++) c->h_alphas[k] = 0.5;
@@ -430,7 +430,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
         c->path_off = c->h_stage_bytes;
         c->h_stage_bytes += ((size_t)c->nnodes * sizeof(PathNode) + 8 * EVT_PATH_BLOCKS + 255) / 256 * 256;
     }
-    c->h_stage_base = c->h_stage_dev_base = static_cast<uint8_t *>(coherent_take(2 * c->h_stage_bytes + 128));
+    c->h_stage_base = c->h_stage_dev_base = static_cast<uint8_t *>(coherent_take(2 * c->h_stage_bytes + 192));
     if (!c->h_stage_base) {
         evt_destroy(c);
         return EVT_ERR_NOMEM;
@@ -440,6 +440,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
         *c->slot_flag[k] = 0;
         if (c->path_off) memset(c->h_stage_base + k * c->h_stage_bytes + c->path_off + (size_t)c->nnodes * sizeof(PathNode), 0, 8 * EVT_PATH_BLOCKS);
     }
+    c->metric_host = reinterpret_cast<double *>(c->h_stage_base + 2 * c->h_stage_bytes + 128);
     c->h_stage = c->h_stage_base;
     c->h_stage_dev = c->h_stage_dev_base;
     // defaults: all numeric, no monotone constraint; queued in stream order ahead of whatever reads them
@@ -1530,10 +1531,9 @@ extern "C" int evt_get_quant(evt_handle c, int32_t *qbits, int32_t *qexp) {
 }
 
 // ---- evaluation metric ------------------------------------------------------------------------
-extern "C" int evt_eval_metric(evt_handle c, int32_t metric, double *value_out) {
+extern "C" int evt_eval_metric_begin(evt_handle c, int32_t metric) {
     return guarded([&]() -> int {
     CTXCHK(c);
-    ARGCHK(value_out, "value_out is NULL");
     ARGCHK(metric >= 0 && metric <= EVT_METRIC_MULTIQUANTILE, "unknown metric");
     ARGCHK(metric != EVT_METRIC_MULTIQUANTILE || c->loss == EVT_LOSS_MULTIQUANTILE,
            "multiquantile is the metric of the multiquantile loss (one target, a level per output) and of no other");
@@ -1546,15 +1546,40 @@ extern "C" int evt_eval_metric(evt_handle c, int32_t metric, double *value_out) 
         evt_set_error("evt_eval_metric: set the target first");
         return EVT_ERR_STATE;
     }
+    c->metric_queued = false;
     prof_begin(c, EVT_K_OTHER, 0);
     int r = launch_apply_pending(c);
-    if (r == EVT_OK) r = launch_eval_metric(c, metric, reinterpret_cast<double *>(c->h_stage_dev));
+    if (r == EVT_OK) r = launch_eval_metric(c, metric, c->metric_host);
     prof_end(c);
     if (r != EVT_OK) return r;
-    HIPCHK(hipStreamSynchronize(c->stream));
-    c->pt_busy = false;
-    memcpy(value_out, c->h_stage, sizeof(double));
+    c->metric_queued = true;
     return EVT_OK;
+    });
+}
+
+extern "C" int evt_eval_metric_end(evt_handle c, double *value_out) {
+    return guarded([&]() -> int {
+    ARGCHK(c != nullptr, "handle is NULL");
+    ARGCHK(value_out, "value_out is NULL");
+    HIPCHK(hipSetDevice(c->device));
+    if (!c->metric_queued) {
+        evt_set_error("evt_eval_metric_end without evt_eval_metric_begin");
+        return EVT_ERR_STATE;
+    }
+    HIPCHK(hipStreamSynchronize(c->stream));
+    c->metric_queued = false;
+    c->pt_busy = false;
+    *value_out = *c->metric_host;
+    return EVT_OK;
+    });
+}
+
+extern "C" int evt_eval_metric(evt_handle c, int32_t metric, double *value_out) {
+    return guarded([&]() -> int {
+    ARGCHK(c != nullptr, "handle is NULL");
+    ARGCHK(value_out, "value_out is NULL");
+    const int r = evt_eval_metric_begin(c, metric);
+    return r == EVT_OK ? evt_eval_metric_end(c, value_out) : r;
     });
 }
 

@@ -187,6 +187,8 @@ struct evt_ctx {
     int q_cur, q_tree;
     bool quant_pending;  // the gradients' fixed-point words are still to be made: by the next tree's first kernel, or by k_quantize
     double *metric_partial; // [2 * EVT_METRIC_BLOCKS + 1] evaluation-metric partial sums, then how many blocks have left theirs (zero between launches)
+    double *metric_host; // pinned: the metric, and whether one is queued that has not been collected
+    bool metric_queued;
     int64_t *stats;    // [D+1] rows built per level
     int32_t *errflag;  // device-side validation flag
     double *ogains;    // oblivious: [maxlvl][F][B]

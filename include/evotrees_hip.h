@@ -293,6 +293,11 @@ int evt_predict_tree(evt_handle h, int32_t nnodes_tree, const int64_t *feat, con
  * new tree is added with evt_predict_tree, then this call returns the metric.  The sum order is
  * fixed, so the result is bit-reproducible. */
 int evt_eval_metric(evt_handle h, int32_t metric, double *value_out);
+/* The same in two halves: the first queues the metric of the predictions as they stand and returns, the second waits for the metric
+ * queued last (EVT_ERR_STATE without one) - the host queues a training round's next tree in between.  What is queued on the handle
+ * after the first half does not change the value. */
+int evt_eval_metric_begin(evt_handle h, int32_t metric);
+int evt_eval_metric_end(evt_handle h, double *value_out);
 
 /* ---- read-back of cache state (parity tests, callbacks) ------------------------------ */
 /* The cache's binned matrix (nobs x nfeats column-major), e.g. after evt_binarize_f64. */
