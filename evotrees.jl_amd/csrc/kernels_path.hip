@@ -119,44 +119,6 @@ __device__ __forceinline__ void path_grads(int loss, float *pr, float y, float w
 #undef PATH_GRAD
 }
 
-// The highest gain over the lanes and, of equal ones, the lowest order; NO_BIN where no lane has a gain.  ROW: the first 16 lanes' only.  The maximum alone goes through the
-// moves; which lane has it is a ballot.
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ double max_move_f64(double g) {
-    const long long v = __double_as_longlong(g);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(v & 0xffffffffll), CTRL, ROW_MASK, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp((int)0xFFF00000, (int)(v >> 32), CTRL, ROW_MASK, 0xf, false); // -inf
-    const double o = __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-    return o > g ? o : g;
-}
-template <bool ROW>
-__device__ __forceinline__ int path_best(double gain, int order, double &best) {
-    double m = gain;
-    m = max_move_f64<0x111, 0xf>(m); // row_shr:1
-    m = max_move_f64<0x112, 0xf>(m); // row_shr:2
-    m = max_move_f64<0x114, 0xf>(m); // row_shr:4
-    m = max_move_f64<0x118, 0xf>(m); // row_shr:8
-    if (!ROW) {
-        m = max_move_f64<0x142, 0xa>(m); // row_bcast:15 into rows 1 and 3
-        m = max_move_f64<0x143, 0xc>(m); // row_bcast:31 into rows 2 and 3
-    }
-    best = __longlong_as_double(readlane_i64(__double_as_longlong(m), ROW ? 15 : 63));
-    unsigned long long who = __ballot(order != NO_BIN && gain == best);
-    if (ROW) who &= 0xFFFFull;
-    int o = NO_BIN;
-    while (who) { // one, but for ties
-        const int v = __builtin_amdgcn_readlane(order, __builtin_ctzll(who));
-        o = v < o ? v : o;
-        who &= who - 1ull;
-    }
-    return o;
-}
-
-// Requests every 64-byte line of the arguments' head at once: read where each is needed, they were as many trips one after the other.
-__device__ __forceinline__ void touch_args(const PathArgs &A) {
-    asm volatile("" ::"s"(A.xcm), "s"(A.js), "s"(A.status), "s"(A.qbits), "s"(A.tree.packed), "s"(A.pred), "s"(A.seed), "s"(A.cond), "s"(A.feat[0]), "s"(A.feat[16]));
-}
-
 // What bounds it: chains, not bytes.  Everything of a row that the levels need - the sampled features' bins side by side, its words - is brought to LDS once, so that a
 // level is two barriers and what lies between: list, record and words out of LDS and into the histograms, the sums and gains of a wavefront, two maxima.
 template <int NAG, int BPL, bool PACK>
@@ -170,7 +132,7 @@ __global__ __launch_bounds__(1024) void k_small_path(PathArgs A) {
     __shared__ double s_S[NK], s_gain_p;  // statistics and gain of the path's node, below the root
     __shared__ int s_len[2], s_in[2];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    touch_args(A);
+    touch_kernargs<sizeof(PathArgs)>();
     const int b = blockIdx.x, B = A.B, N = A.N, nfs = A.nfs, splits = A.D - 1, words = nfs * NA * B, pieces = (nfs + 15) >> 4;
     // [row][piece] of 16 bytes.  A record starts with another feature of the sample from row to row (byte t: feature (row + t) % nfs), so that lanes that add the
     // same byte of their rows add to different features: lanes that add to one bin wait for each other, and of one feature's 64 bins 64 lanes share many (4000 rows x
@@ -458,8 +420,9 @@ __global__ __launch_bounds__(1024) void k_small_path(PathArgs A) {
                 }
             }
         }
-        double bg;
-        int order = path_best<false>(lg, lo, bg);
+        double bg = lg;
+        int order = lo;
+        wave_argmax(bg, order);
         if (order == NO_BIN ? lane == 0 : lo == order) { // an order names one lane
             s_cand[wave].gain = order == NO_BIN ? -INFINITY : bg;
             s_cand[wave].order = order;
@@ -467,7 +430,9 @@ __global__ __launch_bounds__(1024) void k_small_path(PathArgs A) {
             for (int a = 0; a < NAG; a++) s_cand[wave].left[a] = lq[a];
         }
         __syncthreads();
-        order = path_best<true>(s_cand[lane & 15].gain, s_cand[lane & 15].order, bg);
+        bg = s_cand[lane & 15].gain;
+        order = s_cand[lane & 15].order;
+        wave_argmax<true>(bg, order);
         found = order != NO_BIN && bg > A.gamma;
         jw = found ? order >> 8 : 0;
         fw = A.feat[jw];

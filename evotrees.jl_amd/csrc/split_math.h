@@ -34,32 +34,63 @@ __device__ __forceinline__ long long readlane_i64(long long x, int lane) {
 // Sum over the wavefront, in every lane: the scan's last lane (VALU moves; twelve cross-lane shuffles are as many trips through the LDS crossbar)
 __device__ __forceinline__ long long wave_sum_i64(long long x) { return readlane_i64(wave_incl_scan_i64(x), 63); }
 
-// Arg-max over the 64 lanes of a wavefront: highest gain, of equal gains the lowest bin; every lane gets the result.
-// Same data movement as the prefix scan above (row shifts, then row broadcasts; a lane without a source combines with
-// the identity), so the reduction ends in lane 63 - VALU moves only, where a butterfly of cross-lane shuffles goes
-// through the LDS crossbar eighteen times, each a dependent round trip.
+// Maximum over the 64 lanes of a wavefront (ROW: over the first 16), no value a NaN: the scan's moves, a lane without a source meeting itself.
 template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ void argmax_step(double &g, int &b) {
-    const long long gb = __double_as_longlong(g);
-    const int olo = __builtin_amdgcn_update_dpp(0, (int)(gb & 0xffffffffll), CTRL, ROW_MASK, 0xf, false);
-    const int ohi = __builtin_amdgcn_update_dpp((int)0xFFF00000, (int)(gb >> 32), CTRL, ROW_MASK, 0xf, false); // -inf
-    const int ob = __builtin_amdgcn_update_dpp(NO_BIN, b, CTRL, ROW_MASK, 0xf, false);
-    const double og = __longlong_as_double(((long long)ohi << 32) | (unsigned int)olo);
-    if (og > g || (og == g && ob < b)) { g = og; b = ob; }
+__device__ __forceinline__ double max_step_f64(double g) {
+    const long long v = __double_as_longlong(g);
+    const int lo = (int)(v & 0xffffffffll), hi = (int)(v >> 32);
+    const double o = __longlong_as_double(((long long)__builtin_amdgcn_update_dpp(hi, hi, CTRL, ROW_MASK, 0xf, false) << 32) |
+                                          (unsigned int)__builtin_amdgcn_update_dpp(lo, lo, CTRL, ROW_MASK, 0xf, false));
+    double m;
+    asm("v_max_f64 %0, %1, %2" : "=v"(m) : "v"(g), "v"(o)); // fmax first makes a quiet NaN of either that is a signalling one
+    return m;
 }
-__device__ __forceinline__ void wave_argmax(double &g, int &b) {
-    argmax_step<0x111, 0xf>(g, b); // row_shr:1
-    argmax_step<0x112, 0xf>(g, b); // row_shr:2
-    argmax_step<0x114, 0xf>(g, b); // row_shr:4
-    argmax_step<0x118, 0xf>(g, b); // row_shr:8
-    argmax_step<0x142, 0xa>(g, b); // row_bcast:15 into rows 1 and 3
-    argmax_step<0x143, 0xc>(g, b); // row_bcast:31 into rows 2 and 3
-    const long long gb = __double_as_longlong(g);
-    const int lo = __builtin_amdgcn_readlane((int)(gb & 0xffffffffll), 63), hi = __builtin_amdgcn_readlane((int)(gb >> 32), 63);
-    g = __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-    b = __builtin_amdgcn_readlane(b, 63);
+template <bool ROW = false>
+__device__ __forceinline__ double wave_max_f64(double g) {
+    g = max_step_f64<0x111, 0xf>(g); // row_shr:1
+    g = max_step_f64<0x112, 0xf>(g); // row_shr:2
+    g = max_step_f64<0x114, 0xf>(g); // row_shr:4
+    g = max_step_f64<0x118, 0xf>(g); // row_shr:8
+    if (!ROW) {
+        g = max_step_f64<0x142, 0xa>(g); // row_bcast:15 into rows 1 and 3
+        g = max_step_f64<0x143, 0xc>(g); // row_bcast:31 into rows 2 and 3
+    }
+    return __longlong_as_double(readlane_i64(__double_as_longlong(g), ROW ? 15 : 63));
+}
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ int min_step(int v) {
+    const int o = __builtin_amdgcn_update_dpp(v, v, CTRL, ROW_MASK, 0xf, false);
+    return o < v ? o : v;
 }
 
+// Arg-max over the 64 lanes of a wavefront (ROW: the first 16): highest gain, of equal gains the lowest bin (NO_BIN: no gain); every lane gets the result.
+// The maximum alone goes through the moves; which lane has it is a ballot, and the lowest bin is looked for only where several have it.  Gain and bin taken
+// through the moves together cost 80 instructions for 45 (deep levels of the split search, whose wavefronts' instructions are what they take: ARGMAX_FIG).
+template <bool ROW = false>
+__device__ __forceinline__ void wave_argmax(double &g, int &b) {
+    const double m = wave_max_f64<ROW>(g);
+    unsigned long long who = __ballot(g == m && b != NO_BIN);
+    if (ROW) who &= 0xFFFFull;
+    if (who == 0ull) {
+        g = m;
+        b = NO_BIN;
+        return;
+    }
+    if (who & (who - 1ull)) {
+        int v = (who >> (threadIdx.x & 63)) & 1ull ? b : NO_BIN;
+        v = min_step<0x111, 0xf>(v);
+        v = min_step<0x112, 0xf>(v);
+        v = min_step<0x114, 0xf>(v);
+        v = min_step<0x118, 0xf>(v);
+        v = min_step<0x142, 0xa>(v);
+        v = min_step<0x143, 0xc>(v);
+        const int lowest = __builtin_amdgcn_readlane(v, 63);
+        who &= __ballot(b == lowest);
+    }
+    const int lane = __builtin_ctzll(who);
+    g = __longlong_as_double(readlane_i64(__double_as_longlong(g), lane));
+    b = __builtin_amdgcn_readlane(b, lane);
+}
 
 // ---- Float64 gain algebra, expression order as in the reference ------------------------------
 __device__ __forceinline__ double term_gh(double g, double h, double w, double lambda, double L2) {
