@@ -137,7 +137,7 @@ __device__ __forceinline__ void zero_children_slices(const ScanArgs &A, int n) {
 // (scan_finish): one launch per level instead of two where a level is a chain of small kernels.
 template <int NAG, int BPL, bool FUSED>
 __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
     const int n = (1 << (A.level - 1)) + blockIdx.x; // 1-based node id
     // The block's time is a chain of round trips to memory, so requests go out in as few dependent steps as the data
     // allows: node state and feature id first; then, in one batch of unconditional loads, the histogram slices, the
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
     const int jpc = have ? jp : A.nfs - 1;
     int f = (int)A.js[jpc] - 1;
     const int st = A.status[n];
-    asm volatile("" : "+v"(f)); // the feature id is requested ahead of the branch on the node state, not behind it
+    asm volatile("" : "+s"(f)); // the feature id is requested ahead of the branch on the node state, not behind it
     if (st != ST_BUILD && st != ST_SUBTRACT) return;
     const bool is_sub = (st == ST_SUBTRACT);
     // the channel layout fixes the outputs: two-output MLE losses have five channels, every other shape here one output
@@ -245,9 +245,6 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
 
     double wbest = -INFINITY;
     int wjp = NO_BIN, wbin = NO_BIN;
-    long long wq[NAG];
-#pragma unroll
-    for (int ag = 0; ag < NAG; ag++) wq[ag] = 0;
     const int nodeidx = blockIdx.x;
 
     if (have) {
@@ -322,12 +319,10 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
             wave_argmax(lg, lb);
             if (lg > wbest) { wbest = lg; wjp = jp; wbin = lb; }
             if constexpr (!FUSED) {
-                // the lane that holds the winning bin hands its left totals to the whole wave
-                const int owner = (lb != NO_BIN) ? (lb - 1) / BPL : 0;
+                // the lane that holds the winning bin hands its left totals over
+                if (lane == (lb != NO_BIN ? (lb - 1) / BPL : 0)) {
 #pragma unroll
-                for (int ag = 0; ag < NAG; ag++) {
-                    const int lo = __shfl((int)(lq[ag] & 0xffffffffll), owner), hi = __shfl((int)(lq[ag] >> 32), owner);
-                    wq[ag] = ((long long)hi << 32) | (unsigned int)lo;
+                    for (int ag = 0; ag < NAG; ag++) s_wq[wave][ag] = lq[ag];
                 }
             }
         }
@@ -337,18 +332,19 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
     if (lane == 0) {
         s_wg[wave] = wbest; s_wjp[wave] = wjp; s_wbin[wave] = wbin;
         s_wfeat[wave] = numeric ? f + 1 : -(f + 1);
-        if constexpr (!FUSED) {
-#pragma unroll
-            for (int ag = 0; ag < NAG; ag++) s_wq[wave][ag] = wq[ag];
-        }
     }
     __syncthreads();
     double bg = -INFINITY;
     int bj = NO_BIN, bb = NO_BIN, bw = 0;
-    if (tid == 0) {
-        for (int w = 0; w < nwaves; w++) {
-            if (s_wg[w] > bg || (s_wg[w] == bg && s_wjp[w] < bj)) { bg = s_wg[w]; bj = s_wjp[w]; bb = s_wbin[w]; bw = w; }
-        }
+    if (tid == 0) { // the waves' features ascend: only a strictly larger gain replaces an earlier one
+        constexpr int NW = FUSED ? 16 : 4;
+        double g[NW]; // all of them in one trip to LDS
+#pragma unroll
+        for (int w = 0; w < NW; w++) g[w] = s_wg[w];
+#pragma unroll
+        for (int w = 0; w < NW; w++)
+            if (g[w] > bg) { bg = g[w]; bw = w; }
+        if (bg > -INFINITY) { bj = s_wjp[bw]; bb = s_wbin[bw]; }
     }
     if constexpr (FUSED) {
         // the node is finished here: wave jp scanned sampled feature jp, so the winner's left totals are still in the
@@ -757,7 +753,7 @@ __global__ __launch_bounds__(NAG * BPL > 12 ? 512 : 1024) void k_obliv_level(Obl
     __shared__ double s_best;
     const OblivArgs &A = L.o;
     touch_kernargs<sizeof(OblivLevelArgs)>();
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
     constexpr int K = (NAG == 5) ? 2 : 1, NK = 2 * K + 1;
     const int B = A.B, jp = blockIdx.x;
     // all nodes of a level split on the same feature or none does: the level's nodes are all active, or none is
@@ -1048,7 +1044,7 @@ struct ChannelWords {
 template <int BPL, bool LOOP>
 __global__ __launch_bounds__(64 * (EVT_MAX_K / 2)) void k_scan_mc(ScanArgs A) {
     extern __shared__ double s_term[]; // [K][B]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
     touch_kernargs<sizeof(ScanArgs)>();
     const int nodeidx = blockIdx.x, n = (1 << (A.level - 1)) + nodeidx, jp = blockIdx.y;
     int f = (int)A.js[jp] - 1;
