@@ -19,7 +19,7 @@
 #define ST_LEAF 4     // scanned (or last level), leaf
 
 #define EVT_CHUNK 2048        // rows per partition chunk (8 per thread of a 256-thread block); part_chunk_rows() gives the levels of the one-pass form up to
-#define EVT_CHUNK_MAX 8192    // this many
+#define EVT_CHUNK_MAX 16384   // this many
 #define EVT_CHUNK_WORDS 32    // 64-bit ballot words per chunk
 #define EVT_MAX_NK 5  // gradient rows of the one- and two-output losses (register arrays of the specialised kernels)
 #define EVT_MAX_NA 5

@@ -18,6 +18,7 @@
 // No host round trip is needed between levels.
 #include "grad_math.h"
 #include <algorithm>
+#include <type_traits>
 
 // largest i in [0, n) with pre[i] <= v   (pre ascending, pre[0] <= v): the number of such entries, less one.  Every
 // wavefront counts them for itself, 64 entries per step, all loads independent: one trip to memory where a binary
@@ -626,17 +627,25 @@ __global__ __launch_bounds__(256) void k_part_scatter(PartArgs A, NextArgs NX) {
     }
 }
 
+// p's element at a byte offset
+template <typename V>
+__device__ __forceinline__ V &at_offset(V *p, uint32_t bytes) {
+    return *reinterpret_cast<V *>(reinterpret_cast<char *>(const_cast<std::remove_const_t<V> *>(p)) + bytes);
+}
+
 // The partition of a level in one pass: a block decides its chunk's rows, claims as many places of either child with one addition to the
 // node's cursor, and writes the row ids there.  A chunk's rows keep their order; the chunks of a node follow each other in the order of
 // their claims, which nothing depends on: sums are integers, leaves are recorded by row id.  A wavefront owns NI * 64 neighbouring
 // positions, so that one total per wavefront is all that is exchanged.
-// Bound by its chain of trips to memory (descriptor, row ids and node, decision words, claim, stores) below a million rows, by the lists
-// and, deeper, the decision words' lines above.  us a level, count + scan of the counts + scatter -> this: 800k rows x 28 features, depth 8
-// 5.2 + 6.5 -> 7.4; 500k of 100 4.7 + 5.9 -> 7.5; 10M x 100, depth 11, root 17 + 5 + 19 -> 32, level 5 18 + 5 + 18 -> 35, level 9 33 + 5 + 19 -> 46.
+// Bound by its chain of trips to memory (descriptor, row ids and node, decision words, claim, stores) below a million rows; above, by the claims of a node of
+// many chunks, by the lists and, deeper, the decision words' lines.  A chunk's numbers are in scalar registers and a lane's addresses offsets from them, which takes
+// a third of the registers (97 -> 64 for 16 rows a thread) and twice the wavefronts.  us a level, count + scan of the counts + scatter -> one pass -> this: 800k
+// rows x 28 features, depth 8 5.2 + 6.5 -> 7.4 -> 7.1; 500k of 100 4.7 + 5.9 -> 6.3 -> 6.2; 10M x 100, depth 11, root 17 + 5 + 19 -> 32 -> 26, level 5 18 + 5 + 18 -> 36 -> 35, level 9 33 + 5 +
+// 19 -> 45 -> 43.
 template <bool NT, int T, int NI>
-__global__ __launch_bounds__(T) void k_part_move(PartArgs A, NextArgs NX) {
+__global__ __launch_bounds__(T, 8) void k_part_move(PartArgs A, NextArgs NX) {
     constexpr int W = T / 64, CHUNK = NI * T;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __shared__ long long s_tmp[34];
     __shared__ int s_cnt[W];
     __shared__ unsigned long long s_claim;
@@ -651,37 +660,43 @@ __global__ __launch_bounds__(T) void k_part_move(PartArgs A, NextArgs NX) {
     const int64_t n_chunks = A.hdr[LH_N_CHUNKS];
     asm volatile("" : "+v"(cd.x), "+v"(cd.y), "+v"(cd.z), "+v"(cd.w)); // requested with the level's chunk count, not behind the branch on it
     for (int64_t c = blockIdx.x - 1; c < n_chunks; c += G, cd = A.cdesc[c < n_chunks ? c : 0]) {
-        const int n = (int)cd.x;
-        const uint32_t p0 = cd.y, pend = cd.z, seg = p0 - (uint32_t)(c - cd.w) * CHUNK; // positions are 32-bit numbers, as the row ids
+        // a chunk's numbers are the block's, in scalar registers: a lane's addresses are 32-bit offsets from them
+        const int n = __builtin_amdgcn_readfirstlane((int)cd.x);
+        const uint32_t p0 = __builtin_amdgcn_readfirstlane((int)cd.y), pend = __builtin_amdgcn_readfirstlane((int)cd.z), c0 = __builtin_amdgcn_readfirstlane((int)cd.w);
+        const uint32_t seg = p0 - (uint32_t)(c - c0) * CHUNK;                             // positions are 32-bit numbers, as the row ids
         const uint32_t left_of = pend - p0, wofs = wave * (NI * 64) + lane;               // rows from the chunk's first on; this lane's first
         const uint32_t *isp = A.is_cur + p0;
         uint32_t rid[NI], xbv[NI];
 #pragma unroll
-        for (int it = 0; it < NI; it++) rid[it] = isp[wofs + it * 64 < left_of ? wofs + it * 64 : left_of - 1];
-        const int st = A.status[n];
-        uint32_t nd = A.t_packed[n - 1]; // requested with the state, not behind the branch on it
-        uint32_t nl = (uint32_t)A.node_sum[(int64_t)(2 * n) * A.NAg + A.NAg - 1];
-        asm volatile("" : "+v"(nd), "+v"(nl));
+        for (int it = 0; it < NI; it++) rid[it] = at_offset(isp, 4u * (wofs + it * 64 < left_of ? wofs + it * 64 : left_of - 1));
+        int stv = A.status[n];
+        uint32_t ndv = A.t_packed[n - 1]; // requested with the state, not behind the branch on it
+        uint32_t nlv = (uint32_t)A.node_sum[(int64_t)(2 * n) * A.NAg + A.NAg - 1];
+        asm volatile("" : "+v"(stv), "+v"(ndv), "+v"(nlv));
+        const int st = __builtin_amdgcn_readfirstlane(stv);
+        const uint32_t nd = __builtin_amdgcn_readfirstlane((int)ndv), nl = __builtin_amdgcn_readfirstlane((int)nlv);
         if (st == ST_SPLIT) {
             const int f = (int)(nd & 0xFFFFu) - 1;
             const uint32_t cb = (nd >> 16) & 0xFFu;
             const bool numeric = (nd & EVT_NODE_NUMERIC) != 0;
             const uint8_t *col = A.xcm + (size_t)f * A.N;
-            const uint32_t *plane = (A.planes && numeric && cb >= 1u && cb < (uint32_t)A.B) ? A.planes + ((size_t)f * (A.B - 1) + (cb - 1)) * A.plane_words : nullptr;
+            const bool plane = A.planes && numeric && cb >= 1u && cb < (uint32_t)A.B;
+            uint32_t lefts_of = 0; // bit it: the lane's row of step it goes left
             if (plane) {
+                const uint32_t *words = A.planes + ((size_t)f * (A.B - 1) + (cb - 1)) * A.plane_words;
 #pragma unroll
-                for (int it = 0; it < NI; it++) xbv[it] = load_decision<NT>(nullptr, plane, rid[it]);
+                for (int it = 0; it < NI; it++) xbv[it] = NT ? __builtin_nontemporal_load(&at_offset(words, (rid[it] >> 5) * 4u)) : at_offset(words, (rid[it] >> 5) * 4u);
+#pragma unroll
+                for (int it = 0; it < NI; it++) lefts_of |= (wofs + it * 64 < left_of ? (xbv[it] >> (rid[it] & 31u)) & 1u : 0u) << it;
             } else {
 #pragma unroll
-                for (int it = 0; it < NI; it++) xbv[it] = load_decision<NT>(col, nullptr, rid[it]);
+                for (int it = 0; it < NI; it++) xbv[it] = NT ? __builtin_nontemporal_load(&at_offset(col, rid[it])) : at_offset(col, rid[it]);
+#pragma unroll
+                for (int it = 0; it < NI; it++) lefts_of |= (uint32_t)(wofs + it * 64 < left_of && (numeric ? xbv[it] <= cb : xbv[it] == cb)) << it;
             }
-            unsigned long long bal[NI];
             int cnt = 0;
 #pragma unroll
-            for (int it = 0; it < NI; it++) {
-                bal[it] = __ballot(wofs + it * 64 < left_of && decide_left(xbv[it], plane != nullptr, rid[it], numeric, cb));
-                cnt += __popcll(bal[it]);
-            }
+            for (int it = 0; it < NI; it++) cnt += __popcll(__ballot((lefts_of >> it) & 1u));
             if (lane == 0) s_cnt[wave] = cnt;
             __syncthreads();
             int lefts = 0, before = 0; // of the chunk, of the wavefronts before this one
@@ -694,16 +709,20 @@ __global__ __launch_bounds__(T) void k_part_move(PartArgs A, NextArgs NX) {
             const int rows = (int)(left_of < (uint32_t)CHUNK ? left_of : (uint32_t)CHUNK);
             if (tid == 0) s_claim = atomicAdd(A.cursor + EVT_CURSOR_SLOT(n), (unsigned long long)lefts | ((unsigned long long)(rows - lefts) << 32));
             __syncthreads();
-            const unsigned long long claim = s_claim;
-            uint32_t dL = seg + (uint32_t)claim + before, dR = seg + nl + (uint32_t)(claim >> 32) + (wave * (NI * 64) - before);
+            before = __builtin_amdgcn_readfirstlane(before);
+            const uint32_t claim_l = __builtin_amdgcn_readfirstlane((int)(uint32_t)s_claim), claim_r = __builtin_amdgcn_readfirstlane((int)(uint32_t)(s_claim >> 32));
+            uint32_t *out_l = A.is_next + (seg + claim_l + before), *out_r = A.is_next + (seg + nl + claim_r + (wave * (NI * 64) - before));
 #pragma unroll
             for (int it = 0; it < NI; it++) {
-                const int lrank = __popcll(bal[it] & ((1ull << lane) - 1ull));
-                const bool left = (bal[it] >> lane) & 1ull;
-                if (wofs + it * 64 < left_of) A.is_next[left ? dL + lrank : dR + (lane - lrank)] = rid[it];
-                const int k = __popcll(bal[it]);
-                dL += k;
-                dR += 64 - k;
+                const bool left = (lefts_of >> it) & 1u;
+                const unsigned long long bal = __ballot(left);
+                const uint32_t lrank = __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+                if (left) at_offset(out_l, 4u * lrank) = rid[it];
+                asm volatile(""); // two stores from scalar addresses, not one from an address chosen by the lane
+                if (!left && wofs + it * 64 < left_of) at_offset(out_r, 4u * (lane - lrank)) = rid[it];
+                const int k = __popcll(bal);
+                out_l += k;
+                out_r += 64 - k;
             }
         } else if (st == ST_LEAF && (A.write_nidx || A.fuse_pred)) { // rows of a node that stops here, as in k_part_scatter
             for (uint32_t k = tid; k < (uint32_t)CHUNK && k < left_of; k += T) {
@@ -1119,13 +1138,14 @@ static bool part_in_one_pass(const evt_ctx *c) { return c->part_one_pass && c->u
 
 // Rows of a chunk of the level.  A node's chunks queue at its cursor, ~20 ns each: where a node has more than 128 of them they grow (us a level of
 // 1M rows, 2048 | 4096 | 8192 rows a chunk: root 11.7 | 8.9 | 9.0, two nodes 9.0 | 7.6 | 8.4, eight 6.8 | 6.8 | 8.3; 10M: 67 | 39 | 28, 62 | 36 | 28,
-// 34 | 28 | 23).  They grow too where the level is more blocks than the chip holds at once and nodes are many chunks (10M rows, 64 nodes 44 | - | 40).
+// 34 | 28 | 23; 8192 | 16384, blocks of 1024: one to four nodes 31 | 26, 29 | 24, 29 | 26, eight 30 | 34, whose nodes of 1.25M rows keep the narrower).  They grow too where the level is more blocks than the chip holds at once and nodes are many chunks (10M rows, 64 nodes 44 | - | 40).
 int part_chunk_rows(const evt_ctx *c, int level) {
     int rows = EVT_CHUNK;
     if (!part_in_one_pass(c) || level >= c->D - 1) return rows;
     const int64_t per_node = (c->last_all_rows ? c->N : c->N * (c->last_cond + 1) / 256) >> (level - 1);
     const int64_t all = per_node << (level - 1);
-    while (rows < EVT_CHUNK_MAX && (per_node > (int64_t)rows * 128 || (all > (int64_t)rows * 2048 && per_node >= (int64_t)rows * 16))) rows *= 2;
+    while (rows < EVT_CHUNK_MAX / 2 && (per_node > (int64_t)rows * 128 || (all > (int64_t)rows * 2048 && per_node >= (int64_t)rows * 16))) rows *= 2;
+    if (rows == EVT_CHUNK_MAX / 2 && per_node > (int64_t)rows * 256) rows = EVT_CHUNK_MAX;
     return rows;
 }
 
@@ -1181,7 +1201,7 @@ int launch_part_scatter(evt_ctx *c, int level, const uint32_t *is_cur, uint32_t 
         if (A.stream_hint) hipLaunchKernelGGL((k_part_move<true, T_, NI_>), grid, dim3(T_), 0, c->stream, A, NX);    \
         else hipLaunchKernelGGL((k_part_move<false, T_, NI_>), grid, dim3(T_), 0, c->stream, A, NX);                 \
     }
-        PMCASE(256, 8) PMCASE(512, 8) PMCASE(512, 16)
+        PMCASE(256, 8) PMCASE(512, 8) PMCASE(512, 16) PMCASE(1024, 16)
 #undef PMCASE
         HIPCHK(hipGetLastError());
         return EVT_OK;
