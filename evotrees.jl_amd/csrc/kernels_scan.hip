@@ -77,8 +77,9 @@ __device__ __forceinline__ void root_totals(const ScanArgs &A, int n, const long
 // The decision for one node (get_best_split's threshold, src/fit-utils.jl:444-450; the Tree arrays, src/fit.jl:96-103;
 // a node without a split becomes a leaf, src/predict.jl:198-262): thread 0 holds the node's best candidate (bg, bj, bb)
 // and its feature (1-based id, type); S: the node's statistics (in shared memory).  Leaves {found, bj, bb} in s_dec.
+template <int NAG>
 __device__ __forceinline__ void scan_decide(const ScanArgs &A, int n, const double *S, int *s_dec, double bg, int bj, int bb, int feat, bool numeric) {
-    const int K = A.K;
+    constexpr int K = NAG == 5 ? 2 : 1; // the channel layout names the outputs
     const int found = (bb != NO_BIN && bg > A.gamma) ? 1 : 0;
     s_dec[0] = found; s_dec[1] = bj; s_dec[2] = bb;
     if (found) {
@@ -99,7 +100,7 @@ __device__ __forceinline__ void scan_decide(const ScanArgs &A, int n, const doub
 // and state are written here too - what the leaf-level pass would compute from node_sum (same integers, same expressions).
 template <int NAG>
 __device__ __forceinline__ void write_children(const ScanArgs &A, int n, const long long *qL, const long long *s_Sq, const double *s_sc) {
-    const int NK = A.NK, K = A.K;
+    constexpr int K = NAG == 5 ? 2 : 1, NK = 2 * K + 1;
 #pragma unroll
     for (int child = 0; child < 2; child++) {
         const int cn = 2 * n + child;
@@ -110,7 +111,7 @@ __device__ __forceinline__ void write_children(const ScanArgs &A, int n, const l
             A.node_sum[(int64_t)cn * NAG + ag] = qc[ag];
         }
         if (A.fold_leaves) {
-            double v[EVT_MAX_NK];
+            double v[NK];
             decode_vals(qc, s_sc, A.loss, NK, v);
             A.tree.w[cn - 1] = (float)v[NK - 1];
             for (int k = 0; k < K; k++) A.tree.pred[(int64_t)K * (cn - 1) + k] = (float)leaf_value(A.loss, v, k, K, A.eta, A.bagging, A.lambda, A.L2);
@@ -352,7 +353,7 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
         if (tid == 0) {
             A.tree.w[n - 1] = (float)S[NK - 1];
             const int wf = (bb != NO_BIN) ? s_wfeat[bj] : 1;
-            scan_decide(A, n, s_S, s_dec, bg, bj, bb, wf < 0 ? -wf : wf, wf > 0);
+            scan_decide<NAG>(A, n, s_S, s_dec, bg, bj, bb, wf < 0 ? -wf : wf, wf > 0);
         }
         __syncthreads();
         if (!s_dec[0]) return;
@@ -434,7 +435,7 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
             A.counts[(size_t)nodeidx * EVT_SCAN_COUNT_STEP] = 0;
             A.tree.w[n - 1] = (float)S[NK - 1];
             const int feat = found ? (mine.feat < 0 ? -mine.feat : mine.feat) : 1;
-            scan_decide(A, n, S, s_dec, g, j, found ? mine.bin : NO_BIN, feat, found ? mine.feat > 0 : true);
+            scan_decide<NAG>(A, n, S, s_dec, g, j, found ? mine.bin : NO_BIN, feat, found ? mine.feat > 0 : true);
             if (found) {
                 write_children<NAG>(A, n, mine.qL, nsq, sc);
             }
@@ -565,7 +566,7 @@ __global__ __launch_bounds__(256) void k_scan_fin(ScanArgs A, int ngroups) {
     const bool owner = found ? (mine.jp == bj && mine.bin != NO_BIN) : (tid == 0);
     if (owner) {
         const int feat = found ? (mine.feat < 0 ? -mine.feat : mine.feat) : 1;
-        scan_decide(A, n, s_S, s_dec, bg, bj, bb, feat, found ? mine.feat > 0 : true);
+        scan_decide<NAG>(A, n, s_S, s_dec, bg, bj, bb, feat, found ? mine.feat > 0 : true);
         if (found) {
             long long qL[NAG];
 #pragma unroll
