@@ -353,7 +353,7 @@ __host__ __device__ __forceinline__ uint32_t evt_pack_node(int feat, int cond_bi
 // Requests every 64-byte line of a kernel's arguments (BYTES of them) at once.  The compiler loads an argument where it is first needed, behind the branches before it, and
 // each line so found is a trip to memory that nothing else hides: a launch's arguments are in no cache.  us a launch, with a chunk's descriptor requested beside the chunk
 // count: k_part_move 6.2 -> 5.9 (500k rows) and 7.3 -> 7.0 (800k), k_part_count 4.5 -> 4.3, k_part_scatter 5.0 -> 4.6, k_final_fused 5.8 -> 5.3 (60k), k_scan_mc 9.5 -> 9.2,
-// k_obliv_level 9.6 -> 9.3, k_tree_begin 8.3 -> 8.1; k_scan and the histogram kernels gain nothing by it.
+// k_obliv_level 9.6 -> 9.3, k_tree_begin 8.3 -> 8.1; k_scan 6.05 -> 5.8 once its first requests wait for no argument; the histogram kernels gain nothing by it.
 template <size_t BYTES>
 __device__ __forceinline__ void touch_kernargs() {
     constexpr int LAST = (int)(BYTES - 4) / 64;

@@ -136,28 +136,33 @@ __device__ __forceinline__ void zero_children_slices(const ScanArgs &A, int n) {
 // and, for subtract nodes, materialises h[n] = h[parent] - h[sibling].
 // FUSED: one block of 16 waves per node covers every sampled feature (at most 16) and finishes the node itself
 // (scan_finish): one launch per level instead of two where a level is a chain of small kernels.
+// What the first requests are made from comes as arguments of its own, ahead of the rest: these are in scalar registers when a wavefront starts (a struct's fields are not), and the
+// rest is on its way beside the feature id and the node's state, which are now one trip (the id was waited for before the state was asked for, and the block's size was a trip of
+// its own).  us a launch: 500k x 100 of 64 bins, half the features, 6.14 -> 5.8 (5.7 to 5.9; without the registers 6.0), 800k x 28 of 128 bins 8.6 -> 8.1 (8.3), 10M x 100 14.1 -> 13.4.
 template <int NAG, int BPL, bool FUSED>
-__global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
-    const int n = (1 << (A.level - 1)) + blockIdx.x; // 1-based node id
+__global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(const uint32_t *js, const int32_t *status, long long *hist, int64_t node_stride, int level, int nfs, int B,
+                                                             ScanArgs A) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int nwaves = FUSED ? 16 : 4;
+    const int n = (1 << (level - 1)) + blockIdx.x; // 1-based node id
     // The block's time is a chain of round trips to memory, so requests go out in as few dependent steps as the data
     // allows: node state and feature id first; then, in one batch of unconditional loads, the histogram slices, the
     // feature's type and constraint, the node totals and the decode scales.
     const int jp = blockIdx.y * nwaves + wave;
-    const bool have = jp < A.nfs; // wave-uniform; a wave past the last feature loads the last one's data and drops it
-    const int jpc = have ? jp : A.nfs - 1;
-    int f = (int)A.js[jpc] - 1;
-    const int st = A.status[n];
-    asm volatile("" : "+s"(f)); // the feature id is requested ahead of the branch on the node state, not behind it
+    const bool have = jp < nfs; // wave-uniform; a wave past the last feature loads the last one's data and drops it
+    const int jpc = have ? jp : nfs - 1;
+    int f = (int)js[jpc], st = status[n];
+    touch_kernargs<48 + sizeof(ScanArgs)>();
+    asm volatile("" : "+s"(f), "+s"(st)); // both are requested before either is waited for, and ahead of the branch on the state
     if (st != ST_BUILD && st != ST_SUBTRACT) return;
+    f -= 1;
     const bool is_sub = (st == ST_SUBTRACT);
     // the channel layout fixes the outputs: two-output MLE losses have five channels, every other shape here one output
     constexpr int K = (NAG == 5) ? 2 : 1, NK = 2 * K + 1;
-    const int B = A.B;
     // BPL = bins per lane = ceil(nbins / 64), a template parameter so that nbins <= 64 keeps one bin per lane in registers
-    long long *hn = A.hist + (int64_t)(n - 1) * A.node_stride;
-    const long long *hp = A.hist + (int64_t)((n >> 1) - 1) * A.node_stride;
-    const long long *hs = A.hist + (int64_t)((n ^ 1) - 1) * A.node_stride;
+    long long *hn = hist + (int64_t)(n - 1) * node_stride;
+    const long long *hp = hist + (int64_t)((n >> 1) - 1) * node_stride;
+    const long long *hs = hist + (int64_t)((n ^ 1) - 1) * node_stride;
 
     __shared__ long long s_Sq[EVT_MAX_NA];
     __shared__ double s_S[EVT_MAX_NK];
@@ -218,7 +223,7 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
     }
 
     // node totals -> Float64 statistics
-    if (A.level == 1) { // the root's totals are any sampled feature's sums over its bins: the wavefront's own (a wavefront past the last feature has none, and no use for them).
+    if (level == 1) { // the root's totals are any sampled feature's sums over its bins: the wavefront's own (a wavefront past the last feature has none, and no use for them).
         // Read again by one wavefront, with two barriers behind it, they took the root's search from 6.5 to 7.8 us (50 features x 64 bins), from 8.9 to 11.4 (28 x 128).
 #pragma unroll
         for (int ag = 0; ag < NAG; ag++) {
@@ -307,7 +312,7 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
                     }
                 }
                 if (A.oblivious) {
-                    A.ogains[((int64_t)nodeidx * A.nfs + jp) * B + b] = ok ? gain : 0.0; // update_gains!
+                    A.ogains[((int64_t)nodeidx * nfs + jp) * B + b] = ok ? gain : 0.0; // update_gains!
                 } else if (ok && gain > lg) {
                     lg = gain;
                     lb = b + 1;
@@ -403,10 +408,10 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(ScanArgs A) {
         }
         // the children's slices start from zero: a wave clears its feature's bins in both, whatever the node turns out to be
         if (A.zero_children && have) {
-            long long *hc = A.hist + (int64_t)(2 * n - 1) * A.node_stride + o0;
+            long long *hc = hist + (int64_t)(2 * n - 1) * node_stride + o0;
             for (int i = lane; i < NAG * B; i += 64) {
                 hc[i] = 0;
-                hc[A.node_stride + i] = 0;
+                hc[node_stride + i] = 0;
             }
         }
         if (wave != 0 || !__builtin_amdgcn_readfirstlane(last)) return;
@@ -1409,18 +1414,19 @@ int launch_scan(evt_ctx *c, int level, const evt_params *p, bool leaf_level) {
     // few sampled features: one block of 16 waves scans a node's features and finishes the node, no second launch
     const bool fused = !leaf_level && !A.oblivious && A.nfs <= 16 && c->scan_fused;
     if (fused) A.last_decides = 0;
+#define SCAN_FIRST A.js, A.status, A.hist, A.node_stride, A.level, A.nfs, A.B
 #define SCASE(NAG_)                                                                                     \
     case NAG_:                                                                                          \
         if (fused) {                                                                                    \
-            if (bpl == 1) hipLaunchKernelGGL((k_scan<NAG_, 1, true>), dim3(nodes), dim3(1024), 0, c->stream, A);      \
-            else if (bpl == 2) hipLaunchKernelGGL((k_scan<NAG_, 2, true>), dim3(nodes), dim3(1024), 0, c->stream, A); \
-            else hipLaunchKernelGGL((k_scan<NAG_, 4, true>), dim3(nodes), dim3(1024), 0, c->stream, A);               \
+            if (bpl == 1) hipLaunchKernelGGL((k_scan<NAG_, 1, true>), dim3(nodes), dim3(1024), 0, c->stream, SCAN_FIRST, A);      \
+            else if (bpl == 2) hipLaunchKernelGGL((k_scan<NAG_, 2, true>), dim3(nodes), dim3(1024), 0, c->stream, SCAN_FIRST, A); \
+            else hipLaunchKernelGGL((k_scan<NAG_, 4, true>), dim3(nodes), dim3(1024), 0, c->stream, SCAN_FIRST, A);               \
             break;                                                                                      \
         }                                                                                               \
         if (!leaf_level) {                                                                              \
-            if (bpl == 1) hipLaunchKernelGGL((k_scan<NAG_, 1, false>), grid, dim3(256), 0, c->stream, A);      \
-            else if (bpl == 2) hipLaunchKernelGGL((k_scan<NAG_, 2, false>), grid, dim3(256), 0, c->stream, A); \
-            else hipLaunchKernelGGL((k_scan<NAG_, 4, false>), grid, dim3(256), 0, c->stream, A);               \
+            if (bpl == 1) hipLaunchKernelGGL((k_scan<NAG_, 1, false>), grid, dim3(256), 0, c->stream, SCAN_FIRST, A);      \
+            else if (bpl == 2) hipLaunchKernelGGL((k_scan<NAG_, 2, false>), grid, dim3(256), 0, c->stream, SCAN_FIRST, A); \
+            else hipLaunchKernelGGL((k_scan<NAG_, 4, false>), grid, dim3(256), 0, c->stream, SCAN_FIRST, A);               \
         }                                                                                               \
         if (leaf_level || (!A.oblivious && !A.last_decides)) hipLaunchKernelGGL(k_scan_fin<NAG_>, dim3(nodes, 1 + zero_blocks), dim3(256), 0, c->stream, A, ngroups); \
         break;
@@ -1431,6 +1437,7 @@ int launch_scan(evt_ctx *c, int level, const evt_params *p, bool leaf_level) {
     default: evt_set_error("unsupported global channel count %d", c->NAg); return EVT_ERR_ARG;
     }
 #undef SCASE
+#undef SCAN_FIRST
     HIPCHK(hipGetLastError());
     return EVT_OK;
 }
