@@ -66,7 +66,7 @@ struct PathCand { // a wavefront's best split of a node
 };
 
 // Nodes of the tree, one to each of a wavefront's first lanes (n: its number, 0 none), to the device's arrays and to the host.  A node's three words go out by three
-// lanes in one instruction: each store on its own is a write of part of a line over the bus (1000 rows x 10, depth 10: a round 85 us, with them together 57).
+// lanes in one instruction: each store on its own is a write of part of a line over the bus (1000 rows x 10, depth 10: a round 85 us, with them together 45).
 template <int K>
 __device__ __forceinline__ void path_put_nodes(const PathArgs &A, int lane, int n, int rows, float w, uint32_t packed, float gain, const float *pred) {
     const uint32_t feat = packed & 0xFFFFu, bin = (packed >> 16) & 0xFFu, split = packed ? 1u : 0u;
