@@ -647,10 +647,11 @@ def fit(config, dtrain=None, x_train=None, y_train=None, w_train=None, offset_tr
             grow_evotree(m, cache, config, more=(i < config.nrounds and (logger is None or not return_cache)))
             if logger is not None:
                 cb.start(m.trees[-1])  # as the reference: only the round's last tree reaches the eval prediction
-                # while the device evaluates the round and grows the tree behind it, the host queues the one after that (one more that early stopping may drop): of small
-                # fits the host is what a round waits for (2000 rows x 10 with 500 eval rows, 100 rounds 5.5 -> 4.5 ms together with cheaper addresses of arrays;
-                # 100k rows, where it is the device, level)
-                if i + 1 < config.nrounds and not return_cache and config.bagging_size == 1 and len(cache.pending) == 1:
+                # while the device evaluates the round and grows the tree behind it, the host queues the one after that: of small fits the host is what a round waits for
+                # (2000 rows x 10 with 500 eval rows, 100 rounds 5.5 -> 4.5 ms together with cheaper addresses of arrays; 100k rows, where it is the device, level).
+                # Not in a round that may be the last by early stopping, which would drop this tree too
+                last = logger["iter_since_best"] + 1 >= logger["early_stopping_rounds"]
+                if i + 1 < config.nrounds and not last and not return_cache and config.bagging_size == 1 and len(cache.pending) == 1:
                     _begin_tree(cache, config, True)
                 cb.finish(logger, i)
                 if i % print_every_n == 0 and verbosity > 0:

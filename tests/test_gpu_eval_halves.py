@@ -52,3 +52,16 @@ def test_a_fit_that_queues_ahead_of_its_evaluation(evt, rounds):
     assert a.info["logger"]["metrics"] == b.info["logger"]["metrics"] and len(a.trees) == len(b.trees)
     for s, t in zip(a.trees, b.trees):
         assert np.array_equal(s.feat, t.feat) and s.pred.tobytes() == t.pred.tobytes()
+
+
+@pytest.mark.parametrize("patience", [1, 2, 5])
+def test_early_stopping_drops_one_tree(evt, monkeypatch, patience):
+    """Of the trees queued ahead of the evaluation that ends a fit, one at most is grown for nothing."""
+    rng = np.random.default_rng(patience)
+    x, y = rng.random((900, 5)), rng.random(900)  # noise: the metric soon stops improving
+    queued, begin = [], evt._begin_tree
+    monkeypatch.setattr(evt, "_begin_tree", lambda *args: (queued.append(1), begin(*args))[1])
+    config = evt.EvoTreeRegressor(nrounds=60, max_depth=4, eta=0.3, early_stopping_rounds=patience)
+    m = evt.fit(config, x_train=x[:600], y_train=y[:600], x_eval=x[600:], y_eval=y[600:], verbosity=0)
+    kept = len(m.trees) - 1
+    assert kept < 58 and len(queued) == kept + 1
