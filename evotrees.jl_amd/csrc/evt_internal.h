@@ -350,13 +350,26 @@ static int guarded(F &&f) {
 __host__ __device__ __forceinline__ uint32_t evt_pack_node(int feat, int cond_bin, bool numeric) {
     return (uint32_t)feat | ((uint32_t)cond_bin << 16) | EVT_NODE_SPLIT | (numeric ? EVT_NODE_NUMERIC : 0u);
 }
-// Requests every 64-byte line of a kernel's arguments (BYTES of them) at once.  The compiler loads an argument where it is first needed, behind the branches before it, and
+// Bytes of the arguments of a kernel of type void(T...): they lie one after the other, as the members of a struct
+template <typename KERNEL>
+struct KernargBytes;
+template <typename... T>
+struct KernargBytes<void(T...)> {
+    static constexpr size_t sum() {
+        size_t at = 0;
+        ((at = (at + alignof(T) - 1) / alignof(T) * alignof(T) + sizeof(T)), ...);
+        return at;
+    }
+    static constexpr size_t value = sum();
+};
+static_assert(KernargBytes<void(uint8_t, double, int, uint16_t)>::value == 22, "as a struct's members");
+// Requests every 64-byte line of the arguments of a kernel, named by its type, at once.  The compiler loads an argument where it is first needed, behind the branches before it, and
 // each line so found is a trip to memory that nothing else hides: a launch's arguments are in no cache.  us a launch, with a chunk's descriptor requested beside the chunk
 // count: k_part_move 6.2 -> 5.9 (500k rows) and 7.3 -> 7.0 (800k), k_part_count 4.5 -> 4.3, k_part_scatter 5.0 -> 4.6, k_final_fused 5.8 -> 5.3 (60k), k_scan_mc 9.5 -> 9.2,
 // k_obliv_level 9.6 -> 9.3, k_tree_begin 8.3 -> 8.1; k_scan 6.05 -> 5.8 once its first requests wait for no argument; the histogram kernels gain nothing by it.
-template <size_t BYTES>
+template <typename KERNEL>
 __device__ __forceinline__ void touch_kernargs() {
-    constexpr int LAST = (int)(BYTES - 4) / 64;
+    constexpr int LAST = (int)(KernargBytes<KERNEL>::value - 4) / 64;
     static_assert(LAST < 12, "lines");
     const auto *k = (const __attribute__((address_space(4))) uint32_t *)__builtin_amdgcn_kernarg_segment_ptr();
 #define EVT_LINE(i_) "s"(k[((i_) < LAST ? (i_) : LAST) * 16])

@@ -97,7 +97,7 @@ template <bool NT>
 __global__ __launch_bounds__(256) void k_part_count(PartArgs A) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // the first descriptor is requested together with the level's chunk count (the grid never exceeds the table)
-    touch_kernargs<sizeof(PartArgs)>();
+    touch_kernargs<decltype(k_part_count<NT>)>();
     uint4 cd = A.cdesc[blockIdx.x];
     const int64_t n_chunks = A.hdr[LH_N_CHUNKS];
     asm volatile("" : "+v"(cd.x), "+v"(cd.y), "+v"(cd.z), "+v"(cd.w));
@@ -446,7 +446,7 @@ __global__ __launch_bounds__(256) void k_part_scatter(PartArgs A, NextArgs NX) {
     extern __shared__ unsigned long long s_H[]; // HNA > 0: [HNA][sampled features][bins]
     // fold 1: the level's bookkeeping rides along whole and the blocks add up their node's chunk counts themselves;
     // fold 2: the chunk counts were scanned by k_chunk_scan, only the next level's tables ride along
-    touch_kernargs<sizeof(PartArgs) + sizeof(NextArgs)>();
+    touch_kernargs<decltype(k_part_scatter<HNA, PACK>)>();
     const bool fold = A.fold == 1;
     if (blockIdx.x == gridDim.x - 1) { // the level's bookkeeping, beside the blocks that move the rows
         __shared__ uint4 s_child[512];
@@ -649,7 +649,7 @@ __global__ __launch_bounds__(T, 8) void k_part_move(PartArgs A, NextArgs NX) {
     __shared__ long long s_tmp[34];
     __shared__ int s_cnt[W];
     __shared__ unsigned long long s_claim;
-    touch_kernargs<sizeof(PartArgs) + sizeof(NextArgs)>();
+    touch_kernargs<decltype(k_part_move<NT, T, NI>)>();
     const int64_t G = (int64_t)gridDim.x - 1;
     if (blockIdx.x == 0) { // the next level's tables, beside the blocks that move the rows
         __shared__ uint4 s_child[512];
@@ -742,7 +742,7 @@ __global__ __launch_bounds__(T, 8) void k_part_move(PartArgs A, NextArgs NX) {
 template <bool NT>
 __global__ __launch_bounds__(256) void k_final_fused(PartArgs A) {
     const int tid = threadIdx.x;
-    touch_kernargs<sizeof(PartArgs)>();
+    touch_kernargs<decltype(k_final_fused<NT>)>();
     const int64_t G = (int64_t)gridDim.x - A.blob.blocks;
     if ((int64_t)blockIdx.x >= G) {
         // the tree's arrays are complete (this is the tree's last kernel and writes none of them): their way back to the
@@ -893,7 +893,7 @@ __device__ void tree_begin_root(const BeginArgs &A, int blocks) {
 // Blocks from `blocks` on quantise the gradients, which have nothing to do with the set-up: side by side in one launch where the gradients' words are
 // still to be made: set-up + quantisation, us, 500k rows of four channels 4.2 + 6.9 -> 7.0, 60k of 14 channels 3.0 + 7.9 -> 9.3 - and a launch each.
 __global__ __launch_bounds__(1024) void k_tree_begin(BeginArgs A, QuantArgs Q, int blocks) {
-    touch_kernargs<sizeof(BeginArgs) + sizeof(QuantArgs) + 4>();
+    touch_kernargs<decltype(k_tree_begin)>();
     if ((int)blockIdx.x >= blocks) {
         quant_rows(Q, (int)blockIdx.x - blocks, (int)gridDim.x - blocks);
         return;
@@ -953,7 +953,7 @@ template <bool DRAW>
 __global__ __launch_bounds__(256) void k_mask_sample(uint8_t *mask, uint8_t cond, int64_t N, unsigned long long seed, uint32_t *is_out,
                                                      unsigned long long *claims, BeginArgs B, QuantArgs Q, int blocks, int clear) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    touch_kernargs<48 + sizeof(BeginArgs) + sizeof(QuantArgs) + 8>();
+    touch_kernargs<decltype(k_mask_sample<DRAW>)>();
     const int own_block = (int)blockIdx.x - 1, set_up = blocks + clear;
     if (own_block >= set_up) { // as k_tree_begin
         quant_rows(Q, own_block - set_up, (int)gridDim.x - 1 - set_up);

@@ -132,7 +132,7 @@ __global__ __launch_bounds__(1024) void k_small_path(PathArgs A) {
     __shared__ double s_S[NK], s_gain_p;  // statistics and gain of the path's node, below the root
     __shared__ int s_len[2], s_in[2];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    touch_kernargs<sizeof(PathArgs)>();
+    touch_kernargs<decltype(k_small_path<NAG, BPL, PACK>)>();
     const int b = blockIdx.x, B = A.B, N = A.N, nfs = A.nfs, splits = A.D - 1, words = nfs * NA * B, pieces = (nfs + 15) >> 4;
     // [row][piece] of 16 bytes.  A record starts with another feature of the sample from row to row (byte t: feature (row + t) % nfs), so that lanes that add the
     // same byte of their rows add to different features: lanes that add to one bin wait for each other, and of one feature's 64 bins 64 lanes share many (4000 rows x

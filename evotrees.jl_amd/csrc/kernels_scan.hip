@@ -152,7 +152,7 @@ __global__ __launch_bounds__(FUSED ? 1024 : 256) void k_scan(const uint32_t *js,
     const bool have = jp < nfs; // wave-uniform; a wave past the last feature loads the last one's data and drops it
     const int jpc = have ? jp : nfs - 1;
     int f = (int)js[jpc], st = status[n];
-    touch_kernargs<48 + sizeof(ScanArgs)>();
+    touch_kernargs<decltype(k_scan<NAG, BPL, FUSED>)>();
     asm volatile("" : "+s"(f), "+s"(st)); // both are requested before either is waited for, and ahead of the branch on the state
     if (st != ST_BUILD && st != ST_SUBTRACT) return;
     f -= 1;
@@ -758,7 +758,7 @@ __global__ __launch_bounds__(NAG * BPL > 12 ? 512 : 1024) void k_obliv_level(Obl
     __shared__ int s_last, s_bin, s_cell;
     __shared__ double s_best;
     const OblivArgs &A = L.o;
-    touch_kernargs<sizeof(OblivLevelArgs)>();
+    touch_kernargs<decltype(k_obliv_level<NAG, BPL, NPW>)>();
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
     constexpr int K = (NAG == 5) ? 2 : 1, NK = 2 * K + 1;
     const int B = A.B, jp = blockIdx.x;
@@ -1051,7 +1051,7 @@ template <int BPL, bool LOOP>
 __global__ __launch_bounds__(64 * (EVT_MAX_K / 2)) void k_scan_mc(ScanArgs A) {
     extern __shared__ double s_term[]; // [K][B]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
-    touch_kernargs<sizeof(ScanArgs)>();
+    touch_kernargs<decltype(k_scan_mc<BPL, LOOP>)>();
     const int nodeidx = blockIdx.x, n = (1 << (A.level - 1)) + nodeidx, jp = blockIdx.y;
     int f = (int)A.js[jp] - 1;
     const int st = A.status[n];
