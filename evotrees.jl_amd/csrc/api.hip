@@ -426,7 +426,7 @@ extern "C" int evt_create(int64_t nobs, int32_t nfeats, int32_t nbins, int32_t K
     // pinned staging: tree read-back + small per-tree uploads; coherent: wait_for_tree reads it while the kernel that fills it runs
     c->h_stage_bytes = c->blob_bytes + (size_t)c->F * 4 + (size_t)c->RS * 2 + 1024;
     c->h_stage_bytes = (c->h_stage_bytes + 255) / 256 * 256;
-    if (!c->mc && tree_type != EVT_TREE_OBLIVIOUS && c->D >= 2 && c->D <= 10) {
+    if (!c->mc && tree_type != EVT_TREE_OBLIVIOUS && c->D >= 2 && c->D <= EVT_PATH_DEPTH) {
         c->path_off = c->h_stage_bytes;
         c->h_stage_bytes += ((size_t)c->nnodes * sizeof(PathNode) + 8 * EVT_PATH_BLOCKS + 255) / 256 * 256;
     }

@@ -74,7 +74,9 @@ struct PathNode {
     uint32_t rows; // of the sample, of a node that was searched
     float w, gain, pred[2];
 };
-#define EVT_PATH_BLOCKS 256
+// Trees of one launch: the deepest, and its blocks, one to each node of the last level that splits - each has a word of the slot
+#define EVT_PATH_DEPTH 10
+#define EVT_PATH_BLOCKS (1 << (EVT_PATH_DEPTH - 2))
 
 struct TreeDev {
     int32_t *feat;    // 1-based, 0 none
@@ -487,7 +489,7 @@ int small_tree_form(const evt_ctx *c, int nfs, bool all_rows);
 bool small_root_quantises(const evt_ctx *c, int form);
 int launch_small_tree(evt_ctx *c, const evt_params *p, bool draw, int slices);
 #define SMALL_PATH (-1) // of small_tree_form: the whole tree in one launch
-bool small_path_takes(const evt_ctx *c, int nfs, bool whatever);
+bool small_path_takes(const evt_ctx *c, int nfs, bool wherever);
 int launch_small_path(evt_ctx *c, const evt_params *p, bool draw);
 int launch_final_fused(evt_ctx *c, int level, const uint32_t *is_cur, bool fuse_pred, bool send_blob);
 int launch_nidx_from_segments(evt_ctx *c, int level, const uint32_t *is_cur);

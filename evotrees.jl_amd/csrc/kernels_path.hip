@@ -15,7 +15,6 @@
 
 #define PATH_MAX_ROWS 32767 // a row and its mark are 16 bits of a list
 #define PATH_MAX_FEATS 64
-#define PATH_MAX_DEPTH 10
 #define PATH_OUT 0x8000u    // the row is not in the sample
 #define PATH_NUMERIC (1u << 16)
 #define PATH_LDS (148 * 1024)
@@ -628,7 +627,7 @@ int launch_small_path(evt_ctx *c, const evt_params *p, bool draw) {
         A.feat[j] = (uint32_t)f | (c->h_feattypes[f] ? PATH_NUMERIC : 0u) | ((uint32_t)(c->h_mono[f] + 1) << 17);
     }
     const size_t lds = path_lds(c, A.nfs);
-    const unsigned blocks = 1u << (c->D - 2);
+    const unsigned blocks = 1u << (c->D - 2); // at most EVT_PATH_BLOCKS: path_off
     prof_begin(c, EVT_K_PARTITION, 1);
 #define PATH3(NAG_, BPL_, PACK_)                                                                                                                                  \
     {                                                                                                                                                             \
