@@ -365,18 +365,23 @@ struct KernargBytes<void(T...)> {
     static constexpr size_t value = sum();
 };
 static_assert(KernargBytes<void(uint8_t, double, int, uint16_t)>::value == 22, "as a struct's members");
-// Requests every 64-byte line of the arguments of a kernel, named by its type, at once.  The compiler loads an argument where it is first needed, behind the branches before it, and
+// Requests every 64-byte line of a kernel's first BYTES of arguments at once.  The compiler loads an argument where it is first needed, behind the branches before it, and
 // each line so found is a trip to memory that nothing else hides: a launch's arguments are in no cache.  us a launch, with a chunk's descriptor requested beside the chunk
 // count: k_part_move 6.2 -> 5.9 (500k rows) and 7.3 -> 7.0 (800k), k_part_count 4.5 -> 4.3, k_part_scatter 5.0 -> 4.6, k_final_fused 5.8 -> 5.3 (60k), k_scan_mc 9.5 -> 9.2,
 // k_obliv_level 9.6 -> 9.3, k_tree_begin 8.3 -> 8.1; k_scan 6.05 -> 5.8 once its first requests wait for no argument; the histogram kernels gain nothing by it.
-template <typename KERNEL>
-__device__ __forceinline__ void touch_kernargs() {
-    constexpr int LAST = (int)(KernargBytes<KERNEL>::value - 4) / 64;
+template <size_t BYTES>
+__device__ __forceinline__ void touch_kernarg_bytes() {
+    constexpr int LAST = (int)(BYTES - 4) / 64;
     static_assert(LAST < 12, "lines");
     const auto *k = (const __attribute__((address_space(4))) uint32_t *)__builtin_amdgcn_kernarg_segment_ptr();
 #define EVT_LINE(i_) "s"(k[((i_) < LAST ? (i_) : LAST) * 16])
     asm volatile("" ::EVT_LINE(0), EVT_LINE(1), EVT_LINE(2), EVT_LINE(3), EVT_LINE(4), EVT_LINE(5), EVT_LINE(6), EVT_LINE(7), EVT_LINE(8), EVT_LINE(9), EVT_LINE(10), EVT_LINE(11));
 #undef EVT_LINE
+}
+// ... of all arguments of a kernel, named by its type
+template <typename KERNEL>
+__device__ __forceinline__ void touch_kernargs() {
+    touch_kernarg_bytes<KernargBytes<KERNEL>::value>();
 }
 // The word of a row whose one channel shares it with the row count, staged as 32 bits (30 of gradient, half the plane to gather from) and widened here to (q << 16) + 1.
 __device__ __forceinline__ unsigned long long evt_load_narrow(const unsigned long long *__restrict__ gq, uint32_t id) {

@@ -470,10 +470,10 @@ __device__ __forceinline__ void small_search(const SmallArgs &A, const double *q
     }
 }
 
-// Requests every 64-byte line of the arguments at once: read where each is needed, they were ten trips one after the other.
-__device__ __forceinline__ void touch_args(const SmallArgs &A) {
-    asm volatile("" ::"s"(A.xcm), "s"(A.left_in), "s"(A.js_src), "s"(A.qscale), "s"(A.qexp), "s"(A.stats), "s"(A.gamma), "s"(A.nfs), "s"(A.cond));
-}
+// Requests the arguments at once, but for the features, of which a block needs its own: read where each is needed, they were ten trips one after the other.  us a round,
+// with nine fields named by hand before | this: one block a feature, 30k rows x 10 of two outputs, depth 6 135.6 | 134.4, 8k x 30 72.4 | 70.8; shared rows, the same
+// 79.3 | 77.9, 74.9 | 73.2; weighted, two outputs of 192 bins, 21k x 16 198 | 170 (the search of five channels spills less: 87 -> 71 registers of its 256 bins).
+__device__ __forceinline__ void touch_small_args() { touch_kernarg_bytes<offsetof(SmallArgs, feat)>(); }
 
 // An oblivious level's row of one feature (grow_otree!, src/fit.jl:190-217), by one wavefront: the gains of the level's nodes added in
 // node order, zero where one of them is not positive, and the first maximum over the bins.
@@ -520,7 +520,7 @@ __global__ __launch_bounds__(1024) void k_small_level(SmallArgs A) {
     __shared__ int s_nact, s_cnt, s_best;
     __shared__ double s_qs[EVT_MC_MAX_NK], s_qmul[EVT_MC_MAX_NK]; // scales of the channels; multipliers of the gradient rows (raw)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    touch_args(A);
+    touch_small_args();
     constexpr bool ROOT = FORM != SMALL_BELOW, QUANT = FORM == SMALL_ROOT;
     const int B = A.B, N = A.N, level = ROOT ? 1 : A.level;
     __builtin_assume(ROOT || level > 1);
@@ -893,7 +893,7 @@ __global__ __launch_bounds__(1024) void k_small_scan(SmallArgs A) {
     __shared__ uint16_t s_node[SMALL_MAX_NODES];
     __shared__ int s_nact, s_best;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    touch_args(A);
+    touch_small_args();
     const int nag = NAG ? NAG : A.NAg, jp = blockIdx.x, first = 1 << (A.level - 1), words = nag * A.B;
     const int mine = (int)blockIdx.y * 16 + wave;
     const int st = A.status[first + (mine < first ? mine : 0)];
@@ -963,7 +963,7 @@ __global__ __launch_bounds__(1024) void k_small_final(SmallArgs A) {
     constexpr int K = LOSS == 2 || LOSS == 7 ? 2 : 1, NK = 2 * K + 1;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const bool writer = blockIdx.x == 0;
-    touch_args(A);
+    touch_small_args();
     const int np = 1 << (A.level - 2);
     long long *s_tot = reinterpret_cast<long long *>(s_dyn);
     long long *s_own = GRADS ? s_tot + 2 * np * A.NAg : nullptr;
