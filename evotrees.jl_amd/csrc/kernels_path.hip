@@ -6,7 +6,9 @@
 // paths share a node repeat its work on compute units that would have nothing to do otherwise, so no block waits for another and none need be resident
 // together; all of them add the same integers and so decide alike.  The first block under a node is the node's owner: it writes the node's part of the tree, its
 // histogram, and, of a leaf, its rows.
-// What a block reads of other rows (bins, gradients, mask) nobody writes in this launch: the next gradients go to a second array, their maxima to a third set.
+// What a block uses of other blocks' rows (bins, gradients, mask) nobody writes in this launch: the next gradients go to a second array, their maxima to a third set.
+// Predictions alone are read and written in one array: a block requests those of all rows, and by then a block that has finished may have added its leaves' values
+// to its own.  It uses only those of the rows it finishes itself, which no other block writes (each row ends in one leaf, and a leaf's rows are its owner's).
 // The sums are the same integers and the gains the same expressions as in the other kernels: same trees, bit for bit.
 #include "grad_math.h"
 #include "pool.h"
@@ -162,7 +164,7 @@ __global__ __launch_bounds__(1024) void k_small_path(PathArgs A) {
             r.m = A.sampled && !A.draw ? A.mask[row] : 0;
 #pragma unroll
             for (int a = 0; a < NA; a++) r.g[a] = A.raw[(size_t)row * NK + (NAG == 2 && a == 1 ? 2 : a)];
-            if (A.grad_loss >= 0) { // for the next gradients: a trip to memory less at the end
+            if (A.grad_loss >= 0) { // for the next gradients: a trip to memory less at the end; old or new, of rows that another block finishes, and then not used
 #pragma unroll
                 for (int k = 0; k < K; k++) r.pr[k] = A.pred[(size_t)K * row + k];
                 r.y = A.y[row];
@@ -558,9 +560,12 @@ static bool path_can(const evt_ctx *c, int nfs) {
 
 // Whether a tree takes it.  A level costs a round of the searches for every 16 features, by channels and bins, and every path adds all rows of the root; the kernels of
 // one level each (kernels_small.hip) spread the features over blocks and pay a launch and four trips to memory a level.  Both in microseconds a round, fitted to 500
-// rounds of 30 to 6000 rows, 1 to 64 features, 2 to 255 bins and depths 2 to 10 that fit LDS: taken for three in four of them, whose rounds take 0.53 of the time in the
-// mean; one takes more than 3 % longer than without (1.13), against the better of both 1.012 in the mean.  10 features, 64 bins, depth 6, us a round in one launch | one a
-// level: 500 rows 28 | 47, 2000 34 | 50, 4000 44 | 54; 1000 rows, depth 2 16 | 16, 10 45 | 139; 20 features 39 | 48, 32 50 | 48.
+// rounds of an earlier state of the kernel and checked on 1535 shapes that the present one can hold: 30 to 4735 rows (the most, of one feature and two bins), 1 to 64
+// features, 2 to 255 bins, depths 2 to 10.  1201 of them take it, whose rounds take 0.61 of the time in the mean; 33 of these take more than 3 % longer, 12 more than
+// 10, the worst 1.21 (29 to 43 features of two bins; few rows of 255).  Of the 334 others 38 would gain more than 3 %, the most 37; all together 1.005 of the better form.
+// Fitted again to 1035 of them it lost 6 shapes for 33, but 15 of the other 500 took 3 to 37 % longer than by these figures.
+// 10 features, 64 bins, depth 6, us a round in one launch | one a level: 500 rows 26 | 44, 2000 34 | 47, 4000 43 | 50;
+// 1000 rows, depth 2 16 | 13, 10 43 | 123; 1000 rows of 20 features 38 | 46, of 32 49 | 46.
 bool small_path_takes(const evt_ctx *c, int nfs, bool wherever) {
     if (!path_can(c, nfs)) return false;
     if (wherever) return true;
