@@ -1138,7 +1138,8 @@ static bool part_in_one_pass(const evt_ctx *c) { return c->part_one_pass && c->u
 
 // Rows of a chunk of the level.  A node's chunks queue at its cursor, ~20 ns each: where a node has more than 128 of them they grow (us a level of
 // 1M rows, 2048 | 4096 | 8192 rows a chunk: root 11.7 | 8.9 | 9.0, two nodes 9.0 | 7.6 | 8.4, eight 6.8 | 6.8 | 8.3; 10M: 67 | 39 | 28, 62 | 36 | 28,
-// 34 | 28 | 23; 8192 | 16384, blocks of 1024: one to four nodes 31 | 26, 29 | 24, 29 | 26, eight 30 | 34, whose nodes of 1.25M rows keep the narrower).  They grow too where the level is more blocks than the chip holds at once and nodes are many chunks (10M rows, 64 nodes 44 | - | 40).
+// 34 | 28 | 23; 8192 | 16384, blocks of 1024: one to four nodes 31 | 26, 29 | 24, 29 | 26, eight 30 | 34, whose nodes of 1.25M rows keep the narrower;
+// whole rounds of 10 to 40 features: 2.2M to 6M rows level within 0.7 % either way, 7M 290 | 285, 8M 317 | 311, 9M 352 | 346, 20M 1447 | 1439).  They grow too where the level is more blocks than the chip holds at once and nodes are many chunks (10M rows, 64 nodes 44 | - | 40).
 int part_chunk_rows(const evt_ctx *c, int level) {
     int rows = EVT_CHUNK;
     if (!part_in_one_pass(c) || level >= c->D - 1) return rows;

@@ -387,7 +387,10 @@ int evt_predict_static(void *stream, int64_t nobs, int32_t nfeats, const uint8_t
                        int32_t apply_link, float *out_dev, int32_t *status_dev);
 
 /* ---- measurement ---------------------------------------------------------------------
- * Kernel classes timed with HIP events on the handle's stream when profiling is on. */
+ * Kernel classes timed with HIP events on the handle's stream when profiling is on.  Kernels that do the work of several classes
+ * count as one: a tree of one launch is one PARTITION launch, and none of HIST or SCAN; of one kernel per level, the root's is a
+ * HIST launch and the others PARTITION; histograms from the partition's scatter pass and a tree's gradients computed by its last kernel
+ * count with that kernel (see "small_tree", "hist_in_scatter" and "grads_ahead" below). */
 enum {
     EVT_K_GRAD = 0,
     EVT_K_HIST = 1,
