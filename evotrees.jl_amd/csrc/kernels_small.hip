@@ -1106,12 +1106,12 @@ static int small_tree_buffers(evt_ctx *c, bool split) {
 // rows / S, the channels and - through the candidates every block reads and the searches its 16 wavefronts share - the nodes; slices
 // add the words they flush and, where a level is searched apart, a launch.  The other path spreads rows of any number over the chip and pays for its launches.
 // Estimates in microseconds, fitted to rounds of an earlier state of these kernels and checked on the present ones (500 to 300k rows, 3 to 250 features, depths 3 to
-// 10): of 364 shapes of one or two outputs 328 take a form within 4 % of the best and 353 within 10, the worst 1.32 times the best; of 186 of several outputs 149
-// and 157, the worst 1.65, where the other path, which has since become faster than its estimate, is not taken (profiles/rule_small_tree.txt).
+// 10): of 364 shapes of one or two outputs 313 take a form within 4 % of the best and 334 within 10, the worst 1.44 times the best; of 186 of several outputs 141
+// and 154, the worst 1.92, where the other path, which has since become faster than its estimate, is not taken (profiles/rule_small_tree.txt).
 // What a further walk of all channels costs whatever its rows was added for those: 16 classes, 192 bins, 893 rows x 3, depth 6 906 -> 244 us, 14 classes, 160 bins,
 // 1558 x 4, depth 9 1209 -> 337; of 1658 shapes one takes more than 3 % longer by it.
-// A round of depth 6, 64 bins and 8 features as a fit queues it, microseconds for the other path, S = 1 and S > 1: mse 103, 58, 75 at 2k rows, 115, 109, 77 at 30k,
-// 127, -, 91 at 250k; 3 classes 146, 132, 121 at 8k, 161, 501, 139 at 60k, 190, -, 197 at 250k; 7 classes 148, 157, 184 at 2k, 186, -, 225 at 120k, 223, -, 299 at 250k.
+// A round of depth 6, 64 bins and 8 features as a fit queues it, microseconds for the other path, S = 1 and S > 1: mse 82, 48, 64 at 2k rows (31 in one launch), 91, 101, 66 at
+// 30k, 104, -, 79 at 250k; 3 classes 125, 122, 113 at 8k, 147, 482, 129 at 60k, 173, -, 187 at 250k; 7 classes 129, 147, 170 at 2k, 181, -, 254 at 120k, 220, -, 341 at 250k.
 int small_tree_form(const evt_ctx *c, int nfs, bool all_rows) {
     if (!c->small_tree || c->D < 2 || c->D > 10 || nfs > 256 || c->N < 4 || c->N > (1 << 24) || !c->defer_pred || EVT_IS_QUANTILE(c->loss)) return 0;
     if (c->record_nidx && !all_rows) return 0;
